@@ -333,10 +333,11 @@ int pskv_host_trim(void);
 int pskv_table_counters(pskv_table* t, uint64_t* out, size_t cap);
 
 /* Device memory the library keeps for reuse goes back to the system (no counterpart in the
- * reference): the slot arrays and row storage that growths have replaced (they stay in a
- * memory pool of the library, one per device, because releasing a few hundred MB costs
- * hundreds of microseconds that would land in the caller's next wait; the pool reuses them
- * for later growths of any table, and gives them up when this is called) and the workspaces
+ * reference): the slot arrays, row storage and request buffers that growths have replaced or that
+ * destroyed tables have left (up to 8 GiB per device stay on a list of the library, because
+ * releasing and allocating a few hundred MB costs from hundreds of microseconds to hundreds of
+ * milliseconds; the list serves later growths and tables, of any thread and stream), the fixed-size
+ * state and pinned request buffers of destroyed tables (up to 32 of them) and the workspaces
  * and staging buffers of pskv_match, which only grow (a 16M-key host-resident call leaves
  * several GiB behind). Memory in use by live tables is not touched. Calls of pskv_match on
  * the device wait for it and it for them. */

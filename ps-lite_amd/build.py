@@ -10,8 +10,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpskv.so")
-SOURCES = ["table.hip", "slice.hip", "hostmem.hip", "stager.hip", "match.hip", "meta_codec.cc"]
-HEADERS = ["device_common.h", "host_common.h", "scan.h", "stager.h", "table_kernels.h"]
+SOURCES = ["table.hip", "slice.hip", "hostmem.hip", "stager.hip", "devpool.hip", "match.hip", "meta_codec.cc"]
+HEADERS = ["device_common.h", "devpool.h", "host_common.h", "scan.h", "stager.h", "table_kernels.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -18,6 +18,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "devpool.h"
 #include "host_common.h"
 #include "scan.h"
 #include "stager.h"
@@ -76,19 +77,6 @@ struct EventPair {
   hipEvent_t a, b;
 };
 
-// An allocation handed to the library's allocating thread (AllocWorker below).
-struct AllocJob {
-  int device = 0;
-  size_t bytes = 0;
-  hipStream_t stream = nullptr;
-  void* ptr = nullptr;
-  bool pooled = false;
-  int rc = PSKV_OK;
-  double took_us = 0;  // what the allocation cost the allocating thread
-  bool done = false;  // guarded by AllocWorker::mu
-};
-
-
 // What the host reads back of the device state, written by the device into pinned host memory
 // (a one-wavefront kernel is quicker than a copy command for these few words).
 struct StateView {
@@ -98,6 +86,14 @@ struct StateView {
   uint64_t same_epoch;
   unsigned error, req_error, special_present, pad;
 };
+
+// A new table's device state: all zero, the side slot's payload unset. One workgroup.
+__global__ void k_init_state(DevState* st) {
+  unsigned long long* w = reinterpret_cast<unsigned long long*>(st);
+  constexpr unsigned kAt = offsetof(DevState, special_payload) / 8;
+  static_assert(sizeof(DevState) % 8 == 0, "the state is cleared word by word");
+  for (unsigned i = threadIdx.x; i < sizeof(DevState) / 8; i += blockDim.x) w[i] = i == kAt ? kPayloadUnset : 0ull;
+}
 
 // One wavefront per table (blockIdx.x).
 struct StateBatch {
@@ -120,6 +116,84 @@ __global__ void k_read_state(StateBatch sb) {
   out->special_present = st->special_present;
 }
 
+// The parts of a table that have one size whatever the table holds: device state, the pinned words and
+// request buffers, events. Creating them costs the calling thread about a millisecond (every
+// pinned allocation and its release go through the driver), so a table that goes leaves its shell to
+// the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim.
+struct Shell {
+  DevState* st = nullptr;
+  char* pinned = nullptr;  // StateView, Snapshot, outcome word (256 bytes each), small_in, small_out
+  hipEvent_t done[kSmallParts] = {nullptr};
+};
+constexpr size_t kShellsKept = 32;
+
+struct ShellPool {
+  std::mutex mu;
+  std::vector<Shell*> idle;
+};
+ShellPool g_shells[64];
+
+void shell_free(Shell* sh) {
+  if (!sh) return;
+  if (sh->st) (void)hipFree(sh->st);
+  if (sh->pinned) (void)hipHostFree(sh->pinned);
+  for (hipEvent_t e : sh->done)
+    if (e) (void)hipEventDestroy(e);
+  delete sh;
+}
+
+// A shell for a table on `device` (current): one whose last table is gone (nothing on the GPU uses it any
+// more) if there is one.
+Shell* shell_take(int device) {
+  Shell* sh = nullptr;
+  if (device < 64) {
+    ShellPool& p = g_shells[device];
+    std::lock_guard<std::mutex> lk(p.mu);
+    if (!p.idle.empty()) {
+      sh = p.idle.back();
+      p.idle.pop_back();
+    }
+  }
+  if (!sh) {
+    sh = new (std::nothrow) Shell();
+    if (!sh) return nullptr;
+    // coherent: the GPU does not cache this memory, so each request sees what the host just wrote
+    bool ok = hipMalloc(reinterpret_cast<void**>(&sh->st), sizeof(DevState)) == hipSuccess &&
+              hipHostMalloc(reinterpret_cast<void**>(&sh->pinned), 1024 + 2 * kSmallBytes, hipHostMallocCoherent) ==
+                  hipSuccess;
+    for (int q = 0; ok && q < kSmallParts; ++q)
+      ok = hipEventCreateWithFlags(&sh->done[q], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+      shell_free(sh);
+      return nullptr;
+    }
+  }
+  return sh;
+}
+
+void shell_give(int device, Shell* sh) {
+  if (!sh) return;
+  if (device < 64) {
+    ShellPool& p = g_shells[device];
+    std::lock_guard<std::mutex> lk(p.mu);
+    if (p.idle.size() < kShellsKept) {
+      p.idle.push_back(sh);
+      return;
+    }
+  }
+  shell_free(sh);
+}
+
+// pskv_device_trim (with `device` current): idle shells go.
+void shell_trim(int device) {
+  std::vector<Shell*> go;
+  {
+    std::lock_guard<std::mutex> lk(g_shells[device].mu);
+    go.swap(g_shells[device].idle);
+  }
+  for (Shell* sh : go) shell_free(sh);
+}
+
 }  // namespace
 }  // namespace pskv
 
@@ -133,14 +207,12 @@ struct pskv_table {
   float max_load = 0.5f;
 
   Slot* slots = nullptr;
-  bool slots_pooled = false, arena_pooled = false;  // taken from the stream-ordered pool by a growth
   uint64_t cap = 0;        // slots, a power of two
   // The array the next growth will move into, allocated ahead of need (once the table is 40 % of
   // the way to that growth) at the end of a request, while the GPU is busy with that request:
   // allocating costs the host 50-100 us, which would otherwise be spent with the GPU idle.
   Slot* spare = nullptr;
   uint64_t spare_cap = 0;
-  bool spare_pooled = false;
   std::shared_ptr<AllocJob> spare_job;  // the allocation of `spare` while it is under way
   // what the sizing logic did, printed when the table goes if PSKV_STATS is set in the environment
   struct Stats {
@@ -175,6 +247,7 @@ struct pskv_table {
   GrowBuf ws;         // per-request workspace (row references, offsets)
   GrowBuf tiles;      // VARLEN: first key of every request-side tile
   GrowBuf tiles_aff;  // VARLEN: one TileNote per tile
+  Shell* shell = nullptr;     // what st, st_host, snap, outcome and small_* belong to
   char* small_in = nullptr;   // pinned, kSmallBytes: small host-resident requests, read in place
   char* small_out = nullptr;  // pinned, kSmallBytes: their responses, written in place
   // A small host-resident SCALAR push returns once its kernel is queued: nothing comes back from
@@ -227,7 +300,6 @@ struct pskv_table {
   unsigned long long sc_seen = 0;         // the value of *outcome the host last looked at
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
 
-  bool counted = false;  // among the live tables of its device
   bool prof = false;
   std::vector<EventPair> pending[PSKV_KERNEL_COUNT];
   std::vector<EventPair> free_events;
@@ -293,29 +365,6 @@ int prof_collect(pskv_table* t) {
 }
 
 // ---- memory ----------------------------------------------------------------------
-int grow(pskv_table* t, GrowBuf* b, size_t bytes) {
-  if (bytes <= b->bytes) return PSKV_OK;
-  if (t->capturing) return set_error(PSKV_ESTALE, "a recorded request needs a buffer that its first run did not leave");
-  // An eighth to spare (up to 32 MB): the slices of a worker's requests differ by a few keys from one
-  // request to the next, and a reallocation waits for the stream and costs 100-350 us, several
-  // requests' worth, every time a table sees its largest slice so far.
-  size_t want = std::max(bytes + std::min<size_t>(bytes / 8, (size_t)32 << 20), b->bytes + b->bytes / 2);
-  want = (want + 4095) & ~(size_t)4095;
-  if (b == &t->ws || b == &t->tiles || b == &t->tiles_aff || b == &t->cache_keys ||
-      b == &t->cache_lens || b == &t->sc_vals || b == &t->sc_slots)
-    t->cache_valid = false;  // the contents do not survive a reallocation
-  if (b->ptr) {
-    // earlier requests on the stream may still read the old buffer
-    PSKV_HIP(hipStreamSynchronize(t->stream));
-    PSKV_HIP(hipFree(b->ptr));
-    b->ptr = nullptr;
-    b->bytes = 0;
-  }
-  PSKV_HIP(hipMalloc(&b->ptr, want));
-  b->bytes = want;
-  return PSKV_OK;
-}
-
 // Carves aligned pieces out of a GrowBuf that was grown to the total beforehand.
 struct Carver {
   char* base;
@@ -374,151 +423,35 @@ int report_device_errors(pskv_table* t) {
   return set_error(PSKV_ELEN_CHANGED, "a pushed row length differs from the stored length");
 }
 
-// Slot arrays and arenas come from, and go back to, the device's stream-ordered pool where the
-// runtime has one (PSKV_NO_ASYNC_ALLOC in the environment goes back to hipMalloc / hipFree): a
-// growth releases the old array behind the kernel that empties it, without a wait on the host
-// (a plain hipFree of a few hundred MB blocks the host for 150-440 us, longer than the
-// re-insertion itself). `pooled` says how the array must be released later.
-// The pool is the library's own, one per device, and keeps what is freed into it: the default
-// pool hands freed memory back to the system at the next wait of any stream, which for the old
-// array of a growth is an unmapping of hundreds of microseconds in the middle of the caller's
-// loop. pskv_device_trim gives the kept memory back; so does the end of the last table.
-struct DevicePool {
-  std::atomic<int> known{0};  // 0 = not asked yet, 1 = no pool, 2 = pool
-  hipMemPool_t pool = nullptr;
-  std::atomic<long> tables{0};  // live tables on the device
-};
-DevicePool g_pools[64];
-
-hipMemPool_t device_pool(int dev) {
-  if (dev < 0 || dev >= 64) return nullptr;
-  DevicePool& dp = g_pools[dev];
-  int k = dp.known.load(std::memory_order_acquire);
-  if (k == 0) {
-    static std::mutex mu;
-    std::lock_guard<std::mutex> lock(mu);
-    k = dp.known.load(std::memory_order_acquire);
-    if (k == 0) {
-      int ok = 0;
-      if (std::getenv("PSKV_NO_ASYNC_ALLOC") ||
-          hipDeviceGetAttribute(&ok, hipDeviceAttributeMemoryPoolsSupported, dev) != hipSuccess)
-        ok = 0;
-      if (ok) {
-        hipMemPoolProps props;
-        std::memset(&props, 0, sizeof(props));
-        props.allocType = hipMemAllocationTypePinned;
-        props.handleTypes = hipMemHandleTypeNone;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        uint64_t keep = ~0ull;
-        if (hipMemPoolCreate(&dp.pool, &props) != hipSuccess ||
-            hipMemPoolSetAttribute(dp.pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
-          dp.pool = nullptr;
-          ok = 0;
-        }
-      }
-      (void)hipGetLastError();
-      k = ok ? 2 : 1;
-      dp.known.store(k, std::memory_order_release);
-    }
-  }
-  return k == 2 ? dp.pool : nullptr;
-}
-
-int alloc_for_growth(void** out, size_t bytes, hipStream_t stream, bool* pooled) {
-  int dev = 0;
-  hipMemPool_t pool = hipGetDevice(&dev) == hipSuccess ? device_pool(dev) : nullptr;
-  if (pool) {
-    if (hipMallocFromPoolAsync(out, bytes, pool, stream) == hipSuccess) {
-      *pooled = true;
-      return PSKV_OK;
-    }
-    (void)hipGetLastError();
-  }
-  *pooled = false;
-  PSKV_HIP(hipMalloc(out, bytes));
-  return PSKV_OK;
-}
-
-// Allocating a few hundred MB costs the calling thread 50 us on a good day and 800 on a bad one,
-// so the array of a coming growth is allocated by a thread of the library's own while the
-// caller goes on enqueuing requests; the growth picks the result up (and waits for it in the
-// unlikely case that it is not there yet). One thread per process, started with the first job,
-// kept until the process ends.
-class AllocWorker {
- public:
-  static AllocWorker& get() {
-    static AllocWorker* w = new AllocWorker();  // never destroyed: its thread may outlive static destructors
-    return *w;
-  }
-  void submit(const std::shared_ptr<AllocJob>& job) {
-    {
-      std::lock_guard<std::mutex> lk(mu_);
-      if (!started_) {
-        std::thread(&AllocWorker::run, this).detach();
-        started_ = true;
-      }
-      jobs_.push_back(job);
-    }
-    cv_job_.notify_one();
-  }
-  void wait(const std::shared_ptr<AllocJob>& job) {
-    std::unique_lock<std::mutex> lk(mu_);
-    cv_done_.wait(lk, [&] { return job->done; });
-  }
-  bool finished(const std::shared_ptr<AllocJob>& job) {
-    std::lock_guard<std::mutex> lk(mu_);
-    return job->done;
-  }
-
- private:
-  void run() {
-    for (;;) {
-      std::shared_ptr<AllocJob> job;
-      {
-        std::unique_lock<std::mutex> lk(mu_);
-        cv_job_.wait(lk, [&] { return !jobs_.empty(); });
-        job = jobs_.front();
-        jobs_.pop_front();
-      }
-      const auto a0 = std::chrono::steady_clock::now();
-      if (hipSetDevice(job->device) != hipSuccess) {
-        (void)hipGetLastError();
-        job->rc = PSKV_EHIP;
-      } else {
-        job->rc = alloc_for_growth(&job->ptr, job->bytes, job->stream, &job->pooled);
-      }
-      job->took_us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - a0).count();
-      {
-        std::lock_guard<std::mutex> lk(mu_);
-        job->done = true;
-      }
-      cv_done_.notify_all();
-    }
-  }
-  std::mutex mu_;
-  std::condition_variable cv_job_, cv_done_;
-  std::deque<std::shared_ptr<AllocJob>> jobs_;
-  bool started_ = false;
-};
-
-// Releases an array that kernels already enqueued on `stream` may still use.
-int release_after(void* ptr, bool pooled, hipStream_t stream) {
-  if (!ptr) return PSKV_OK;
-  if (pooled) {
-    PSKV_HIP(hipFreeAsync(ptr, stream));
-    return PSKV_OK;
-  }
-  PSKV_HIP(hipStreamSynchronize(stream));
-  PSKV_HIP(hipFree(ptr));
-  return PSKV_OK;
-}
-
-int alloc_slots(uint64_t cap, Slot** out, hipStream_t stream, bool* pooled, bool fill = true) {
-  int rc = alloc_for_growth(reinterpret_cast<void**>(out), cap * sizeof(Slot), stream, pooled);
+int alloc_slots(uint64_t cap, Slot** out, hipStream_t stream, bool fill = true) {
+  int rc = array_alloc(reinterpret_cast<void**>(out), cap * sizeof(Slot), stream);
   if (rc) return rc;
   // all-ones bytes: key = empty marker (k_regrow writes every slot itself and needs no fill)
   if (fill) PSKV_HIP(hipMemsetAsync(*out, 0xFF, cap * sizeof(Slot), stream));
+  return PSKV_OK;
+}
+
+int grow(pskv_table* t, GrowBuf* b, size_t bytes) {
+  if (bytes <= b->bytes) return PSKV_OK;
+  if (t->capturing) return set_error(PSKV_ESTALE, "a recorded request needs a buffer that its first run did not leave");
+  // An eighth to spare (up to 32 MB): the slices of a worker's requests differ by a few keys from one
+  // request to the next, and a reallocation costs the calling thread several requests' worth when the
+  // pool has to ask the system, every time a table sees its largest slice so far.
+  size_t want = std::max(bytes + std::min<size_t>(bytes / 8, (size_t)32 << 20), b->bytes + b->bytes / 2);
+  want = (want + 4095) & ~(size_t)4095;
+  if (b == &t->ws || b == &t->tiles || b == &t->tiles_aff || b == &t->cache_keys ||
+      b == &t->cache_lens || b == &t->sc_vals || b == &t->sc_slots)
+    t->cache_valid = false;  // the contents do not survive a reallocation
+  // (earlier requests on the stream may still read the old buffer)
+  int rc = array_release(b->ptr, t->stream);
+  if (rc) return rc;
+  b->ptr = nullptr;
+  b->bytes = 0;
+  rc = array_alloc(&b->ptr, want, t->stream);
+  if (rc) return rc;
+  // the staging buffers are filled and read by copy streams, which know nothing of this stream's order
+  if (b == &t->stage || b == &t->stage_out) PSKV_HIP(hipStreamSynchronize(t->stream));
+  b->bytes = want;
   return PSKV_OK;
 }
 
@@ -576,15 +509,14 @@ void collect_spare(pskv_table* t, bool wait) {
   if (!t->spare_job) return;
   if (wait) {
     const auto w0 = std::chrono::steady_clock::now();
-    AllocWorker::get().wait(t->spare_job);
+    alloc_wait(t->spare_job);
     t->stats.alloc_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - w0).count();
-  } else if (!AllocWorker::get().finished(t->spare_job)) {
+  } else if (!alloc_finished(t->spare_job)) {
     return;
   }
   t->stats.ahead_us += t->spare_job->took_us;
   if (t->spare_job->rc == PSKV_OK && t->spare_job->ptr) {
     t->spare = static_cast<Slot*>(t->spare_job->ptr);
-    t->spare_pooled = t->spare_job->pooled;
   } else {
     t->spare_cap = 0;  // (the growth will ask again itself and report)
   }
@@ -609,21 +541,19 @@ int grow_slots(pskv_table* t, uint64_t keys_needed) {
     if (rc) return rc;
     t->cache_valid = false;
   }
-  bool pooled = false;
   ++t->stats.growths;
   collect_spare(t, true);
   if (t->spare && t->spare_cap >= want) {
     ++t->stats.spare_used;
     fresh = t->spare;
     want = t->spare_cap;
-    pooled = t->spare_pooled;
   } else {
     if (t->spare) {  // too small after all
-      rc = release_after(t->spare, t->spare_pooled, t->stream);
+      rc = array_release(t->spare, t->stream);
       if (rc) return rc;
     }
     const auto a0 = std::chrono::steady_clock::now();
-    rc = alloc_slots(want, &fresh, t->stream, &pooled, false);
+    rc = alloc_slots(want, &fresh, t->stream, false);
     t->stats.alloc_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - a0).count();
     if (rc) return rc;
   }
@@ -647,10 +577,9 @@ int grow_slots(pskv_table* t, uint64_t keys_needed) {
   }
   PSKV_HIP(hipGetLastError());
   const auto r0 = std::chrono::steady_clock::now();
-  rc = release_after(t->slots, t->slots_pooled, t->stream);
+  rc = array_release(t->slots, t->stream);
   t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
   t->slots = fresh;
-  t->slots_pooled = pooled;
   t->cap = want;
   return rc;
 }
@@ -674,23 +603,21 @@ void prepare_growth(pskv_table* t) {
   job->stream = t->stream;
   t->spare_cap = want;
   t->spare_job = job;
-  AllocWorker::get().submit(job);
+  alloc_submit(job);
 }
 
 int grow_arena(pskv_table* t, uint64_t floats_needed, uint64_t live_floats) {
   uint64_t want = std::max(floats_needed, t->arena_cap + t->arena_cap / 2);
   want = (want + 1023) & ~(uint64_t)1023;
   float* fresh = nullptr;
-  bool pooled = false;
-  int rc = alloc_for_growth(reinterpret_cast<void**>(&fresh), want * sizeof(float), t->stream, &pooled);
+  int rc = array_alloc(reinterpret_cast<void**>(&fresh), want * sizeof(float), t->stream);
   if (rc) return rc;
   if (live_floats && t->arena) {
     PSKV_HIP(hipMemcpyAsync(fresh, t->arena, live_floats * sizeof(float), hipMemcpyDeviceToDevice,
                             t->stream));
   }
-  rc = release_after(t->arena, t->arena_pooled, t->stream);
+  rc = array_release(t->arena, t->stream);
   t->arena = fresh;
-  t->arena_pooled = pooled;
   t->arena_cap = want;
   return rc;
 }
@@ -1928,6 +1855,8 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
     pskv_table_destroy(t);
     return rc;
   };
+  t->shell = shell_take(t->device);
+  if (!t->shell) return fail(set_error(PSKV_ENOMEM, "cannot allocate table state"));
   if (opts->stream) {
     t->stream = static_cast<hipStream_t>(opts->stream);
   } else {
@@ -1935,43 +1864,28 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
       return fail(set_error(PSKV_EHIP, "hipStreamCreateWithFlags failed"));
     t->own_stream = true;
   }
-  const uint64_t keys = opts->initial_capacity ? opts->initial_capacity : kDefaultCapacity;
-  t->cap = std::max(kMinSlots, next_pow2((uint64_t)((double)keys / t->max_load) + 1));
-  int rc = alloc_slots(t->cap, &t->slots, t->stream, &t->slots_pooled);
-  if (rc) return fail(rc);
-  if (hipMalloc(reinterpret_cast<void**>(&t->st), sizeof(DevState)) != hipSuccess ||
-      hipMemsetAsync(t->st, 0, sizeof(DevState), t->stream) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&t->st_host), sizeof(StateView), hipHostMallocCoherent) !=
-          hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&t->snap), sizeof(Snapshot), hipHostMallocDefault) !=
-          hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&t->outcome), sizeof(unsigned long long), hipHostMallocCoherent) !=
-          hipSuccess ||
-      // coherent: the GPU does not cache these two, so each request sees what the host just wrote
-      hipHostMalloc(reinterpret_cast<void**>(&t->small_in), kSmallBytes, hipHostMallocCoherent) !=
-          hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&t->small_out), kSmallBytes, hipHostMallocCoherent) !=
-          hipSuccess)
-    return fail(set_error(PSKV_ENOMEM, "cannot allocate table state"));
-  for (int q = 0; q < kSmallParts; ++q)
-    if (hipEventCreateWithFlags(&t->small_done[q], hipEventDisableTiming) != hipSuccess)
-      return fail(set_error(PSKV_ENOMEM, "cannot allocate table state"));
+  t->st = t->shell->st;
+  t->st_host = reinterpret_cast<StateView*>(t->shell->pinned);
+  t->snap = reinterpret_cast<Snapshot*>(t->shell->pinned + 256);
+  t->outcome = reinterpret_cast<unsigned long long*>(t->shell->pinned + 512);
+  t->small_in = t->shell->pinned + 1024;
+  t->small_out = t->small_in + kSmallBytes;
+  for (int q = 0; q < kSmallParts; ++q) t->small_done[q] = t->shell->done[q];
+  std::memset(t->st_host, 0, sizeof(StateView));
   std::memset(t->snap, 0xFF, sizeof(Snapshot));  // names no request
   *t->outcome = 0ull;
+  k_init_state<<<dim3(1), dim3(256), 0, t->stream>>>(t->st);
+  if (hipGetLastError() != hipSuccess) return fail(set_error(PSKV_EHIP, "table initialisation failed"));
+  const uint64_t keys = opts->initial_capacity ? opts->initial_capacity : kDefaultCapacity;
+  t->cap = std::max(kMinSlots, next_pow2((uint64_t)((double)keys / t->max_load) + 1));
+  int rc = alloc_slots(t->cap, &t->slots, t->stream);
+  if (rc) return fail(rc);
   if (t->mode != PSKV_MODE_SCALAR && opts->arena_floats) {
     t->arena_cap = (opts->arena_floats + 1023) & ~(uint64_t)1023;
-    if (alloc_for_growth(reinterpret_cast<void**>(&t->arena), t->arena_cap * sizeof(float), t->stream,
-                         &t->arena_pooled) != PSKV_OK)
+    if (array_alloc(reinterpret_cast<void**>(&t->arena), t->arena_cap * sizeof(float), t->stream) != PSKV_OK)
       return fail(set_error(PSKV_ENOMEM, "cannot allocate %llu floats of row storage",
                             (unsigned long long)t->arena_cap));
   }
-  const uint64_t unset = kPayloadUnset;
-  if (hipMemcpyAsync(&t->st->special_payload, &unset, sizeof(unset), hipMemcpyHostToDevice, t->stream) !=
-          hipSuccess ||
-      hipStreamSynchronize(t->stream) != hipSuccess)
-    return fail(set_error(PSKV_EHIP, "table initialisation failed"));
-  g_pools[t->device < 64 ? t->device : 63].tables.fetch_add(1);
-  t->counted = true;
   *out = t;
   return PSKV_OK;
 }
@@ -1988,6 +1902,7 @@ int pskv_table_destroy(pskv_table* t) {
             (unsigned long long)t->stats.spare_used, (unsigned long long)t->stats.waits,
             (unsigned long long)t->stats.catch_ups, t->stats.catch_up_us, (unsigned long long)t->stats.records,
             t->stats.alloc_us, t->stats.ahead_us, t->stats.release_us);
+  collect_spare(t, true);  // (the stream may have been made to wait for what used that array before)
   if (t->stream) (void)hipStreamSynchronize(t->stream);
   for (int k = 0; k < PSKV_KERNEL_COUNT; ++k)
     for (const EventPair& ev : t->pending[k]) t->free_events.push_back(ev);
@@ -1995,46 +1910,14 @@ int pskv_table_destroy(pskv_table* t) {
     (void)hipEventDestroy(ev.a);
     (void)hipEventDestroy(ev.b);
   }
-  // (arrays that a growth took from the stream-ordered pool go back to it)
-  if (t->slots && t->slots_pooled) {
-    (void)hipFreeAsync(t->slots, t->stream);
-  } else if (t->slots) {
-    (void)hipFree(t->slots);
-  }
-  if (t->arena && t->arena_pooled) {
-    (void)hipFreeAsync(t->arena, t->stream);
-    t->arena = nullptr;
-  }
-  collect_spare(t, true);
-  if (t->spare && t->spare_pooled) {
-    (void)hipFreeAsync(t->spare, t->stream);
-  } else if (t->spare) {
-    (void)hipFree(t->spare);
-  }
-  if (t->slots_pooled || t->arena_pooled || t->spare_pooled) (void)hipStreamSynchronize(t->stream);
-  if (t->st) (void)hipFree(t->st);
-  if (t->st_host) (void)hipHostFree(t->st_host);
-  if (t->snap) (void)hipHostFree(t->snap);
-  if (t->outcome) (void)hipHostFree(t->outcome);
-  if (t->sc_vals.ptr) (void)hipFree(t->sc_vals.ptr);
-  if (t->sc_slots.ptr) (void)hipFree(t->sc_slots.ptr);
-  for (int q = 0; q < kSmallParts; ++q)
-    if (t->small_done[q]) (void)hipEventDestroy(t->small_done[q]);
-  if (t->small_in) (void)hipHostFree(t->small_in);
-  if (t->small_out) (void)hipHostFree(t->small_out);
-  if (t->arena) (void)hipFree(t->arena);
-  if (t->ws.ptr) (void)hipFree(t->ws.ptr);
-  if (t->stage.ptr) (void)hipFree(t->stage.ptr);
-  if (t->tiles.ptr) (void)hipFree(t->tiles.ptr);
-  if (t->tiles_aff.ptr) (void)hipFree(t->tiles_aff.ptr);
-  if (t->cache_keys.ptr) (void)hipFree(t->cache_keys.ptr);
-  if (t->cache_lens.ptr) (void)hipFree(t->cache_lens.ptr);
-  if (t->stage_out.ptr) (void)hipFree(t->stage_out.ptr);
-  if (t->own_stream && t->stream) (void)hipStreamDestroy(t->stream);
-  // the last table of a device to go takes the memory the pool has kept with it
-  DevicePool& dp = g_pools[t->device < 64 ? t->device : 63];
-  if (t->counted && dp.tables.fetch_sub(1) == 1 && dp.known.load(std::memory_order_acquire) == 2 && dp.pool)
-    (void)hipMemPoolTrimTo(dp.pool, 0);
+  // the stream is idle: the arrays are free to go to any other table at once
+  for (void* ptr : {static_cast<void*>(t->slots), static_cast<void*>(t->arena), static_cast<void*>(t->spare)})
+    (void)array_release(ptr, t->stream, true);
+  for (const GrowBuf* b : {&t->ws, &t->tiles, &t->tiles_aff, &t->stage, &t->stage_out, &t->cache_keys, &t->cache_lens,
+                           &t->sc_vals, &t->sc_slots})
+    (void)array_release(b->ptr, t->stream, true);
+  shell_give(t->device, t->shell);
+  if (t->own_stream) (void)hipStreamDestroy(t->stream);
   delete t;
   return PSKV_OK;
 }
@@ -2380,13 +2263,10 @@ int pskv_table_counters(pskv_table* t, uint64_t* out, size_t cap) {
 int pskv_device_trim(int device) {
   clear_error();
   if (device < 0 || device >= 64) return set_error(PSKV_EINVAL, "device %d out of range", device);
-  DevicePool& dp = g_pools[device];
   DeviceGuard guard(device);
   if (!guard.ok()) return set_error(PSKV_EHIP, "cannot select device %d", device);
-  if (dp.known.load(std::memory_order_acquire) == 2 && dp.pool) {
-    PSKV_HIP(hipDeviceSynchronize());  // what streams have freed into the pool is the pool's once they got there
-    PSKV_HIP(hipMemPoolTrimTo(dp.pool, 0));
-  }
+  array_trim(device);
+  shell_trim(device);
   return match_trim(device);
 }
 
