@@ -120,6 +120,96 @@ __global__ __launch_bounds__(kFusedWaves * 64) void k_bounds_fused(
   announce_done(pos_host, S, done_seq);
 }
 
+// Boundaries and the lens sums of the slices between them in one launch (few boundaries, in ascending
+// order). A workgroup takes one stretch of the request: two keys tell it which boundaries fall inside,
+// it searches those there, adds up the lens between them, and hands positions and sums over past the
+// L2; the workgroup that finishes last writes everything to pinned memory. The lens of a request are
+// read once and nothing else is: 2M keys over 16 ranges took three launches (6.8 + 10.1 us, and the sums'
+// way to the host) and a stream wait, 38 us per call; this is one launch and the watched word.
+constexpr unsigned kSumsMaxBlocks = 256;  // (every workgroup takes a ticket of one counter, about 10 ns each)
+struct SumsState {                         // device memory of one slicer context, all zero between calls
+  unsigned long long pos[kFusedTargets];
+  unsigned long long sums[kFusedTargets];
+  unsigned ticket;
+};
+__global__ __launch_bounds__(kBlock) void k_bounds_sums(const uint64_t* __restrict__ keys,
+                                                       const int32_t* __restrict__ lens, uint64_t n, uint64_t chunk,
+                                                       FusedTargets targets, unsigned S, SumsState* state,
+                                                       uint64_t* __restrict__ pos_host,
+                                                       unsigned long long* __restrict__ sums_host,
+                                                       unsigned long long done_seq) {
+  __shared__ uint64_t s_b[kFusedTargets];
+  __shared__ unsigned long long s_red[kBlock / 64];
+  __shared__ unsigned s_last;
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t c0 = (uint64_t)blockIdx.x * chunk;
+  const uint64_t c1 = n - c0 < chunk ? n : c0 + chunk;
+  const uint64_t before = c0 ? keys[c0 - 1] : 0, last = keys[c1 - 1];
+  for (unsigned i = wave; i <= S; i += kBlock / 64) {  // whole wavefronts
+    const uint64_t target = targets.v[i];
+    const bool after_start = c0 == 0 || before < target;  // the boundary does not lie before this stretch
+    const bool mine = after_start && (c1 == n || last >= target);
+    uint64_t at = after_start ? c1 : c0;
+    if (mine) at = c0 + wave_lower_bound(keys + c0, c1 - c0, target, lane);
+    if (lane == 0) {
+      s_b[i] = at;
+      if (mine) __hip_atomic_store(&state->pos[i], (unsigned long long)at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  __syncthreads();
+  for (unsigned i = 0; i < S; ++i) {
+    const uint64_t b = s_b[i], e = s_b[i + 1];
+    if (e <= b) continue;  // (the same for the whole workgroup)
+    unsigned long long sum = 0;
+    uint64_t j = b + threadIdx.x;
+    for (; j + 7 * kBlock < e; j += 8 * kBlock) {  // loads of a round before its adds
+      int32_t l[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) l[u] = lens[j + (uint64_t)u * kBlock];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += (unsigned long long)(long long)l[u];
+    }
+    for (; j < e; j += kBlock) sum += (unsigned long long)(long long)lens[j];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if (lane == 0) s_red[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned long long t = 0;
+      for (unsigned w = 0; w < kBlock / 64; ++w) t += s_red[w];
+      if (t) atomicAdd(&state->sums[i], t);
+    }
+    __syncthreads();
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // what this lane has handed over is there before the ticket is taken
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s_last = atomicAdd(&state->ticket, 1u) == gridDim.x - 1 ? 1u : 0u;
+    if (s_last) __threadfence();
+  }
+  __syncthreads();
+  if (!s_last) return;
+  if (threadIdx.x < S) {
+    sums_host[threadIdx.x] = __hip_atomic_load(&state->sums[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    state->sums[threadIdx.x] = 0ull;
+  }
+  if (threadIdx.x <= S) {
+    s_b[threadIdx.x] = __hip_atomic_load(&state->pos[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    state->pos[threadIdx.x] = 0ull;  // (keys that are not sorted may leave a boundary without an owner)
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  state->ticket = 0;
+  uint64_t p = s_b[0];
+  pos_host[0] = p;
+  for (unsigned i = 0; i < S; ++i) {
+    p = s_b[i + 1] > p ? s_b[i + 1] : p;
+    pos_host[i + 1] = p;
+  }
+  announce_done(pos_host, S, done_seq);
+}
+
 // ---- the slicer for callers that cannot allocate ------------------------------------------
 // Working memory of pskv_slice_noalloc: the lower bounds of the boundary searches followed by
 // the per-slice sums of lens. It lives in the code object, so every GPU that loads the library
@@ -286,6 +376,7 @@ struct SliceCtx {
   unsigned long long calls = 0;  // numbers the calls whose completion the host watches for
   int device = -1;
   hipStream_t stream = nullptr;
+  SumsState* sums_state = nullptr;
   void* dev = nullptr;      // device scratch: targets, lower bounds, positions, sums
   size_t dev_bytes = 0;
   void* pinned = nullptr;   // pinned host memory the kernels read targets from and answer into
@@ -309,7 +400,11 @@ SliceCtx* take_ctx(int device) {
   SliceCtx* c = new (std::nothrow) SliceCtx();
   if (!c) return nullptr;
   c->device = device;
-  if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
+      hipMalloc(reinterpret_cast<void**>(&c->sums_state), sizeof(SumsState)) != hipSuccess ||
+      hipMemset(c->sums_state, 0, sizeof(SumsState)) != hipSuccess) {
+    if (c->sums_state) (void)hipFree(c->sums_state);
+    if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return nullptr;
   }
@@ -454,16 +549,25 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     uint64_t* h_targets = reinterpret_cast<uint64_t*>(h);
     uint64_t* h_pos = reinterpret_cast<uint64_t*>(h + arr);
     unsigned long long* h_sums = reinterpret_cast<unsigned long long*>(h + 2 * arr);
-    const int32_t* d_lens = lens;
     h_targets[0] = range_begin[0];
     for (size_t i = 0; i < S; ++i) h_targets[i + 1] = range_end[i];
-    // Without lens the positions are all this call waits for, and the kernel that writes them
-    // says so in pinned memory: watching that word costs about 5 us less than a stream wait.
-    const unsigned long long watch = do_sums ? 0ull : ++c->calls;
+    // With few boundaries one kernel leaves everything this call waits for in pinned memory and says so in
+    // a word behind it: watching that word costs about 5 us less than a stream wait. (With lens the
+    // boundaries must ascend, as those of contiguous ranges do unless a range ends before it begins.)
+    const bool few = S + 1 <= kFusedTargets;
+    const bool sums_too = do_sums && few && std::is_sorted(h_targets, h_targets + S + 1);
+    const unsigned long long watch = !do_sums || sums_too ? ++c->calls : 0ull;
     h_pos[S + 1] = 0;  // (whatever an earlier call with other ranges left at this place)
-    if (S + 1 <= kFusedTargets) {  // one launch for the boundaries when they are few
-      FusedTargets ft = {};
+    FusedTargets ft = {};
+    if (few)
       for (size_t i = 0; i <= S; ++i) ft.v[i] = h_targets[i];
+    if (sums_too) {
+      // (a stretch of at least 2,048 keys, a multiple of four)
+      const uint64_t chunk = std::max<uint64_t>(2048, ((n + kSumsMaxBlocks - 1) / kSumsMaxBlocks + 3) & ~(uint64_t)3);
+      k_bounds_sums<<<dim3((unsigned)((n + chunk - 1) / chunk)), dim3(kBlock), 0, c->stream>>>(
+          keys, lens, n, chunk, ft, (unsigned)S, c->sums_state, h_pos, h_sums, watch);
+      PSKV_HIP(hipGetLastError());
+    } else if (few) {  // one launch for the boundaries
       const unsigned waves = (unsigned)std::min<size_t>(S + 1, kFusedWaves);
       k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, c->stream>>>(keys, n, ft, S, d_pos, h_pos,
                                                                  do_sums ? d_sums : nullptr, watch);
@@ -475,11 +579,10 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
                                                           watch);
       PSKV_HIP(hipGetLastError());
     }
-    if (do_sums) {
+    if (do_sums && !sums_too) {
       uint64_t per = n / S / (kBlock * 8) + 1;
       if (per > 1024) per = 1024;
-      k_segment_sums<<<dim3((unsigned)per, (unsigned)S), dim3(kBlock), 0, c->stream>>>(d_lens, d_pos,
-                                                                                      d_sums);
+      k_segment_sums<<<dim3((unsigned)per, (unsigned)S), dim3(kBlock), 0, c->stream>>>(lens, d_pos, d_sums);
       PSKV_HIP(hipGetLastError());
       k_export_sums<<<dim3((unsigned)((S + 255) / 256)), dim3(256), 0, c->stream>>>(d_sums, S, h_sums);
       PSKV_HIP(hipGetLastError());

@@ -66,6 +66,25 @@ def test_slice_sixteen_million_keys(capi, dev, S):
     assert np.array_equal(pos2, pos) and np.array_equal(vpos2.astype(np.int64), 2 * pos.astype(np.int64))
 
 
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 4096, 256 * 2048, 256 * 2048 + 1, 600001])
+@pytest.mark.parametrize("S", [1, 5, 31])
+def test_slice_with_lens_at_the_edges_of_a_stretch(capi, orc, dev, n, S):
+    """Boundaries on, next to and far from the edges of the stretches that a workgroup of the one-launch
+    lens slicer takes; empty slices between them; twice in a row (the kernel clears up behind itself)."""
+    announce("slice_lens_edges", n, S)
+    rng = np.random.default_rng(n + S)
+    keys = unique_keys(rng, n)
+    chunk = max(2048, ((n + 255) // 256 + 3) & ~3)
+    spots = np.array([0, 1, chunk - 1, chunk, chunk + 1, 2 * chunk, n - 1, n // 2, n // 2])
+    cuts = keys[np.minimum(rng.choice(spots, S - 1), n - 1)] + rng.integers(0, 2, S - 1).astype(np.uint64) if S > 1 else keys[:0]
+    cuts = np.sort(cuts)
+    rb = np.concatenate([np.zeros(1, np.uint64), cuts])
+    re = np.concatenate([cuts, np.array([KMAX], np.uint64)])
+    lens = rng.integers(0, 9, n).astype(np.int32)
+    for _ in range(2):
+        assert _compare(capi, orc, keys, rb, re, lens, int(lens.sum()), dev, "device") == 0
+
+
 @pytest.mark.parametrize("S", [1, 4, 1024])
 def test_slice_sixteen_million_keys_in_host_memory(capi, orc, dev, S):
     """The same request with its keys (and lens) in ordinary host memory, as the worker's slicer
