@@ -4,10 +4,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#ifndef PSKV_TILE_VAR
-#define PSKV_TILE_VAR 256
-#endif
-
 namespace pskv {
 
 // ps::kMaxKey (include/ps/base.h:18). The stock server ranges never cover it

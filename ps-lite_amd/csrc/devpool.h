@@ -21,6 +21,9 @@ namespace pskv {
 int array_alloc(void** out, size_t bytes, hipStream_t stream);
 // Gives an array back (null: nothing). Work already enqueued on `stream` may still use it; `idle`: nothing does.
 int array_release(void* ptr, hipStream_t stream, bool idle = false);
+// `stream` (of the current device) has just been waited for and may be destroyed: nothing on the list
+// depends on it any more.
+void array_settle(hipStream_t stream);
 // Frees every array on the list of `device` (current). Waits for those that are still in use.
 void array_trim(int device);
 

@@ -95,7 +95,8 @@ class Worker {
 
 void free_now(Pool* p, const Idle& i) {
   if (i.done) {
-    (void)hipEventSynchronize(i.done);
+    // (an event of a stream that is gone by now is an error; hipFree waits for the device anyway)
+    if (hipEventSynchronize(i.done) != hipSuccess) (void)hipGetLastError();
     std::lock_guard<std::mutex> lk(p->mu);
     p->events.push_back(i.done);
   }
@@ -233,6 +234,18 @@ int array_release(void* ptr, hipStream_t stream, bool idle) {
   }
   if (!over.empty()) Worker::get().free_later(dev, std::move(over));
   return PSKV_OK;
+}
+
+void array_settle(hipStream_t stream) {
+  int dev = 0;
+  Pool* p = hipGetDevice(&dev) == hipSuccess ? pool_of(dev) : nullptr;
+  if (!p) return;
+  std::lock_guard<std::mutex> lk(p->mu);
+  for (Idle& i : p->idle) {
+    if (!i.done || i.stream != stream) continue;
+    p->events.push_back(i.done);
+    i.done = nullptr;
+  }
 }
 
 void array_trim(int device) {

@@ -606,11 +606,14 @@ void prepare_growth(pskv_table* t) {
   alloc_submit(job);
 }
 
+// Room behind an arena's last row: the row kernels read a row's last quad whole.
+constexpr size_t kArenaEnd = 16;
+
 int grow_arena(pskv_table* t, uint64_t floats_needed, uint64_t live_floats) {
   uint64_t want = std::max(floats_needed, t->arena_cap + t->arena_cap / 2);
   want = (want + 1023) & ~(uint64_t)1023;
   float* fresh = nullptr;
-  int rc = array_alloc(reinterpret_cast<void**>(&fresh), want * sizeof(float), t->stream);
+  int rc = array_alloc(reinterpret_cast<void**>(&fresh), want * sizeof(float) + kArenaEnd, t->stream);
   if (rc) return rc;
   if (live_floats && t->arena) {
     PSKV_HIP(hipMemcpyAsync(fresh, t->arena, live_floats * sizeof(float), hipMemcpyDeviceToDevice,
@@ -1074,15 +1077,30 @@ int run_scalar(Batch& bt, bool push, bool pull) {
 // requests of a busy server they do not survive in the caches anyway.
 constexpr uint64_t kStreamFloats = 1u << 20;
 
-// The row kernel over `floats` request-side floats of the batch's only table, starting at float
-// `first` (a multiple of the tile size): one piece of a request that is served as it arrives.
+// FIXED: quads (see k_rows) that lie, whole (`started`: or in part), within the first `floats` floats of a
+// request with rows of k floats.
+uint64_t quads_within(uint64_t floats, uint64_t k, bool started) {
+  const uint64_t in_row = floats % k;
+  return floats / k * ((k + 3) / 4) + (started ? (in_row + 3) / 4 : in_row / 4);
+}
+
+// The row kernel over the request-side floats [first, first + floats) of the batch's only table (`first`
+// is a multiple of a VARLEN workgroup's stretch): one piece of a request that is served as it arrives.
 template <bool VARLEN>
 int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
-  const uint64_t tile = VARLEN ? kRowsVarPerBlock : kTileFixed;
   Item& it = bt[0];
   const bool stream = it.d.total >= kStreamFloats;
-  it.d.tile_base = (uint32_t)(first / tile);
-  auto nblk = [&](const Item&) { return (floats + tile - 1) / tile; };
+  uint64_t blocks;
+  if (VARLEN) {
+    it.d.tile_base = (uint32_t)(first / kRowsVarPerBlock);
+    blocks = (floats + kRowsVarPerBlock - 1) / kRowsVarPerBlock;
+  } else {
+    // a quad on the edge of two pieces goes with the second when it is read, with the first when written
+    it.d.nvals = quads_within(first, it.d.k, op == kOpGather);
+    it.d.ntiles = quads_within(first + floats, it.d.k, op == kOpGather);
+    blocks = (it.d.ntiles - it.d.nvals + kQuadsFixed - 1) / kQuadsFixed;
+  }
+  auto nblk = [&](const Item&) { return blocks; };
   int rc;
   if (op == kOpAcc) {
     rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, true>, nblk)
@@ -1098,9 +1116,14 @@ int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
 // The row kernel over every table of the batch whose TableReq::total is not zero.
 template <bool VARLEN>
 int launch_rows(Batch& bt, int op) {
-  const uint64_t tile = VARLEN ? kRowsVarPerBlock : kTileFixed;  // request-side floats per workgroup
   uint64_t floats = 0;
-  for (const Item& it : bt) floats += it.d.total;
+  for (Item& it : bt) {
+    floats += it.d.total;
+    if (!VARLEN) {
+      it.d.nvals = 0;
+      it.d.ntiles = it.d.total ? it.d.n * ((it.d.k + 3) / 4) : 0;
+    }
+  }
   if (!floats) return PSKV_OK;
   if (bt.size() == 1 && op == kOpAcc && bt[0].r.pipe_in) {
     // the values are still in the caller's memory: every piece is accumulated as soon as it is here
@@ -1117,7 +1140,9 @@ int launch_rows(Batch& bt, int op) {
     bt[0].r.gather_varlen = VARLEN;
     return PSKV_OK;
   }
-  auto nblk = [&](const Item& it) { return (it.d.total + tile - 1) / tile; };
+  auto nblk = [&](const Item& it) {
+    return VARLEN ? (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock : (it.d.ntiles + kQuadsFixed - 1) / kQuadsFixed;
+  };
   const bool stream = floats >= kStreamFloats;
   if (op == kOpAcc) {
     if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, true>, nblk);
@@ -1205,7 +1230,6 @@ int run_fixed(Batch& bt, bool push, bool pull) {
       if (!it.r.n) continue;
       it.d.req = const_cast<float*>(it.r.vals);
       it.d.total = it.r.n * it.d.k;
-      it.d.force_scalar = ((it.d.k & 3) || (reinterpret_cast<uintptr_t>(it.r.vals) & 15)) ? 1u : 0u;
       it.d.ignore_new = 0;
     }
     rc = launch_rows<false>(bt, kOpAcc);
@@ -1216,7 +1240,6 @@ int run_fixed(Batch& bt, bool push, bool pull) {
       if (!it.r.n) continue;
       it.d.req = it.r.out;
       it.d.total = it.r.n * it.d.k;
-      it.d.force_scalar = ((it.d.k & 3) || (reinterpret_cast<uintptr_t>(it.r.out) & 15)) ? 1u : 0u;
       it.d.ignore_new = push ? 1u : 0u;
     }
     rc = launch_rows<false>(bt, kOpGather);
@@ -1350,7 +1373,6 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       it.t->cache_nvals = it.r.nvals;
       it.d.req = const_cast<float*>(it.r.vals);
       it.d.total = it.r.nvals;
-      it.d.force_scalar = (reinterpret_cast<uintptr_t>(it.r.vals) & 15) ? 1u : 0u;
       it.d.ignore_new = 0;
       it.d.total_on_device = 0;
     }
@@ -1394,7 +1416,6 @@ int run_varlen(Batch& bt, bool push, bool pull) {
         it.d.req = it.r.out;
         it.d.total = it.r.out_cap;
         it.d.total_on_device = 1;
-        it.d.force_scalar = (reinterpret_cast<uintptr_t>(it.r.out) & 15) ? 1u : 0u;
         it.d.ignore_new = 1;
       }
       rc = make_tile_tables(bt, items);
@@ -1434,7 +1455,6 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       it.d.req = r.out;
       it.d.total = total;
       it.d.total_on_device = 0;
-      it.d.force_scalar = (reinterpret_cast<uintptr_t>(r.out) & 15) ? 1u : 0u;
       it.d.ignore_new = 1;
     }
     rc = make_tile_tables(bt, items);
@@ -1882,7 +1902,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   if (rc) return fail(rc);
   if (t->mode != PSKV_MODE_SCALAR && opts->arena_floats) {
     t->arena_cap = (opts->arena_floats + 1023) & ~(uint64_t)1023;
-    if (array_alloc(reinterpret_cast<void**>(&t->arena), t->arena_cap * sizeof(float), t->stream) != PSKV_OK)
+    if (array_alloc(reinterpret_cast<void**>(&t->arena), t->arena_cap * sizeof(float) + kArenaEnd, t->stream) != PSKV_OK)
       return fail(set_error(PSKV_ENOMEM, "cannot allocate %llu floats of row storage",
                             (unsigned long long)t->arena_cap));
   }
@@ -1910,7 +1930,8 @@ int pskv_table_destroy(pskv_table* t) {
     (void)hipEventDestroy(ev.a);
     (void)hipEventDestroy(ev.b);
   }
-  // the stream is idle: the arrays are free to go to any other table at once
+  // the stream is idle: the arrays are free to go to any other table at once, as are those given up before
+  if (t->stream) array_settle(t->stream);
   for (void* ptr : {static_cast<void*>(t->slots), static_cast<void*>(t->arena), static_cast<void*>(t->spare)})
     (void)array_release(ptr, t->stream, true);
   for (const GrowBuf* b : {&t->ws, &t->tiles, &t->tiles_aff, &t->stage, &t->stage_out, &t->cache_keys, &t->cache_lens,

@@ -25,7 +25,7 @@ struct TableReq {
   const float* vals;     // SCALAR push: n values
   float* out;            // SCALAR pull: n values
   uint64_t n;
-  uint64_t nvals;        // VARLEN push: floats pushed
+  uint64_t nvals;        // VARLEN push: floats pushed; FIXED row kernels: the quad the launch starts at
   // row modes
   float* arena;              // row storage
   uint64_t* ref;             // n row references, written by the lookup kernel
@@ -33,7 +33,8 @@ struct TableReq {
   unsigned long long* part;  // VARLEN: per-workgroup totals of the lens scan
   uint32_t* tile_key;        // VARLEN: first key of every request-side tile, ntiles+1 entries
   TileNote* tile_aff;        // VARLEN: one note per tile
-  uint64_t ntiles;           // VARLEN: tiles of the request (push) / room in the tile table (pull)
+  uint64_t ntiles;           // VARLEN: tiles of the request (push) / room in the tile table (pull);
+                             // FIXED row kernels: the quad the launch ends before
   uint64_t* cache_keys;      // keys (and lens) of the request whose references the workspace holds
   int32_t* cache_lens;
   int32_t* out_lens;         // VARLEN pull: n answered lengths
@@ -44,7 +45,7 @@ struct TableReq {
   float* req;             // push: request values (read); pull: response values (written)
   uint64_t total;         // floats in req
   uint64_t k;             // FIXED: floats per row
-  uint32_t force_scalar;  // request buffer or k not 16-byte friendly
+  uint32_t reserved;
   uint32_t ignore_new;    // pull half of a push+pull: rows created by the push half hold data
   uint32_t total_on_device;  // VARLEN pull without a host round trip: the floats to move are
                              // DevState::scan_total and `total` is the room in req
@@ -54,7 +55,7 @@ struct TableReq {
   // `tile_key`
   unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null
   uint32_t cache_mode;          // kCache* below
-  uint32_t tile_base;           // row kernels: the launch starts at this tile of the request (a large
+  uint32_t tile_base;           // VARLEN row kernels: the launch starts at this tile of the request (a large
                                 // host-resident request is served piece by piece as it arrives)
 };
 constexpr uint32_t kCacheOff = 0;     // SCALAR: the request neither uses nor fills the key cache
@@ -544,6 +545,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
 // slots for its keys, then the workgroup takes the rows of all created keys from the arena
 // with ONE atomic add and a workgroup-wide scan hands them out in request order, so rows of
 // neighbouring keys are neighbours in the arena.
+constexpr unsigned kTileVar = 256;  // request-side floats per wavefront of the var-len row kernel: one quad per lane
 constexpr unsigned long long kArenaPadUnits = 8;  // 128 bytes in 16-byte allocation units
 
 template <int kItems>
@@ -561,7 +563,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_lookup(ReqBatch b) {
   uint64_t* __restrict__ off = d.off;
   uint32_t* __restrict__ tile_key = d.tile_key;
   const uint64_t ntiles = d.ntiles;
-  constexpr uint64_t tile = PSKV_TILE_VAR;
+  constexpr uint64_t tile = kTileVar;
   uint64_t* __restrict__ ref = d.ref;
   uint64_t* __restrict__ cache_keys = d.cache_keys;
   int32_t* __restrict__ cache_lens = d.cache_lens;
@@ -725,7 +727,7 @@ __global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch b) {
   uint64_t* __restrict__ off = d.off;
   uint32_t* __restrict__ tile_key = d.tile_key;
   const uint64_t ntiles_cap = d.ntiles;
-  constexpr uint64_t tile = PSKV_TILE_VAR;
+  constexpr uint64_t tile = kTileVar;
   const DevState* st = d.st;
   const ReqTag tag = d.tag;
   if (cache_same(st, tag) || tag.replay) return;  // offsets and tile table of the cached request hold
@@ -741,12 +743,14 @@ __global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch b) {
 
 // ---------------------------------------------------------------------------------
 // Row modes, step 2: stream the values.
-// A workgroup owns one tile of consecutive floats of the request-side
-// buffer, whatever rows they belong to, so the load is balanced for any mix of row
-// lengths and the request side is read or written fully coalesced with 128-bit
-// accesses. FIXED locates the row of an element by division; VARLEN stages the
-// offsets and row references of the keys that overlap the tile in LDS and locates
-// rows by binary search there.
+// The unit of work is a quad: four consecutive floats of the request-side buffer (one 128-bit access
+// per lane), so the load is balanced for any mix of row lengths. Quads need not lie on 16-byte
+// boundaries: a 128-bit access to global memory may start at any float, and costs a wavefront of
+// consecutive quads one 128-byte line in eight at most.
+// FIXED cuts every row into quads of its own (the last one shorter when k is not a multiple of four) and
+// locates the row of a quad by division; VARLEN cuts the request into quads, stages the offsets and row
+// references of the keys that overlap a wavefront's stretch in LDS and locates rows by binary search
+// there.
 // ---------------------------------------------------------------------------------
 struct RowsParams {
   float* req;                // push: request values (read); pull: response values (written)
@@ -757,124 +761,121 @@ struct RowsParams {
   TileNote* tile_aff;        // VARLEN: one note per tile
   DevState* st;
   uint64_t n;
-  uint64_t total;         // floats in req
+  uint64_t total;         // VARLEN: floats in req
   uint64_t k;             // FIXED: floats per row
-  uint32_t force_scalar;  // request buffer or k not 16-byte friendly
   uint32_t ignore_new;    // pull half of a push+pull: rows created by the push half hold data
   uint32_t total_on_device;  // VARLEN pull without a host round trip: the floats to move are
                              // DevState::scan_total and `total` is the room in req
-  uint32_t blk;              // the workgroup's number among those that cover the request
+  uint32_t blk;              // VARLEN: the workgroup's number among those that cover the request
   ReqTag tag;
 };
 
 constexpr int kOpAcc = 0;
 constexpr int kOpGather = 1;
 
-// VEC floats moved by one lane per access. STREAM selects non-temporal accesses: a
+// Four (three, two) floats that start at any float. STREAM selects non-temporal accesses: a
 // request far larger than the caches is read and written once per launch, and telling
 // the memory system so is worth 10-15 % of bandwidth on this GPU.
-template <int VEC>
-struct VecT;
-template <>
-struct VecT<4> {
-  using type = f32x4;
-  __device__ static f32x4 zero() { return (f32x4)(0.f); }
-};
-template <>
-struct VecT<1> {
-  using type = float;
-  __device__ static float zero() { return 0.f; }
-};
-template <bool STREAM, typename V>
-__device__ __forceinline__ V vload(const V* p) {
-  return STREAM ? __builtin_nontemporal_load(p) : *p;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x3u __attribute__((ext_vector_type(3), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+template <bool STREAM>
+__device__ __forceinline__ f32x4 load_quad(const float* p) {
+  const f32x4u* q = reinterpret_cast<const f32x4u*>(p);
+  return STREAM ? __builtin_nontemporal_load(q) : *q;
 }
-template <bool STREAM, typename V>
-__device__ __forceinline__ void vstore(V v, V* p) {
-  if (STREAM) __builtin_nontemporal_store(v, p); else *p = v;
+template <bool STREAM>
+__device__ __forceinline__ void store_quad(f32x4 v, float* p) {
+  f32x4u* q = reinterpret_cast<f32x4u*>(p);
+  if (STREAM) __builtin_nontemporal_store((f32x4u)v, q); else *q = v;
+}
+// The first `count` (1 to 4) floats of a quad, one access each.
+template <bool STREAM>
+__device__ __forceinline__ f32x4 load_part(const float* p, unsigned count) {
+  f32x4 v = (f32x4)(0.f);
+  if (count == 4) {
+    v = load_quad<STREAM>(p);
+  } else if (count == 3) {
+    const f32x3u* q = reinterpret_cast<const f32x3u*>(p);
+    const f32x3u w = STREAM ? __builtin_nontemporal_load(q) : *q;
+    v.x = w.x, v.y = w.y, v.z = w.z;
+  } else if (count == 2) {
+    const f32x2u* q = reinterpret_cast<const f32x2u*>(p);
+    const f32x2u w = STREAM ? __builtin_nontemporal_load(q) : *q;
+    v.x = w.x, v.y = w.y;
+  } else {
+    v.x = STREAM ? __builtin_nontemporal_load(p) : *p;
+  }
+  return v;
+}
+template <bool STREAM>
+__device__ __forceinline__ void store_part(f32x4 v, float* p, unsigned count) {
+  if (count == 4) {
+    store_quad<STREAM>(v, p);
+  } else if (count == 3) {
+    f32x3u* q = reinterpret_cast<f32x3u*>(p);
+    const f32x3u w = {v.x, v.y, v.z};
+    if (STREAM) __builtin_nontemporal_store(w, q); else *q = w;
+  } else if (count == 2) {
+    f32x2u* q = reinterpret_cast<f32x2u*>(p);
+    const f32x2u w = {v.x, v.y};
+    if (STREAM) __builtin_nontemporal_store(w, q); else *q = w;
+  } else {
+    if (STREAM) __builtin_nontemporal_store(v.x, p); else *p = v.x;
+  }
 }
 
-// FIXED rows: a workgroup owns TILE consecutive request-side floats; the row of an element
-// follows from a division (one compare when a row is at least a tile long).
-template <int OP, int VEC, bool STREAM, unsigned TILE>
-__device__ __forceinline__ void rows_tile_fixed(const RowsParams& p, uint64_t total) {
+// FIXED rows: one quad per lane. `quads` = ceil(k/4) per row, `rest` = k mod 4 floats in a row's last one
+// (REST: not zero). A row's quads are its own, so a lane deals with one row whatever k is. (Rows with a
+// rest used to go float by float, four 32-bit accesses and four divisions per lane: 500,000 rows of 33
+// floats 78 us to accumulate and 47 to gather, now 49 and 35; 160 rows of 825,153 floats 1.39 times faster.)
+template <int OP, bool STREAM, bool REST>
+__device__ __forceinline__ void rows_quads_fixed(const RowsParams& p, uint64_t q0, uint64_t q_end) {
   // a refused push (it repeats a key) changes no stored value; rows it created stay, as zero rows
   const bool rejected = OP == kOpAcc && p.st->refused_epoch == p.tag.epoch;
-  using V = typename VecT<VEC>::type;
-  constexpr int kIter = TILE / (VEC * kBlock);      // elements per thread
-  constexpr int kGroup = kIter < 4 ? kIter : 4;     // loads issued back to back
-  static_assert(kIter >= 1 && kIter % kGroup == 0, "tile does not divide over the workgroup");
-  const uint64_t f0 = (uint64_t)p.blk * TILE;
-  if (f0 >= total) return;
-  const uint32_t tile_floats = (uint32_t)((total - f0 < (uint64_t)TILE) ? (total - f0) : (uint64_t)TILE);
-  const uint32_t nelem = tile_floats / VEC;
-
-  // The request-side loads depend on nothing but the tile index: issue them first so that
-  // they are in flight while the row references are fetched.
-  V x[kIter];
-  if (OP == kOpAcc) {
-#pragma unroll
-    for (int i = 0; i < kIter; ++i) {
-      const uint32_t le = (uint32_t)i * kBlock + threadIdx.x;
-      x[i] = VecT<VEC>::zero();
-      if (le < nelem) x[i] = vload<STREAM>(reinterpret_cast<const V*>(p.req + f0 + le * VEC));
-    }
+  const uint64_t quads = (p.k + 3) >> 2;
+  const unsigned rest = REST ? (unsigned)p.k & 3u : 0u;
+  const bool live = threadIdx.x < q_end - q0;
+  f32x4 x = (f32x4)(0.f);
+  // Without a rest the request side depends on nothing but the quad's number: asked for first, so that
+  // it is in flight while the row reference is fetched.
+  if (OP == kOpAcc && !REST && live) x = load_quad<STREAM>(p.req + (q0 + threadIdx.x) * 4);
+  // one division per workgroup; a lane is at most kBlock quads further on
+  const uint64_t row0 = q0 / quads;
+  const uint64_t c0 = q0 - row0 * quads + threadIdx.x;
+  uint64_t over, c;
+  if (quads >= kBlock) {
+    over = c0 >= quads ? 1u : 0u;
+    c = over ? c0 - quads : c0;
+  } else {
+    const unsigned o32 = (unsigned)c0 / (unsigned)quads;
+    over = o32;
+    c = (unsigned)c0 - o32 * (unsigned)quads;
   }
-  const uint64_t j0 = f0 / p.k;           // row of the tile's first float
-  const uint64_t rem0 = f0 - j0 * p.k;    // and its offset in that row
-
-#pragma unroll
-  for (int g = 0; g < kIter; g += kGroup) {
-    V y[kGroup];
-    V* dst[kGroup];
-    uint32_t lf[kGroup];
-    bool live[kGroup], fresh[kGroup];
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      const uint32_t le = (uint32_t)(g + u) * kBlock + threadIdx.x;
-      live[u] = le < nelem;
-      lf[u] = le * VEC;
-      dst[u] = nullptr;
-      fresh[u] = false;
-      if (!live[u]) continue;
-      const uint64_t xoff = rem0 + lf[u];
-      uint64_t q, within;
-      if (p.k >= (uint64_t)TILE) {
-        q = xoff >= p.k ? 1u : 0u;
-        within = q ? xoff - p.k : xoff;
-      } else {
-        const uint32_t q32 = (uint32_t)xoff / (uint32_t)p.k;
-        q = q32;
-        within = (uint32_t)xoff - q32 * (uint32_t)p.k;
-      }
-      const uint64_t r = p.ref[j0 + q];
-      dst[u] = reinterpret_cast<V*>(p.arena + (r & ~kRefNew) * p.k + within);
-      if (r == kRefAbsent) {  // a key the lookup refused (duplicate in the request, full table)
-        live[u] = false;
-        continue;
-      }
-      fresh[u] = (r & kRefNew) != 0 && !p.ignore_new;
+  if (!live) return;
+  const uint64_t row = row0 + over;
+  const unsigned count = REST && c + 1 == quads ? rest : 4u;
+  float* side = p.req + row * p.k + c * 4;
+  // (a shorter quad is read whole: what follows it is the next row, or the room behind the last row of the
+  // arena; only the end of the request's values is the end of what may be read)
+  if (OP == kOpAcc && REST) x = count == 4 || row + 1 < p.n ? load_quad<STREAM>(side) : load_part<STREAM>(side, rest);
+  const uint64_t r = p.ref[row];
+  if (r == kRefAbsent) return;  // a key the lookup refused (duplicate in the request, full table)
+  const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
+  float* dst = p.arena + (r & ~kRefNew) * p.k + c * 4;
+  f32x4 y = (f32x4)(0.f);
+  if (!fresh) y = load_quad<STREAM>(dst);
+  if (OP == kOpAcc) {
+    if (rejected) {
+      if (!fresh) return;
+    } else {
+      y = y + x;  // a created row is a zero row first (0.0f + v), kv_app.h:454
     }
-    // all stored-row loads of the group before the first add
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      y[u] = VecT<VEC>::zero();
-      if (live[u] && !fresh[u]) y[u] = vload<STREAM>(dst[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kGroup; ++u) {
-      if (!live[u]) continue;
-      if (OP == kOpAcc) {
-        if (rejected) {
-          if (fresh[u]) vstore<STREAM>(VecT<VEC>::zero(), dst[u]);
-        } else {
-          // a created row is a zero row first (0.0f + v), kv_app.h:454
-          vstore<STREAM>(y[u] + x[g + u], dst[u]);
-        }
-      } else {
-        vstore<STREAM>(y[u], reinterpret_cast<V*>(p.req + f0 + lf[u]));
-        if (fresh[u]) vstore<STREAM>(VecT<VEC>::zero(), dst[u]);  // pull created the row: zeros
-      }
+    if (!REST || count == 4) store_quad<STREAM>(y, dst); else store_part<STREAM>(y, dst, rest);
+  } else {
+    if (!REST || count == 4) store_quad<STREAM>(y, side); else store_part<STREAM>(y, side, rest);
+    if (fresh) {  // pull created the row: zeros
+      if (!REST || count == 4) store_quad<STREAM>(y, dst); else store_part<STREAM>(y, dst, rest);
     }
   }
 }
@@ -891,29 +892,27 @@ constexpr unsigned kWaveSpan = 128;
 // even when it turns out not to be needed, so that it is not a second round trip after the
 // decision) and the request-side values. `bound` is what the host knows of the request's
 // length; the data may be shorter.
-template <int OP, int VEC, bool STREAM, unsigned WTILE>
-__device__ __forceinline__ void rows_wave_ask(const RowsParams& p, uint64_t bound,
-                                              typename VecT<VEC>::type* x, TileNote& aff) {
-  using V = typename VecT<VEC>::type;
-  constexpr int kIter = WTILE / (VEC * 64);
+template <int OP, bool STREAM>
+__device__ __forceinline__ void rows_wave_ask(const RowsParams& p, uint64_t bound, f32x4& x, TileNote& aff) {
   const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t wt = (uint64_t)p.blk * (kBlock / 64) + wave;
-  const uint64_t f0 = wt * WTILE;
+  const uint64_t f0 = wt * kTileVar;
   const uint64_t left = bound > f0 ? bound - f0 : 0;  // 0: the tile lies past the data
-  const uint32_t nelem = (uint32_t)(left < (uint64_t)WTILE ? left : (uint64_t)WTILE) / VEC;
+  const uint32_t floats = (uint32_t)(left < (uint64_t)kTileVar ? left : (uint64_t)kTileVar);
   aff.first = kTileNotAffine;
   aff.second = 0;
-  if (VEC == 4 && left) {
+  if (left) {
     const u64x2 w = *reinterpret_cast<const u64x2*>(&p.tile_aff[wt]);  // one 128-bit load
     aff.first = w.x;
     aff.second = w.y;
   }
+  x = (f32x4)(0.f);
   if (OP == kOpAcc) {
-#pragma unroll
-    for (int i = 0; i < kIter; ++i) {
-      const uint32_t le = (uint32_t)i * 64 + lane;
-      x[i] = VecT<VEC>::zero();
-      if (le < nelem) x[i] = vload<STREAM>(reinterpret_cast<const V*>(p.req + f0 + le * VEC));
+    const uint32_t lf = lane * 4;
+    if (lf + 4 <= floats) {
+      x = load_quad<STREAM>(p.req + f0 + lf);
+    } else if (lf < floats) {  // the end of the request
+      x = load_part<STREAM>(p.req + f0 + lf, floats - lf);
     }
   }
 }
@@ -923,60 +922,48 @@ __device__ __forceinline__ void rows_wave_ask(const RowsParams& p, uint64_t boun
 // lookup that created them), the note the row kernel of the cached request left maps every
 // float with an offset and neither the row table nor a search is needed. Returns false when the
 // tile has to take the general way. Wavefront-uniform.
-template <int OP, bool STREAM, unsigned WTILE>
-__device__ __forceinline__ bool rows_wave_affine(const RowsParams& p, uint64_t total,
-                                                 const f32x4* x, const TileNote& aff) {
-  using V = f32x4;
-  constexpr int VEC = 4;
-  constexpr int kIter = WTILE / (VEC * 64);
-  static_assert(WTILE < (1u << kTileSplitBits), "the split index does not fit the note");
+template <int OP, bool STREAM>
+__device__ __forceinline__ bool rows_wave_affine(const RowsParams& p, uint64_t total, const f32x4& x,
+                                                 const TileNote& aff) {
+  static_assert(kTileVar < (1u << kTileSplitBits), "the split index does not fit the note");
   if (aff.first == kTileNotAffine) return false;
   const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t wt = (uint64_t)p.blk * (kBlock / 64) + wave;
-  const uint64_t f0 = wt * WTILE;
+  const uint64_t f0 = ((uint64_t)p.blk * (kBlock / 64) + wave) * kTileVar;
   if (f0 >= total) return true;
-  const uint32_t nelem = (uint32_t)((total - f0 < (uint64_t)WTILE) ? (total - f0) : (uint64_t)WTILE) / VEC;
-  // rows start on multiples of four floats here, so no 128-bit element straddles the split
+  const uint32_t lf = lane * 4;
+  if (lf >= (total - f0 < (uint64_t)kTileVar ? (uint32_t)(total - f0) : kTileVar)) return true;
+  // rows start on multiples of four floats here, so no quad straddles the split
   const uint32_t split = aff.second ? (uint32_t)(aff.second & ((1u << kTileSplitBits) - 1)) : ~0u;
   const int64_t first = (int64_t)aff.first;
   const int64_t second = (int64_t)(aff.second >> kTileSplitBits) - kTileNoteBias;  // may be negative
-  V y[kIter];
-  V* dst[kIter];
-#pragma unroll
-  for (int i = 0; i < kIter; ++i) {
-    const uint32_t le = (uint32_t)i * 64 + lane;
-    dst[i] = reinterpret_cast<V*>(p.arena + ((le * VEC >= split ? second : first) + (int64_t)(le * VEC)));
-    y[i] = VecT<VEC>::zero();
-    if (le < nelem) y[i] = vload<STREAM>(dst[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < kIter; ++i) {
-    const uint32_t le = (uint32_t)i * 64 + lane;
-    if (le >= nelem) continue;
-    if (OP == kOpAcc) {
-      vstore<STREAM>(y[i] + x[i], dst[i]);
-    } else {
-      vstore<STREAM>(y[i], reinterpret_cast<V*>(p.req + f0 + le * VEC));
-    }
+  float* dst = p.arena + ((lf >= split ? second : first) + (int64_t)lf);
+  const f32x4 y = load_quad<STREAM>(dst);
+  if (OP == kOpAcc) {
+    store_quad<STREAM>(y + x, dst);
+  } else {
+    store_quad<STREAM>(y, p.req + f0 + lf);
   }
   return true;
 }
 
-// `x` comes from rows_wave_ask; x[i] is used only below `total`.
-template <int OP, int VEC, bool STREAM, unsigned WTILE>
+// `x` comes from rows_wave_ask; it is used only below `total`. RAGGED: some row's length is not a
+// multiple of four, so a quad may hold the end of one row and the start of the next (rows themselves
+// start on multiples of four floats in the arena). The part in the row of its first float and the part in
+// the next row are one access each, both asked for before either is used; where rows of one or two floats
+// make it more than two parts, the floats are moved one by one, their loads together. (Every float used to
+// be looked up and moved on its own.) The arena side of such rows is read and written through the caches
+// whatever the size of the request: a 128-byte line holds pieces of several rows, and lines that are
+// written piecewise past the caches cost a third of the bandwidth (1M rows of 1 to 60 floats: 345 us per
+// push + pull against 221).
+template <int OP, bool RAGGED, bool STREAM>
 __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t total,
                                                  int32_t* s_off_all, uint64_t* s_ref_all,
-                                                 bool rejected, bool same,
-                                                 const typename VecT<VEC>::type* x) {
-  using V = typename VecT<VEC>::type;
-  constexpr int kIter = WTILE / (VEC * 64);  // elements per lane
-  static_assert(kIter >= 1 && kIter <= 8, "wave tile out of range");
+                                                 bool rejected, bool same, const f32x4& x) {
   const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t wt = (uint64_t)p.blk * (kBlock / 64) + wave;
-  const uint64_t f0 = wt * WTILE;
+  const uint64_t f0 = wt * kTileVar;
   if (f0 >= total) return;  // the whole wavefront leaves; nothing below synchronises workgroups
-  const uint32_t tile_floats = (uint32_t)((total - f0 < (uint64_t)WTILE) ? (total - f0) : (uint64_t)WTILE);
-  const uint32_t nelem = tile_floats / VEC;
+  const uint32_t tile_floats = (uint32_t)((total - f0 < (uint64_t)kTileVar) ? (total - f0) : (uint64_t)kTileVar);
 
   const uint64_t j_lo = p.tile_key[wt];
   const uint32_t span = (uint32_t)((uint64_t)p.tile_key[wt + 1] - j_lo + 1);
@@ -999,7 +986,7 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
     // piece when all distances are equal (the rows lie back to back, in request order, without
     // padding between them) and two pieces when they change once.
     TileNote note = {kTileNotAffine, 0};
-    if (VEC == 4 && staged) {
+    if (!RAGGED && staged) {
       bool absent = false;
       int64_t d[(kWaveSpan + 63) / 64];
       bool has[(kWaveSpan + 63) / 64];
@@ -1049,71 +1036,122 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
     if (lane == 0) p.tile_aff[wt] = note;
   }
 
-  V y[kIter];
-  V* dst[kIter];
-  bool live[kIter], fresh[kIter];
-#pragma unroll
-  for (int i = 0; i < kIter; ++i) {
-    const uint32_t le = (uint32_t)i * 64 + lane;
-    const uint32_t lf = le * VEC;
-    live[i] = le < nelem;
-    dst[i] = nullptr;
-    fresh[i] = false;
-    if (!live[i]) continue;
-    uint64_t r, within;
-    if (staged) {
-      // last key whose first float is at or before lf (zero-length rows repeat an offset)
-      uint32_t lo = 0, hi = span;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (s_off[mid] <= (int32_t)lf) lo = mid + 1; else hi = mid;
-      }
-      r = s_ref[lo - 1];
-      within = (uint64_t)((int32_t)lf - s_off[lo - 1]);
-    } else {
-      const uint64_t f = f0 + lf;
-      uint64_t lo = j_lo, hi = j_lo + span;
-      while (lo < hi) {
-        const uint64_t mid = (lo + hi) >> 1;
-        if (p.off[mid] <= f) lo = mid + 1; else hi = mid;
-      }
-      r = p.ref[lo - 1];
-      within = f - p.off[lo - 1];
-    }
-    dst[i] = reinterpret_cast<V*>(p.arena + (((r & ~kRefNew) >> kLenBits) << 2) + within);
-    if (r == kRefAbsent) {  // a key the lookup refused (duplicate in the request, full table)
-      live[i] = false;
-      continue;
-    }
-    fresh[i] = (r & kRefNew) != 0 && !p.ignore_new;
+  const uint32_t lf = lane * 4;
+  if (lf >= tile_floats) return;
+  // offsets (from the tile's first float) and references of the keys that overlap the tile, from LDS or,
+  // where there are too many, from where they lie
+  auto off_of = [&](uint32_t s) { return staged ? (int64_t)s_off[s] : (int64_t)(p.off[j_lo + s] - f0); };
+  auto ref_of = [&](uint32_t s) { return staged ? s_ref[s] : p.ref[j_lo + s]; };
+  auto place = [&](uint64_t r, int64_t within) {
+    return p.arena + (((r & ~kRefNew) >> kLenBits) << 2) + within;
+  };
+  // the key that holds the quad's first float: the last one whose first float is at or before it
+  // (zero-length rows repeat an offset)
+  uint32_t lo = 0, hi = span;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (off_of(mid) <= (int64_t)lf) lo = mid + 1; else hi = mid;
   }
-#pragma unroll
-  for (int i = 0; i < kIter; ++i) {
-    y[i] = VecT<VEC>::zero();
-    if (live[i] && !fresh[i]) y[i] = vload<STREAM>(dst[i]);
+  const uint64_t r = ref_of(lo - 1);
+  float* dst = place(r, (int64_t)lf - off_of(lo - 1));
+  // a key the lookup refused (duplicate in the request, full table) is neither read nor written
+  const bool here = r != kRefAbsent;
+  const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
+  float* side = p.req + f0 + lf;
+  if (!RAGGED) {
+    if (!here) return;
+    f32x4 y = (f32x4)(0.f);
+    if (!fresh) y = load_quad<STREAM>(dst);
+    if (OP == kOpGather) {
+      store_quad<STREAM>(y, side);
+    } else if (!rejected) {
+      store_quad<STREAM>(y + x, dst);  // a created row is a zero row first (0.0f + v)
+    } else if (fresh) {
+      // a refused push changes no stored value; rows it created stay, as zero rows
+      store_quad<STREAM>(y, dst);
+    }
+    return;
   }
-#pragma unroll
-  for (int i = 0; i < kIter; ++i) {
-    if (!live[i]) continue;
-    const uint32_t lf = ((uint32_t)i * 64 + lane) * VEC;
-    if (OP == kOpAcc) {
-      if (rejected) {
-        // a refused push changes no stored value; rows it created stay, as zero rows
-        if (fresh[i]) vstore<STREAM>(VecT<VEC>::zero(), dst[i]);
+  const uint32_t upto = tile_floats - lf < 4u ? tile_floats - lf : 4u;
+  const int64_t end = off_of(lo);
+  const uint32_t count = end - (int64_t)lf < (int64_t)upto ? (uint32_t)(end - (int64_t)lf) : upto;
+  // the next row, when the quad reaches into it
+  uint64_t r2 = kRefAbsent;
+  float* dst2 = nullptr;
+  uint32_t two = upto;  // floats of the quad that the two rows hold
+  if (count < upto) {
+    uint32_t key = lo;  // (zero-length rows are stepped over; the key table closes with the end of the request)
+    while (off_of(key + 1) <= end) ++key;
+    r2 = ref_of(key);
+    dst2 = place(r2, 0);
+    const int64_t end2 = off_of(key + 1);
+    if (end2 - (int64_t)lf < (int64_t)upto) two = (uint32_t)(end2 - (int64_t)lf);
+  }
+  const bool here2 = r2 != kRefAbsent;
+  const bool fresh2 = (r2 & kRefNew) != 0 && !p.ignore_new;
+  if (two == upto) {
+    // (reading a quad whole is safe: what follows its row is another row, or the room behind the arena's last)
+    f32x4 y = (f32x4)(0.f), y2 = (f32x4)(0.f);
+    if (here && !fresh) y = load_quad<false>(dst);
+    if (here2 && !fresh2) y2 = load_quad<false>(dst2);
+    if (OP == kOpGather) {
+      f32x4 v = y;
+      if (count == 1) v.y = y2.x, v.z = y2.y, v.w = y2.z;
+      if (count == 2) v.z = y2.x, v.w = y2.y;
+      if (count == 3) v.w = y2.x;
+      if (upto == 4 && here && (here2 || count == 4)) {
+        store_quad<STREAM>(v, side);
       } else {
-        vstore<STREAM>(y[i] + x[i], dst[i]);  // a created row is a zero row first (0.0f + v)
+        if (here) store_part<false>(y, side, count);
+        if (here2) store_part<false>(y2, side + count, upto - count);
       }
-    } else {
-      vstore<STREAM>(y[i], reinterpret_cast<V*>(p.req + f0 + lf));
+      return;
+    }
+    if (here && (!rejected || fresh)) store_part<false>(rejected ? y : y + x, dst, count);
+    if (here2 && (!rejected || fresh2)) {
+      f32x4 x2 = x;
+      if (count == 1) x2.x = x.y, x2.y = x.z, x2.z = x.w;
+      if (count == 2) x2.x = x.z, x2.y = x.w;
+      if (count == 3) x2.x = x.w;
+      store_part<false>(rejected ? y2 : y2 + x2, dst2, upto - count);
+    }
+    return;
+  }
+  // three rows or more
+  float* at[4];
+  float cur[4];
+  bool made[4];
+  uint32_t key = lo - 1;
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) {
+    at[e] = nullptr;
+    made[e] = false;
+    if (e >= upto) continue;
+    while (off_of(key + 1) <= (int64_t)(lf + e)) ++key;
+    const uint64_t q = ref_of(key);
+    if (q == kRefAbsent) continue;
+    made[e] = (q & kRefNew) != 0 && !p.ignore_new;
+    at[e] = place(q, (int64_t)(lf + e) - off_of(key));
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) cur[e] = at[e] && !made[e] ? *at[e] : 0.f;
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) {
+    if (!at[e]) continue;
+    if (OP == kOpGather) {
+      side[e] = cur[e];
+    } else if (!rejected) {
+      *at[e] = cur[e] + x[e];
+    } else if (made[e]) {
+      *at[e] = cur[e];
     }
   }
 }
 
-// Request-side floats per workgroup (fixed rows) and per wavefront (var-len rows). One
+// Quads per workgroup (fixed rows) and request-side floats per wavefront (var-len rows). One
 // 128-bit access per lane and many small workgroups stream fastest on this GPU (6.5 TB/s for
 // `row += in` against 5.5 TB/s with four accesses per lane).
-constexpr unsigned kTileFixed = 1024;
-constexpr unsigned kTileVar = PSKV_TILE_VAR;        // per wavefront; the tile table's granularity
+constexpr unsigned kQuadsFixed = kBlock;
 constexpr unsigned kRowsVarPerBlock = kTileVar * (kBlock / 64);
 
 template <int OP, bool VARLEN, bool STREAM>
@@ -1121,9 +1159,11 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch b) {
   const TableReq& d = b.t[blockIdx.y];
   // the grid is sized for the largest table of the launch: workgroups (VARLEN: wavefronts) past
   // this table's floats leave before they touch anything
-  if ((((uint64_t)blockIdx.x + d.tile_base) * (kBlock / 64) + (VARLEN ? (threadIdx.x >> 6) : 0u)) *
-          (VARLEN ? kTileVar : kTileFixed / (kBlock / 64)) >= d.total)
-    return;
+  if (VARLEN) {
+    if ((((uint64_t)blockIdx.x + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total) return;
+  } else {
+    if (d.nvals + (uint64_t)blockIdx.x * kQuadsFixed >= d.ntiles) return;
+  }
   RowsParams p;
   p.req = d.req;
   p.arena = d.arena;
@@ -1135,40 +1175,32 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch b) {
   p.n = d.n;
   p.total = d.total;
   p.k = d.k;
-  p.force_scalar = d.force_scalar;
   p.ignore_new = d.ignore_new;
   p.total_on_device = d.total_on_device;
   p.blk = blockIdx.x + d.tile_base;
   p.tag = d.tag;
   __shared__ int32_t s_off[VARLEN ? (kWaveSpan + 1) * (kBlock / 64) : 1];
   __shared__ uint64_t s_ref[VARLEN ? kWaveSpan * (kBlock / 64) : 1];
-  bool rejected = false;
-  bool scalar = p.force_scalar != 0;
-  uint64_t total = p.total;
   // What the device knows about the request: one load, one wait per wavefront.
   const ReqFacts facts = load_req_facts(p.st);
   if (VARLEN) {
     // every argument the common path uses, asked for at once (the compiler otherwise fetches them
     // group by group where they are first used, one wait each)
     asm volatile("" ::"s"(p.req), "s"(p.arena), "s"(p.tile_aff), "s"(p.total),
-                 "s"(p.force_scalar), "s"(p.total_on_device), "s"(p.tag.epoch));
-  }
-  if (VARLEN) {
-    // the grid covers the room in the caller's buffer, which may be more than the data
-    const uint64_t f0 = ((uint64_t)p.blk * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar;
-    if (f0 >= p.total) return;
-    // the loads that need no facts are on their way before the facts are looked at
-    f32x4 x4[kTileVar / 256];
+                 "s"(p.total_on_device), "s"(p.tag.epoch));
+    // the grid covers the room in the caller's buffer, which may be more than the data; the loads
+    // that need no facts are on their way before the facts are looked at
+    uint64_t total = p.total;
+    f32x4 x;
     TileNote aff = {kTileNotAffine, 0};
-    if (!scalar) rows_wave_ask<OP, 4, STREAM, kTileVar>(p, p.total, x4, aff);
+    rows_wave_ask<OP, STREAM>(p, total, x, aff);
     // a request served from the cached references creates nothing and cannot have been refused
     const bool same = facts.same_epoch == p.tag.epoch;
     if (p.tag.replay && !same) return;
     if (same) p.ignore_new = 1;
     const unsigned err = same ? 0u : facts.req_error;
     if (err & (kDevErrBadLen | kDevErrSizeMismatch | kDevErrDuplicate)) return;
-    rejected = (err & kDevErrLenChanged) != 0;
-    scalar = scalar || (facts.misaligned != 0);
+    const bool rejected = (err & kDevErrLenChanged) != 0;
     if (p.total_on_device) {
       total = facts.scan_total;
       if (total > p.total) {  // the response does not fit the caller's buffer: write nothing
@@ -1176,22 +1208,26 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch b) {
         return;
       }
     }
-    if (scalar) {
-      float x1[kTileVar / 64];
-      TileNote none;
-      rows_wave_ask<OP, 1, STREAM, kTileVar>(p, total, x1, none);
-      rows_wave_varlen<OP, 1, STREAM, kTileVar>(p, total, s_off, s_ref, rejected, same, x1);
+    if (facts.misaligned != 0) {
+      rows_wave_varlen<OP, true, STREAM>(p, total, s_off, s_ref, rejected, same, x);
     } else {
-      if (same && rows_wave_affine<OP, STREAM, kTileVar>(p, total, x4, aff)) return;
-      rows_wave_varlen<OP, 4, STREAM, kTileVar>(p, total, s_off, s_ref, rejected, same, x4);
+      if (same && rows_wave_affine<OP, STREAM>(p, total, x, aff)) return;
+      rows_wave_varlen<OP, false, STREAM>(p, total, s_off, s_ref, rejected, same, x);
     }
   } else {
     if (p.tag.replay && facts.same_epoch != p.tag.epoch) return;
     if (facts.same_epoch == p.tag.epoch) p.ignore_new = 1;
-    if (scalar) {
-      rows_tile_fixed<OP, 1, STREAM, kTileFixed>(p, total);
+    const uint64_t q0 = d.nvals + (uint64_t)blockIdx.x * kQuadsFixed;
+    if (p.k & 3) {
+      // (short rows share 128-byte lines with their neighbours, which lie in other workgroups' hands: lines
+      // written piecewise past the caches made rows of 33 floats a third slower)
+      if (p.k >= 1024) {
+        rows_quads_fixed<OP, STREAM, true>(p, q0, d.ntiles);
+      } else {
+        rows_quads_fixed<OP, false, true>(p, q0, d.ntiles);
+      }
     } else {
-      rows_tile_fixed<OP, 4, STREAM, kTileFixed>(p, total);
+      rows_quads_fixed<OP, STREAM, false>(p, q0, d.ntiles);
     }
   }
 }

@@ -1,0 +1,91 @@
+"""Rows that do not fit 16-byte quads: every remainder of the row length, quads that hold two rows or more,
+buffers on any float, pieces of a host-resident request that end inside a quad. Against the CPU oracle, bit
+for bit."""
+import numpy as np
+import pytest
+
+from helpers import assert_bits_equal, to_dev, unique_keys
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+
+def _off_by(a, dev, shift):
+    """The values on the device, `shift` floats behind a 16-byte boundary."""
+    import torch
+    room = torch.zeros(a.size + shift, dtype=torch.float32, device=dev)
+    room[shift:] = to_dev(a, dev)
+    return room[shift:]
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 31, 64, 66, 255, 1021, 1022, 1023, 1024, 1025, 1030])
+def test_fixed_rows_of_any_length(capi, orc, dev, k, shift):
+    announce("fixed rows", k, shift)
+    import torch
+    rng = np.random.default_rng(k)
+    n = max(3, 60_000 // k) | 1
+    t, o = capi.Table(capi.MODE_FIXED, row_len=k), orc.Store(orc.MODE_FIXED, k)
+    keys = unique_keys(rng, 2 * n)
+    for turn in range(4):
+        some = np.sort(rng.choice(keys, n, replace=False))
+        vals = rng.standard_normal(n * k).astype(np.float32)
+        t.push(to_dev(some, dev), _off_by(vals, dev, shift))
+        o.push(some, vals)
+        if turn == 2:  # keys that the store has not seen are answered, and kept, as zero rows
+            some = keys
+        out = _off_by(np.full(some.size * k, 7, np.float32), dev, 3 * shift)
+        t.pull(to_dev(some, dev), out)
+        torch.cuda.synchronize()
+        assert_bits_equal(out.cpu().numpy(), o.pull(some)[0], "k = %d" % k)
+    assert_bits_equal(t.dump()[2], o.dump()[2])
+
+
+LENGTHS = {"any": lambda rng, n: rng.integers(0, 101, n), "short": lambda rng, n: rng.integers(0, 4, n),
+           "ones": lambda rng, n: np.ones(n, np.int64), "mixed": lambda rng, n: rng.choice([0, 1, 2, 3, 5, 258, 1025], n),
+           "tail": lambda rng, n: np.where(np.arange(n) == n - 1, 3, 8)}
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n", [1, 130, 5000])
+@pytest.mark.parametrize("which", sorted(LENGTHS))
+def test_varlen_rows_of_any_length(capi, orc, dev, which, n, shift):
+    announce("varlen rows", which, n, shift)
+    import torch
+    rng = np.random.default_rng(n)
+    t, o = capi.Table(capi.MODE_VARLEN), orc.Store(orc.MODE_VARLEN)
+    keys = unique_keys(rng, 2 * n)
+    all_lens = LENGTHS[which](rng, 2 * n).astype(np.int32)
+    for turn in range(4):
+        pick = np.sort(rng.choice(2 * n, n, replace=False)) if turn != 1 else pick  # (turn 1: the same keys again)
+        some, lens = keys[pick], all_lens[pick]
+        vals = rng.standard_normal(int(lens.sum())).astype(np.float32)
+        t.push(to_dev(some, dev), _off_by(vals, dev, shift), to_dev(lens, dev))
+        o.push(some, vals, lens)
+        if turn == 2:
+            some = keys  # some of them absent: answered with length 0
+        want, want_lens = o.pull(some)
+        out = _off_by(np.full(want.size + 5, 7, np.float32), dev, 3 * shift)
+        out_lens = torch.empty(some.size, dtype=torch.int32, device=dev)
+        got = t.pull(to_dev(some, dev), out, out_lens)
+        torch.cuda.synchronize()
+        assert got == want.size and np.array_equal(out_lens.cpu().numpy(), want_lens)
+        host = out.cpu().numpy()
+        assert_bits_equal(host[:got], want, which)
+        assert (host[got:] == 7).all()
+
+
+@pytest.mark.parametrize("n,k", [(3, 1_500_001), (5, 1_048_579), (40_001, 131)])
+def test_host_resident_rows_in_pieces(capi, orc, dev, n, k):
+    """Several pieces of the ring per request; their edges fall inside rows and inside quads."""
+    announce("host pieces", n, k)
+    rng = np.random.default_rng(k)
+    t, o = capi.Table(capi.MODE_FIXED, row_len=k), orc.Store(orc.MODE_FIXED, k)
+    keys = unique_keys(rng, n)
+    for _ in range(2):
+        vals = rng.random(n * k, dtype=np.float32) - np.float32(0.5)
+        t.push(keys, vals)
+        o.push(keys, vals)
+        out = np.zeros(n * k, np.float32)
+        t.pull(keys, out)
+        assert_bits_equal(out, o.pull(keys)[0])
