@@ -10,10 +10,11 @@
 
 namespace pskv {
 
-// Keys per thread: 4 for long requests (fewer atomic adds on the arena counter and fewer
-// tickets), 1 for short ones so that even 100k keys spread over a few hundred workgroups.
-constexpr int kScanItemsLarge = 4;
-constexpr uint64_t kScanLargeKeys = 1u << 20;
+// Pass 1 takes four keys per thread whatever the size of the request: kScanPart keys per workgroup, one
+// total each. (With one key per thread the 782 totals and tickets of a 200,000-key push were most of
+// the kernel's time.)
+constexpr int kScanItems = 4;
+constexpr uint64_t kScanPart = (uint64_t)kBlock * kScanItems;
 
 // Sum of `x` and OR of `f` over the workgroup; results valid in every thread. `red` and
 // `fred` hold kBlock/64 entries each.
@@ -97,39 +98,41 @@ __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned 
   return *s_last != 0u;
 }
 
-// Pass 1, what the last workgroup does once all totals are there: it turns them into
-// exclusive offsets in place, stores the grand total, publishes the request's flags and folds
-// the previous request's error bits into the sticky ones, which makes this the point where
-// one request's flags end and the next begin. Every thread of that workgroup calls it;
-// the facts collected from all workgroups are returned in thread 0.
-__device__ __forceinline__ unsigned scan_pass1_last(unsigned long long* part, DevState* st,
-                                                    unsigned nblk, unsigned long long epoch,
-                                                    unsigned long long* red,
-                                                    unsigned long long* carry_s) {
-  scan_spine(part, nblk, red, carry_s);
-  unsigned flags = 0;
-  if (threadIdx.x == 0) {
-    flags = atomicExch(&st->req_flags, 0u);
-    st->scan_total = *carry_s;
-    st->error |= st->req_error;
-    const bool bad_len = (flags & kReqBadLen) != 0u;
-    const bool dup = (flags & kReqDuplicate) != 0u;
-    st->req_error = (bad_len ? kDevErrBadLen : 0u) | (dup ? kDevErrDuplicate : 0u);
-    if (bad_len || dup) st->bad_epoch = epoch;
-    st->misaligned = flags & kReqMisaligned;
-  }
-  return flags;
+// Pass 1, what the last workgroup does once all totals are there, first half: the facts that the
+// workgroups have collected. Every thread of that workgroup calls it and gets them. `shared` is a word of LDS.
+__device__ __forceinline__ unsigned scan_pass1_facts(DevState* st, unsigned* shared) {
+  if (threadIdx.x == 0) *shared = atomicExch(&st->req_flags, 0u);
+  __syncthreads();
+  return *shared;
 }
 
-// Pass 2, the workgroup's part: every thread passes its kScanItems consecutive lens
+// Second half: turns the totals into exclusive offsets in place and stores the grand total, unless the
+// request repeats the cached one (`same`: offsets and total are there), publishes the request's flags and
+// folds the previous request's error bits into the sticky ones, which makes this the point where
+// one request's flags end and the next begin. Every thread of that workgroup calls it.
+__device__ __forceinline__ void scan_pass1_last(unsigned long long* part, DevState* st, unsigned nparts,
+                                                unsigned long long epoch, unsigned flags, bool same,
+                                                unsigned long long* red, unsigned long long* carry_s) {
+  if (!same) scan_spine(part, nparts, red, carry_s);
+  if (threadIdx.x != 0) return;
+  if (!same) st->scan_total = *carry_s;
+  st->error |= st->req_error;
+  const bool bad_len = (flags & kReqBadLen) != 0u;
+  const bool dup = (flags & kReqDuplicate) != 0u;
+  st->req_error = (bad_len ? kDevErrBadLen : 0u) | (dup ? kDevErrDuplicate : 0u);
+  if (bad_len || dup) st->bad_epoch = epoch;
+  st->misaligned = flags & kReqMisaligned;
+}
+
+// Pass 2, the workgroup's part: every thread passes its kItems consecutive lens
 // (sign-extended; zero past the end) starting at index `base`; the workgroup rescans them from
 // its exclusive offset `part_b` and writes off[]. With a tile table it also records, for each
 // request-side tile of `tile` floats, the key that owns the tile's first float: key j owns
 // floats [off[j], off[j+1]), so every tile gets exactly one writer and the row kernel needs no
 // search to find where a tile starts. Entry `ntiles` closes the table. `wsum` holds kBlock/64
 // words.
-template <int kScanItems>
-__device__ __forceinline__ void scan_pass2_offsets(const unsigned long long (&v)[kScanItems],
+template <int kItems>
+__device__ __forceinline__ void scan_pass2_offsets(const unsigned long long (&v)[kItems],
                                                    uint64_t base, uint64_t n,
                                                    unsigned long long part_b,
                                                    uint64_t* __restrict__ off,
@@ -137,7 +140,7 @@ __device__ __forceinline__ void scan_pass2_offsets(const unsigned long long (&v)
                                                    uint64_t tile, unsigned long long* wsum) {
   unsigned long long s = 0;
 #pragma unroll
-  for (int j = 0; j < kScanItems; ++j) s += v[j];
+  for (int j = 0; j < kItems; ++j) s += v[j];
   const unsigned long long inc = wave_incl_scan_u64(s);
   const unsigned wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 63) wsum[wave] = inc;
@@ -146,7 +149,7 @@ __device__ __forceinline__ void scan_pass2_offsets(const unsigned long long (&v)
   for (unsigned w = 0; w < wave; ++w) run += wsum[w];
   if (tile_key && base == 0) tile_key[ntiles] = (uint32_t)(n - 1);
 #pragma unroll
-  for (int j = 0; j < kScanItems; ++j) {
+  for (int j = 0; j < kItems; ++j) {
     if (base + j < n) {
       off[base + j] = run;
       const unsigned long long end = run + v[j];
@@ -162,12 +165,7 @@ __device__ __forceinline__ void scan_pass2_offsets(const unsigned long long (&v)
   }
 }
 
-// `n_largest`: the longest key list among the tables a launch serves; all of them use one split.
-inline int scan_items(uint64_t n_largest) { return n_largest >= kScanLargeKeys ? kScanItemsLarge : 1; }
-inline uint64_t scan_num_parts(uint64_t n, int items) {
-  const uint64_t chunk = (uint64_t)kBlock * items;
-  return (n + chunk - 1) / chunk;
-}
+inline uint64_t scan_num_parts(uint64_t n) { return (n + kScanPart - 1) / kScanPart; }
 
 }  // namespace pskv
 #endif  // PSKV_SCAN_H_

@@ -275,6 +275,7 @@ struct pskv_table {
   GrowBuf cache_keys, cache_lens;
   bool cache_valid = false;
   uint64_t cache_n = 0, cache_nvals = 0;
+  uint64_t known_n = 0;  // FIXED: positions of cache_keys whose reference in the workspace belongs to the key there
   uint64_t epoch = 0;  // number of the last request that took part in this
 
   // SCALAR: the same idea with the VALUES of the cached keys kept in request order (and the
@@ -1152,13 +1153,13 @@ int launch_rows(Batch& bt, int op) {
   return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, k_rows<kOpGather, VARLEN, false>, nblk);
 }
 
-// Starts a row-mode request on every table with keys: numbers it and, where the key cache has
-// the right shape, lets the device compare the request with the cached one. Call after every
+// Starts a row-mode request on every table with keys: numbers it and (`compare`: a recorded one), where the
+// key cache has the right shape, lets the device compare the request with the cached one. Call after every
 // buffer the cache lives in has been grown for this request.
-int begin_row_request(Batch& bt) {
+int begin_row_request(Batch& bt, bool compare) {
   for (Item& it : bt) {
     if (!it.r.n) continue;
-    it.tag = next_tag(it.t, it.r, true);
+    it.tag = next_tag(it.t, it.r, it.t->mode == PSKV_MODE_VARLEN);
     if (it.r.replay == kReplayCapture && !it.tag.try_cache)
       return set_error(PSKV_ESTALE, "the key cache does not hold the request that is being recorded%s",
                        it.t->mode == PSKV_MODE_VARLEN ? " (a PSKV_MODE_VARLEN pull leaves no key cache behind: record "
@@ -1167,6 +1168,7 @@ int begin_row_request(Batch& bt) {
     it.d.tag = it.tag;
     it.d.outcome = it.t->outcome;
   }
+  if (!compare) return PSKV_OK;
   return launch_batch(bt, PSKV_KERNEL_SAME_KEYS, k_same_keys, [](const Item& it) {
     return (it.r.n && it.tag.try_cache) ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems)
                                         : 0ull;
@@ -1188,8 +1190,10 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     if (rc) return rc;
     rc = grow(t, &t->cache_keys, r.n * sizeof(uint64_t));
     if (rc) return rc;
+    if (!t->cache_valid) t->known_n = 0;
     Carver c(t->ws.ptr);
     TableReq& d = it.d;
+    d.cached = (uint32_t)std::min<uint64_t>(t->known_n, 0xffffffffu);
     d.slots = t->slots;
     d.mask = t->cap - 1;
     d.st = t->st;
@@ -1204,10 +1208,10 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     n_largest = std::max(n_largest, r.n);
   }
   if (!n_largest) return PSKV_OK;
-  int rc = begin_row_request(bt);
+  int rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
   if (rc) return rc;
   if (bt[0].r.replay == kReplayCapture) {
-    // a recorded repeat uses the references that are there: no lookup
+    // a recorded repeat is compared as a whole and uses the references that are there: no lookup
   } else if (n_largest >= kLookupLargeKeys) {
     rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, k_lookup_fixed<kLookupItemsLarge>, [](const Item& it) {
       return it.r.n ? (uint64_t)grid_for(it.r.n, kBlock * kLookupItemsLarge, kMaxGrid) : 0ull;
@@ -1224,6 +1228,7 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     it.t->cache_valid = true;
     it.t->cache_n = it.r.n;
     it.t->cache_nvals = it.r.n * it.d.k;
+    it.t->known_n = std::max(it.t->known_n, it.r.n);  // (what lies behind this request's last key holds still)
   }
   if (push) {
     for (Item& it : bt) {
@@ -1256,18 +1261,22 @@ int grow_tile_tables(pskv_table* t, uint64_t floats, uint64_t* ntiles_cap) {
   return grow(t, &t->tiles_aff, (*ntiles_cap + 1) * sizeof(TileNote));
 }
 
-// The kernels of a var-len request that work key by key: one workgroup per kBlock*items keys,
-// `items` per thread, the same split in every kernel of the request and for every table of the
-// batch (the scan's per-workgroup totals are indexed by it).
-int launch_keys(Batch& bt, int prof_kernel, int items, void (*k1)(ReqBatch), void (*k4)(ReqBatch)) {
-  return launch_batch(bt, prof_kernel, items == kScanItemsLarge ? k4 : k1,
-                      [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+// Keys per thread of the creating lookup: 4 for long requests (fewer atomic adds on the arena counter), 1 for
+// short ones so that even 100k keys spread over a few hundred workgroups.
+constexpr uint64_t kVarLookupLargeKeys = 1u << 20;
+
+// Workgroups for a kernel over `chunks` stretches of a request that returns at once when the request repeats
+// the cached one: one per stretch, or a few hundred that stride over them where the newest comparison of
+// requests of this kind has found the cached keys (a launch costs by the workgroup even then).
+uint64_t may_return_at_once(const Item& it, bool push, uint64_t chunks, size_t tables) {
+  const bool expected = it.tag.try_cache && it.t->sc_track[push ? 0 : 1].hit;
+  return expected ? std::min<uint64_t>(chunks, std::max<uint64_t>(32, 512 / tables)) : chunks;
 }
 
 // Pass 2 of a pull's scan for every table with a response: the request-side offsets of the
 // response and the tile table for Item::d.total floats of room (the row kernel fills the other
 // table).
-int make_tile_tables(Batch& bt, int items) {
+int make_tile_tables(Batch& bt) {
   for (Item& it : bt) {
     if (!it.d.total) continue;
     uint64_t ntiles_cap = 0;
@@ -1278,12 +1287,13 @@ int make_tile_tables(Batch& bt, int items) {
     it.d.ntiles = ntiles_cap;
   }
   if (bt[0].r.replay == kReplayCapture) return PSKV_OK;  // (a recorded repeat: the tables that are there)
-  return launch_batch(bt, -1, items == kScanItemsLarge ? k_var_offsets<kScanItemsLarge> : k_var_offsets<1>,
-                      [](const Item& it) { return (it.r.n && it.d.total) ? it.nparts : 0ull; });
+  return launch_batch(bt, -1, k_var_offsets, [&](const Item& it) {
+    return (it.r.n && it.d.total) ? may_return_at_once(it, false, it.nparts, bt.size()) : 0ull;
+  });
 }
 
 // Launches per var-len request: a push takes three (compare + scan pass 1; scan pass 2 +
-// find-or-create + counter record; rows), a pull four (compare; stored lengths + scan pass 1;
+// find-or-create + counter record; rows), a pull three (compare + stored lengths + scan pass 1;
 // scan pass 2 + tile table; rows), whatever the number of tables.
 int run_varlen(Batch& bt, bool push, bool pull) {
   uint64_t n_largest = 0;
@@ -1297,13 +1307,14 @@ int run_varlen(Batch& bt, bool push, bool pull) {
   // (keys per thread of the key-by-key kernels: by the keys of the whole launch, not of its largest table)
   uint64_t n_launch = 0;
   for (const Item& it : bt) n_launch += it.r.n;
-  const int items = scan_items(n_launch);
+  const bool large = n_launch >= kVarLookupLargeKeys;
+  const uint64_t chunk = kBlock * (large ? 4 : 1);  // keys per workgroup of the creating lookup
   const bool async_pull = pull && !push && !bt[0].r.need_total;
   for (Item& it : bt) {
     pskv_table* t = it.t;
     Request& r = it.r;
     if (!r.n) continue;
-    it.nparts = scan_num_parts(r.n, items);
+    it.nparts = scan_num_parts(r.n);
     const size_t need = Carver::need(r.n, 8) + Carver::need(r.n + 1, 8) + Carver::need(it.nparts, 8) +
                         Carver::need(r.n, 4);
     // Every buffer the key cache lives in is grown BEFORE the request is compared with the
@@ -1338,7 +1349,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       // every key may round its row up to a 16-byte unit, every workgroup may pad its rows' start
       int rc = r.replay == kReplayCapture
                    ? PSKV_OK
-                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * it.nparts, 4, &it.pub);
+                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * ((r.n + chunk - 1) / chunk), 4, &it.pub);
       if (rc) return rc;
       if (t->cache_nvals != r.nvals) t->cache_valid = false;  // same lens would mean the same total
       it.tag = next_tag(t, r, true);
@@ -1360,11 +1371,13 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
     }
-    int rc = launch_keys(bt, -1, items, k_var_push_begin<1>, k_var_push_begin<kScanItemsLarge>);
+    int rc = launch_batch(bt, -1, k_var_push_begin, [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
     if (rc) return rc;
     // (a recorded repeat uses the offsets, tile table and references that are there)
     if (bt[0].r.replay != kReplayCapture)
-      rc = launch_keys(bt, PSKV_KERNEL_LOOKUP, items, k_var_push_lookup<1>, k_var_push_lookup<kScanItemsLarge>);
+      rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, large ? k_var_push_lookup<4> : k_var_push_lookup<1>, [&](const Item& it) {
+        return it.r.n ? may_return_at_once(it, true, (it.r.n + chunk - 1) / chunk, bt.size()) : 0ull;
+      });
     if (rc) return rc;
     for (Item& it : bt) {
       if (!it.r.n) continue;
@@ -1401,11 +1414,11 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     }
     // A pull with the keys of the cached push finds every key present with the cached length
     // and reuses its references; any other pull recomputes them and so ends the cache.
-    rc = begin_row_request(bt);
+    rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
     if (rc) return rc;
     for (Item& it : bt)
       if (it.r.n && !it.tag.try_cache) it.t->cache_valid = false;
-    rc = launch_keys(bt, PSKV_KERNEL_LOOKUP, items, k_var_pull_lookup<1>, k_var_pull_lookup<kScanItemsLarge>);
+    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, k_var_pull_lookup, [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
     if (rc) return rc;
     if (async_pull) {
       // No host round trip: the grid covers the caller's buffer, the kernels take the real
@@ -1418,7 +1431,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
         it.d.total_on_device = 1;
         it.d.ignore_new = 1;
       }
-      rc = make_tile_tables(bt, items);
+      rc = make_tile_tables(bt);
       if (rc) return rc;
       return launch_rows<true>(bt, kOpGather);
     }
@@ -1457,7 +1470,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       it.d.total_on_device = 0;
       it.d.ignore_new = 1;
     }
-    rc = make_tile_tables(bt, items);
+    rc = make_tile_tables(bt);
     if (rc) return rc;
     rc = launch_rows<true>(bt, kOpGather);
     if (rc) return rc;

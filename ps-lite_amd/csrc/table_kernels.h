@@ -45,7 +45,7 @@ struct TableReq {
   float* req;             // push: request values (read); pull: response values (written)
   uint64_t total;         // floats in req
   uint64_t k;             // FIXED: floats per row
-  uint32_t reserved;
+  uint32_t cached;        // FIXED lookup: the first so many positions of cache_keys and ref belong together
   uint32_t ignore_new;    // pull half of a push+pull: rows created by the push half hold data
   uint32_t total_on_device;  // VARLEN pull without a host round trip: the floats to move are
                              // DevState::scan_total and `total` is the room in req
@@ -288,16 +288,15 @@ __global__ __launch_bounds__(kBlock) void k_scalar_flush(ReqBatch b) {
 // Row modes, step 1: key -> row reference.
 // ---------------------------------------------------------------------------------
 
-// The decision about a request that may repeat the cached one, taken by one thread after
-// every workgroup has compared its share (`different`: any of them found a difference). If
-// the decision is "different" (or the cache was not usable, or not even tried), the request
-// is going to refill the cache, so it becomes the cached request right here. Epochs start
+// The decision about a request that may repeat the cached one, written down by one thread after
+// every workgroup has compared its share (`same`: none found a difference and the cache was
+// usable). If it is not the same, the request is going to refill the cache, so it becomes the cached request right here. Epochs start
 // at 1.
-__device__ __forceinline__ void decide_same(DevState* st, const ReqTag& tag, bool different,
+__device__ __forceinline__ bool cache_usable(const DevState* st, const ReqTag& tag) {
+  return tag.try_cache && st->cache_epoch != 0ull && st->bad_epoch != st->cache_epoch;
+}
+__device__ __forceinline__ void decide_same(DevState* st, const ReqTag& tag, bool same,
                                             unsigned long long* outcome = nullptr) {
-  const bool usable =
-      tag.try_cache && st->cache_epoch != 0ull && st->bad_epoch != st->cache_epoch;
-  const bool same = !different && usable;
   if (tag.replay && !same) {
     // (an earlier replay of this very request may have left its number here)
     st->same_epoch = 0ull;
@@ -361,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch b) {
   __syncthreads();
   if (!s_last) return;
   if (threadIdx.x == 0)
-    decide_same(st, tag, (atomicExch(&st->req_flags, 0u) & kReqDiffer) != 0u, d.outcome);
+    decide_same(st, tag, (atomicExch(&st->req_flags, 0u) & kReqDiffer) == 0u && cache_usable(st, tag), d.outcome);
 }
 
 // The counter record of a request, written by the kernel that creates its keys once every
@@ -387,6 +386,12 @@ constexpr uint64_t kLookupLargeKeys = 1u << 20;
 // every thread claims slots for its keys, then the workgroup takes the rows of all
 // created keys from the arena with ONE atomic add and a workgroup-wide scan hands them
 // out in request order, so rows of neighbouring keys are neighbours in the arena.
+// A key's row never changes, so a reference that an earlier request has left at the key's position
+// (cache_keys holds the key it was left for) is the key's still: it is used as it is, and only the other
+// keys are looked up. A request that repeats the last one, or a push behind the pull of its keys, streams
+// through 24 B per key here. (It used to be compared as a whole by a launch of its own in front of this one:
+// 6.8 us of comparison and 4.5 us of a lookup that returned at once for 1M keys, and both for every small
+// request.)
 // FIXED: request `tag` repeats a key. Reported by the next wait; the request's row kernels
 // change no stored value.
 __device__ __forceinline__ void refuse_fixed(DevState* st, const ReqTag& tag) {
@@ -410,12 +415,8 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
   const ReqTag tag = d.tag;
   Snapshot* snap = d.snap;
   const uint64_t snap_seq = d.snap_seq;
-  if (cache_same(st, tag)) {  // the references of the cached request are this request's
-    if (snap && blockIdx.x == 0 && threadIdx.x < 64) publish_snapshot(st, snap, snap_seq);
-    return;
-  }
-  if (tag.replay) return;
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->cache_epoch = cache_keys ? tag.epoch : 0ull;
+  const uint64_t cached = d.cached;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->cache_epoch = tag.epoch;
   __shared__ unsigned long long red[kBlock / 64];
   __shared__ unsigned cred[kBlock / 64];
   __shared__ unsigned long long s_first;
@@ -425,6 +426,7 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
   for (uint64_t base = (uint64_t)blockIdx.x * kRound; base < n; base += (uint64_t)nblk * kRound) {
     uint64_t* p[kLookupItems];
     uint64_t seen[kLookupItems];
+    uint64_t was[kLookupItems];  // the reference that is there already, if it is this key's
     bool is_new[kLookupItems];
     unsigned mine = 0;
 #pragma unroll
@@ -433,14 +435,22 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
       p[j] = nullptr;
       is_new[j] = false;
       seen[j] = 0;
+      was[j] = kRefAbsent;
       if (i < n) {
+        // (all asked for at once: none of them waits for another)
         const uint64_t key = keys[i];
-        if (cache_keys) cache_keys[i] = key;
+        const uint64_t left = i > 0 ? keys[i - 1] : ~key;
+        const uint64_t cached_key = i < cached ? cache_keys[i] : ~key;
+        const uint64_t cached_ref = i < cached ? ref[i] : kRefAbsent;
         // keys are sorted and must be unique (kv_app.h:17): a key that equals its left neighbour
         // refuses the request, whether the key is new or has been in the table for long
-        if (i > 0 && keys[i - 1] == key) {
+        if (left == key) {
           refuse_fixed(st, tag);
+          cache_keys[i] = key;
+        } else if (cached_key == key && cached_ref != kRefAbsent) {
+          was[j] = cached_ref;
         } else {
+          cache_keys[i] = key;
           p[j] = find_or_insert(slots, mask, st, key, is_new[j], seen[j]);
         }
       }
@@ -460,6 +470,10 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
     for (int j = 0; j < kLookupItems; ++j) {
       const uint64_t i = base + (uint64_t)threadIdx.x * kLookupItems + j;
       if (i >= n) continue;
+      if (was[j] != kRefAbsent) {  // (created by the request that left it, but not by this one)
+        if (was[j] & kRefNew) ref[i] = was[j] & ~kRefNew;
+        continue;
+      }
       if (!p[j]) {
         ref[i] = kRefAbsent;
         continue;
@@ -478,13 +492,42 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
   publish_after_lookup(st, snap, snap_seq, nblk, &s_last);
 }
 
+// Four consecutive keys of a request with a word each, starting at index `at`: 128-bit loads where all four are
+// there (keys on any 8-byte, words on any 4-byte boundary), `fill` and zero keys past the end.
+typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
+template <typename W>
+struct FourKeys {
+  uint64_t k[4];
+  W v[4];
+};
+template <typename W>
+__device__ __forceinline__ void load_four(FourKeys<W>& f, const uint64_t* keys, const W* words, uint64_t at, uint64_t n,
+                                          W fill) {
+  static_assert(kScanItems == 4, "four keys per thread");
+  if (at + 4 <= n) {
+    const u64x2u a = *reinterpret_cast<const u64x2u*>(keys + at);
+    const u64x2u b = *reinterpret_cast<const u64x2u*>(keys + at + 2);
+    typedef W W4 __attribute__((ext_vector_type(4), aligned(sizeof(W))));
+    const W4 w = *reinterpret_cast<const W4*>(words + at);
+    f.k[0] = a.x, f.k[1] = a.y, f.k[2] = b.x, f.k[3] = b.y;
+    f.v[0] = w.x, f.v[1] = w.y, f.v[2] = w.z, f.v[3] = w.w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f.k[j] = at + j < n ? keys[at + j] : 0;
+      f.v[j] = at + j < n ? words[at + j] : fill;
+    }
+  }
+}
+
 // VARLEN push, first kernel: one pass over the request's keys and lens that
 //   - compares them with the cached request (when the host found the cache usable),
 //   - takes pass 1 of the lens scan (per-workgroup totals, flags),
 // and whose last workgroup decides whether the request repeats the cached one and scans the
 // totals. Always launched for a push, so the decision and the scan cost no launch of their
 // own.
-template <int kItems>
+// (Bound by its tail, not by its bytes: the tickets, and the scan of the totals, which a request that
+// repeats the cached one does without.)
 __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
@@ -492,8 +535,6 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
   const uint64_t* __restrict__ keys = d.keys;
   const int32_t* __restrict__ lens = d.lens;
   const uint64_t n = d.n;
-  const uint64_t* __restrict__ cache_keys = d.cache_keys;
-  const int32_t* __restrict__ cache_lens = d.cache_lens;
   unsigned long long* __restrict__ part = d.part;
   DevState* st = d.st;
   constexpr unsigned max_len = PSKV_MAX_VARLEN_ROW;
@@ -501,48 +542,47 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
   __shared__ unsigned long long red[kBlock / 64];
   __shared__ unsigned fred[kBlock / 64];
   __shared__ unsigned long long carry_s;
-  __shared__ unsigned s_last;
-  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kItems;
+  __shared__ unsigned s_last, s_same;
+  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kScanItems;
   // all loads first, then the arithmetic
-  int32_t l[kItems], cl[kItems];
-  uint64_t k[kItems], ck[kItems];
-#pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const bool in = base + j < n;
-    l[j] = in ? lens[base + j] : 0;
-    k[j] = in ? keys[base + j] : 0;
-    ck[j] = k[j];
-    cl[j] = l[j];
-    if (in && tag.try_cache) {
-      ck[j] = cache_keys[base + j];
-      cl[j] = cache_lens[base + j];
-    }
+  FourKeys<int32_t> mine, old;
+  load_four(mine, keys, lens, base, n, 0);
+  if (tag.try_cache) {
+    load_four(old, d.cache_keys, d.cache_lens, base, n, 0);
+  } else {
+    old = mine;
   }
   // the key in front of this thread's first one (its neighbour has asked for that line already)
   const uint64_t left = (base > 0 && base < n) ? keys[base - 1] : 0;
   unsigned long long s = 0;
   unsigned flags = 0;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    s += (unsigned long long)(long long)l[j];
-    flags |= (unsigned)l[j] & kReqMisaligned;
-    flags |= (l[j] < 0 || (unsigned)l[j] > max_len) ? kReqBadLen : 0u;
-    flags |= (k[j] != ck[j] || l[j] != cl[j]) ? kReqDiffer : 0u;
+  for (int j = 0; j < kScanItems; ++j) {
+    const int32_t l = mine.v[j];
+    s += (unsigned long long)(long long)l;
+    flags |= (unsigned)l & kReqMisaligned;
+    flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
+    flags |= (mine.k[j] != old.k[j] || l != old.v[j]) ? kReqDiffer : 0u;
     // keys are sorted and must be unique (kv_app.h:17): a key that equals its left neighbour
     // refuses the request before anything of it is applied
     const bool has_left = base + j < n && base + j > 0;
-    flags |= (has_left && k[j] == (j ? k[j - 1] : left)) ? kReqDuplicate : 0u;
+    flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
   }
   if (!scan_pass1_block(s, flags, part, st, nblk, red, fred, &s_last)) return;
-  flags = scan_pass1_last(part, st, nblk, tag.epoch, red, &carry_s);
-  if (threadIdx.x == 0) decide_same(st, tag, (flags & kReqDiffer) != 0u, d.outcome);
+  flags = scan_pass1_facts(st, &s_last);
+  if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && cache_usable(st, tag) ? 1u : 0u;
+  __syncthreads();
+  const bool same = s_same != 0u;
+  scan_pass1_last(part, st, nblk, tag.epoch, flags, same, red, &carry_s);
+  if (threadIdx.x == 0) decide_same(st, tag, same, d.outcome);
 }
 
 // VARLEN push, second kernel: pass 2 of the lens scan (request-side offsets and the tile
 // table) and, for the same keys, find-or-create: a created row gets ceil(len/4) 16-byte
 // units of the arena, so every row starts 16-byte aligned; a present row must have the
-// pushed length. A workgroup handles kBlock*kItems consecutive keys: every thread claims
-// slots for its keys, then the workgroup takes the rows of all created keys from the arena
+// pushed length. A workgroup handles chunks of kBlock*kItems consecutive keys (one each, or, when the
+// request is expected to repeat the cached one and the kernel to return at once, several): every thread
+// claims slots for its keys, then the workgroup takes the rows of all created keys from the arena
 // with ONE atomic add and a workgroup-wide scan hands them out in request order, so rows of
 // neighbouring keys are neighbours in the arena.
 constexpr unsigned kTileVar = 256;  // request-side floats per wavefront of the var-len row kernel: one quad per lane
@@ -593,80 +633,98 @@ __global__ __launch_bounds__(kBlock) void k_var_push_lookup(ReqBatch b) {
   __shared__ unsigned cred[kBlock / 64];
   __shared__ unsigned long long s_first;
   __shared__ unsigned s_last;
-  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kItems;
-  unsigned long long len[kItems];
+  unsigned created = 0;
+  constexpr uint64_t kChunk = (uint64_t)kBlock * kItems;
+  static_assert(kScanPart % kChunk == 0, "a part of the scan is a whole number of chunks");
+  for (uint64_t first_key = (uint64_t)blockIdx.x * kChunk; first_key < n; first_key += (uint64_t)nblk * kChunk) {
+    const uint64_t base = first_key + (uint64_t)threadIdx.x * kItems;
+    unsigned long long len[kItems];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) len[j] = base + j < n ? (unsigned long long)(uint32_t)lens[base + j] : 0ull;
-  scan_pass2_offsets<kItems>(len, base, n, part[blockIdx.x], off, tile_key, ntiles, tile, wsum);
+    for (int j = 0; j < kItems; ++j) len[j] = base + j < n ? (unsigned long long)(uint32_t)lens[base + j] : 0ull;
+    // where the chunk's first row starts in the request: the offset of its part of the scan, and the lens
+    // of that part in front of the chunk
+    const uint64_t part_key = first_key / kScanPart * kScanPart;
+    unsigned long long start = 0;
+    if (kChunk < kScanPart) {
+      for (uint64_t i = part_key + threadIdx.x; i < first_key; i += kBlock) start += (unsigned long long)(uint32_t)lens[i];
+      unsigned none = 0;
+      block_sum_or(start, none, red, cred);
+    }
+    start += part[first_key / kScanPart];
+    scan_pass2_offsets<kItems>(len, base, n, start, off, tile_key, ntiles, tile, wsum);
 
-  uint64_t* p[kItems];
-  uint64_t seen[kItems];
-  bool is_new[kItems];
-  unsigned long long units = 0;
-  unsigned mine = 0;
+    uint64_t* p[kItems];
+    uint64_t seen[kItems];
+    bool is_new[kItems];
+    unsigned long long units = 0;
+    unsigned mine = 0;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint64_t i = base + j;
-    p[j] = nullptr;
-    is_new[j] = false;
-    seen[j] = 0;
-    if (i < n) {
-      const uint64_t key = keys[i];
-      cache_keys[i] = key;
-      cache_lens[i] = (int32_t)len[j];
-      p[j] = find_or_insert(slots, mask, st, key, is_new[j], seen[j]);
-      if (p[j] && !is_new[j] && seen[j] == kPayloadUnset) {
-        atomicOr(&st->error, kDevErrDuplicate);  // the same key twice in this request
-        st->bad_epoch = tag.epoch;
-        p[j] = nullptr;
+    for (int j = 0; j < kItems; ++j) {
+      const uint64_t i = base + j;
+      p[j] = nullptr;
+      is_new[j] = false;
+      seen[j] = 0;
+      if (i < n) {
+        const uint64_t key = keys[i];
+        cache_keys[i] = key;
+        cache_lens[i] = (int32_t)len[j];
+        p[j] = find_or_insert(slots, mask, st, key, is_new[j], seen[j]);
+        if (p[j] && !is_new[j] && seen[j] == kPayloadUnset) {
+          atomicOr(&st->error, kDevErrDuplicate);  // the same key twice in this request
+          st->bad_epoch = tag.epoch;
+          p[j] = nullptr;
+        }
+      }
+      if (p[j] && is_new[j]) {
+        units += (len[j] + 3) >> 2;
+        ++mine;
       }
     }
-    if (p[j] && is_new[j]) {
-      units += (len[j] + 3) >> 2;
-      ++mine;
+    unsigned long long total;
+    unsigned long long at = block_excl_scan_u64(units, red, total);
+    if (threadIdx.x == 0 && total) {
+      // kArenaPadUnits - 1 units of slack let the chunk's rows start at an arena address that
+      // is congruent, modulo 128 bytes, to the request-side offset of the chunk's first key.
+      // When all its keys are new (a first push) the rows then mirror the request 128-byte line
+      // for 128-byte line, and the row kernels' arena accesses are as aligned as their
+      // request-side ones (misaligned ones cost about 5 % of their bandwidth).
+      const unsigned long long first = atomicAdd(&st->arena_top, total + (kArenaPadUnits - 1));
+      const unsigned long long want = (start >> 2) & (kArenaPadUnits - 1);
+      s_first = first + ((want - first) & (kArenaPadUnits - 1));
     }
-  }
-  unsigned long long total;
-  unsigned long long at = block_excl_scan_u64(units, red, total);
-  if (threadIdx.x == 0 && total) {
-    // kArenaPadUnits - 1 units of slack let the workgroup's rows start at an arena address that
-    // is congruent, modulo 128 bytes, to the request-side offset of the workgroup's first key.
-    // When all its keys are new (a first push) the rows then mirror the request 128-byte line
-    // for 128-byte line, and the row kernels' arena accesses are as aligned as their
-    // request-side ones (misaligned ones cost about 5 % of their bandwidth).
-    const unsigned long long first = atomicAdd(&st->arena_top, total + (kArenaPadUnits - 1));
-    const unsigned long long want = (part[blockIdx.x] >> 2) & (kArenaPadUnits - 1);
-    s_first = first + ((want - first) & (kArenaPadUnits - 1));
-  }
-  __syncthreads();
-  at += total ? s_first : 0ull;
+    __syncthreads();
+    at += total ? s_first : 0ull;
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint64_t i = base + j;
-    if (i >= n) continue;
-    if (!p[j]) {
-      ref[i] = kRefAbsent;
-      continue;
+    for (int j = 0; j < kItems; ++j) {
+      const uint64_t i = base + j;
+      if (i >= n) continue;
+      if (!p[j]) {
+        ref[i] = kRefAbsent;
+        continue;
+      }
+      uint64_t payload = seen[j];
+      if (is_new[j]) {
+        payload = ((uint64_t)at << kLenBits) | len[j];
+        at += (len[j] + 3) >> 2;
+        *p[j] = payload;
+      } else if ((payload & kLenMask) != len[j]) {
+        raise_error(st, kDevErrLenChanged, tag.epoch);
+      }
+      ref[i] = payload | (is_new[j] ? kRefNew : 0ull);
     }
-    uint64_t payload = seen[j];
-    if (is_new[j]) {
-      payload = ((uint64_t)at << kLenBits) | len[j];
-      at += (len[j] + 3) >> 2;
-      *p[j] = payload;
-    } else if ((payload & kLenMask) != len[j]) {
-      raise_error(st, kDevErrLenChanged, tag.epoch);
-    }
-    ref[i] = payload | (is_new[j] ? kRefNew : 0ull);
+    created += mine;
+    __syncthreads();  // the shared words are reused by the next chunk
   }
-  block_count_add(st, mine, cred);
+  block_count_add(st, created, cred);
   publish_after_lookup(st, snap, snap_seq, nblk, &s_last);
 }
 
 // VARLEN pull, first kernel: the stored length of every key (an absent key answers length 0
-// and is not created) together with pass 1 of the scan over those lengths. With the keys of
-// the cached push the answer is known without a single probe: every key is present with the
-// cached length, and the offsets of that push are the offsets of this response.
-template <int kItems>
+// and is not created) together with pass 1 of the scan over those lengths. A key that sits where the
+// cached push had it is present with the cached length, and its reference is in the workspace: only the
+// others are looked up. When every key does, the offsets of that push are the offsets of this response
+// as well, and the scan of the totals falls away. (The comparison was a launch of its own in front of this
+// one; a recorded request, which must not answer anything before the decision is there, still has it.)
 __global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
@@ -678,46 +736,100 @@ __global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch b) {
   const uint64_t n = d.n;
   uint64_t* __restrict__ ref = d.ref;
   int32_t* __restrict__ out_lens = d.out_lens;
-  const int32_t* __restrict__ cache_lens = d.cache_lens;
   unsigned long long* __restrict__ part = d.part;
   const ReqTag tag = d.tag;
   __shared__ unsigned long long red[kBlock / 64];
   __shared__ unsigned fred[kBlock / 64];
   __shared__ unsigned long long carry_s;
-  __shared__ unsigned s_last;
-  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kItems;
-  if (cache_same(st, tag)) {
+  __shared__ unsigned s_last, s_same;
+  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kScanItems;
+  if (tag.replay) {
+    if (!cache_same(st, tag)) return;
 #pragma unroll
-    for (int j = 0; j < kItems; ++j)
-      if (base + j < n) out_lens[base + j] = cache_lens[base + j];
+    for (int j = 0; j < kScanItems; ++j)
+      if (base + j < n) out_lens[base + j] = d.cache_lens[base + j];
     return;
   }
-  if (tag.replay) return;
-  // this pull rewrites the references and offsets in the workspace: the cached push is gone
-  if (blockIdx.x == 0 && threadIdx.x == 0) st->bad_epoch = st->cache_epoch;
-  unsigned long long s = 0;
-  unsigned bits = 0;
+  // (the last workgroup alone changes what this reads, after every workgroup has read it)
+  const bool usable = cache_usable(st, tag);
+  FourKeys<int32_t> old;
+  uint64_t key[kScanItems];
+  bool known[kScanItems], hit[kScanItems];
+  uint64_t payload[kScanItems];
+  int32_t l[kScanItems];
+  if (base + kScanItems <= n) {
+    const u64x2u a = *reinterpret_cast<const u64x2u*>(keys + base);
+    const u64x2u c = *reinterpret_cast<const u64x2u*>(keys + base + 2);
+    key[0] = a.x, key[1] = a.y, key[2] = c.x, key[3] = c.y;
+  } else {
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint64_t i = base + j;
-    if (i < n) {
-      uint64_t payload;
-      const bool hit = find_only(slots, mask, st, keys[i], payload);
-      const uint32_t l = hit ? (uint32_t)(payload & kLenMask) : 0u;
-      ref[i] = hit ? payload : kRefAbsent;
-      out_lens[i] = (int32_t)l;
-      s += l;
-      bits |= l & 3u;
+    for (int j = 0; j < kScanItems; ++j) key[j] = base + j < n ? keys[base + j] : 0;
+  }
+  if (usable) load_four(old, d.cache_keys, d.cache_lens, base, n, 0);
+  bool all = true;
+#pragma unroll
+  for (int j = 0; j < kScanItems; ++j) {
+    known[j] = base + j >= n || (usable && old.k[j] == key[j]);
+    l[j] = known[j] && base + j < n ? old.v[j] : 0;
+    all = all && known[j];
+  }
+  unsigned bits = 0;
+  if (!all) {
+    bits = kReqDiffer;
+    // the home slots of the thread's keys together: a probe is one line from memory
+    u64x2 home[kScanItems];
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j)
+      if (!known[j]) home[j] = load_slot(&slots[home_slot(key[j], mask)]);
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j) {
+      if (known[j]) continue;
+      if (home[j].x == key[j] && key[j] != kEmptyKey) {
+        hit[j] = true;
+        payload[j] = home[j].y;
+      } else {
+        hit[j] = find_only(slots, mask, st, key[j], payload[j]);
+      }
+      l[j] = hit[j] ? (int32_t)(payload[j] & kLenMask) : 0;
+      ref[base + j] = hit[j] ? payload[j] : kRefAbsent;
     }
   }
+  unsigned long long s = 0;
+#pragma unroll
+  for (int j = 0; j < kScanItems; ++j) {
+    s += (uint32_t)l[j];
+    bits |= (unsigned)l[j] & kReqMisaligned;
+  }
+  if (base + kScanItems <= n) {
+    typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    i32x4u w;
+    w.x = l[0], w.y = l[1], w.z = l[2], w.w = l[3];
+    *reinterpret_cast<i32x4u*>(out_lens + base) = w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < kScanItems; ++j)
+      if (base + j < n) out_lens[base + j] = l[j];
+  }
   if (!scan_pass1_block(s, bits, part, st, nblk, red, fred, &s_last)) return;
-  scan_pass1_last(part, st, nblk, tag.epoch, red, &carry_s);
+  const unsigned flags = scan_pass1_facts(st, &s_last);
+  if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && usable ? 1u : 0u;
+  __syncthreads();
+  const bool same = s_same != 0u;
+  scan_pass1_last(part, st, nblk, tag.epoch, flags, same, red, &carry_s);
+  if (threadIdx.x == 0) {
+    if (same) {
+      st->same_epoch = tag.epoch;
+    } else {
+      // this pull has rewritten references in the workspace, and its offsets will: the cached push is gone
+      st->bad_epoch = st->cache_epoch;
+    }
+    if (d.outcome && tag.try_cache) *d.outcome = (tag.epoch << 1) | (same ? 1ull : 0ull);
+  }
 }
 
 // VARLEN pull, second kernel: pass 2 of the scan over the answered lengths: the request-side
 // offsets of the response and its tile table. `ntiles_cap` is the room in the table; the
 // tiles in use follow from the scanned total.
-template <int kItems>
 __global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch b) {
   const TableReq& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;
@@ -734,11 +846,14 @@ __global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch b) {
   __shared__ unsigned long long wsum[kBlock / 64];
   uint64_t ntiles = (st->scan_total + tile - 1) / tile;
   if (ntiles > ntiles_cap) ntiles = ntiles_cap;
-  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kItems;
-  unsigned long long len[kItems];
+  for (uint64_t first = (uint64_t)blockIdx.x * kScanPart; first < n; first += (uint64_t)d.nblk * kScanPart) {
+    const uint64_t base = first + (uint64_t)threadIdx.x * kScanItems;
+    unsigned long long len[kScanItems];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) len[j] = base + j < n ? (unsigned long long)(uint32_t)lens[base + j] : 0ull;
-  scan_pass2_offsets<kItems>(len, base, n, part[blockIdx.x], off, tile_key, ntiles, tile, wsum);
+    for (int j = 0; j < kScanItems; ++j) len[j] = base + j < n ? (unsigned long long)(uint32_t)lens[base + j] : 0ull;
+    scan_pass2_offsets<kScanItems>(len, base, n, part[first / kScanPart], off, tile_key, ntiles, tile, wsum);
+    __syncthreads();  // wsum is reused by the next part
+  }
 }
 
 // ---------------------------------------------------------------------------------

@@ -89,3 +89,41 @@ def test_host_resident_rows_in_pieces(capi, orc, dev, n, k):
         out = np.zeros(n * k, np.float32)
         t.pull(keys, out)
         assert_bits_equal(out, o.pull(keys)[0])
+
+
+@pytest.mark.parametrize("mode", ["fixed", "varlen"])
+@pytest.mark.parametrize("n", [1, 255, 257, 1023, 1025, 140_001, (1 << 20) + 3])
+def test_requests_that_partly_repeat(capi, orc, dev, mode, n):
+    """The same keys several times (the kernels then expect them), then a few or all of them others, and a
+    shorter request in between: references left at a position are used exactly where their key still is."""
+    announce("partly repeat", mode, n)
+    import torch
+    rng = np.random.default_rng(n)
+    m, k = (capi.MODE_FIXED, 5) if mode == "fixed" else (capi.MODE_VARLEN, 0)
+    t, o = capi.Table(m, row_len=k), orc.Store(m, k)
+    keys = unique_keys(rng, n + n // 2 + 2)
+    all_lens = rng.integers(1, 6, keys.size).astype(np.int32)
+    base = np.sort(rng.choice(keys.size, n, replace=False))
+    near = base.copy()
+    spare = np.setdiff1d(np.arange(keys.size), base)
+    near[rng.integers(0, n, 3)] = spare[0]
+    near = np.unique(near)
+    other = np.sort(rng.choice(keys.size, n, replace=False))
+    for pick in (base, base, base, near, base, base[: n // 2 + 1], base, base, other, base):
+        some, lens = keys[pick], all_lens[pick]
+        vals = rng.standard_normal(int(lens.sum()) if mode == "varlen" else some.size * k).astype(np.float32)
+        args = (to_dev(lens, dev),) if mode == "varlen" else ()
+        t.push(to_dev(some, dev), to_dev(vals, dev), *args)
+        o.push(some, vals, lens if mode == "varlen" else None)
+        want, want_lens = o.pull(some)
+        out = torch.empty(want.size, dtype=torch.float32, device=dev)
+        if mode == "varlen":
+            out_lens = torch.empty(some.size, dtype=torch.int32, device=dev)
+            t.pull(to_dev(some, dev), out, out_lens)
+            torch.cuda.synchronize()
+            assert np.array_equal(out_lens.cpu().numpy(), want_lens)
+        else:
+            t.pull(to_dev(some, dev), out)
+            torch.cuda.synchronize()
+        assert_bits_equal(out.cpu().numpy(), want)
+    assert_bits_equal(t.dump()[2], o.dump()[2])
