@@ -14,6 +14,7 @@
 #include <new>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -60,7 +61,9 @@ constexpr uint64_t kSpareMaxBytes = 16384ull << 20;  // no array larger than thi
 // Host-resident requests up to this size (per direction) skip the copy commands: the kernels
 // read the request from, and write the response to, pinned host memory mapped into the GPU.
 constexpr size_t kSmallBytes = 1024u << 10;
-constexpr int kSmallParts = 8;  // (128 KiB each: a SCALAR push of up to 10,000 keys)
+// Requests up to a quarter of that take their room in turn, so that several can be in flight (small_room).
+constexpr int kSmallParts = 4;
+constexpr size_t kSmallPart = kSmallBytes / kSmallParts;
 // Host-resident buffers from this size on travel piece by piece through the ring of pinned memory
 // (stager.h), copying, transfer and kernels overlapping; smaller ones take one copy command.
 constexpr size_t kPipeBytes = 4u << 20;
@@ -85,6 +88,7 @@ struct StateView {
   uint64_t scan_total;
   uint64_t same_epoch;
   unsigned error, req_error, special_present, pad;
+  unsigned long long seq;  // written last: the number of the reading (StateBatch::seq)
 };
 
 // A new table's device state: all zero, the side slot's payload unset. One workgroup.
@@ -99,6 +103,7 @@ __global__ void k_init_state(DevState* st) {
 struct StateBatch {
   const DevState* st[kMaxBatch];
   StateView* out[kMaxBatch];
+  unsigned long long seq;
 };
 __global__ void k_read_state(StateBatch sb) {
   const DevState* st = sb.st[blockIdx.x];
@@ -114,6 +119,7 @@ __global__ void k_read_state(StateBatch sb) {
   out->error = st->error;
   out->req_error = st->req_error;
   out->special_present = st->special_present;
+  __hip_atomic_store(&out->seq, sb.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The parts of a table that have one size whatever the table holds: device state, the pinned words and
@@ -122,7 +128,7 @@ __global__ void k_read_state(StateBatch sb) {
 // the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim.
 struct Shell {
   DevState* st = nullptr;
-  char* pinned = nullptr;  // StateView, Snapshot, outcome word (256 bytes each), small_in, small_out
+  char* pinned = nullptr;  // StateView, Snapshot, outcome word, done word (256 bytes each), small_in, small_out
   hipEvent_t done[kSmallParts] = {nullptr};
 };
 constexpr size_t kShellsKept = 32;
@@ -251,12 +257,17 @@ struct pskv_table {
   char* small_in = nullptr;   // pinned, kSmallBytes: small host-resident requests, read in place
   char* small_out = nullptr;  // pinned, kSmallBytes: their responses, written in place
   // A small host-resident SCALAR push returns once its kernel is queued: nothing comes back from
-  // it. Such pushes take the kSmallParts parts of small_in in turn (when they fit one), so that
-  // several can be in flight; a request that writes a part waits for the event its last user left.
+  // it. Requests of up to kSmallPart bytes take their room in small_in one behind the other, so that
+  // as many pushes as fit can be in flight. An event is left when a part has been used up and
+  // waited for when the part comes round again: one event for 21 pushes of 1,000 keys (an event behind
+  // every push cost the calling thread 3.6 us of its 11.5).
   hipEvent_t small_done[kSmallParts] = {nullptr};
-  bool small_pending[kSmallParts] = {false};
-  int small_next = 0;      // the part the next such push takes
-  int small_newest = -1;   // the part whose event was recorded last (everything before it is done when it is)
+  bool small_pending[kSmallParts] = {false};  // the part's event has been recorded and not been waited for
+  int small_part = 0;             // the part that is being used up,
+  size_t small_at = 0;            // and the bytes of it that have been given away
+  bool small_in_flight = false;   // requests that nobody has waited for may still be reading small_in
+  unsigned long long* done = nullptr;  // pinned: done_seq of the newest request that had to tell its end
+  unsigned long long done_seq = 0;
   GrowBuf stage;      // device copies of host-resident request buffers
   GrowBuf stage_out;  // device-side response of a host-resident or undersized pull
   bool no_growth = false;  // set while dumping: every key is known to be present
@@ -313,12 +324,11 @@ namespace {
 
 // ---- profiling -------------------------------------------------------------------
 // Launches `kernel` on the table's stream. While profiling is on, the launch carries
-// a start and a stop event of its own (hipExtLaunchKernelGGL), which take the
+// a start and a stop event of its own (hipExtLaunchKernel), which take the
 // begin/end timestamps of that very dispatch: the same clock a profiler reads,
 // without the idle time that events recorded around a launch would add.
-template <typename... KArgs, typename... Args>
-void launch_lds(pskv_table* t, int prof_kernel, void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds,
-                Args... args) {
+hipError_t launch_args(pskv_table* t, int prof_kernel, const void* kernel, dim3 grid, dim3 block, size_t lds,
+                       void** args) {
   if (t->prof && prof_kernel >= 0 && !t->capturing) {
     EventPair ev;
     bool have = false;
@@ -334,18 +344,24 @@ void launch_lds(pskv_table* t, int prof_kernel, void (*kernel)(KArgs...), dim3 g
       }
     }
     if (have) {
-      hipExtLaunchKernelGGL(kernel, grid, block, lds, t->stream, ev.a, ev.b, 0, static_cast<KArgs>(args)...);
       t->pending[prof_kernel].push_back(ev);
-      return;
+      return hipExtLaunchKernel(kernel, grid, block, args, lds, t->stream, ev.a, ev.b, 0);
     }
   }
-  hipLaunchKernelGGL(kernel, grid, block, lds, t->stream, static_cast<KArgs>(args)...);
+  return hipLaunchKernel(kernel, grid, block, args, lds, t->stream);
 }
 
 template <typename... KArgs, typename... Args>
-void launch(pskv_table* t, int prof_kernel, void (*kernel)(KArgs...), dim3 grid, dim3 block,
-            Args... args) {
-  launch_lds(t, prof_kernel, kernel, grid, block, 0, args...);
+int launch(pskv_table* t, int prof_kernel, void (*kernel)(KArgs...), dim3 grid, dim3 block, size_t lds,
+           Args... given) {
+  std::tuple<KArgs...> as_declared(static_cast<KArgs>(given)...);
+  return std::apply(
+      [&](KArgs&... a) {
+        void* args[] = {static_cast<void*>(&a)...};
+        PSKV_HIP(launch_args(t, prof_kernel, reinterpret_cast<const void*>(kernel), grid, block, lds, args));
+        return PSKV_OK;
+      },
+      as_declared);
 }
 
 int prof_collect(pskv_table* t) {
@@ -391,17 +407,38 @@ void adopt_state(pskv_table* t) {
   t->pend_keys = t->pend_units = 0;
 }
 
-int read_state(pskv_table* t) {
+// Watches a word of pinned host memory for `want` for up to about 200 us; false when it did not show up
+// in that time (the caller then waits for the stream as usual). A stream wait costs about 5 us more.
+bool seen_in_time(const unsigned long long* word, unsigned long long want) {
+  const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+  for (;;) {
+    for (int spin = 0; spin < 256; ++spin)
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return true;
+    if (std::chrono::steady_clock::now() > give_up) return false;
+  }
+}
+
+// Reads the device state of up to kMaxBatch tables on one stream, with one launch and one wait. `watch`: what the
+// caller wants to see afterwards lies in pinned memory (the state itself, answers that kernels have written
+// there): it is enough that this kernel, the last one on the stream, has run.
+std::atomic<unsigned long long> g_readings{0};
+int read_states(pskv_table* const* tables, size_t count, bool watch) {
   StateBatch sb;
-  std::memset(&sb, 0, sizeof(sb));
-  sb.st[0] = t->st;
-  sb.out[0] = t->st_host;
-  k_read_state<<<dim3(1), dim3(64), 0, t->stream>>>(sb);
+  sb.seq = ++g_readings;
+  for (size_t i = 0; i < count; ++i) {
+    sb.st[i] = tables[i]->st;
+    sb.out[i] = tables[i]->st_host;
+  }
+  k_read_state<<<dim3((unsigned)count), dim3(64), 0, tables[0]->stream>>>(sb);
   PSKV_HIP(hipGetLastError());
-  PSKV_HIP(hipStreamSynchronize(t->stream));
-  adopt_state(t);
+  bool seen = watch;
+  for (size_t i = 0; seen && i < count; ++i) seen = seen_in_time(&tables[i]->st_host->seq, sb.seq);
+  if (!seen) PSKV_HIP(hipStreamSynchronize(tables[0]->stream));
+  for (size_t i = 0; i < count; ++i) adopt_state(tables[i]);
   return PSKV_OK;
 }
+
+int read_state(pskv_table* t, bool watch = false) { return read_states(&t, 1, watch); }
 
 // Turns device error bits into a status, clearing them on the device.
 int report_device_errors(pskv_table* t) {
@@ -487,7 +524,7 @@ void adopt_snapshot(pskv_table* t) {
 // anything but the kernels of a request that repeats the cached keys looks at the slots.
 int flush_scalar_cache(pskv_table* t) {
   if (!t->sc_dirty) return PSKV_OK;
-  ReqBatch rb;
+  ReqBatch<1> rb;
   std::memset(&rb, 0, sizeof(rb));
   TableReq& d = rb.t[0];
   d.slots = t->slots;
@@ -498,7 +535,7 @@ int flush_scalar_cache(pskv_table* t) {
   d.tile_key = static_cast<uint32_t*>(t->sc_slots.ptr);
   d.cache_mode = kFlushAlways;
   d.nblk = grid_for(t->cache_n, kBlock, kFlushGrid);
-  hipLaunchKernelGGL(k_scalar_flush, dim3(d.nblk, 1), dim3(kBlock), 0, t->stream, rb);
+  hipLaunchKernelGGL(k_scalar_flush<1>, dim3(d.nblk, 1), dim3(kBlock), 0, t->stream, rb);
   PSKV_HIP(hipGetLastError());
   t->sc_dirty = false;
   return PSKV_OK;
@@ -565,18 +602,19 @@ int grow_slots(pskv_table* t, uint64_t keys_needed) {
     // two streaming passes: the new array is written whole, slot by slot, from LDS
     const unsigned nblk = (unsigned)(t->cap / kRegrowOld);
     const size_t lds = (size_t)kRegrowOld * factor * 2 * sizeof(unsigned long long);
-    launch_lds(t, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk), dim3(kBlock), lds, t->slots, fresh, t->cap - 1,
-               want - 1, (unsigned)factor);
-    PSKV_HIP(hipGetLastError());
-    launch(t, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock), dim3(kBlock),
-           (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
+    rc = launch(t, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk), dim3(kBlock), lds, t->slots, fresh, t->cap - 1,
+                want - 1, (unsigned)factor);
+    if (rc) return rc;
+    rc = launch(t, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock), dim3(kBlock), 0,
+                (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
+    if (rc) return rc;
   } else {
     // (a small table that a large request makes much larger: fill and scatter)
     PSKV_HIP(hipMemsetAsync(fresh, 0xFF, want * sizeof(Slot), t->stream));
-    launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(t->cap, kBlock, kMaxGrid)), dim3(kBlock),
-           (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
+    rc = launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(t->cap, kBlock, kMaxGrid)), dim3(kBlock), 0,
+                (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
+    if (rc) return rc;
   }
-  PSKV_HIP(hipGetLastError());
   const auto r0 = std::chrono::steady_clock::now();
   rc = array_release(t->slots, t->stream);
   t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
@@ -774,6 +812,9 @@ struct Request {
   // that have arrived. pipe_out: the gather kernel is not launched with the request; the caller
   // launches it piece by piece in step with the transfer of the response (gather_deferred says
   // that it is still owed, gather_varlen which kernel it is).
+  bool pinned;               // keys, vals and lens lie in pinned host memory
+  unsigned long long* done;  // SCALAR, pinned: the word that takes done_seq when the request is done, or null
+  unsigned long long done_seq;
   const float* vals_host;
   bool pipe_in, pipe_out, gather_deferred, gather_varlen;
   // pskv_replay_record: kReplayPrime = the run that brings the tables into the state a repeat of the
@@ -809,11 +850,24 @@ pskv_table* lead_of(Batch& bt) {
   return bt[0].t;
 }
 
-// A launch as pskv_replay_record keeps it: everything hipLaunchKernelGGL needs to make it again.
+// One kernel of the store in its three sizes (ReqBatch).
+struct KernelSet {
+  const void* one;
+  const void* four;
+  const void* most;
+};
+#define PSKV_KSET(name)                                                                                        \
+  (KernelSet{reinterpret_cast<const void*>(&name<1>), reinterpret_cast<const void*>(&name<4>),                   \
+             reinterpret_cast<const void*>(&name<kMaxBatch>)})
+#define PSKV_KSET_OF(name, ...)                                                                                \
+  (KernelSet{reinterpret_cast<const void*>(&name<__VA_ARGS__, 1>), reinterpret_cast<const void*>(&name<__VA_ARGS__, 4>), \
+             reinterpret_cast<const void*>(&name<__VA_ARGS__, kMaxBatch>)})
+
+// A launch as pskv_replay_record keeps it: everything it takes to make it again.
 struct SavedLaunch {
-  void (*kernel)(ReqBatch);
+  const void* kernel;
   dim3 grid;
-  ReqBatch rb;
+  ReqBatch<kMaxBatch> rb;  // (the kernel takes as much of it as its size says)
 };
 // Where launch_batch leaves a copy of its launches while a request is being recorded (the thread
 // that records is the thread that launches).
@@ -822,37 +876,30 @@ thread_local std::vector<SavedLaunch>* g_recording = nullptr;
 // One launch for the whole batch: blockIdx.y selects the table, `nblk_of` says how many
 // workgroups serve each (0: none, the table sits this step out).
 template <typename F>
-int launch_batch(Batch& bt, int prof_kernel, void (*kernel)(ReqBatch), F nblk_of) {
-  ReqBatch rb;
-  std::memset(&rb, 0, sizeof(rb));
+int launch_batch(Batch& bt, int prof_kernel, const KernelSet& kernels, F nblk_of) {
+  SavedLaunch l;
+  const size_t room = bt.size() <= 1 ? 1 : bt.size() <= 4 ? 4 : kMaxBatch;
+  l.kernel = room == 1 ? kernels.one : room == 4 ? kernels.four : kernels.most;
   uint64_t gx = 0;
   for (size_t i = 0; i < bt.size(); ++i) {
     const uint64_t nb = nblk_of(bt[i]);
     if (nb > 0x7fffffffull) return set_error(PSKV_EINVAL, "request too large");
-    rb.t[i] = bt[i].d;
-    rb.t[i].nblk = (uint32_t)nb;
+    l.rb.t[i] = bt[i].d;
+    l.rb.t[i].nblk = (uint32_t)nb;
     gx = std::max(gx, nb);
   }
   if (!gx) return PSKV_OK;
-  launch(lead_of(bt), prof_kernel, kernel, dim3((unsigned)gx, (unsigned)bt.size()), dim3(kBlock), rb);
-  PSKV_HIP(hipGetLastError());
-  if (g_recording) g_recording->push_back(SavedLaunch{kernel, dim3((unsigned)gx, (unsigned)bt.size()), rb});
+  l.grid = dim3((unsigned)gx, (unsigned)bt.size());
+  void* args[] = {&l.rb};
+  PSKV_HIP(launch_args(lead_of(bt), prof_kernel, l.kernel, l.grid, dim3(kBlock), 0, args));
+  if (g_recording) g_recording->push_back(l);
   return PSKV_OK;
 }
 
-// The device state of every table of the batch with one launch and one wait.
-int read_state_batch(Batch& bt) {
-  StateBatch sb;
-  std::memset(&sb, 0, sizeof(sb));
-  for (size_t i = 0; i < bt.size(); ++i) {
-    sb.st[i] = bt[i].t->st;
-    sb.out[i] = bt[i].t->st_host;
-  }
-  k_read_state<<<dim3((unsigned)bt.size()), dim3(64), 0, bt[0].t->stream>>>(sb);
-  PSKV_HIP(hipGetLastError());
-  PSKV_HIP(hipStreamSynchronize(bt[0].t->stream));
-  for (Item& it : bt) adopt_state(it.t);
-  return PSKV_OK;
+int read_state_batch(Batch& bt, bool watch) {
+  pskv_table* tables[kMaxBatch];
+  for (size_t i = 0; i < bt.size(); ++i) tables[i] = bt[i].t;
+  return read_states(tables, bt.size(), watch);
 }
 
 // What the device has reported about the comparisons of earlier requests with the cached keys
@@ -999,7 +1046,10 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       rc = grow(t, &t->sc_slots, r.n * sizeof(uint32_t));
       if (rc) return rc;
     }
-    if (use[i] != kScPlain) {
+    if (use[i] == kScPlain) {
+      d.outcome = r.done;
+      d.tag.epoch = r.done_seq;
+    } else {
       it.tag = next_tag(t, r);
       t->sc_kind[it.tag.epoch % pskv_table::kScKinds] = r.push ? 0 : 1;
       d.tag = it.tag;
@@ -1030,7 +1080,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   if (!n_largest) return PSKV_OK;
   int rc;
   if (any_cache) {
-    rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, k_same_keys, [](const Item& it) {
+    rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
       return (it.d.cache_mode == kCacheOn && it.tag.try_cache)
                  ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems) : 0ull;
     });
@@ -1038,7 +1088,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     // slots that lag behind the cache are written back once the device knows that the request
     // does NOT repeat the cached keys (cache_mode reads as kFlushUnlessSame in that kernel)
     static_assert(kFlushUnlessSame == kCacheOn, "one descriptor serves both kernels");
-    rc = launch_batch(bt, -1, k_scalar_flush, [](const Item& it) {
+    rc = launch_batch(bt, -1, PSKV_KSET(k_scalar_flush), [](const Item& it) {
       return it.flush_unless_same ? (uint64_t)grid_for(it.r.n, kBlock, kFlushGrid) : 0ull;
     });
     if (rc) return rc;
@@ -1052,16 +1102,23 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     const bool four = (it.d.cache_mode == kCacheOn && it.tag.try_cache) || it.d.cache_mode == kCachePerKey;
     return grid_for(it.d.n, four ? kBlock * 4 : kBlock, kMaxGrid);
   };
+  const bool pinned = bt[0].r.pinned;
+  if (any_cache) {
+    for (Item& it : bt) it.r.done = nullptr;  // (the word of such a launch says how the comparison went)
+  }
   if (push && pull) {
-    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, k_scalar<true, true, true>, nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, k_scalar<true, true, false>, nblk);
+    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, true, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, true), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, false), nblk);
   } else if (push) {
-    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, k_scalar<true, false, true>, nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, k_scalar<true, false, false>, nblk);
+    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, true, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, true), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, false), nblk);
   } else {
     const int kind = bt[0].d.cache_mode == kCachePerKey ? PSKV_KERNEL_PULL_PER_KEY : PSKV_KERNEL_PULL_SCALAR;
-    rc = any_cache ? launch_batch(bt, kind, k_scalar<false, true, true>, nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, k_scalar<false, true, false>, nblk);
+    rc = any_cache ? launch_batch(bt, kind, PSKV_KSET_OF(k_scalar, false, true, true, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, true), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, false), nblk);
   }
   if (rc) return rc;
   for (size_t i = 0; i < bt.size(); ++i) {
@@ -1104,11 +1161,11 @@ int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
   auto nblk = [&](const Item&) { return blocks; };
   int rc;
   if (op == kOpAcc) {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, true>, nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, false>, nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false), nblk);
   } else {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, k_rows<kOpGather, VARLEN, true>, nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, k_rows<kOpGather, VARLEN, false>, nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false), nblk);
   }
   it.d.tile_base = 0;
   return rc;
@@ -1146,11 +1203,11 @@ int launch_rows(Batch& bt, int op) {
   };
   const bool stream = floats >= kStreamFloats;
   if (op == kOpAcc) {
-    if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, true>, nblk);
-    return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, k_rows<kOpAcc, VARLEN, false>, nblk);
+    if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true), nblk);
+    return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false), nblk);
   }
-  if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, k_rows<kOpGather, VARLEN, true>, nblk);
-  return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, k_rows<kOpGather, VARLEN, false>, nblk);
+  if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true), nblk);
+  return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false), nblk);
 }
 
 // Starts a row-mode request on every table with keys: numbers it and (`compare`: a recorded one), where the
@@ -1169,7 +1226,7 @@ int begin_row_request(Batch& bt, bool compare) {
     it.d.outcome = it.t->outcome;
   }
   if (!compare) return PSKV_OK;
-  return launch_batch(bt, PSKV_KERNEL_SAME_KEYS, k_same_keys, [](const Item& it) {
+  return launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
     return (it.r.n && it.tag.try_cache) ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems)
                                         : 0ull;
   });
@@ -1213,11 +1270,11 @@ int run_fixed(Batch& bt, bool push, bool pull) {
   if (bt[0].r.replay == kReplayCapture) {
     // a recorded repeat is compared as a whole and uses the references that are there: no lookup
   } else if (n_largest >= kLookupLargeKeys) {
-    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, k_lookup_fixed<kLookupItemsLarge>, [](const Item& it) {
+    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET_OF(k_lookup_fixed, kLookupItemsLarge), [](const Item& it) {
       return it.r.n ? (uint64_t)grid_for(it.r.n, kBlock * kLookupItemsLarge, kMaxGrid) : 0ull;
     });
   } else {
-    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, k_lookup_fixed<1>, [](const Item& it) {
+    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET_OF(k_lookup_fixed, 1), [](const Item& it) {
       return it.r.n ? (uint64_t)grid_for(it.r.n, kBlock, kMaxGrid) : 0ull;
     });
   }
@@ -1287,7 +1344,7 @@ int make_tile_tables(Batch& bt) {
     it.d.ntiles = ntiles_cap;
   }
   if (bt[0].r.replay == kReplayCapture) return PSKV_OK;  // (a recorded repeat: the tables that are there)
-  return launch_batch(bt, -1, k_var_offsets, [&](const Item& it) {
+  return launch_batch(bt, -1, PSKV_KSET(k_var_offsets), [&](const Item& it) {
     return (it.r.n && it.d.total) ? may_return_at_once(it, false, it.nparts, bt.size()) : 0ull;
   });
 }
@@ -1371,11 +1428,11 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
     }
-    int rc = launch_batch(bt, -1, k_var_push_begin, [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+    int rc = launch_batch(bt, -1, PSKV_KSET(k_var_push_begin), [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
     if (rc) return rc;
     // (a recorded repeat uses the offsets, tile table and references that are there)
     if (bt[0].r.replay != kReplayCapture)
-      rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, large ? k_var_push_lookup<4> : k_var_push_lookup<1>, [&](const Item& it) {
+      rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, large ? PSKV_KSET_OF(k_var_push_lookup, 4) : PSKV_KSET_OF(k_var_push_lookup, 1), [&](const Item& it) {
         return it.r.n ? may_return_at_once(it, true, (it.r.n + chunk - 1) / chunk, bt.size()) : 0ull;
       });
     if (rc) return rc;
@@ -1396,7 +1453,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     int rc;
     if (push) {
       // a refused push must not be followed by its pull half
-      rc = read_state_batch(bt);
+      rc = read_state_batch(bt, true);
       if (rc) return rc;
       for (Item& it : bt) {
         rc = report_device_errors(it.t);
@@ -1418,7 +1475,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     if (rc) return rc;
     for (Item& it : bt)
       if (it.r.n && !it.tag.try_cache) it.t->cache_valid = false;
-    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, k_var_pull_lookup, [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET(k_var_pull_lookup), [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
     if (rc) return rc;
     if (async_pull) {
       // No host round trip: the grid covers the caller's buffer, the kernels take the real
@@ -1435,7 +1492,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       if (rc) return rc;
       return launch_rows<true>(bt, kOpGather);
     }
-    rc = read_state_batch(bt);  // the response sizes are data dependent
+    rc = read_state_batch(bt, true);  // the response sizes are data dependent
     if (rc) return rc;
     int fit = PSKV_OK;
     for (Item& it : bt) {
@@ -1547,6 +1604,36 @@ int validate(pskv_table* t, bool push, bool pull, uint64_t n, uint64_t nvals, co
   }
 }
 
+// Everything enqueued on the table has been waited for: small_in is free.
+void small_idle(pskv_table* t) {
+  t->small_part = 0;
+  t->small_at = 0;
+  t->small_in_flight = false;
+  for (bool& p : t->small_pending) p = false;
+}
+
+// Room for a small host-resident request of `bytes` bytes in small_in that no request in flight reads.
+int small_room(pskv_table* t, size_t bytes, char** out) {
+  if (bytes > kSmallPart) {  // all of it (such a request is waited for)
+    if (t->small_in_flight) PSKV_HIP(hipStreamSynchronize(t->stream));
+    small_idle(t);
+  } else if (t->small_at + bytes > kSmallPart) {
+    // the requests that lie in the part that is full now are queued
+    PSKV_HIP(hipEventRecord(t->small_done[t->small_part], t->stream));
+    t->small_pending[t->small_part] = true;
+    t->small_part = (t->small_part + 1) % kSmallParts;
+    t->small_at = 0;
+    if (t->small_pending[t->small_part]) {
+      PSKV_HIP(hipEventSynchronize(t->small_done[t->small_part]));
+      t->small_pending[t->small_part] = false;
+    }
+  }
+  *out = t->small_in + (size_t)t->small_part * kSmallPart + t->small_at;
+  t->small_at = std::min(t->small_at + bytes, kSmallPart);
+  t->small_in_flight = true;
+  return PSKV_OK;
+}
+
 int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n, const float* vals,
             size_t nvals, const int32_t* lens, size_t nlens, float* out, size_t out_cap,
             int32_t* out_lens, size_t* out_nvals, int memkind) {
@@ -1564,7 +1651,7 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
   const bool host = memkind == PSKV_MEM_HOST;
   const bool varlen = t->mode == PSKV_MODE_VARLEN;
   bool small = false;        // host-resident request served from the pinned buffers
-  int small_part = -1;       // the part of small_in it lies in when it does not take all of it
+  bool early = false;        // a small push that returns once its kernel is queued
   size_t small_out_at = 0;   // bytes of small_out already given away
 
   // SCALAR and FIXED know the response size up front. A response that does not fit is
@@ -1595,11 +1682,12 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
         Carver::need(n, 8) + Carver::need(r.nvals, 4) + Carver::need(want_lens ? n : 0, 4);
     const size_t out_lens_need = Carver::need(want_out_lens ? n : 0, 4);
     small = in_need <= kSmallBytes && out_lens_need <= kSmallBytes;
-    char* base = t->small_in;
-    // a push that returns at once takes one part of the pinned buffer, the others all of it
-    const bool early = small && t->mode == PSKV_MODE_SCALAR && !pull && t->small_done[0] != nullptr;
-    small_part = (early && in_need <= kSmallBytes / kSmallParts) ? t->small_next : -1;
-    if (small_part >= 0) base += (size_t)small_part * (kSmallBytes / kSmallParts);
+    char* base = nullptr;
+    early = small && t->mode == PSKV_MODE_SCALAR && !pull && in_need <= kSmallPart;
+    if (small) {
+      rc = small_room(t, in_need, &base);
+      if (rc) return rc;
+    }
     if (!small) {
       rc = grow(t, &t->stage, in_need + out_lens_need);
       if (rc) return rc;
@@ -1611,17 +1699,6 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
     int32_t* dlens = c.take<int32_t>(want_lens ? n : 0);
     int32_t* dout_lens = nullptr;
     if (small) {
-      // earlier requests are done with what this one overwrites: they ended with a wait, or left an event
-      if (small_part >= 0) {
-        if (t->small_pending[small_part]) {
-          PSKV_HIP(hipEventSynchronize(t->small_done[small_part]));
-          t->small_pending[small_part] = false;
-        }
-      } else if (t->small_newest >= 0) {
-        PSKV_HIP(hipEventSynchronize(t->small_done[t->small_newest]));  // (one stream: the others came before)
-        for (int q = 0; q < kSmallParts; ++q) t->small_pending[q] = false;
-        t->small_newest = -1;
-      }
       if (n) std::memcpy(dkeys, keys, n * 8);
       if (r.nvals) std::memcpy(dvals, vals, r.nvals * 4);
       if (want_lens && n) std::memcpy(dlens, lens, n * 4);
@@ -1662,6 +1739,7 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
     r.vals = dvals;
     r.lens = dlens;
     r.out_lens = want_out_lens ? dout_lens : nullptr;
+    r.pinned = small;
     r.lazy_out = pull && varlen;
     if (small && r.lazy_out) {
       r.small_out = t->small_out + small_out_at;
@@ -1671,6 +1749,10 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
   if (pull && !varlen && (host || too_small) && fixed_out) {
     if (small && !too_small && fixed_out * sizeof(float) <= kSmallBytes - small_out_at) {
       r.out = reinterpret_cast<float*>(t->small_out + small_out_at);
+      if (t->mode == PSKV_MODE_SCALAR) {  // the host watches for the end of the request
+        r.done = t->done;
+        r.done_seq = ++t->done_seq;
+      }
     } else {
       rc = grow(t, &t->stage_out, fixed_out * sizeof(float));
       if (rc) return rc;
@@ -1687,7 +1769,10 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
   if (out_nvals) *out_nvals = r.out_nvals;
   // Kernels of this request may still be reading the pinned request buffer, which the next
   // host-resident request overwrites from the host: no early return without a wait.
-  if (small && (rc || too_small)) (void)hipStreamSynchronize(t->stream);
+  if (small && (rc || too_small)) {
+    (void)hipStreamSynchronize(t->stream);
+    small_idle(t);
+  }
   if (rc) {
     t->cache_valid = false;
     return rc;
@@ -1721,18 +1806,17 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
     }
     if (pull && varlen && out_lens && n && !lens_pinned)
       PSKV_HIP(hipMemcpyAsync(out_lens, r.out_lens, n * 4, hipMemcpyDeviceToHost, t->stream));
-    if (small_part >= 0) {
+    if (early) {
       // no device-detected errors in this mode and nothing to hand back: the caller's buffers have
       // been copied, the kernel is queued, later requests follow it on the stream
-      PSKV_HIP(hipEventRecord(t->small_done[small_part], t->stream));
-      t->small_pending[small_part] = true;
-      t->small_newest = small_part;
-      t->small_next = (small_part + 1) % kSmallParts;
-    } else if (t->mode == PSKV_MODE_SCALAR) {
-      // no device-detected errors in this mode: waiting for the stream is all that is left
-      PSKV_HIP(hipStreamSynchronize(t->stream));
+      return PSKV_OK;
+    }
+    if (t->mode == PSKV_MODE_SCALAR) {
+      // no device-detected errors in this mode: the end of the request is all that is left to wait for
+      if (!r.done || !seen_in_time(r.done, r.done_seq)) PSKV_HIP(hipStreamSynchronize(t->stream));
     } else {
-      rc = read_state(t);  // also waits for the copies above
+      // (also waits for the copies above, where there were any)
+      rc = read_state(t, small && (!pull || !r.out_nvals || out_pinned));
       if (rc) return rc;
       rc = report_device_errors(t);
       if (rc) {
@@ -1740,6 +1824,7 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
         return rc;
       }
     }
+    small_idle(t);
     if (out_pinned) std::memcpy(out, r.out, r.out_nvals * 4);
     if (pull && varlen && out_lens && n && lens_pinned) std::memcpy(out_lens, r.out_lens, n * 4);
   }
@@ -1901,6 +1986,8 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   t->st_host = reinterpret_cast<StateView*>(t->shell->pinned);
   t->snap = reinterpret_cast<Snapshot*>(t->shell->pinned + 256);
   t->outcome = reinterpret_cast<unsigned long long*>(t->shell->pinned + 512);
+  t->done = reinterpret_cast<unsigned long long*>(t->shell->pinned + 768);
+  *t->done = 0ull;
   t->small_in = t->shell->pinned + 1024;
   t->small_out = t->small_in + kSmallBytes;
   for (int q = 0; q < kSmallParts; ++q) t->small_done[q] = t->shell->done[q];
@@ -2098,8 +2185,10 @@ int pskv_replay_run(pskv_replay* r) {
     PSKV_HIP(hipGraphLaunch(r->exec, r->stream));
     return PSKV_OK;
   }
-  for (const SavedLaunch& l : r->launches) hipLaunchKernelGGL(l.kernel, l.grid, dim3(kBlock), 0, r->stream, l.rb);
-  PSKV_HIP(hipGetLastError());
+  for (SavedLaunch& l : r->launches) {
+    void* args[] = {&l.rb};
+    PSKV_HIP(hipLaunchKernel(l.kernel, l.grid, dim3(kBlock), args, 0, r->stream));
+  }
   return PSKV_OK;
 }
 
@@ -2123,7 +2212,7 @@ int pskv_sync_multi(pskv_table* const* tables, size_t S) {
   for (size_t at = 0; at < S; at += kMaxBatch) {
     Batch bt(std::min<size_t>(S - at, kMaxBatch));
     for (size_t i = 0; i < bt.size(); ++i) bt[i].t = tables[at + i];
-    rc = read_state_batch(bt);
+    rc = read_state_batch(bt, false);
     if (rc) return rc;
     for (Item& it : bt) {
       rc = report_device_errors(it.t);  // every table's error bits are cleared; the first is reported
@@ -2278,10 +2367,8 @@ int pskv_copy_probe(pskv_table* t, void* dst, const void* src, size_t bytes) {
   DeviceGuard guard(t->device);
   const uint64_t n16 = bytes / 16;
   if ((n16 + kBlock - 1) / kBlock > 0x7fffffffull) return set_error(PSKV_EINVAL, "copy too large");
-  launch(t, PSKV_KERNEL_COPY, k_copy, dim3((unsigned)((n16 + kBlock - 1) / kBlock)), dim3(kBlock),
-         static_cast<f32x4*>(dst), static_cast<const f32x4*>(src), n16);
-  PSKV_HIP(hipGetLastError());
-  return PSKV_OK;
+  return launch(t, PSKV_KERNEL_COPY, k_copy, dim3((unsigned)((n16 + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                static_cast<f32x4*>(dst), static_cast<const f32x4*>(src), n16);
 }
 
 int pskv_table_counters(pskv_table* t, uint64_t* out, size_t cap) {

@@ -53,7 +53,8 @@ struct TableReq {
   // SCALAR key cache (a request that repeats the cached sorted key set is served from a
   // request-ordered value array): cache_keys above, the values in `arena`, the slot numbers in
   // `tile_key`
-  unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null
+  unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null; SCALAR
+                                // without the key cache: the word that takes tag.epoch when the request is done
   uint32_t cache_mode;          // kCache* below
   uint32_t tile_base;           // VARLEN row kernels: the launch starts at this tile of the request (a large
                                 // host-resident request is served piece by piece as it arrives)
@@ -65,10 +66,13 @@ constexpr uint32_t kCachePerKey = 3;  // SCALAR pull, slots up to date: every ke
 constexpr uint32_t kFlushUnlessSame = 1;  // k_scalar_flush: skip when the request in flight repeats the cache
 constexpr uint32_t kFlushAlways = 2;
 constexpr uint32_t kSlotSpecial = 0xffffffffu;  // cached slot number of key 2^64-1 (the side slot)
+// Every kernel comes for one, for up to four and for up to kMaxBatch tables: an argument of 3.8 KB costs the
+// calling thread 4.6 us per launch, one of 240 bytes 3.
+template <int TABLES>
 struct ReqBatch {
-  TableReq t[kMaxBatch];
+  TableReq t[TABLES];
 };
-static_assert(sizeof(ReqBatch) <= 3840, "kernel arguments are limited to 4 KiB");
+static_assert(sizeof(ReqBatch<kMaxBatch>) <= 3840, "kernel arguments are limited to 4 KiB");
 
 // ---------------------------------------------------------------------------------
 // SCALAR mode: one float per key, kept in the low word of the slot payload so that a
@@ -94,8 +98,12 @@ static_assert(sizeof(ReqBatch) <= 3840, "kernel arguments are limited to 4 KiB")
 // way and leaves its keys, their values and their slot numbers behind as the new cache.
 // A pull that comes right behind the push that filled the cache (the slots are up to date then)
 // needs no decision for the whole request: kCachePerKey compares key by key, in the same pass.
-template <bool PUSH, bool PULL, bool CACHE>
-__global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch b) {
+// PINNED: the request lies in pinned host memory, whose every read is a round trip over the host link
+// (about 2 us): everything the lane needs of it is asked for at once, the neighbours of the wavefront's
+// first and last key included. (From device memory the plain order is 2 % faster: those two reads are
+// mostly in the cache by the time they are made.)
+template <bool PUSH, bool PULL, bool CACHE, bool PINNED, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   const uint64_t n = d.n;
   const unsigned nblk = d.nblk;  // (the grid is sized for the table with the most workgroups)
@@ -202,17 +210,28 @@ __global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch b) {
   for (uint64_t first = (uint64_t)blockIdx.x * kBlock; first < n_turns; first += stride) {
     const uint64_t i = first + threadIdx.x;
     const bool live = i < n;
+    uint64_t outside = 0;  // PINNED: the key next to the wavefront's 64 keys on this lane's side
+    float v = 0.0f;
+    if (PINNED) {
+      const bool up = lane == 0 && i > 0 && live, down = lane == 63 && i + 1 < n;
+      if (up || down) outside = keys[up ? i - 1 : i + 1];
+      if (PUSH && live) v = vals[i];
+    }
     const uint64_t key = live ? keys[i] : 0;
     uint64_t before = __shfl_up(key, 1);
     uint64_t after = __shfl_down(key, 1);
     // the first and the last lane look just outside the wavefront's 64 keys; their neighbours have
     // fetched those lines already
-    if (lane == 0) before = (live && i > 0) ? keys[i - 1] : ~key;
-    if (lane == 63) after = (i + 1 < n) ? keys[i + 1] : ~key;
+    if (PINNED) {
+      if (lane == 0) before = outside;
+      if (lane == 63) after = outside;
+    } else {
+      if (lane == 0) before = (live && i > 0) ? keys[i - 1] : ~key;
+      if (lane == 63) after = (i + 1 < n) ? keys[i + 1] : ~key;
+    }
     if (!live || (i > 0 && before == key)) continue;  // past the end, or inside a run
     const bool run = i + 1 < n && after == key;
-    float v = 0.0f;
-    if (PUSH) v = vals[i];
+    if (PUSH && !PINNED) v = vals[i];
     bool is_new;
     uint64_t seen;
     uint64_t* p = find_or_insert(slots, mask, st, key, is_new, seen);
@@ -241,10 +260,17 @@ __global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch b) {
   // The workgroup that finishes last tells the host, which never waits for either, whether every
   // key of a key-by-key pull sat at its cached position and, when the host asked for it (the
   // table is close to a limit), what the counters are after this request.
+  // (A request without the key cache may have a host that watches a word for its end: the answers, in
+  // pinned memory, come before the word.)
   const bool want_outcome = kPerKey && d.cache_mode == kCachePerKey;
-  if (want_outcome || d.snap) {
+  const bool want_done = !CACHE && d.outcome != nullptr;
+  if (want_outcome || want_done || d.snap) {
     __shared__ unsigned s_last;
     const int any = want_outcome ? __syncthreads_or(differs ? 1 : 0) : 0;
+    if (want_done) {
+      __threadfence_system();
+      __syncthreads();
+    }
     if (threadIdx.x == 0) {
       if (any) atomicOr(&st->req_flags, kReqDiffer);
       s_last = ticket_last(st, nblk) ? 1u : 0u;
@@ -256,13 +282,16 @@ __global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch b) {
       if (d.outcome) *d.outcome = (d.tag.epoch << 1) | (all ? 1ull : 0ull);
     }
     if (d.snap && threadIdx.x < 64) publish_snapshot(st, d.snap, d.snap_seq);
+    if (want_done && threadIdx.x == 0)
+      __hip_atomic_store(d.outcome, d.tag.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
 // Writes the cached values back to their slots. Launched before anything reads or changes the
 // slots of a table whose cache may be ahead of them: a request that does not repeat the cached
 // keys (kFlushUnlessSame: the comparison of that request has run), a growth, a dump.
-__global__ __launch_bounds__(kBlock) void k_scalar_flush(ReqBatch b) {
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_scalar_flush(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;
   // nothing changes these two while this kernel runs except its own last workgroup, which writes
@@ -317,7 +346,8 @@ __device__ __forceinline__ void decide_same(DevState* st, const ReqTag& tag, boo
 // request: the workgroup that finishes last sees whether any workgroup found a difference and
 // writes same_epoch. (A var-len push, whose lens count as well, compares in k_var_push_begin.)
 constexpr int kSameKeysItems = 4;
-__global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch b) {
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;  // tables that have nothing to compare have no workgroups
   const uint64_t* __restrict__ keys = d.keys;
@@ -400,8 +430,8 @@ __device__ __forceinline__ void refuse_fixed(DevState* st, const ReqTag& tag) {
   st->refused_epoch = tag.epoch;
 }
 
-template <int kLookupItems>
-__global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch b) {
+template <int kLookupItems, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
@@ -528,7 +558,8 @@ __device__ __forceinline__ void load_four(FourKeys<W>& f, const uint64_t* keys, 
 // own.
 // (Bound by its tail, not by its bytes: the tickets, and the scan of the totals, which a request that
 // repeats the cached one does without.)
-__global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
@@ -588,8 +619,8 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch b) {
 constexpr unsigned kTileVar = 256;  // request-side floats per wavefront of the var-len row kernel: one quad per lane
 constexpr unsigned long long kArenaPadUnits = 8;  // 128 bytes in 16-byte allocation units
 
-template <int kItems>
-__global__ __launch_bounds__(kBlock) void k_var_push_lookup(ReqBatch b) {
+template <int kItems, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_push_lookup(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
@@ -725,7 +756,8 @@ __global__ __launch_bounds__(kBlock) void k_var_push_lookup(ReqBatch b) {
 // others are looked up. When every key does, the offsets of that push are the offsets of this response
 // as well, and the scan of the totals falls away. (The comparison was a launch of its own in front of this
 // one; a recorded request, which must not answer anything before the decision is there, still has it.)
-__global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch b) {
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
@@ -830,7 +862,8 @@ __global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch b) {
 // VARLEN pull, second kernel: pass 2 of the scan over the answered lengths: the request-side
 // offsets of the response and its tile table. `ntiles_cap` is the room in the table; the
 // tiles in use follow from the scanned total.
-__global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch b) {
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_offsets(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;
   const int32_t* __restrict__ lens = d.out_lens;  // the lengths the lookup kernel answered
@@ -1269,8 +1302,8 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
 constexpr unsigned kQuadsFixed = kBlock;
 constexpr unsigned kRowsVarPerBlock = kTileVar * (kBlock / 64);
 
-template <int OP, bool VARLEN, bool STREAM>
-__global__ __launch_bounds__(kBlock) void k_rows(ReqBatch b) {
+template <int OP, bool VARLEN, bool STREAM, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   // the grid is sized for the largest table of the launch: workgroups (VARLEN: wavefronts) past
   // this table's floats leave before they touch anything
