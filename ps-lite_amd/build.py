@@ -5,11 +5,13 @@ built file and never fall back to anything else.
 """
 import os
 import subprocess
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpskv.so")
+NATIVE = os.path.join(HERE, "_native.so")
 SOURCES = ["table.hip", "slice.hip", "hostmem.hip", "stager.hip", "devpool.hip", "match.hip", "meta_codec.cc"]
 HEADERS = ["device_common.h", "devpool.h", "host_common.h", "scan.h", "stager.h", "table_kernels.h"]
 
@@ -31,7 +33,7 @@ def lib_path():
 
 
 def is_built():
-    return os.path.exists(LIB)
+    return os.path.exists(LIB) and os.path.exists(NATIVE)
 
 
 def build_lib(verbose=False):
@@ -54,7 +56,18 @@ def build_lib(verbose=False):
             print(out, flush=True)
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", LIB]
     subprocess.run(cmd, check=True)
+    build_native()
     return LIB
+
+
+def build_native():
+    """Compiles the per-request half of the Python binding (csrc/pymodule.cc) against the library."""
+    cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+           "-I" + os.path.join(REPO, "include"), "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "pymodule.cc"), "-L" + HERE, "-lpskv", "-Wl,-rpath,$ORIGIN", "-L/opt/rocm/lib",
+           "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-o", NATIVE]
+    subprocess.run(cmd, check=True)
+    return NATIVE
 
 
 HOST_TEST = os.path.join(REPO, "tests", "test_kv_app_gpu")

@@ -1,4 +1,5 @@
-"""ctypes binding of libpskv.so, the C ABI declared in include/pskv/capi.h.
+"""Binding of libpskv.so, the C ABI declared in include/pskv/capi.h: ctypes, and the extension module _native
+(csrc/pymodule.cc) for the calls that a request takes.
 
 Buffers are either numpy arrays (host memory, PSKV_MEM_HOST) or torch tensors
 on the table's device (PSKV_MEM_DEVICE). torch is only the owner of device
@@ -67,6 +68,24 @@ class Opts(ctypes.Structure):
 
 
 _lib = None
+_native = None
+
+
+def _load_native():
+    """The extension module behind push, pull and their like, told what tensors look like where torch is there."""
+    global _native
+    from . import _native as native
+    try:
+        import torch
+    except ImportError:
+        pass
+    else:
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is None:
+            def raw(device):
+                return torch.cuda.current_stream(device).cuda_stream
+        native.setup(torch.Tensor, torch.int64, getattr(torch, "uint64", torch.int64), torch.float32, torch.int32, raw)
+    _native = native
 
 
 def load():
@@ -120,6 +139,7 @@ def load():
     lib.pskv_table_counters.argtypes = [vp, vp, sz]
     lib.pskv_last_error.restype = ctypes.c_char_p
     lib.pskv_version.restype = ctypes.c_char_p
+    _load_native()
     _lib = lib
     return lib
 
@@ -166,14 +186,23 @@ class _Holder:
     next wait, so that a temporary (`t.push(to_dev(keys), ...)`) is not handed to someone else by
     torch's allocator while a kernel is still to read it. The *_raw methods leave that to the caller."""
 
+    _held = None
+
     def _hold(self, *tensors):
-        held = self.__dict__.setdefault("_held", [])
-        held.extend(x for x in tensors if x is not None and _is_tensor(x) and x.is_cuda)
-        if len(held) > 4096:
+        self._holding().extend(x for x in tensors if x is not None and _is_tensor(x) and x.is_cuda)
+
+    def _holding(self):
+        """The list that device tensors of a call go to."""
+        held = self._held
+        if held is None:
+            self._held = held = []
+        elif len(held) > 4096:
             self.sync()
+            held = self._held
+        return held
 
     def _release(self):
-        self.__dict__["_held"] = []
+        self._held = []
 
 
 class Table(_Holder):
@@ -185,6 +214,7 @@ class Table(_Holder):
         self._h = ctypes.c_void_p()
         o = Opts(device, mode, initial_capacity, row_len, arena_floats, max_load, 0, stream)
         _check(self._lib.pskv_table_create(ctypes.byref(self._h), ctypes.byref(o)))
+        self._at = self._h.value
         self.mode = mode
         self.device = device
 
@@ -192,6 +222,7 @@ class Table(_Holder):
         if self._h:
             self._lib.pskv_table_destroy(self._h)
             self._h = ctypes.c_void_p()
+            self._at = 0
         self._release()
 
     def __del__(self):
@@ -205,6 +236,11 @@ class Table(_Holder):
             pass
 
     def push(self, keys, vals, lens=None):
+        rc = _native.table_push(self._at, keys, vals, lens, self._holding())
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return
         kp, n, k1 = _buf(keys, np.uint64, "int64")
         vp, nv, k2 = _buf(vals, np.float32, "float32")
         lp, nl, k3 = _buf(lens, np.int32, "int32")
@@ -213,6 +249,9 @@ class Table(_Holder):
 
     def pull(self, keys, out, out_lens=None):
         """Returns the number of floats of the response."""
+        got = _native.table_pull(self._at, keys, out, out_lens, self._holding())
+        if got is not None:
+            return self._sized(got)
         kp, n, k1 = _buf(keys, np.uint64, "int64")
         op, cap, k2 = _buf(out, np.float32, "float32")
         lp, _, k3 = _buf(out_lens, np.int32, "int32")
@@ -224,7 +263,16 @@ class Table(_Holder):
         _check(rc)
         return got.value
 
+    def _sized(self, got):
+        rc, self.last_out_nvals = got if isinstance(got, tuple) else (OK, got)
+        if rc:
+            _check(rc)
+        return self.last_out_nvals
+
     def pushpull(self, keys, vals, out, lens=None, out_lens=None):
+        got = _native.table_pushpull(self._at, keys, vals, lens, out, out_lens, self._holding())
+        if got is not None:
+            return self._sized(got)
         kp, n, k1 = _buf(keys, np.uint64, "int64")
         vp, nv, k2 = _buf(vals, np.float32, "float32")
         lp, nl, k3 = _buf(lens, np.int32, "int32")
@@ -322,6 +370,7 @@ class Group(_Holder):
         self.S = S
         self.mode = mode
         self._arr = (ctypes.c_void_p * max(S, 1))(*[t._h for t in self.tables])
+        self._at = ctypes.addressof(self._arr)
         self._lib = load()
 
     def close(self):
@@ -377,6 +426,13 @@ class Group(_Holder):
 
     def pushpull(self, keys, pos, vals, val_pos, out, lens=None, out_pos=None, out_lens=None, want_sizes=False):
         """pskv_pushpull_multi: one request with both halves over all slices."""
+        if not want_sizes:
+            rc = _native.group_pushpull(self._at, self.S, keys, vals, lens, out, out_lens, pos, val_pos, out_pos, None,
+                                        self._holding())
+            if rc is not None:
+                if rc:
+                    _check(rc)
+                return None
         _memkind(MEM_DEVICE)
         self._hold(keys, vals, lens, out, out_lens)
         pos = np.ascontiguousarray(pos, dtype=np.uint64)
@@ -394,6 +450,11 @@ class Group(_Holder):
         return sizes[:self.S] if want_sizes else None
 
     def push(self, keys, pos, vals, val_pos, lens=None):
+        rc = _native.group_push(self._at, self.S, keys, vals, lens, pos, val_pos, self._holding())
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return
         _memkind(MEM_DEVICE)
         self._hold(keys, vals, lens)
         self.push_raw(keys.data_ptr() if keys.numel() else None, pos,
@@ -401,6 +462,13 @@ class Group(_Holder):
                       None if lens is None else (lens.data_ptr() if lens.numel() else None))
 
     def pull(self, keys, pos, out, out_pos=None, out_lens=None, want_sizes=False):
+        if not want_sizes:
+            rc = _native.group_pull(self._at, self.S, keys, out, out_lens, pos, out_pos, None, self._holding())
+            if rc is not None:
+                self.last_sizes = None
+                if rc:
+                    _check(rc)
+                return None
         _memkind(MEM_DEVICE)
         self._hold(keys, out, out_lens)
         return self.pull_raw(keys.data_ptr() if keys.numel() else None, pos,
@@ -445,16 +513,20 @@ class Replay:
 
     def __init__(self, handle, held):
         self._h = handle
+        self._at = handle.value
         self._held = held
         self._lib = load()
 
     def run(self):
-        _check(self._lib.pskv_replay_run(self._h))
+        rc = _native.replay_run(self._at)
+        if rc:
+            _check(rc)
 
     def close(self):
         if self._h:
             self._lib.pskv_replay_destroy(self._h)
             self._h = None
+            self._at = 0
             self._held = None
 
     def __del__(self):
@@ -476,6 +548,17 @@ def server_ranges(num_servers):
 
 def slice_keys(keys, range_begin, range_end, lens=None, nvals=0, device=0):
     """KVWorker::DefaultSlicer (kv_app.h:517-572): returns (pos, val_pos, used)."""
+    if _native is None:
+        load()
+    if isinstance(range_begin, np.ndarray) and range_begin.ndim == 1:
+        S = range_begin.size
+        pos, val_pos = np.zeros((2, S + 1), np.uint64)
+        used = np.zeros(max(S, 1), np.uint8)
+        rc = _native.slice(device, keys, lens, nvals, range_begin, range_end, pos, val_pos, used)
+        if rc is not None:
+            if rc:
+                _check(rc)
+            return pos, val_pos, used if S else used[:0]
     kp, n, k1 = _buf(keys, np.uint64, "int64")
     lp, nl, k2 = _buf(lens, np.int32, "int32")
     rb = np.ascontiguousarray(range_begin, dtype=np.uint64)
@@ -536,6 +619,14 @@ def match(src_keys, src_vals, dst_keys, dst_vals, k=1, op=OP_ASSIGN, device=0, k
     dst_keys[i] == src_keys[j], in place. numpy arrays (host memory) or torch tensors on the device.
     Returns the number of matched VALUES (k per matched key). kernel_ms: None, or a float32 numpy array of
     two entries that receives the device time of the call's key kernel and row kernel."""
+    if _native is None:
+        load()
+    if kernel_ms is None and (_is_tensor(dst_vals) or isinstance(dst_vals, np.ndarray)):
+        got = _native.match(device, src_keys, src_vals, dst_keys, dst_vals, k, op)
+        if got is not None:
+            if isinstance(got, tuple):
+                _check(got[0])
+            return got
     skp, ns, m1 = _buf(src_keys, np.uint64, "int64")
     svp, nsv, m2 = _buf(src_vals, np.float32, "float32")
     dkp, nd, m3 = _buf(dst_keys, np.uint64, "int64")
