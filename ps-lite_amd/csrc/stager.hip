@@ -8,6 +8,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <vector>
 
 #include "host_common.h"
 
@@ -15,10 +16,12 @@ namespace pskv {
 
 struct Stager::Impl {
   int device = 0;
-  hipStream_t copy = nullptr;  // the stream of the copy commands (default priority)
+  // The streams of the copy commands (default priority), which take turns: one stream leaves the link idle for
+  // about 15 us between two commands, a tenth of a piece's time.
+  hipStream_t copy[kStreams] = {nullptr};
   char* ring = nullptr;        // kSlots pieces of pinned memory
   hipEvent_t dma_done[kSlots];   // the copy command that last used the slot has finished
-  hipEvent_t prod_done[kSlots];  // device -> host: the producer has written the slot's piece
+  hipEvent_t prod_done[2];       // device -> host: the producer has written the first piece, and everything
 
   std::mutex op_mu;  // one transfer at a time: the host link is what they would share anyway
 
@@ -91,13 +94,14 @@ Stager* Stager::get(int device) {
   Impl* im = new (std::nothrow) Impl();
   if (!im) return nullptr;
   im->device = device;
-  bool ok = hipStreamCreateWithFlags(&im->copy, hipStreamNonBlocking) == hipSuccess;
+  bool ok = true;
+  for (int q = 0; ok && q < kStreams; ++q) ok = hipStreamCreateWithFlags(&im->copy[q], hipStreamNonBlocking) == hipSuccess;
   ok = ok && hipHostMalloc(reinterpret_cast<void**>(&im->ring), (size_t)kSlots * kPiece, hipHostMallocDefault) ==
                  hipSuccess;
   for (int s = 0; ok && s < kSlots; ++s) {
-    ok = hipEventCreateWithFlags(&im->dma_done[s], hipEventDisableTiming) == hipSuccess &&
-         hipEventCreateWithFlags(&im->prod_done[s], hipEventDisableTiming) == hipSuccess;
+    ok = hipEventCreateWithFlags(&im->dma_done[s], hipEventDisableTiming) == hipSuccess;
   }
+  for (hipEvent_t& e : im->prod_done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     failed[device] = true;  // (what was created stays; this happens once)
@@ -108,13 +112,34 @@ Stager* Stager::get(int device) {
   return table[device];
 }
 
+namespace {
+
+// Where the pieces of a transfer begin (and, last, where it ends). Whatever the workers copy before the first
+// command can go out, or after the last one has come in, is time in which the link stands still: on the way to
+// the device the first pieces are short and double up to kPiece, on the way back the last ones halve.
+std::vector<size_t> cut(size_t bytes, bool to_device) {
+  constexpr size_t kLeast = 512u << 10, kUnit = 64u << 10;
+  std::vector<size_t> at(1, 0);
+  for (size_t len = kLeast; at.back() < bytes;) {
+    const size_t left = bytes - at.back();
+    if (!to_device) len = std::max(kLeast, (left / 2 + kUnit - 1) / kUnit * kUnit);
+    at.push_back(at.back() + std::min(left, std::min(len, Stager::kPiece)));
+    if (to_device) len = std::min(2 * len, Stager::kPiece);
+  }
+  return at;
+}
+
+}  // namespace
+
 int Stager::to_device(void* dst, const void* src, size_t bytes, hipStream_t consumer,
-                      const std::function<int(size_t, size_t)>& after_piece) {
+                      const std::function<int(size_t, size_t)>& consume) {
+  static_assert(kStreams == 2, "the last two commands are the last of each stream");
   Impl* im = impl_;
   std::lock_guard<std::mutex> op(im->op_mu);
-  const size_t npieces = (bytes + kPiece - 1) / kPiece;
-  auto len_of = [&](size_t c) { return c + 1 < npieces ? kPiece : bytes - c * kPiece; };
-  size_t issued = 0, sent = 0;
+  const std::vector<size_t> at = cut(bytes, true);
+  const size_t npieces = at.size() - 1;
+  auto len_of = [&](size_t c) { return at[c + 1] - at[c]; };
+  size_t issued = 0, sent = 0, consumed = 0;
   int status = PSKV_OK;
   auto check = [&](hipError_t e) {
     if (e != hipSuccess && !status)
@@ -129,19 +154,27 @@ int Stager::to_device(void* dst, const void* src, size_t bytes, hipStream_t cons
       const int slot = (int)(issued % kSlots);
       // the copy command that last read this slot (this transfer's or an earlier one's) is done
       if (!check(hipEventSynchronize(im->dma_done[slot]))) break;
-      im->submit(im->slot_ptr(slot), static_cast<const char*>(src) + issued * kPiece, len_of(issued), slot);
+      im->submit(im->slot_ptr(slot), static_cast<const char*>(src) + at[issued], len_of(issued), slot);
       ++issued;
     }
     if (status) break;
     const int slot = (int)(sent % kSlots);
-    const size_t off = sent * kPiece, len = len_of(sent);
+    const size_t off = at[sent], len = len_of(sent);
+    hipStream_t copy = im->copy[sent % kStreams];
     im->wait_slot(slot);
-    if (!check(hipMemcpyAsync(static_cast<char*>(dst) + off, im->slot_ptr(slot), len, hipMemcpyHostToDevice,
-                              im->copy)) ||
-        !check(hipEventRecord(im->dma_done[slot], im->copy)) ||
-        !check(hipStreamWaitEvent(consumer, im->dma_done[slot], 0)))
+    if (!check(hipMemcpyAsync(static_cast<char*>(dst) + off, im->slot_ptr(slot), len, hipMemcpyHostToDevice, copy)) ||
+        !check(hipEventRecord(im->dma_done[slot], copy)))
       break;
-    if (after_piece) status = after_piece(off, len);
+    // The consumer works through what has arrived in stretches of kStretch pieces, and at the end on the last
+    // piece alone: it needs a fortieth of the transfer's time, and a stream that waits for every piece holds
+    // up the copy commands where it shares a hardware queue with one of theirs.
+    if ((sent + 1) % kStretch == 0 || sent + 2 >= npieces) {
+      bool ok = check(hipStreamWaitEvent(consumer, im->dma_done[slot], 0));
+      if (ok && sent > 0) ok = check(hipStreamWaitEvent(consumer, im->dma_done[(sent - 1) % kSlots], 0));
+      if (!ok) break;
+      if (consume) status = consume(at[consumed], off + len - at[consumed]);
+      consumed = sent + 1;
+    }
     ++sent;
   }
   if (status) {
@@ -152,11 +185,12 @@ int Stager::to_device(void* dst, const void* src, size_t bytes, hipStream_t cons
 }
 
 int Stager::to_host(void* dst, const void* src, size_t bytes, hipStream_t producer,
-                    const std::function<int(size_t, size_t)>& before_piece) {
+                    const std::function<int(size_t, size_t)>& produce) {
   Impl* im = impl_;
   std::lock_guard<std::mutex> op(im->op_mu);
-  const size_t npieces = (bytes + kPiece - 1) / kPiece;
-  auto len_of = [&](size_t c) { return c + 1 < npieces ? kPiece : bytes - c * kPiece; };
+  const std::vector<size_t> at = cut(bytes, false);
+  const size_t npieces = at.size() - 1;
+  auto len_of = [&](size_t c) { return at[c + 1] - at[c]; };
   size_t launched = 0, drained = 0;
   int status = PSKV_OK;
   while (drained < npieces && status == PSKV_OK) {
@@ -169,17 +203,26 @@ int Stager::to_host(void* dst, const void* src, size_t bytes, hipStream_t produc
         if (drained < launched) break;  // hand out what has arrived first
         im->wait_slot(slot);
       }
-      const size_t off = launched * kPiece, len = len_of(launched);
-      if (before_piece) {
-        status = before_piece(off, len);
-        if (status) break;
+      const size_t off = at[launched], len = len_of(launched);
+      hipStream_t copy = im->copy[launched % kStreams];
+      // The producer's work is done for the first piece, then for all the others at once: it takes a fortieth of
+      // the transfer's time, and a producer that takes turns with the copy commands holds them up (9 to 20 us a
+      // piece).
+      hipError_t e = hipSuccess;
+      if (launched < 2) {
+        if (produce) {
+          status = produce(off, launched == 0 ? len : bytes - off);
+          if (status) break;
+        }
+        e = hipEventRecord(im->prod_done[launched], producer);
+        if (e == hipSuccess) e = hipStreamWaitEvent(copy, im->prod_done[launched], 0);
+      } else if (launched < 1 + kStreams) {
+        e = hipStreamWaitEvent(copy, im->prod_done[1], 0);
       }
-      hipError_t e = hipEventRecord(im->prod_done[slot], producer);
-      if (e == hipSuccess) e = hipStreamWaitEvent(im->copy, im->prod_done[slot], 0);
       if (e == hipSuccess)
         e = hipMemcpyAsync(im->slot_ptr(slot), static_cast<const char*>(src) + off, len, hipMemcpyDeviceToHost,
-                           im->copy);
-      if (e == hipSuccess) e = hipEventRecord(im->dma_done[slot], im->copy);
+                           copy);
+      if (e == hipSuccess) e = hipEventRecord(im->dma_done[slot], copy);
       if (e != hipSuccess) {
         status = set_error(PSKV_EHIP, "staging a response failed: %s", hipGetErrorString(e));
         break;
@@ -193,12 +236,13 @@ int Stager::to_host(void* dst, const void* src, size_t bytes, hipStream_t produc
       status = set_error(PSKV_EHIP, "staging a response failed: %s", hipGetErrorString(e));
       break;
     }
-    im->submit(static_cast<char*>(dst) + drained * kPiece, im->slot_ptr(slot), len_of(drained), slot);
+    im->submit(static_cast<char*>(dst) + at[drained], im->slot_ptr(slot), len_of(drained), slot);
     ++drained;
   }
   // nothing of this transfer may be left in the ring or in flight when the caller gets its buffer
   for (int s = 0; s < kSlots; ++s) im->wait_slot(s);
-  if (status) (void)hipStreamSynchronize(im->copy);
+  if (status)
+    for (hipStream_t copy : im->copy) (void)hipStreamSynchronize(copy);
   return status;
 }
 

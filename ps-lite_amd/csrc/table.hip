@@ -1788,7 +1788,7 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
     Stager* sg = Stager::get(t->device);
     if (pull && r.out_nvals && !out_pinned) {
       if (r.gather_deferred || (sg && r.out_nvals * 4 >= kPipeBytes && !host_pool_owns(out, r.out_nvals * 4))) {
-        // piece by piece: the gather of a piece (when it is still owed), its transfer, and the copy
+        // piece by piece: the gather (when it is still owed), the transfer of a piece, and the copy
         // into the caller's buffer overlap with those of the neighbouring pieces
         if (!sg) return set_error(PSKV_ENOMEM, "no pinned memory to stage the response through");
         std::function<int(size_t, size_t)> gather;
