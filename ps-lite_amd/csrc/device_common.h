@@ -140,6 +140,18 @@ struct Snapshot {
   volatile uint64_t seq_end;
 };
 
+// Adds a workgroup's facts (one thread calls it) to those of the other workgroups of a launch of `nblk`. Every
+// workgroup of a request that differs from the cached one finds the same fact, and atomics on one address are
+// served one at a time: a large launch looks first whether somebody has reported it already (a comparison of
+// 4M keys that differ took 52 us, of 4M that do not 12).
+__device__ __forceinline__ void report_facts(DevState* st, unsigned facts, unsigned nblk) {
+  constexpr unsigned kFew = 512;  // so many are under way before anybody could see them
+  if (nblk > kFew &&
+      (facts & ~__hip_atomic_load(&st->req_flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u)
+    return;
+  atomicOr(&st->req_flags, facts);
+}
+
 // What a row-mode kernel needs to know about the request it belongs to.
 struct ReqTag {
   unsigned long long epoch;  // number of the request

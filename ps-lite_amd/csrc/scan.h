@@ -80,7 +80,7 @@ __device__ __forceinline__ void scan_spine(unsigned long long* part, uint64_t np
 // Pass 1, the workgroup's part. Every thread calls it with the sum of its lens, taken as
 // sign-extended 64-bit values modulo 2^64 (what `size_t val_end += int l` does in the
 // reference, kv_app.h:565), and the kReq* facts it found. The workgroup's total goes to
-// part[blockIdx.x], its facts to DevState::req_flags (one atomic per workgroup at most).
+// part[blockIdx.x], its facts to DevState::req_flags.
 // Returns true in every thread of the workgroup that finishes last of the `nblk` that scan this
 // table's request. `red`/`fred` hold kBlock/64 words each.
 __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned flags,
@@ -90,7 +90,7 @@ __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned 
                                                  unsigned* s_last) {
   block_sum_or(s, flags, red, fred);
   if (threadIdx.x == 0) {
-    if (flags) atomicOr(&st->req_flags, flags);
+    if (flags) report_facts(st, flags, nblk);
     publish_u64(&part[blockIdx.x], s);
     *s_last = ticket_last(st, nblk) ? 1u : 0u;
   }

@@ -684,7 +684,8 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
   // Two limits. `limit` is the fill the table is kept below; `hard` (0.85 unless max_load is higher) is
   // the fill it must never exceed. The keys in flight count in full against the second, and against the
   // first with the share of them that is going to be new if requests go on as the latest records say
-  // (twice that share plus a tenth, to be on the safe side; in full while no record has said anything).
+  // (a quarter more than that share plus a tenth, to be on the safe side; in full while no record has said
+  // anything).
   // A server whose requests mostly name keys it holds, the steady state of a parameter server, then does
   // not grow, or wait, for keys that are not coming, however far ahead of the device its caller runs; if
   // the requests change their ways the table runs fuller than `limit` for as long as it takes the next
@@ -693,7 +694,7 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
   const double hard = std::max((double)t->max_load, kHardLoad) * (double)t->cap;
   auto slots_short = [&]() {
     // (looked up on every call: a record adopted further down may have changed it)
-    const double share = t->share_known ? std::min(1.0, 2.0 * t->new_share + 0.1) : 1.0;
+    const double share = t->share_known ? std::min(1.0, 1.25 * t->new_share + 0.1) : 1.0;
     const double in_flight = (double)(t->pend_keys + n);
     return (double)t->base_count + in_flight > hard || (double)t->base_count + share * in_flight > limit;
   };

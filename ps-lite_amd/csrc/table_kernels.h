@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch<TABLES> b) {
       __syncthreads();
     }
     if (threadIdx.x == 0) {
-      if (any) atomicOr(&st->req_flags, kReqDiffer);
+      if (any) report_facts(st, kReqDiffer, nblk);
       s_last = ticket_last(st, nblk) ? 1u : 0u;
     }
     __syncthreads();
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch<TABLES> b) {
   for (int j = 0; j < kItems; ++j) differ |= a[j] != c[j];
   const int any = __syncthreads_or(differ ? 1 : 0);
   if (threadIdx.x == 0) {
-    if (any) atomicOr(&st->req_flags, kReqDiffer);
+    if (any) report_facts(st, kReqDiffer, d.nblk);
     s_last = ticket_last(st, d.nblk) ? 1u : 0u;
   }
   __syncthreads();
