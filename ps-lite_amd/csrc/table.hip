@@ -91,12 +91,18 @@ struct StateView {
   unsigned long long seq;  // written last: the number of the reading (StateBatch::seq)
 };
 
-// A new table's device state: all zero, the side slot's payload unset. One workgroup.
-__global__ void k_init_state(DevState* st) {
+// A new table: its device state all zero, the side slot's payload unset, its slots all ones (key = empty
+// marker). One launch: a memset command behind a kernel of its own left the GPU idle for 5 to 12 us per table.
+__global__ __launch_bounds__(kBlock) void k_init_table(DevState* st, Slot* slots, uint64_t cap) {
   unsigned long long* w = reinterpret_cast<unsigned long long*>(st);
   constexpr unsigned kAt = offsetof(DevState, special_payload) / 8;
   static_assert(sizeof(DevState) % 8 == 0, "the state is cleared word by word");
-  for (unsigned i = threadIdx.x; i < sizeof(DevState) / 8; i += blockDim.x) w[i] = i == kAt ? kPayloadUnset : 0ull;
+  if (blockIdx.x == 0)
+    for (unsigned i = threadIdx.x; i < sizeof(DevState) / 8; i += kBlock) w[i] = i == kAt ? kPayloadUnset : 0ull;
+  const u64x2 empty = {kEmptyKey, kPayloadUnset};
+  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < cap; i += stride)
+    *reinterpret_cast<u64x2*>(&slots[i]) = empty;
 }
 
 // One wavefront per table (blockIdx.x).
@@ -123,13 +129,14 @@ __global__ void k_read_state(StateBatch sb) {
 }
 
 // The parts of a table that have one size whatever the table holds: device state, the pinned words and
-// request buffers, events. Creating them costs the calling thread about a millisecond (every
+// request buffers, events, its stream. Creating them costs the calling thread about a millisecond (every
 // pinned allocation and its release go through the driver), so a table that goes leaves its shell to
 // the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim.
 struct Shell {
   DevState* st = nullptr;
   char* pinned = nullptr;  // StateView, Snapshot, outcome word, done word (256 bytes each), small_in, small_out
   hipEvent_t done[kSmallParts] = {nullptr};
+  hipStream_t stream = nullptr;  // the stream of a table that was not given one
 };
 constexpr size_t kShellsKept = 32;
 
@@ -141,6 +148,7 @@ ShellPool g_shells[64];
 
 void shell_free(Shell* sh) {
   if (!sh) return;
+  if (sh->stream) (void)hipStreamDestroy(sh->stream);
   if (sh->st) (void)hipFree(sh->st);
   if (sh->pinned) (void)hipHostFree(sh->pinned);
   for (hipEvent_t e : sh->done)
@@ -209,7 +217,6 @@ struct pskv_table {
   int device = 0;
   int mode = PSKV_MODE_SCALAR;
   hipStream_t stream = nullptr;
-  bool own_stream = false;
   float max_load = 0.5f;
 
   Slot* slots = nullptr;
@@ -461,12 +468,9 @@ int report_device_errors(pskv_table* t) {
   return set_error(PSKV_ELEN_CHANGED, "a pushed row length differs from the stored length");
 }
 
-int alloc_slots(uint64_t cap, Slot** out, hipStream_t stream, bool fill = true) {
-  int rc = array_alloc(reinterpret_cast<void**>(out), cap * sizeof(Slot), stream);
-  if (rc) return rc;
-  // all-ones bytes: key = empty marker (k_regrow writes every slot itself and needs no fill)
-  if (fill) PSKV_HIP(hipMemsetAsync(*out, 0xFF, cap * sizeof(Slot), stream));
-  return PSKV_OK;
+// (not filled: whoever asks for the array writes every slot of it)
+int alloc_slots(uint64_t cap, Slot** out, hipStream_t stream) {
+  return array_alloc(reinterpret_cast<void**>(out), cap * sizeof(Slot), stream);
 }
 
 int grow(pskv_table* t, GrowBuf* b, size_t bytes) {
@@ -591,7 +595,7 @@ int grow_slots(pskv_table* t, uint64_t keys_needed) {
       if (rc) return rc;
     }
     const auto a0 = std::chrono::steady_clock::now();
-    rc = alloc_slots(want, &fresh, t->stream, false);
+    rc = alloc_slots(want, &fresh, t->stream);
     t->stats.alloc_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - a0).count();
     if (rc) return rc;
   }
@@ -1979,9 +1983,9 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   if (opts->stream) {
     t->stream = static_cast<hipStream_t>(opts->stream);
   } else {
-    if (hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking) != hipSuccess)
+    if (!t->shell->stream && hipStreamCreateWithFlags(&t->shell->stream, hipStreamNonBlocking) != hipSuccess)
       return fail(set_error(PSKV_EHIP, "hipStreamCreateWithFlags failed"));
-    t->own_stream = true;
+    t->stream = t->shell->stream;
   }
   t->st = t->shell->st;
   t->st_host = reinterpret_cast<StateView*>(t->shell->pinned);
@@ -1995,12 +1999,12 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   std::memset(t->st_host, 0, sizeof(StateView));
   std::memset(t->snap, 0xFF, sizeof(Snapshot));  // names no request
   *t->outcome = 0ull;
-  k_init_state<<<dim3(1), dim3(256), 0, t->stream>>>(t->st);
-  if (hipGetLastError() != hipSuccess) return fail(set_error(PSKV_EHIP, "table initialisation failed"));
   const uint64_t keys = opts->initial_capacity ? opts->initial_capacity : kDefaultCapacity;
   t->cap = std::max(kMinSlots, next_pow2((uint64_t)((double)keys / t->max_load) + 1));
   int rc = alloc_slots(t->cap, &t->slots, t->stream);
   if (rc) return fail(rc);
+  k_init_table<<<dim3(grid_for(t->cap, kBlock, 1u << 16)), dim3(kBlock), 0, t->stream>>>(t->st, t->slots, t->cap);
+  if (hipGetLastError() != hipSuccess) return fail(set_error(PSKV_EHIP, "table initialisation failed"));
   if (t->mode != PSKV_MODE_SCALAR && opts->arena_floats) {
     t->arena_cap = (opts->arena_floats + 1023) & ~(uint64_t)1023;
     if (array_alloc(reinterpret_cast<void**>(&t->arena), t->arena_cap * sizeof(float) + kArenaEnd, t->stream) != PSKV_OK)
@@ -2039,7 +2043,6 @@ int pskv_table_destroy(pskv_table* t) {
                            &t->sc_vals, &t->sc_slots})
     (void)array_release(b->ptr, t->stream, true);
   shell_give(t->device, t->shell);
-  if (t->own_stream) (void)hipStreamDestroy(t->stream);
   delete t;
   return PSKV_OK;
 }
@@ -2241,7 +2244,7 @@ int pskv_size(pskv_table* t, uint64_t* n_keys, uint64_t* n_vals) {
   clear_error();
   if (!t) return set_error(PSKV_EINVAL, "null table");
   DeviceGuard guard(t->device);
-  int rc = read_state(t);
+  int rc = read_state(t, true);
   if (rc) return rc;
   const uint64_t nk = t->count;  // includes key 2^64-1 when present
   if (n_keys) *n_keys = nk;
