@@ -23,9 +23,12 @@ namespace {
 constexpr unsigned kMatchBlock = 256;
 constexpr unsigned kMatchItems = 4;
 constexpr unsigned kMatchTile = kMatchBlock * kMatchItems;  // destination keys per workgroup
-constexpr unsigned kMatchLds = 2048;    // source keys a workgroup holds in LDS at a time (16 KiB)
+constexpr unsigned kMatchLds = 1536;    // source keys (and values) a workgroup holds in LDS at a time (18 KiB)
+constexpr unsigned kMatchTurn = 3;      // source keys a lane asks for at a time
 constexpr unsigned kMatchPieces = 8;    // a longer stretch than this many pieces is searched in place
 constexpr uint64_t kNoMatch = ~0ull;
+constexpr unsigned kCounts = 64;        // counters of matched keys, each on a line of its own
+constexpr unsigned kCountStride = 16;
 
 // first index in [lo, hi) whose key is not below `key`
 __device__ __forceinline__ uint64_t lower_bound_of(const uint64_t* __restrict__ a, uint64_t lo, uint64_t hi,
@@ -56,36 +59,65 @@ __device__ __forceinline__ f32x4 combine(int op, f32x4 d, f32x4 s) {
 
 // spans[t] = first source key not below the first destination key of tile t; spans[tiles] = n_src.
 // The stretch of tile t is [spans[t], spans[t+1]): it may hold source keys that lie between two
-// tiles, which match nothing. One wavefront per tile: 64 probes per round narrow the range by a
-// factor of 64, so 16M source keys take four dependent loads where halving takes 24.
-__global__ __launch_bounds__(kMatchBlock) void k_match_spans(const uint64_t* __restrict__ src, uint64_t n_src,
-                                                             const uint64_t* __restrict__ dst, uint64_t tiles,
-                                                             uint64_t* __restrict__ spans) {
-  const uint64_t t = (uint64_t)blockIdx.x * (kMatchBlock / 64) + (threadIdx.x >> 6);
-  const unsigned lane = threadIdx.x & 63;
-  if (t > tiles) return;  // (whole wavefronts)
-  if (t == tiles) {
-    if (lane == 0) spans[t] = n_src;
-    return;
+// tiles, which match nothing. Bound by the round trips to memory that follow from each other: a workgroup
+// samples the whole source evenly into LDS (one round trip, the same lines for every workgroup), its
+// kSpanTiles tiles find the step they lie in there, and kSpanLanes lanes each narrow it down by a factor of 16
+// per round: four round trips in all for 16M keys. (A wavefront per tile with 64 probes per round takes as many
+// but reads 72 lines a tile.)
+constexpr unsigned kSpanLanes = 16;
+constexpr unsigned kSpanTiles = 64;
+constexpr unsigned kSpanBlock = kSpanTiles * kSpanLanes;
+constexpr unsigned kSpanSamples = 4 * kSpanBlock;
+__global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __restrict__ src, uint64_t n_src,
+                                                            const uint64_t* __restrict__ dst, uint64_t tiles,
+                                                            uint64_t* __restrict__ spans) {
+  __shared__ uint64_t s_sample[kSpanSamples];
+  const uint64_t t = (uint64_t)blockIdx.x * kSpanTiles + threadIdx.x / kSpanLanes;
+  const unsigned lane = threadIdx.x & 63, sub = threadIdx.x % kSpanLanes;
+  const bool live = t < tiles;
+  const uint64_t key = live ? dst[t * kMatchTile] : 0;
+  const uint64_t step = (n_src + kSpanSamples - 1) / kSpanSamples;
+  const unsigned samples = (unsigned)((n_src + step - 1) / step);
+  uint64_t x[kSpanSamples / kSpanBlock];
+#pragma unroll
+  for (unsigned q = 0; q < kSpanSamples / kSpanBlock; ++q) {
+    const unsigned i = q * kSpanBlock + threadIdx.x;
+    x[q] = i < samples ? src[i * step] : 0;
   }
-  const uint64_t key = dst[t * kMatchTile];
+#pragma unroll
+  for (unsigned q = 0; q < kSpanSamples / kSpanBlock; ++q) s_sample[q * kSpanBlock + threadIdx.x] = x[q];
+  if (t == 0 && sub == 0) spans[tiles] = n_src;
+  __syncthreads();
+  unsigned a = 0, b = samples;  // samples before a are below the key, none from b on is
+  while (a < b) {
+    const unsigned mid = (a + b) >> 1;
+    if (s_sample[mid] < key) a = mid + 1; else b = mid;
+  }
   // every source key before lo is below the key, none from hi on is
-  uint64_t lo = 0, hi = n_src;
-  while (lo < hi) {
-    const uint64_t step = (hi - lo + 63) / 64;
-    const uint64_t p = lo + lane * step;
-    const bool below = p < hi && src[p] < key;
-    const unsigned cnt = (unsigned)__popcll(__ballot(below));  // the probes are sorted: the first cnt are below
-    if (cnt == 0) break;
-    const uint64_t next = lo + cnt * step;  // the first probe that is not below, if there is one
-    lo += (cnt - 1) * step + 1;
-    if (cnt < 64 && next < hi) hi = next;
+  uint64_t lo = a ? (a - 1) * step + 1 : 0, hi = a < samples ? a * step : n_src;
+  // (the lanes of a group stay together; a wavefront takes as many rounds as the longest of its groups)
+  while (__any(live && lo < hi)) {
+    const uint64_t stride = (hi - lo + kSpanLanes - 1) / kSpanLanes;
+    const uint64_t p = lo + sub * stride;
+    const bool below = live && p < hi && src[p] < key;
+    // the probes are sorted: the first cnt are below
+    const unsigned cnt =
+        (unsigned)__popcll((__ballot(below) >> (lane / kSpanLanes * kSpanLanes)) & ((1ull << kSpanLanes) - 1));
+    if (cnt == 0) {
+      hi = lo;
+    } else {
+      const uint64_t next = lo + cnt * stride;  // the first probe that is not below, if there is one
+      lo += (cnt - 1) * stride + 1;
+      if (cnt < kSpanLanes && next < hi) hi = next;
+    }
   }
-  if (lane == 0) spans[t] = lo;
+  if (live && sub == 0) spans[t] = lo;
 }
 
-// One workgroup per kMatchTile destination keys. K1: values are single floats and are combined
-// here; otherwise where[i] receives the index of the matching source key, or kNoMatch.
+// One workgroup per kMatchTile destination keys. Bound by memory once the loads do not wait for each other: 12M
+// against 16M keys took 100 us with one source key per lane asked for at a time, 77 with three (5.2 TB/s).
+// K1: values are single floats and are combined here; otherwise where[i] receives the index of the matching
+// source key, or kNoMatch.
 template <bool K1>
 __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __restrict__ src, uint64_t n_src,
                                                             const uint64_t* __restrict__ dst, uint64_t n_dst,
@@ -93,8 +125,9 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
                                                             uint64_t* __restrict__ where,
                                                             const float* __restrict__ src_vals,
                                                             float* __restrict__ dst_vals, int op,
-                                                            unsigned* __restrict__ tile_count) {
+                                                            unsigned long long* __restrict__ counts) {
   __shared__ uint64_t s_keys[kMatchLds];
+  __shared__ float s_vals[K1 ? kMatchLds : 1];
   __shared__ unsigned s_red[kMatchBlock / 64];
   const uint64_t first = (uint64_t)blockIdx.x * kMatchTile;
   const uint64_t tile_n = n_dst - first < kMatchTile ? n_dst - first : kMatchTile;
@@ -115,6 +148,13 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
   }
   const uint64_t lo = spans[blockIdx.x], hi = spans[blockIdx.x + 1];
   const uint64_t span = hi > lo ? hi - lo : 0;  // (hi >= lo when the keys are sorted)
+  // K1: the values follow the keys without waiting for what the search finds: those of the destination are
+  // asked for here (a line of 32 of them without a match is rare), those of a stretch that fits into LDS come
+  // with its keys.
+  const bool vec = K1 && whole && (reinterpret_cast<uintptr_t>(dst_vals) & 15) == 0;
+  const bool vals_here = K1 && span <= kMatchLds;
+  f32x4 mine = (f32x4)(0.f);
+  if (vec) mine = *reinterpret_cast<const f32x4*>(dst_vals + i0);
   // The stretch goes through LDS in pieces of kMatchLds keys. A key is looked up in the first
   // piece whose last key is not below it (or in the last piece).
   const bool staged = span <= (uint64_t)kMatchLds * kMatchPieces;
@@ -130,7 +170,24 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
       const unsigned len = span - base < kMatchLds ? (unsigned)(span - base) : kMatchLds;
       const bool last_piece = base + len == span;
       if (base) __syncthreads();  // everyone is done with the piece before
-      for (unsigned t = threadIdx.x; t < len; t += kMatchBlock) s_keys[t] = src[lo + base + t];
+      // (all loads of a turn before the first of them is waited for)
+      for (unsigned t0 = threadIdx.x; t0 < len; t0 += kMatchBlock * kMatchTurn) {
+        uint64_t ks[kMatchTurn];
+        float vs[kMatchTurn];
+#pragma unroll
+        for (unsigned q = 0; q < kMatchTurn; ++q) {
+          const unsigned t = t0 + q * kMatchBlock;
+          ks[q] = t < len ? src[lo + base + t] : 0;
+          vs[q] = vals_here && t < len ? src_vals[lo + base + t] : 0.0f;
+        }
+#pragma unroll
+        for (unsigned q = 0; q < kMatchTurn; ++q) {
+          const unsigned t = t0 + q * kMatchBlock;
+          if (t >= len) continue;
+          s_keys[t] = ks[q];
+          if (vals_here) s_vals[t] = vs[q];
+        }
+      }
       __syncthreads();
       const uint64_t top = s_keys[len - 1];
       unsigned pos = 0;     // the lane's open keys are above every source key before this one
@@ -170,21 +227,15 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
 #pragma unroll
   for (unsigned r = 0; r < kMatchItems; ++r) found += j[r] != kNoMatch ? 1u : 0u;
   if (K1) {
-    const bool vec = whole && (reinterpret_cast<uintptr_t>(dst_vals) & 15) == 0;
-    float d[kMatchItems] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (vec) {
-      if (op != PSKV_OP_ASSIGN || (found && found != kMatchItems)) {  // what is combined, or what stays
-        const f32x4 v = *reinterpret_cast<const f32x4*>(dst_vals + i0);
-        d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
-      }
-    } else if (op != PSKV_OP_ASSIGN) {
+    float d[kMatchItems] = {mine.x, mine.y, mine.z, mine.w};
+    if (!vec && op != PSKV_OP_ASSIGN) {
 #pragma unroll
       for (unsigned r = 0; r < kMatchItems; ++r)
         if (j[r] != kNoMatch) d[r] = dst_vals[i0 + r];
     }
 #pragma unroll
     for (unsigned r = 0; r < kMatchItems; ++r)
-      if (j[r] != kNoMatch) d[r] = combine(op, d[r], src_vals[j[r]]);
+      if (j[r] != kNoMatch) d[r] = combine(op, d[r], vals_here ? s_vals[j[r] - lo] : src_vals[j[r]]);
     if (vec) {
       if (found) {
         f32x4 v;
@@ -215,32 +266,25 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
   if (threadIdx.x == 0) {
     unsigned total = 0;
     for (unsigned w = 0; w < kMatchBlock / 64; ++w) total += s_red[w];
-    tile_count[blockIdx.x] = total;  // (thousands of atomic adds on one counter would take turns)
+    // (spread over kCounts lines: adds on one address take turns)
+    if (total) atomicAdd(&counts[(blockIdx.x % kCounts) * kCountStride], (unsigned long long)total);
   }
 }
 
-// The matched keys of all tiles: one workgroup of 1024 threads, four loads in flight per thread.
-constexpr unsigned kTotalBlock = 1024;
-__global__ __launch_bounds__(kTotalBlock) void k_match_total(const unsigned* __restrict__ tile_count, uint64_t tiles,
-                                                             unsigned long long* __restrict__ count) {
-  __shared__ unsigned long long s_sum[kTotalBlock / 64];
-  unsigned long long sum = 0;
-  for (uint64_t t = threadIdx.x; t < tiles; t += 4 * kTotalBlock) {
-    const unsigned a = tile_count[t];
-    const unsigned b = t + kTotalBlock < tiles ? tile_count[t + kTotalBlock] : 0;
-    const unsigned c = t + 2 * kTotalBlock < tiles ? tile_count[t + 2 * kTotalBlock] : 0;
-    const unsigned d = t + 3 * kTotalBlock < tiles ? tile_count[t + 3 * kTotalBlock] : 0;
-    sum += (unsigned long long)a + b + c + d;
-  }
+// The matched keys of all tiles, for the host to see, and the counts clear for the next call. One wavefront,
+// behind the kernels of the match: when `done` shows `seq`, what those have written is there.
+struct MatchDone {
+  unsigned long long count, seq;
+};
+__global__ void k_match_total(unsigned long long* counts, MatchDone* done, unsigned long long seq) {
+  static_assert(kCounts == 64, "one lane per count");
+  unsigned long long x = counts[threadIdx.x * kCountStride];
+  counts[threadIdx.x * kCountStride] = 0ull;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-  if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long total = 0;
-    for (unsigned w = 0; w < kTotalBlock / 64; ++w) total += s_sum[w];
-    *count = total;
-  }
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+  if (threadIdx.x != 0) return;
+  done->count = x;
+  __hip_atomic_store(&done->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Rows of kq units (floats, or groups of four floats): dst row i op= src row where[i].
@@ -274,12 +318,14 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_rows(const uint64_t* __re
 struct MatchCtx {
   std::mutex mu;
   hipStream_t stream = nullptr;
-  unsigned long long* count_host = nullptr;  // pinned; the kernel that adds the tiles up writes it
+  MatchDone* done = nullptr;            // pinned; the last kernel of a call writes it
+  unsigned long long seq = 0;           // number of the newest call
+  unsigned long long* counts = nullptr;  // kCounts lines, zero between calls
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // begin/end of the key kernel and of the row kernel
   struct Buf {
     void* ptr = nullptr;
     size_t cap = 0;
-  } where, spans, tile_count, stage[4];
+  } where, spans, stage[4];
 };
 
 int room(MatchCtx::Buf* b, size_t bytes, hipStream_t stream) {
@@ -306,18 +352,21 @@ MatchCtx* match_ctx(int device, bool create = true) {
   MatchCtx* c = new (std::nothrow) MatchCtx();  // kept until the process ends
   if (!c) return nullptr;
   bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
-  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&c->count_host), sizeof(unsigned long long),
-                           hipHostMallocDefault) == hipSuccess;
+  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&c->done), sizeof(MatchDone), hipHostMallocCoherent) == hipSuccess;
+  ok = ok && hipMalloc(reinterpret_cast<void**>(&c->counts), kCounts * kCountStride * 8) == hipSuccess;
+  ok = ok && hipMemset(c->counts, 0, kCounts * kCountStride * 8) == hipSuccess;
   for (int e = 0; ok && e < 4; ++e) ok = hipEventCreate(&c->ev[e]) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     for (int e = 0; e < 4; ++e)
       if (c->ev[e]) (void)hipEventDestroy(c->ev[e]);
-    if (c->count_host) (void)hipHostFree(c->count_host);
+    if (c->done) (void)hipHostFree(c->done);
+    if (c->counts) (void)hipFree(c->counts);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return nullptr;
   }
+  c->done->seq = 0;
   table[device] = c;
   return c;
 }
@@ -332,7 +381,7 @@ int match_trim(int device) {
   DeviceGuard guard(device);
   if (!guard.ok()) return set_error(PSKV_EHIP, "cannot select device %d", device);
   std::lock_guard<std::mutex> lk(c->mu);
-  MatchCtx::Buf* bufs[] = {&c->where, &c->spans, &c->tile_count, &c->stage[0], &c->stage[1], &c->stage[2], &c->stage[3]};
+  MatchCtx::Buf* bufs[] = {&c->where, &c->spans, &c->stage[0], &c->stage[1], &c->stage[2], &c->stage[3]};
   for (MatchCtx::Buf* b : bufs) {
     if (b->ptr) PSKV_HIP(hipFree(b->ptr));
     b->ptr = nullptr;
@@ -389,25 +438,20 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
     if (rc) return rc;
   }
   uint64_t* spans = static_cast<uint64_t*>(c->spans.ptr);
-  {
-    int rc = room(&c->tile_count, (size_t)blocks * sizeof(unsigned), st);
-    if (rc) return rc;
-  }
-  unsigned* tile_count = static_cast<unsigned*>(c->tile_count.ptr);
-  hipLaunchKernelGGL(k_match_spans, dim3(blocks / (kMatchBlock / 64) + 1), dim3(kMatchBlock), 0, st, d_src, (uint64_t)n_src,
-                     d_dst, (uint64_t)blocks, spans);
+  hipLaunchKernelGGL(k_match_spans, dim3((blocks + kSpanTiles - 1) / kSpanTiles), dim3(kSpanBlock), 0, st, d_src,
+                     (uint64_t)n_src, d_dst, (uint64_t)blocks, spans);
   // (a launch can carry events of its own, which read the begin and the end of that very dispatch)
   hipEvent_t e0 = kernel_ms ? c->ev[0] : nullptr, e1 = kernel_ms ? c->ev[1] : nullptr;
   hipEvent_t e2 = kernel_ms ? c->ev[2] : nullptr, e3 = kernel_ms ? c->ev[3] : nullptr;
   if (k == 1) {
     hipExtLaunchKernelGGL(k_match_keys<true>, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, d_src, (uint64_t)n_src, d_dst,
-                       (uint64_t)n_dst, spans, static_cast<uint64_t*>(nullptr), d_sv, d_dv, op, tile_count);
+                       (uint64_t)n_dst, spans, static_cast<uint64_t*>(nullptr), d_sv, d_dv, op, c->counts);
   } else {
     int rc = room(&c->where, n_dst * sizeof(uint64_t), st);
     if (rc) return rc;
     uint64_t* where = static_cast<uint64_t*>(c->where.ptr);
     hipExtLaunchKernelGGL(k_match_keys<false>, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, d_src, (uint64_t)n_src, d_dst,
-                       (uint64_t)n_dst, spans, where, d_sv, d_dv, op, tile_count);
+                       (uint64_t)n_dst, spans, where, d_sv, d_dv, op, c->counts);
     const bool vec = k % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_sv) | reinterpret_cast<uintptr_t>(d_dv)) & 15) == 0;
     const uint64_t kq = vec ? k / 4 : k;
     const unsigned grid = grid_for(n_dst * kq, kMatchBlock, 1u << 20);
@@ -419,12 +463,13 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
                          d_dv, op);
     }
   }
-  hipLaunchKernelGGL(k_match_total, dim3(1), dim3(kTotalBlock), 0, st, tile_count, (uint64_t)blocks, c->count_host);
+  const unsigned long long seq = ++c->seq;
+  hipLaunchKernelGGL(k_match_total, dim3(1), dim3(64), 0, st, c->counts, c->done, seq);
   PSKV_HIP(hipGetLastError());
   if (memkind == PSKV_MEM_HOST)
     PSKV_HIP(hipMemcpyAsync(dst_vals, d_dv, n_dst * k * 4, hipMemcpyDeviceToHost, st));
-  PSKV_HIP(hipStreamSynchronize(st));
-  if (matched) *matched = (uint64_t)*static_cast<volatile unsigned long long*>(c->count_host) * k;  // values, not keys (:52)
+  if (memkind == PSKV_MEM_HOST || kernel_ms || !seen_in_time(&c->done->seq, seq)) PSKV_HIP(hipStreamSynchronize(st));
+  if (matched) *matched = (uint64_t)c->done->count * k;  // values, not keys (:52)
   if (kernel_ms) {
     PSKV_HIP(hipEventElapsedTime(&kernel_ms[0], c->ev[0], c->ev[1]));
     if (k > 1) PSKV_HIP(hipEventElapsedTime(&kernel_ms[1], c->ev[2], c->ev[3]));

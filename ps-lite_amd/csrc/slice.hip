@@ -2,7 +2,6 @@
 // (include/ps/kv_app.h:517-572) and the device-side reassembly of pulled slices
 // that mirrors the callback of KVWorker::AddPullCB (kv_app.h:663-714).
 #include <algorithm>
-#include <chrono>
 #include <cstring>
 #include <limits>
 #include <mutex>
@@ -361,17 +360,6 @@ __global__ __launch_bounds__(kBlock) void k_concat(const Segment* __restrict__ s
 // Per-call state of the slicer. Calls may come from any thread at once
 // (KVWorker::Push is thread-safe, kv_app.h:101-104), so each call takes a context
 // of its own from a pool and returns it afterwards.
-// Watches a word of pinned host memory for `want` for up to about 200 us; false when it did
-// not show up in that time (the caller then waits for the stream as usual).
-bool seen_in_time(const unsigned long long* word, unsigned long long want) {
-  const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-  for (;;) {
-    for (int spin = 0; spin < 256; ++spin)
-      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return true;
-    if (std::chrono::steady_clock::now() > give_up) return false;
-  }
-}
-
 struct SliceCtx {
   unsigned long long calls = 0;  // numbers the calls whose completion the host watches for
   int device = -1;

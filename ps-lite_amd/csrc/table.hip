@@ -414,17 +414,6 @@ void adopt_state(pskv_table* t) {
   t->pend_keys = t->pend_units = 0;
 }
 
-// Watches a word of pinned host memory for `want` for up to about 200 us; false when it did not show up
-// in that time (the caller then waits for the stream as usual). A stream wait costs about 5 us more.
-bool seen_in_time(const unsigned long long* word, unsigned long long want) {
-  const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-  for (;;) {
-    for (int spin = 0; spin < 256; ++spin)
-      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return true;
-    if (std::chrono::steady_clock::now() > give_up) return false;
-  }
-}
-
 // Reads the device state of up to kMaxBatch tables on one stream, with one launch and one wait. `watch`: what the
 // caller wants to see afterwards lies in pinned memory (the state itself, answers that kernels have written
 // there): it is enough that this kernel, the last one on the stream, has run.

@@ -107,3 +107,21 @@ def test_match_at_the_size_of_a_model(capi, dev):
         d_self = torch.ones(dk.size * k, dtype=torch.float32, device=dev)
         assert capi.match(d_dk, d_dv, d_dk, d_self, k, capi.OP_TIMES) == dk.size * k
         assert_bits_equal(from_dev(d_self), once, "a key set against itself, k=%d" % k)
+
+
+@pytest.mark.parametrize("n_src,n_dst", [(1536, 1024), (1537, 1024), (1535, 1025), (4096, 65536), (4097, 65537),
+                                         (200_000, 66_000), (3072 * 4, 1024), (20_000, 1024)])
+def test_match_edges_of_stretches(capi, orc, dev, n_src, n_dst):
+    """Source stretches at the edges of what a workgroup stages in LDS with its values (1,536 keys), of the
+    sampled search (4,096 samples, 64 tiles of 1,024 destination keys), and called twice: the counters of one call
+    are clear for the next."""
+    announce("match_stretches", n_src, n_dst)
+    rng = np.random.default_rng(n_src + n_dst)
+    sk, dk = key_sets(rng, n_src, n_dst, min(n_src, n_dst) // 2)
+    sv, dv = values(rng, sk.size, 1), values(rng, dk.size, 1)
+    for op in (0, 1):
+        _, want, want_n = orc.ordered_match(sk, sv, dk, dv, 1, op)
+        for _ in range(2):
+            got, n = run(capi, dev, "device", sk, sv, dk, dv, 1, op)
+            assert n == want_n
+            assert_bits_equal(got, want, "op %d" % op)
