@@ -860,7 +860,7 @@ struct KernelSet {
 // A launch as pskv_replay_record keeps it: everything it takes to make it again.
 struct SavedLaunch {
   const void* kernel;
-  dim3 grid;
+  dim3 grid, block;
   ReqBatch<kMaxBatch> rb;  // (the kernel takes as much of it as its size says)
 };
 // Where launch_batch leaves a copy of its launches while a request is being recorded (the thread
@@ -870,7 +870,7 @@ thread_local std::vector<SavedLaunch>* g_recording = nullptr;
 // One launch for the whole batch: blockIdx.y selects the table, `nblk_of` says how many
 // workgroups serve each (0: none, the table sits this step out).
 template <typename F>
-int launch_batch(Batch& bt, int prof_kernel, const KernelSet& kernels, F nblk_of) {
+int launch_batch(Batch& bt, int prof_kernel, const KernelSet& kernels, F nblk_of, unsigned threads = kBlock) {
   SavedLaunch l;
   const size_t room = bt.size() <= 1 ? 1 : bt.size() <= 4 ? 4 : kMaxBatch;
   l.kernel = room == 1 ? kernels.one : room == 4 ? kernels.four : kernels.most;
@@ -884,8 +884,9 @@ int launch_batch(Batch& bt, int prof_kernel, const KernelSet& kernels, F nblk_of
   }
   if (!gx) return PSKV_OK;
   l.grid = dim3((unsigned)gx, (unsigned)bt.size());
+  l.block = dim3(threads);
   void* args[] = {&l.rb};
-  PSKV_HIP(launch_args(lead_of(bt), prof_kernel, l.kernel, l.grid, dim3(kBlock), 0, args));
+  PSKV_HIP(launch_args(lead_of(bt), prof_kernel, l.kernel, l.grid, l.block, 0, args));
   if (g_recording) g_recording->push_back(l);
   return PSKV_OK;
 }
@@ -1073,7 +1074,23 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   }
   if (!n_largest) return PSKV_OK;
   int rc;
-  if (any_cache) {
+  // a recorded repeat, where the workgroups that compare it can wait for each other: one launch
+  unsigned repeat_quads = 0;
+  auto repeat_groups = [&](const Item& it) -> uint64_t {
+    const uint64_t per = (uint64_t)kRepeatBlock * 4 * repeat_quads;
+    return (it.d.n + per - 1) / per;
+  };
+  if (bt[0].r.replay == kReplayCapture) {
+    for (unsigned quads : {kRepeatFew, kRepeatMany}) {
+      uint64_t groups = 0;
+      repeat_quads = quads;
+      for (const Item& it : bt) groups += repeat_groups(it);
+      if (groups <= kRepeatGroups) break;
+      repeat_quads = 0;
+    }
+  }
+  const bool one_launch = repeat_quads != 0;
+  if (any_cache && !one_launch) {
     rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
       return (it.d.cache_mode == kCacheOn && it.tag.try_cache)
                  ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems) : 0ull;
@@ -1100,7 +1117,14 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   if (any_cache) {
     for (Item& it : bt) it.r.done = nullptr;  // (the word of such a launch says how the comparison went)
   }
-  if (push && pull) {
+  if (one_launch) {
+    const bool few = repeat_quads == kRepeatFew;
+    const KernelSet kernels =
+        push && pull ? (few ? PSKV_KSET_OF(k_scalar_repeat, true, true, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, true, true, kRepeatMany))
+        : push       ? (few ? PSKV_KSET_OF(k_scalar_repeat, true, false, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, true, false, kRepeatMany))
+                     : (few ? PSKV_KSET_OF(k_scalar_repeat, false, true, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, false, true, kRepeatMany));
+    rc = launch_batch(bt, push ? PSKV_KERNEL_PUSH_SCALAR : PSKV_KERNEL_PULL_SCALAR, kernels, repeat_groups, kRepeatBlock);
+  } else if (push && pull) {
     rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, true, false), nblk)
          : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, true), nblk)
                    : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, false), nblk);
@@ -2180,7 +2204,7 @@ int pskv_replay_run(pskv_replay* r) {
   }
   for (SavedLaunch& l : r->launches) {
     void* args[] = {&l.rb};
-    PSKV_HIP(hipLaunchKernel(l.kernel, l.grid, dim3(kBlock), args, 0, r->stream));
+    PSKV_HIP(hipLaunchKernel(l.kernel, l.grid, l.block, args, 0, r->stream));
   }
   return PSKV_OK;
 }

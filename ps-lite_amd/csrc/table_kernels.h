@@ -393,6 +393,109 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch<TABLES> b) {
     decide_same(st, tag, (atomicExch(&st->req_flags, 0u) & kReqDiffer) == 0u && cache_usable(st, tag), d.outcome);
 }
 
+// A recorded SCALAR request of up to kRepeatGroups workgroups: comparison and values in ONE launch. Nothing
+// may change or be answered before every key of the table's share is known to be the cached one, so the
+// workgroups of a table wait for each other in between: all loads are under way by then, and the wait (an atomic
+// and a look at its outcome) is shorter than the end of one kernel and the start of the next (4 tables of 25,000
+// keys: 4.6 + 3.6 us and the gap between them, now 5.7; the calling thread makes one launch instead of two, and a
+// recorded step 8.8 -> 4.2 us).
+// All workgroups have to be on the GPU together: 64 of 1,024 threads are an eighth of what it holds, so twice as
+// many such launches fit side by side as a process has hardware queues to run them from. A workgroup whose wait
+// does not end within about a second all the same (kRepeatSpins) applies nothing and leaves the replay error.
+constexpr unsigned kRepeatBlock = 1024;
+constexpr unsigned kRepeatGroups = 64;
+constexpr unsigned kRepeatSpins = 1u << 20;
+// Quads of keys per thread: one while the request fits into kRepeatGroups workgroups that way (262,144 keys), two
+// up to twice that; beyond it the two kernels that fill the GPU are as quick (with four quads the registers spill).
+constexpr unsigned kRepeatFew = 1, kRepeatMany = 2;
+typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool PUSH, bool PULL, unsigned QUADS, int TABLES>
+__global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(ReqBatch<TABLES> b) {
+  const TableReq& d = b.t[blockIdx.y];
+  const unsigned nblk = d.nblk;
+  if (blockIdx.x >= nblk) return;
+  DevState* st = d.st;
+  const ReqTag tag = d.tag;
+  __shared__ unsigned s_same;
+  unsigned long long before = 0;  // (nobody changes the verdict before this workgroup has arrived)
+  if (threadIdx.x == 0)
+    before = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint64_t n = d.n;
+  const uint64_t first = ((uint64_t)blockIdx.x * kRepeatBlock * QUADS + threadIdx.x) * 4;
+  f32x4 cur[QUADS], add[QUADS];
+  u64x2u x0[QUADS], x1[QUADS];
+  u64x2 y0[QUADS], y1[QUADS];
+#pragma unroll
+  for (unsigned q = 0; q < QUADS; ++q) {
+    const uint64_t i = first + (uint64_t)q * kRepeatBlock * 4;
+    cur[q] = add[q] = (f32x4)(0.f);
+    x0[q] = x1[q] = (u64x2u)(0ull);
+    y0[q] = y1[q] = (u64x2)(0ull);
+    if (i + 4 <= n) {
+      x0[q] = *reinterpret_cast<const u64x2u*>(d.keys + i), x1[q] = *reinterpret_cast<const u64x2u*>(d.keys + i + 2);
+      y0[q] = *reinterpret_cast<const u64x2*>(d.cache_keys + i);
+      y1[q] = *reinterpret_cast<const u64x2*>(d.cache_keys + i + 2);
+      cur[q] = *reinterpret_cast<const f32x4*>(d.arena + i);
+      if (PUSH) add[q] = *reinterpret_cast<const f32x4u*>(d.vals + i);
+    } else {
+#pragma unroll
+      for (unsigned j = 0; j < 4; ++j) {
+        if (i + j >= n) continue;
+        const uint64_t x = d.keys[i + j], y = d.cache_keys[i + j];
+        if (j < 2) x0[q][j] = x, y0[q][j] = y; else x1[q][j - 2] = x, y1[q][j - 2] = y;
+        cur[q][j] = d.arena[i + j];
+        if (PUSH) add[q][j] = d.vals[i + j];
+      }
+    }
+  }
+  bool differ = false;
+#pragma unroll
+  for (unsigned q = 0; q < QUADS; ++q)
+    differ |= x0[q].x != y0[q].x || x0[q].y != y0[q].y || x1[q].x != y1[q].x || x1[q].y != y1[q].y;
+  const bool any = __syncthreads_or(differ ? 1 : 0) != 0;
+  if (threadIdx.x == 0) {
+    const unsigned old = atomicAdd(&st->repeat_arrived, any ? 0x10001u : 1u);
+    bool same = false;
+    if ((old & 0xffffu) == nblk - 1) {
+      same = !any && (old >> 16) == 0u && cache_usable(st, tag);
+      decide_same(st, tag, same, d.outcome);
+      if (PUSH && same) st->dirty_epoch = tag.epoch;  // the slots fall behind
+      st->repeat_arrived = 0u;
+      __hip_atomic_store(&st->repeat_verdict, ((before >> 1) + 1) << 1 | (same ? 1ull : 0ull), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      unsigned long long now = before;
+      for (unsigned spin = 0; spin < kRepeatSpins; ++spin) {
+        now = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (now != before) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      same = now != before && (now & 1ull) != 0ull;
+      if (now == before) atomicOr(&st->error, kDevErrReplay);
+    }
+    s_same = same ? 1u : 0u;
+  }
+  __syncthreads();
+  if (!s_same) return;
+#pragma unroll
+  for (unsigned q = 0; q < QUADS; ++q) {
+    const uint64_t i = first + (uint64_t)q * kRepeatBlock * 4;
+    if (PUSH) cur[q] = cur[q] + add[q];
+    if (i + 4 <= n) {
+      if (PULL) *reinterpret_cast<f32x4u*>(d.out + i) = cur[q];
+      if (PUSH) *reinterpret_cast<f32x4*>(d.arena + i) = cur[q];
+    } else {
+#pragma unroll
+      for (unsigned j = 0; j < 4; ++j) {
+        if (i + j >= n) continue;
+        if (PULL) d.out[i + j] = cur[q][j];
+        if (PUSH) d.arena[i + j] = cur[q][j];
+      }
+    }
+  }
+}
+
 // The counter record of a request, written by the kernel that creates its keys once every
 // workgroup has taken its rows (or at once when the request creates nothing): the record then
 // holds the counters as they are AFTER the request. Every thread of the workgroup calls it;
@@ -524,7 +627,6 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch<TABLES> b) {
 
 // Four consecutive keys of a request with a word each, starting at index `at`: 128-bit loads where all four are
 // there (keys on any 8-byte, words on any 4-byte boundary), `fill` and zero keys past the end.
-typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
 template <typename W>
 struct FourKeys {
   uint64_t k[4];
@@ -924,7 +1026,6 @@ constexpr int kOpGather = 1;
 // Four (three, two) floats that start at any float. STREAM selects non-temporal accesses: a
 // request far larger than the caches is read and written once per launch, and telling
 // the memory system so is worth 10-15 % of bandwidth on this GPU.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x3u __attribute__((ext_vector_type(3), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 template <bool STREAM>

@@ -316,3 +316,38 @@ def test_replay_misuse_is_a_status_code(capi, dev):
     assert torch.equal(out, vals) and torch.equal(out_lens, lens)
     rec.close()
     g.close()
+
+
+@pytest.mark.parametrize("S,n", [(1, 1), (1, 3), (1, 4095), (1, 4097), (1, 262_144), (1, 262_145), (4, 262_140),
+                                 (1, 524_287), (1, 524_289)])
+@pytest.mark.parametrize("how", [0, 4])
+def test_scalar_repeats_at_the_edges_of_their_launches(capi, orc, dev, S, n, how):
+    """One launch with one quad of keys per thread, with two, and the two kernels behind; a last key that differs,
+    in the last workgroup, stops all of the table's."""
+    announce("replay_edges", S, n, how)
+    rng = np.random.default_rng(n)
+    g, o = capi.Group(S, MODES["scalar"]), orc.Store(MODES["scalar"], 0)
+    keys = unique_keys(rng, n, S)
+    st = _Step(capi, dev, rng, "scalar", S, keys, None, n)
+    vals = rng.normal(0, 1, size=n).astype(np.float32)
+    st.set_vals(vals)
+    rec = g.record(capi.REPLAY_PUSH | capi.REPLAY_PULL | how, st.dk, st.pos, st.dv, st.vpos, out=st.out, out_pos=st.out_pos)
+    for _ in range(4):
+        rec.run()
+    for _ in range(5):
+        o.push(keys, vals)
+    g.sync()
+    assert_bits_equal(st.answered(), o.pull(keys)[0], "repeats")
+    st.dk[n - 1] = st.dk[n - 1] + 1
+    st.set_vals(vals)
+    rec.run()
+    with pytest.raises(capi.PskvError) as e:
+        g.sync()
+    assert e.value.code == capi.ESTALE
+    assert np.all(st.answered()[int(st.pos[S - 1]):] == 7.0)
+    rest = slice(0, int(st.pos[S - 1]))
+    if rest.stop:
+        o.push(keys[rest], vals[rest])
+    rec.close()
+    _check_dump(g, o, "after a repeat with another key")
+    g.close()
