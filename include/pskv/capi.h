@@ -174,8 +174,8 @@ int pskv_sync_multi(pskv_table* const* tables, size_t S);
  * arguments (device memory only; out_vals, out_pos and out_lens as pskv_pull_multi's out,
  * out_pos and out_lens; a PSKV_MODE_VARLEN response that does not fit is reported by the next
  * sync), waits for it, and keeps the launches that a repeat of it takes as a HIP graph on the
- * tables' stream (which must not be the null stream), or, with PSKV_REPLAY_LAUNCHES, as the
- * launches themselves. It allocates and waits; it is a set-up call.
+ * tables' stream (which must not be the null stream), or, with PSKV_REPLAY_LAUNCHES or where they are so
+ * few that a graph would cost more, as the launches themselves. It allocates and waits; it is a set-up call.
  * pskv_replay_run enqueues that graph (makes those launches again): the request is applied
  * again, to whatever the value buffers hold by the time the stream gets to it (keys, lens, positions and addresses are part
  * of the recording). It allocates nothing, waits for nothing and reads nothing back: the host

@@ -2101,10 +2101,14 @@ int pskv_pull_multi(pskv_table* const* tables, size_t S, const uint64_t* keys, c
                        out_nvals, memkind);
 }
 
+// Up to so many launches are made again one by one whatever the caller asked for: they take the calling thread
+// 2.7 us each, a graph of one or two kernels 16 us.
+constexpr size_t kGraphLaunches = 5;
+
 struct pskv_replay {
   std::vector<pskv_table*> tables;
   std::vector<uint64_t> gen;  // pskv_table::gen of each when the recording was made
-  std::vector<SavedLaunch> launches;  // PSKV_REPLAY_LAUNCHES: made again one by one instead of as a graph
+  std::vector<SavedLaunch> launches;  // made again one by one: PSKV_REPLAY_LAUNCHES, or few of them
   hipGraphExec_t exec = nullptr;
   hipStream_t stream = nullptr;
   int device = 0;
@@ -2117,7 +2121,6 @@ int pskv_replay_record(pskv_replay** out, pskv_table* const* tables, size_t S, i
   if (!out) return set_error(PSKV_EINVAL, "null argument");
   *out = nullptr;
   const bool push = (what & PSKV_REPLAY_PUSH) != 0, pull = (what & PSKV_REPLAY_PULL) != 0;
-  const bool as_graph = (what & PSKV_REPLAY_LAUNCHES) == 0;
   if ((!push && !pull) || (what & ~(PSKV_REPLAY_PUSH | PSKV_REPLAY_PULL | PSKV_REPLAY_LAUNCHES)))
     return set_error(PSKV_EINVAL, "what = %d names neither a push nor a pull", what);
   if (S == 0) return set_error(PSKV_EINVAL, "no tables");
@@ -2174,6 +2177,7 @@ int pskv_replay_record(pskv_replay** out, pskv_table* const* tables, size_t S, i
     (void)hipGraphDestroy(graph);
     return set_error(PSKV_ENOMEM, "out of host memory");
   }
+  const bool as_graph = (what & PSKV_REPLAY_LAUNCHES) == 0 && saved.size() > kGraphLaunches;
   const hipError_t ei = as_graph ? hipGraphInstantiate(&r->exec, graph, nullptr, nullptr, 0) : hipSuccess;
   (void)hipGraphDestroy(graph);
   if (ei != hipSuccess) {
