@@ -27,7 +27,7 @@ class Stager {
   static constexpr int kStreams = 2;          // streams that the copy commands alternate between
   static constexpr int kStretch = 8;          // pieces that the consumer of a transfer takes at a time
   static constexpr int kWorkers = 8;          // threads that copy between caller memory and the ring
-  static constexpr int kParts = 4;            // a piece is copied in this many parts, by as many workers
+  static constexpr int kParts = 8;            // a piece is copied in this many parts, by as many workers
 
   // The stager of `device`, created on first use and kept until the process ends; nullptr when
   // its pinned memory cannot be had (the caller then falls back to plain copy commands).

@@ -1,7 +1,11 @@
 // The ring of pinned pieces and the worker threads behind Stager (stager.h).
 #include "stager.h"
 
+#include <emmintrin.h>
+
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <deque>
@@ -13,6 +17,28 @@
 #include "host_common.h"
 
 namespace pskv {
+
+// memcpy whose stores go past the caches: what it writes is read by the copy engine, or by the caller a while
+// later, and stores through the caches read every line from memory before they write it.
+static void copy_past_caches(void* dst, const void* src, size_t len) {
+  char* d = static_cast<char*>(dst);
+  const char* s = static_cast<const char*>(src);
+  const size_t head = std::min(len, (size_t)(-reinterpret_cast<uintptr_t>(d) & 63));
+  std::memcpy(d, s, head);
+  d += head, s += head, len -= head;
+  for (; len >= 64; d += 64, s += 64, len -= 64) {
+    const __m128i a = _mm_loadu_si128(reinterpret_cast<const __m128i*>(s));
+    const __m128i b = _mm_loadu_si128(reinterpret_cast<const __m128i*>(s + 16));
+    const __m128i c = _mm_loadu_si128(reinterpret_cast<const __m128i*>(s + 32));
+    const __m128i e = _mm_loadu_si128(reinterpret_cast<const __m128i*>(s + 48));
+    _mm_stream_si128(reinterpret_cast<__m128i*>(d), a);
+    _mm_stream_si128(reinterpret_cast<__m128i*>(d + 16), b);
+    _mm_stream_si128(reinterpret_cast<__m128i*>(d + 32), c);
+    _mm_stream_si128(reinterpret_cast<__m128i*>(d + 48), e);
+  }
+  std::memcpy(d, s, len);
+  _mm_sfence();
+}
 
 struct Stager::Impl {
   int device = 0;
@@ -35,51 +61,75 @@ struct Stager::Impl {
   std::mutex mu;
   std::condition_variable cv_job, cv_done;
   std::deque<Job> jobs;
-  int pending[kSlots] = {0};  // parts of the slot's piece that workers still owe
+  std::atomic<int> queued{0};                 // jobs.size()
+  std::atomic<int> pending[kSlots] = {};      // parts of the slot's piece that workers still owe
+  std::atomic<int> sleepers{0}, waiters{0};   // threads in cv_job and cv_done
 
   char* slot_ptr(int s) const { return ring + (size_t)s * kPiece; }
 
+  // Looks for `ready` for about 100 us before a thread goes to sleep: the next piece, or the next transfer, is
+  // mostly nearer than that, and waking a thread costs the start and the end of a transfer 30 to 50 us each.
+  template <typename F>
+  static bool look_for(F ready) {
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+    do {
+      for (int spin = 0; spin < 64; ++spin) {
+        if (ready()) return true;
+        __builtin_ia32_pause();
+      }
+    } while (std::chrono::steady_clock::now() < until);
+    return ready();
+  }
+
   void work() {
     for (;;) {
+      (void)look_for([&] { return queued.load() > 0; });
       Job j;
       {
         std::unique_lock<std::mutex> lk(mu);
-        cv_job.wait(lk, [&] { return !jobs.empty(); });
+        if (jobs.empty()) {
+          ++sleepers;
+          cv_job.wait(lk, [&] { return !jobs.empty(); });
+          --sleepers;
+        }
         j = jobs.front();
         jobs.pop_front();
+        --queued;
       }
-      std::memcpy(j.dst, j.src, j.len);
-      bool last;
-      {
+      copy_past_caches(j.dst, j.src, j.len);
+      // (a waiter counts itself in before it looks at `pending` for the last time)
+      if (--pending[j.slot] == 0 && waiters.load() > 0) {
         std::lock_guard<std::mutex> lk(mu);
-        last = --pending[j.slot] == 0;
+        cv_done.notify_all();
       }
-      if (last) cv_done.notify_all();
     }
   }
-  // A piece is copied in kParts parts by as many workers: it is ready (or gone) in a quarter of
+  // A piece is copied in kParts parts by as many workers: it is ready (or gone) in an eighth of
   // the time, which is what a transfer of a few dozen pieces waits for at its start and its end.
   void submit(void* dst, const void* src, size_t len, int slot) {
     const size_t part = ((len + kParts - 1) / kParts + 4095) & ~(size_t)4095;
-    int n = 0;
+    if (len == 0) return;
+    bool wake;
     {
       std::lock_guard<std::mutex> lk(mu);
+      int n = 0;
       for (size_t at = 0; at < len; at += part, ++n)
         jobs.push_back(Job{static_cast<char*>(dst) + at, static_cast<const char*>(src) + at,
                            std::min(part, len - at), slot});
       pending[slot] = n;
+      queued += n;
+      wake = sleepers.load() > 0;
     }
-    if (n == 0) return;
-    cv_job.notify_all();
+    if (wake) cv_job.notify_all();
   }
   void wait_slot(int slot) {
+    if (look_for([&] { return pending[slot].load() == 0; })) return;
     std::unique_lock<std::mutex> lk(mu);
-    cv_done.wait(lk, [&] { return pending[slot] == 0; });
+    ++waiters;
+    cv_done.wait(lk, [&] { return pending[slot].load() == 0; });
+    --waiters;
   }
-  bool slot_free(int slot) {
-    std::lock_guard<std::mutex> lk(mu);
-    return pending[slot] == 0;
-  }
+  bool slot_free(int slot) { return pending[slot].load() == 0; }
 };
 
 Stager* Stager::get(int device) {

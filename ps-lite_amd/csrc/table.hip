@@ -1804,6 +1804,7 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
                             r.out < reinterpret_cast<float*>(t->small_out + kSmallBytes);
     const bool lens_pinned = r.out_lens == reinterpret_cast<int32_t*>(t->small_out);
     Stager* sg = Stager::get(t->device);
+    bool copying = false;  // a copy command of its own is on the stream
     if (pull && r.out_nvals && !out_pinned) {
       if (r.gather_deferred || (sg && r.out_nvals * 4 >= kPipeBytes && !host_pool_owns(out, r.out_nvals * 4))) {
         // piece by piece: the gather (when it is still owed), the transfer of a piece, and the copy
@@ -1820,10 +1821,13 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
         if (rc) return rc;
       } else {
         PSKV_HIP(hipMemcpyAsync(out, r.out, r.out_nvals * 4, hipMemcpyDeviceToHost, t->stream));
+        copying = true;
       }
     }
-    if (pull && varlen && out_lens && n && !lens_pinned)
+    if (pull && varlen && out_lens && n && !lens_pinned) {
       PSKV_HIP(hipMemcpyAsync(out_lens, r.out_lens, n * 4, hipMemcpyDeviceToHost, t->stream));
+      copying = true;
+    }
     if (early) {
       // no device-detected errors in this mode and nothing to hand back: the caller's buffers have
       // been copied, the kernel is queued, later requests follow it on the stream
@@ -1833,8 +1837,8 @@ int request(pskv_table* t, bool push, bool pull, const uint64_t* keys, size_t n,
       // no device-detected errors in this mode: the end of the request is all that is left to wait for
       if (!r.done || !seen_in_time(r.done, r.done_seq)) PSKV_HIP(hipStreamSynchronize(t->stream));
     } else {
-      // (also waits for the copies above, where there were any)
-      rc = read_state(t, small && (!pull || !r.out_nvals || out_pinned));
+      // (also waits for the copies above, where there were any; what the staging ring has carried is here)
+      rc = read_state(t, !copying);
       if (rc) return rc;
       rc = report_device_errors(t);
       if (rc) {
