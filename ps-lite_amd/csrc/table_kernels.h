@@ -74,6 +74,17 @@ struct ReqBatch {
 };
 static_assert(sizeof(ReqBatch<kMaxBatch>) <= 3840, "kernel arguments are limited to 4 KiB");
 
+// Small requests are bound by the loads that wait for each other. Left to itself the compiler puts a load where
+// its value is first used, behind whatever branch that is, and a kernel argument likewise: what a kernel is going
+// to need is asked for together, from where there is something to read (past the end: the last element again),
+// and held here until all of it has arrived.
+template <typename T>
+__device__ __forceinline__ void arrived(T& x) {
+  asm volatile("" : "+v"(x));
+}
+// (kernel arguments: scalar registers)
+#define PSKV_ASK_ARGS(...) asm volatile("" ::__VA_ARGS__)
+
 // ---------------------------------------------------------------------------------
 // SCALAR mode: one float per key, kept in the low word of the slot payload so that a
 // probe reads key and value with one 128-bit load.
@@ -536,6 +547,8 @@ __device__ __forceinline__ void refuse_fixed(DevState* st, const ReqTag& tag) {
 template <int kLookupItems, int TABLES>
 __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
+  PSKV_ASK_ARGS("s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.n), "s"(d.ref), "s"(d.cache_keys),
+                "s"(d.snap), "s"(d.tag.epoch), "s"(d.cached), "s"(d.nblk));
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
   Slot* __restrict__ slots = d.slots;
@@ -562,6 +575,18 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch<TABLES> b) {
     uint64_t was[kLookupItems];  // the reference that is there already, if it is this key's
     bool is_new[kLookupItems];
     unsigned mine = 0;
+    // (the buffers have room for n keys; what lies beyond `cached` is not looked at)
+    uint64_t key[kLookupItems], left[kLookupItems], cached_key[kLookupItems], cached_ref[kLookupItems];
+#pragma unroll
+    for (int j = 0; j < kLookupItems; ++j) {
+      const uint64_t i = base + (uint64_t)threadIdx.x * kLookupItems + j, at = i < n ? i : n - 1;
+      key[j] = keys[at];
+      left[j] = keys[at ? at - 1 : 0];
+      cached_key[j] = cache_keys[at];
+      cached_ref[j] = ref[at];
+    }
+#pragma unroll
+    for (int j = 0; j < kLookupItems; ++j) arrived(key[j]), arrived(left[j]), arrived(cached_key[j]), arrived(cached_ref[j]);
 #pragma unroll
     for (int j = 0; j < kLookupItems; ++j) {
       const uint64_t i = base + (uint64_t)threadIdx.x * kLookupItems + j;
@@ -570,21 +595,16 @@ __global__ __launch_bounds__(kBlock) void k_lookup_fixed(ReqBatch<TABLES> b) {
       seen[j] = 0;
       was[j] = kRefAbsent;
       if (i < n) {
-        // (all asked for at once: none of them waits for another)
-        const uint64_t key = keys[i];
-        const uint64_t left = i > 0 ? keys[i - 1] : ~key;
-        const uint64_t cached_key = i < cached ? cache_keys[i] : ~key;
-        const uint64_t cached_ref = i < cached ? ref[i] : kRefAbsent;
         // keys are sorted and must be unique (kv_app.h:17): a key that equals its left neighbour
         // refuses the request, whether the key is new or has been in the table for long
-        if (left == key) {
+        if (i > 0 && left[j] == key[j]) {
           refuse_fixed(st, tag);
-          cache_keys[i] = key;
-        } else if (cached_key == key && cached_ref != kRefAbsent) {
-          was[j] = cached_ref;
+          cache_keys[i] = key[j];
+        } else if (i < cached && cached_key[j] == key[j] && cached_ref[j] != kRefAbsent) {
+          was[j] = cached_ref[j];
         } else {
-          cache_keys[i] = key;
-          p[j] = find_or_insert(slots, mask, st, key, is_new[j], seen[j]);
+          cache_keys[i] = key[j];
+          p[j] = find_or_insert(slots, mask, st, key[j], is_new[j], seen[j]);
         }
       }
       if (p[j] && !is_new[j] && seen[j] == kPayloadUnset) {
@@ -1221,8 +1241,10 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
   uint64_t* s_ref = s_ref_all + wave * kWaveSpan;
   if (staged) {
     for (uint32_t s = lane; s <= span; s += 64) {
-      s_off[s] = (int32_t)(int64_t)(p.off[j_lo + s] - f0);
-      if (s < span) s_ref[s] = p.ref[j_lo + s];
+      uint64_t at = p.off[j_lo + s], r = p.ref[j_lo + (s < span ? s : span - 1)];  // (one trip, not two)
+      arrived(at), arrived(r);
+      s_off[s] = (int32_t)(int64_t)(at - f0);
+      if (s < span) s_ref[s] = r;
     }
     // the wavefront's own LDS writes, visible to all of its lanes before the reads below
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
