@@ -517,9 +517,9 @@ void adopt_snapshot(pskv_table* t) {
 // anything but the kernels of a request that repeats the cached keys looks at the slots.
 int flush_scalar_cache(pskv_table* t) {
   if (!t->sc_dirty) return PSKV_OK;
-  ReqBatch<1> rb;
+  HeadBatch<1> rb;
   std::memset(&rb, 0, sizeof(rb));
-  TableReq& d = rb.t[0];
+  TableHead& d = rb.t[0];
   d.slots = t->slots;
   d.mask = t->cap - 1;
   d.st = t->st;
@@ -844,24 +844,32 @@ pskv_table* lead_of(Batch& bt) {
   return bt[0].t;
 }
 
-// One kernel of the store in its three sizes (ReqBatch).
+// One kernel of the store in its three sizes (ReqBatch, or HeadBatch: `head`).
 struct KernelSet {
   const void* one;
   const void* four;
   const void* most;
+  bool head;
 };
+template <typename B>
+constexpr bool takes_heads(void (*)(B)) { return false; }
+template <int TABLES>
+constexpr bool takes_heads(void (*)(HeadBatch<TABLES>)) { return true; }
 #define PSKV_KSET(name)                                                                                        \
   (KernelSet{reinterpret_cast<const void*>(&name<1>), reinterpret_cast<const void*>(&name<4>),                   \
-             reinterpret_cast<const void*>(&name<kMaxBatch>)})
+             reinterpret_cast<const void*>(&name<kMaxBatch>), takes_heads(&name<1>)})
 #define PSKV_KSET_OF(name, ...)                                                                                \
   (KernelSet{reinterpret_cast<const void*>(&name<__VA_ARGS__, 1>), reinterpret_cast<const void*>(&name<__VA_ARGS__, 4>), \
-             reinterpret_cast<const void*>(&name<__VA_ARGS__, kMaxBatch>)})
+             reinterpret_cast<const void*>(&name<__VA_ARGS__, kMaxBatch>), takes_heads(&name<__VA_ARGS__, 1>)})
 
 // A launch as pskv_replay_record keeps it: everything it takes to make it again.
 struct SavedLaunch {
   const void* kernel;
   dim3 grid, block;
-  ReqBatch<kMaxBatch> rb;  // (the kernel takes as much of it as its size says)
+  union {  // (the kernel takes as much of it as its size says)
+    ReqBatch<kMaxBatch> rb;
+    HeadBatch<kMaxBatch> heads;
+  };
 };
 // Where launch_batch leaves a copy of its launches while a request is being recorded (the thread
 // that records is the thread that launches).
@@ -878,8 +886,8 @@ int launch_batch(Batch& bt, int prof_kernel, const KernelSet& kernels, F nblk_of
   for (size_t i = 0; i < bt.size(); ++i) {
     const uint64_t nb = nblk_of(bt[i]);
     if (nb > 0x7fffffffull) return set_error(PSKV_EINVAL, "request too large");
-    l.rb.t[i] = bt[i].d;
-    l.rb.t[i].nblk = (uint32_t)nb;
+    bt[i].d.nblk = (uint32_t)nb;
+    if (kernels.head) l.heads.t[i] = bt[i].d; else l.rb.t[i] = bt[i].d;
     gx = std::max(gx, nb);
   }
   if (!gx) return PSKV_OK;

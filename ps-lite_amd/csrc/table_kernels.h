@@ -16,31 +16,42 @@ namespace pskv {
 // to kMaxBatch of these by value (blockIdx.y selects one), so that a request which the slicer
 // has cut into per-server pieces (kv_app.h:562-612) costs one launch per step and not one per
 // server; the single-table entry points launch with one of them.
-struct TableReq {
+// (The first half, all that the SCALAR kernels need, is a record of its own: a launch costs the calling thread by
+// what it carries, 2.45 us with 64 bytes of arguments, 2.9 with 240, 3.8 with 3,840.)
+struct TableHead {
   Slot* slots;
   uint64_t mask;
   DevState* st;
   const uint64_t* keys;  // n sorted unique keys
-  const int32_t* lens;   // VARLEN push: n row lengths
   const float* vals;     // SCALAR push: n values
   float* out;            // SCALAR pull: n values
   uint64_t n;
-  uint64_t nvals;        // VARLEN push: floats pushed; FIXED row kernels: the quad the launch starts at
-  // row modes
+  uint64_t* cache_keys;  // keys (and lens) of the request whose references the workspace holds
+  // SCALAR key cache (a request that repeats the cached sorted key set is served from a
+  // request-ordered value array): cache_keys above, the values in `arena`, the slot numbers in
+  // `tile_key`
   float* arena;              // row storage
-  uint64_t* ref;             // n row references, written by the lookup kernel
-  uint64_t* off;             // VARLEN: n+1 request-side row offsets in floats
-  unsigned long long* part;  // VARLEN: per-workgroup totals of the lens scan
   uint32_t* tile_key;        // VARLEN: first key of every request-side tile, ntiles+1 entries
-  TileNote* tile_aff;        // VARLEN: one note per tile
-  uint64_t ntiles;           // VARLEN: tiles of the request (push) / room in the tile table (pull);
-                             // FIXED row kernels: the quad the launch ends before
-  uint64_t* cache_keys;      // keys (and lens) of the request whose references the workspace holds
-  int32_t* cache_lens;
-  int32_t* out_lens;         // VARLEN pull: n answered lengths
   Snapshot* snap;            // where the kernel that creates the request's keys leaves the counters
   uint64_t snap_seq;
   ReqTag tag;
+  unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null; SCALAR
+                                // without the key cache: the word that takes tag.epoch when the request is done
+  uint32_t nblk;        // workgroups of the launch in flight that serve this table
+  uint32_t cache_mode;  // kCache* below
+};
+struct TableReq : TableHead {
+  const int32_t* lens;   // VARLEN push: n row lengths
+  uint64_t nvals;        // VARLEN push: floats pushed; FIXED row kernels: the quad the launch starts at
+  // row modes
+  uint64_t* ref;             // n row references, written by the lookup kernel
+  uint64_t* off;             // VARLEN: n+1 request-side row offsets in floats
+  unsigned long long* part;  // VARLEN: per-workgroup totals of the lens scan
+  TileNote* tile_aff;        // VARLEN: one note per tile
+  uint64_t ntiles;           // VARLEN: tiles of the request (push) / room in the tile table (pull);
+                             // FIXED row kernels: the quad the launch ends before
+  int32_t* cache_lens;
+  int32_t* out_lens;         // VARLEN pull: n answered lengths
   // row kernels
   float* req;             // push: request values (read); pull: response values (written)
   uint64_t total;         // floats in req
@@ -49,13 +60,6 @@ struct TableReq {
   uint32_t ignore_new;    // pull half of a push+pull: rows created by the push half hold data
   uint32_t total_on_device;  // VARLEN pull without a host round trip: the floats to move are
                              // DevState::scan_total and `total` is the room in req
-  uint32_t nblk;          // workgroups of the launch in flight that serve this table
-  // SCALAR key cache (a request that repeats the cached sorted key set is served from a
-  // request-ordered value array): cache_keys above, the values in `arena`, the slot numbers in
-  // `tile_key`
-  unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null; SCALAR
-                                // without the key cache: the word that takes tag.epoch when the request is done
-  uint32_t cache_mode;          // kCache* below
   uint32_t tile_base;           // VARLEN row kernels: the launch starts at this tile of the request (a large
                                 // host-resident request is served piece by piece as it arrives)
 };
@@ -71,6 +75,10 @@ constexpr uint32_t kSlotSpecial = 0xffffffffu;  // cached slot number of key 2^6
 template <int TABLES>
 struct ReqBatch {
   TableReq t[TABLES];
+};
+template <int TABLES>
+struct HeadBatch {
+  TableHead t[TABLES];
 };
 static_assert(sizeof(ReqBatch<kMaxBatch>) <= 3840, "kernel arguments are limited to 4 KiB");
 
@@ -114,8 +122,8 @@ __device__ __forceinline__ void arrived(T& x) {
 // first and last key included. (From device memory the plain order is 2 % faster: those two reads are
 // mostly in the cache by the time they are made.)
 template <bool PUSH, bool PULL, bool CACHE, bool PINNED, int TABLES>
-__global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch<TABLES> b) {
-  const TableReq& d = b.t[blockIdx.y];
+__global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
+  const TableHead& d = b.t[blockIdx.y];
   const uint64_t n = d.n;
   const unsigned nblk = d.nblk;  // (the grid is sized for the table with the most workgroups)
   if (blockIdx.x >= nblk) return;
@@ -302,8 +310,8 @@ __global__ __launch_bounds__(kBlock) void k_scalar(ReqBatch<TABLES> b) {
 // slots of a table whose cache may be ahead of them: a request that does not repeat the cached
 // keys (kFlushUnlessSame: the comparison of that request has run), a growth, a dump.
 template <int TABLES>
-__global__ __launch_bounds__(kBlock) void k_scalar_flush(ReqBatch<TABLES> b) {
-  const TableReq& d = b.t[blockIdx.y];
+__global__ __launch_bounds__(kBlock) void k_scalar_flush(HeadBatch<TABLES> b) {
+  const TableHead& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;
   // nothing changes these two while this kernel runs except its own last workgroup, which writes
   // after every workgroup has read them
@@ -358,8 +366,8 @@ __device__ __forceinline__ void decide_same(DevState* st, const ReqTag& tag, boo
 // writes same_epoch. (A var-len push, whose lens count as well, compares in k_var_push_begin.)
 constexpr int kSameKeysItems = 4;
 template <int TABLES>
-__global__ __launch_bounds__(kBlock) void k_same_keys(ReqBatch<TABLES> b) {
-  const TableReq& d = b.t[blockIdx.y];
+__global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
+  const TableHead& d = b.t[blockIdx.y];
   if (blockIdx.x >= d.nblk) return;  // tables that have nothing to compare have no workgroups
   const uint64_t* __restrict__ keys = d.keys;
   const uint64_t* __restrict__ cache_keys = d.cache_keys;
@@ -422,8 +430,8 @@ constexpr unsigned kRepeatFew = 1, kRepeatMany = 2;
 typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 template <bool PUSH, bool PULL, unsigned QUADS, int TABLES>
-__global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(ReqBatch<TABLES> b) {
-  const TableReq& d = b.t[blockIdx.y];
+__global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(HeadBatch<TABLES> b) {
+  const TableHead& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
   DevState* st = d.st;
