@@ -1223,6 +1223,129 @@ __device__ __forceinline__ bool rows_wave_affine(const RowsParams& p, uint64_t t
   return true;
 }
 
+// The second half of it: moves the tile's floats. STAGED: offsets and references lie in LDS (all of it in 32 bits:
+// a row is shorter than 2^28 floats), else where they were.
+template <int OP, bool RAGGED, bool STREAM, bool STAGED>
+__device__ __forceinline__ void rows_wave_move(const RowsParams& p, uint64_t f0, uint32_t tile_floats, uint64_t j_lo,
+                                               uint32_t span, const int32_t* s_off, const uint64_t* s_ref, bool rejected,
+                                               const f32x4& x) {
+  const unsigned lane = threadIdx.x & 63;
+  const uint32_t lf = lane * 4;
+  if (lf >= tile_floats) return;
+  // offsets (from the tile's first float; those of a row that ends far behind the tile are cut off) and references
+  // of the keys that overlap the tile
+  auto off_of = [&](uint32_t s) -> int32_t {
+    if (STAGED) return s_off[s];
+    const int64_t o = (int64_t)(p.off[j_lo + s] - f0);
+    return (int32_t)(o < (int64_t)PSKV_MAX_VARLEN_ROW * 2 ? o : (int64_t)PSKV_MAX_VARLEN_ROW * 2);
+  };
+  auto ref_of = [&](uint32_t s) { return STAGED ? s_ref[s] : p.ref[j_lo + s]; };
+  auto place = [&](uint64_t r, int32_t within) {
+    return p.arena + (((r & ~kRefNew) >> kLenBits) << 2) + within;
+  };
+  // the key that holds the quad's first float: the last one whose first float is at or before it
+  // (zero-length rows repeat an offset)
+  uint32_t lo = 0, hi = span;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (off_of(mid) <= (int32_t)lf) lo = mid + 1; else hi = mid;
+  }
+  const uint64_t r = ref_of(lo - 1);
+  float* dst = place(r, (int32_t)lf - off_of(lo - 1));
+  // a key the lookup refused (duplicate in the request, full table) is neither read nor written
+  const bool here = r != kRefAbsent;
+  const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
+  float* side = p.req + f0 + lf;
+  if (!RAGGED) {
+    if (!here) return;
+    f32x4 y = (f32x4)(0.f);
+    if (!fresh) y = load_quad<STREAM>(dst);
+    if (OP == kOpGather) {
+      store_quad<STREAM>(y, side);
+    } else if (!rejected) {
+      store_quad<STREAM>(y + x, dst);  // a created row is a zero row first (0.0f + v)
+    } else if (fresh) {
+      // a refused push changes no stored value; rows it created stay, as zero rows
+      store_quad<STREAM>(y, dst);
+    }
+    return;
+  }
+  const uint32_t upto = tile_floats - lf < 4u ? tile_floats - lf : 4u;
+  const int32_t end = off_of(lo);
+  const uint32_t count = end - (int32_t)lf < (int32_t)upto ? (uint32_t)(end - (int32_t)lf) : upto;
+  // the next row, when the quad reaches into it
+  uint64_t r2 = kRefAbsent;
+  float* dst2 = nullptr;
+  uint32_t two = upto;  // floats of the quad that the two rows hold
+  if (count < upto) {
+    uint32_t key = lo;  // (zero-length rows are stepped over; the key table closes with the end of the request)
+    while (off_of(key + 1) <= end) ++key;
+    r2 = ref_of(key);
+    dst2 = place(r2, 0);
+    const int32_t end2 = off_of(key + 1);
+    if (end2 - (int32_t)lf < (int32_t)upto) two = (uint32_t)(end2 - (int32_t)lf);
+  }
+  const bool here2 = r2 != kRefAbsent;
+  const bool fresh2 = (r2 & kRefNew) != 0 && !p.ignore_new;
+  if (two == upto) {
+    // (reading a quad whole is safe: what follows its row is another row, or the room behind the arena's last)
+    f32x4 y = (f32x4)(0.f), y2 = (f32x4)(0.f);
+    if (here && !fresh) y = load_quad<false>(dst);
+    if (here2 && !fresh2) y2 = load_quad<false>(dst2);
+    if (OP == kOpGather) {
+      f32x4 v = y;
+      if (count == 1) v.y = y2.x, v.z = y2.y, v.w = y2.z;
+      if (count == 2) v.z = y2.x, v.w = y2.y;
+      if (count == 3) v.w = y2.x;
+      if (upto == 4 && here && (here2 || count == 4)) {
+        store_quad<STREAM>(v, side);
+      } else {
+        if (here) store_part<false>(y, side, count);
+        if (here2) store_part<false>(y2, side + count, upto - count);
+      }
+      return;
+    }
+    if (here && (!rejected || fresh)) store_part<false>(rejected ? y : y + x, dst, count);
+    if (here2 && (!rejected || fresh2)) {
+      f32x4 x2 = x;
+      if (count == 1) x2.x = x.y, x2.y = x.z, x2.z = x.w;
+      if (count == 2) x2.x = x.z, x2.y = x.w;
+      if (count == 3) x2.x = x.w;
+      store_part<false>(rejected ? y2 : y2 + x2, dst2, upto - count);
+    }
+    return;
+  }
+  // three rows or more
+  float* at[4];
+  float cur[4];
+  bool made[4];
+  uint32_t key = lo - 1;
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) {
+    at[e] = nullptr;
+    made[e] = false;
+    if (e >= upto) continue;
+    while (off_of(key + 1) <= (int32_t)(lf + e)) ++key;
+    const uint64_t q = ref_of(key);
+    if (q == kRefAbsent) continue;
+    made[e] = (q & kRefNew) != 0 && !p.ignore_new;
+    at[e] = place(q, (int32_t)(lf + e) - off_of(key));
+  }
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) cur[e] = at[e] && !made[e] ? *at[e] : 0.f;
+#pragma unroll
+  for (uint32_t e = 0; e < 4; ++e) {
+    if (!at[e]) continue;
+    if (OP == kOpGather) {
+      side[e] = cur[e];
+    } else if (!rejected) {
+      *at[e] = cur[e] + x[e];
+    } else if (made[e]) {
+      *at[e] = cur[e];
+    }
+  }
+}
+
 // `x` comes from rows_wave_ask; it is used only below `total`. RAGGED: some row's length is not a
 // multiple of four, so a quad may hold the end of one row and the start of the next (rows themselves
 // start on multiples of four floats in the arena). The part in the row of its first float and the part in
@@ -1315,115 +1438,10 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
     if (lane == 0) p.tile_aff[wt] = note;
   }
 
-  const uint32_t lf = lane * 4;
-  if (lf >= tile_floats) return;
-  // offsets (from the tile's first float) and references of the keys that overlap the tile, from LDS or,
-  // where there are too many, from where they lie
-  auto off_of = [&](uint32_t s) { return staged ? (int64_t)s_off[s] : (int64_t)(p.off[j_lo + s] - f0); };
-  auto ref_of = [&](uint32_t s) { return staged ? s_ref[s] : p.ref[j_lo + s]; };
-  auto place = [&](uint64_t r, int64_t within) {
-    return p.arena + (((r & ~kRefNew) >> kLenBits) << 2) + within;
-  };
-  // the key that holds the quad's first float: the last one whose first float is at or before it
-  // (zero-length rows repeat an offset)
-  uint32_t lo = 0, hi = span;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (off_of(mid) <= (int64_t)lf) lo = mid + 1; else hi = mid;
-  }
-  const uint64_t r = ref_of(lo - 1);
-  float* dst = place(r, (int64_t)lf - off_of(lo - 1));
-  // a key the lookup refused (duplicate in the request, full table) is neither read nor written
-  const bool here = r != kRefAbsent;
-  const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
-  float* side = p.req + f0 + lf;
-  if (!RAGGED) {
-    if (!here) return;
-    f32x4 y = (f32x4)(0.f);
-    if (!fresh) y = load_quad<STREAM>(dst);
-    if (OP == kOpGather) {
-      store_quad<STREAM>(y, side);
-    } else if (!rejected) {
-      store_quad<STREAM>(y + x, dst);  // a created row is a zero row first (0.0f + v)
-    } else if (fresh) {
-      // a refused push changes no stored value; rows it created stay, as zero rows
-      store_quad<STREAM>(y, dst);
-    }
-    return;
-  }
-  const uint32_t upto = tile_floats - lf < 4u ? tile_floats - lf : 4u;
-  const int64_t end = off_of(lo);
-  const uint32_t count = end - (int64_t)lf < (int64_t)upto ? (uint32_t)(end - (int64_t)lf) : upto;
-  // the next row, when the quad reaches into it
-  uint64_t r2 = kRefAbsent;
-  float* dst2 = nullptr;
-  uint32_t two = upto;  // floats of the quad that the two rows hold
-  if (count < upto) {
-    uint32_t key = lo;  // (zero-length rows are stepped over; the key table closes with the end of the request)
-    while (off_of(key + 1) <= end) ++key;
-    r2 = ref_of(key);
-    dst2 = place(r2, 0);
-    const int64_t end2 = off_of(key + 1);
-    if (end2 - (int64_t)lf < (int64_t)upto) two = (uint32_t)(end2 - (int64_t)lf);
-  }
-  const bool here2 = r2 != kRefAbsent;
-  const bool fresh2 = (r2 & kRefNew) != 0 && !p.ignore_new;
-  if (two == upto) {
-    // (reading a quad whole is safe: what follows its row is another row, or the room behind the arena's last)
-    f32x4 y = (f32x4)(0.f), y2 = (f32x4)(0.f);
-    if (here && !fresh) y = load_quad<false>(dst);
-    if (here2 && !fresh2) y2 = load_quad<false>(dst2);
-    if (OP == kOpGather) {
-      f32x4 v = y;
-      if (count == 1) v.y = y2.x, v.z = y2.y, v.w = y2.z;
-      if (count == 2) v.z = y2.x, v.w = y2.y;
-      if (count == 3) v.w = y2.x;
-      if (upto == 4 && here && (here2 || count == 4)) {
-        store_quad<STREAM>(v, side);
-      } else {
-        if (here) store_part<false>(y, side, count);
-        if (here2) store_part<false>(y2, side + count, upto - count);
-      }
-      return;
-    }
-    if (here && (!rejected || fresh)) store_part<false>(rejected ? y : y + x, dst, count);
-    if (here2 && (!rejected || fresh2)) {
-      f32x4 x2 = x;
-      if (count == 1) x2.x = x.y, x2.y = x.z, x2.z = x.w;
-      if (count == 2) x2.x = x.z, x2.y = x.w;
-      if (count == 3) x2.x = x.w;
-      store_part<false>(rejected ? y2 : y2 + x2, dst2, upto - count);
-    }
-    return;
-  }
-  // three rows or more
-  float* at[4];
-  float cur[4];
-  bool made[4];
-  uint32_t key = lo - 1;
-#pragma unroll
-  for (uint32_t e = 0; e < 4; ++e) {
-    at[e] = nullptr;
-    made[e] = false;
-    if (e >= upto) continue;
-    while (off_of(key + 1) <= (int64_t)(lf + e)) ++key;
-    const uint64_t q = ref_of(key);
-    if (q == kRefAbsent) continue;
-    made[e] = (q & kRefNew) != 0 && !p.ignore_new;
-    at[e] = place(q, (int64_t)(lf + e) - off_of(key));
-  }
-#pragma unroll
-  for (uint32_t e = 0; e < 4; ++e) cur[e] = at[e] && !made[e] ? *at[e] : 0.f;
-#pragma unroll
-  for (uint32_t e = 0; e < 4; ++e) {
-    if (!at[e]) continue;
-    if (OP == kOpGather) {
-      side[e] = cur[e];
-    } else if (!rejected) {
-      *at[e] = cur[e] + x[e];
-    } else if (made[e]) {
-      *at[e] = cur[e];
-    }
+  if (staged) {
+    rows_wave_move<OP, RAGGED, STREAM, true>(p, f0, tile_floats, j_lo, span, s_off, s_ref, rejected, x);
+  } else {
+    rows_wave_move<OP, RAGGED, STREAM, false>(p, f0, tile_floats, j_lo, span, s_off, s_ref, rejected, x);
   }
 }
 
