@@ -1178,7 +1178,7 @@ __device__ __forceinline__ void rows_wave_ask(const RowsParams& p, uint64_t boun
   const uint32_t floats = (uint32_t)(left < (uint64_t)kTileVar ? left : (uint64_t)kTileVar);
   aff.first = kTileNotAffine;
   aff.second = 0;
-  if (left) {
+  if (left && p.tag.try_cache) {
     const u64x2 w = *reinterpret_cast<const u64x2*>(&p.tile_aff[wt]);  // one 128-bit load
     aff.first = w.x;
     aff.second = w.y;
@@ -1382,13 +1382,13 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  if (!same) {
+  if (!same && !RAGGED) {  // (nobody looks at the notes of a request with ragged rows)
     // Leave a note for requests that repeat this one. Every row with floats in the tile has a
     // distance between its place in the arena and its place in the request; the tile is one
     // piece when all distances are equal (the rows lie back to back, in request order, without
     // padding between them) and two pieces when they change once.
     TileNote note = {kTileNotAffine, 0};
-    if (!RAGGED && staged) {
+    if (staged) {
       bool absent = false;
       int64_t d[(kWaveSpan + 63) / 64];
       bool has[(kWaveSpan + 63) / 64];
