@@ -2,12 +2,12 @@
 // sketches in ParallelOrderedMatch (include/ps/internal/parallel_kv_match.h:29-120) with the
 // operators of assign_op.h:12-41:
 //     if (dst_key[i] == src_key[j]) dst_val[i] op= src_val[j]        (k floats per key)
-// Both key sets are sorted, so the source keys that can match a tile of destination keys are
+// Both key sets are sorted, so the keys of one that can match a tile of the other's are
 // one contiguous stretch. A first small kernel finds where every tile's stretch begins (one
-// search per tile, all tiles at once); a workgroup then stages its stretch in LDS and resolves
-// its destination keys there, so all key traffic is streamed, once. For k == 1 the values
-// are combined in the same kernel; for longer values the kernel leaves the matched source
-// index of every destination key behind and a second kernel streams the rows.
+// search per tile, all tiles at once); a workgroup then stages its stretch in LDS, or samples it there
+// where it is long, and resolves its keys, so where the sets are of like size all key traffic is streamed, once. For
+// k == 1 the values are combined in the same kernel; for longer values the kernel leaves the index of every key's match
+// behind and a second kernel streams the rows.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -21,24 +21,19 @@ namespace pskv {
 namespace {
 
 constexpr unsigned kMatchBlock = 256;
+// Keys per lane: four neighbouring ones, the first found by halving and the others a few keys further on; one where
+// four would leave the GPU with fewer than two workgroups per compute unit, or a tile's stretch would not fit into LDS
+// because the other set is twice as large or more.
 constexpr unsigned kMatchItems = 4;
-constexpr unsigned kMatchTile = kMatchBlock * kMatchItems;  // destination keys per workgroup
+constexpr uint64_t kFewKeys = 2ull * 256 * kMatchBlock * kMatchItems;
 constexpr unsigned kMatchLds = 1536;    // source keys (and values) a workgroup holds in LDS at a time (18 KiB)
 constexpr unsigned kMatchTurn = 3;      // source keys a lane asks for at a time
-constexpr unsigned kMatchPieces = 8;    // a longer stretch than this many pieces is searched in place
+// A longer stretch than so many pieces is sampled, not staged. (Pieces follow from each other, but read in one go
+// what the sampled search reads key by key: they pay while there are workgroups enough to fill the GPU.)
+constexpr unsigned kMatchPieces = 8, kMatchPiecesFew = 3;
 constexpr uint64_t kNoMatch = ~0ull;
 constexpr unsigned kCounts = 64;        // counters of matched keys, each on a line of its own
 constexpr unsigned kCountStride = 16;
-
-// first index in [lo, hi) whose key is not below `key`
-__device__ __forceinline__ uint64_t lower_bound_of(const uint64_t* __restrict__ a, uint64_t lo, uint64_t hi,
-                                                   uint64_t key) {
-  while (lo < hi) {
-    const uint64_t mid = lo + ((hi - lo) >> 1);
-    if (a[mid] < key) lo = mid + 1; else hi = mid;
-  }
-  return lo;
-}
 
 // assign_op.h:26-36: right op= left
 __device__ __forceinline__ float combine(int op, float d, float s) {
@@ -57,8 +52,9 @@ __device__ __forceinline__ f32x4 combine(int op, f32x4 d, f32x4 s) {
   return r;
 }
 
-// spans[t] = first source key not below the first destination key of tile t; spans[tiles] = n_src.
-// The stretch of tile t is [spans[t], spans[t+1]): it may hold source keys that lie between two
+// The match walks the tiles of one key set and finds their keys in the other. spans[t] = first key of the set that is
+// searched (`src`, n_src keys) not below the first key of tile t of the other; spans[tiles] = n_src.
+// The stretch of tile t is [spans[t], spans[t+1]): it may hold keys that lie between two
 // tiles, which match nothing. Bound by the round trips to memory that follow from each other: a workgroup
 // samples the whole source evenly into LDS (one round trip, the same lines for every workgroup), its
 // kSpanTiles tiles find the step they lie in there, and kSpanLanes lanes each narrow it down by a factor of 16
@@ -70,12 +66,12 @@ constexpr unsigned kSpanBlock = kSpanTiles * kSpanLanes;
 constexpr unsigned kSpanSamples = 4 * kSpanBlock;
 __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __restrict__ src, uint64_t n_src,
                                                             const uint64_t* __restrict__ dst, uint64_t tiles,
-                                                            uint64_t* __restrict__ spans) {
+                                                            unsigned tile, uint64_t* __restrict__ spans) {
   __shared__ uint64_t s_sample[kSpanSamples];
   const uint64_t t = (uint64_t)blockIdx.x * kSpanTiles + threadIdx.x / kSpanLanes;
   const unsigned lane = threadIdx.x & 63, sub = threadIdx.x % kSpanLanes;
   const bool live = t < tiles;
-  const uint64_t key = live ? dst[t * kMatchTile] : 0;
+  const uint64_t key = live ? dst[t * tile] : 0;
   const uint64_t step = (n_src + kSpanSamples - 1) / kSpanSamples;
   const unsigned samples = (unsigned)((n_src + step - 1) / step);
   uint64_t x[kSpanSamples / kSpanBlock];
@@ -114,58 +110,65 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
   if (live && sub == 0) spans[t] = lo;
 }
 
-// One workgroup per kMatchTile destination keys. Bound by memory once the loads do not wait for each other: 12M
-// against 16M keys took 100 us with one source key per lane asked for at a time, 77 with three (5.2 TB/s).
-// K1: values are single floats and are combined here; otherwise where[i] receives the index of the matching
-// source key, or kNoMatch.
-template <bool K1>
-__global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __restrict__ src, uint64_t n_src,
-                                                            const uint64_t* __restrict__ dst, uint64_t n_dst,
+// One workgroup per tile of kMatchBlock * ITEMS keys of `near`, which it finds in `far`. Those are the destination's
+// and the source's keys, or with SWAP, where the source is much the smaller set, the other way round: the walk then
+// reads, and the row kernel visits, what there is in the source. Bound by memory once the loads do not wait for each
+// other: 12M source against 16M destination keys took 100 us with one source key per lane asked for at a time, 77 with
+// three (5.2 TB/s).
+// K1: values are single floats and are combined here; otherwise where[i] receives the index in `far` of the match of
+// key i, or kNoMatch.
+template <bool K1, bool SWAP, unsigned ITEMS>
+__global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __restrict__ far, uint64_t n_far,
+                                                            const uint64_t* __restrict__ near, uint64_t n_near,
                                                             const uint64_t* __restrict__ spans,
                                                             uint64_t* __restrict__ where,
                                                             const float* __restrict__ src_vals,
                                                             float* __restrict__ dst_vals, int op,
                                                             unsigned long long* __restrict__ counts) {
+  static_assert(ITEMS == 4 || ITEMS == 1, "128-bit accesses of four keys, or one key");
   __shared__ uint64_t s_keys[kMatchLds];
-  __shared__ float s_vals[K1 ? kMatchLds : 1];
+  __shared__ float s_vals[K1 && !SWAP ? kMatchLds : 1];
   __shared__ unsigned s_red[kMatchBlock / 64];
-  const uint64_t first = (uint64_t)blockIdx.x * kMatchTile;
-  const uint64_t tile_n = n_dst - first < kMatchTile ? n_dst - first : kMatchTile;
-  // A lane takes kMatchItems neighbouring destination keys (requested before anything else): the
-  // first is found by halving, the others a few source keys further on.
-  const unsigned idx0 = threadIdx.x * kMatchItems;
+  constexpr unsigned kTile = kMatchBlock * ITEMS;
+  const uint64_t first = (uint64_t)blockIdx.x * kTile;
+  const uint64_t tile_n = n_near - first < kTile ? n_near - first : kTile;
+  const unsigned idx0 = threadIdx.x * ITEMS;
   const uint64_t i0 = first + idx0;
-  uint64_t key[kMatchItems];
-  const bool whole = idx0 + kMatchItems <= tile_n;
-  if (whole && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-    static_assert(kMatchItems == 4, "two 128-bit loads");
-    const u64x2 x = *reinterpret_cast<const u64x2*>(dst + i0);
-    const u64x2 y = *reinterpret_cast<const u64x2*>(dst + i0 + 2);
-    key[0] = x.x, key[1] = x.y, key[2] = y.x, key[3] = y.y;
+  uint64_t key[ITEMS];
+  const bool whole = ITEMS == 4 && idx0 + ITEMS <= tile_n;
+  if (whole && (reinterpret_cast<uintptr_t>(near) & 15) == 0) {
+    const u64x2 x = *reinterpret_cast<const u64x2*>(near + i0);
+    const u64x2 y = *reinterpret_cast<const u64x2*>(near + i0 + 2);
+    key[0] = x.x, key[1 % ITEMS] = x.y, key[2 % ITEMS] = y.x, key[3 % ITEMS] = y.y;
   } else {
 #pragma unroll
-    for (unsigned r = 0; r < kMatchItems; ++r) key[r] = idx0 + r < tile_n ? dst[i0 + r] : 0;
+    for (unsigned r = 0; r < ITEMS; ++r) key[r] = near[idx0 + r < tile_n ? i0 + r : first];
   }
   const uint64_t lo = spans[blockIdx.x], hi = spans[blockIdx.x + 1];
   const uint64_t span = hi > lo ? hi - lo : 0;  // (hi >= lo when the keys are sorted)
-  // K1: the values follow the keys without waiting for what the search finds: those of the destination are
+  // K1: the values follow the keys without waiting for what the search finds: those of this side are
   // asked for here (a line of 32 of them without a match is rare), those of a stretch that fits into LDS come
   // with its keys.
-  const bool vec = K1 && whole && (reinterpret_cast<uintptr_t>(dst_vals) & 15) == 0;
-  const bool vals_here = K1 && span <= kMatchLds;
+  const float* near_vals = SWAP ? src_vals : dst_vals;
+  const bool vec = K1 && whole && (reinterpret_cast<uintptr_t>(near_vals) & 15) == 0;
+  const bool vals_here = K1 && !SWAP && span <= kMatchLds;
   f32x4 mine = (f32x4)(0.f);
-  if (vec) mine = *reinterpret_cast<const f32x4*>(dst_vals + i0);
-  // The stretch goes through LDS in pieces of kMatchLds keys. A key is looked up in the first
-  // piece whose last key is not below it (or in the last piece).
-  const bool staged = span <= (uint64_t)kMatchLds * kMatchPieces;
-  uint64_t j[kMatchItems];
-  bool open[kMatchItems];
+  if (vec) {
+    mine = *reinterpret_cast<const f32x4*>(near_vals + i0);
+  } else if (K1) {
 #pragma unroll
-  for (unsigned r = 0; r < kMatchItems; ++r) {
+    for (unsigned r = 0; r < ITEMS; ++r) mine[r] = near_vals[idx0 + r < tile_n ? i0 + r : first];
+  }
+  uint64_t j[ITEMS];
+  bool open[ITEMS];
+#pragma unroll
+  for (unsigned r = 0; r < ITEMS; ++r) {
     j[r] = kNoMatch;
     open[r] = idx0 + r < tile_n;
   }
-  if (staged) {
+  if (span <= (uint64_t)kMatchLds * (ITEMS == 1 ? kMatchPiecesFew : kMatchPieces)) {
+    // The stretch goes through LDS in pieces of kMatchLds keys. A key is looked up in the first
+    // piece whose last key is not below it (or in the last piece).
     for (uint64_t base = 0; base < span; base += kMatchLds) {
       const unsigned len = span - base < kMatchLds ? (unsigned)(span - base) : kMatchLds;
       const bool last_piece = base + len == span;
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
 #pragma unroll
         for (unsigned q = 0; q < kMatchTurn; ++q) {
           const unsigned t = t0 + q * kMatchBlock;
-          ks[q] = t < len ? src[lo + base + t] : 0;
+          ks[q] = t < len ? far[lo + base + t] : 0;
           vs[q] = vals_here && t < len ? src_vals[lo + base + t] : 0.0f;
         }
 #pragma unroll
@@ -190,10 +193,10 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
       }
       __syncthreads();
       const uint64_t top = s_keys[len - 1];
-      unsigned pos = 0;     // the lane's open keys are above every source key before this one
+      unsigned pos = 0;     // the lane's open keys are above every key before this one
       bool on_foot = false;  // whether a key of this lane has been placed in this piece already
 #pragma unroll
-      for (unsigned r = 0; r < kMatchItems; ++r) {
+      for (unsigned r = 0; r < ITEMS; ++r) {
         if (!open[r] || !(key[r] <= top || last_piece)) continue;
         unsigned at = pos;
         if (on_foot) {
@@ -213,49 +216,78 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
         on_foot = true;
       }
     }
-  } else {  // far more source keys than destination keys here: search the stretch where it lies
-    uint64_t from = lo;
+  } else {
+    // Far more keys there than here: the stretch is sampled evenly into LDS, a key finds the step it lies in there and
+    // halves that step where it lies, a line or two. (Halving the whole stretch in memory took 14 trips that follow
+    // from each other for 13,000 keys, 50 us.)
+    const uint64_t step = (span + kMatchLds - 1) / kMatchLds;
+    const unsigned samples = (unsigned)((span + step - 1) / step);
+    for (unsigned t0 = threadIdx.x; t0 < samples; t0 += kMatchBlock * kMatchTurn) {
+      uint64_t ks[kMatchTurn];
 #pragma unroll
-    for (unsigned r = 0; r < kMatchItems; ++r) {
-      if (!open[r]) continue;
-      const uint64_t p = lower_bound_of(src, from, hi, key[r]);
-      if (p < hi && src[p] == key[r]) j[r] = p;
-      from = p;
+      for (unsigned q = 0; q < kMatchTurn; ++q) {
+        const unsigned t = t0 + q * kMatchBlock;
+        ks[q] = far[lo + (t < samples ? t : samples - 1) * step];
+      }
+#pragma unroll
+      for (unsigned q = 0; q < kMatchTurn; ++q)
+        if (t0 + q * kMatchBlock < samples) s_keys[t0 + q * kMatchBlock] = ks[q];
     }
+    __syncthreads();
+    uint64_t a[ITEMS], b[ITEMS];  // every key before a is below the lane's, none from b on is
+#pragma unroll
+    for (unsigned r = 0; r < ITEMS; ++r) {
+      unsigned at = 0, end = samples;
+      while (at < end) {
+        const unsigned mid = (at + end) >> 1;
+        if (s_keys[mid] < key[r]) at = mid + 1; else end = mid;
+      }
+      a[r] = at ? lo + (at - 1) * step + 1 : lo;
+      b[r] = at < samples ? lo + at * step : hi;
+      if (!open[r]) b[r] = a[r];
+    }
+    for (uint64_t left = step; left > 0; left >>= 1) {  // (the lane's keys side by side)
+#pragma unroll
+      for (unsigned r = 0; r < ITEMS; ++r) {
+        if (a[r] >= b[r]) continue;
+        const uint64_t mid = a[r] + ((b[r] - a[r]) >> 1);
+        if (far[mid] < key[r]) a[r] = mid + 1; else b[r] = mid;
+      }
+    }
+#pragma unroll
+    for (unsigned r = 0; r < ITEMS; ++r)
+      if (open[r] && a[r] < n_far && far[a[r]] == key[r]) j[r] = a[r];
   }
   unsigned found = 0;
 #pragma unroll
-  for (unsigned r = 0; r < kMatchItems; ++r) found += j[r] != kNoMatch ? 1u : 0u;
-  if (K1) {
-    float d[kMatchItems] = {mine.x, mine.y, mine.z, mine.w};
-    if (!vec && op != PSKV_OP_ASSIGN) {
+  for (unsigned r = 0; r < ITEMS; ++r) found += j[r] != kNoMatch ? 1u : 0u;
+  if (K1 && SWAP) {
+    float d[ITEMS];
 #pragma unroll
-      for (unsigned r = 0; r < kMatchItems; ++r)
-        if (j[r] != kNoMatch) d[r] = dst_vals[i0 + r];
-    }
+    for (unsigned r = 0; r < ITEMS; ++r) d[r] = op != PSKV_OP_ASSIGN && j[r] != kNoMatch ? dst_vals[j[r]] : 0.0f;
 #pragma unroll
-    for (unsigned r = 0; r < kMatchItems; ++r)
-      if (j[r] != kNoMatch) d[r] = combine(op, d[r], vals_here ? s_vals[j[r] - lo] : src_vals[j[r]]);
+    for (unsigned r = 0; r < ITEMS; ++r)
+      if (j[r] != kNoMatch) dst_vals[j[r]] = combine(op, d[r], mine[r]);
+  } else if (K1) {
+#pragma unroll
+    for (unsigned r = 0; r < ITEMS; ++r)
+      if (j[r] != kNoMatch) mine[r] = combine(op, mine[r], vals_here ? s_vals[j[r] - lo] : src_vals[j[r]]);
     if (vec) {
-      if (found) {
-        f32x4 v;
-        v.x = d[0], v.y = d[1], v.z = d[2], v.w = d[3];
-        *reinterpret_cast<f32x4*>(dst_vals + i0) = v;
-      }
+      if (found) *reinterpret_cast<f32x4*>(dst_vals + i0) = mine;
     } else {
 #pragma unroll
-      for (unsigned r = 0; r < kMatchItems; ++r)
-        if (j[r] != kNoMatch) dst_vals[i0 + r] = d[r];
+      for (unsigned r = 0; r < ITEMS; ++r)
+        if (j[r] != kNoMatch) dst_vals[i0 + r] = mine[r];
     }
   } else {
     if (whole) {
       u64x2 x, y;
-      x.x = j[0], x.y = j[1], y.x = j[2], y.y = j[3];
+      x.x = j[0], x.y = j[1 % ITEMS], y.x = j[2 % ITEMS], y.y = j[3 % ITEMS];
       *reinterpret_cast<u64x2*>(where + i0) = x;  // (the workspace is 256-byte aligned)
       *reinterpret_cast<u64x2*>(where + i0 + 2) = y;
     } else {
 #pragma unroll
-      for (unsigned r = 0; r < kMatchItems; ++r)
+      for (unsigned r = 0; r < ITEMS; ++r)
         if (idx0 + r < tile_n) where[i0 + r] = j[r];
     }
   }
@@ -287,12 +319,13 @@ __global__ void k_match_total(unsigned long long* counts, MatchDone* done, unsig
   __hip_atomic_store(&done->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Rows of kq units (floats, or groups of four floats): dst row i op= src row where[i].
-template <typename V>
-__global__ __launch_bounds__(kMatchBlock) void k_match_rows(const uint64_t* __restrict__ where, uint64_t n_dst,
+// Rows of kq units (floats, or groups of four floats): dst row i op= src row where[i], or with SWAP dst row where[i]
+// op= src row i.
+template <typename V, bool SWAP>
+__global__ __launch_bounds__(kMatchBlock) void k_match_rows(const uint64_t* __restrict__ where, uint64_t n_near,
                                                             uint64_t kq, const V* __restrict__ src,
                                                             V* __restrict__ dst, int op) {
-  const uint64_t total = n_dst * kq;
+  const uint64_t total = n_near * kq;
   const uint64_t stride = (uint64_t)gridDim.x * kMatchBlock;
   for (uint64_t base = (uint64_t)blockIdx.x * kMatchBlock; base < total; base += stride) {
     // one division per workgroup and turn; a lane is at most kMatchBlock units further on
@@ -300,11 +333,11 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_rows(const uint64_t* __re
     const uint64_t c = base - row0 * kq + threadIdx.x;
     const uint64_t over = kq >= kMatchBlock ? (c >= kq ? 1u : 0u) : (uint64_t)((unsigned)c / (unsigned)kq);
     const uint64_t row = row0 + over, col = c - over * kq;
-    if (row >= n_dst) continue;
+    if (row >= n_near) continue;
     const uint64_t j = where[row];
     if (j == kNoMatch) continue;
-    const V s = __builtin_nontemporal_load(src + j * kq + col);
-    V* p = dst + row * kq + col;
+    const V s = __builtin_nontemporal_load(src + (SWAP ? row : j) * kq + col);
+    V* p = dst + (SWAP ? j : row) * kq + col;
     if (op == PSKV_OP_ASSIGN) {
       __builtin_nontemporal_store(s, p);
     } else {
@@ -432,35 +465,50 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
     d_sv = static_cast<const float*>(c->stage[2].ptr);
     d_dv = static_cast<float*>(c->stage[3].ptr);
   }
-  const unsigned blocks = (unsigned)((n_dst + kMatchTile - 1) / kMatchTile);
+  const bool vec = k % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_sv) | reinterpret_cast<uintptr_t>(d_dv)) & 15) == 0;
+  const uint64_t kq = vec ? k / 4 : k;
+  // The walk goes over the destination's keys, which streams through everything once, unless the source is so much
+  // smaller that finding its keys in the destination reads less. Single values: from 16 times on, and where the
+  // destination is not a matter of a few microseconds anyway (320,000 into 6.6M keys: 41 -> 36 us, but 44,000 into
+  // 1M 25 -> 27, 1.3M into 8.7M 53 -> 108). Longer ones: the row kernel visits the walk's keys, so from twice or four
+  // times on (450,000 into 1.6M keys with 3 floats: 53 -> 39 us; 1M into 3M with 4: 58 -> 62).
+  const uint64_t ratio = n_dst / n_src;
+  const bool swap = k == 1 ? ratio >= 16 && n_dst >= (4u << 20) : ratio >= (kq == 1 ? 4 : 2);
+  const uint64_t n_near = swap ? n_src : n_dst, n_far = swap ? n_dst : n_src;
+  const uint64_t *near = swap ? d_src : d_dst, *far = swap ? d_dst : d_src;
+  const bool few = n_near < kFewKeys || n_far / n_near >= 2;
+  const unsigned tile = kMatchBlock * (few ? 1 : kMatchItems);
+  const unsigned blocks = (unsigned)((n_near + tile - 1) / tile);
   {
     int rc = room(&c->spans, ((size_t)blocks + 1) * sizeof(uint64_t), st);
     if (rc) return rc;
   }
   uint64_t* spans = static_cast<uint64_t*>(c->spans.ptr);
-  hipLaunchKernelGGL(k_match_spans, dim3((blocks + kSpanTiles - 1) / kSpanTiles), dim3(kSpanBlock), 0, st, d_src,
-                     (uint64_t)n_src, d_dst, (uint64_t)blocks, spans);
+  hipLaunchKernelGGL(k_match_spans, dim3((blocks + kSpanTiles - 1) / kSpanTiles), dim3(kSpanBlock), 0, st, far, n_far, near,
+                     (uint64_t)blocks, tile, spans);
   // (a launch can carry events of its own, which read the begin and the end of that very dispatch)
   hipEvent_t e0 = kernel_ms ? c->ev[0] : nullptr, e1 = kernel_ms ? c->ev[1] : nullptr;
   hipEvent_t e2 = kernel_ms ? c->ev[2] : nullptr, e3 = kernel_ms ? c->ev[3] : nullptr;
-  if (k == 1) {
-    hipExtLaunchKernelGGL(k_match_keys<true>, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, d_src, (uint64_t)n_src, d_dst,
-                       (uint64_t)n_dst, spans, static_cast<uint64_t*>(nullptr), d_sv, d_dv, op, c->counts);
-  } else {
-    int rc = room(&c->where, n_dst * sizeof(uint64_t), st);
+  uint64_t* where = nullptr;
+  if (k > 1) {
+    int rc = room(&c->where, n_near * sizeof(uint64_t), st);
     if (rc) return rc;
-    uint64_t* where = static_cast<uint64_t*>(c->where.ptr);
-    hipExtLaunchKernelGGL(k_match_keys<false>, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, d_src, (uint64_t)n_src, d_dst,
-                       (uint64_t)n_dst, spans, where, d_sv, d_dv, op, c->counts);
-    const bool vec = k % 4 == 0 && ((reinterpret_cast<uintptr_t>(d_sv) | reinterpret_cast<uintptr_t>(d_dv)) & 15) == 0;
-    const uint64_t kq = vec ? k / 4 : k;
-    const unsigned grid = grid_for(n_dst * kq, kMatchBlock, 1u << 20);
+    where = static_cast<uint64_t*>(c->where.ptr);
+  }
+  auto keys = k == 1 ? (swap ? (few ? k_match_keys<true, true, 1> : k_match_keys<true, true, kMatchItems>)
+                             : (few ? k_match_keys<true, false, 1> : k_match_keys<true, false, kMatchItems>))
+                     : (few ? k_match_keys<false, false, 1> : k_match_keys<false, false, kMatchItems>);
+  hipExtLaunchKernelGGL(keys, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, far, n_far, near, n_near, spans, where, d_sv,
+                        d_dv, op, c->counts);
+  if (k > 1) {
+    const unsigned grid = grid_for(n_near * kq, kMatchBlock, 1u << 20);
     if (vec) {
-      hipExtLaunchKernelGGL(k_match_rows<f32x4>, dim3(grid), dim3(kMatchBlock), 0, st, e2, e3, 0, where, (uint64_t)n_dst, kq,
-                         reinterpret_cast<const f32x4*>(d_sv), reinterpret_cast<f32x4*>(d_dv), op);
+      auto rows = swap ? k_match_rows<f32x4, true> : k_match_rows<f32x4, false>;
+      hipExtLaunchKernelGGL(rows, dim3(grid), dim3(kMatchBlock), 0, st, e2, e3, 0, where, n_near, kq,
+                            reinterpret_cast<const f32x4*>(d_sv), reinterpret_cast<f32x4*>(d_dv), op);
     } else {
-      hipExtLaunchKernelGGL(k_match_rows<float>, dim3(grid), dim3(kMatchBlock), 0, st, e2, e3, 0, where, (uint64_t)n_dst, kq, d_sv,
-                         d_dv, op);
+      auto rows = swap ? k_match_rows<float, true> : k_match_rows<float, false>;
+      hipExtLaunchKernelGGL(rows, dim3(grid), dim3(kMatchBlock), 0, st, e2, e3, 0, where, n_near, kq, d_sv, d_dv, op);
     }
   }
   const unsigned long long seq = ++c->seq;

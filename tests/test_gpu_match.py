@@ -110,18 +110,22 @@ def test_match_at_the_size_of_a_model(capi, dev):
 
 
 @pytest.mark.parametrize("n_src,n_dst", [(1536, 1024), (1537, 1024), (1535, 1025), (4096, 65536), (4097, 65537),
-                                         (200_000, 66_000), (3072 * 4, 1024), (20_000, 1024)])
+                                         (200_000, 66_000), (3072 * 4, 1024), (20_000, 1024), (256, 1023), (256, 1024),
+                                         (257, 1028), (1_000_000, 257), (530_000 * 14, 530_000), (200_000, 4_300_000), (530_000, 8_500_000)])
 def test_match_edges_of_stretches(capi, orc, dev, n_src, n_dst):
-    """Source stretches at the edges of what a workgroup stages in LDS with its values (1,536 keys), of the
-    sampled search (4,096 samples, 64 tiles of 1,024 destination keys), and called twice: the counters of one call
-    are clear for the next."""
+    """Stretches at the edges of what a workgroup stages in LDS with its values (1,536 keys) and in pieces (3 or 8
+    of them), longer ones, which are sampled; tiles of 256 and (from 524,288 keys on) of 1,024 keys; the walk over
+    the source where it is much smaller than the destination; and called twice: the counters of one call are clear
+    for the next."""
     announce("match_stretches", n_src, n_dst)
     rng = np.random.default_rng(n_src + n_dst)
     sk, dk = key_sets(rng, n_src, n_dst, min(n_src, n_dst) // 2)
-    sv, dv = values(rng, sk.size, 1), values(rng, dk.size, 1)
-    for op in (0, 1):
-        _, want, want_n = orc.ordered_match(sk, sv, dk, dv, 1, op)
+    for op, k in ((0, 1), (1, 1), (2, 3), (1, 4)):
+        if k > 1 and max(n_src, n_dst) > 1_000_000:
+            continue
+        sv, dv = values(rng, sk.size * k, op), values(rng, dk.size * k, op)
+        _, want, want_n = orc.ordered_match(sk, sv, dk, dv, k, op)
         for _ in range(2):
-            got, n = run(capi, dev, "device", sk, sv, dk, dv, 1, op)
+            got, n = run(capi, dev, "device", sk, sv, dk, dv, k, op)
             assert n == want_n
-            assert_bits_equal(got, want, "op %d" % op)
+            assert_bits_equal(got, want, "op %d k %d" % (op, k))
