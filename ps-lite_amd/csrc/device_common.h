@@ -101,7 +101,8 @@ struct alignas(32) DevState {
   unsigned long long repeat_verdict;
   // keys held (slot array plus the side slot) = sum of the shards
   unsigned long long count_shard[kCountShards * kShardStride];
-  // first level of the last-workgroup ticket: one counter per 128-byte line
+  // first level of the last-workgroup ticket: one counter per 128-byte line, and behind it the facts of its
+  // workgroups (report_facts)
   unsigned int ticket_sub[kTicketShards * 32];
 };
 
@@ -143,18 +144,6 @@ struct Snapshot {
   volatile uint64_t arena_top;
   volatile uint64_t seq_end;
 };
-
-// Adds a workgroup's facts (one thread calls it) to those of the other workgroups of a launch of `nblk`. Every
-// workgroup of a request that differs from the cached one finds the same fact, and atomics on one address are
-// served one at a time: a large launch looks first whether somebody has reported it already (a comparison of
-// 4M keys that differ took 52 us, of 4M that do not 12).
-__device__ __forceinline__ void report_facts(DevState* st, unsigned facts, unsigned nblk) {
-  constexpr unsigned kFew = 512;  // so many are under way before anybody could see them
-  if (nblk > kFew &&
-      (facts & ~__hip_atomic_load(&st->req_flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u)
-    return;
-  atomicOr(&st->req_flags, facts);
-}
 
 // What a row-mode kernel needs to know about the request it belongs to.
 struct ReqTag {
@@ -218,6 +207,27 @@ __device__ __forceinline__ bool ticket_last(DevState* st, unsigned nblk) {
   st->ticket_top = 0;
   __threadfence();  // acquire, once per grid: nothing stale is left in this XCD's L2
   return true;
+}
+
+// Adds a workgroup's facts (one thread calls it, before its ticket) to those of the other workgroups of a launch of
+// `nblk`. Every workgroup of a request that differs from the cached one, or has ragged rows, finds the same fact, and
+// accesses to one address past the L2 are served one at a time: they go next to the tickets, one word per line (a
+// comparison of 4M keys that differ took 46 us with one word for all, of keys that do not 12).
+__device__ __forceinline__ void report_facts(DevState* st, unsigned facts, unsigned nblk) {
+  atomicOr(nblk > (unsigned)kTicketShards ? &st->ticket_sub[blockIdx.x % kTicketShards * 32 + 1] : &st->req_flags, facts);
+}
+// All of them, taken away: called by the 64 lanes of one wavefront of the workgroup that finished last.
+__device__ __forceinline__ unsigned take_facts(DevState* st, unsigned nblk) {
+  const unsigned lane = threadIdx.x & 63;
+  unsigned f = 0;
+  if (nblk > (unsigned)kTicketShards) {
+    if (lane < (unsigned)kTicketShards) f = atomicExch(&st->ticket_sub[lane * 32 + 1], 0u);
+  } else if (lane == 0) {
+    f = atomicExch(&st->req_flags, 0u);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) f |= __shfl_xor(f, o);
+  return f;
 }
 
 // A 64-bit value for the workgroup that ticket_last elects: stored past the L2.

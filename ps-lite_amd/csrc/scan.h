@@ -80,7 +80,7 @@ __device__ __forceinline__ void scan_spine(unsigned long long* part, uint64_t np
 // Pass 1, the workgroup's part. Every thread calls it with the sum of its lens, taken as
 // sign-extended 64-bit values modulo 2^64 (what `size_t val_end += int l` does in the
 // reference, kv_app.h:565), and the kReq* facts it found. The workgroup's total goes to
-// part[blockIdx.x], its facts to DevState::req_flags.
+// part[blockIdx.x], its facts to where they are collected.
 // Returns true in every thread of the workgroup that finishes last of the `nblk` that scan this
 // table's request. `red`/`fred` hold kBlock/64 words each.
 __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned flags,
@@ -100,8 +100,11 @@ __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned 
 
 // Pass 1, what the last workgroup does once all totals are there, first half: the facts that the
 // workgroups have collected. Every thread of that workgroup calls it and gets them. `shared` is a word of LDS.
-__device__ __forceinline__ unsigned scan_pass1_facts(DevState* st, unsigned* shared) {
-  if (threadIdx.x == 0) *shared = atomicExch(&st->req_flags, 0u);
+__device__ __forceinline__ unsigned scan_pass1_facts(DevState* st, unsigned nblk, unsigned* shared) {
+  if (threadIdx.x < 64) {
+    const unsigned f = take_facts(st, nblk);
+    if (threadIdx.x == 0) *shared = f;
+  }
   __syncthreads();
   return *shared;
 }

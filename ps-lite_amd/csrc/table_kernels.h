@@ -296,9 +296,9 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
     }
     __syncthreads();
     if (!s_last) return;
-    if (want_outcome && threadIdx.x == 0) {
-      const bool all = (atomicExch(&st->req_flags, 0u) & kReqDiffer) == 0u && per_key;
-      if (d.outcome) *d.outcome = (d.tag.epoch << 1) | (all ? 1ull : 0ull);
+    if (want_outcome && threadIdx.x < 64) {
+      const bool all = (take_facts(st, nblk) & kReqDiffer) == 0u && per_key;
+      if (threadIdx.x == 0 && d.outcome) *d.outcome = (d.tag.epoch << 1) | (all ? 1ull : 0ull);
     }
     if (d.snap && threadIdx.x < 64) publish_snapshot(st, d.snap, d.snap_seq);
     if (want_done && threadIdx.x == 0)
@@ -408,8 +408,9 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
   }
   __syncthreads();
   if (!s_last) return;
-  if (threadIdx.x == 0)
-    decide_same(st, tag, (atomicExch(&st->req_flags, 0u) & kReqDiffer) == 0u && cache_usable(st, tag), d.outcome);
+  if (threadIdx.x >= 64) return;
+  const bool same = (take_facts(st, d.nblk) & kReqDiffer) == 0u && cache_usable(st, tag);
+  if (threadIdx.x == 0) decide_same(st, tag, same, d.outcome);
 }
 
 // A recorded SCALAR request of up to kRepeatGroups workgroups: comparison and values in ONE launch. Nothing
@@ -730,7 +731,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
     flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
   }
   if (!scan_pass1_block(s, flags, part, st, nblk, red, fred, &s_last)) return;
-  flags = scan_pass1_facts(st, &s_last);
+  flags = scan_pass1_facts(st, nblk, &s_last);
   if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && cache_usable(st, tag) ? 1u : 0u;
   __syncthreads();
   const bool same = s_same != 0u;
@@ -973,7 +974,7 @@ __global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch<TABLES> b) 
       if (base + j < n) out_lens[base + j] = l[j];
   }
   if (!scan_pass1_block(s, bits, part, st, nblk, red, fred, &s_last)) return;
-  const unsigned flags = scan_pass1_facts(st, &s_last);
+  const unsigned flags = scan_pass1_facts(st, nblk, &s_last);
   if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && usable ? 1u : 0u;
   __syncthreads();
   const bool same = s_same != 0u;
