@@ -247,6 +247,7 @@ struct pskv_table {
   uint64_t log_keys[kLog] = {0}, log_units[kLog] = {0};
   Snapshot* snap = nullptr;  // pinned host memory the device publishes into
   uint64_t record_seq = ~0ull;  // the newest request that was asked to publish its counters (all ones: none yet)
+  uint64_t unrecorded_keys = 0;  // keys that requests behind it have named
   double new_share = 0.0;  // share of the keys named by requests that were new, over the latest records
   bool share_known = false;  // (a record has said so)
   DevState* st = nullptr;  // device
@@ -672,13 +673,18 @@ struct PublishReq {
   uint64_t seq = 0;
 };
 
+// The share of the keys in flight that is taken to be new: what the latest records say, a quarter more and a
+// tenth, to be on the safe side; all of them while no record has said anything.
+double new_share_at_most(const pskv_table* t) {
+  return t->share_known ? std::min(1.0, 1.25 * t->new_share + 0.1) : 1.0;
+}
+
 int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit, PublishReq* pub) {
   if (t->no_growth) return PSKV_OK;
   // Two limits. `limit` is the fill the table is kept below; `hard` (0.85 unless max_load is higher) is
   // the fill it must never exceed. The keys in flight count in full against the second, and against the
   // first with the share of them that is going to be new if requests go on as the latest records say
-  // (a quarter more than that share plus a tenth, to be on the safe side; in full while no record has said
-  // anything).
+  // (new_share_at_most).
   // A server whose requests mostly name keys it holds, the steady state of a parameter server, then does
   // not grow, or wait, for keys that are not coming, however far ahead of the device its caller runs; if
   // the requests change their ways the table runs fuller than `limit` for as long as it takes the next
@@ -687,9 +693,9 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
   const double hard = std::max((double)t->max_load, kHardLoad) * (double)t->cap;
   auto slots_short = [&]() {
     // (looked up on every call: a record adopted further down may have changed it)
-    const double share = t->share_known ? std::min(1.0, 1.25 * t->new_share + 0.1) : 1.0;
     const double in_flight = (double)(t->pend_keys + n);
-    return (double)t->base_count + in_flight > hard || (double)t->base_count + share * in_flight > limit;
+    return (double)t->base_count + in_flight > hard ||
+           (double)t->base_count + new_share_at_most(t) * in_flight > limit;
   };
   auto arena_short = [&]() {
     return units && (t->base_top + t->pend_units + units) * floats_per_unit > t->arena_cap;
@@ -762,13 +768,23 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
   t->log_units[q % pskv_table::kLog] = units;
   t->pend_keys += n;
   t->pend_units += units;
-  // Close to a limit every request leaves a record; from a third of the way to the next growth on,
-  // every fourth one does (the election of a kernel's last workgroup costs a 1M-key launch about
-  // 6 us): the host then knows how full the table is early enough to have the next array allocated
-  // by the time it is needed.
+  // Close to a limit, as the latest records say how many of the keys in flight are going to be new, every
+  // request leaves a record. From a third of the way to the next growth on every fourth one does, and every
+  // one behind which an eighth of the room below `hard` is unaccounted for (a host that is made to wait there
+  // then has a record near enough to wait for): the host knows how full the table is early enough to have the
+  // next array allocated by the time it is needed. The election of a kernel's last workgroup costs a 1M-key
+  // launch about 6 us, so it is not made for the mere length of the queue: minibatches of keys that are all
+  // held left a record with 96 of 100 requests while keys in flight counted in full here, as soon as the
+  // caller ran a dozen requests ahead (4 pushes and pulls of 1M of 20M held keys: 281 us, with a record for
+  // every fourth 255).
   const double limit_now = (double)t->max_load * (double)t->cap;
-  const double reach = (double)(t->base_count + t->pend_keys + 2 * n);
-  const bool tight_slots = reach > limit_now || (reach > 0.35 * limit_now && q % 4 == 0);
+  const double hard_now = std::max((double)t->max_load, kHardLoad) * (double)t->cap;
+  const double ahead = (double)(t->pend_keys + 2 * n);
+  t->unrecorded_keys += n;
+  const bool tight_slots =
+      (double)t->base_count + new_share_at_most(t) * ahead > limit_now ||
+      ((double)t->base_count + ahead > 0.35 * limit_now &&
+       (q % 4 == 0 || (double)t->unrecorded_keys > 0.125 * (hard_now - (double)t->base_count)));
   const bool tight_arena =
       units && (t->base_top + t->pend_units + 2 * units) * floats_per_unit > t->arena_cap;
   // (a base that merely grows old asks for a record every eighth request, not every one)
@@ -779,6 +795,7 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
     pub->snap = t->snap;
     pub->seq = q;
     t->record_seq = q;
+    t->unrecorded_keys = 0;
     ++t->stats.records;
   }
   return PSKV_OK;

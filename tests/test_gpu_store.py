@@ -277,6 +277,49 @@ def test_a_table_does_not_grow_for_keys_that_are_not_coming(capi, orc, dev, mode
     t.close()
 
 
+@pytest.mark.parametrize("n", [120_000, 700_000])
+def test_held_keys_in_flight_leave_a_record_now_and_then(capi, orc, dev, n):
+    """A caller that runs dozens of requests ahead of the GPU with keys that the table holds (a fill of a third):
+    the queue alone is no reason for a request to leave a counter record, which costs its kernel the election of a
+    last workgroup. Every fourth request leaves one, or every one where a few of them would fill the array (n =
+    700,000 against room for 4.3M); the table neither grows nor waits either way, and holds the right values."""
+    import torch
+    announce("records_of_held_keys", n)
+    rng = np.random.default_rng(n)
+    held, sets, rounds = 2_800_000, 8, 15
+    t, o = capi.Table(capi.MODE_SCALAR, initial_capacity=4_000_000), orc.Store(orc.MODE_SCALAR)
+    base = unique_keys(rng, held)
+    first = rng.standard_normal(held).astype(np.float32)
+    t.push(to_dev(base, dev), to_dev(first, dev))
+    o.push(base, first)
+    t.sync()
+    requests = []
+    for s in range(sets):  # (sizes that differ: no request is compared with the one before it)
+        keys = base[np.sort(rng.choice(held, size=n + s, replace=False))]
+        vals = rng.standard_normal(keys.size).astype(np.float32)
+        requests.append((keys, vals, to_dev(keys, dev), to_dev(vals, dev)))
+    for _, _, dk, dv in requests[:2]:  # the host learns that such requests bring nothing new
+        t.push(dk, dv)
+        torch.cuda.synchronize()
+    before = t.counters()
+    for _ in range(rounds):
+        for _, _, dk, dv in requests:
+            t.push(dk, dv)
+    after = t.counters()
+    made = after["requests"] - before["requests"]
+    records = after["records"] - before["records"]
+    assert made == rounds * sets and after["growths"] == 0 and after["waits"] == 0, after
+    assert made / 5 <= records, (records, made)
+    if n * 4 < (0.85 * after["slots"] - held) / 8:
+        assert records <= made / 3, (records, made)
+    for keys, vals, _, _ in requests[:2]:
+        o.push(keys, vals)
+    for _ in range(rounds):
+        for keys, vals, _, _ in requests:
+            o.push(keys, vals)
+    _check_dump(t, o, "records of held keys")
+
+
 @pytest.mark.parametrize("mode", ["scalar", "fixed", "varlen"])
 def test_many_requests_in_flight_while_the_table_grows(capi, orc, dev, mode):
     """Device-resident requests are enqueued without waiting, so the host only has bounds on the
