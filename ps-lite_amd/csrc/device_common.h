@@ -95,8 +95,7 @@ struct alignas(32) DevState {
   // the value of dirty_epoch up to which the slots have been brought up to date since
   unsigned long long dirty_epoch;
   unsigned long long clean_epoch;
-  // k_scalar_repeat: arrivals of the launch in flight (low half: workgroups, high half: those that found
-  // other keys), and launches served so far << 1 | verdict of the newest
+  // k_scalar_repeat: votes of the launch in flight (vote.h), and launches served so far << 1 | verdict of the newest
   unsigned int repeat_arrived;
   unsigned long long repeat_verdict;
   // keys held (slot array plus the side slot) = sum of the shards

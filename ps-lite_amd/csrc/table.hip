@@ -445,8 +445,8 @@ int report_device_errors(pskv_table* t) {
   PSKV_HIP(hipStreamSynchronize(t->stream));
   if (bits & kDevErrFull) return set_error(PSKV_ENOMEM, "slot array full (internal sizing error)");
   if (bits & kDevErrReplay)
-    return set_error(PSKV_ESTALE, "a replayed request no longer named the keys it was recorded with: that run of it "
-                                  "changed and answered nothing on this table");
+    return set_error(PSKV_ESTALE, "a replayed request no longer named the keys it was recorded with (or was held up for "
+                                  "good): that run of it changed and answered nothing on this table");
   if (bits & kDevErrBadLen)
     return set_error(PSKV_EINVAL, "a length is negative or above PSKV_MAX_VARLEN_ROW");
   if (bits & kDevErrSizeMismatch)
@@ -1144,6 +1144,10 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   }
   if (one_launch) {
     const bool few = repeat_quads == kRepeatFew;
+    // (the environment variable, read when a request is recorded, is for tests of the wait that runs out)
+    unsigned looks = kRepeatLooks;
+    if (const char* e = std::getenv("PSKV_REPEAT_LOOKS")) looks = (unsigned)std::strtoul(e, nullptr, 10);
+    for (Item& it : bt) it.d.cache_mode = looks;
     const KernelSet kernels =
         push && pull ? (few ? PSKV_KSET_OF(k_scalar_repeat, true, true, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, true, true, kRepeatMany))
         : push       ? (few ? PSKV_KSET_OF(k_scalar_repeat, true, false, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, true, false, kRepeatMany))

@@ -9,6 +9,7 @@
 #define PSKV_TABLE_KERNELS_H_
 #include "device_common.h"
 #include "scan.h"
+#include "vote.h"
 
 namespace pskv {
 
@@ -38,7 +39,7 @@ struct TableHead {
   unsigned long long* outcome;  // pinned host word that learns how the comparison went, or null; SCALAR
                                 // without the key cache: the word that takes tag.epoch when the request is done
   uint32_t nblk;        // workgroups of the launch in flight that serve this table
-  uint32_t cache_mode;  // kCache* below
+  uint32_t cache_mode;  // kCache* below; k_scalar_repeat: looks for the outcome before a workgroup leaves
 };
 struct TableReq : TableHead {
   const int32_t* lens;   // VARLEN push: n row lengths
@@ -420,23 +421,49 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
 // keys: 4.6 + 3.6 us and the gap between them, now 5.7; the calling thread makes one launch instead of two, and a
 // recorded step 8.8 -> 4.2 us).
 // All workgroups have to be on the GPU together: 64 of 1,024 threads are an eighth of what it holds, so twice as
-// many such launches fit side by side as a process has hardware queues to run them from. A workgroup whose wait
-// does not end within about a second all the same (kRepeatSpins) applies nothing and leaves the replay error.
+// many such launches fit side by side as a process has hardware queues to run them from. Something else may hold up
+// a part of them all the same (a long kernel of small workgroups on another stream, another process): a workgroup
+// that has looked for the outcome for about a second (kRepeatLooks) leaves, and nobody applies anything then
+// (vote.h); the run counts as one that named other keys.
 constexpr unsigned kRepeatBlock = 1024;
 constexpr unsigned kRepeatGroups = 64;
-constexpr unsigned kRepeatSpins = 1u << 20;
+constexpr unsigned kRepeatLooks = 1u << 20;
 // Quads of keys per thread: one while the request fits into kRepeatGroups workgroups that way (262,144 keys), two
 // up to twice that; beyond it the two kernels that fill the GPU are as quick (with four quads the registers spill).
 constexpr unsigned kRepeatFew = 1, kRepeatMany = 2;
 typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+// (the memory of vote(): words that are only ever touched by atomics, past the per-XCD L2)
+template <bool PUSH>
+struct RepeatVotes {
+  DevState* st;
+  const TableHead& d;
+  unsigned long long before;  // the verdict of the launch before this one
+  __device__ unsigned add(unsigned x) { return atomicAdd(&st->repeat_arrived, x); }
+  __device__ unsigned word() { return __hip_atomic_load(&st->repeat_arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  __device__ bool swap(unsigned from, unsigned to) { return atomicCAS(&st->repeat_arrived, from, to) == from; }
+  __device__ bool publish(bool yes) {
+    const bool same = yes && cache_usable(st, d.tag);
+    decide_same(st, d.tag, same, d.outcome);
+    if (PUSH && same) st->dirty_epoch = d.tag.epoch;  // the slots fall behind
+    __hip_atomic_store(&st->repeat_arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&st->repeat_verdict, ((before >> 1) + 1) << 1 | (same ? 1ull : 0ull), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    return same;
+  }
+  __device__ int outcome() {
+    const unsigned long long now = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return now == before ? -1 : (int)(now & 1ull);
+  }
+  __device__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
+
 template <bool PUSH, bool PULL, unsigned QUADS, int TABLES>
 __global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(HeadBatch<TABLES> b) {
   const TableHead& d = b.t[blockIdx.y];
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
   DevState* st = d.st;
-  const ReqTag tag = d.tag;
   __shared__ unsigned s_same;
   unsigned long long before = 0;  // (nobody changes the verdict before this workgroup has arrived)
   if (threadIdx.x == 0)
@@ -475,26 +502,10 @@ __global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(HeadBatch<TABLES
     differ |= x0[q].x != y0[q].x || x0[q].y != y0[q].y || x1[q].x != y1[q].x || x1[q].y != y1[q].y;
   const bool any = __syncthreads_or(differ ? 1 : 0) != 0;
   if (threadIdx.x == 0) {
-    const unsigned old = atomicAdd(&st->repeat_arrived, any ? 0x10001u : 1u);
-    bool same = false;
-    if ((old & 0xffffu) == nblk - 1) {
-      same = !any && (old >> 16) == 0u && cache_usable(st, tag);
-      decide_same(st, tag, same, d.outcome);
-      if (PUSH && same) st->dirty_epoch = tag.epoch;  // the slots fall behind
-      st->repeat_arrived = 0u;
-      __hip_atomic_store(&st->repeat_verdict, ((before >> 1) + 1) << 1 | (same ? 1ull : 0ull), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-      unsigned long long now = before;
-      for (unsigned spin = 0; spin < kRepeatSpins; ++spin) {
-        now = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (now != before) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      same = now != before && (now & 1ull) != 0ull;
-      if (now == before) atomicOr(&st->error, kDevErrReplay);
-    }
-    s_same = same ? 1u : 0u;
+    // (the old verdict has to be here before the vote goes out, behind which it may change)
+    asm volatile("" : "+v"(before) : : "memory");
+    RepeatVotes<PUSH> votes{st, d, before};
+    s_same = vote(votes, nblk, !any, d.cache_mode) ? 1u : 0u;
   }
   __syncthreads();
   if (!s_same) return;

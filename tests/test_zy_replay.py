@@ -351,3 +351,56 @@ def test_scalar_repeats_at_the_edges_of_their_launches(capi, orc, dev, S, n, how
     rec.close()
     _check_dump(g, o, "after a repeat with another key")
     g.close()
+
+
+@pytest.mark.parametrize("S,n", [(1, 9000), (1, 262_144), (1, 400_000), (4, 100_000), (4, 200_001)])
+@pytest.mark.parametrize("what", ["push+pull", "push"])
+def test_a_replay_that_nobody_waits_for_is_applied_whole_or_not_at_all(capi, orc, dev, monkeypatch, S, n, what):
+    """The workgroups of a recorded SCALAR request wait for each other before they apply anything. With a wait of no
+    looks at all, a workgroup leaves as soon as it finds that the others have not arrived: of every table's share
+    either all is applied and answered or nothing is, the error says which, and the run after it is as good as
+    any."""
+    import torch
+    announce("replay_no_wait", S, n, what)
+    monkeypatch.setenv("PSKV_REPEAT_LOOKS", "0")
+    rng = np.random.default_rng(n + S)
+    g = capi.Group(S, capi.MODE_SCALAR, initial_capacity=4 * n)
+    keys = unique_keys(rng, n, S)
+    st = _Step(capi, dev, rng, "scalar", S, keys, None, n)
+    first = rng.normal(0, 1, size=n).astype(np.float32)
+    st.set_vals(first)
+    flags = capi.REPLAY_PUSH | capi.REPLAY_LAUNCHES | (capi.REPLAY_PULL if "pull" in what else 0)
+    rec = g.record(flags, st.dk, st.pos, st.dv, st.vpos, None, st.out if "pull" in what else None,
+                   st.out_pos if "pull" in what else None)
+    held = first.copy()  # what the tables hold, in request order
+    applied = refused = 0
+    for rnd in range(12):
+        vals = rng.normal(0, 1, size=n).astype(np.float32)
+        st.set_vals(vals)
+        rec.run()
+        left = [False] * S
+        for s in range(S):  # (table by table: the error word is the table's own)
+            try:
+                g.tables[s].sync()
+            except capi.PskvError as e:
+                assert e.code == capi.ESTALE, e
+                left[s] = True
+        out = st.answered()
+        for s in range(S):
+            at = slice(int(st.pos[s]), int(st.pos[s + 1]))
+            if left[s]:
+                refused += 1
+                if "pull" in what:
+                    assert (out[at] == 7.0).all(), (rnd, s, "answered although it was given up")
+            else:
+                applied += 1
+                held[at] = held[at] + vals[at]
+                if "pull" in what:
+                    assert_bits_equal(out[at], held[at], "round %d table %d" % (rnd, s))
+    print("[case] applied", applied, "given up", refused, flush=True)
+    monkeypatch.delenv("PSKV_REPEAT_LOOKS")
+    rec.close()
+    gk, _, gv = _dump_all(g)  # (what the slots hold once the cached values have been written back)
+    assert np.array_equal(gk, keys)
+    assert_bits_equal(gv, held, "held")
+    g.close()
