@@ -27,12 +27,14 @@ struct Idle {
   size_t bytes;
   hipStream_t stream;  // whose work may still use it ...
   hipEvent_t done;     // ... until this event; null: nothing does
+  unsigned long long number;  // of its release
 };
 
 struct Pool {
   std::mutex mu;
   std::list<Idle> idle;  // oldest first
   size_t kept = 0;
+  unsigned long long releases = 0;  // so far
   std::unordered_map<void*, size_t> size_of;  // every array handed out
   std::vector<hipEvent_t> events;             // for reuse
 };
@@ -146,7 +148,7 @@ int array_alloc(void** out, size_t bytes, hipStream_t stream) {
   Pool* p = pool_of(dev);
   if (!p) return set_error(PSKV_EINVAL, "device %d out of range", dev);
   bytes = rounded(bytes ? bytes : 1);
-  Idle got = {nullptr, 0, nullptr, nullptr};
+  Idle got = {nullptr, 0, nullptr, nullptr, 0};
   {
     std::lock_guard<std::mutex> lk(p->mu);
     // the smallest that fits without wasting more than a quarter; among equals one that nothing waits for
@@ -200,7 +202,7 @@ int array_release(void* ptr, hipStream_t stream, bool idle) {
   int dev = 0;
   PSKV_HIP(hipGetDevice(&dev));
   Pool* p = pool_of(dev);
-  Idle i = {ptr, 0, stream, nullptr};
+  Idle i = {ptr, 0, stream, nullptr, 0};
   std::vector<Idle> over;
   {
     std::lock_guard<std::mutex> lk(p->mu);
@@ -223,6 +225,7 @@ int array_release(void* ptr, hipStream_t stream, bool idle) {
       }
     }
     i.bytes = it->second;
+    i.number = ++p->releases;
     p->size_of.erase(it);
     p->idle.push_back(i);
     p->kept += i.bytes;
@@ -236,13 +239,21 @@ int array_release(void* ptr, hipStream_t stream, bool idle) {
   return PSKV_OK;
 }
 
-void array_settle(hipStream_t stream) {
+unsigned long long array_mark() {
+  int dev = 0;
+  Pool* p = hipGetDevice(&dev) == hipSuccess ? pool_of(dev) : nullptr;
+  if (!p) return 0;
+  std::lock_guard<std::mutex> lk(p->mu);
+  return p->releases;
+}
+
+void array_settle(hipStream_t stream, unsigned long long mark) {
   int dev = 0;
   Pool* p = hipGetDevice(&dev) == hipSuccess ? pool_of(dev) : nullptr;
   if (!p) return;
   std::lock_guard<std::mutex> lk(p->mu);
   for (Idle& i : p->idle) {
-    if (!i.done || i.stream != stream) continue;
+    if (!i.done || i.stream != stream || i.number > mark) continue;
     p->events.push_back(i.done);
     i.done = nullptr;
   }

@@ -85,3 +85,42 @@ def test_an_array_another_stream_is_still_using(capi, orc, dev):
             assert np.array_equal(dk, ok)
             assert_bits_equal(dv, ov)
             t.close()
+
+
+def test_tables_of_several_threads_on_one_stream(capi, orc, dev):
+    """Two threads drive tables of their own on ONE stream of the caller's while a third creates tables on streams of
+    their own, which take over what the others give up: the end of a table, which waits for the shared stream, says
+    nothing about arrays that the other thread gives up after that wait."""
+    import torch
+    announce("pool shared stream")
+    shared = torch.cuda.Stream(device=dev)
+    failed = []
+
+    def work(seed, stream):
+        try:
+            rng = np.random.default_rng(seed)
+            for _ in range(8):
+                n = 60_000 + 1000 * seed
+                t, o = capi.Table(capi.MODE_SCALAR, initial_capacity=2000, stream=stream), orc.Store(orc.MODE_SCALAR)
+                keep = []
+                for _ in range(3):
+                    keys, vals = unique_keys(rng, n), rng.standard_normal(n).astype(np.float32)
+                    keep.append((to_dev(keys, dev), to_dev(vals, dev)))
+                    torch.cuda.current_stream().synchronize()
+                    t.push(*keep[-1])
+                    o.push(keys, vals)
+                dk, _, dv = t.dump()
+                ok, _, ov = o.dump()
+                assert np.array_equal(dk, ok)
+                assert_bits_equal(dv, ov)
+                t.close()
+        except BaseException as e:  # noqa: B036 (reported by the main thread)
+            failed.append((seed, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(s, stream)) for s, stream in
+               enumerate([shared.cuda_stream, shared.cuda_stream, 0])]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not failed, failed
