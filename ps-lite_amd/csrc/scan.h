@@ -99,14 +99,17 @@ __device__ __forceinline__ bool scan_pass1_block(unsigned long long s, unsigned 
 }
 
 // Pass 1, what the last workgroup does once all totals are there, first half: the facts that the
-// workgroups have collected. Every thread of that workgroup calls it and gets them. `shared` is a word of LDS.
-__device__ __forceinline__ unsigned scan_pass1_facts(DevState* st, unsigned nblk, unsigned* shared) {
+// workgroups have collected. Every thread of that workgroup calls it and gets them.
+// (The word is its own: the one that says which workgroup is the last may still be unread by a wavefront that is
+// late when the first one gets here.)
+__device__ __forceinline__ unsigned scan_pass1_facts(DevState* st, unsigned nblk) {
+  __shared__ unsigned s_facts;
   if (threadIdx.x < 64) {
     const unsigned f = take_facts(st, nblk);
-    if (threadIdx.x == 0) *shared = f;
+    if (threadIdx.x == 0) s_facts = f;
   }
   __syncthreads();
-  return *shared;
+  return s_facts;
 }
 
 // Second half: turns the totals into exclusive offsets in place and stores the grand total, unless the

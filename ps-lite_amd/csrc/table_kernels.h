@@ -742,7 +742,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
     flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
   }
   if (!scan_pass1_block(s, flags, part, st, nblk, red, fred, &s_last)) return;
-  flags = scan_pass1_facts(st, nblk, &s_last);
+  flags = scan_pass1_facts(st, nblk);
   if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && cache_usable(st, tag) ? 1u : 0u;
   __syncthreads();
   const bool same = s_same != 0u;
@@ -985,7 +985,7 @@ __global__ __launch_bounds__(kBlock) void k_var_pull_lookup(ReqBatch<TABLES> b) 
       if (base + j < n) out_lens[base + j] = l[j];
   }
   if (!scan_pass1_block(s, bits, part, st, nblk, red, fred, &s_last)) return;
-  const unsigned flags = scan_pass1_facts(st, nblk, &s_last);
+  const unsigned flags = scan_pass1_facts(st, nblk);
   if (threadIdx.x == 0) s_same = !(flags & kReqDiffer) && usable ? 1u : 0u;
   __syncthreads();
   const bool same = s_same != 0u;
