@@ -236,6 +236,9 @@ int Stager::to_device(void* dst, const void* src, size_t bytes, hipStream_t cons
 
 int Stager::to_host(void* dst, const void* src, size_t bytes, hipStream_t producer,
                     const std::function<int(size_t, size_t)>& produce) {
+  // A slot that this transfer fills may still be read by a copy command of the transfer before it: no wait is made
+  // for that, both are on the same stream (piece c lies in slot c % kSlots and goes over stream c % kStreams).
+  static_assert(kSlots % kStreams == 0, "a slot always meets the same stream");
   Impl* im = impl_;
   std::lock_guard<std::mutex> op(im->op_mu);
   const std::vector<size_t> at = cut(bytes, false);
