@@ -769,22 +769,20 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
   t->pend_keys += n;
   t->pend_units += units;
   // Close to a limit, as the latest records say how many of the keys in flight are going to be new, every
-  // request leaves a record. From a third of the way to the next growth on every fourth one does, and every
-  // one behind which an eighth of the room below `hard` is unaccounted for (a host that is made to wait there
-  // then has a record near enough to wait for): the host knows how full the table is early enough to have the
-  // next array allocated by the time it is needed. The election of a kernel's last workgroup costs a 1M-key
-  // launch about 6 us, so it is not made for the mere length of the queue: minibatches of keys that are all
-  // held left a record with 96 of 100 requests while keys in flight counted in full here, as soon as the
-  // caller ran a dozen requests ahead (4 pushes and pulls of 1M of 20M held keys: 281 us, with a record for
-  // every fourth 255).
+  // request leaves a record; from a third of the way to the next growth on, every fourth one does: the host then
+  // knows how full the table is early enough to have the next array allocated by the time it is needed. The
+  // election of a kernel's last workgroup costs a 1M-key launch about 6 us, so it is not made with every request for
+  // the mere length of the queue: minibatches of keys that are all held left a record with 96 of 100 requests while
+  // keys in flight counted in full here, as soon as the caller ran a dozen requests ahead (4 pushes and pulls of 1M of
+  // 20M held keys: 281 us, with a record for every fourth 255). A long queue leaves them by the keys as well, one for
+  // an eighth of the room below `hard`: a host that is held back there waits for the next record.
   const double limit_now = (double)t->max_load * (double)t->cap;
   const double hard_now = std::max((double)t->max_load, kHardLoad) * (double)t->cap;
-  const double ahead = (double)(t->pend_keys + 2 * n);
+  const double base = (double)t->base_count, ahead = (double)(t->pend_keys + 2 * n);
   t->unrecorded_keys += n;
   const bool tight_slots =
-      (double)t->base_count + new_share_at_most(t) * ahead > limit_now ||
-      ((double)t->base_count + ahead > 0.35 * limit_now &&
-       (q % 4 == 0 || (double)t->unrecorded_keys > 0.125 * (hard_now - (double)t->base_count)));
+      base + new_share_at_most(t) * ahead > limit_now || (base + ahead > 0.35 * limit_now && q % 4 == 0) ||
+      (base + ahead > limit_now && (double)t->unrecorded_keys > 0.125 * (hard_now - base));
   const bool tight_arena =
       units && (t->base_top + t->pend_units + 2 * units) * floats_per_unit > t->arena_cap;
   // (a base that merely grows old asks for a record every eighth request, not every one)
