@@ -339,7 +339,8 @@ int pskv_table_counters(pskv_table* t, uint64_t* out, size_t cap);
  * milliseconds; the list serves later growths and tables, of any thread and stream), the fixed-size
  * state and pinned request buffers of destroyed tables (up to 32 of them) and the workspaces
  * and staging buffers of pskv_match, which only grow (a 16M-key host-resident call leaves
- * several GiB behind). Memory in use by live tables is not touched. Calls of pskv_match on
+ * several GiB behind). All but the last goes back by itself some time (two seconds) after the last table of
+ * the device has gone. Memory in use by live tables is not touched. Calls of pskv_match on
  * the device wait for it and it for them. */
 int pskv_device_trim(int device);
 

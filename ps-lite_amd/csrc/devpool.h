@@ -28,6 +28,15 @@ unsigned long long array_mark();
 void array_settle(hipStream_t stream, unsigned long long mark);
 // Frees every array on the list of `device` (current). Waits for those that are still in use.
 void array_trim(int device);
+// False with PSKV_NO_ASYNC_ALLOC in the environment: arrays come from hipMalloc and go to hipFree, nothing is kept.
+bool arrays_are_kept();
+
+// A table of `device` has come (`tables` = 1) or gone (-1). What tables leave is there for the next ones, so it goes
+// back when there are none: kLingerMs after the last table of the device has gone, unless another has come by then,
+// a thread of the library's own calls `give_back` (with the device current). A program that drops its tables and makes others, the
+// case the lists are for, does so within that time; giving back at once is what cost it 25 to 160 ms.
+constexpr int kLingerMs = 2000;
+void device_tables(int device, int tables, void (*give_back)(int device));
 
 // Allocations made by a thread of the library's own: allocating a few hundred MB costs the calling
 // thread 50 us on a good day and 800 on a bad one, so the array of a coming growth is asked for

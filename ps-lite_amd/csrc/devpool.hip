@@ -1,10 +1,11 @@
-// The lists of device arrays behind devpool.h and the thread that allocates ahead and frees behind.
+// The lists of device arrays behind devpool.h and the threads that allocate ahead, free behind and give back.
 #include "devpool.h"
 
+#include <algorithm>
 #include <chrono>
 #include <condition_variable>
+#include <cstdlib>
 #include <deque>
-#include <algorithm>
 #include <list>
 #include <mutex>
 #include <thread>
@@ -49,6 +50,47 @@ size_t rounded(size_t bytes) {
   return (bytes + step - 1) / step * step;
 }
 
+// The threads below must not be inside the runtime when the process takes that down: once it is ending they free and
+// give back nothing any more, and what they are at is waited for. (An array that somebody still asks for is still
+// allocated: whoever asks waits for it.)
+class Gate {
+ public:
+  static Gate& get() {
+    static Gate* g = new Gate();  // never destroyed, like the threads
+    return *g;
+  }
+  bool enter() {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (ending_) return false;
+    ++inside_;
+    return true;
+  }
+  void leave() {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (--inside_ == 0) cv_.notify_all();
+  }
+
+ private:
+  Gate() {
+    std::atexit([] {
+      Gate& g = get();
+      std::unique_lock<std::mutex> lk(g.mu_);
+      g.ending_ = true;
+      g.cv_.wait(lk, [&] { return g.inside_ == 0; });
+    });
+  }
+  std::mutex mu_;
+  std::condition_variable cv_;
+  int inside_ = 0;
+  bool ending_ = false;
+};
+
+// (other threads of the process may be capturing a stream: what the threads here allocate and free is no part of that)
+void relaxed_capture() {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
 // One thread per process, started with the first job, kept until the process ends.
 class Worker {
  public:
@@ -84,6 +126,7 @@ class Worker {
  private:
   void start() {
     if (started_) return;
+    (void)Gate::get();
     std::thread(&Worker::run, this).detach();
     started_ = true;
   }
@@ -92,6 +135,77 @@ class Worker {
   std::condition_variable cv_job_, cv_done_;
   std::deque<std::shared_ptr<AllocJob>> jobs_;
   std::deque<std::pair<int, Idle>> frees_;
+  bool started_ = false;
+};
+
+// Counts the tables of every device and gives back what they have left some time after the last one has gone, by a
+// thread of its own (one that waits with a timer costs the arrays that the other one allocates 2 us each).
+class Keeper {
+ public:
+  static Keeper& get() {
+    static Keeper* k = new Keeper();  // never destroyed
+    return *k;
+  }
+  void tables(int device, int change, void (*give_back)(int)) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      Device& d = devices_[device];
+      d.tables += change;
+      d.due = change < 0 && d.tables == 0;
+      if (!d.due) return;
+      d.when = Clock::now() + std::chrono::milliseconds(kLingerMs);
+      d.give_back = give_back;
+      if (!started_) {
+        (void)Gate::get();
+        std::thread(&Keeper::run, this).detach();
+        started_ = true;
+      }
+      // (waking the thread costs a program that makes and drops one table after the other 5 us each time: one that is
+      // going to look in time anyway is left alone)
+      if (wakes_ <= d.when) return;
+    }
+    cv_.notify_one();
+  }
+
+ private:
+  typedef std::chrono::steady_clock Clock;
+  struct Device {
+    long tables = 0;
+    bool due = false;  // what is kept goes back at `when`
+    Clock::time_point when;
+    void (*give_back)(int) = nullptr;
+  };
+  void run() {
+    relaxed_capture();
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+      Clock::time_point next = Clock::time_point::max();
+      int device = -1;
+      const Clock::time_point now = Clock::now();
+      for (int d = 0; d < kMaxDevices; ++d) {
+        if (!devices_[d].due) continue;
+        if (devices_[d].when <= now) device = d; else next = std::min(next, devices_[d].when);
+      }
+      if (device < 0) {
+        wakes_ = next;
+        if (next == Clock::time_point::max()) cv_.wait(lk); else cv_.wait_until(lk, next);
+        wakes_ = Clock::time_point::min();
+        continue;
+      }
+      devices_[device].due = false;
+      void (*give_back)(int) = devices_[device].give_back;
+      lk.unlock();
+      if (Gate::get().enter()) {
+        if (hipSetDevice(device) == hipSuccess) give_back(device);
+        Gate::get().leave();
+      }
+      lk.lock();
+    }
+  }
+  std::mutex mu_;
+  std::condition_variable cv_;
+  Device devices_[kMaxDevices];
+  Clock::time_point wakes_ = Clock::time_point::min();  // when the thread is going to look by itself
   bool started_ = false;
 };
 
@@ -106,6 +220,7 @@ void free_now(Pool* p, const Idle& i) {
 }
 
 void Worker::run() {
+  relaxed_capture();
   for (;;) {
     std::shared_ptr<AllocJob> job;
     std::pair<int, Idle> gone;
@@ -120,8 +235,10 @@ void Worker::run() {
         frees_.pop_front();
       }
     }
+    const bool inside = Gate::get().enter();
     if (!job) {
-      if (hipSetDevice(gone.first) == hipSuccess) free_now(pool_of(gone.first), gone.second);
+      if (inside && hipSetDevice(gone.first) == hipSuccess) free_now(pool_of(gone.first), gone.second);
+      if (inside) Gate::get().leave();
       continue;
     }
     const auto a0 = std::chrono::steady_clock::now();
@@ -137,6 +254,7 @@ void Worker::run() {
       job->done = true;
     }
     cv_done_.notify_all();
+    if (inside) Gate::get().leave();
   }
 }
 
@@ -148,6 +266,10 @@ int array_alloc(void** out, size_t bytes, hipStream_t stream) {
   Pool* p = pool_of(dev);
   if (!p) return set_error(PSKV_EINVAL, "device %d out of range", dev);
   bytes = rounded(bytes ? bytes : 1);
+  if (!arrays_are_kept()) {
+    PSKV_HIP(hipMalloc(out, bytes));
+    return PSKV_OK;
+  }
   Idle got = {nullptr, 0, nullptr, nullptr, 0};
   {
     std::lock_guard<std::mutex> lk(p->mu);
@@ -197,8 +319,18 @@ int array_alloc(void** out, size_t bytes, hipStream_t stream) {
   return PSKV_OK;
 }
 
+bool arrays_are_kept() {
+  static const bool kept = std::getenv("PSKV_NO_ASYNC_ALLOC") == nullptr;
+  return kept;
+}
+
 int array_release(void* ptr, hipStream_t stream, bool idle) {
   if (!ptr) return PSKV_OK;
+  if (!arrays_are_kept()) {
+    if (!idle) PSKV_HIP(hipStreamSynchronize(stream));
+    PSKV_HIP(hipFree(ptr));
+    return PSKV_OK;
+  }
   int dev = 0;
   PSKV_HIP(hipGetDevice(&dev));
   Pool* p = pool_of(dev);
@@ -269,6 +401,10 @@ void array_trim(int device) {
     p->kept = 0;
   }
   for (const Idle& i : all) free_now(p, i);
+}
+
+void device_tables(int device, int tables, void (*give_back)(int device)) {
+  if (device >= 0 && device < kMaxDevices) Keeper::get().tables(device, tables, give_back);
 }
 
 void alloc_submit(const std::shared_ptr<AllocJob>& job) { Worker::get().submit(job); }

@@ -131,7 +131,8 @@ __global__ void k_read_state(StateBatch sb) {
 // The parts of a table that have one size whatever the table holds: device state, the pinned words and
 // request buffers, events, its stream. Creating them costs the calling thread about a millisecond (every
 // pinned allocation and its release go through the driver), so a table that goes leaves its shell to
-// the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim.
+// the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim, and
+// some time after the last table of the device has gone.
 struct Shell {
   DevState* st = nullptr;
   char* pinned = nullptr;  // StateView, Snapshot, outcome word, done word (256 bytes each), small_in, small_out
@@ -187,7 +188,7 @@ Shell* shell_take(int device) {
 
 void shell_give(int device, Shell* sh) {
   if (!sh) return;
-  if (device < 64) {
+  if (device < 64 && arrays_are_kept()) {
     ShellPool& p = g_shells[device];
     std::lock_guard<std::mutex> lk(p.mu);
     if (p.idle.size() < kShellsKept) {
@@ -198,7 +199,7 @@ void shell_give(int device, Shell* sh) {
   shell_free(sh);
 }
 
-// pskv_device_trim (with `device` current): idle shells go.
+// With `device` current: idle shells go.
 void shell_trim(int device) {
   std::vector<Shell*> go;
   {
@@ -206,6 +207,12 @@ void shell_trim(int device) {
     go.swap(g_shells[device].idle);
   }
   for (Shell* sh : go) shell_free(sh);
+}
+
+// What tables that are gone have left (`device` is current).
+void give_back(int device) {
+  array_trim(device);
+  if (device < 64) shell_trim(device);
 }
 
 }  // namespace
@@ -2016,6 +2023,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   t->mode = opts->mode;
   t->max_load = opts->max_load > 0.f ? opts->max_load : 0.5f;
   t->row_len = opts->mode == PSKV_MODE_FIXED ? opts->row_len : 0;
+  device_tables(t->device, 1, give_back);
   t->sc_min_keys = kScalarCacheMinKeys;
   if (const char* e = std::getenv("PSKV_SCALAR_CACHE_MIN_KEYS")) t->sc_min_keys = std::strtoull(e, nullptr, 10);
   auto fail = [&](int rc) {
@@ -2089,6 +2097,7 @@ int pskv_table_destroy(pskv_table* t) {
                            &t->sc_vals, &t->sc_slots})
     (void)array_release(b->ptr, t->stream, idle);
   shell_give(t->device, t->shell);
+  device_tables(t->device, -1, give_back);
   delete t;
   return PSKV_OK;
 }
@@ -2440,8 +2449,7 @@ int pskv_device_trim(int device) {
   if (device < 0 || device >= 64) return set_error(PSKV_EINVAL, "device %d out of range", device);
   DeviceGuard guard(device);
   if (!guard.ok()) return set_error(PSKV_EHIP, "cannot select device %d", device);
-  array_trim(device);
-  shell_trim(device);
+  give_back(device);
   return match_trim(device);
 }
 

@@ -12,6 +12,7 @@
 #include <vector>
 
 enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorInvalidValue = 1 };
+enum hipStreamCaptureMode { hipStreamCaptureModeRelaxed = 2 };
 struct HostStream {
   unsigned long queued = 0, done = 0;
 };
@@ -39,6 +40,7 @@ inline const char* hipGetErrorString(hipError_t) { return "error"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t bytes) {
   std::lock_guard<std::mutex> lk(host_hip().mu);
   if (host_hip().live_bytes + bytes > host_hip().room) return hipErrorOutOfMemory;

@@ -18,7 +18,11 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["settle"])
-def test_arrays_change_hands_safely(program, what):
-    out = subprocess.run([program, what], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+@pytest.mark.parametrize("what", ["settle", "linger", "bound", "unkept"])
+def test_arrays_change_hands_and_go_back(program, what):
+    env = dict(os.environ)
+    env.pop("PSKV_NO_ASYNC_ALLOC", None)
+    if what == "unkept":
+        env["PSKV_NO_ASYNC_ALLOC"] = "1"
+    out = subprocess.run([program, what], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60, env=env)
     assert out.returncode == 0 and out.stdout.endswith("ok\n"), out.stdout

@@ -1,11 +1,14 @@
 """Device arrays and table state that one table leaves and the next one takes over."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
 import pytest
 
 from helpers import assert_bits_equal, to_dev, unique_keys
-from conftest import announce
+from conftest import REPO, announce
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +127,62 @@ def test_tables_of_several_threads_on_one_stream(capi, orc, dev):
     for th in threads:
         th.join()
     assert not failed, failed
+
+
+_GIVES_BACK = """
+import importlib, sys, time
+sys.path.insert(0, %r)
+import numpy as np, torch
+capi = importlib.import_module("ps-lite_amd").capi
+kept = sys.argv[1] == "kept"
+x, g = torch.zeros(1000, device="cuda"), torch.cuda.CUDAGraph()
+free = lambda: torch.cuda.mem_get_info()[0]
+def table():
+    t = capi.Table(capi.MODE_SCALAR, initial_capacity=1 << 26)  # 2 GiB of slots
+    keys = np.arange(1, 100_000, dtype=np.uint64)
+    t.push(keys, np.ones(keys.size, np.float32))
+    t.sync()
+    return t
+table().close()
+capi.device_trim()
+torch.cuda.synchronize()
+before = free()
+t = table()
+assert free() <= before - (2 << 30), "a table of 2 GiB takes 2 GiB"
+t.close()
+left = before - free()
+assert (left >= (2 << 30)) == kept, left
+if kept:  # in the middle of somebody's capture, which must not notice
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        x += 1
+        torch.cuda.synchronize()
+        g.capture_begin()
+        x += 1
+        time.sleep(3)
+        g.capture_end()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+    assert (x == 4).all(), x[:4]
+assert before - free() < (64 << 20), before - free()
+t = table()  # and again
+t.close()
+print("ok", flush=True)
+"""
+
+
+@pytest.mark.parametrize("how", ["kept", "not kept"])
+def test_the_last_table_gives_the_memory_back(capi, dev, how):
+    """What tables have left goes back to the system some time after the last one has gone, also while another thread
+    captures a stream; with PSKV_NO_ASYNC_ALLOC in the environment nothing is kept to begin with. (In a process of
+    its own, where no other table is.)"""
+    announce("gives back", how)
+    env = dict(os.environ)
+    env.pop("PSKV_NO_ASYNC_ALLOC", None)
+    if how != "kept":
+        env["PSKV_NO_ASYNC_ALLOC"] = "1"
+    out = subprocess.run([sys.executable, "-c", _GIVES_BACK % REPO, how], stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                         text=True, timeout=90, env=env)
+    assert out.returncode == 0 and out.stdout.strip().endswith("ok"), out.stdout
