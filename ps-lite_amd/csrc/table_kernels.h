@@ -418,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
 // may change or be answered before every key of the table's share is known to be the cached one, so the
 // workgroups of a table wait for each other in between: all loads are under way by then, and the wait (an atomic
 // and a look at its outcome) is shorter than the end of one kernel and the start of the next (4 tables of 25,000
-// keys: 4.6 + 3.6 us and the gap between them, now 5.7; the calling thread makes one launch instead of two, and a
+// keys: 4.6 + 3.6 us and the gap between them, now 5.5; the calling thread makes one launch instead of two, and a
 // recorded step 8.8 -> 4.2 us).
 // All workgroups have to be on the GPU together: 64 of 1,024 threads are an eighth of what it holds, so twice as
 // many such launches fit side by side as a process has hardware queues to run them from. Something else may hold up
@@ -437,15 +437,15 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 template <bool PUSH>
 struct RepeatVotes {
   DevState* st;
-  const TableHead& d;
+  ReqTag tag;
+  unsigned long long* told;   // (pinned: the outcome for the host)
   unsigned long long before;  // the verdict of the launch before this one
   __device__ unsigned add(unsigned x) { return atomicAdd(&st->repeat_arrived, x); }
   __device__ unsigned word() { return __hip_atomic_load(&st->repeat_arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
   __device__ bool swap(unsigned from, unsigned to) { return atomicCAS(&st->repeat_arrived, from, to) == from; }
-  __device__ bool publish(bool yes) {
-    const bool same = yes && cache_usable(st, d.tag);
-    decide_same(st, d.tag, same, d.outcome);
-    if (PUSH && same) st->dirty_epoch = d.tag.epoch;  // the slots fall behind
+  __device__ bool publish(bool same) {
+    decide_same(st, tag, same, told);
+    if (PUSH && same) st->dirty_epoch = tag.epoch;  // the slots fall behind
     __hip_atomic_store(&st->repeat_arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&st->repeat_verdict, ((before >> 1) + 1) << 1 | (same ? 1ull : 0ull), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
@@ -464,10 +464,18 @@ __global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(HeadBatch<TABLES
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
   DevState* st = d.st;
+  const unsigned looks = d.cache_mode;
   __shared__ unsigned s_same;
-  unsigned long long before = 0;  // (nobody changes the verdict before this workgroup has arrived)
-  if (threadIdx.x == 0)
-    before = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // (nobody changes the verdict before this workgroup has voted, nor what says that the cache is usable; both are asked
+  // for with the keys, and the arguments that the last vote needs as well: between the votes and the outcome nothing
+  // is fetched)
+  RepeatVotes<PUSH> votes{st, d.tag, d.outcome, 0ull};
+  PSKV_ASK_ARGS("s"(votes.told), "s"(votes.tag.epoch), "s"(looks));
+  bool usable = false;
+  if (threadIdx.x == 0) {
+    votes.before = __hip_atomic_load(&st->repeat_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    usable = cache_usable(st, votes.tag);
+  }
   const uint64_t n = d.n;
   const uint64_t first = ((uint64_t)blockIdx.x * kRepeatBlock * QUADS + threadIdx.x) * 4;
   f32x4 cur[QUADS], add[QUADS];
@@ -503,9 +511,8 @@ __global__ __launch_bounds__(kRepeatBlock) void k_scalar_repeat(HeadBatch<TABLES
   const bool any = __syncthreads_or(differ ? 1 : 0) != 0;
   if (threadIdx.x == 0) {
     // (the old verdict has to be here before the vote goes out, behind which it may change)
-    asm volatile("" : "+v"(before) : : "memory");
-    RepeatVotes<PUSH> votes{st, d, before};
-    s_same = vote(votes, nblk, !any, d.cache_mode) ? 1u : 0u;
+    asm volatile("" : "+v"(votes.before) : : "memory");
+    s_same = vote(votes, nblk, usable && !any, looks) ? 1u : 0u;
   }
   __syncthreads();
   if (!s_same) return;

@@ -18,8 +18,8 @@ constexpr unsigned vote_count(unsigned word) { return word & 0xffffu; }
 //   unsigned add(unsigned)                   adds to the word of the votes and returns what it was
 //   unsigned word()                          the word as it is
 //   bool swap(unsigned from, unsigned to)    exchanges it if it is `from`
-//   bool publish(bool yes)                   called by the last vote: clears the word and lets the others see the
-//                                            outcome, which it returns (it may turn a yes into a no)
+//   bool publish(bool yes)                   called by the last vote: clears the word, lets the others see the
+//                                            outcome and returns it
 //   int outcome()                            1 or 0, and -1 while it has not been published
 //   void pause()
 // `looks`: how often a workgroup looks for the outcome before it means to leave.
