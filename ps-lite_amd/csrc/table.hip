@@ -130,7 +130,7 @@ __global__ void k_read_state(StateBatch sb) {
 // request buffers, events, its stream. Creating them costs the calling thread about a millisecond (every
 // pinned allocation and its release go through the driver), so a table that goes leaves its shell to
 // the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim, and
-// some time after the last table of the device has gone.
+// (but for the streams) some time after the last table of the device has gone.
 struct Shell {
   DevState* st = nullptr;
   char* pinned = nullptr;  // StateView, Snapshot, outcome word, done word (256 bytes each), small_in, small_out
@@ -142,6 +142,7 @@ constexpr size_t kShellsKept = 32;
 struct ShellPool {
   std::mutex mu;
   std::vector<Shell*> idle;
+  std::vector<hipStream_t> streams;  // of shells that have gone back (shell_trim)
 };
 ShellPool g_shells[64];
 
@@ -197,20 +198,46 @@ void shell_give(int device, Shell* sh) {
   shell_free(sh);
 }
 
-// With `device` current: idle shells go.
-void shell_trim(int device) {
+// The stream that the next shell without one gets: one that a shell has left, or null.
+hipStream_t shell_stream(int device) {
+  if (device >= 64) return nullptr;
+  ShellPool& p = g_shells[device];
+  std::lock_guard<std::mutex> lk(p.mu);
+  if (p.streams.empty()) return nullptr;
+  hipStream_t s = p.streams.back();
+  p.streams.pop_back();
+  return s;
+}
+
+// With `device` current: idle shells go. Their streams stay (`streams_too`: or not): they are no memory, and a new
+// stream may come to share a hardware queue with other streams than the old one did, which moves a caller with
+// several tables by a tenth either way.
+void shell_trim(int device, bool streams_too) {
   std::vector<Shell*> go;
+  std::vector<hipStream_t> streams;
   {
-    std::lock_guard<std::mutex> lk(g_shells[device].mu);
-    go.swap(g_shells[device].idle);
+    ShellPool& p = g_shells[device];
+    std::lock_guard<std::mutex> lk(p.mu);
+    go.swap(p.idle);
+    if (streams_too) {
+      streams.swap(p.streams);
+    } else {
+      for (Shell* sh : go) {
+        if (sh->stream && p.streams.size() < kShellsKept) {
+          p.streams.push_back(sh->stream);
+          sh->stream = nullptr;
+        }
+      }
+    }
   }
   for (Shell* sh : go) shell_free(sh);
+  for (hipStream_t s : streams) (void)hipStreamDestroy(s);
 }
 
 // What tables that are gone have left (`device` is current).
 void give_back(int device) {
   array_trim(device);
-  if (device < 64) shell_trim(device);
+  if (device < 64) shell_trim(device, false);
 }
 
 }  // namespace
@@ -2033,6 +2060,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   if (opts->stream) {
     t->stream = static_cast<hipStream_t>(opts->stream);
   } else {
+    if (!t->shell->stream) t->shell->stream = shell_stream(t->device);
     if (!t->shell->stream && hipStreamCreateWithFlags(&t->shell->stream, hipStreamNonBlocking) != hipSuccess)
       return fail(set_error(PSKV_EHIP, "hipStreamCreateWithFlags failed"));
     t->stream = t->shell->stream;
@@ -2447,7 +2475,8 @@ int pskv_device_trim(int device) {
   if (device < 0 || device >= 64) return set_error(PSKV_EINVAL, "device %d out of range", device);
   DeviceGuard guard(device);
   if (!guard.ok()) return set_error(PSKV_EHIP, "cannot select device %d", device);
-  give_back(device);
+  array_trim(device);
+  shell_trim(device, true);
   return match_trim(device);
 }
 
