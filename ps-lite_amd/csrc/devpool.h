@@ -21,11 +21,11 @@ namespace pskv {
 int array_alloc(void** out, size_t bytes, hipStream_t stream);
 // Gives an array back (null: nothing). Work already enqueued on `stream` may still use it; `idle`: nothing does.
 int array_release(void* ptr, hipStream_t stream, bool idle = false);
-// For a stream (of the current device) that is waited for and may be destroyed: array_mark() before the wait, and
+// For a stream of `device` that is waited for and may be destroyed: array_mark() before the wait, and
 // behind it array_settle() with what it said: nothing that had been released by then depends on the stream any
 // more. (What another thread releases on the same stream meanwhile does.)
-unsigned long long array_mark();
-void array_settle(hipStream_t stream, unsigned long long mark);
+unsigned long long array_mark(int device);
+void array_settle(int device, hipStream_t stream, unsigned long long mark);
 // Frees every array on the list of `device` (current). Waits for those that are still in use.
 void array_trim(int device);
 // False with PSKV_NO_ASYNC_ALLOC in the environment: arrays come from hipMalloc and go to hipFree, nothing is kept.

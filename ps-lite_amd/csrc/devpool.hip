@@ -371,17 +371,15 @@ int array_release(void* ptr, hipStream_t stream, bool idle) {
   return PSKV_OK;
 }
 
-unsigned long long array_mark() {
-  int dev = 0;
-  Pool* p = hipGetDevice(&dev) == hipSuccess ? pool_of(dev) : nullptr;
+unsigned long long array_mark(int device) {
+  Pool* p = pool_of(device);
   if (!p) return 0;
   std::lock_guard<std::mutex> lk(p->mu);
   return p->releases;
 }
 
-void array_settle(hipStream_t stream, unsigned long long mark) {
-  int dev = 0;
-  Pool* p = hipGetDevice(&dev) == hipSuccess ? pool_of(dev) : nullptr;
+void array_settle(int device, hipStream_t stream, unsigned long long mark) {
+  Pool* p = pool_of(device);
   if (!p) return;
   std::lock_guard<std::mutex> lk(p->mu);
   for (Idle& i : p->idle) {

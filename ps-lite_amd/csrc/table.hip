@@ -2106,7 +2106,7 @@ int pskv_table_destroy(pskv_table* t) {
             (unsigned long long)t->stats.catch_ups, t->stats.catch_up_us, (unsigned long long)t->stats.records,
             t->stats.alloc_us, t->stats.ahead_us, t->stats.release_us);
   collect_spare(t, true);  // (the stream may have been made to wait for what used that array before)
-  const unsigned long long mark = array_mark();
+  const unsigned long long mark = array_mark(t->device);
   const bool idle = !t->stream || hipStreamSynchronize(t->stream) == hipSuccess;
   for (int k = 0; k < PSKV_KERNEL_COUNT; ++k)
     for (const EventPair& ev : t->pending[k]) t->free_events.push_back(ev);
@@ -2116,7 +2116,7 @@ int pskv_table_destroy(pskv_table* t) {
   }
   // this table's work is done: its arrays are free to go to any other table at once, as are those that were given up
   // before the wait. (Others may use the stream: what they have given up since waits for its own event.)
-  if (t->stream && idle) array_settle(t->stream, mark);
+  if (t->stream && idle) array_settle(t->device, t->stream, mark);
   for (void* ptr : {static_cast<void*>(t->slots), static_cast<void*>(t->arena), static_cast<void*>(t->spare)})
     (void)array_release(ptr, t->stream, idle);
   for (const GrowBuf* b : {&t->ws, &t->tiles, &t->tiles_aff, &t->stage, &t->stage_out, &t->cache_keys, &t->cache_lens,

@@ -42,11 +42,11 @@ static int settle() {
   CHECK(array_alloc(&between, 8 << 20, &shared) == PSKV_OK);
   shared.queued = 5;
   CHECK(array_release(before, &shared) == PSKV_OK);
-  const unsigned long long mark = array_mark();
+  const unsigned long long mark = array_mark(0);
   CHECK(hipStreamSynchronize(&shared) == hipSuccess);
   shared.queued = 9;  // (the kernel of a growth that reads the old array)
   CHECK(array_release(between, &shared) == PSKV_OK);
-  array_settle(&shared, mark);
+  array_settle(0, &shared, mark);
   CHECK(array_alloc(&got, 8 << 20, &other) == PSKV_OK && got == between);
   CHECK(safe(&other, &shared, 9));
   const size_t waits = host_hip().waits.size();
