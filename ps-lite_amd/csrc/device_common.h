@@ -103,6 +103,9 @@ struct alignas(32) DevState {
   // first level of the last-workgroup ticket: one counter per 128-byte line, and behind it the facts of its
   // workgroups (report_facts)
   unsigned int ticket_sub[kTicketShards * 32];
+  // k_fixed_own: pushes served so far << 1 | whether the newest one repeated a key; everyone watches it, so the line is its own
+  unsigned long long push_verdict;
+  unsigned long long pad[15];
 };
 
 // The head of DevState as one load.
@@ -320,13 +323,22 @@ __device__ __forceinline__ void publish_snapshot(const DevState* st, Snapshot* o
   unsigned long long c = lane < kCountShards ? st->count_shard[lane * kShardStride] : 0ull;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  const unsigned long long top = st->arena_top;
   if (lane != 0) return;
-  out->seq_begin = seq;
-  __threadfence_system();
-  out->count = c;
-  out->arena_top = st->arena_top;
-  __threadfence_system();
-  out->seq_end = seq;
+  // (one behind the other, each once the one before it has arrived; a fence would write back what else lies in the L2)
+  auto tell = [](volatile uint64_t* to, uint64_t x) {
+    __hip_atomic_store(const_cast<uint64_t*>(to), x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  auto arrive = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+  };
+  tell(&out->seq_begin, seq);
+  arrive();
+  tell(&out->count, c);
+  tell(&out->arena_top, top);
+  arrive();
+  tell(&out->seq_end, seq);
 }
 
 // Finds `key` or claims an empty slot for it. Returns the address of the slot's

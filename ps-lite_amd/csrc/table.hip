@@ -19,6 +19,7 @@
 
 #include "devpool.h"
 #include "host_common.h"
+#include "one_launch.h"
 #include "scan.h"
 #include "stager.h"
 #include "table_kernels.h"
@@ -350,6 +351,7 @@ struct pskv_table {
   unsigned char sc_kind[kScKinds] = {0};  // kind of the request with number e, at e % kScKinds
   unsigned long long* outcome = nullptr;  // pinned: epoch << 1 | same of the newest comparison
   unsigned long long sc_seen = 0;         // the value of *outcome the host last looked at
+  unsigned push_looks = 0;                // k_fixed_own: how often a workgroup looks for the verdict
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
 
   bool prof = false;
@@ -1309,6 +1311,23 @@ int begin_row_request(Batch& bt, bool compare) {
   });
 }
 
+// Whether a FIXED request is one launch (k_fixed_own): not where it arrives, or leaves, piece by piece or is being
+// recorded, nor where a row is more than a workgroup takes. A push needs its workgroups on the GPU together. A pull of rows
+// that do not end on a quad is better off with the lookup in front of it when it is large (500,000 rows of 33 floats,
+// three tables in turn: 309 us per step against 298; 193,521 of 30: 120 against 126).
+constexpr uint64_t kOwnRaggedFloats = 1u << 23;
+bool fixed_in_one(const Batch& bt, bool push) {
+  if (bt[0].r.replay || bt[0].r.pipe_in || bt[0].r.pipe_out) return false;
+  uint64_t groups = 0, floats = 0;
+  for (const Item& it : bt) {
+    if (!it.r.n) continue;
+    if ((it.d.k + 3) / 4 > kOwnQuads || it.r.n > ((uint64_t)1 << 40) / it.d.k) return false;
+    groups += (it.r.n + own_keys(it.d.k) - 1) / own_keys(it.d.k);
+    floats += it.d.k % 4 ? it.r.n * it.d.k : 0;
+  }
+  return push ? groups <= kOwnPushGroups : floats <= kOwnRaggedFloats;
+}
+
 int run_fixed(Batch& bt, bool push, bool pull) {
   uint64_t n_largest = 0;
   for (Item& it : bt) {
@@ -1344,7 +1363,28 @@ int run_fixed(Batch& bt, bool push, bool pull) {
   if (!n_largest) return PSKV_OK;
   int rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
   if (rc) return rc;
-  if (bt[0].r.replay == kReplayCapture) {
+  const bool one = fixed_in_one(bt, push);
+  if (one) {
+    uint64_t floats = 0;
+    bool apart = true;  // (rows that share no line with their neighbours; the others go through the caches, see k_rows)
+    for (Item& it : bt) {
+      if (!it.r.n) continue;
+      it.d.vals = it.r.vals;
+      it.d.out = it.r.out;
+      it.d.cache_mode = it.t->push_looks;
+      floats += it.r.n * it.d.k;
+      apart = apart && it.d.k >= 32 && (it.d.k % 4 == 0 || it.d.k >= 1024);
+    }
+    const bool stream = floats >= kStreamFloats && apart;
+    const KernelSet kernels = push && pull ? PSKV_KSET_OF(k_fixed_own, true, true, false)
+                              : push       ? stream ? PSKV_KSET_OF(k_fixed_own, true, false, true)
+                                                    : PSKV_KSET_OF(k_fixed_own, true, false, false)
+                              : stream     ? PSKV_KSET_OF(k_fixed_own, false, true, true)
+                                           : PSKV_KSET_OF(k_fixed_own, false, true, false);
+    rc = launch_batch(bt, push ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, [](const Item& it) {
+      return it.r.n ? (it.r.n + own_keys(it.d.k) - 1) / own_keys(it.d.k) : 0ull;
+    });
+  } else if (bt[0].r.replay == kReplayCapture) {
     // a recorded repeat is compared as a whole and uses the references that are there: no lookup
   } else if (n_largest >= kLookupLargeKeys) {
     rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET_OF(k_lookup_fixed, kLookupItemsLarge), [](const Item& it) {
@@ -1364,6 +1404,7 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     it.t->cache_nvals = it.r.n * it.d.k;
     it.t->known_n = std::max(it.t->known_n, it.r.n);  // (what lies behind this request's last key holds still)
   }
+  if (one) return PSKV_OK;
   if (push) {
     for (Item& it : bt) {
       if (!it.r.n) continue;
@@ -2049,6 +2090,9 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   t->max_load = opts->max_load > 0.f ? opts->max_load : 0.5f;
   t->row_len = opts->mode == PSKV_MODE_FIXED ? opts->row_len : 0;
   device_tables(t->device, 1, give_back);
+  // (the environment variable is for tests of workgroups that do not see the verdict)
+  t->push_looks = kOwnLooks;
+  if (const char* e = std::getenv("PSKV_PUSH_LOOKS")) t->push_looks = (unsigned)std::strtoul(e, nullptr, 10);
   t->sc_min_keys = kScalarCacheMinKeys;
   if (const char* e = std::getenv("PSKV_SCALAR_CACHE_MIN_KEYS")) t->sc_min_keys = std::strtoull(e, nullptr, 10);
   auto fail = [&](int rc) {
