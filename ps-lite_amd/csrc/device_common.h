@@ -66,6 +66,7 @@ struct __align__(16) Slot {
 constexpr int kCountShards = 32;
 constexpr int kShardStride = 16;  // in 8-byte words: one shard per 128-byte line
 constexpr int kTicketShards = 32;
+constexpr unsigned kVarParts = 256;  // workgroups of a var-len request that tell each other about it (one_launch.h)
 
 struct alignas(32) DevState {
   // The first 32 bytes are what a row kernel needs to know about its request (ReqFacts below):
@@ -88,8 +89,8 @@ struct alignas(32) DevState {
   unsigned int ticket_top;             // second level of the last-workgroup ticket (ticket_last)
   unsigned long long cache_epoch;
   unsigned long long bad_epoch;
-  // FIXED: the request with this number was refused (it repeats a key): its row kernels change
-  // no stored value and leave the rows it created as zero rows
+  // The request with this number was refused (FIXED: it repeats a key; k_var_push_start: a length differs from the stored
+  // one): its row kernels change no stored value and leave the rows it created as zero rows
   unsigned long long refused_epoch;
   // SCALAR key cache: the last request that changed cached values without touching the slots, and
   // the value of dirty_epoch up to which the slots have been brought up to date since
@@ -103,9 +104,11 @@ struct alignas(32) DevState {
   // first level of the last-workgroup ticket: one counter per 128-byte line, and behind it the facts of its
   // workgroups (report_facts)
   unsigned int ticket_sub[kTicketShards * 32];
-  // k_fixed_own: pushes served so far << 1 | whether the newest one repeated a key; everyone watches it, so the line is its own
+  // one_launch.h: pushes served so far << 2 | the verdict on the newest one; everyone watches it, so the line is its own
   unsigned long long push_verdict;
   unsigned long long pad[15];
+  // one_launch.h: what the workgroups of a var-len request tell each other, all zero between requests
+  unsigned long long parts[kVarParts];
 };
 
 // The head of DevState as one load.
@@ -341,6 +344,51 @@ __device__ __forceinline__ void publish_snapshot(const DevState* st, Snapshot* o
   tell(&out->seq_end, seq);
 }
 
+// Tries to settle `key` at slot `at`, whose contents `s` were read a moment ago: 1 = found (`seen` is the payload), 2 =
+// claimed, 0 = the slot belongs to another key.
+__device__ __forceinline__ int settle_slot(Slot* __restrict__ slots, uint64_t at, const u64x2& s, uint64_t key,
+                                           uint64_t& seen) {
+  if (s.x == key) {
+    seen = s.y;
+    return 1;
+  }
+  if (s.x == kEmptyKey) {
+    unsigned long long old = atomicCAS(reinterpret_cast<unsigned long long*>(&slots[at].key),
+                                       (unsigned long long)kEmptyKey, (unsigned long long)key);
+    if (old == kEmptyKey) return 2;
+    if (old == key) {  // same key twice in one request: undefined for callers, but stay sane
+      seen = slots[at].payload;
+      return 1;
+    }
+  }
+  return 0;
+}
+
+// The walk behind slot `h`, which belongs to another key: three slots at once (a walk of one slot per round trip made
+// a push a tenth slower at a fill of 0.4 than at 0.1). The first three may have been asked for already (`there`).
+__device__ __forceinline__ uint64_t* walk_slots(Slot* __restrict__ slots, uint64_t mask, DevState* st, uint64_t key,
+                                                uint64_t h, bool& is_new, uint64_t& seen, u64x2 s1, u64x2 s2, u64x2 s3,
+                                                bool there) {
+  for (uint64_t probes = 0; probes <= mask; probes += 3) {
+    const uint64_t h1 = (h + 1) & mask, h2 = (h + 2) & mask, h3 = (h + 3) & mask;
+    if (!there) s1 = load_slot(&slots[h1]), s2 = load_slot(&slots[h2]), s3 = load_slot(&slots[h3]);
+    there = false;
+    if (const int r = settle_slot(slots, h1, s1, key, seen)) return is_new = r == 2, &slots[h1].payload;
+    if (const int r = settle_slot(slots, h2, s2, key, seen)) return is_new = r == 2, &slots[h2].payload;
+    if (const int r = settle_slot(slots, h3, s3, key, seen)) return is_new = r == 2, &slots[h3].payload;
+    h = h3;
+  }
+  atomicOr(&st->error, kDevErrFull);
+  return nullptr;
+}
+
+// Key 2^64-1, which marks an empty slot, lives in the side slot.
+__device__ __forceinline__ uint64_t* special_slot(DevState* st, bool& is_new, uint64_t& seen) {
+  is_new = atomicExch(&st->special_present, 1u) == 0u;
+  seen = st->special_payload;
+  return reinterpret_cast<uint64_t*>(&st->special_payload);
+}
+
 // Finds `key` or claims an empty slot for it. Returns the address of the slot's
 // payload (nullptr if the table has no free slot, which the host-side sizing
 // rules out). `seen` is the payload read together with the key when the key was
@@ -350,53 +398,54 @@ __device__ __forceinline__ uint64_t* find_or_insert(Slot* __restrict__ slots, ui
                                                     uint64_t& seen) {
   is_new = false;
   seen = 0;
-  if (key == kEmptyKey) {
-    is_new = atomicExch(&st->special_present, 1u) == 0u;
-    seen = st->special_payload;
-    return reinterpret_cast<uint64_t*>(&st->special_payload);
-  }
-  uint64_t h = home_slot(key, mask);
-  // Tries to settle the key at slot `at`, whose contents `s` were read a moment ago: 1 = found,
-  // 2 = claimed, 0 = the slot belongs to another key.
-  auto settle = [&](uint64_t at, const u64x2& s) -> int {
-    if (s.x == key) {
-      seen = s.y;
-      return 1;
-    }
-    if (s.x == kEmptyKey) {
-      unsigned long long old = atomicCAS(reinterpret_cast<unsigned long long*>(&slots[at].key),
-                                         (unsigned long long)kEmptyKey, (unsigned long long)key);
-      if (old == kEmptyKey) {
-        is_new = true;
-        return 2;
-      }
-      if (old == key) {  // same key twice in one request: undefined for callers, but stay sane
-        seen = slots[at].payload;
-        return 1;
-      }
-    }
-    return 0;
-  };
+  if (key == kEmptyKey) return special_slot(st, is_new, seen);
+  const uint64_t h = home_slot(key, mask);
   // The home slot alone first: at the fills this table runs at, most keys are settled there, and
-  // one load per lane keeps the most wavefronts in flight. A key that has to walk on asks for the
-  // next three slots at once (a walk of one slot per round trip made a push a tenth slower at a
-  // fill of 0.4 than at 0.1).
-  {
-    const u64x2 s = load_slot(&slots[h]);
-    if (settle(h, s)) return &slots[h].payload;
+  // one load per lane keeps the most wavefronts in flight.
+  const u64x2 s = load_slot(&slots[h]);
+  if (const int r = settle_slot(slots, h, s, key, seen)) return is_new = r == 2, &slots[h].payload;
+  return walk_slots(slots, mask, st, key, h, is_new, seen, s, s, s, false);
+}
+
+// The same for the N keys of a lane, whose home slots have been read a moment ago, side by side: in a wavefront there
+// is nearly always a lane that has to claim a slot or to walk on, and N keys one after the other are N round trips.
+template <int N>
+__device__ __forceinline__ void find_or_insert_all(Slot* __restrict__ slots, uint64_t mask, DevState* st,
+                                                   const uint64_t (&key)[N], const u64x2 (&home)[N], const bool (&live)[N],
+                                                   uint64_t* (&p)[N], bool (&is_new)[N], uint64_t (&seen)[N]) {
+  unsigned long long old[N];
+  bool walk[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    p[j] = nullptr, is_new[j] = false, seen[j] = 0, old[j] = home[j].x;
+    walk[j] = live[j] && key[j] != kEmptyKey;
+    if (walk[j] && home[j].x == kEmptyKey)
+      old[j] = atomicCAS(reinterpret_cast<unsigned long long*>(&slots[home_slot(key[j], mask)].key),
+                         (unsigned long long)kEmptyKey, (unsigned long long)key[j]);
   }
-  for (uint64_t probes = 0; probes <= mask; probes += 3) {
-    const uint64_t h1 = (h + 1) & mask, h2 = (h + 2) & mask, h3 = (h + 3) & mask;
-    const u64x2 s1 = load_slot(&slots[h1]);
-    const u64x2 s2 = load_slot(&slots[h2]);
-    const u64x2 s3 = load_slot(&slots[h3]);
-    if (settle(h1, s1)) return &slots[h1].payload;
-    if (settle(h2, s2)) return &slots[h2].payload;
-    if (settle(h3, s3)) return &slots[h3].payload;
-    h = h3;
+  u64x2 s[N][3];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const uint64_t h = home_slot(key[j], mask);
+    s[j][0] = s[j][1] = s[j][2] = home[j];
+    if (!walk[j]) continue;
+    if (old[j] == kEmptyKey || old[j] == key[j]) {
+      walk[j] = false;
+      p[j] = &slots[h].payload;
+      is_new[j] = old[j] == kEmptyKey;
+      seen[j] = home[j].x == key[j] ? home[j].y : is_new[j] ? 0 : slots[h].payload;
+    } else {
+      s[j][0] = load_slot(&slots[(h + 1) & mask]);
+      s[j][1] = load_slot(&slots[(h + 2) & mask]);
+      s[j][2] = load_slot(&slots[(h + 3) & mask]);
+    }
   }
-  atomicOr(&st->error, kDevErrFull);
-  return nullptr;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if (walk[j])
+      p[j] = walk_slots(slots, mask, st, key[j], home_slot(key[j], mask), is_new[j], seen[j], s[j][0], s[j][1], s[j][2], true);
+    if (live[j] && key[j] == kEmptyKey) p[j] = special_slot(st, is_new[j], seen[j]);
+  }
 }
 
 // Lookup without insertion. Returns false when the key is absent.

@@ -1,6 +1,6 @@
-// Requests of the row modes that are ONE launch: what a lookup kernel and a row kernel of table_kernels.h do one after the
-// other. A small request is bound by its launches (2.2 us of the calling thread for each, and 3 to 5 us of the GPU's
-// between dependent ones), not by what they do.
+// Requests of the row modes in fewer launches: what kernels of table_kernels.h do one after the other in one. A small
+// request is bound by its launches (2.2 us of the calling thread for each, and 3 to 5 us of the GPU's between dependent
+// ones), not by what they do.
 #ifndef PSKV_ONE_LAUNCH_H_
 #define PSKV_ONE_LAUNCH_H_
 #include "table_kernels.h"
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
       if (PUSH) {
         verdict = take_facts(st, nblk) & kReqDuplicate ? 1u : 0u;
         if (threadIdx.x == 0)
-          __hip_atomic_store(&st->push_verdict, ((before >> 1) + 1) << 1 | verdict, __ATOMIC_RELAXED,
+          __hip_atomic_store(&st->push_verdict, ((before >> 2) + 1) << 2 | verdict, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT);
       }
       if (d.snap) publish_snapshot(st, d.snap, d.snap_seq);
@@ -180,6 +180,322 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
     if (fresh || (PUSH && !rejected)) store_part<STREAM>(y[q], d.arena + (ref[q] & ~kRefNew) * k + col[q], count[q]);
     if (PULL) store_part<STREAM>(y[q], d.out + (first + row[q]) * k + col[q], count[q]);
   }
+}
+
+// VARLEN requests of up to kVarParts workgroups: what the first two kernels of a push, or of a pull, do, in one. A
+// workgroup takes kStartPart consecutive keys, two a thread, and keeps them in registers. What it has to know of the
+// others (where its rows start in the request, what is the matter with any key or length) it reads off one word of
+// each, which it watches until all of them are there: no election, no scan by one for all (with those, and the outcome in
+// a word for everyone, 15,826 rows over 3 tables took 14.8 us to start a push, now 8.6; begin + lookup 6.7 + 7.2 and the
+// launch between them). With four keys a thread it was the walks of a wavefront's keys one after the other, 13.4. The
+// workgroups have to be on the GPU together, and kVarParts of them are a fifth of what it holds; who does not see all
+// words in time (d.cache_mode looks: something else may keep a part of the workgroups off the GPU) goes through the
+// request itself, so nobody depends on the others but for time.
+// The row kernel behind it takes the words away again, and leaves the counter record of a push (finish_start).
+// Measured (us per step of slice, push and pull, other rows in every step, three tables in turn): 10,562 rows of 8 to 128
+// floats over 4 tables 36.3 -> 35.5, 15,826 of 1 to 90 over 3 42.2 -> 38.6, 50,000 of 8 to 64 over 4 43.9 -> 38.6.
+constexpr int kStartItems = 2;
+constexpr uint64_t kStartPart = (uint64_t)kBlock * kStartItems;
+inline uint64_t start_parts(uint64_t n) { return (n + kStartPart - 1) / kStartPart; }
+constexpr unsigned long long kPartHere = 1ull << 63;
+constexpr unsigned kPartFlagsAt = 40;  // (512 lengths below 2^28 add up to less)
+static_assert(kStartPart <= 1u << 10 && PSKV_MAX_VARLEN_ROW < (1u << 28), "a part's total fits below its flags");
+
+struct OfAllParts {
+  unsigned long long before, all;  // floats in front of this workgroup's part, and in the request
+  unsigned flags;                  // kReq*
+  bool known;
+};
+struct PartRed {
+  unsigned long long before[kBlock / 64], all[kBlock / 64];
+  unsigned flags[kBlock / 64];
+};
+__device__ __forceinline__ void reduce_parts(OfAllParts& x, PartRed* red) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    x.before += __shfl_xor(x.before, o);
+    x.all += __shfl_xor(x.all, o);
+    x.flags |= __shfl_xor(x.flags, o);
+  }
+  const unsigned wave = threadIdx.x >> 6;
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red->before[wave] = x.before, red->all[wave] = x.all, red->flags[wave] = x.flags;
+  __syncthreads();
+  x.before = x.all = 0, x.flags = 0;
+#pragma unroll
+  for (unsigned w = 0; w < kBlock / 64; ++w) x.before += red->before[w], x.all += red->all[w], x.flags |= red->flags[w];
+}
+// Every thread of the workgroup calls it with its own floats and flags.
+__device__ __forceinline__ OfAllParts meet_parts(DevState* st, unsigned nblk, unsigned long long floats, unsigned flags,
+                                                 unsigned looks, PartRed* red) {
+  OfAllParts mine{0, floats, flags, true};
+  reduce_parts(mine, red);
+  if (threadIdx.x == 0)
+    publish_u64(&st->parts[blockIdx.x], kPartHere | (unsigned long long)mine.flags << kPartFlagsAt |
+                                            (mine.flags & kReqBadLen ? 0ull : mine.all));
+  OfAllParts x{0, 0, 0, true};
+#pragma unroll
+  for (unsigned q = 0; q < kVarParts / kBlock; ++q) {
+    const unsigned i = q * kBlock + threadIdx.x;
+    if (i >= nblk) continue;
+    unsigned long long w = 0;
+    for (unsigned look = looks;; --look) {
+      w = __hip_atomic_load(&st->parts[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((w & kPartHere) || !look) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    const unsigned long long sum = w & ((1ull << kPartFlagsAt) - 1);
+    x.known = x.known && (w & kPartHere) != 0;
+    x.all += sum;
+    if (i < blockIdx.x) x.before += sum;
+    x.flags |= (unsigned)(w >> kPartFlagsAt) & 31u;
+  }
+  x.known = __syncthreads_and(x.known ? 1 : 0) != 0;
+  if (x.known) reduce_parts(x, red);
+  return x;
+}
+static_assert(kReqDuplicate == 16u && (kReqMisaligned | kReqBadLen | kReqDiffer) == 15u, "five bits of flags");
+
+typedef int32_t i32x2u __attribute__((ext_vector_type(2), aligned(4)));
+struct TwoKeys {
+  uint64_t k[kStartItems];
+  int32_t v[kStartItems];
+};
+__device__ __forceinline__ void load_two(TwoKeys& f, const uint64_t* keys, const int32_t* lens, uint64_t at, uint64_t n) {
+  static_assert(kStartItems == 2, "two keys per thread");
+  if (at + 2 <= n) {
+    const u64x2u a = *reinterpret_cast<const u64x2u*>(keys + at);
+    const i32x2u w = *reinterpret_cast<const i32x2u*>(lens + at);
+    f.k[0] = a.x, f.k[1] = a.y, f.v[0] = w.x, f.v[1] = w.y;
+  } else {
+    f.k[0] = at < n ? keys[at] : 0, f.v[0] = at < n ? lens[at] : 0;
+    f.k[1] = 0, f.v[1] = 0;
+  }
+}
+
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
+  const TableReq& d = b.t[blockIdx.y];
+  PSKV_ASK_ARGS("s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.lens), "s"(d.n), "s"(d.nvals), "s"(d.ref),
+                "s"(d.off), "s"(d.tile_key), "s"(d.ntiles), "s"(d.cache_keys), "s"(d.cache_lens), "s"(d.tag.epoch),
+                "s"(d.nblk));
+  const unsigned nblk = d.nblk;
+  if (blockIdx.x >= nblk) return;
+  DevState* st = d.st;
+  const uint64_t n = d.n;
+  constexpr unsigned max_len = PSKV_MAX_VARLEN_ROW;
+  __shared__ PartRed red;
+  __shared__ unsigned long long wsum[kBlock / 64 + 1];
+  __shared__ unsigned cred[kBlock / 64];
+  __shared__ unsigned long long s_start;
+  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kStartItems;
+  TwoKeys mine;
+  load_two(mine, d.keys, d.lens, base, n);
+  const uint64_t left = (base > 0 && base < n) ? d.keys[base - 1] : 0;
+  // The keys' home slots are on the way while the workgroups wait (an empty slot that has been taken since shows when it
+  // is claimed).
+  u64x2 home[kStartItems];
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) home[j] = load_slot(&d.slots[home_slot(mine.k[j], d.mask)]);
+  unsigned long long len[kStartItems], s = 0;
+  unsigned flags = 0;
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) {  // (as in k_var_push_begin)
+    const int32_t l = mine.v[j];
+    len[j] = (unsigned long long)(uint32_t)l;
+    s += len[j];
+    flags |= (unsigned)l & kReqMisaligned;
+    flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
+    const bool has_left = base + j < n && base + j > 0;
+    flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
+  }
+  OfAllParts of = meet_parts(st, nblk, s, flags, d.cache_mode, &red);
+  if (!of.known) {
+    of = OfAllParts{0, 0, 0, true};
+    for (uint64_t i = threadIdx.x; i < n; i += kBlock) {
+      const int32_t l = d.lens[i];
+      of.all += (unsigned long long)(uint32_t)l;
+      if (i < (uint64_t)blockIdx.x * kStartPart) of.before += (unsigned long long)(uint32_t)l;
+      of.flags |= (unsigned)l & kReqMisaligned;
+      of.flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
+      of.flags |= i > 0 && d.keys[i] == d.keys[i - 1] ? kReqDuplicate : 0u;
+    }
+    reduce_parts(of, &red);
+  }
+  const unsigned refused = (of.flags & kReqBadLen ? kDevErrBadLen : 0u) | (of.flags & kReqDuplicate ? kDevErrDuplicate : 0u);
+  const unsigned bad = refused ? refused : of.all != d.nvals ? kDevErrSizeMismatch : 0u;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    // what k_var_push_begin's last workgroup leaves of a request that does not repeat the cached one
+    if (st->req_error) atomicOr(&st->error, st->req_error);
+    st->req_error = bad;
+    st->scan_total = of.all;
+    st->misaligned = of.flags & kReqMisaligned;
+    st->cache_epoch = d.tag.epoch;
+    if (bad) st->bad_epoch = d.tag.epoch;
+  }
+  if (bad) return;  // nothing is created
+  scan_pass2_offsets<kStartItems>(len, base, n, of.before, d.off, d.tile_key, d.ntiles, kTileVar, wsum);
+  uint64_t* p[kStartItems];
+  uint64_t seen[kStartItems];
+  bool is_new[kStartItems], live[kStartItems];
+  unsigned long long units = 0;
+  unsigned created = 0;
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) live[j] = base + j < n;
+  find_or_insert_all<kStartItems>(d.slots, d.mask, st, mine.k, home, live, p, is_new, seen);
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) {
+    const uint64_t i = base + j;
+    if (live[j]) {
+      d.cache_keys[i] = mine.k[j];
+      d.cache_lens[i] = mine.v[j];
+      if (p[j] && !is_new[j] && seen[j] == kPayloadUnset) {
+        atomicOr(&st->error, kDevErrDuplicate);  // the same key twice in this request
+        st->bad_epoch = d.tag.epoch;
+        p[j] = nullptr;
+      }
+    }
+    if (p[j] && is_new[j]) {
+      units += (len[j] + 3) >> 2;
+      ++created;
+    }
+  }
+  if (__syncthreads_or(created ? 1 : 0)) {
+    unsigned long long total;
+    unsigned long long at = block_excl_scan_u64(units, wsum, total);
+    if (threadIdx.x == 0) {
+      // (the rows of the part start where the request's do, modulo 128 bytes: see k_var_push_lookup)
+      const unsigned long long first = atomicAdd(&st->arena_top, total + (kArenaPadUnits - 1));
+      const unsigned long long want = (of.before >> 2) & (kArenaPadUnits - 1);
+      s_start = first + ((want - first) & (kArenaPadUnits - 1));
+    }
+    __syncthreads();
+    at += s_start;
+#pragma unroll
+    for (int j = 0; j < kStartItems; ++j) {
+      if (!p[j] || !is_new[j]) continue;
+      seen[j] = ((uint64_t)at << kLenBits) | len[j];
+      at += (len[j] + 3) >> 2;
+      *p[j] = seen[j];
+    }
+    block_count_add(st, created, cred);
+  }
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) {
+    const uint64_t i = base + j;
+    if (i >= n) continue;
+    if (!p[j]) {
+      d.ref[i] = kRefAbsent;
+      continue;
+    }
+    if (!is_new[j] && (seen[j] & kLenMask) != len[j]) {
+      atomicOr(&st->error, kDevErrLenChanged);
+      st->bad_epoch = d.tag.epoch;
+      st->refused_epoch = d.tag.epoch;  // (req_error is the first workgroup's, which may be behind this one)
+    }
+    d.ref[i] = seen[j] | (is_new[j] ? kRefNew : 0ull);
+  }
+}
+
+// VARLEN pull: k_var_pull_lookup and k_var_offsets in one. d.ntiles: room in the tile table.
+template <int TABLES>
+__global__ __launch_bounds__(kBlock) void k_var_pull_start(ReqBatch<TABLES> b) {
+  const TableReq& d = b.t[blockIdx.y];
+  PSKV_ASK_ARGS("s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.n), "s"(d.ref), "s"(d.off), "s"(d.tile_key),
+                "s"(d.ntiles), "s"(d.cache_keys), "s"(d.cache_lens), "s"(d.out_lens), "s"(d.tag.epoch), "s"(d.nblk));
+  const unsigned nblk = d.nblk;
+  if (blockIdx.x >= nblk) return;
+  DevState* st = d.st;
+  const uint64_t n = d.n;
+  const ReqTag tag = d.tag;
+  __shared__ PartRed red;
+  __shared__ unsigned long long wsum[kBlock / 64];
+  const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kStartItems;
+  // (the first workgroup alone changes what this reads, after every workgroup has handed in its word; one that has not
+  // seen the words may read it late, and looks up its keys)
+  const bool usable = cache_usable(st, tag);
+  uint64_t key[kStartItems];
+  TwoKeys old;
+  bool known[kStartItems];
+  uint64_t payload[kStartItems];
+  int32_t l[kStartItems];
+  if (base + kStartItems <= n) {
+    const u64x2u a = *reinterpret_cast<const u64x2u*>(d.keys + base);
+    key[0] = a.x, key[1] = a.y;
+  } else {
+#pragma unroll
+    for (int j = 0; j < kStartItems; ++j) key[j] = base + j < n ? d.keys[base + j] : 0;
+  }
+  if (usable) load_two(old, d.cache_keys, d.cache_lens, base, n);
+  unsigned flags = 0;
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) {
+    known[j] = base + j >= n || (usable && old.k[j] == key[j]);
+    l[j] = known[j] && base + j < n ? old.v[j] : 0;
+    if (!known[j]) flags = kReqDiffer;
+  }
+  if (flags) {
+    u64x2 home[kStartItems];
+#pragma unroll
+    for (int j = 0; j < kStartItems; ++j)
+      if (!known[j]) home[j] = load_slot(&d.slots[home_slot(key[j], d.mask)]);
+#pragma unroll
+    for (int j = 0; j < kStartItems; ++j) {
+      if (known[j]) continue;
+      bool hit = home[j].x == key[j] && key[j] != kEmptyKey;
+      payload[j] = home[j].y;
+      if (!hit) hit = find_only(d.slots, d.mask, st, key[j], payload[j]);
+      l[j] = hit ? (int32_t)(payload[j] & kLenMask) : 0;
+      d.ref[base + j] = hit ? payload[j] : kRefAbsent;
+    }
+  }
+  unsigned long long len[kStartItems], s = 0;
+#pragma unroll
+  for (int j = 0; j < kStartItems; ++j) {
+    len[j] = (unsigned long long)(uint32_t)l[j];
+    s += len[j];
+    flags |= (unsigned)l[j] & kReqMisaligned;
+  }
+  if (base + kStartItems <= n) {
+    i32x2u w;
+    w.x = l[0], w.y = l[1];
+    *reinterpret_cast<i32x2u*>(d.out_lens + base) = w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < kStartItems; ++j)
+      if (base + j < n) d.out_lens[base + j] = l[j];
+  }
+  OfAllParts of = meet_parts(st, nblk, s, flags, d.cache_mode, &red);
+  if (!of.known) {
+    of = OfAllParts{0, 0, kReqDiffer, true};
+    for (uint64_t i = threadIdx.x; i < n; i += kBlock) {
+      uint64_t r = 0;
+      const unsigned x = find_only(d.slots, d.mask, st, d.keys[i], r) ? (unsigned)(r & kLenMask) : 0u;
+      of.all += x;
+      if (i < (uint64_t)blockIdx.x * kStartPart) of.before += x;
+      of.flags |= x & kReqMisaligned;
+    }
+    reduce_parts(of, &red);
+  }
+  const bool same = !(of.flags & kReqDiffer) && usable;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    // what k_var_pull_lookup's last workgroup leaves
+    if (st->req_error) atomicOr(&st->error, st->req_error);
+    st->req_error = 0;
+    st->misaligned = of.flags & kReqMisaligned;
+    if (same) {
+      st->same_epoch = tag.epoch;
+    } else {
+      st->scan_total = of.all;
+      // this pull rewrites references and offsets in the workspace: the cached push is gone
+      st->bad_epoch = st->cache_epoch;
+    }
+    if (d.outcome && tag.try_cache) *d.outcome = (tag.epoch << 1) | (same ? 1ull : 0ull);
+  }
+  if (same) return;  // offsets and tile table of the cached request hold
+  uint64_t ntiles = (of.all + kTileVar - 1) / kTileVar;
+  if (ntiles > d.ntiles) ntiles = d.ntiles;
+  scan_pass2_offsets<kStartItems>(len, base, n, of.before, d.off, d.tile_key, ntiles, kTileVar, wsum);
 }
 
 }  // namespace pskv

@@ -1240,11 +1240,11 @@ int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
   auto nblk = [&](const Item&) { return blocks; };
   int rc;
   if (op == kOpAcc) {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true), nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false), nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true, false), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false, false), nblk);
   } else {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true), nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false), nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true, false), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false, false), nblk);
   }
   it.d.tile_base = 0;
   return rc;
@@ -1278,15 +1278,19 @@ int launch_rows(Batch& bt, int op) {
     return PSKV_OK;
   }
   auto nblk = [&](const Item& it) {
-    return VARLEN ? (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock : (it.d.ntiles + kQuadsFixed - 1) / kQuadsFixed;
+    if (VARLEN) return (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock + (it.d.started ? 1 : 0);
+    return (it.d.ntiles + kQuadsFixed - 1) / kQuadsFixed;
   };
   const bool stream = floats >= kStreamFloats;
-  if (op == kOpAcc) {
-    if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true), nblk);
-    return launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false), nblk);
-  }
-  if (stream) return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true), nblk);
-  return launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false), nblk);
+  bool started = false;
+  for (const Item& it : bt) started = started || (VARLEN && it.d.started);
+  const KernelSet kernels =
+      op == kOpAcc
+          ? (started ? (stream ? PSKV_KSET_OF(k_rows, kOpAcc, true, true, true) : PSKV_KSET_OF(k_rows, kOpAcc, true, false, true))
+                     : (stream ? PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true, false) : PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false, false)))
+          : (started ? (stream ? PSKV_KSET_OF(k_rows, kOpGather, true, true, true) : PSKV_KSET_OF(k_rows, kOpGather, true, false, true))
+                     : (stream ? PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true, false) : PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false, false)));
+  return launch_batch(bt, op == kOpAcc ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, nblk);
 }
 
 // Starts a row-mode request on every table with keys: numbers it and (`compare`: a recorded one), where the
@@ -1451,7 +1455,7 @@ uint64_t may_return_at_once(const Item& it, bool push, uint64_t chunks, size_t t
 // Pass 2 of a pull's scan for every table with a response: the request-side offsets of the
 // response and the tile table for Item::d.total floats of room (the row kernel fills the other
 // table).
-int make_tile_tables(Batch& bt) {
+int make_tile_tables(Batch& bt, bool there = false) {
   for (Item& it : bt) {
     if (!it.d.total) continue;
     uint64_t ntiles_cap = 0;
@@ -1461,15 +1465,36 @@ int make_tile_tables(Batch& bt) {
     it.d.tile_aff = static_cast<TileNote*>(it.t->tiles_aff.ptr);
     it.d.ntiles = ntiles_cap;
   }
-  if (bt[0].r.replay == kReplayCapture) return PSKV_OK;  // (a recorded repeat: the tables that are there)
+  if (there || bt[0].r.replay == kReplayCapture) return PSKV_OK;  // (k_var_pull_start's; a recorded repeat's)
   return launch_batch(bt, -1, PSKV_KSET(k_var_offsets), [&](const Item& it) {
     return (it.r.n && it.d.total) ? may_return_at_once(it, false, it.nparts, bt.size()) : 0ull;
   });
 }
 
+// Whether a var-len request starts with one launch (k_var_push_start, k_var_pull_start) and not with two: not where it is
+// being recorded, or arrives piece by piece, nor where its workgroups are too many to wait for each other (200,000 rows
+// in 391 of them, other rows in every step, three tables in turn: 233 us with two launches, 243 with one). The row kernel
+// behind it cleans up, so every table has to have one (`floats`). Of requests that may repeat the cached one those of
+// more than kVarCompareKeys keys are better off with two: the second returns at once (100,000 rows over 16 tables, the
+// same in every step: 51 us against 54; 20,000: 49 against 47).
+constexpr uint64_t kVarCompareKeys = 1u << 16;
+template <typename F>
+bool start_together(const Batch& bt, uint64_t n_launch, F floats) {
+  uint64_t parts = 0;
+  bool compared = false;
+  for (const Item& it : bt) {
+    if (it.r.replay || it.r.pipe_in) return false;
+    if (!it.r.n) continue;
+    if (!floats(it)) return false;
+    parts += start_parts(it.r.n);
+    compared = compared || it.tag.try_cache;
+  }
+  return parts <= kVarParts && (!compared || n_launch <= kVarCompareKeys);
+}
+
 // Launches per var-len request: a push takes three (compare + scan pass 1; scan pass 2 +
 // find-or-create + counter record; rows), a pull three (compare + stored lengths + scan pass 1;
-// scan pass 2 + tile table; rows), whatever the number of tables.
+// scan pass 2 + tile table; rows), whatever the number of tables; a small one two (start_together).
 int run_varlen(Batch& bt, bool push, bool pull) {
   uint64_t n_largest = 0;
   for (Item& it : bt) {
@@ -1484,6 +1509,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
   for (const Item& it : bt) n_launch += it.r.n;
   const bool large = n_launch >= kVarLookupLargeKeys;
   const uint64_t chunk = kBlock * (large ? 4 : 1);  // keys per workgroup of the creating lookup
+  const uint64_t pad_chunk = std::min(chunk, kStartPart);  // (and of k_var_push_start)
   const bool async_pull = pull && !push && !bt[0].r.need_total;
   for (Item& it : bt) {
     pskv_table* t = it.t;
@@ -1524,7 +1550,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       // every key may round its row up to a 16-byte unit, every workgroup may pad its rows' start
       int rc = r.replay == kReplayCapture
                    ? PSKV_OK
-                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * ((r.n + chunk - 1) / chunk), 4, &it.pub);
+                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * ((r.n + pad_chunk - 1) / pad_chunk), 4, &it.pub);
       if (rc) return rc;
       if (t->cache_nvals != r.nvals) t->cache_valid = false;  // same lens would mean the same total
       it.tag = next_tag(t, r, true);
@@ -1546,10 +1572,21 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
     }
-    int rc = launch_batch(bt, -1, PSKV_KSET(k_var_push_begin), [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+    const bool start = start_together(bt, n_launch, [](const Item& it) { return it.r.nvals; });
+    int rc;
+    if (start) {
+      for (Item& it : bt) {
+        it.tag.try_cache = it.d.tag.try_cache = 0;
+        it.d.started = (uint32_t)start_parts(it.r.n);
+        it.d.cache_mode = it.t->push_looks;
+      }
+      rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET(k_var_push_start), [](const Item& it) { return start_parts(it.r.n); });
+    } else {
+      rc = launch_batch(bt, -1, PSKV_KSET(k_var_push_begin), [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+    }
     if (rc) return rc;
     // (a recorded repeat uses the offsets, tile table and references that are there)
-    if (bt[0].r.replay != kReplayCapture)
+    if (!start && bt[0].r.replay != kReplayCapture)
       rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, large ? PSKV_KSET_OF(k_var_push_lookup, 4) : PSKV_KSET_OF(k_var_push_lookup, 1), [&](const Item& it) {
         return it.r.n ? may_return_at_once(it, true, (it.r.n + chunk - 1) / chunk, bt.size()) : 0ull;
       });
@@ -1557,6 +1594,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     for (Item& it : bt) {
       if (!it.r.n) continue;
       it.t->cache_valid = true;  // whichever way the device decided, the cache now is this request
+      if (!start) it.d.snap = nullptr;  // (its lookup leaves the counter record)
       it.t->cache_n = it.r.n;
       it.t->cache_nvals = it.r.nvals;
       it.d.req = const_cast<float*>(it.r.vals);
@@ -1586,6 +1624,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       it.d.out_lens = it.r.out_lens ? it.r.out_lens : it.tmp_lens;
       it.d.total = 0;
       it.d.snap = nullptr;
+      it.d.started = 0;
     }
     // A pull with the keys of the cached push finds every key present with the cached length
     // and reuses its references; any other pull recomputes them and so ends the cache.
@@ -1593,7 +1632,18 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     if (rc) return rc;
     for (Item& it : bt)
       if (it.r.n && !it.tag.try_cache) it.t->cache_valid = false;
-    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, PSKV_KSET(k_var_pull_lookup), [](const Item& it) { return it.r.n ? it.nparts : 0ull; });
+    const bool start = async_pull && start_together(bt, n_launch, [](const Item& it) { return it.r.out ? it.r.out_cap : 0; });
+    if (start) {
+      for (Item& it : bt) {
+        if (!it.r.n) continue;
+        it.d.tile_key = static_cast<uint32_t*>(it.t->tiles.ptr);
+        it.d.ntiles = it.tiles_cap;
+        it.d.started = (uint32_t)start_parts(it.r.n);
+        it.d.cache_mode = it.t->push_looks;
+      }
+    }
+    rc = launch_batch(bt, PSKV_KERNEL_LOOKUP, start ? PSKV_KSET(k_var_pull_start) : PSKV_KSET(k_var_pull_lookup),
+                      [&](const Item& it) { return start ? start_parts(it.r.n) : it.r.n ? it.nparts : 0ull; });
     if (rc) return rc;
     if (async_pull) {
       // No host round trip: the grid covers the caller's buffer, the kernels take the real
@@ -1606,7 +1656,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
         it.d.total_on_device = 1;
         it.d.ignore_new = 1;
       }
-      rc = make_tile_tables(bt);
+      rc = make_tile_tables(bt, start);
       if (rc) return rc;
       return launch_rows<true>(bt, kOpGather);
     }

@@ -86,3 +86,117 @@ def test_a_push_that_repeats_a_key_changes_nothing(capi, orc, dev, monkeypatch, 
         o.push(some, more)
         assert_bits_equal(t.dump()[2], o.dump()[2], "repeat at %d" % at)
         t.close()
+
+
+def _lens(rng, n, kind):
+    if kind == "quads":
+        return rng.choice(np.array([8, 16, 32, 64], np.int32), n)
+    return rng.integers(0, 70, n).astype(np.int32)  # (rows without floats among them)
+
+
+def _pull_async(t, dev, keys, out, out_lens=None):
+    """A pull that does not wait for the size of its response."""
+    import torch
+    d_keys = to_dev(keys, dev)
+    torch.cuda.synchronize()
+    t.pull_raw(d_keys.data_ptr(), keys.size, out.data_ptr(), out.numel(), None if out_lens is None else out_lens.data_ptr())
+    t.sync()
+
+
+VAR = [("any", 1), ("any", 511), ("quads", 512), ("any", 513), ("any", 40_000), ("quads", 256 * 512), ("any", 256 * 512 + 1)]
+
+
+@pytest.mark.parametrize("looks", [None, "0"])
+@pytest.mark.parametrize("kind,n", VAR)
+def test_varlen_started_by_one_launch(capi, orc, dev, monkeypatch, kind, n, looks):
+    """Other keys in every request (some held, some new, some that a pull does not find), and a pull right behind the push of
+    its keys; with `looks` 0 every workgroup goes through the request itself."""
+    import torch
+    announce("varlen in one launch", kind, n, looks)
+    if looks is not None:
+        monkeypatch.setenv("PSKV_PUSH_LOOKS", looks)
+    rng = np.random.default_rng(n)
+    t, o = capi.Table(capi.MODE_VARLEN), orc.Store(orc.MODE_VARLEN)
+    keys = unique_keys(rng, 2 * n + 2)
+    length = _lens(rng, keys.size, kind)
+    length[0] = 3
+    for turn in range(3):
+        at = np.sort(rng.choice(keys.size, n, replace=False))
+        lens = length[at]
+        vals = rng.standard_normal(int(lens.sum())).astype(np.float32)
+        t.push(to_dev(keys[at], dev), _shifted(vals, dev, turn), lens=to_dev(lens, dev))
+        o.push(keys[at], vals, lens)
+        for again in (True, False):
+            if not again:
+                at = np.sort(rng.choice(keys.size, n, replace=False))
+            want, want_lens = o.pull(keys[at])[:2]
+            out = _shifted(np.full(int(length[at].sum()) + 5, 7, np.float32), dev, turn)
+            out_lens = torch.full((n,), 7, dtype=torch.int32, device=dev)
+            _pull_async(t, dev, keys[at], out, out_lens)
+            assert np.array_equal(out_lens.cpu().numpy(), want_lens), (turn, again)
+            assert_bits_equal(out.cpu().numpy()[:want.size], want, "turn %d again %d" % (turn, again))
+            assert (out.cpu().numpy()[want.size:] == 7).all()
+    assert_bits_equal(t.dump()[2], o.dump()[2])
+
+
+@pytest.mark.parametrize("looks", [None, "0"])
+@pytest.mark.parametrize("n", [2, 700, 20_000])
+def test_refused_varlen_requests(capi, orc, dev, monkeypatch, n, looks):
+    """A repeated key, a length that is negative or too long, lens that do not add up: nothing is created or changed. A length
+    that differs from the stored one: no stored value changes, rows it created are zero. A response without room:
+    nothing is written. The request behind each is served."""
+    import torch
+    announce("varlen refused", n, looks)
+    if looks is not None:
+        monkeypatch.setenv("PSKV_PUSH_LOOKS", looks)
+    rng = np.random.default_rng(n)
+    t, o = capi.Table(capi.MODE_VARLEN), orc.Store(orc.MODE_VARLEN)
+    keys = unique_keys(rng, 2 * n)
+    length = rng.integers(1, 40, keys.size).astype(np.int32)
+    held = np.arange(0, 2 * n, 2)
+
+    def push(at, lens=None, ks=None):
+        lens = length[at] if lens is None else lens
+        ks = keys[at] if ks is None else ks
+        vals = rng.standard_normal(int(length[at].sum())).astype(np.float32)
+        t.push(to_dev(ks, dev), to_dev(vals, dev), lens=to_dev(lens, dev))
+        return ks, vals, lens
+
+    o.push(*push(held))
+    t.sync()
+    for what in ("repeat", "negative", "long", "sum"):
+        at = np.sort(rng.choice(2 * n, n, replace=False))
+        lens, ks, code = length[at].copy(), keys[at].copy(), capi.EINVAL
+        j = int(rng.integers(1, n))
+        if what == "repeat":
+            ks[j] = ks[j - 1]
+        elif what == "negative":
+            lens[j] = -1
+        elif what == "long":
+            lens[j] = 1 << 28
+        else:
+            lens[j] += 1
+            code = capi.ESIZE_MISMATCH
+        push(at, lens, ks)
+        with pytest.raises(capi.PskvError) as e:
+            t.sync()
+        assert e.value.code == code, what
+        assert t.size() == (o.size()[0], o.size()[1]), what
+        o.push(*push(held))
+        t.sync()
+    # a held row comes with another length, a new one with it
+    at = np.array([held[0], held[0] + 1])
+    lens = np.array([length[held[0]] + 1, 6], np.int32)
+    t.push(to_dev(keys[at], dev), to_dev(np.ones(int(lens.sum()), np.float32), dev), lens=to_dev(lens, dev))
+    with pytest.raises(capi.PskvError) as e:
+        t.sync()
+    assert e.value.code == capi.ELEN_CHANGED
+    o.push(keys[at[1:]], np.zeros(6, np.float32), lens[1:])
+    want = o.pull(keys)[0]
+    out = torch.full((want.size,), 7.0, device=dev)
+    with pytest.raises(capi.PskvError) as e:
+        _pull_async(t, dev, keys, out[:want.size - 1])
+    assert e.value.code == capi.ESIZE_MISMATCH and bool((out == 7).all())
+    _pull_async(t, dev, keys, out)
+    assert_bits_equal(out.cpu().numpy(), want)
+    assert_bits_equal(t.dump()[2], o.dump()[2])
