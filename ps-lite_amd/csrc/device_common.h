@@ -96,6 +96,8 @@ struct alignas(32) DevState {
   // the value of dirty_epoch up to which the slots have been brought up to date since
   unsigned long long dirty_epoch;
   unsigned long long clean_epoch;
+  // the write-back that k_scalar does itself: pieces given away and pieces written (k_same_keys clears both)
+  unsigned int flush_next, flush_done;
   // k_scalar_repeat: votes of the launch in flight (vote.h), and launches served so far << 1 | verdict of the newest
   unsigned int repeat_arrived;
   unsigned long long repeat_verdict;

@@ -1052,7 +1052,7 @@ ScalarCacheUse scalar_cache_use(pskv_table* t, const Request& r) {
 
 int run_scalar(Batch& bt, bool push, bool pull) {
   uint64_t n_largest = 0;
-  bool any_cache = false;
+  bool any_cache = false, behind = false;
   std::vector<ScalarCacheUse> use(bt.size(), kScPlain);
   for (size_t i = 0; i < bt.size(); ++i) {
     Item& it = bt[i];
@@ -1117,6 +1117,12 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       any_cache = true;
       // (a recorded repeat is served from the cache or not at all: nothing to write back first)
       it.flush_unless_same = !per_key && it.tag.try_cache && t->sc_dirty && r.replay != kReplayCapture;
+      // (expected to repeat it: the request's own kernel writes them back if need be)
+      if (it.flush_unless_same && t->sc_track[r.push ? 0 : 1].hit) {
+        it.flush_unless_same = false;
+        d.cache_mode = kCacheOnBehind;
+        behind = true;
+      }
     }
     d.slots = t->slots;
     d.mask = t->cap - 1;
@@ -1149,7 +1155,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   const bool one_launch = repeat_quads != 0;
   if (any_cache && !one_launch) {
     rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
-      return (it.d.cache_mode == kCacheOn && it.tag.try_cache)
+      return ((it.d.cache_mode == kCacheOn || it.d.cache_mode == kCacheOnBehind) && it.tag.try_cache)
                  ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems) : 0ull;
     });
     if (rc) return rc;
@@ -1167,7 +1173,8 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   // lane takes four turns).
   auto nblk = [&](const Item& it) -> uint64_t {
     if (!it.d.n) return 0;
-    const bool four = (it.d.cache_mode == kCacheOn && it.tag.try_cache) || it.d.cache_mode == kCachePerKey;
+    const bool four = (it.d.cache_mode == kCacheOn && it.tag.try_cache) || it.d.cache_mode == kCacheOnBehind ||
+                      it.d.cache_mode == kCachePerKey;
     return grid_for(it.d.n, four ? kBlock * 4 : kBlock, kMaxGrid);
   };
   const bool pinned = bt[0].r.pinned;
@@ -1186,18 +1193,21 @@ int run_scalar(Batch& bt, bool push, bool pull) {
                      : (few ? PSKV_KSET_OF(k_scalar_repeat, false, true, kRepeatFew) : PSKV_KSET_OF(k_scalar_repeat, false, true, kRepeatMany));
     rc = launch_batch(bt, push ? PSKV_KERNEL_PUSH_SCALAR : PSKV_KERNEL_PULL_SCALAR, kernels, repeat_groups, kRepeatBlock);
   } else if (push && pull) {
-    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, true, false), nblk)
-         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, true), nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, false), nblk);
+    rc = behind    ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, true, false, true), nblk)
+         : any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, true, false, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, true, false), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, true, false, false, false), nblk);
   } else if (push) {
-    rc = any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, true, false), nblk)
-         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, true), nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, false), nblk);
+    rc = behind    ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, true, false, true), nblk)
+         : any_cache ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, true, false, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, true, false), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PUSH_SCALAR, PSKV_KSET_OF(k_scalar, true, false, false, false, false), nblk);
   } else {
     const int kind = bt[0].d.cache_mode == kCachePerKey ? PSKV_KERNEL_PULL_PER_KEY : PSKV_KERNEL_PULL_SCALAR;
-    rc = any_cache ? launch_batch(bt, kind, PSKV_KSET_OF(k_scalar, false, true, true, false), nblk)
-         : pinned  ? launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, true), nblk)
-                   : launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, false), nblk);
+    rc = behind    ? launch_batch(bt, kind, PSKV_KSET_OF(k_scalar, false, true, true, false, true), nblk)
+         : any_cache ? launch_batch(bt, kind, PSKV_KSET_OF(k_scalar, false, true, true, false, false), nblk)
+         : pinned  ? launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, true, false), nblk)
+                   : launch_batch(bt, PSKV_KERNEL_PULL_SCALAR, PSKV_KSET_OF(k_scalar, false, true, false, false, false), nblk);
   }
   if (rc) return rc;
   for (size_t i = 0; i < bt.size(); ++i) {

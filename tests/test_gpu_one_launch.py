@@ -200,3 +200,46 @@ def test_refused_varlen_requests(capi, orc, dev, monkeypatch, n, looks):
     _pull_async(t, dev, keys, out)
     assert_bits_equal(out.cpu().numpy(), want)
     assert_bits_equal(t.dump()[2], o.dump()[2])
+
+
+@pytest.mark.parametrize("kind", ["push", "pull", "both"])
+@pytest.mark.parametrize("n", [1, 4096, 4097, 2_500_001])
+def test_cached_values_written_back_by_the_request_that_differs(capi, orc, dev, monkeypatch, kind, n):
+    """The same keys often enough for the host to expect them, then others of the same number (2.5M: more workgroups than
+    the GPU holds): the cached values reach the slots before the first of the others is looked up."""
+    import torch
+    announce("write back", kind, n)
+    monkeypatch.setenv("PSKV_SCALAR_CACHE_MIN_KEYS", "1")
+    rng = np.random.default_rng(n)
+    t, o = capi.Table(capi.MODE_SCALAR), orc.Store(orc.MODE_SCALAR)
+    pool = unique_keys(rng, n + n // 2 + 1)
+    same = np.sort(rng.choice(pool, n, replace=False))
+    if n > 1:
+        same[-1] = 2**64 - 1  # (the key that lives in the side slot)
+    other = np.sort(rng.choice(pool, n, replace=False))
+    other[-1] = max(other[-1], same[-1])
+    vals = [rng.standard_normal(n).astype(np.float32) for _ in range(2)]
+
+    def request(keys, v):
+        out = torch.zeros(n, device=dev)
+        torch.cuda.synchronize()
+        want = None
+        if kind == "both":
+            t.pushpull(to_dev(keys, dev), to_dev(v, dev), out)
+            want = o.pushpull(keys, v)[0]
+        else:
+            if kind == "push" or keys is same:
+                t.push(to_dev(keys, dev), to_dev(v, dev))
+                o.push(keys, v)
+            if kind == "pull":
+                t.pull(to_dev(keys, dev), out)
+                want = o.pull(keys)[0]
+        t.sync()
+        if want is not None:
+            assert_bits_equal(out.cpu().numpy(), want)
+
+    for _ in range(2):
+        for turn in range(4):
+            request(same, vals[turn & 1])
+        request(other, vals[0])
+    assert_bits_equal(t.dump()[2], o.dump()[2])
