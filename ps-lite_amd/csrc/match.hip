@@ -4,8 +4,8 @@
 //     if (dst_key[i] == src_key[j]) dst_val[i] op= src_val[j]        (k floats per key)
 // Both key sets are sorted, so the keys of one that can match a tile of the other's are
 // one contiguous stretch. A first small kernel finds where every tile's stretch begins (one
-// search per tile, all tiles at once); a workgroup then stages its stretch in LDS, or samples it there
-// where it is long, and resolves its keys, so where the sets are of like size all key traffic is streamed, once. For
+// search per tile, all tiles at once; where there are few, the workgroups do so themselves); a workgroup then stages its
+// stretch in LDS, or samples it there where it is long, and resolves its keys, so where the sets are of like size all key traffic is streamed, once. For
 // k == 1 the values are combined in the same kernel; for longer values the kernel leaves the index of every key's match
 // behind and a second kernel streams the rows.
 #include <hip/hip_ext.h>
@@ -13,6 +13,7 @@
 
 #include <mutex>
 #include <new>
+#include <type_traits>
 
 #include "device_common.h"
 #include "host_common.h"
@@ -31,6 +32,7 @@ constexpr unsigned kMatchTurn = 3;      // source keys a lane asks for at a time
 // A longer stretch than so many pieces is sampled, not staged. (Pieces follow from each other, but read in one go
 // what the sampled search reads key by key: they pay while there are workgroups enough to fill the GPU.)
 constexpr unsigned kMatchPieces = 8, kMatchPiecesFew = 3;
+constexpr unsigned kOwnSpans = 4096;
 constexpr uint64_t kNoMatch = ~0ull;
 constexpr unsigned kCounts = 64;        // counters of matched keys, each on a line of its own
 constexpr unsigned kCountStride = 16;
@@ -115,9 +117,14 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
 // reads, and the row kernel visits, what there is in the source. Bound by memory once the loads do not wait for each
 // other: 12M source against 16M destination keys took 100 us with one source key per lane asked for at a time, 77 with
 // three (5.2 TB/s).
+// OWN: the workgroup finds where its stretch begins and ends itself (a wavefront each) instead of reading it from `spans`:
+// the search is hidden behind the keys of the tile, and a launch of 10 to 13 us in front of this one falls away, but every
+// workgroup reads lines for it that nobody else needs. Up to kOwnSpans tiles that is the better way (us per call:
+// 45,928 into 44,225 keys 16.6 -> 13.5, 1M into 1M 28.0 -> 21.4, 2.6M into 1.4M 39.3 -> 32.6, 4M into 4M 47.9 -> 46.2;
+// beyond it 6M into 6M 56.4 -> 58).
 // K1: values are single floats and are combined here; otherwise where[i] receives the index in `far` of the match of
 // key i, or kNoMatch.
-template <bool K1, bool SWAP, unsigned ITEMS>
+template <bool K1, bool SWAP, unsigned ITEMS, bool OWN>
 __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __restrict__ far, uint64_t n_far,
                                                             const uint64_t* __restrict__ near, uint64_t n_near,
                                                             const uint64_t* __restrict__ spans,
@@ -144,7 +151,17 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
 #pragma unroll
     for (unsigned r = 0; r < ITEMS; ++r) key[r] = near[idx0 + r < tile_n ? i0 + r : first];
   }
-  const uint64_t lo = spans[blockIdx.x], hi = spans[blockIdx.x + 1];
+  __shared__ uint64_t s_span[OWN ? 2 : 1];
+  if (OWN) {
+    const unsigned wave = threadIdx.x >> 6;
+    if (wave < 2) {
+      const uint64_t at = first + wave * kTile;
+      const uint64_t end = at < n_near ? wave_lower_bound(far, n_far, near[at], threadIdx.x & 63) : n_far;
+      if ((threadIdx.x & 63) == 0) s_span[wave] = end;
+    }
+    __syncthreads();
+  }
+  const uint64_t lo = OWN ? s_span[0] : spans[blockIdx.x], hi = OWN ? s_span[OWN ? 1 : 0] : spans[blockIdx.x + 1];
   const uint64_t span = hi > lo ? hi - lo : 0;  // (hi >= lo when the keys are sorted)
   // K1: the values follow the keys without waiting for what the search finds: those of this side are
   // asked for here (a line of 32 of them without a match is rare), those of a stretch that fits into LDS come
@@ -479,13 +496,15 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
   const bool few = n_near < kFewKeys || n_far / n_near >= 2;
   const unsigned tile = kMatchBlock * (few ? 1 : kMatchItems);
   const unsigned blocks = (unsigned)((n_near + tile - 1) / tile);
-  {
+  const bool own = blocks <= kOwnSpans;
+  if (!own) {
     int rc = room(&c->spans, ((size_t)blocks + 1) * sizeof(uint64_t), st);
     if (rc) return rc;
   }
   uint64_t* spans = static_cast<uint64_t*>(c->spans.ptr);
-  hipLaunchKernelGGL(k_match_spans, dim3((blocks + kSpanTiles - 1) / kSpanTiles), dim3(kSpanBlock), 0, st, far, n_far, near,
-                     (uint64_t)blocks, tile, spans);
+  if (!own)
+    hipLaunchKernelGGL(k_match_spans, dim3((blocks + kSpanTiles - 1) / kSpanTiles), dim3(kSpanBlock), 0, st, far, n_far, near,
+                       (uint64_t)blocks, tile, spans);
   // (a launch can carry events of its own, which read the begin and the end of that very dispatch)
   hipEvent_t e0 = kernel_ms ? c->ev[0] : nullptr, e1 = kernel_ms ? c->ev[1] : nullptr;
   hipEvent_t e2 = kernel_ms ? c->ev[2] : nullptr, e3 = kernel_ms ? c->ev[3] : nullptr;
@@ -495,9 +514,13 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
     if (rc) return rc;
     where = static_cast<uint64_t*>(c->where.ptr);
   }
-  auto keys = k == 1 ? (swap ? (few ? k_match_keys<true, true, 1> : k_match_keys<true, true, kMatchItems>)
-                             : (few ? k_match_keys<true, false, 1> : k_match_keys<true, false, kMatchItems>))
-                     : (few ? k_match_keys<false, false, 1> : k_match_keys<false, false, kMatchItems>);
+  auto pick = [&](auto o) {
+    constexpr bool OWN = decltype(o)::value;
+    return k == 1 ? (swap ? (few ? k_match_keys<true, true, 1, OWN> : k_match_keys<true, true, kMatchItems, OWN>)
+                          : (few ? k_match_keys<true, false, 1, OWN> : k_match_keys<true, false, kMatchItems, OWN>))
+                  : (few ? k_match_keys<false, false, 1, OWN> : k_match_keys<false, false, kMatchItems, OWN>);
+  };
+  auto keys = own ? pick(std::true_type()) : pick(std::false_type());
   hipExtLaunchKernelGGL(keys, dim3(blocks), dim3(kMatchBlock), 0, st, e0, e1, 0, far, n_far, near, n_near, spans, where, d_sv,
                         d_dv, op, c->counts);
   if (k > 1) {
