@@ -333,10 +333,19 @@ __global__ __launch_bounds__(kBlock) void k_concat(const Segment* __restrict__ s
 // Per-call state of the slicer. Calls may come from any thread at once
 // (KVWorker::Push is thread-safe, kv_app.h:101-104), so each call takes a context
 // of its own from a pool and returns it afterwards.
+// A process has few hardware queues (four), and a stream shares its one with others: where those are tables with
+// requests queued, every call waits behind them (20 pushes of 1M keys, sliced one by one: 2,250 us, or 2,040 where it
+// does not). Nothing says which queue a stream is on, but the calls themselves: a context whose calls take long tries
+// other streams and keeps to the one on which they took least.
+constexpr int kSliceStreams = 4;
+constexpr float kSliceSlow = 20.0f;  // us; a call that waits for nobody takes 9 to 12
 struct SliceCtx {
   unsigned long long calls = 0;  // numbers the calls whose completion the host watches for
   int device = -1;
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr;  // the one in use, of
+  hipStream_t streams[kSliceStreams] = {nullptr};
+  float took[kSliceStreams] = {0.0f};  // us per call lately; forgotten little by little while another one is in use
+  int at = 0;
   SumsState* sums_state = nullptr;
   void* dev = nullptr;      // device scratch: targets, lower bounds, positions, sums
   size_t dev_bytes = 0;
@@ -361,15 +370,33 @@ SliceCtx* take_ctx(int device) {
   SliceCtx* c = new (std::nothrow) SliceCtx();
   if (!c) return nullptr;
   c->device = device;
-  if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
+  // (all of them at once: a stream gets the queue that the fewest are on, so they end up on one each and leave the tables'
+  // streams spread as they were)
+  bool streams = true;
+  for (hipStream_t& s : c->streams) streams = streams && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess;
+  if (!streams ||
       hipMalloc(reinterpret_cast<void**>(&c->sums_state), sizeof(SumsState)) != hipSuccess ||
       hipMemset(c->sums_state, 0, sizeof(SumsState)) != hipSuccess) {
     if (c->sums_state) (void)hipFree(c->sums_state);
-    if (c->stream) (void)hipStreamDestroy(c->stream);
+    for (hipStream_t s : c->streams)
+      if (s) (void)hipStreamDestroy(s);
     delete c;
     return nullptr;
   }
+  c->stream = c->streams[0];
   return c;
+}
+
+// A call on the context's stream has taken `us` and nothing of it is left: the stream of the next one.
+void note_call(SliceCtx* c, float us) {
+  for (int i = 0; i < kSliceStreams; ++i) c->took[i] *= i == c->at ? 0.75f : 0.98f;
+  c->took[c->at] += 0.25f * us;
+  if (c->took[c->at] < kSliceSlow) return;
+  int best = c->at;
+  for (int i = 0; i < kSliceStreams; ++i)
+    if (c->took[i] < 0.8f * c->took[best]) best = i;
+  c->at = best;
+  c->stream = c->streams[best];
 }
 
 void give_ctx(SliceCtx* c) {
@@ -518,6 +545,7 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     const bool few = S + 1 <= kFusedTargets;
     const bool sums_too = do_sums && few && std::is_sorted(h_targets, h_targets + S + 1);
     const unsigned long long watch = !do_sums || sums_too ? ++c->calls : 0ull;
+    const auto asked = std::chrono::steady_clock::now();
     h_pos[S + 1] = 0;  // (whatever an earlier call with other ranges left at this place)
     FusedTargets ft = {};
     if (few)
@@ -551,6 +579,8 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     if (!watch || !seen_in_time(reinterpret_cast<unsigned long long*>(h_pos + S + 1), watch))
       PSKV_HIP(hipStreamSynchronize(c->stream));
     lease.idle = true;  // (the kernel's last act was that word)
+    if (watch)
+      note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count());
     for (size_t i = 0; i <= S; ++i) pos[i] = h_pos[i];
     if (do_sums)
       for (size_t i = 0; i < S; ++i) val_pos[i + 1] = h_sums[i];  // per-slice sums for now

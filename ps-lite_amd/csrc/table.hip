@@ -131,25 +131,22 @@ __global__ void k_read_state(StateBatch sb) {
 // request buffers, events, its stream. Creating them costs the calling thread about a millisecond (every
 // pinned allocation and its release go through the driver), so a table that goes leaves its shell to
 // the next one: up to kShellsKept per device (2.1 MiB of pinned memory each), given back by pskv_device_trim, and
-// (but for the streams) some time after the last table of the device has gone.
+// some time after the last table of the device has gone.
 struct Shell {
   DevState* st = nullptr;
   char* pinned = nullptr;  // StateView, Snapshot, outcome word, done word (256 bytes each), small_in, small_out
   hipEvent_t done[kSmallParts] = {nullptr};
-  hipStream_t stream = nullptr;  // the stream of a table that was not given one
 };
 constexpr size_t kShellsKept = 32;
 
 struct ShellPool {
   std::mutex mu;
   std::vector<Shell*> idle;
-  std::vector<hipStream_t> streams;  // of shells that have gone back (shell_trim)
 };
 ShellPool g_shells[64];
 
 void shell_free(Shell* sh) {
   if (!sh) return;
-  if (sh->stream) (void)hipStreamDestroy(sh->stream);
   if (sh->st) (void)hipFree(sh->st);
   if (sh->pinned) (void)hipHostFree(sh->pinned);
   for (hipEvent_t e : sh->done)
@@ -199,46 +196,92 @@ void shell_give(int device, Shell* sh) {
   shell_free(sh);
 }
 
-// The stream that the next shell without one gets: one that a shell has left, or null.
-hipStream_t shell_stream(int device) {
-  if (device >= 64) return nullptr;
-  ShellPool& p = g_shells[device];
-  std::lock_guard<std::mutex> lk(p.mu);
-  if (p.streams.empty()) return nullptr;
-  hipStream_t s = p.streams.back();
-  p.streams.pop_back();
-  return s;
-}
-
-// With `device` current: idle shells go. Their streams stay (`streams_too`: or not): they are no memory, and a new
-// stream may come to share a hardware queue with other streams than the old one did, which moves a caller with
-// several tables by a tenth either way.
-void shell_trim(int device, bool streams_too) {
+// With `device` current: idle shells go.
+void shell_trim(int device) {
   std::vector<Shell*> go;
-  std::vector<hipStream_t> streams;
   {
     ShellPool& p = g_shells[device];
     std::lock_guard<std::mutex> lk(p.mu);
     go.swap(p.idle);
-    if (streams_too) {
-      streams.swap(p.streams);
-    } else {
-      for (Shell* sh : go) {
-        if (sh->stream && p.streams.size() < kShellsKept) {
-          p.streams.push_back(sh->stream);
-          sh->stream = nullptr;
-        }
-      }
-    }
   }
   for (Shell* sh : go) shell_free(sh);
-  for (hipStream_t s : streams) (void)hipStreamDestroy(s);
+}
+
+// The streams of tables that were not given one. A process has four hardware queues, and a stream is put on the one that
+// the fewest streams are on when it is made, used or not: streams that are made one by one, as tables come and go, end
+// up anywhere, and tables whose streams share a queue run one after the other. Four that are made together lie on one
+// queue each, so they are, and a new table gets a stream of the place among the four that the fewest tables are on.
+// (Three tables of 200,000 rows in turn, other rows in every step: 196 us a step on a queue each, 223 on the same one.)
+// They stay when their tables go: they are no memory, and the ones that took their place might lie elsewhere.
+constexpr int kQueues = 4;
+struct StreamPool {
+  std::mutex mu;
+  struct Entry {
+    hipStream_t stream;
+    int place;
+    bool used;
+  };
+  std::vector<Entry> all;
+};
+StreamPool g_streams[64];
+
+// A stream for a table on `device` (current), or null.
+hipStream_t stream_take(int device) {
+  hipStream_t alone = nullptr;
+  if (device >= 64) return hipStreamCreateWithFlags(&alone, hipStreamNonBlocking) == hipSuccess ? alone : nullptr;
+  StreamPool& p = g_streams[device];
+  std::lock_guard<std::mutex> lk(p.mu);
+  int used[kQueues] = {0};
+  for (const StreamPool::Entry& e : p.all) used[e.place] += e.used ? 1 : 0;
+  auto best = [&]() -> StreamPool::Entry* {
+    StreamPool::Entry* b = nullptr;
+    for (StreamPool::Entry& e : p.all)
+      if (!e.used && (!b || used[e.place] < used[b->place])) b = &e;
+    return b;
+  };
+  StreamPool::Entry* e = best();
+  if (!e || used[e->place] > *std::min_element(used, used + kQueues)) {
+    for (int q = 0; q < kQueues; ++q) {
+      hipStream_t s = nullptr;
+      if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess)
+        p.all.push_back({s, q, false});
+      else
+        (void)hipGetLastError();
+    }
+    e = best();
+  }
+  if (!e) return nullptr;
+  e->used = true;
+  return e->stream;
+}
+
+void stream_give(int device, hipStream_t stream) {
+  if (device >= 64) {
+    (void)hipStreamDestroy(stream);
+    return;
+  }
+  StreamPool& p = g_streams[device];
+  std::lock_guard<std::mutex> lk(p.mu);
+  for (StreamPool::Entry& e : p.all)
+    if (e.stream == stream) e.used = false;
+}
+
+// With `device` current: the streams that no table has go.
+void stream_trim(int device) {
+  if (device >= 64) return;
+  StreamPool& p = g_streams[device];
+  std::lock_guard<std::mutex> lk(p.mu);
+  for (size_t i = p.all.size(); i-- > 0;) {
+    if (p.all[i].used) continue;
+    (void)hipStreamDestroy(p.all[i].stream);
+    p.all.erase(p.all.begin() + (ptrdiff_t)i);
+  }
 }
 
 // What tables that are gone have left (`device` is current).
 void give_back(int device) {
   array_trim(device);
-  if (device < 64) shell_trim(device, false);
+  if (device < 64) shell_trim(device);
 }
 
 }  // namespace
@@ -250,6 +293,7 @@ struct pskv_table {
   int device = 0;
   int mode = PSKV_MODE_SCALAR;
   hipStream_t stream = nullptr;
+  hipStream_t own_stream = nullptr;  // the same, where the table was not given one
   float max_load = 0.5f;
 
   Slot* slots = nullptr;
@@ -2164,10 +2208,9 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   if (opts->stream) {
     t->stream = static_cast<hipStream_t>(opts->stream);
   } else {
-    if (!t->shell->stream) t->shell->stream = shell_stream(t->device);
-    if (!t->shell->stream && hipStreamCreateWithFlags(&t->shell->stream, hipStreamNonBlocking) != hipSuccess)
-      return fail(set_error(PSKV_EHIP, "hipStreamCreateWithFlags failed"));
-    t->stream = t->shell->stream;
+    t->own_stream = stream_take(t->device);
+    if (!t->own_stream) return fail(set_error(PSKV_EHIP, "hipStreamCreateWithFlags failed"));
+    t->stream = t->own_stream;
   }
   t->st = t->shell->st;
   t->st_host = reinterpret_cast<StateView*>(t->shell->pinned);
@@ -2227,6 +2270,7 @@ int pskv_table_destroy(pskv_table* t) {
                            &t->sc_vals, &t->sc_slots})
     (void)array_release(b->ptr, t->stream, idle);
   shell_give(t->device, t->shell);
+  if (t->own_stream) stream_give(t->device, t->own_stream);
   device_tables(t->device, -1, give_back);
   delete t;
   return PSKV_OK;
@@ -2580,7 +2624,8 @@ int pskv_device_trim(int device) {
   DeviceGuard guard(device);
   if (!guard.ok()) return set_error(PSKV_EHIP, "cannot select device %d", device);
   array_trim(device);
-  shell_trim(device, true);
+  shell_trim(device);
+  stream_trim(device);
   return match_trim(device);
 }
 
