@@ -25,12 +25,23 @@ __global__ __launch_bounds__(kBlock) void k_bounds(const uint64_t* __restrict__ 
   if (lane == 0) lb[w] = lo;
 }
 
-// The word behind the S+1 positions in pinned host memory tells a host that is watching it that
-// the positions of call number `done_seq` are all there (0: nobody is watching).
-__device__ __forceinline__ void announce_done(uint64_t* pos_host, uint64_t S, unsigned long long done_seq) {
-  if (pos_host && done_seq)
-    __hip_atomic_store(reinterpret_cast<unsigned long long*>(pos_host + S + 1), done_seq, __ATOMIC_RELEASE,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
+// What the host reads goes to pinned memory, every word with a mark of its own that it is there (the host has cleared it):
+// the host watches all of them, nothing has to arrive before anything else, and no fence writes back what the requests that
+// run meanwhile have left in the L2. Positions and sums are below 2^62 in size.
+constexpr uint64_t kHere = 1ull << 63;
+__device__ __forceinline__ void tell(uint64_t* to, uint64_t x) {
+  __hip_atomic_store(to, x | kHere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+uint64_t told(uint64_t word) { return (uint64_t)((int64_t)(word << 1) >> 1); }  // (sums of lens may be negative)
+
+// The largest of this lane's and all lower lanes' values.
+__device__ __forceinline__ uint64_t wave_running_max(uint64_t x, unsigned lane) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y = __shfl_up(x, o);
+    if (lane >= (unsigned)o && y > x) x = y;
+  }
+  return x;
 }
 
 // kv_app.h:528-541: pos[0] = lower_bound(keys, ranges[0].begin); every further
@@ -41,21 +52,20 @@ __device__ __forceinline__ void announce_done(uint64_t* pos_host, uint64_t S, un
 // cleared for the kernel that follows.
 __global__ void k_bounds_chain(const uint64_t* __restrict__ lb, uint64_t S,
                                uint64_t* __restrict__ pos, uint64_t* __restrict__ pos_host,
-                               unsigned long long* __restrict__ sums, unsigned long long done_seq) {
+                               unsigned long long* __restrict__ sums) {
   if (blockIdx.x != 0) return;
   if (sums)
     for (uint64_t i = threadIdx.x; i < S; i += blockDim.x) sums[i] = 0ull;
   if (threadIdx.x != 0) return;
   uint64_t p = lb[0];
   pos[0] = p;
-  if (pos_host) pos_host[0] = p;
+  if (pos_host) tell(&pos_host[0], p);
   for (uint64_t i = 0; i < S; ++i) {
     const uint64_t e = lb[i + 1];
     p = e > p ? e : p;
     pos[i + 1] = p;
-    if (pos_host) pos_host[i + 1] = p;
+    if (pos_host) tell(&pos_host[i + 1], p);
   }
-  announce_done(pos_host, S, done_seq);
 }
 
 // Both of the above in one launch when the boundaries are few (the stock case: one per server):
@@ -68,8 +78,7 @@ struct FusedTargets {
 };
 __global__ __launch_bounds__(kFusedWaves * 64) void k_bounds_fused(
     const uint64_t* __restrict__ keys, uint64_t n, FusedTargets targets, uint64_t S,
-    uint64_t* __restrict__ pos, uint64_t* __restrict__ pos_host, unsigned long long* __restrict__ sums,
-    unsigned long long done_seq) {
+    uint64_t* __restrict__ pos, uint64_t* __restrict__ pos_host, unsigned long long* __restrict__ sums) {
   __shared__ uint64_t s_lb[kFusedTargets];
   const unsigned lane = threadIdx.x & 63, waves = blockDim.x >> 6;
   for (unsigned w = threadIdx.x >> 6; w <= S; w += waves) {  // whole wavefronts
@@ -79,17 +88,14 @@ __global__ __launch_bounds__(kFusedWaves * 64) void k_bounds_fused(
   __syncthreads();
   if (sums)
     for (uint64_t i = threadIdx.x; i < S; i += blockDim.x) sums[i] = 0ull;
-  if (threadIdx.x != 0) return;
-  uint64_t p = s_lb[0];
-  pos[0] = p;
-  if (pos_host) pos_host[0] = p;
-  for (uint64_t i = 0; i < S; ++i) {
-    const uint64_t e = s_lb[i + 1];
-    p = e > p ? e : p;
-    pos[i + 1] = p;
-    if (pos_host) pos_host[i + 1] = p;
+  if (threadIdx.x >= 64) return;
+  static_assert(kFusedTargets <= 64, "a lane per position");
+  uint64_t p = 0;  // (the reads of LDS do not wait for each other, the steps of a scan over the lanes would)
+  for (unsigned i = 0; i <= S; ++i) p = i <= lane && s_lb[i] > p ? s_lb[i] : p;
+  if (lane <= S) {
+    pos[lane] = p;
+    if (pos_host) tell(&pos_host[lane], p);
   }
-  announce_done(pos_host, S, done_seq);
 }
 
 // Boundaries and the lens sums of the slices between them in one launch (few boundaries, in ascending
@@ -104,12 +110,118 @@ struct SumsState {                         // device memory of one slicer contex
   unsigned long long sums[kFusedTargets];
   unsigned ticket;
 };
+// What the workgroup that finishes last hands to the host. One wavefront.
+__device__ __forceinline__ void hand_over(SumsState* state, unsigned S, unsigned lane, uint64_t* pos_host,
+                                          unsigned long long* sums_host) {
+  uint64_t p = 0;
+  if (lane <= S) p = __hip_atomic_load(&state->pos[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (lane < S)
+    tell(reinterpret_cast<uint64_t*>(&sums_host[lane]),
+         __hip_atomic_load(&state->sums[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  p = wave_running_max(p, lane);
+  if (lane <= S) tell(&pos_host[lane], p);
+  // (the next call's kernel is behind this one on the stream)
+  if (lane < S) state->sums[lane] = 0ull;
+  if (lane <= S) state->pos[lane] = 0ull;  // (keys that are not sorted may leave a boundary without an owner)
+  if (lane == 0) state->ticket = 0;
+}
+
+// A request of up to kFewSumsKeys keys: everything that a workgroup needs is asked for at once, eight keys and lens a
+// thread, the lens are added up by one scan, and the key that a boundary falls in front of says where that is and what lies
+// below. (The searches of the kernel below are trips to memory that follow from each other, and every slice is added up for
+// itself. us per call: 5,000 keys over 16 ranges 19.2 -> 13.5, 15,826 over 3 15.1 -> 12.3, 100,000 over 16 17.0 -> 13.7.)
+constexpr unsigned kFewSumsBlock = 256, kFewSumsItems = 8;  // (larger workgroups find no place on a busy GPU)
+constexpr uint64_t kFewSumsPart = (uint64_t)kFewSumsBlock * kFewSumsItems;
+constexpr uint64_t kFewSumsKeys = 128 * kFewSumsPart;
+__global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_t* __restrict__ keys,
+                                                                   const int32_t* __restrict__ lens, uint64_t n,
+                                                                   FusedTargets targets, unsigned S, SumsState* state,
+                                                                   uint64_t* __restrict__ pos_host,
+                                                                   unsigned long long* __restrict__ sums_host) {
+  constexpr unsigned kWaves = kFewSumsBlock / 64;
+  typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
+  __shared__ unsigned long long s_wave[kWaves];
+  __shared__ uint64_t s_at[kFusedTargets];
+  __shared__ unsigned long long s_below[kFusedTargets];
+  __shared__ uint64_t s_before, s_end;
+  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t c0 = (uint64_t)blockIdx.x * kFewSumsPart;
+  const uint64_t c1 = n - c0 < kFewSumsPart ? n : c0 + kFewSumsPart;
+  const uint64_t i0 = c0 + (uint64_t)threadIdx.x * kFewSumsItems;
+  const unsigned mine = i0 >= c1 ? 0u : c1 - i0 < kFewSumsItems ? (unsigned)(c1 - i0) : kFewSumsItems;
+  uint64_t key[kFewSumsItems], prev = 0;
+  unsigned long long len[kFewSumsItems];
+  if (mine == kFewSumsItems) {
+#pragma unroll
+    for (unsigned j = 0; j < kFewSumsItems; j += 4) {
+      const u64x2u a = *reinterpret_cast<const u64x2u*>(keys + i0 + j), b = *reinterpret_cast<const u64x2u*>(keys + i0 + j + 2);
+      const i32x4u l = *reinterpret_cast<const i32x4u*>(lens + i0 + j);
+      key[j] = a.x, key[j + 1] = a.y, key[j + 2] = b.x, key[j + 3] = b.y;
+#pragma unroll
+      for (unsigned r = 0; r < 4; ++r) len[j + r] = (unsigned long long)(long long)l[r];
+    }
+  } else {
+#pragma unroll
+    for (unsigned j = 0; j < kFewSumsItems; ++j) {
+      key[j] = j < mine ? keys[i0 + j] : 0;
+      len[j] = j < mine ? (unsigned long long)(long long)lens[i0 + j] : 0ull;
+    }
+  }
+  if (mine && i0) prev = keys[i0 - 1];
+  if (threadIdx.x == 0) s_before = prev;
+  uint64_t top = key[0];  // the thread's last key
+#pragma unroll
+  for (unsigned j = 1; j < kFewSumsItems; ++j) top = j < mine ? key[j] : top;
+  if (mine && i0 + mine == c1) s_end = top;
+  unsigned long long sum = 0;
+#pragma unroll
+  for (unsigned j = 0; j < kFewSumsItems; ++j) sum += len[j];
+  const unsigned long long upto = wave_incl_scan_u64(sum);
+  if (lane == 63) s_wave[wave] = upto;
+  __syncthreads();
+  unsigned long long below = upto - sum, all = 0;
+#pragma unroll
+  for (unsigned w = 0; w < kWaves; ++w) {
+    if (w < wave) below += s_wave[w];
+    all += s_wave[w];
+  }
+  for (unsigned i = 0; i <= S; ++i) {  // (few threads hold a boundary, most boundaries lie elsewhere)
+    const uint64_t target = targets.v[i];
+    if (!mine || top < target || (i0 && prev >= target)) continue;
+    unsigned long long x = below;
+    uint64_t at = i0;
+#pragma unroll
+    for (unsigned j = 0; j + 1 < kFewSumsItems; ++j)
+      if (j < mine && key[j] < target) x += len[j], ++at;
+    s_at[i] = at;
+    s_below[i] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const uint64_t before = s_before, end = s_end;
+  unsigned long long under = 0;
+  if (lane <= S) {
+    const uint64_t target = targets.v[lane];
+    const bool after_start = c0 == 0 || before < target, inside = after_start && end >= target;
+    under = inside ? s_below[lane] : after_start ? all : 0ull;
+    // the boundary is this stretch's if it does not lie before it, nor behind it unless it is the last one
+    if (after_start && (c1 == n || inside)) publish_u64(&state->pos[lane], inside ? s_at[lane] : c1);
+  }
+  const unsigned long long next = __shfl_down(under, 1);
+  if (lane < S && next != under) atomicAdd(&state->sums[lane], next - under);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);  // what this lane has handed over is there before the ticket is taken
+  unsigned last = 0;
+  if (lane == 0) last = atomicAdd(&state->ticket, 1u) == gridDim.x - 1 ? 1u : 0u;
+  if (__shfl(last, 0)) hand_over(state, S, lane, pos_host, sums_host);
+}
+
 __global__ __launch_bounds__(kBlock) void k_bounds_sums(const uint64_t* __restrict__ keys,
                                                        const int32_t* __restrict__ lens, uint64_t n, uint64_t chunk,
                                                        FusedTargets targets, unsigned S, SumsState* state,
                                                        uint64_t* __restrict__ pos_host,
-                                                       unsigned long long* __restrict__ sums_host,
-                                                       unsigned long long done_seq) {
+                                                       unsigned long long* __restrict__ sums_host) {
   __shared__ uint64_t s_b[kFusedTargets];
   __shared__ unsigned long long s_red[kBlock / 64];
   __shared__ unsigned s_last;
@@ -161,25 +273,8 @@ __global__ __launch_bounds__(kBlock) void k_bounds_sums(const uint64_t* __restri
   }
   __syncthreads();
   if (!s_last) return;
-  if (threadIdx.x < S) {
-    sums_host[threadIdx.x] = __hip_atomic_load(&state->sums[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    state->sums[threadIdx.x] = 0ull;
-  }
-  if (threadIdx.x <= S) {
-    s_b[threadIdx.x] = __hip_atomic_load(&state->pos[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    state->pos[threadIdx.x] = 0ull;  // (keys that are not sorted may leave a boundary without an owner)
-  }
-  __threadfence_system();
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  state->ticket = 0;
-  uint64_t p = s_b[0];
-  pos_host[0] = p;
-  for (unsigned i = 0; i < S; ++i) {
-    p = s_b[i + 1] > p ? s_b[i + 1] : p;
-    pos_host[i + 1] = p;
-  }
-  announce_done(pos_host, S, done_seq);
+  if (threadIdx.x >= 64) return;
+  hand_over(state, S, lane, pos_host, sums_host);
 }
 
 // ---- the slicer for callers that cannot allocate ------------------------------------------
@@ -340,7 +435,6 @@ __global__ __launch_bounds__(kBlock) void k_concat(const Segment* __restrict__ s
 constexpr int kSliceStreams = 4;
 constexpr float kSliceSlow = 20.0f;  // us; a call that waits for nobody takes 9 to 12
 struct SliceCtx {
-  unsigned long long calls = 0;  // numbers the calls whose completion the host watches for
   int device = -1;
   hipStream_t stream = nullptr;  // the one in use, of
   hipStream_t streams[kSliceStreams] = {nullptr};
@@ -387,14 +481,32 @@ SliceCtx* take_ctx(int device) {
   return c;
 }
 
+// Watches `count` marked words (tell()) of pinned memory for up to about 200 us each; false when one did not show up.
+bool all_here(const uint64_t* words, size_t count) {
+  for (size_t i = 0; i < count; ++i) {
+    if (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0) continue;
+    const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    for (bool here = false; !here;) {
+      for (int spin = 0; spin < 256 && !here; ++spin) here = __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0;
+      if (!here && std::chrono::steady_clock::now() > give_up) return false;
+    }
+  }
+  return true;
+}
+
 // A call on the context's stream has taken `us` and nothing of it is left: the stream of the next one.
 void note_call(SliceCtx* c, float us) {
-  for (int i = 0; i < kSliceStreams; ++i) c->took[i] *= i == c->at ? 0.75f : 0.98f;
-  c->took[c->at] += 0.25f * us;
-  if (c->took[c->at] < kSliceSlow) return;
+  float& mine = c->took[c->at];
+  mine = mine == 0.0f ? us : 0.75f * mine + 0.25f * us;
+  for (int i = 0; i < kSliceStreams; ++i)
+    if (i != c->at) c->took[i] *= 0.995f;
+  if (mine < kSliceSlow) return;
+  // (by a good margin: a stream wait comes with it, and where the GPU itself is what calls wait for all are alike)
   int best = c->at;
   for (int i = 0; i < kSliceStreams; ++i)
-    if (c->took[i] < 0.8f * c->took[best]) best = i;
+    if (c->took[i] < 0.75f * mine && c->took[i] < c->took[best]) best = i;
+  if (best == c->at) return;
+  if (hipStreamSynchronize(c->stream) != hipSuccess) return;  // (the kernel may still be clearing its state)
   c->at = best;
   c->stream = c->streams[best];
 }
@@ -526,7 +638,7 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     if (!c) return set_error(PSKV_EHIP, "cannot create a slicer context on device %d", device);
     lease.idle = false;
     // device: lb[S+1] | pos[S+1] | sums[S]      pinned: targets[S+1] | pos[S+1] | sums[S]
-    const size_t arr = pad256((S + 2) * 8);  // S+1 positions and the word that says they are there
+    const size_t arr = pad256((S + 1) * 8);
     int rc = ctx_reserve(c, 3 * arr, 3 * arr);
     if (rc) return rc;
     char* d = static_cast<char*>(c->dev);
@@ -539,33 +651,37 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     unsigned long long* h_sums = reinterpret_cast<unsigned long long*>(h + 2 * arr);
     h_targets[0] = range_begin[0];
     for (size_t i = 0; i < S; ++i) h_targets[i + 1] = range_end[i];
-    // With few boundaries one kernel leaves everything this call waits for in pinned memory and says so in
-    // a word behind it: watching that word costs about 5 us less than a stream wait. (With lens the
+    // With few boundaries one kernel leaves everything this call waits for in pinned memory, word by word:
+    // watching for those costs about 5 us less than a stream wait. (With lens the
     // boundaries must ascend, as those of contiguous ranges do unless a range ends before it begins.)
     const bool few = S + 1 <= kFusedTargets;
-    const bool sums_too = do_sums && few && std::is_sorted(h_targets, h_targets + S + 1);
-    const unsigned long long watch = !do_sums || sums_too ? ++c->calls : 0ull;
+    const bool sums_too = do_sums && few && n < (1ull << 31) && std::is_sorted(h_targets, h_targets + S + 1);
+    const bool watch = !do_sums || sums_too;
     const auto asked = std::chrono::steady_clock::now();
-    h_pos[S + 1] = 0;  // (whatever an earlier call with other ranges left at this place)
+    std::memset(h_pos, 0, (S + 1) * 8);
+    if (sums_too) std::memset(h_sums, 0, S * 8);
     FusedTargets ft = {};
     if (few)
       for (size_t i = 0; i <= S; ++i) ft.v[i] = h_targets[i];
-    if (sums_too) {
+    if (sums_too && n <= kFewSumsKeys) {
+      k_bounds_sums_few<<<dim3((unsigned)((n + kFewSumsPart - 1) / kFewSumsPart)), dim3(kFewSumsBlock), 0, c->stream>>>(
+          keys, lens, n, ft, (unsigned)S, c->sums_state, h_pos, h_sums);
+      PSKV_HIP(hipGetLastError());
+    } else if (sums_too) {
       // (a stretch of at least 2,048 keys, a multiple of four)
       const uint64_t chunk = std::max<uint64_t>(2048, ((n + kSumsMaxBlocks - 1) / kSumsMaxBlocks + 3) & ~(uint64_t)3);
       k_bounds_sums<<<dim3((unsigned)((n + chunk - 1) / chunk)), dim3(kBlock), 0, c->stream>>>(
-          keys, lens, n, chunk, ft, (unsigned)S, c->sums_state, h_pos, h_sums, watch);
+          keys, lens, n, chunk, ft, (unsigned)S, c->sums_state, h_pos, h_sums);
       PSKV_HIP(hipGetLastError());
     } else if (few) {  // one launch for the boundaries
       const unsigned waves = (unsigned)std::min<size_t>(S + 1, kFusedWaves);
       k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, c->stream>>>(keys, n, ft, S, d_pos, h_pos,
-                                                                 do_sums ? d_sums : nullptr, watch);
+                                                                 do_sums ? d_sums : nullptr);
       PSKV_HIP(hipGetLastError());
     } else {
       rc = launch_bounds_search(keys, n, h_targets, S + 1, d_lb, c->stream);
       if (rc) return rc;
-      k_bounds_chain<<<dim3(1), dim3(64), 0, c->stream>>>(d_lb, S, d_pos, h_pos, do_sums ? d_sums : nullptr,
-                                                          watch);
+      k_bounds_chain<<<dim3(1), dim3(64), 0, c->stream>>>(d_lb, S, d_pos, h_pos, do_sums ? d_sums : nullptr);
       PSKV_HIP(hipGetLastError());
     }
     if (do_sums && !sums_too) {
@@ -576,14 +692,14 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
       k_export_sums<<<dim3((unsigned)((S + 255) / 256)), dim3(256), 0, c->stream>>>(d_sums, S, h_sums);
       PSKV_HIP(hipGetLastError());
     }
-    if (!watch || !seen_in_time(reinterpret_cast<unsigned long long*>(h_pos + S + 1), watch))
+    if (!watch || !all_here(h_pos, S + 1) || (sums_too && !all_here(reinterpret_cast<uint64_t*>(h_sums), S)))
       PSKV_HIP(hipStreamSynchronize(c->stream));
-    lease.idle = true;  // (the kernel's last act was that word)
+    lease.idle = true;  // (what the kernel still does is clear its state for the next one on the stream)
     if (watch)
       note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count());
-    for (size_t i = 0; i <= S; ++i) pos[i] = h_pos[i];
+    for (size_t i = 0; i <= S; ++i) pos[i] = told(h_pos[i]);
     if (do_sums)
-      for (size_t i = 0; i < S; ++i) val_pos[i + 1] = h_sums[i];  // per-slice sums for now
+      for (size_t i = 0; i < S; ++i) val_pos[i + 1] = sums_too ? told(h_sums[i]) : h_sums[i];  // per-slice sums for now
   }
 
   for (size_t i = 0; i < S; ++i) used[i] = pos[i + 1] != pos[i];  // kv_app.h:540
@@ -684,7 +800,7 @@ int pskv_slice_noalloc(int device, void* stream, const uint64_t* keys, size_t n,
     ft.v[0] = range_begin[0];
     for (size_t i = 0; i < S; ++i) ft.v[i + 1] = range_end[i];
     const unsigned waves = (unsigned)std::min<size_t>(S + 1, kFusedWaves);
-    k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, st>>>(keys, n, ft, S, pos, (uint64_t*)nullptr, d_sums, 0ull);
+    k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, st>>>(keys, n, ft, S, pos, (uint64_t*)nullptr, d_sums);
     PSKV_HIP(hipGetLastError());
   } else {
     for (size_t first = 0; first <= S; first += kFusedTargets) {
@@ -699,7 +815,7 @@ int pskv_slice_noalloc(int device, void* stream, const uint64_t* keys, size_t n,
       PSKV_HIP(hipGetLastError());
     }
     k_bounds_chain<<<dim3(1), dim3(64), 0, st>>>(reinterpret_cast<const uint64_t*>(d_lb), S, pos,
-                                                (uint64_t*)nullptr, d_sums, 0ull);
+                                                (uint64_t*)nullptr, d_sums);
     PSKV_HIP(hipGetLastError());
   }
   if (do_sums) {

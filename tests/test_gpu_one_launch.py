@@ -243,3 +243,24 @@ def test_cached_values_written_back_by_the_request_that_differs(capi, orc, dev, 
             request(same, vals[turn & 1])
         request(other, vals[0])
     assert_bits_equal(t.dump()[2], o.dump()[2])
+
+
+@pytest.mark.parametrize("S", [1, 3, 16, 31])
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 30_001, 128 * 2048, 128 * 2048 + 1])
+def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
+    """Boundaries and sums of lens by one scan (up to 262,144 keys): the edges of a workgroup's stretch, boundaries on a key,
+    between keys, in front of all and behind all, several in one stretch; called twice, from either kind of memory."""
+    announce("few slices", n, S)
+    rng = np.random.default_rng(n * 31 + S)
+    begin, end = orc.server_ranges(S)
+    sets = [unique_keys(rng, n, S), np.arange(n, dtype=np.uint64) + begin[S // 2]]
+    if S > 1:
+        near = np.concatenate([np.arange(-3, 4).astype(np.int64).astype(np.uint64) + e for e in end[:-1]])
+        sets.append(np.unique(np.concatenate([near, unique_keys(rng, max(1, n - near.size), S)])))
+    for keys in sets:
+        lens = rng.integers(0, 1000, keys.size).astype(np.int32)
+        want = orc.slice_keys(keys, begin, end, lens, int(lens.sum()))
+        for _ in range(2):
+            got = capi.slice_keys(to_dev(keys, dev), begin, end, lens=to_dev(lens, dev), nvals=int(lens.sum()))
+            for a, b in zip(got, want):
+                assert np.array_equal(np.asarray(a), np.asarray(b))
