@@ -210,6 +210,10 @@ int pskv_sync(pskv_table* t);
  * Waits for the device. */
 int pskv_size(pskv_table* t, uint64_t* n_keys, uint64_t* n_vals);
 
+/* The same for tables that share a stream (see pskv_push_multi), with one wait for up to 16 of them:
+ * n_keys and n_vals (either may be null) receive S entries. */
+int pskv_size_multi(pskv_table* const* tables, size_t S, uint64_t* n_keys, uint64_t* n_vals);
+
 /* All stored pairs sorted by key, for stored-key parity checks (the reference has
  * no such call; it is the equivalent of iterating the store, kv_app.h:462).
  * Host buffers only. lens may be NULL. Too small a buffer gives

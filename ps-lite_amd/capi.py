@@ -45,7 +45,7 @@ ERROR_NAMES = {
 # every symbol include/pskv/capi.h declares
 SYMBOLS = [
     "pskv_table_create", "pskv_table_destroy", "pskv_push", "pskv_pull", "pskv_pushpull",
-    "pskv_sync", "pskv_table_stream", "pskv_push_multi", "pskv_pull_multi", "pskv_pushpull_multi", "pskv_sync_multi", "pskv_replay_record", "pskv_replay_run", "pskv_replay_destroy", "pskv_size", "pskv_dump", "pskv_slice", "pskv_slice_noalloc", "pskv_server_ranges",
+    "pskv_sync", "pskv_table_stream", "pskv_push_multi", "pskv_pull_multi", "pskv_pushpull_multi", "pskv_sync_multi", "pskv_replay_record", "pskv_replay_run", "pskv_replay_destroy", "pskv_size", "pskv_size_multi", "pskv_dump", "pskv_slice", "pskv_slice_noalloc", "pskv_server_ranges",
     "pskv_assemble_pull", "pskv_match", "pskv_prof_enable", "pskv_prof_reset", "pskv_prof_read", "pskv_prof_samples",
     "pskv_copy_probe", "pskv_host_alloc", "pskv_host_free", "pskv_host_trim", "pskv_device_trim", "pskv_table_counters", "pskv_last_error",
     "pskv_version",
@@ -119,6 +119,7 @@ def load():
     lib.pskv_replay_run.argtypes = [vp]
     lib.pskv_replay_destroy.argtypes = [vp]
     lib.pskv_size.argtypes = [vp, ctypes.POINTER(u64), ctypes.POINTER(u64)]
+    lib.pskv_size_multi.argtypes = [vp, sz, vp, vp]
     lib.pskv_dump.argtypes = [vp, vp, vp, sz, vp, sz, ctypes.POINTER(sz), ctypes.POINTER(sz)]
     lib.pskv_slice.argtypes = [i32, vp, sz, vp, sz, sz, vp, vp, sz, vp, vp, vp, i32]
     lib.pskv_slice_noalloc.argtypes = [i32, vp, vp, sz, vp, sz, sz, vp, vp, sz, vp, vp, vp, vp]
@@ -501,11 +502,12 @@ class Group(_Holder):
         return rec
 
     def size(self):
-        nk = nv = 0
-        for t in self.tables:
-            a, b = t.size()
-            nk, nv = nk + a, nv + b
-        return nk, nv
+        if self.S == 1:
+            return self.tables[0].size()
+        n = np.zeros((2, max(self.S, 1)), np.uint64)
+        if self.tables:
+            _check(self._lib.pskv_size_multi(self._arr, self.S, n[0].ctypes.data, n[1].ctypes.data))
+        return int(n[0].sum()), int(n[1].sum())
 
 
 class Replay:

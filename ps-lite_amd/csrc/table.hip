@@ -634,14 +634,74 @@ void collect_spare(pskv_table* t, bool wait) {
 }
 
 // The slots a growth goes to when the table has to hold `keys_needed` keys: at least twice the
-// slots; four times while that stays a small array (a table that starts at the default size and
-// keeps growing then moves its keys half as often on the way up).
+// slots; four or eight times while that stays a small array (a table that starts at the default size and
+// keeps growing then moves its keys a half or a third as often on the way up).
 uint64_t grown_cap(const pskv_table* t, uint64_t keys_needed) {
   const uint64_t want = next_pow2((uint64_t)((double)keys_needed / t->max_load) + 1);
-  return std::max(want, t->cap * 4 * sizeof(Slot) <= kSlackBytes ? t->cap * 4 : t->cap * 2);
+  uint64_t factor = 2;
+  while (factor < (uint64_t)kRegrowMaxFactor && t->cap * factor * 2 * sizeof(Slot) <= kSlackBytes) factor *= 2;
+  return std::max(want, t->cap * factor);
 }
 
-int grow_slots(pskv_table* t, uint64_t keys_needed) {
+// Slot arrays that are to move, all tables' of a request with as few launches as there can be. They do so before
+// anything else of the request, when move() is called or, where a request ends early, when the list goes.
+struct Growths {
+  struct One {
+    pskv_table* t;
+    Slot* from;
+    uint64_t cap;  // of `from`; t has the array and the size that it moves to
+  };
+  std::vector<One> list;
+  int move();
+  ~Growths() { (void)move(); }
+};
+
+int Growths::move() {
+  std::vector<One> todo;
+  todo.swap(list);
+  int rc = PSKV_OK;
+  for (size_t first = 0; first < todo.size() && !rc;) {
+    RegrowBatch b;
+    std::memset(&b, 0, sizeof(b));
+    pskv_table* lead = todo[first].t;
+    uint64_t most = 0, factors = 0;
+    unsigned count = 0;
+    for (; first < todo.size() && count < (unsigned)kMaxBatch && !rc; ++first) {
+      const One& g = todo[first];
+      pskv_table* t = g.t;
+      const uint64_t factor = t->cap / g.cap;
+      if (factor > (uint64_t)kRegrowMaxFactor) {
+        // (a small table that a large request makes much larger: fill and scatter)
+        if (hipMemsetAsync(t->slots, 0xFF, t->cap * sizeof(Slot), t->stream) != hipSuccess)
+          rc = set_error(PSKV_EHIP, "hipMemsetAsync failed");
+        if (!rc)
+          rc = launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(g.cap, kBlock, kMaxGrid)), dim3(kBlock), 0,
+                      (const Slot*)g.from, g.cap, t->slots, t->cap - 1, t->st);
+        continue;
+      }
+      b.t[count++] = RegrowOf{g.from, t->slots, g.cap - 1, t->cap - 1, t->st, factor};
+      most = std::max(most, g.cap);
+      factors = std::max(factors, factor);
+    }
+    if (!count || rc) continue;
+    // two streaming passes: the new array is written whole, slot by slot, from LDS
+    const unsigned nblk = (unsigned)(most / kRegrowOld);
+    const size_t lds = (size_t)kRegrowOld * factors * 2 * sizeof(unsigned long long);
+    rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk, count), dim3(kBlock), lds, b);
+    if (!rc)
+      rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock, count),
+                  dim3(kBlock), 0, b);
+  }
+  for (const One& g : todo) {
+    const auto r0 = std::chrono::steady_clock::now();
+    const int gone = array_release(g.from, g.t->stream);
+    g.t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
+    if (!rc) rc = gone;
+  }
+  return rc;
+}
+
+int grow_slots(pskv_table* t, uint64_t keys_needed, Growths* growths) {
   uint64_t want = grown_cap(t, keys_needed);
   Slot* fresh = nullptr;
   int rc = PSKV_OK;
@@ -669,30 +729,10 @@ int grow_slots(pskv_table* t, uint64_t keys_needed) {
   }
   t->spare = nullptr;
   t->spare_cap = 0;
-  const uint64_t factor = want / t->cap;
-  if (factor <= (uint64_t)kRegrowMaxFactor) {
-    // two streaming passes: the new array is written whole, slot by slot, from LDS
-    const unsigned nblk = (unsigned)(t->cap / kRegrowOld);
-    const size_t lds = (size_t)kRegrowOld * factor * 2 * sizeof(unsigned long long);
-    rc = launch(t, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk), dim3(kBlock), lds, t->slots, fresh, t->cap - 1,
-                want - 1, (unsigned)factor);
-    if (rc) return rc;
-    rc = launch(t, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock), dim3(kBlock), 0,
-                (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
-    if (rc) return rc;
-  } else {
-    // (a small table that a large request makes much larger: fill and scatter)
-    PSKV_HIP(hipMemsetAsync(fresh, 0xFF, want * sizeof(Slot), t->stream));
-    rc = launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(t->cap, kBlock, kMaxGrid)), dim3(kBlock), 0,
-                (const Slot*)t->slots, t->cap, fresh, want - 1, t->st);
-    if (rc) return rc;
-  }
-  const auto r0 = std::chrono::steady_clock::now();
-  rc = array_release(t->slots, t->stream);
-  t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
+  growths->list.push_back({t, t->slots, t->cap});
   t->slots = fresh;
   t->cap = want;
-  return rc;
+  return PSKV_OK;
 }
 
 // Called at the end of a request, with its kernels queued: allocates the array of the next growth
@@ -757,7 +797,7 @@ double new_share_at_most(const pskv_table* t) {
   return t->share_known ? std::min(1.0, 1.25 * t->new_share + 0.1) : 1.0;
 }
 
-int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit, PublishReq* pub) {
+int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit, PublishReq* pub, Growths* growths) {
   if (t->no_growth) return PSKV_OK;
   // Two limits. `limit` is the fill the table is kept below; `hard` (0.85 unless max_load is higher) is
   // the fill it must never exceed. The keys in flight count in full against the second, and against the
@@ -817,7 +857,7 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
       const uint64_t most = t->base_count + t->pend_keys + n;
       // (room for two more such requests while that keeps the array a small one)
       const uint64_t slack_n = grown_cap(t, most + 2 * n) * sizeof(Slot) <= kSlackBytes ? 2 * n : 0;
-      int rc = grow_slots(t, most + slack_n);
+      int rc = grow_slots(t, most + slack_n, growths);
       if (rc) return rc;
       ++t->stats.growths_unasked;
     } else if (slots_short() || arena_short() || old_log) {
@@ -831,7 +871,7 @@ int reserve(pskv_table* t, uint64_t n, uint64_t units, uint64_t floats_per_unit,
       const uint64_t slack_n = grown_cap(t, t->base_count + 3 * n) * sizeof(Slot) <= kSlackBytes ? 2 * n : 0;
       const uint64_t slack_u = t->arena_cap * sizeof(float) <= kSlackBytes ? 2 * units : 0;
       if ((double)(t->base_count + n + slack_n) > limit) {
-        rc = grow_slots(t, t->base_count + n + slack_n);
+        rc = grow_slots(t, t->base_count + n + slack_n, growths);
         if (rc) return rc;
       }
       if (units && (t->base_top + units + slack_u) * floats_per_unit > t->arena_cap) {
@@ -1095,6 +1135,7 @@ ScalarCacheUse scalar_cache_use(pskv_table* t, const Request& r) {
 }
 
 int run_scalar(Batch& bt, bool push, bool pull) {
+  Growths growths;
   uint64_t n_largest = 0;
   bool any_cache = false, behind = false;
   std::vector<ScalarCacheUse> use(bt.size(), kScPlain);
@@ -1106,7 +1147,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     it.d = TableReq{};
     if (r.n == 0) continue;
     // (a growth writes the cache back and drops it; a recorded repeat creates no key)
-    int rc = r.replay == kReplayCapture ? PSKV_OK : reserve(t, r.n, 0, 0, &it.pub);
+    int rc = r.replay == kReplayCapture ? PSKV_OK : reserve(t, r.n, 0, 0, &it.pub, &growths);
     if (rc) return rc;
     const int kind_before = t->sc_last_kind;
     if (r.replay) {
@@ -1180,7 +1221,8 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     n_largest = std::max(n_largest, r.n);
   }
   if (!n_largest) return PSKV_OK;
-  int rc;
+  int rc = growths.move();
+  if (rc) return rc;
   // a recorded repeat, where the workgroups that compare it can wait for each other: one launch
   unsigned repeat_quads = 0;
   auto repeat_groups = [&](const Item& it) -> uint64_t {
@@ -1387,6 +1429,7 @@ bool fixed_in_one(const Batch& bt, bool push) {
 }
 
 int run_fixed(Batch& bt, bool push, bool pull) {
+  Growths growths;
   uint64_t n_largest = 0;
   for (Item& it : bt) {
     pskv_table* t = it.t;
@@ -1395,7 +1438,7 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     r.out_nvals = pull ? r.n * k : 0;
     it.d = TableReq{};
     if (r.n == 0) continue;
-    int rc = r.replay == kReplayCapture ? PSKV_OK : reserve(t, r.n, r.n, k, &it.pub);
+    int rc = r.replay == kReplayCapture ? PSKV_OK : reserve(t, r.n, r.n, k, &it.pub, &growths);
     if (rc) return rc;
     rc = grow(t, &t->ws, Carver::need(r.n, sizeof(uint64_t)));
     if (rc) return rc;
@@ -1419,7 +1462,9 @@ int run_fixed(Batch& bt, bool push, bool pull) {
     n_largest = std::max(n_largest, r.n);
   }
   if (!n_largest) return PSKV_OK;
-  int rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
+  int rc = growths.move();
+  if (rc) return rc;
+  rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
   if (rc) return rc;
   const bool one = fixed_in_one(bt, push);
   if (one) {
@@ -1597,6 +1642,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
   }
 
   if (push) {
+    Growths growths;
     for (Item& it : bt) {
       pskv_table* t = it.t;
       Request& r = it.r;
@@ -1604,7 +1650,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       // every key may round its row up to a 16-byte unit, every workgroup may pad its rows' start
       int rc = r.replay == kReplayCapture
                    ? PSKV_OK
-                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * ((r.n + pad_chunk - 1) / pad_chunk), 4, &it.pub);
+                   : reserve(t, r.n, r.nvals / 4 + r.n + kArenaPadUnits * ((r.n + pad_chunk - 1) / pad_chunk), 4, &it.pub, &growths);
       if (rc) return rc;
       if (t->cache_nvals != r.nvals) t->cache_valid = false;  // same lens would mean the same total
       it.tag = next_tag(t, r, true);
@@ -1626,8 +1672,9 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
     }
+    int rc = growths.move();
+    if (rc) return rc;
     const bool start = start_together(bt, n_launch, [](const Item& it) { return it.r.nvals; });
-    int rc;
     if (start) {
       for (Item& it : bt) {
         it.tag.try_cache = it.d.tag.try_cache = 0;
@@ -2473,32 +2520,53 @@ int pskv_sync(pskv_table* t) {
   return report_device_errors(t);
 }
 
+// The keys and floats that a table holds, its state having just been read.
+static int size_of(pskv_table* t, uint64_t* n_keys, uint64_t* n_vals) {
+  const uint64_t nk = t->count;  // includes key 2^64-1 when present
+  if (n_keys) *n_keys = nk;
+  if (!n_vals) return PSKV_OK;
+  if (t->mode == PSKV_MODE_SCALAR) {
+    *n_vals = nk;
+  } else if (t->mode == PSKV_MODE_FIXED) {
+    *n_vals = nk * t->row_len;
+  } else {
+    unsigned long long* d_total = nullptr;
+    PSKV_HIP(hipMalloc(reinterpret_cast<void**>(&d_total), sizeof(unsigned long long)));
+    PSKV_HIP(hipMemsetAsync(d_total, 0, sizeof(unsigned long long), t->stream));
+    k_sum_lens<<<dim3(grid_for(t->cap, kBlock, 4096)), dim3(kBlock), 0, t->stream>>>(
+        t->slots, t->cap, t->st, d_total);
+    unsigned long long total = 0;
+    hipError_t e = hipMemcpyAsync(&total, d_total, sizeof(total), hipMemcpyDeviceToHost, t->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
+    (void)hipFree(d_total);
+    PSKV_HIP(e);
+    *n_vals = total;
+  }
+  return PSKV_OK;
+}
+
 int pskv_size(pskv_table* t, uint64_t* n_keys, uint64_t* n_vals) {
   clear_error();
   if (!t) return set_error(PSKV_EINVAL, "null table");
   DeviceGuard guard(t->device);
   int rc = read_state(t, true);
   if (rc) return rc;
-  const uint64_t nk = t->count;  // includes key 2^64-1 when present
-  if (n_keys) *n_keys = nk;
-  if (n_vals) {
-    if (t->mode == PSKV_MODE_SCALAR) {
-      *n_vals = nk;
-    } else if (t->mode == PSKV_MODE_FIXED) {
-      *n_vals = nk * t->row_len;
-    } else {
-      unsigned long long* d_total = nullptr;
-      PSKV_HIP(hipMalloc(reinterpret_cast<void**>(&d_total), sizeof(unsigned long long)));
-      PSKV_HIP(hipMemsetAsync(d_total, 0, sizeof(unsigned long long), t->stream));
-      k_sum_lens<<<dim3(grid_for(t->cap, kBlock, 4096)), dim3(kBlock), 0, t->stream>>>(
-          t->slots, t->cap, t->st, d_total);
-      unsigned long long total = 0;
-      hipError_t e = hipMemcpyAsync(&total, d_total, sizeof(total), hipMemcpyDeviceToHost, t->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
-      (void)hipFree(d_total);
-      PSKV_HIP(e);
-      *n_vals = total;
-    }
+  return size_of(t, n_keys, n_vals);
+}
+
+int pskv_size_multi(pskv_table* const* tables, size_t S, uint64_t* n_keys, uint64_t* n_vals) {
+  clear_error();
+  if (S == 0) return PSKV_OK;
+  int rc = check_group(tables, S);
+  if (rc) return rc;
+  DeviceGuard guard(tables[0]->device);
+  for (size_t at = 0; at < S; at += kMaxBatch) {
+    rc = read_states(tables + at, std::min<size_t>(S - at, kMaxBatch), true);
+    if (rc) return rc;
+  }
+  for (size_t s = 0; s < S; ++s) {
+    rc = size_of(tables[s], n_keys ? n_keys + s : nullptr, n_vals ? n_vals + s : nullptr);
+    if (rc) return rc;
   }
   return PSKV_OK;
 }

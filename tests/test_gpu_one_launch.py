@@ -264,3 +264,43 @@ def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
             got = capi.slice_keys(to_dev(keys, dev), begin, end, lens=to_dev(lens, dev), nvals=int(lens.sum()))
             for a, b in zip(got, want):
                 assert np.array_equal(np.asarray(a), np.asarray(b))
+
+
+@pytest.mark.parametrize("mode", ["scalar", "fixed", "varlen"])
+def test_tables_of_a_group_grow_and_are_counted_together(capi, orc, dev, mode):
+    """Eighteen tables of different sizes (two launches' worth) that one request makes grow, by two, four and eight and by
+    more (which fills and scatters), or not at all; their sizes in one call."""
+    announce("group growth", mode)
+    rng = np.random.default_rng(7)
+    S = 18
+    code = {"scalar": capi.MODE_SCALAR, "fixed": capi.MODE_FIXED, "varlen": capi.MODE_VARLEN}[mode]
+    k = 3 if mode == "fixed" else 0
+    tables = []
+    for s in range(S):
+        stream = capi.load().pskv_table_stream(tables[0]._h) if tables else None
+        tables.append(capi.Table(code, initial_capacity=1 << (4 + s), row_len=k, stream=stream))
+    group = object.__new__(capi.Group)
+    group.__dict__.update(tables=tables, S=S, mode=code, _lib=capi.load())
+    import ctypes
+    group._arr = (ctypes.c_void_p * S)(*[t._h for t in tables])
+    group._at = ctypes.addressof(group._arr)
+    stores = [orc.Store(code, k) for _ in range(S)]
+    begin, end = orc.server_ranges(S)
+    for turn, n in enumerate((2_000, 40_000, 60_000, 300_000)):
+        keys = unique_keys(rng, n, S)
+        lens = (keys % np.uint64(7)).astype(np.int32) if mode == "varlen" else None
+        nvals = int(lens.sum()) if mode == "varlen" else n * max(k, 1)
+        vals = rng.standard_normal(nvals).astype(np.float32)
+        pos, val_pos, _ = orc.slice_keys(keys, begin, end, lens, nvals)
+        group.push(to_dev(keys, dev), pos, to_dev(vals, dev), val_pos, lens=None if lens is None else to_dev(lens, dev))
+        for s in range(S):
+            a, b, va, vb = int(pos[s]), int(pos[s + 1]), int(val_pos[s]), int(val_pos[s + 1])
+            stores[s].push(keys[a:b], vals[va:vb], None if lens is None else lens[a:b])
+        sizes = [o.size() for o in stores]
+        assert group.size() == (sum(x for x, _ in sizes), sum(y for _, y in sizes))
+        assert [t.size() for t in tables] == [tuple(x) for x in sizes]
+    for t, o in zip(tables, stores):
+        got, want = t.dump(), o.dump()
+        assert np.array_equal(got[0], want[0])
+        assert_bits_equal(got[2], want[2])
+    group.close()
