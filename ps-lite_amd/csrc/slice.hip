@@ -128,16 +128,33 @@ __device__ __forceinline__ void hand_over(SumsState* state, unsigned S, unsigned
 
 // A request of up to kFewSumsKeys keys: everything that a workgroup needs is asked for at once, eight keys and lens a
 // thread, the lens are added up by one scan, and the key that a boundary falls in front of says where that is and what lies
-// below. (The searches of the kernel below are trips to memory that follow from each other, and every slice is added up for
-// itself. us per call: 5,000 keys over 16 ranges 19.2 -> 13.5, 15,826 over 3 15.1 -> 12.3, 100,000 over 16 17.0 -> 13.7.)
+// below. The workgroups do not meet: each tells the host what its part's lens add up to, which boundaries are its own and,
+// for each of those, where in the part it is and what lies below it there, and the host puts the parts together (a word a
+// part, told of in the order they arrive). (The searches of the kernel below are trips to memory that follow from each other,
+// every slice is added up for itself, and a sum passes through the L2, a ticket and the workgroup that finishes last.
+// us per call: 1,000 keys over 3 ranges 10.6 (12.2 when the workgroups met over a ticket and the last handed everything
+// over), 5,000 over 16 11.9 (13.6; the searches of the kernel below 19.2), 15,826 over 3 11.1 (12.6; 15.1), 262,144 over 4
+// 12.0 (13.6). The searches against this: 400,000 over 8 15.5 and 12.8, 1M over 16 16.9 and 14.9, but with a thousand words
+// for the host to read 2M over 16 17.0 and 17.3: up to 512 parts.)
 constexpr unsigned kFewSumsBlock = 256, kFewSumsItems = 8;  // (larger workgroups find no place on a busy GPU)
 constexpr uint64_t kFewSumsPart = (uint64_t)kFewSumsBlock * kFewSumsItems;
-constexpr uint64_t kFewSumsKeys = 128 * kFewSumsPart;
+constexpr unsigned kFewSumsParts = 512;
+constexpr uint64_t kFewSumsKeys = kFewSumsParts * kFewSumsPart;
+// The words a part tells: lens in the lower kPartLensBits (2,048 of 32 bits, a sign), and above them for the part the first
+// of its boundaries and their number, for a boundary its place in the part.
+constexpr unsigned kPartLensBits = 45, kPartCountAt = kPartLensBits + 6;
+static_assert(kFewSumsPart <= 1u << 11 && kFusedTargets < 64, "a place and two numbers of boundaries fit above the lens");
+__host__ __device__ constexpr unsigned long long part_word(unsigned long long lens, unsigned long long upper) {
+  return (lens & ((1ull << kPartLensBits) - 1)) | upper << kPartLensBits;
+}
+inline uint64_t part_lens(uint64_t word) {
+  return (uint64_t)((int64_t)(word << (64 - kPartLensBits)) >> (64 - kPartLensBits));
+}
 __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_t* __restrict__ keys,
                                                                    const int32_t* __restrict__ lens, uint64_t n,
-                                                                   FusedTargets targets, unsigned S, SumsState* state,
-                                                                   uint64_t* __restrict__ pos_host,
-                                                                   unsigned long long* __restrict__ sums_host) {
+                                                                   FusedTargets targets, unsigned S,
+                                                                   uint64_t* __restrict__ bounds_host,
+                                                                   uint64_t* __restrict__ parts_host) {
   constexpr unsigned kWaves = kFewSumsBlock / 64;
   typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
   typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
@@ -200,21 +217,18 @@ __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_
   __syncthreads();
   if (threadIdx.x >= 64) return;
   const uint64_t before = s_before, end = s_end;
-  unsigned long long under = 0;
+  bool own = false;
   if (lane <= S) {
     const uint64_t target = targets.v[lane];
     const bool after_start = c0 == 0 || before < target, inside = after_start && end >= target;
-    under = inside ? s_below[lane] : after_start ? all : 0ull;
-    // the boundary is this stretch's if it does not lie before it, nor behind it unless it is the last one
-    if (after_start && (c1 == n || inside)) publish_u64(&state->pos[lane], inside ? s_at[lane] : c1);
+    // the boundary is this part's if it does not lie before it, nor behind it unless it is the last one
+    own = after_start && (c1 == n || inside);
+    if (own) tell(&bounds_host[lane], part_word(inside ? s_below[lane] : all, (inside ? s_at[lane] : c1) - c0));
   }
-  const unsigned long long next = __shfl_down(under, 1);
-  if (lane < S && next != under) atomicAdd(&state->sums[lane], next - under);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(0);  // what this lane has handed over is there before the ticket is taken
-  unsigned last = 0;
-  if (lane == 0) last = atomicAdd(&state->ticket, 1u) == gridDim.x - 1 ? 1u : 0u;
-  if (__shfl(last, 0)) hand_over(state, S, lane, pos_host, sums_host);
+  const unsigned long long owned = __ballot(own);  // (the boundaries ascend: these follow each other)
+  if (lane == 0)
+    tell(&parts_host[blockIdx.x],
+         part_word(all, owned ? (unsigned long long)__builtin_ctzll(owned) | (unsigned long long)__popcll(owned) << 6 : 0ull));
 }
 
 __global__ __launch_bounds__(kBlock) void k_bounds_sums(const uint64_t* __restrict__ keys,
@@ -494,6 +508,32 @@ bool all_here(const uint64_t* words, size_t count) {
   return true;
 }
 
+// What the parts of k_bounds_sums_few have told: the positions of the boundaries and the sums of the slices between them.
+// False when a word did not show up, or when keys that are not sorted have left a boundary without an owner, or with
+// two: what comes late may then still be on its way.
+bool join_parts(const uint64_t* parts, const uint64_t* bounds, uint64_t n, size_t S, uint64_t* pos, uint64_t* sums) {
+  uint64_t before = 0, below[kFusedTargets], seen = 0;
+  bool clear = true;
+  for (size_t i = 0; i <= S; ++i) pos[i] = below[i] = 0;
+  for (uint64_t b = 0; b * kFewSumsPart < n; ++b) {
+    clear = all_here(parts + b, 1) && clear;
+    const uint64_t word = parts[b];
+    const unsigned first = (unsigned)(word >> kPartLensBits) & 63u, count = (unsigned)(word >> kPartCountAt) & 63u;
+    for (unsigned i = first; i < first + count; ++i) {
+      clear = all_here(bounds + i, 1) && !(seen >> i & 1u) && clear;
+      seen |= 1ull << i;
+      pos[i] = b * kFewSumsPart + ((bounds[i] & ~kHere) >> kPartLensBits);
+      below[i] = before + part_lens(bounds[i]);
+    }
+    before += part_lens(word);
+  }
+  for (size_t i = 1; i <= S; ++i) {
+    if (pos[i] < pos[i - 1]) pos[i] = pos[i - 1], below[i] = below[i - 1];
+    sums[i - 1] = below[i] - below[i - 1];
+  }
+  return clear && seen == (2ull << S) - 1;
+}
+
 // A call on the context's stream has taken `us` and nothing of it is left: the stream of the next one.
 void note_call(SliceCtx* c, float us) {
   float& mine = c->took[c->at];
@@ -637,9 +677,10 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     SliceCtx* c = lease.c;
     if (!c) return set_error(PSKV_EHIP, "cannot create a slicer context on device %d", device);
     lease.idle = false;
-    // device: lb[S+1] | pos[S+1] | sums[S]      pinned: targets[S+1] | pos[S+1] | sums[S]
+    // device: lb[S+1] | pos[S+1] | sums[S]      pinned: targets[S+1] | pos[S+1] | sums[S] | parts[kFewSumsParts]
     const size_t arr = pad256((S + 1) * 8);
-    int rc = ctx_reserve(c, 3 * arr, 3 * arr);
+    constexpr size_t kParts = kFewSumsParts * 8;
+    int rc = ctx_reserve(c, 3 * arr, 3 * arr + kParts);
     if (rc) return rc;
     char* d = static_cast<char*>(c->dev);
     uint64_t* d_lb = reinterpret_cast<uint64_t*>(d);
@@ -649,6 +690,7 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     uint64_t* h_targets = reinterpret_cast<uint64_t*>(h);
     uint64_t* h_pos = reinterpret_cast<uint64_t*>(h + arr);
     unsigned long long* h_sums = reinterpret_cast<unsigned long long*>(h + 2 * arr);
+    uint64_t* h_parts = reinterpret_cast<uint64_t*>(h + 3 * arr);
     h_targets[0] = range_begin[0];
     for (size_t i = 0; i < S; ++i) h_targets[i + 1] = range_end[i];
     // With few boundaries one kernel leaves everything this call waits for in pinned memory, word by word:
@@ -659,13 +701,16 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     const bool watch = !do_sums || sums_too;
     const auto asked = std::chrono::steady_clock::now();
     std::memset(h_pos, 0, (S + 1) * 8);
-    if (sums_too) std::memset(h_sums, 0, S * 8);
+    const bool in_parts = sums_too && n <= kFewSumsKeys;
+    const uint64_t nparts = in_parts ? (n + kFewSumsPart - 1) / kFewSumsPart : 0;
+    if (in_parts) std::memset(h_parts, 0, nparts * 8);
+    if (sums_too && !in_parts) std::memset(h_sums, 0, S * 8);
     FusedTargets ft = {};
     if (few)
       for (size_t i = 0; i <= S; ++i) ft.v[i] = h_targets[i];
-    if (sums_too && n <= kFewSumsKeys) {
-      k_bounds_sums_few<<<dim3((unsigned)((n + kFewSumsPart - 1) / kFewSumsPart)), dim3(kFewSumsBlock), 0, c->stream>>>(
-          keys, lens, n, ft, (unsigned)S, c->sums_state, h_pos, h_sums);
+    if (in_parts) {
+      k_bounds_sums_few<<<dim3((unsigned)nparts), dim3(kFewSumsBlock), 0, c->stream>>>(keys, lens, n, ft, (unsigned)S, h_pos,
+                                                                                      h_parts);
       PSKV_HIP(hipGetLastError());
     } else if (sums_too) {
       // (a stretch of at least 2,048 keys, a multiple of four)
@@ -692,13 +737,19 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
       k_export_sums<<<dim3((unsigned)((S + 255) / 256)), dim3(256), 0, c->stream>>>(d_sums, S, h_sums);
       PSKV_HIP(hipGetLastError());
     }
-    if (!watch || !all_here(h_pos, S + 1) || (sums_too && !all_here(reinterpret_cast<uint64_t*>(h_sums), S)))
+    if (in_parts) {
+      if (!join_parts(h_parts, h_pos, n, S, pos, val_pos + 1)) {
+        PSKV_HIP(hipStreamSynchronize(c->stream));
+        (void)join_parts(h_parts, h_pos, n, S, pos, val_pos + 1);
+      }
+    } else if (!watch || !all_here(h_pos, S + 1) || (sums_too && !all_here(reinterpret_cast<uint64_t*>(h_sums), S))) {
       PSKV_HIP(hipStreamSynchronize(c->stream));
+    }
     lease.idle = true;  // (what the kernel still does is clear its state for the next one on the stream)
     if (watch)
       note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count());
-    for (size_t i = 0; i <= S; ++i) pos[i] = told(h_pos[i]);
-    if (do_sums)
+    for (size_t i = 0; i <= S && !in_parts; ++i) pos[i] = told(h_pos[i]);
+    if (do_sums && !in_parts)
       for (size_t i = 0; i < S; ++i) val_pos[i + 1] = sums_too ? told(h_sums[i]) : h_sums[i];  // per-slice sums for now
   }
 

@@ -246,9 +246,9 @@ def test_cached_values_written_back_by_the_request_that_differs(capi, orc, dev, 
 
 
 @pytest.mark.parametrize("S", [1, 3, 16, 31])
-@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 30_001, 128 * 2048, 128 * 2048 + 1])
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 30_001, 128 * 2048 + 1, 512 * 2048, 512 * 2048 + 1])
 def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
-    """Boundaries and sums of lens by one scan (up to 262,144 keys): the edges of a workgroup's stretch, boundaries on a key,
+    """Boundaries and sums of lens by one scan (up to 1,048,576 keys): the edges of a workgroup's stretch, boundaries on a key,
     between keys, in front of all and behind all, several in one stretch; called twice, from either kind of memory."""
     announce("few slices", n, S)
     rng = np.random.default_rng(n * 31 + S)
@@ -264,6 +264,35 @@ def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
             got = capi.slice_keys(to_dev(keys, dev), begin, end, lens=to_dev(lens, dev), nvals=int(lens.sum()))
             for a, b in zip(got, want):
                 assert np.array_equal(np.asarray(a), np.asarray(b))
+
+
+@pytest.mark.parametrize("n", [2049, 70_000])
+def test_slices_with_lens_of_any_size_and_order(capi, orc, dev, n):
+    """Ranges without keys that end where they begin, lens whose sums need all the bits of a part's word and negative ones;
+    and keys that are not sorted, which give no slices worth having but an answer, and leave the next call alone."""
+    announce("few slices, lens of any size", n)
+    rng = np.random.default_rng(n)
+    keys = unique_keys(rng, n, 4)
+    cut = [0, int(keys[n // 3]), int(keys[n // 3]), int(keys[2 * n // 3]) + 1, 2**64 - 1]
+    begin, end = np.array(cut[:-1], np.uint64), np.array(cut[1:], np.uint64)
+    for lens in (np.full(n, 2**31 - 1, np.int32), rng.integers(-2**31, 2**31, n).astype(np.int32) | 1):
+        nvals = max(0, int(lens.astype(np.int64).sum()))
+        for shuffled in (False, True):
+            k = rng.permutation(keys) if shuffled else keys
+            results = []
+            for who, arrays in ((capi, (to_dev(k, dev), to_dev(lens, dev))), (orc, (k, lens))):
+                try:
+                    if who is capi:
+                        results.append(capi.slice_keys(arrays[0], begin, end, lens=arrays[1], nvals=nvals))
+                    else:
+                        results.append(orc.slice_keys(arrays[0], begin, end, arrays[1], nvals))
+                except Exception as e:
+                    results.append(type(e).__name__)
+            if not shuffled and not isinstance(results[0], str):
+                for a, b in zip(*results):
+                    assert np.array_equal(np.asarray(a), np.asarray(b))
+            elif not shuffled:
+                assert isinstance(results[1], str), results
 
 
 @pytest.mark.parametrize("mode", ["scalar", "fixed", "varlen"])
