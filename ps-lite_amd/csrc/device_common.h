@@ -320,33 +320,6 @@ __device__ __forceinline__ unsigned long long wave_incl_scan_u64(unsigned long l
   return x;
 }
 
-// A 64-ary lower_bound by one wavefront. Each round the 64 lanes probe evenly spaced keys of
-// the remaining interval, a ballot counts how many are below the target (the probes are
-// sorted, so the votes are a prefix of ones) and the interval shrinks 64-fold:
-// ceil(log64 n) dependent loads instead of ceil(log2 n). Every lane returns the answer.
-__device__ __forceinline__ uint64_t wave_lower_bound(const uint64_t* __restrict__ keys, uint64_t n,
-                                                     uint64_t target, unsigned lane) {
-  uint64_t lo = 0, hi = n;  // the answer lies in [lo, hi]; keys[lo..hi) are undecided
-  while (hi > lo) {
-    const uint64_t len = hi - lo;
-    if (len <= 64) {
-      const bool below = lane < len && keys[lo + lane] < target;
-      lo += __popcll(__ballot(below));
-      break;
-    }
-    const uint64_t step = (len + 63) / 64;
-    const uint64_t idx = lo + (uint64_t)(lane + 1) * step - 1;
-    const bool below = idx < hi && keys[idx] < target;
-    const uint64_t c = __popcll(__ballot(below));
-    // probes 0..c-1 are below the target, probe c (if any) is not
-    const uint64_t new_lo = lo + c * step;
-    const uint64_t cap = lo + (c + 1) * step - 1;
-    hi = cap < hi ? cap : hi;
-    lo = new_lo < hi ? new_lo : hi;
-  }
-  return lo;
-}
-
 // Writes the table's counters to `out` (pinned host memory). Called by all 64 lanes of one
 // wavefront, at a point of the stream where no kernel is changing the counters.
 __device__ __forceinline__ void publish_snapshot(const DevState* st, Snapshot* out, uint64_t seq) {

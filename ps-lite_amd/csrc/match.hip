@@ -17,6 +17,7 @@
 
 #include "device_common.h"
 #include "host_common.h"
+#include "search.h"
 
 namespace pskv {
 namespace {
