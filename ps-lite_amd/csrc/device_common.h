@@ -4,6 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+// Asks for all of a kernel's arguments at once (the compiler otherwise fetches them group by group where they are first
+// used, one wait each).
+#define PSKV_ASK_ARGS(...) asm volatile("" ::__VA_ARGS__)
+
 namespace pskv {
 
 // ps::kMaxKey (include/ps/base.h:18). The stock server ranges never cover it

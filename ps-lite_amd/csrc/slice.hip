@@ -69,8 +69,8 @@ __global__ void k_bounds_chain(const uint64_t* __restrict__ lb, uint64_t S,
   }
 }
 
-// Both of the above in one launch when the boundaries are few (the stock case: one per server):
-// one workgroup of up to 16 wavefronts, each searching one or two boundaries, then the chain.
+// Both of the above in one launch when the boundaries are few and the positions are for a kernel behind it: one
+// workgroup of up to 16 wavefronts, each searching one or two boundaries, then the chain.
 // The boundaries travel with the launch: no read across the host link before the search.
 constexpr unsigned kFusedWaves = 16;
 constexpr unsigned kFusedTargets = 2 * kFusedWaves;
@@ -78,18 +78,24 @@ struct FusedTargets {
   uint64_t v[kFusedTargets];
 };
 __global__ __launch_bounds__(kFusedWaves * 64) void k_bounds_fused(
-    const uint64_t* __restrict__ keys, uint64_t n, FusedTargets targets, uint64_t S,
-    uint64_t* __restrict__ pos, uint64_t* __restrict__ pos_host, unsigned long long* __restrict__ sums) {
+    const uint64_t* __restrict__ keys, uint64_t n, uint64_t* __restrict__ pos, uint64_t* __restrict__ pos_host,
+    unsigned long long* __restrict__ sums, unsigned S, unsigned waves, FusedTargets targets) {
   __shared__ uint64_t s_lb[kFusedTargets];
-  const unsigned lane = threadIdx.x & 63, waves = blockDim.x >> 6;
-  for (unsigned w = threadIdx.x >> 6; w <= S; w += waves) {  // whole wavefronts
-    const uint64_t lo = wave_lower_bound(keys, n, targets.v[w], lane);
+  const unsigned lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  static_assert(kFusedTargets == 2 * kFusedWaves, "two boundaries for a wavefront at most");
+  const unsigned second = wave + waves < kFusedTargets ? wave + waves : 0u;
+  const uint64_t target[2] = {targets.v[wave], targets.v[second]};
+  PSKV_ASK_ARGS("s"(keys), "s"(n), "s"(pos), "s"(pos_host), "s"(sums), "s"(S), "s"(target[0]), "s"(target[1]));
+#pragma unroll
+  for (unsigned q = 0; q < 2; ++q) {
+    const unsigned w = wave + q * waves;
+    if (w > S) continue;
+    const uint64_t lo = wave_lower_bound(keys, n, target[q], lane);
     if (lane == 0) s_lb[w] = lo;
   }
   __syncthreads();
-  if (sums)
-    for (uint64_t i = threadIdx.x; i < S; i += blockDim.x) sums[i] = 0ull;
   if (threadIdx.x >= 64) return;
+  if (sums && lane < S) sums[lane] = 0ull;
   static_assert(kFusedTargets <= 64, "a lane per position");
   uint64_t p = 0;  // (the reads of LDS do not wait for each other, the steps of a scan over the lanes would)
   for (unsigned i = 0; i <= S; ++i) p = i <= lane && s_lb[i] > p ? s_lb[i] : p;
@@ -97,6 +103,19 @@ __global__ __launch_bounds__(kFusedWaves * 64) void k_bounds_fused(
     pos[lane] = p;
     if (pos_host) tell(&pos_host[lane], p);
   }
+}
+
+// The searches of a request without lens, or whose lens nobody adds up here: a wavefront and compute unit for each boundary,
+// which tells the host what it has found; the host takes the larger of each and the one before. (A round of a search is 64
+// lines, and one compute unit asks for a line a clock: 17 searches in one workgroup took 2 us longer than two. us per call,
+// one workgroup -> this: 1,000 keys over 4 ranges 9.6 -> 8.4, 20,000 over 1 9.5 -> 8.7, over 16 11.6 -> 9.2, 1M over 4 9.9 ->
+// 9.0, 16M over 16 11.8 -> 9.4. More probes a round, to save rounds: slower, a round that follows is 0.3 us.)
+__global__ __launch_bounds__(64) void k_bounds_tell(const uint64_t* __restrict__ keys, uint64_t n,
+                                                   uint64_t* __restrict__ lb_host, FusedTargets targets) {
+  const uint64_t target = targets.v[blockIdx.x];
+  PSKV_ASK_ARGS("s"(keys), "s"(n), "s"(lb_host), "s"(target));
+  const uint64_t lo = wave_lower_bound(keys, n, target, threadIdx.x);
+  if (threadIdx.x == 0) tell(&lb_host[blockIdx.x], lo);
 }
 
 // Boundaries and the lens sums of the slices between them in one launch (few boundaries, in ascending
@@ -153,14 +172,15 @@ inline uint64_t part_lens(uint64_t word) {
 }
 __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_t* __restrict__ keys,
                                                                    const int32_t* __restrict__ lens, uint64_t n,
-                                                                   FusedTargets targets, unsigned S,
                                                                    uint64_t* __restrict__ bounds_host,
-                                                                   uint64_t* __restrict__ parts_host) {
+                                                                   uint64_t* __restrict__ parts_host, unsigned S,
+                                                                   FusedTargets targets) {
+  PSKV_ASK_ARGS("s"(keys), "s"(lens), "s"(n), "s"(bounds_host), "s"(parts_host), "s"(S));
   constexpr unsigned kWaves = kFewSumsBlock / 64;
   typedef int32_t i32x4u __attribute__((ext_vector_type(4), aligned(4)));
   typedef unsigned long long u64x2u __attribute__((ext_vector_type(2), aligned(8)));
   __shared__ unsigned long long s_wave[kWaves];
-  __shared__ uint64_t s_at[kFusedTargets];
+  __shared__ uint64_t s_at[kFusedTargets], s_target[kFusedTargets];
   __shared__ unsigned long long s_below[kFusedTargets];
   __shared__ uint64_t s_before, s_end;
   const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -187,6 +207,7 @@ __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_
     }
   }
   if (mine && i0) prev = keys[i0 - 1];
+  if (threadIdx.x < kFusedTargets) s_target[threadIdx.x] = targets.v[threadIdx.x];
   if (threadIdx.x == 0) s_before = prev;
   uint64_t top = key[0];  // the thread's last key
 #pragma unroll
@@ -204,8 +225,10 @@ __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_
     if (w < wave) below += s_wave[w];
     all += s_wave[w];
   }
+  uint64_t near = s_target[0];
   for (unsigned i = 0; i <= S; ++i) {  // (few threads hold a boundary, most boundaries lie elsewhere)
-    const uint64_t target = targets.v[i];
+    const uint64_t target = near;
+    near = s_target[i < S ? i + 1 : S];  // (the next one is on its way)
     if (!mine || top < target || (i0 && prev >= target)) continue;
     unsigned long long x = below;
     uint64_t at = i0;
@@ -220,7 +243,7 @@ __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_
   const uint64_t before = s_before, end = s_end;
   bool own = false;
   if (lane <= S) {
-    const uint64_t target = targets.v[lane];
+    const uint64_t target = s_target[lane];
     const bool after_start = c0 == 0 || before < target, inside = after_start && end >= target;
     // the boundary is this part's if it does not lie before it, nor behind it unless it is the last one
     own = after_start && (c1 == n || inside);
@@ -710,8 +733,8 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     if (few)
       for (size_t i = 0; i <= S; ++i) ft.v[i] = h_targets[i];
     if (in_parts) {
-      k_bounds_sums_few<<<dim3((unsigned)nparts), dim3(kFewSumsBlock), 0, c->stream>>>(keys, lens, n, ft, (unsigned)S, h_pos,
-                                                                                      h_parts);
+      k_bounds_sums_few<<<dim3((unsigned)nparts), dim3(kFewSumsBlock), 0, c->stream>>>(keys, lens, n, h_pos, h_parts,
+                                                                                      (unsigned)S, ft);
       PSKV_HIP(hipGetLastError());
     } else if (sums_too) {
       // (a stretch of at least 2,048 keys, a multiple of four)
@@ -719,10 +742,12 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
       k_bounds_sums<<<dim3((unsigned)((n + chunk - 1) / chunk)), dim3(kBlock), 0, c->stream>>>(
           keys, lens, n, chunk, ft, (unsigned)S, c->sums_state, h_pos, h_sums);
       PSKV_HIP(hipGetLastError());
+    } else if (few && !do_sums) {
+      k_bounds_tell<<<dim3((unsigned)(S + 1)), dim3(64), 0, c->stream>>>(keys, n, h_pos, ft);
+      PSKV_HIP(hipGetLastError());
     } else if (few) {  // one launch for the boundaries
       const unsigned waves = (unsigned)std::min<size_t>(S + 1, kFusedWaves);
-      k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, c->stream>>>(keys, n, ft, S, d_pos, h_pos,
-                                                                 do_sums ? d_sums : nullptr);
+      k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, c->stream>>>(keys, n, d_pos, h_pos, d_sums, (unsigned)S, waves, ft);
       PSKV_HIP(hipGetLastError());
     } else {
       rc = launch_bounds_search(keys, n, h_targets, S + 1, d_lb, c->stream);
@@ -749,7 +774,7 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     lease.idle = true;  // (what the kernel still does is clear its state for the next one on the stream)
     if (watch)
       note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count());
-    for (size_t i = 0; i <= S && !in_parts; ++i) pos[i] = told(h_pos[i]);
+    for (size_t i = 0; i <= S && !in_parts; ++i) pos[i] = std::max(told(h_pos[i]), i ? pos[i - 1] : 0);
     if (do_sums && !in_parts)
       for (size_t i = 0; i < S; ++i) val_pos[i + 1] = sums_too ? told(h_sums[i]) : h_sums[i];  // per-slice sums for now
   }
@@ -852,7 +877,7 @@ int pskv_slice_noalloc(int device, void* stream, const uint64_t* keys, size_t n,
     ft.v[0] = range_begin[0];
     for (size_t i = 0; i < S; ++i) ft.v[i + 1] = range_end[i];
     const unsigned waves = (unsigned)std::min<size_t>(S + 1, kFusedWaves);
-    k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, st>>>(keys, n, ft, S, pos, (uint64_t*)nullptr, d_sums);
+    k_bounds_fused<<<dim3(1), dim3(waves * 64), 0, st>>>(keys, n, pos, (uint64_t*)nullptr, d_sums, (unsigned)S, waves, ft);
     PSKV_HIP(hipGetLastError());
   } else {
     for (size_t first = 0; first <= S; first += kFusedTargets) {

@@ -95,8 +95,6 @@ template <typename T>
 __device__ __forceinline__ void arrived(T& x) {
   asm volatile("" : "+v"(x));
 }
-// (kernel arguments: scalar registers)
-#define PSKV_ASK_ARGS(...) asm volatile("" ::__VA_ARGS__)
 
 // ---------------------------------------------------------------------------------
 // SCALAR mode: one float per key, kept in the low word of the slot payload so that a

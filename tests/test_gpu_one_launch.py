@@ -266,6 +266,23 @@ def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
                 assert np.array_equal(np.asarray(a), np.asarray(b))
 
 
+@pytest.mark.parametrize("S", [1, 16, 31, 32])
+@pytest.mark.parametrize("n", [1, 64, 65, 4096, 4097, 300_000])
+def test_slices_without_lens(capi, orc, dev, n, S):
+    """A wavefront for each boundary, up to 32 of them: where its search takes a round more, keys on the boundaries and beside
+    them, and no key in most of the ranges."""
+    announce("slices without lens", n, S)
+    rng = np.random.default_rng(n * 37 + S)
+    begin, end = orc.server_ranges(S)
+    near = np.concatenate([np.arange(-3, 4).astype(np.int64).astype(np.uint64) + e for e in end[:-1]] or [end[:0]])
+    for keys in (unique_keys(rng, n, S), np.arange(n, dtype=np.uint64) + begin[S // 2],
+                 np.unique(np.concatenate([near, unique_keys(rng, n, S)]))):
+        want = orc.slice_keys(keys, begin, end, None, 3 * keys.size)
+        for _ in range(2):
+            for a, b in zip(capi.slice_keys(to_dev(keys, dev), begin, end, nvals=3 * keys.size), want):
+                assert np.array_equal(np.asarray(a), np.asarray(b))
+
+
 @pytest.mark.parametrize("n", [2049, 70_000])
 def test_slices_with_lens_of_any_size_and_order(capi, orc, dev, n):
     """Ranges without keys that end where they begin, lens whose sums need all the bits of a part's word and negative ones;
