@@ -112,7 +112,9 @@ struct alignas(32) DevState {
   unsigned int ticket_sub[kTicketShards * 32];
   // one_launch.h: pushes served so far << 2 | the verdict on the newest one; everyone watches it, so the line is its own
   unsigned long long push_verdict;
-  unsigned long long pad[15];
+  // k_fixed_long: the newest of its requests that has created a row, and how many rows there were before it
+  unsigned long long fresh_from;
+  unsigned long long pad[14];
   // one_launch.h: what the workgroups of a var-len request tell each other, all zero between requests
   unsigned long long parts[kVarParts];
 };
@@ -201,23 +203,35 @@ __device__ __forceinline__ void raise_error(DevState* st, unsigned bit, unsigned
 // Two levels of counters, the first spread over kTicketShards cache lines, because atomics
 // on one address are served one at a time (about 15 ns each).
 // The counters are left at zero; kernels that use it must not overlap on one table.
-__device__ __forceinline__ bool ticket_last(DevState* st, unsigned nblk) {
-  // this thread's atomics and atomic stores are complete before its ticket is taken
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(0);
-  unsigned shards = nblk;  // a small grid goes straight to the second level
+// In two halves, for a thread that has something to ask for in between: what it has to see to is that its atomics and
+// atomic stores are complete before it takes the ticket.
+__device__ __forceinline__ unsigned ticket_take(DevState* st, unsigned nblk) {
+  // (a small grid goes straight to the second level)
+  return atomicAdd(nblk > (unsigned)kTicketShards ? &st->ticket_sub[blockIdx.x % kTicketShards * 32] : &st->ticket_top, 1u);
+}
+__device__ __forceinline__ bool ticket_is_last(DevState* st, unsigned nblk, unsigned ticket) {
+  unsigned shards = nblk;
   if (nblk > (unsigned)kTicketShards) {
     shards = (unsigned)kTicketShards;
     const unsigned sub = blockIdx.x % shards;
     const unsigned members = (nblk - sub + shards - 1) / shards;  // workgroups b with b % shards == sub
-    unsigned* c = &st->ticket_sub[sub * 32];
-    if (atomicAdd(c, 1u) != members - 1) return false;
-    *c = 0;
+    if (ticket != members - 1) return false;
+    st->ticket_sub[sub * 32] = 0;
+    ticket = atomicAdd(&st->ticket_top, 1u);
   }
-  if (atomicAdd(&st->ticket_top, 1u) != shards - 1) return false;
+  if (ticket != shards - 1) return false;
   st->ticket_top = 0;
-  __threadfence();  // acquire, once per grid: nothing stale is left in this XCD's L2
+  // once per grid: nothing stale is left in this XCD's L2 (__threadfence would also write back what others have left there)
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   return true;
+}
+__device__ __forceinline__ void my_atomics_are_there() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0);
+}
+__device__ __forceinline__ bool ticket_last(DevState* st, unsigned nblk) {
+  my_atomics_are_there();
+  return ticket_is_last(st, nblk, ticket_take(st, nblk));
 }
 
 // Adds a workgroup's facts (one thread calls it, before its ticket) to those of the other workgroups of a launch of

@@ -17,9 +17,10 @@ namespace pskv {
 // to be on the GPU together for that: kOwnPushGroups of them are a third of what it holds. Who does not see the verdict
 // in time all the same (d.cache_mode looks: something else may keep a part of the workgroups off the GPU) reads all
 // keys of the request itself, so nobody depends on the others but for time.
-// Measured (us per step of three pulls and two pushes, three tables in turn; lookup and rows as two launches -> one):
-// 9,639 rows of 7 floats 37.2 -> 23.2, 59,871 of 16 36.4 -> 26.2, 30,000 of 64 43.3 -> 33.4; pulls alone as one launch:
-// 193,521 rows of 30 126 -> 120, 1M of 64 663 -> 645.
+// Measured (us per two steps of pull and push and a pull, lookup and rows as two launches -> one): 49,881 rows of 15 floats
+// one table 49-53 -> 40, three in turn 28-39 -> 20.4; 30,000 of 64 53-59 -> 41, 37-45 -> 30.6; 1M of 64, whose pushes are two
+// launches, 668 -> 633, 643 -> 633. Of that the loads of a lane's rows side by side, the ticket in front of them and its
+// fence without a write-back are 45.6 -> 40, 24 -> 20.4 and 48.8 -> 41, 33.2 -> 30.6.
 constexpr unsigned kOwnTurns = 4;
 constexpr unsigned kOwnQuads = kBlock * kOwnTurns;
 constexpr uint64_t kOwnPushGroups = 512;
@@ -68,21 +69,26 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
   }
   // the values of the workgroup's quads, which lie one behind the other in the request
   const unsigned all = mine * quads;
+  // (a lane behind the end takes the last one and does not store it: a load under a condition is waited for before the next
+  // is asked for)
   f32x4 x[kOwnTurns];
   unsigned row[kOwnTurns], col[kOwnTurns], count[kOwnTurns];
 #pragma unroll
   for (unsigned q = 0; q < kOwnTurns; ++q) {
-    const unsigned quad = q * kBlock + threadIdx.x;
-    row[q] = quad / quads;
-    const unsigned c = quad - row[q] * quads;
+    const unsigned quad = q * kBlock + threadIdx.x, there = quad < all ? quad : all - 1;
+    row[q] = there / quads;
+    const unsigned c = there - row[q] * quads;
     col[q] = c * 4;
     count[q] = quad >= all ? 0u : rest && c + 1 == quads ? rest : 4u;
     x[q] = (f32x4)(0.f);
-    if (PUSH && count[q]) {
-      const float* side = d.vals + (first + row[q]) * k + col[q];
-      // (a shorter quad is read whole where the next row follows it)
-      x[q] = count[q] == 4 || first + row[q] + 1 < n ? load_quad<STREAM>(side) : load_part<STREAM>(side, count[q]);
-    }
+  }
+  if (PUSH && (!rest || first + mine < n)) {  // a shorter quad is read whole where the next row follows it
+#pragma unroll
+    for (unsigned q = 0; q < kOwnTurns; ++q) x[q] = load_quad<STREAM>(d.vals + (first + row[q]) * k + col[q]);
+  } else if (PUSH) {
+#pragma unroll
+    for (unsigned q = 0; q < kOwnTurns; ++q)
+      if (count[q]) x[q] = load_part<STREAM>(d.vals + (first + row[q]) * k + col[q], count[q]);
   }
   uint64_t* p = nullptr;
   uint64_t seen = 0;
@@ -119,31 +125,40 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
       *p = s_first + at;
       r = (s_first + at) | kRefNew;
     }
+    if (threadIdx.x == 0) my_atomics_are_there();
   }
   if (live) {
     s_ref[threadIdx.x] = r;
     if (r != was) d.ref[i] = r;
   }
   __syncthreads();
+  // The ticket goes out in front of the loads of the rows: behind them it would wait for them.
+  unsigned ticket = 0;
+  if ((PUSH || d.snap) && threadIdx.x == 0) {
+    if (PUSH && any_repeated) {
+      report_facts(st, kReqDuplicate, nblk);
+      my_atomics_are_there();
+    }
+    asm volatile("" : "+v"(before) : : "memory");  // (the old verdict has to be here before the ticket goes out)
+    ticket = ticket_take(st, nblk);
+  }
   // the rows
   f32x4 y[kOwnTurns];
   uint64_t ref[kOwnTurns];
 #pragma unroll
   for (unsigned q = 0; q < kOwnTurns; ++q) {
     ref[q] = count[q] ? s_ref[row[q]] : kRefAbsent;
-    y[q] = (f32x4)(0.f);
-    // (a key that was refused has no row; a created row is zero)
-    if (ref[q] != kRefAbsent && !(ref[q] & kRefNew)) y[q] = load_quad<STREAM>(d.arena + ref[q] * k + col[q]);
+    // (a key that was refused has no row, a created row is zero: read is the table's first one then)
+    y[q] = load_quad<STREAM>(d.arena + (ref[q] & kRefNew ? 0 : ref[q]) * k + col[q]);
   }
+#pragma unroll
+  for (unsigned q = 0; q < kOwnTurns; ++q)
+    if (ref[q] & kRefNew) y[q] = (f32x4)(0.f);
   // (before anything is stored: the counter record goes past the caches and would wait for the rows)
   unsigned verdict = 2;  // not known yet
   if ((PUSH || d.snap) && threadIdx.x < 64) {
     unsigned last = 0;
-    if (threadIdx.x == 0) {
-      if (PUSH && any_repeated) report_facts(st, kReqDuplicate, nblk);
-      asm volatile("" : "+v"(before) : : "memory");  // (the old verdict has to be here before the ticket goes out)
-      last = ticket_last(st, nblk) ? 1u : 0u;
-    }
+    if (threadIdx.x == 0) last = ticket_is_last(st, nblk, ticket) ? 1u : 0u;
     if (__shfl(last, 0)) {
       if (PUSH) {
         verdict = take_facts(st, nblk) & kReqDuplicate ? 1u : 0u;
@@ -180,6 +195,147 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
     if (fresh || (PUSH && !rejected)) store_part<STREAM>(y[q], d.arena + (ref[q] & ~kRefNew) * k + col[q], count[q]);
     if (PULL) store_part<STREAM>(y[q], d.out + (first + row[q]) * k + col[q], count[q]);
   }
+}
+
+// FIXED rows of more than kOwnQuads quads: a workgroup moves an even part of one row, up to kOwnQuads quads, and every
+// workgroup of a row looks up the row's key, so nobody waits for the others' lookups. Whoever claims the slot of a new key
+// gives it its row; the others find the key and wait for its payload, which follows from nothing but the claim. That the
+// row is new they can see from DevState::fresh_from: before the first creator of a request counts the rows up it notes
+// there, under the number of the request, how many there were, so every row from there on is new to this request. (Number
+// and rows are one word: 2^26 rows of 4,100 floats are four times what the GPU holds, 2^38 requests years.)
+// Whether a request repeats a key every workgroup sees for itself: there are at most as many keys as threads.
+// Bound by the chain from a key to its slot, from there to the row, and back. Up to kLongFloats floats that is better than
+// the two launches of lookup and rows (us per push + pull, one table; three in turn, of which the launches are most:
+// 5,000 floats 19.6 -> 18.7; 12.7-15 -> 8.1-9.5, 43 rows of 36,505 27 -> 22; 12.4-15.9 -> 9.3, 200 of 10,000 28 -> 23;
+// 12.4-15.5 -> 11.1, and per four pushes + pull 40 of 100,000 92 -> 71; 71 -> 61). Beyond it other requests' rows fill the
+// gap in front of theirs, and workgroups that ask for less before their rows stream faster (three pushes + pull of 8 rows
+// of 960,704 100 -> 82; 73 -> 81). Quads a lane: 4, with 2 30 rows of 262,144 38 -> 41, with 1 47; past the caches 42.
+constexpr uint64_t kLongFloats = 1u << 22;
+constexpr uint64_t kLongKeys = kBlock;
+constexpr unsigned kFreshBits = 26;
+constexpr unsigned kLongLooks = 1u << 16;  // (nobody gets that far: a claimed slot has its row some 2 us later)
+__host__ __device__ constexpr unsigned long_groups(uint64_t k) { return (unsigned)(((k + 3) / 4 + kOwnQuads - 1) / kOwnQuads); }
+
+// The row of `key`, with kRefNew if this call has created it. One thread.
+__device__ __forceinline__ uint64_t find_or_make_row(const TableReq& d, uint64_t key) {
+  DevState* st = d.st;
+  bool is_new;
+  uint64_t seen;
+  uint64_t* p = find_or_insert(d.slots, d.mask, st, key, is_new, seen);
+  if (!p) return kRefAbsent;
+  if (!is_new) {
+    for (unsigned looks = kLongLooks; seen == kPayloadUnset && looks; --looks)
+      seen = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (seen != kPayloadUnset) return seen;
+    refuse_fixed(st, d.tag);
+    return kRefAbsent;
+  }
+  const unsigned long long word = __hip_atomic_load(&st->fresh_from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (word >> kFreshBits != d.tag.epoch) {
+    // (as long as the word can be exchanged, nobody has counted up)
+    const unsigned long long rows = __hip_atomic_load(&st->arena_top, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long was = atomicCAS(&st->fresh_from, word, (unsigned long long)d.tag.epoch << kFreshBits | rows);
+    asm volatile("" : "+v"(was) : : "memory");  // (it is there before the count changes)
+  }
+  const unsigned long long row = atomicAdd(&st->arena_top, 1ull);
+  atomicAdd(&st->count_shard[(blockIdx.x % kCountShards) * kShardStride], 1ull);
+  __hip_atomic_store(p, row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  my_atomics_are_there();
+  return row | kRefNew;
+}
+
+template <bool PUSH, bool PULL, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_fixed_long(ReqBatch<TABLES> b) {
+  const TableReq& d = b.t[blockIdx.y];
+  PSKV_ASK_ARGS("s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.n), "s"(d.ref), "s"(d.cache_keys), "s"(d.vals),
+                "s"(d.out), "s"(d.arena), "s"(d.k), "s"(d.snap), "s"(d.tag.epoch), "s"(d.nblk));
+  const unsigned nblk = d.nblk;
+  if (blockIdx.x >= nblk) return;
+  DevState* st = d.st;
+  const uint64_t k = d.k;
+  const unsigned n = (unsigned)d.n;
+  __shared__ uint64_t s_ref;
+  const unsigned quads = (unsigned)((k + 3) >> 2), rest = (unsigned)k & 3u;
+  const unsigned per = long_groups(k), i = blockIdx.x / per, part = blockIdx.x - i * per;
+  const uint64_t key = d.keys[i], left = d.keys[i ? i - 1 : 0];
+  // whole quads, four a lane, and the rest of the row, which is one lane's (a case of its own: with the rest as a case of
+  // every quad the code was half as long again, and a small request reads all of it for the first time)
+  const unsigned wholes = quads - (rest ? 1u : 0u), share = (quads + per - 1) / per, c0 = part * share + threadIdx.x;
+  const unsigned end = (part + 1) * share < wholes ? (part + 1) * share : wholes;
+  const bool tail = rest && part + 1 == per && threadIdx.x == kBlock - 1;
+  // (a lane behind the end moves the last whole quad, and does not store it: a load under a condition is waited for)
+  unsigned at[kOwnTurns];
+#pragma unroll
+  for (unsigned q = 0; q < kOwnTurns; ++q) at[q] = (c0 + q * kBlock < end ? c0 + q * kBlock : end - 1) * 4;
+  const float* side = d.vals + i * k;
+  f32x4 x[kOwnTurns], x_tail = (f32x4)(0.f);
+  if (PUSH) {
+#pragma unroll
+    for (unsigned q = 0; q < kOwnTurns; ++q) x[q] = load_quad<false>(side + at[q]);
+    if (tail) x_tail = load_part<false>(side + wholes * 4, rest);
+  }
+  bool repeated = false, twice = false, unsorted = false;
+  uint64_t r = kRefAbsent;
+  if (threadIdx.x == 0) {
+    if (blockIdx.x == 0) st->cache_epoch = d.tag.epoch;
+    repeated = i > 0 && left == key;
+    if (!repeated) r = find_or_make_row(d, key);
+    s_ref = r;
+  }
+  if (threadIdx.x && threadIdx.x < n) {
+    const uint64_t a = d.keys[threadIdx.x - 1], c = d.keys[threadIdx.x];
+    twice = a == c;
+    unsorted = a > c;
+  }
+  bool rejected = __syncthreads_or(twice ? 1 : 0) != 0;  // (s_ref is there)
+  bool again = false;
+  if (__syncthreads_or(unsorted ? 1 : 0)) {  // (then a key may be anywhere again)
+    const unsigned j = threadIdx.x;
+    again = j < n && j != i && d.keys[j] == key;
+    for (unsigned l = 0; PUSH && j < n && l < j; ++l) twice |= d.keys[l] == d.keys[j];
+    again = __syncthreads_or(again ? 1 : 0) != 0;
+    rejected = __syncthreads_or(twice ? 1 : 0) != 0;
+  }
+  unsigned ticket = 0;  // (in front of the loads of the row, see k_fixed_own)
+  if (d.snap && threadIdx.x == 0) ticket = ticket_take(st, nblk);
+  r = s_ref;
+  const uint64_t row = r & ~kRefNew;
+  float* const base = d.arena + (r != kRefAbsent ? row : 0) * k;  // (a refused key reads the table's first row)
+  f32x4 y[kOwnTurns], y_tail = (f32x4)(0.f);
+#pragma unroll
+  for (unsigned q = 0; q < kOwnTurns; ++q) y[q] = load_quad<false>(base + at[q]);
+  if (tail) y_tail = load_part<false>(base + wholes * 4, rest);
+  // (behind the row's number, which its creator leaves behind this word; the row is on its way meanwhile)
+  const unsigned long long word = __hip_atomic_load(&st->fresh_from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool fresh = r != kRefAbsent && word >> kFreshBits == d.tag.epoch && row >= (word & ((1ull << kFreshBits) - 1));
+  if (threadIdx.x == 0 && part == 0) {
+    // (a pull is served from the rows that are there however often a key comes; none is created twice)
+    if (repeated || (PUSH ? rejected && again : fresh && again)) refuse_fixed(st, d.tag);
+    d.cache_keys[i] = key;
+    d.ref[i] = fresh ? row | kRefNew : r;
+  }
+  if (d.snap && threadIdx.x < 64) {
+    unsigned last = 0;
+    if (threadIdx.x == 0) last = ticket_is_last(st, nblk, ticket) ? 1u : 0u;
+    if (__shfl(last, 0)) publish_snapshot(st, d.snap, d.snap_seq);
+  }
+  if (r == kRefAbsent) return;
+  // a refused push changes no stored value; rows it created stay, as zero rows
+  const bool add = PUSH && !rejected, keep = fresh || add;
+  float* const out = PULL ? d.out + i * k : nullptr;
+#pragma unroll
+  for (unsigned q = 0; q < kOwnTurns; ++q) {
+    if (c0 + q * kBlock >= end) continue;
+    if (fresh) y[q] = (f32x4)(0.f);
+    if (add) y[q] = y[q] + x[q];  // a created row is a zero row first (0.0f + v), kv_app.h:454
+    if (keep) store_quad<false>(y[q], base + at[q]);
+    if (PULL) store_quad<false>(y[q], out + at[q]);
+  }
+  if (!tail) return;
+  if (fresh) y_tail = (f32x4)(0.f);
+  if (add) y_tail = y_tail + x_tail;
+  if (keep) store_part<false>(y_tail, base + wholes * 4, rest);
+  if (PULL) store_part<false>(y_tail, out + wholes * 4, rest);
 }
 
 // VARLEN requests of up to kVarParts workgroups: what the first two kernels of a push, or of a pull, do, in one. A

@@ -1428,6 +1428,18 @@ bool fixed_in_one(const Batch& bt, bool push) {
   return push ? groups <= kOwnPushGroups : floats <= kOwnRaggedFloats;
 }
 
+// The same of longer rows (k_fixed_long, which says why the lines lie there).
+bool fixed_long(const Batch& bt) {
+  if (bt[0].r.replay || bt[0].r.pipe_in || bt[0].r.pipe_out) return false;
+  uint64_t floats = 0;
+  for (const Item& it : bt) {
+    if (!it.r.n) continue;
+    if ((it.d.k + 3) / 4 <= kOwnQuads || it.r.n > kLongKeys || it.d.k > kLongFloats) return false;
+    floats += it.r.n * it.d.k;
+  }
+  return floats <= kLongFloats;
+}
+
 int run_fixed(Batch& bt, bool push, bool pull) {
   Growths growths;
   uint64_t n_largest = 0;
@@ -1466,7 +1478,7 @@ int run_fixed(Batch& bt, bool push, bool pull) {
   if (rc) return rc;
   rc = begin_row_request(bt, bt[0].r.replay == kReplayCapture);
   if (rc) return rc;
-  const bool one = fixed_in_one(bt, push);
+  const bool lengthy = fixed_long(bt), one = lengthy || fixed_in_one(bt, push);
   if (one) {
     uint64_t floats = 0;
     bool apart = true;  // (rows that share no line with their neighbours; the others go through the caches, see k_rows)
@@ -1479,13 +1491,17 @@ int run_fixed(Batch& bt, bool push, bool pull) {
       apart = apart && it.d.k >= 32 && (it.d.k % 4 == 0 || it.d.k >= 1024);
     }
     const bool stream = floats >= kStreamFloats && apart;
-    const KernelSet kernels = push && pull ? PSKV_KSET_OF(k_fixed_own, true, true, false)
+    const KernelSet kernels = lengthy ? (push && pull ? PSKV_KSET_OF(k_fixed_long, true, true)
+                                         : push       ? PSKV_KSET_OF(k_fixed_long, true, false)
+                                                      : PSKV_KSET_OF(k_fixed_long, false, true))
+                              : push && pull ? PSKV_KSET_OF(k_fixed_own, true, true, false)
                               : push       ? stream ? PSKV_KSET_OF(k_fixed_own, true, false, true)
                                                     : PSKV_KSET_OF(k_fixed_own, true, false, false)
                               : stream     ? PSKV_KSET_OF(k_fixed_own, false, true, true)
                                            : PSKV_KSET_OF(k_fixed_own, false, true, false);
-    rc = launch_batch(bt, push ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, [](const Item& it) {
-      return it.r.n ? (it.r.n + own_keys(it.d.k) - 1) / own_keys(it.d.k) : 0ull;
+    rc = launch_batch(bt, push ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, [&](const Item& it) -> uint64_t {
+      if (!it.r.n) return 0;
+      return lengthy ? it.r.n * long_groups(it.d.k) : (it.r.n + own_keys(it.d.k) - 1) / own_keys(it.d.k);
     });
   } else if (bt[0].r.replay == kReplayCapture) {
     // a recorded repeat is compared as a whole and uses the references that are there: no lookup

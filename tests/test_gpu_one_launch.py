@@ -24,7 +24,9 @@ def _shifted(a, dev, shift):
 # floats per row, keys: one workgroup's share and a key more or less, the last share of a push and one beyond, rows
 # that are a workgroup's all, and longer ones
 FIXED = [(1, 1), (1, 256), (1, 257), (3, 511), (4, 513), (15, 256 * 512), (16, 256 * 512 + 1), (64, 63), (64, 65),
-         (64, 64 * 512), (64, 64 * 512 + 1), (500, 9), (4093, 4), (4096, 3), (4097, 3)]
+         (64, 64 * 512), (64, 64 * 512 + 1), (500, 9), (4093, 4), (4096, 3),
+         # and those of several workgroups: a part of one quad, whole parts, one row, as many keys as go this way, too many floats
+         (4097, 3), (4097, 256), (4097, 257), (8192, 2), (8195, 5), (100_003, 7), (1 << 22, 1), (16_384, 256), (16_385, 256)]
 
 
 @pytest.mark.parametrize("looks", [None, "0"])
@@ -58,7 +60,7 @@ def test_fixed_in_one_launch(capi, orc, dev, monkeypatch, k, n, looks):
 
 
 @pytest.mark.parametrize("looks", [None, "0"])
-@pytest.mark.parametrize("k,n", [(5, 1), (5, 700), (64, 64 * 512 - 1)])
+@pytest.mark.parametrize("k,n", [(5, 1), (5, 700), (64, 64 * 512 - 1), (4100, 1), (4100, 255), (9001, 3)])
 def test_a_push_that_repeats_a_key_changes_nothing(capi, orc, dev, monkeypatch, k, n, looks):
     """The repeat sits in the first, in the last or in any workgroup's share: no stored value changes, created rows are
     zero, the next sync says EINVAL, and the push behind it is served."""
@@ -86,6 +88,39 @@ def test_a_push_that_repeats_a_key_changes_nothing(capi, orc, dev, monkeypatch, 
         o.push(some, more)
         assert_bits_equal(t.dump()[2], o.dump()[2], "repeat at %d" % at)
         t.close()
+
+
+@pytest.mark.parametrize("k", [4097, 20_000])
+def test_long_rows_in_any_order(capi, orc, dev, k):
+    """Keys that are not sorted, the key that marks an empty slot among them, rows made by pulls, many requests (whose counter
+    records come from the same launch); a push that repeats a key it does not stand next to is refused, a pull served."""
+    announce("long rows", k)
+    rng = np.random.default_rng(k)
+    pool = np.append(unique_keys(rng, 40), np.uint64(2**64 - 1))
+    t, o = capi.Table(capi.MODE_FIXED, row_len=k, initial_capacity=8), orc.Store(orc.MODE_FIXED, k)
+
+    def pull(keys):
+        out = _shifted(np.full(keys.size * k, 7, np.float32), dev, 0)
+        t.pull(to_dev(keys, dev), out)
+        t.sync()
+        return out.cpu().numpy()
+
+    for turn in range(12):
+        some = rng.permutation(pool)[:rng.integers(1, 17)]
+        vals = rng.standard_normal(some.size * k).astype(np.float32)
+        t.push(to_dev(some, dev), to_dev(vals, dev))
+        o.push(some, vals)
+        some = rng.permutation(pool)[:9]
+        assert_bits_equal(pull(some), o.pull(some)[0], "turn %d" % turn)
+    twice = np.append(pool[:5], pool[2])[::-1].copy()
+    o.pull(pool[:5])
+    with pytest.raises(capi.PskvError) as e:
+        t.push(to_dev(twice, dev), to_dev(np.ones(twice.size * k, np.float32), dev))
+        t.sync()
+    assert e.value.code == capi.EINVAL
+    assert_bits_equal(pull(twice), o.pull(twice)[0])
+    assert_bits_equal(t.dump()[2], o.dump()[2])
+    assert t.size() == o.size()
 
 
 def _lens(rng, n, kind):
