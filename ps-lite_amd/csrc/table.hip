@@ -566,15 +566,13 @@ int grow(pskv_table* t, GrowBuf* b, size_t bytes) {
 }
 
 // Moves the base of the bounds forward to the newest record the device has published: the
-// counters after request `seq_end`.
+// counters after request `s1`.
 void adopt_snapshot(pskv_table* t) {
   const Snapshot* sn = t->snap;
-  const uint64_t s1 = sn->seq_end;
-  std::atomic_thread_fence(std::memory_order_acquire);
-  const uint64_t c = sn->count, top = sn->arena_top;
-  std::atomic_thread_fence(std::memory_order_acquire);
-  const uint64_t s0 = sn->seq_begin;
-  if (s0 != s1 || s1 < t->base_seq || s1 >= t->seq) return;  // (the initial record is all ones)
+  const uint64_t s1 = sn->seq, count = sn->count, units = sn->arena_top;
+  if (count >> kRecordTagAt != (record_word(0, s1) >> kRecordTagAt) || units >> kRecordTagAt != count >> kRecordTagAt) return;
+  if (s1 < t->base_seq || s1 >= t->seq) return;  // (the initial record is all ones)
+  const uint64_t c = count & (((uint64_t)1 << kRecordTagAt) - 1), top = units & (((uint64_t)1 << kRecordTagAt) - 1);
   uint64_t named = 0;
   for (uint64_t r = t->base_seq; r <= s1; ++r) {
     named += t->log_keys[r % pskv_table::kLog];
