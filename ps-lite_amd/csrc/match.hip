@@ -29,7 +29,7 @@ constexpr unsigned kMatchBlock = 256;
 constexpr unsigned kMatchItems = 4;
 constexpr uint64_t kFewKeys = 2ull * 256 * kMatchBlock * kMatchItems;
 constexpr unsigned kMatchLds = 1536;    // source keys (and values) a workgroup holds in LDS at a time (18 KiB)
-constexpr unsigned kMatchTurn = 3;      // source keys a lane asks for at a time
+constexpr unsigned kMatchTurn = kMatchLds / kMatchBlock;  // source keys a lane asks for: all that there is room for
 // A longer stretch than so many pieces is sampled, not staged. (Pieces follow from each other, but read in one go
 // what the sampled search reads key by key: they pay while there are workgroups enough to fill the GPU.)
 constexpr unsigned kMatchPieces = 8, kMatchPiecesFew = 3;
@@ -116,8 +116,8 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
 // One workgroup per tile of kMatchBlock * ITEMS keys of `near`, which it finds in `far`. Those are the destination's
 // and the source's keys, or with SWAP, where the source is much the smaller set, the other way round: the walk then
 // reads, and the row kernel visits, what there is in the source. Bound by memory once the loads do not wait for each
-// other: 12M source against 16M destination keys took 100 us with one source key per lane asked for at a time, 77 with
-// three (5.2 TB/s).
+// other: 12M source against 16M destination keys, the whole call, took 125 us with one source key per lane asked for at a
+// time, 104.7 with three under a condition each, 101 without it, and 99.5 with all six that LDS has room for.
 // OWN: the workgroup finds where its stretch begins and ends itself (a wavefront each) instead of reading it from `spans`:
 // the search is hidden behind the keys of the tile, and a launch of 10 to 13 us in front of this one falls away, but every
 // workgroup reads lines for it that nobody else needs. Up to kOwnSpans tiles that is the better way (us per call:
@@ -191,15 +191,23 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
       const unsigned len = span - base < kMatchLds ? (unsigned)(span - base) : kMatchLds;
       const bool last_piece = base + len == span;
       if (base) __syncthreads();  // everyone is done with the piece before
-      // (all loads of a turn before the first of them is waited for)
-      for (unsigned t0 = threadIdx.x; t0 < len; t0 += kMatchBlock * kMatchTurn) {
+      // (all loads before the first of them is waited for; with values, a lane behind the end asks for the last key, as a
+      // load under a condition waits for those in front of it)
+      {
+        const unsigned t0 = threadIdx.x;
         uint64_t ks[kMatchTurn];
-        float vs[kMatchTurn];
+        float vs[kMatchTurn] = {};
 #pragma unroll
         for (unsigned q = 0; q < kMatchTurn; ++q) {
           const unsigned t = t0 + q * kMatchBlock;
-          ks[q] = t < len ? far[lo + base + t] : 0;
-          vs[q] = vals_here && t < len ? src_vals[lo + base + t] : 0.0f;
+          ks[q] = K1 ? far[lo + base + (t < len ? t : len - 1)] : t < len ? far[lo + base + t] : 0;
+        }
+        if (vals_here) {
+#pragma unroll
+          for (unsigned q = 0; q < kMatchTurn; ++q) {
+            const unsigned t = t0 + q * kMatchBlock;
+            vs[q] = src_vals[lo + base + (t < len ? t : len - 1)];
+          }
         }
 #pragma unroll
         for (unsigned q = 0; q < kMatchTurn; ++q) {
@@ -240,7 +248,8 @@ __global__ __launch_bounds__(kMatchBlock) void k_match_keys(const uint64_t* __re
     // from each other for 13,000 keys, 50 us.)
     const uint64_t step = (span + kMatchLds - 1) / kMatchLds;
     const unsigned samples = (unsigned)((span + step - 1) / step);
-    for (unsigned t0 = threadIdx.x; t0 < samples; t0 += kMatchBlock * kMatchTurn) {
+    {
+      const unsigned t0 = threadIdx.x;
       uint64_t ks[kMatchTurn];
 #pragma unroll
       for (unsigned q = 0; q < kMatchTurn; ++q) {
