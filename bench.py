@@ -1070,11 +1070,12 @@ def run_embed(args, capi, dev):
         # gradient in, row in, row out: 12 B/float, the rows scattered over the arena
         "roofline": dict(roofline(12.0 * n * k, acc[0], acc[1], traffic("rows_acc_embed", n * k), acc[2]),
                          kernel="k_rows<acc,fixed> (row += in, rows scattered)", bytes_per_float=12),
-        "kernels": {"rows_gather": dict(roofline(8.0 * n * k, gat[0], gat[1],
+        "kernels": {"rows_gather": dict(roofline(8.0 * n * k + 24.0 * n, gat[0], gat[1],
                                                  traffic("rows_gather_embed", n * k), gat[2]),
-                                        bytes_per_float=8),
+                                        kernel="k_fixed_own (key -> row, and the rows)", bytes_per_float=8,
+                                        bytes_per_key=24),
                     "lookup": dict(roofline(24.0 * n, look[0], look[1], traffic("lookup_embed", n), look[2]),
-                                   kernel="k_lookup_fixed (key -> row, the pull's; the push reuses it)",
+                                   kernel="k_lookup_fixed (the push's, which finds the references that the pull has left)",
                                    bytes_per_key=24)},
     }
     return res, (all_keys, batches[args.warmup:], g.reshape(-1), n, rows, k)
