@@ -471,7 +471,7 @@ __global__ __launch_bounds__(kBlock) void k_concat(const Segment* __restrict__ s
 // does not). Nothing says which queue a stream is on, but the calls themselves: a context whose calls take long tries
 // other streams and keeps to the one on which they took least.
 constexpr int kSliceStreams = 4;
-constexpr float kSliceSlow = 20.0f;  // us; a call that waits for nobody takes 9 to 12
+constexpr float kSliceSlow = 20.0f;  // us; a call that waits for nobody takes 8 to 15
 struct SliceCtx {
   int device = -1;
   hipStream_t stream = nullptr;  // the one in use, of
