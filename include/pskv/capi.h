@@ -30,7 +30,8 @@
  *    PSKV_EINVAL (no stored value changes; PSKV_MODE_FIXED may leave the keys it named as
  *    zero rows, as a pull of them would), PSKV_MODE_SCALAR gives the result of the
  *    reference's loop (kv_app.h:451-459). An unsorted request that repeats a key has an
- *    unspecified result in every mode (no memory other than its keys' values is touched).
+ *    unspecified result in every mode (no memory other than its keys' values is touched;
+ *    where PSKV_MODE_FIXED notices and says PSKV_EINVAL, no stored value has changed).
  *    A table must not be used from two threads at once (the reference
  *    runs the handle on one Customer thread, src/customer.cc:49-63).
  *    pskv_slice is re-entrant.

@@ -110,11 +110,13 @@ struct alignas(32) DevState {
   // first level of the last-workgroup ticket: one counter per 128-byte line, and behind it the facts of its
   // workgroups (report_facts)
   unsigned int ticket_sub[kTicketShards * 32];
-  // one_launch.h: pushes served so far << 2 | the verdict on the newest one; everyone watches it, so the line is its own
+  // k_fixed_own: the word of the verdict (handover.h); everyone watches it, so the line is its own
   unsigned long long push_verdict;
   // k_fixed_long: the newest of its requests that has created a row, and how many rows there were before it
   unsigned long long fresh_from;
-  unsigned long long pad[14];
+  // k_fixed_own: a bit for every workgroup of a push that has left its rows to the last one, all zero between requests
+  unsigned long long shares_left[8];
+  unsigned long long pad[6];
   // one_launch.h: what the workgroups of a var-len request tell each other, all zero between requests
   unsigned long long parts[kVarParts];
 };

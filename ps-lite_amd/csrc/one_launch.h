@@ -3,6 +3,7 @@
 // ones), not by what they do.
 #ifndef PSKV_ONE_LAUNCH_H_
 #define PSKV_ONE_LAUNCH_H_
+#include "handover.h"
 #include "table_kernels.h"
 
 namespace pskv {
@@ -15,8 +16,10 @@ namespace pskv {
 // A push changes nothing before it is known that the request repeats no key: the workgroups hand in what they have
 // found once their keys are looked up, ask for their rows, and the verdict is there by the time those are. They have
 // to be on the GPU together for that: kOwnPushGroups of them are a third of what it holds. Who does not see the verdict
-// in time all the same (d.cache_mode looks: something else may keep a part of the workgroups off the GPU) reads all
-// keys of the request itself, so nobody depends on the others but for time.
+// in time all the same (d.cache_mode looks: something else may keep a part of the workgroups off the GPU) leaves its rows to
+// the workgroup that reaches the verdict (handover.h), so nobody depends on the others but for time, and there is one
+// verdict for the whole request, whatever it rests on: that a new key comes twice in a request that is not sorted only those
+// notice who claim its slot. (Shares that are left take some 10 us each.)
 // Measured (us per two steps of pull and push and a pull, lookup and rows as two launches -> one): 49,881 rows of 15 floats
 // one table 49-53 -> 40, three in turn 28-39 -> 20.4; 30,000 of 64 53-59 -> 41, 37-45 -> 30.6; 1M of 64, whose pushes are two
 // launches, 668 -> 633, 643 -> 633. Of that the loads of a lane's rows side by side, the ticket in front of them and its
@@ -33,6 +36,53 @@ __host__ __device__ constexpr unsigned own_keys(uint64_t k) {
 
 __device__ __forceinline__ unsigned long long ask_verdict(const DevState* st) {
   return __hip_atomic_load(&st->push_verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The memory of leave_share.
+struct ShareMem {
+  DevState* st;
+  __device__ unsigned long long* word() { return &st->shares_left[blockIdx.x / 64]; }
+  __device__ unsigned long long bit() { return 1ull << (blockIdx.x % 64); }
+  __device__ void mark() {
+    unsigned long long was = atomicOr(word(), bit());
+    asm volatile("" : "+v"(was) : : "memory");  // (it is there before anything that follows)
+  }
+  __device__ bool unmark() { return (atomicAnd(word(), ~bit()) & bit()) != 0; }
+  __device__ unsigned long long swap(unsigned long long from, unsigned long long to) {
+    unsigned long long was = atomicCAS(&st->push_verdict, from, to);
+    asm volatile("" : "+v"(was) : : "memory");
+    return was;
+  }
+};
+static_assert(kOwnPushGroups == 64 * (sizeof(DevState::shares_left) / 8), "a bit for every workgroup of a push");
+
+// The rows of the workgroups that have left theirs to this one. Every thread calls it.
+template <bool PULL, bool STREAM>
+__device__ __forceinline__ void serve_shares_left(const TableReq& d, bool rejected) {
+  __shared__ unsigned long long s_left;
+  const unsigned quads = (unsigned)((d.k + 3) >> 2), rest = (unsigned)d.k & 3u, share = own_keys(d.k);
+  for (unsigned w = 0; w * 64 < d.nblk; ++w) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_left = atomicExch(&d.st->shares_left[w], 0ull);
+    __syncthreads();
+    __threadfence();  // nothing stale is left of what those workgroups have written in front of their marks
+    for (unsigned long long left = s_left; left; left &= left - 1) {
+      const uint64_t first = ((uint64_t)w * 64 + __builtin_ctzll(left)) * share;
+      const unsigned mine = d.n - first < share ? (unsigned)(d.n - first) : share;
+      for (unsigned quad = threadIdx.x; quad < mine * quads; quad += kBlock) {
+        const unsigned row = quad / quads, c = quad - row * quads, col = c * 4, count = rest && c + 1 == quads ? rest : 4u;
+        const uint64_t ref = d.ref[first + row];
+        if (ref == kRefAbsent) continue;
+        const bool fresh = (ref & kRefNew) != 0;
+        float* const at = d.arena + (ref & ~kRefNew) * d.k + col;
+        f32x4 y = (f32x4)(0.f);
+        if (!fresh) y = load_part<STREAM>(at, count);
+        if (!rejected) y = y + load_part<STREAM>(d.vals + (first + row) * d.k + col, count);
+        if (fresh || !rejected) store_part<STREAM>(y, at, count);
+        if (PULL) store_part<STREAM>(y, d.out + (first + row) * d.k + col, count);
+      }
+    }
+  }
 }
 
 template <bool PUSH, bool PULL, bool STREAM, int TABLES>
@@ -155,22 +205,25 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
   for (unsigned q = 0; q < kOwnTurns; ++q)
     if (ref[q] & kRefNew) y[q] = (f32x4)(0.f);
   // (before anything is stored: the counter record goes past the caches and would wait for the rows)
-  unsigned verdict = 2;  // not known yet
+  constexpr unsigned kUnknown = 2, kIsLast = 4;
+  unsigned verdict = kUnknown;
+  // The last workgroup: what the word of the verdict was in front of its own. (Nobody waits for it in front of the rows: it
+  // has no other value, and it is looked at behind them. With a wait small pushes took 0.35 us of 11 longer.)
+  unsigned long long exchanged;
+  asm volatile("" : "=v"(exchanged));
   if ((PUSH || d.snap) && threadIdx.x < 64) {
     unsigned last = 0;
     if (threadIdx.x == 0) last = ticket_is_last(st, nblk, ticket) ? 1u : 0u;
     if (__shfl(last, 0)) {
       if (PUSH) {
-        verdict = take_facts(st, nblk) & kReqDuplicate ? 1u : 0u;
-        if (threadIdx.x == 0)
-          __hip_atomic_store(&st->push_verdict, ((before >> 2) + 1) << 2 | verdict, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+        verdict = (take_facts(st, nblk) & kReqDuplicate ? 1u : 0u) | kIsLast;
+        if (threadIdx.x == 0) exchanged = atomicExch(&st->push_verdict, next_verdict(before, verdict & 1u));
       }
       if (d.snap) publish_snapshot(st, d.snap, d.snap_seq);
     } else if (PUSH && threadIdx.x == 0) {
-      for (unsigned looks = d.cache_mode; looks && verdict == 2; --looks) {
+      for (unsigned looks = d.cache_mode; looks && verdict == kUnknown; --looks) {
         const unsigned long long now = ask_verdict(st);
-        if (now != before) verdict = (unsigned)now & 1u; else __builtin_amdgcn_s_sleep(1);
+        if (has_verdict(now, before)) verdict = (unsigned)(now & kVerdictYes); else __builtin_amdgcn_s_sleep(1);
       }
     }
     if (threadIdx.x == 0) s_verdict = verdict;
@@ -179,12 +232,19 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
   if (PUSH) {
     __syncthreads();
     verdict = s_verdict;
-    if (verdict == 2) {
-      bool any = false;
-      for (uint64_t at = 1 + threadIdx.x; at < n; at += kBlock) any |= d.keys[at] == d.keys[at - 1];
-      verdict = __syncthreads_or(any ? 1 : 0) ? 1u : 0u;
+    if (verdict == kUnknown) {
+      __threadfence();  // the rows of its keys are there for whoever moves them
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        ShareMem m{st};
+        const int late = leave_share(m, before);
+        s_verdict = late < 0 ? kUnknown : (unsigned)late;
+      }
+      __syncthreads();
+      verdict = s_verdict;
+      if (verdict == kUnknown) return;
     }
-    rejected = verdict != 0;
+    rejected = (verdict & 1u) != 0;
   }
 #pragma unroll
   for (unsigned q = 0; q < kOwnTurns; ++q) {
@@ -194,6 +254,13 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
     if (PUSH && !rejected) y[q] = y[q] + x[q];  // a created row is a zero row first (0.0f + v), kv_app.h:454
     if (fresh || (PUSH && !rejected)) store_part<STREAM>(y[q], d.arena + (ref[q] & ~kRefNew) * k + col[q], count[q]);
     if (PULL) store_part<STREAM>(y[q], d.out + (first + row[q]) * k + col[q], count[q]);
+  }
+  if (PUSH && (verdict & kIsLast)) {
+    __syncthreads();
+    asm volatile("" : "+v"(exchanged));
+    if (threadIdx.x == 0) s_verdict = exchanged & kSharesLeft ? 1u : 0u;
+    __syncthreads();
+    if (s_verdict) serve_shares_left<PULL, STREAM>(d, rejected);
   }
 }
 

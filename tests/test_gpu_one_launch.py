@@ -33,7 +33,7 @@ FIXED = [(1, 1), (1, 256), (1, 257), (3, 511), (4, 513), (15, 256 * 512), (16, 2
 @pytest.mark.parametrize("k,n", FIXED)
 def test_fixed_in_one_launch(capi, orc, dev, monkeypatch, k, n, looks):
     """New keys, held ones and a mix, pushed, pulled and both in one; with `looks` 0 no workgroup of a push waits for the
-    verdict: every one reads all keys."""
+    verdict: the last one moves the rows of all."""
     import torch
     announce("fixed in one launch", k, n, looks)
     if looks is not None:
@@ -88,6 +88,46 @@ def test_a_push_that_repeats_a_key_changes_nothing(capi, orc, dev, monkeypatch, 
         o.push(some, more)
         assert_bits_equal(t.dump()[2], o.dump()[2], "repeat at %d" % at)
         t.close()
+
+
+@pytest.mark.parametrize("looks", [None, "0"])
+@pytest.mark.parametrize("k,n", [(1, 256 * 65), (5, 700), (64, 64 * 511), (300, 20)])
+def test_a_new_key_twice_in_a_request_that_is_not_sorted(capi, orc, dev, monkeypatch, k, n, looks):
+    """Next to each other in no workgroup's eyes, but both of them one workgroup's, which therefore notices when it makes the
+    row: the push is refused as a whole, whoever has waited for the verdict. In front of it and behind it pushes of keys in
+    any order, new ones among them."""
+    import torch
+    announce("fixed, not sorted", k, n, looks)
+    if looks is not None:
+        monkeypatch.setenv("PSKV_PUSH_LOOKS", looks)
+    rng = np.random.default_rng(n)
+    t, o = capi.Table(capi.MODE_FIXED, row_len=k, initial_capacity=4 * n), orc.Store(orc.MODE_FIXED, k)
+    pool = rng.permutation(unique_keys(rng, 2 * n + 1))
+
+    def push(keys, both=False):
+        vals = rng.standard_normal(keys.size * k).astype(np.float32)
+        if not both:
+            t.push(to_dev(keys, dev), _shifted(vals, dev, 1))
+            return o.push(keys, vals)
+        out = torch.full((keys.size * k,), 7.0, device=dev)
+        t.pushpull(to_dev(keys, dev), to_dev(vals, dev), out)
+        t.sync()
+        assert_bits_equal(out.cpu().numpy(), o.pushpull(keys, vals)[0])
+
+    push(pool[:n])
+    push(pool[n // 2:n // 2 + n], both=True)
+    # (three keys into the request, or two: a workgroup has at least that many)
+    twice = pool[:n - 2]
+    twice = np.concatenate([pool[-1:], twice[:1], pool[-1:], twice[1:]])
+    t.push(to_dev(twice, dev), to_dev(rng.standard_normal(twice.size * k).astype(np.float32), dev))
+    with pytest.raises(capi.PskvError) as e:
+        t.sync()
+    assert e.value.code == capi.EINVAL
+    o.pull(pool[-1:])  # (the row it made stays, as a zero row)
+    assert_bits_equal(t.dump()[2], o.dump()[2])
+    push(rng.permutation(pool)[:n])
+    push(rng.permutation(pool)[:n], both=True)
+    assert_bits_equal(t.dump()[2], o.dump()[2])
 
 
 @pytest.mark.parametrize("k", [4097, 20_000])
