@@ -10,6 +10,7 @@
 
 #include "device_common.h"
 #include "host_common.h"
+#include "parts.h"
 #include "search.h"
 
 namespace pskv {
@@ -26,14 +27,10 @@ __global__ __launch_bounds__(kBlock) void k_bounds(const uint64_t* __restrict__ 
   if (lane == 0) lb[w] = lo;
 }
 
-// What the host reads goes to pinned memory, every word with a mark of its own that it is there (the host has cleared it):
-// the host watches all of them, nothing has to arrive before anything else, and no fence writes back what the requests that
-// run meanwhile have left in the L2. Positions and sums are below 2^62 in size.
-constexpr uint64_t kHere = 1ull << 63;
+// (a marked word of parts.h)
 __device__ __forceinline__ void tell(uint64_t* to, uint64_t x) {
   __hip_atomic_store(to, x | kHere, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-uint64_t told(uint64_t word) { return (uint64_t)((int64_t)(word << 1) >> 1); }  // (sums of lens may be negative)
 
 // The largest of this lane's and all lower lanes' values.
 __device__ __forceinline__ uint64_t wave_running_max(uint64_t x, unsigned lane) {
@@ -73,7 +70,6 @@ __global__ void k_bounds_chain(const uint64_t* __restrict__ lb, uint64_t S,
 // workgroup of up to 16 wavefronts, each searching one or two boundaries, then the chain.
 // The boundaries travel with the launch: no read across the host link before the search.
 constexpr unsigned kFusedWaves = 16;
-constexpr unsigned kFusedTargets = 2 * kFusedWaves;
 struct FusedTargets {
   uint64_t v[kFusedTargets];
 };
@@ -156,20 +152,6 @@ __device__ __forceinline__ void hand_over(SumsState* state, unsigned S, unsigned
 // over), 5,000 over 16 11.9 (13.6; the searches of the kernel below 19.2), 15,826 over 3 11.1 (12.6; 15.1), 262,144 over 4
 // 12.0 (13.6). The searches against this: 400,000 over 8 15.5 and 12.8, 1M over 16 16.9 and 14.9, but with a thousand words
 // for the host to read 2M over 16 17.0 and 17.3: up to 512 parts.)
-constexpr unsigned kFewSumsBlock = 256, kFewSumsItems = 8;  // (larger workgroups find no place on a busy GPU)
-constexpr uint64_t kFewSumsPart = (uint64_t)kFewSumsBlock * kFewSumsItems;
-constexpr unsigned kFewSumsParts = 512;
-constexpr uint64_t kFewSumsKeys = kFewSumsParts * kFewSumsPart;
-// The words a part tells: lens in the lower kPartLensBits (2,048 of 32 bits, a sign), and above them for the part the first
-// of its boundaries and their number, for a boundary its place in the part.
-constexpr unsigned kPartLensBits = 45, kPartCountAt = kPartLensBits + 6;
-static_assert(kFewSumsPart <= 1u << 11 && kFusedTargets < 64, "a place and two numbers of boundaries fit above the lens");
-__host__ __device__ constexpr unsigned long long part_word(unsigned long long lens, unsigned long long upper) {
-  return (lens & ((1ull << kPartLensBits) - 1)) | upper << kPartLensBits;
-}
-inline uint64_t part_lens(uint64_t word) {
-  return (uint64_t)((int64_t)(word << (64 - kPartLensBits)) >> (64 - kPartLensBits));
-}
 __global__ __launch_bounds__(kFewSumsBlock) void k_bounds_sums_few(const uint64_t* __restrict__ keys,
                                                                    const int32_t* __restrict__ lens, uint64_t n,
                                                                    uint64_t* __restrict__ bounds_host,
@@ -519,45 +501,6 @@ SliceCtx* take_ctx(int device) {
   return c;
 }
 
-// Watches `count` marked words (tell()) of pinned memory for up to about 200 us each; false when one did not show up.
-bool all_here(const uint64_t* words, size_t count) {
-  for (size_t i = 0; i < count; ++i) {
-    if (__atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0) continue;
-    const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-    for (bool here = false; !here;) {
-      for (int spin = 0; spin < 256 && !here; ++spin) here = __atomic_load_n(words + i, __ATOMIC_ACQUIRE) != 0;
-      if (!here && std::chrono::steady_clock::now() > give_up) return false;
-    }
-  }
-  return true;
-}
-
-// What the parts of k_bounds_sums_few have told: the positions of the boundaries and the sums of the slices between them.
-// False when a word did not show up, or when keys that are not sorted have left a boundary without an owner, or with
-// two: what comes late may then still be on its way.
-bool join_parts(const uint64_t* parts, const uint64_t* bounds, uint64_t n, size_t S, uint64_t* pos, uint64_t* sums) {
-  uint64_t before = 0, below[kFusedTargets], seen = 0;
-  bool clear = true;
-  for (size_t i = 0; i <= S; ++i) pos[i] = below[i] = 0;
-  for (uint64_t b = 0; b * kFewSumsPart < n; ++b) {
-    clear = all_here(parts + b, 1) && clear;
-    const uint64_t word = parts[b];
-    const unsigned first = (unsigned)(word >> kPartLensBits) & 63u, count = (unsigned)(word >> kPartCountAt) & 63u;
-    for (unsigned i = first; i < first + count; ++i) {
-      clear = all_here(bounds + i, 1) && !(seen >> i & 1u) && clear;
-      seen |= 1ull << i;
-      pos[i] = b * kFewSumsPart + ((bounds[i] & ~kHere) >> kPartLensBits);
-      below[i] = before + part_lens(bounds[i]);
-    }
-    before += part_lens(word);
-  }
-  for (size_t i = 1; i <= S; ++i) {
-    if (pos[i] < pos[i - 1]) pos[i] = pos[i - 1], below[i] = below[i - 1];
-    sums[i - 1] = below[i] - below[i - 1];
-  }
-  return clear && seen == (2ull << S) - 1;
-}
-
 // A call on the context's stream has taken `us` and nothing of it is left: the stream of the next one.
 void note_call(SliceCtx* c, float us) {
   float& mine = c->took[c->at];
@@ -763,12 +706,14 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
       k_export_sums<<<dim3((unsigned)((S + 255) / 256)), dim3(256), 0, c->stream>>>(d_sums, S, h_sums);
       PSKV_HIP(hipGetLastError());
     }
+    const WatchEnd end = watch_end(std::chrono::steady_clock::now());
     if (in_parts) {
-      if (!join_parts(h_parts, h_pos, n, S, pos, val_pos + 1)) {
+      if (!join_parts(h_parts, h_pos, n, S, pos, val_pos + 1, end)) {
         PSKV_HIP(hipStreamSynchronize(c->stream));
-        (void)join_parts(h_parts, h_pos, n, S, pos, val_pos + 1);
+        (void)join_parts(h_parts, h_pos, n, S, pos, val_pos + 1, end);
       }
-    } else if (!watch || !all_here(h_pos, S + 1) || (sums_too && !all_here(reinterpret_cast<uint64_t*>(h_sums), S))) {
+    } else if (!watch || !all_here(h_pos, S + 1, end) ||
+               (sums_too && !all_here(reinterpret_cast<uint64_t*>(h_sums), S, end))) {
       PSKV_HIP(hipStreamSynchronize(c->stream));
     }
     lease.idle = true;  // (what the kernel still does is clear its state for the next one on the stream)
