@@ -12,6 +12,7 @@
 #include "host_common.h"
 #include "parts.h"
 #include "search.h"
+#include "stream_choice.h"
 
 namespace pskv {
 namespace {
@@ -448,18 +449,11 @@ __global__ __launch_bounds__(kBlock) void k_concat(const Segment* __restrict__ s
 // Per-call state of the slicer. Calls may come from any thread at once
 // (KVWorker::Push is thread-safe, kv_app.h:101-104), so each call takes a context
 // of its own from a pool and returns it afterwards.
-// A process has few hardware queues (four), and a stream shares its one with others: where those are tables with
-// requests queued, every call waits behind them (20 pushes of 1M keys, sliced one by one: 2,250 us, or 2,040 where it
-// does not). Nothing says which queue a stream is on, but the calls themselves: a context whose calls take long tries
-// other streams and keeps to the one on which they took least.
-constexpr int kSliceStreams = 4;
-constexpr float kSliceSlow = 20.0f;  // us; a call that waits for nobody takes 8 to 15
 struct SliceCtx {
   int device = -1;
   hipStream_t stream = nullptr;  // the one in use, of
   hipStream_t streams[kSliceStreams] = {nullptr};
-  float took[kSliceStreams] = {0.0f};  // us per call lately; forgotten little by little while another one is in use
-  int at = 0;
+  StreamChoice choice;
   SumsState* sums_state = nullptr;
   void* dev = nullptr;      // device scratch: targets, lower bounds, positions, sums
   size_t dev_bytes = 0;
@@ -501,21 +495,13 @@ SliceCtx* take_ctx(int device) {
   return c;
 }
 
-// A call on the context's stream has taken `us` and nothing of it is left: the stream of the next one.
-void note_call(SliceCtx* c, float us) {
-  float& mine = c->took[c->at];
-  mine = mine == 0.0f ? us : 0.75f * mine + 0.25f * us;
-  for (int i = 0; i < kSliceStreams; ++i)
-    if (i != c->at) c->took[i] *= 0.995f;
-  if (mine < kSliceSlow) return;
-  // (by a good margin: a stream wait comes with it, and where the GPU itself is what calls wait for all are alike)
-  int best = c->at;
-  for (int i = 0; i < kSliceStreams; ++i)
-    if (c->took[i] < 0.75f * mine && c->took[i] < c->took[best]) best = i;
-  if (best == c->at) return;
+// A call on the context's stream has taken `us`, `own` by itself, and nothing of it is left: the stream of the next one.
+void note_call(SliceCtx* c, float us, float own) {
+  const int next = c->choice.note(us, own);
+  if (next == c->choice.at) return;
   if (hipStreamSynchronize(c->stream) != hipSuccess) return;  // (the kernel may still be clearing its state)
-  c->at = best;
-  c->stream = c->streams[best];
+  c->choice.at = next;
+  c->stream = c->streams[next];
 }
 
 void give_ctx(SliceCtx* c) {
@@ -718,7 +704,8 @@ int pskv_slice(int device, const uint64_t* keys, size_t n, const int32_t* lens, 
     }
     lease.idle = true;  // (what the kernel still does is clear its state for the next one on the stream)
     if (watch)
-      note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count());
+      note_call(c, std::chrono::duration<float, std::micro>(std::chrono::steady_clock::now() - asked).count(),
+                own_slice_us(n, S, do_sums));
     for (size_t i = 0; i <= S && !in_parts; ++i) pos[i] = std::max(told(h_pos[i]), i ? pos[i - 1] : 0);
     if (do_sums && !in_parts)
       for (size_t i = 0; i < S; ++i) val_pos[i + 1] = sums_too ? told(h_sums[i]) : h_sums[i];  // per-slice sums for now
