@@ -132,7 +132,7 @@ __global__ __launch_bounds__(kBlock) void k_fixed_own(ReqBatch<TABLES> b) {
     count[q] = quad >= all ? 0u : rest && c + 1 == quads ? rest : 4u;
     x[q] = (f32x4)(0.f);
   }
-  if (PUSH && (!rest || first + mine < n)) {  // a shorter quad is read whole where the next row follows it
+  if (PUSH && whole_quads(first + mine, k, n)) {  // a shorter quad is read whole where rows enough follow it
 #pragma unroll
     for (unsigned q = 0; q < kOwnTurns; ++q) x[q] = load_quad<STREAM>(d.vals + (first + row[q]) * k + col[q]);
   } else if (PUSH) {

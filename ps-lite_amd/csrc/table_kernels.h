@@ -8,6 +8,7 @@
 #ifndef PSKV_TABLE_KERNELS_H_
 #define PSKV_TABLE_KERNELS_H_
 #include "device_common.h"
+#include "quads.h"
 #include "scan.h"
 #include "vote.h"
 
@@ -1197,9 +1198,10 @@ __device__ __forceinline__ void rows_quads_fixed(const RowsParams& p, uint64_t q
   const uint64_t row = row0 + over;
   const unsigned count = REST && c + 1 == quads ? rest : 4u;
   float* side = p.req + row * p.k + c * 4;
-  // (a shorter quad is read whole: what follows it is the next row, or the room behind the last row of the
+  // (a shorter quad is read whole: what follows it is other rows, or the room behind the last row of the
   // arena; only the end of the request's values is the end of what may be read)
-  if (OP == kOpAcc && REST) x = count == 4 || row + 1 < p.n ? load_quad<STREAM>(side) : load_part<STREAM>(side, rest);
+  if (OP == kOpAcc && REST)
+    x = count == 4 || whole_quads(row + 1, p.k, p.n) ? load_quad<STREAM>(side) : load_part<STREAM>(side, rest);
   const uint64_t r = p.ref[row];
   if (r == kRefAbsent) return;  // a key the lookup refused (duplicate in the request, full table)
   const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
