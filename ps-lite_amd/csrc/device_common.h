@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "start_rule.h"
+
 // Asks for all of a kernel's arguments at once (the compiler otherwise fetches them group by group where they are first
 // used, one wait each).
 #define PSKV_ASK_ARGS(...) asm volatile("" ::__VA_ARGS__)
@@ -70,7 +72,6 @@ struct __align__(16) Slot {
 constexpr int kCountShards = 32;
 constexpr int kShardStride = 16;  // in 8-byte words: one shard per 128-byte line
 constexpr int kTicketShards = 32;
-constexpr unsigned kVarParts = 256;  // workgroups of a var-len request that tell each other about it (one_launch.h)
 
 struct alignas(32) DevState {
   // The first 32 bytes are what a row kernel needs to know about its request (ReqFacts below):
@@ -104,6 +105,7 @@ struct alignas(32) DevState {
   unsigned int flush_next, flush_done;
   // k_scalar_repeat: votes of the launch in flight (vote.h), and launches served so far << 1 | verdict of the newest
   unsigned int repeat_arrived;
+  unsigned int told_ragged;  // what the host has been told of the rows of var-len pushes (tell_ragged)
   unsigned long long repeat_verdict;
   // keys held (slot array plus the side slot) = sum of the shards
   unsigned long long count_shard[kCountShards * kShardStride];

@@ -555,6 +555,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
     st->misaligned = of.flags & kReqMisaligned;
     st->cache_epoch = d.tag.epoch;
     if (bad) st->bad_epoch = d.tag.epoch;
+    tell_ragged(st, d.outcome, of.flags);
   }
   if (bad) return;  // nothing is created
   scan_pass2_offsets<kStartItems>(len, base, n, of.before, d.off, d.tile_key, d.ntiles, kTileVar, wsum);

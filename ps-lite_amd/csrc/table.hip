@@ -393,7 +393,7 @@ struct pskv_table {
   } sc_track[2];
   static const int kScKinds = 64;
   unsigned char sc_kind[kScKinds] = {0};  // kind of the request with number e, at e % kScKinds
-  unsigned long long* outcome = nullptr;  // pinned: epoch << 1 | same of the newest comparison
+  unsigned long long* outcome = nullptr;  // pinned: epoch << 1 | same of the newest comparison; VARLEN: whether pushes have ragged rows
   unsigned long long sc_seen = 0;         // the value of *outcome the host last looked at
   unsigned push_looks = 0;                // k_fixed_own: how often a workgroup looks for the verdict
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
@@ -1584,25 +1584,24 @@ int make_tile_tables(Batch& bt, bool there = false) {
   });
 }
 
-// Whether a var-len request starts with one launch (k_var_push_start, k_var_pull_start) and not with two: not where it is
-// being recorded, or arrives piece by piece, nor where its workgroups are too many to wait for each other (200,000 rows
-// in 391 of them, other rows in every step, three tables in turn: 233 us with two launches, 243 with one). The row kernel
-// behind it cleans up, so every table has to have one (`floats`). Of requests that may repeat the cached one those of
-// more than kVarCompareKeys keys are better off with two: the second returns at once (100,000 rows over 16 tables, the
-// same in every step: 51 us against 54; 20,000: 49 against 47).
-constexpr uint64_t kVarCompareKeys = 1u << 16;
+// Whether a var-len request starts with one launch (start_rule.h): not where it is being recorded, or arrives piece by piece.
+// The row kernel behind it cleans up, so every table has to have one (`floats`).
 template <typename F>
-bool start_together(const Batch& bt, uint64_t n_launch, F floats) {
-  uint64_t parts = 0;
-  bool compared = false;
+bool start_together(const Batch& bt, bool push, F floats) {
+  StartOf r;
+  r.tables = (unsigned)bt.size();
+  r.push = push;
   for (const Item& it : bt) {
     if (it.r.replay || it.r.pipe_in) return false;
     if (!it.r.n) continue;
     if (!floats(it)) return false;
-    parts += start_parts(it.r.n);
-    compared = compared || it.tag.try_cache;
+    r.keys += it.r.n;
+    r.floats += floats(it);
+    r.parts += start_parts(it.r.n);
+    r.compared = r.compared || it.tag.try_cache;
+    r.shortcut = r.shortcut || (it.tag.try_cache && !const_cast<volatile unsigned long long*>(it.t->outcome)[1]);
   }
-  return parts <= kVarParts && (!compared || n_launch <= kVarCompareKeys);
+  return one_start(r);
 }
 
 // Launches per var-len request: a push takes three (compare + scan pass 1; scan pass 2 +
@@ -1688,7 +1687,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     }
     int rc = growths.move();
     if (rc) return rc;
-    const bool start = start_together(bt, n_launch, [](const Item& it) { return it.r.nvals; });
+    const bool start = start_together(bt, push, [](const Item& it) { return it.r.nvals; });
     if (start) {
       for (Item& it : bt) {
         it.tag.try_cache = it.d.tag.try_cache = 0;
@@ -1747,7 +1746,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
     if (rc) return rc;
     for (Item& it : bt)
       if (it.r.n && !it.tag.try_cache) it.t->cache_valid = false;
-    const bool start = async_pull && start_together(bt, n_launch, [](const Item& it) { return it.r.out ? it.r.out_cap : 0; });
+    const bool start = async_pull && start_together(bt, false, [](const Item& it) { return it.r.out ? it.r.out_cap : 0; });
     if (start) {
       for (Item& it : bt) {
         if (!it.r.n) continue;
@@ -2284,7 +2283,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   for (int q = 0; q < kSmallParts; ++q) t->small_done[q] = t->shell->done[q];
   std::memset(t->st_host, 0, sizeof(StateView));
   std::memset(t->snap, 0xFF, sizeof(Snapshot));  // names no request
-  *t->outcome = 0ull;
+  t->outcome[0] = t->outcome[1] = 0ull;
   const uint64_t keys = opts->initial_capacity ? opts->initial_capacity : kDefaultCapacity;
   t->cap = std::max(kMinSlots, next_pow2((uint64_t)((double)keys / t->max_load) + 1));
   int rc = alloc_slots(t->cap, &t->slots, t->stream);

@@ -745,6 +745,14 @@ __device__ __forceinline__ void load_four(FourKeys<W>& f, const uint64_t* keys, 
   }
 }
 
+// Tells the host, in the word behind that of the outcomes, when a table's pushes come to have ragged rows or cease to.
+__device__ __forceinline__ void tell_ragged(DevState* st, unsigned long long* outcome, unsigned flags) {
+  const unsigned ragged = flags & kReqMisaligned ? 1u : 0u;
+  if (!outcome || ragged == st->told_ragged) return;
+  st->told_ragged = ragged;
+  outcome[1] = ragged;
+}
+
 // VARLEN push, first kernel: one pass over the request's keys and lens that
 //   - compares them with the cached request (when the host found the cache usable),
 //   - takes pass 1 of the lens scan (per-workgroup totals, flags),
@@ -800,7 +808,10 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
   __syncthreads();
   const bool same = s_same != 0u;
   scan_pass1_last(part, st, nblk, tag.epoch, flags, same, red, &carry_s);
-  if (threadIdx.x == 0) decide_same(st, tag, same, d.outcome);
+  if (threadIdx.x == 0) {
+    decide_same(st, tag, same, d.outcome);
+    tell_ragged(st, d.outcome, flags);
+  }
 }
 
 // VARLEN push, second kernel: pass 2 of the lens scan (request-side offsets and the tile

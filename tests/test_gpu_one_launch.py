@@ -277,6 +277,42 @@ def test_refused_varlen_requests(capi, orc, dev, monkeypatch, n, looks):
     assert_bits_equal(t.dump()[2], o.dump()[2])
 
 
+@pytest.mark.parametrize("S", [1, 5])
+def test_varlen_requests_that_repeat(capi, orc, dev, S):
+    """The same rows often enough to be expected, others of the same number, ragged ones and the first again: each starts with
+    one launch or with two, as the rule has it, and finds what the others have left."""
+    import torch
+    announce("varlen repeats", S)
+    rng = np.random.default_rng(S)
+    n = 5000
+    group, stores = capi.Group(S, capi.MODE_VARLEN), [orc.Store(orc.MODE_VARLEN) for _ in range(S)]
+    begin, end = orc.server_ranges(S)
+    pool = np.sort(rng.permutation(unique_keys(rng, 3 * n, S)))
+    sets = []
+    for i in range(3):
+        lens = (rng.integers(1, 33, n) * (1 if i == 2 else 4)).astype(np.int32)
+        sets.append((pool[i::3], lens))
+    for which in (0, 0, 0, 0, 1, 0, 2, 2, 2, 1, 2, 0, 0, 0):
+        keys, lens = sets[which]
+        total = int(lens.sum())
+        pos, val_pos, _ = orc.slice_keys(keys, begin, end, lens, total)
+        vals = rng.standard_normal(total).astype(np.float32)
+        out = torch.full((total,), 7.0, device=dev)
+        out_lens = torch.zeros(n, dtype=torch.int32, device=dev)
+        d_keys, d_lens = to_dev(keys, dev), to_dev(lens, dev)
+        group.push(d_keys, pos, to_dev(vals, dev), val_pos, lens=d_lens)
+        group.pull(d_keys, pos, out, out_pos=val_pos, out_lens=out_lens)
+        group.sync()
+        want = []
+        for s in range(S):
+            a, b, va, vb = int(pos[s]), int(pos[s + 1]), int(val_pos[s]), int(val_pos[s + 1])
+            stores[s].push(keys[a:b], vals[va:vb], lens[a:b])
+            want.append(stores[s].pull(keys[a:b])[0])
+        assert_bits_equal(out.cpu().numpy(), np.concatenate(want))
+        assert np.array_equal(out_lens.cpu().numpy(), lens)
+    group.close()
+
+
 @pytest.mark.parametrize("kind", ["push", "pull", "both"])
 @pytest.mark.parametrize("n", [1, 4096, 4097, 2_500_001])
 def test_cached_values_written_back_by_the_request_that_differs(capi, orc, dev, monkeypatch, kind, n):
