@@ -18,6 +18,7 @@
 #include <hip/hip_ext.h>
 
 #include "devpool.h"
+#include "growths.h"
 #include "host_common.h"
 #include "one_launch.h"
 #include "scan.h"
@@ -641,62 +642,56 @@ uint64_t grown_cap(const pskv_table* t, uint64_t keys_needed) {
   return std::max(want, t->cap * factor);
 }
 
-// Slot arrays that are to move, all tables' of a request with as few launches as there can be. They do so before
-// anything else of the request, when move() is called or, where a request ends early, when the list goes.
+// The slot arrays that are to move for a request (growths.h). They do so before anything else of it, when move() is called or,
+// where it ends early, when the list goes.
 struct Growths {
-  struct One {
-    pskv_table* t;
-    Slot* from;
-    uint64_t cap;  // of `from`; t has the array and the size that it moves to
-  };
-  std::vector<One> list;
+  std::vector<Growth<pskv_table, Slot>> list;
   int move();
   ~Growths() { (void)move(); }
 };
 
-int Growths::move() {
-  std::vector<One> todo;
-  todo.swap(list);
-  int rc = PSKV_OK;
-  for (size_t first = 0; first < todo.size() && !rc;) {
+struct GrowthLaunches {
+  int scatter(const Growth<pskv_table, Slot>& g) {  // (a small table that a large request makes much larger)
+    pskv_table* t = g.t;
+    PSKV_HIP(hipMemsetAsync(t->slots, 0xFF, t->cap * sizeof(Slot), t->stream));
+    return launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(g.cap, kBlock, kMaxGrid)), dim3(kBlock), 0,
+                  (const Slot*)g.from, g.cap, t->slots, t->cap - 1, t->st);
+  }
+  // two streaming passes: the new array is written whole, slot by slot, from LDS
+  int stream(Growth<pskv_table, Slot>* const* some, unsigned count, bool& begun) {
     RegrowBatch b;
     std::memset(&b, 0, sizeof(b));
-    pskv_table* lead = todo[first].t;
+    pskv_table* lead = some[0]->t;
     uint64_t most = 0, factors = 0;
-    unsigned count = 0;
-    for (; first < todo.size() && count < (unsigned)kMaxBatch && !rc; ++first) {
-      const One& g = todo[first];
-      pskv_table* t = g.t;
-      const uint64_t factor = t->cap / g.cap;
-      if (factor > (uint64_t)kRegrowMaxFactor) {
-        // (a small table that a large request makes much larger: fill and scatter)
-        if (hipMemsetAsync(t->slots, 0xFF, t->cap * sizeof(Slot), t->stream) != hipSuccess)
-          rc = set_error(PSKV_EHIP, "hipMemsetAsync failed");
-        if (!rc)
-          rc = launch(t, PSKV_KERNEL_REHASH, k_rehash, dim3(grid_for(g.cap, kBlock, kMaxGrid)), dim3(kBlock), 0,
-                      (const Slot*)g.from, g.cap, t->slots, t->cap - 1, t->st);
-        continue;
-      }
-      b.t[count++] = RegrowOf{g.from, t->slots, g.cap - 1, t->cap - 1, t->st, factor};
+    for (unsigned i = 0; i < count; ++i) {
+      const Growth<pskv_table, Slot>& g = *some[i];
+      const uint64_t factor = g.t->cap / g.cap;
+      b.t[i] = RegrowOf{g.from, g.t->slots, g.cap - 1, g.t->cap - 1, g.t->st, factor};
       most = std::max(most, g.cap);
       factors = std::max(factors, factor);
     }
-    if (!count || rc) continue;
-    // two streaming passes: the new array is written whole, slot by slot, from LDS
     const unsigned nblk = (unsigned)(most / kRegrowOld);
     const size_t lds = (size_t)kRegrowOld * factors * 2 * sizeof(unsigned long long);
-    rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk, count), dim3(kBlock), lds, b);
-    if (!rc)
-      rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock, count),
+    int rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow, dim3(nblk, count), dim3(kBlock), lds, b);
+    if (rc) return rc;
+    begun = true;
+    return launch(lead, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((nblk * kRestLanes + kBlock - 1) / kBlock, count),
                   dim3(kBlock), 0, b);
   }
-  for (const One& g : todo) {
+  int release(pskv_table* t, Slot* slots) {
     const auto r0 = std::chrono::steady_clock::now();
-    const int gone = array_release(g.from, g.t->stream);
-    g.t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
-    if (!rc) rc = gone;
+    const int rc = array_release(slots, t->stream);
+    t->stats.release_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - r0).count();
+    return rc;
   }
-  return rc;
+};
+
+int Growths::move() {
+  if (list.empty()) return PSKV_OK;
+  std::vector<Growth<pskv_table, Slot>> todo;
+  todo.swap(list);
+  GrowthLaunches launches;
+  return move_growths(todo, (unsigned)kMaxBatch, (uint64_t)kRegrowMaxFactor, launches);
 }
 
 int grow_slots(pskv_table* t, uint64_t keys_needed, Growths* growths) {
@@ -727,7 +722,7 @@ int grow_slots(pskv_table* t, uint64_t keys_needed, Growths* growths) {
   }
   t->spare = nullptr;
   t->spare_cap = 0;
-  growths->list.push_back({t, t->slots, t->cap});
+  growths->list.push_back({t, t->slots, t->cap, false});
   t->slots = fresh;
   t->cap = want;
   return PSKV_OK;
