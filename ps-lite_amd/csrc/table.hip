@@ -13,6 +13,7 @@
 #include <string>
 #include <thread>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -712,7 +713,7 @@ int grow_slots(pskv_table* t, uint64_t keys_needed, Growths* growths) {
     want = t->spare_cap;
   } else {
     if (t->spare) {  // too small after all
-      rc = array_release(t->spare, t->stream);
+      rc = array_release(std::exchange(t->spare, nullptr), t->stream);
       if (rc) return rc;
     }
     const auto a0 = std::chrono::steady_clock::now();
