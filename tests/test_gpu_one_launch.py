@@ -397,30 +397,37 @@ def test_slices_without_lens(capi, orc, dev, n, S):
 @pytest.mark.parametrize("n", [2049, 70_000])
 def test_slices_with_lens_of_any_size_and_order(capi, orc, dev, n):
     """Ranges without keys that end where they begin, lens whose sums need all the bits of a part's word and negative ones;
-    and keys that are not sorted, which give no slices worth having but an answer, and leave the next call alone."""
+    and keys that are not sorted, which give no slices worth having but an answer, and leave the next call alone, which is one
+    of the same keys in order. Refused is what the oracle refuses."""
     announce("few slices, lens of any size", n)
     rng = np.random.default_rng(n)
     keys = unique_keys(rng, n, 4)
     cut = [0, int(keys[n // 3]), int(keys[n // 3]), int(keys[2 * n // 3]) + 1, 2**64 - 1]
     begin, end = np.array(cut[:-1], np.uint64), np.array(cut[1:], np.uint64)
-    for lens in (np.full(n, 2**31 - 1, np.int32), rng.integers(-2**31, 2**31, n).astype(np.int32) | 1):
-        nvals = max(0, int(lens.astype(np.int64).sum()))
-        for shuffled in (False, True):
-            k = rng.permutation(keys) if shuffled else keys
-            results = []
-            for who, arrays in ((capi, (to_dev(k, dev), to_dev(lens, dev))), (orc, (k, lens))):
-                try:
-                    if who is capi:
-                        results.append(capi.slice_keys(arrays[0], begin, end, lens=arrays[1], nvals=nvals))
-                    else:
-                        results.append(orc.slice_keys(arrays[0], begin, end, arrays[1], nvals))
-                except Exception as e:
-                    results.append(type(e).__name__)
-            if not shuffled and not isinstance(results[0], str):
-                for a, b in zip(*results):
-                    assert np.array_equal(np.asarray(a), np.asarray(b))
-            elif not shuffled:
-                assert isinstance(results[1], str), results
+    d_keys, d_shuffled = to_dev(keys, dev), to_dev(rng.permutation(keys), dev)
+
+    def sliced(slice_keys, error, *args, **more):
+        try:
+            return slice_keys(*args, **more)
+        except error as e:
+            return e.code
+
+    largest, some = np.full(n, 2**31 - 1, np.int32), rng.integers(-300, 1000, n).astype(np.int32)
+    for lens, short in ((largest, 0), (largest, 1), (some, 0), (rng.integers(-2**31, 2**31, n).astype(np.int32) | 1, 0)):
+        nvals, d_lens = max(0, int(lens.astype(np.int64).sum()) - short), to_dev(lens, dev)
+        want = sliced(orc.slice_keys, orc.OracleError, keys, begin, end, lens, nvals)
+        refused = isinstance(want, int)
+        assert refused or not short
+        for k in (d_keys, d_shuffled, d_keys):
+            got = sliced(capi.slice_keys, capi.PskvError, k, begin, end, lens=d_lens, nvals=nvals)
+            if k is d_shuffled:
+                continue
+            if refused:
+                assert got == want
+                continue
+            assert not isinstance(got, int), got
+            for a, b in zip(got, want):
+                assert np.array_equal(np.asarray(a), np.asarray(b))
 
 
 @pytest.mark.parametrize("mode", ["scalar", "fixed", "varlen"])
