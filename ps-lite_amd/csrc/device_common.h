@@ -101,8 +101,8 @@ struct alignas(32) DevState {
   // the value of dirty_epoch up to which the slots have been brought up to date since
   unsigned long long dirty_epoch;
   unsigned long long clean_epoch;
-  // the write-back that k_scalar does itself: pieces given away and pieces written (k_same_keys clears both)
-  unsigned int flush_next, flush_done;
+  // the newest request that found cached values ahead of the slots and named other keys (k_scalar<BEHIND>)
+  unsigned long long behind_epoch;
   // k_scalar_repeat: votes of the launch in flight (vote.h), and launches served so far << 1 | verdict of the newest
   unsigned int repeat_arrived;
   unsigned int told_ragged;  // what the host has been told of the rows of var-len pushes (tell_ragged)

@@ -605,9 +605,8 @@ int flush_scalar_cache(pskv_table* t) {
   d.n = t->cache_n;
   d.arena = static_cast<float*>(t->sc_vals.ptr);
   d.tile_key = static_cast<uint32_t*>(t->sc_slots.ptr);
-  d.cache_mode = kFlushAlways;
   d.nblk = grid_for(t->cache_n, kBlock, kFlushGrid);
-  hipLaunchKernelGGL(k_scalar_flush<1>, dim3(d.nblk, 1), dim3(kBlock), 0, t->stream, rb);
+  hipLaunchKernelGGL(k_scalar_flush, dim3(d.nblk, 1), dim3(kBlock), 0, t->stream, rb);
   PSKV_HIP(hipGetLastError());
   t->sc_dirty = false;
   return PSKV_OK;
@@ -958,9 +957,6 @@ struct Item {
   // var-len workspace of the request
   int32_t* tmp_lens = nullptr;
   uint64_t nparts = 0, tiles_cap = 0;
-  // SCALAR: the slots may lag behind the key cache and must be written back if the device finds
-  // that this request does not repeat the cached keys
-  bool flush_unless_same = false;
 };
 typedef std::vector<Item> Batch;
 
@@ -1194,11 +1190,8 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       const bool per_key = use[i] == kScTry && !push && !t->sc_dirty && kind_before == 0 && r.replay != kReplayCapture;
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
-      // (a recorded repeat is served from the cache or not at all: nothing to write back first)
-      it.flush_unless_same = !per_key && it.tag.try_cache && t->sc_dirty && r.replay != kReplayCapture;
-      // (expected to repeat it: the request's own kernel writes them back if need be)
-      if (it.flush_unless_same && t->sc_track[r.push ? 0 : 1].hit) {
-        it.flush_unless_same = false;
+      // (a recorded repeat is served from the cache or not at all: nothing to write back)
+      if (!per_key && it.tag.try_cache && t->sc_dirty && r.replay != kReplayCapture) {
         d.cache_mode = kCacheOnBehind;
         behind = true;
       }
@@ -1237,13 +1230,6 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
       return ((it.d.cache_mode == kCacheOn || it.d.cache_mode == kCacheOnBehind) && it.tag.try_cache)
                  ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems) : 0ull;
-    });
-    if (rc) return rc;
-    // slots that lag behind the cache are written back once the device knows that the request
-    // does NOT repeat the cached keys (cache_mode reads as kFlushUnlessSame in that kernel)
-    static_assert(kFlushUnlessSame == kCacheOn, "one descriptor serves both kernels");
-    rc = launch_batch(bt, -1, PSKV_KSET(k_scalar_flush), [](const Item& it) {
-      return it.flush_unless_same ? (uint64_t)grid_for(it.r.n, kBlock, kFlushGrid) : 0ull;
     });
     if (rc) return rc;
   }

@@ -72,9 +72,8 @@ constexpr uint32_t kCacheOff = 0;     // SCALAR: the request neither uses nor fi
 constexpr uint32_t kCacheOn = 1;      // SCALAR: serve from the cache when the keys match, else refill it
 constexpr uint32_t kCachePerKey = 3;  // SCALAR pull, slots up to date: every key that sits at its cached
                                       // position is answered from the cache, the others through the slots
-constexpr uint32_t kCacheOnBehind = 4;  // SCALAR: as kCacheOn, and the slots may lag behind the cache (k_scalar<BEHIND>)
-constexpr uint32_t kFlushUnlessSame = 1;  // k_scalar_flush: skip when the request in flight repeats the cache
-constexpr uint32_t kFlushAlways = 2;
+constexpr uint32_t kCacheOnBehind = 5;  // SCALAR: as kCacheOn, and the slots may lag behind the cache (k_scalar<BEHIND>)
+constexpr uint32_t kCacheRecords = 3;   // the bits that say so: a request that is served from the cache, or fills it
 constexpr uint32_t kSlotSpecial = 0xffffffffu;  // cached slot number of key 2^64-1 (the side slot)
 // Every kernel comes for one, for up to four and for up to kMaxBatch tables: an argument of 3.8 KB costs the
 // calling thread 4.6 us per launch, one of 240 bytes 3.
@@ -125,47 +124,15 @@ __device__ __forceinline__ void arrived(T& x) {
 // (about 2 us): everything the lane needs of it is asked for at once, the neighbours of the wavefront's
 // first and last key included. (From device memory the plain order is 2 % faster: those two reads are
 // mostly in the cache by the time they are made.)
-// BEHIND: the request is expected to repeat the cached one, and the cached values may be ahead of the slots. Should it
-// name other keys after all, its workgroups write them back first (write_back_together). Usually there is nothing to
-// write back, and a launch in front of every request that found that out took 4.7 us of the 70 of 16M keys.
-constexpr unsigned kWriteBackPiece = kBlock * 16;  // cached values
-__device__ __forceinline__ void write_back_together(const TableHead& d) {
-  DevState* st = d.st;
-  const unsigned long long dirty = st->dirty_epoch;  // (nothing changes it in this launch)
-  auto clean = [&] { return __hip_atomic_load(&st->clean_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  __shared__ unsigned s_piece;
-  const unsigned pieces = (unsigned)((d.n + kWriteBackPiece - 1) / kWriteBackPiece);
-  // Whoever is on the GPU takes pieces until all are given away, and waits then for those that others have: they are
-  // running, whichever workgroups have not started yet. Past the L2, for the other XCDs.
-  for (;;) {
-    __syncthreads();
-    if (threadIdx.x == 0) s_piece = clean() >= dirty ? pieces : atomicAdd(&st->flush_next, 1u);
-    __syncthreads();
-    const unsigned piece = s_piece;
-    if (piece >= pieces) break;
-    for (unsigned j = 0; j < kWriteBackPiece / kBlock; ++j) {
-      const uint64_t i = (uint64_t)piece * kWriteBackPiece + j * kBlock + threadIdx.x;
-      if (i >= d.n) break;
-      const uint32_t slot = d.tile_key[i];
-      float* dst = slot == kSlotSpecial ? reinterpret_cast<float*>(&st->special_payload)
-                                        : reinterpret_cast<float*>(&d.slots[slot].payload);
-      __hip_atomic_store(dst, d.arena[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(&st->flush_done, 1u) == pieces - 1)
-      __hip_atomic_store(&st->clean_epoch, dirty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (threadIdx.x == 0) {
-    while (clean() < dirty) __builtin_amdgcn_s_sleep(8);
-    __threadfence();  // nothing stale is left in this XCD's L2
-  }
-  __syncthreads();
-}
-
+// BEHIND: the cached values may be ahead of the slots. Should the request name other keys than the cached one, k_same_keys has
+// written back those of the positions where it does, which may be anybody's here; a position where it does not is this lane's
+// alone, which takes the value from the cache. (Usually the request names the same keys: a launch in front of every request
+// that found out whether there is something to write back took 4.7 us of the 75 of 16M keys and 4.3 of the 12.8 of 500,000.
+// Workgroups that wrote everything back here and waited for each other took 706 us for 4M other keys, now 202 behind 98.)
+// (Eight wavefronts per SIMD, said to the compiler: it came to 7 for pulls with BEHIND, 4M keys 20.4 us and not 20.0, and to
+// 24.0 and not 23.0 for pushes.)
 template <bool PUSH, bool PULL, bool CACHE, bool PINNED, bool BEHIND, int TABLES>
-__global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
+__global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
   const TableHead& d = b.t[blockIdx.y];
   const uint64_t n = d.n;
   const unsigned nblk = d.nblk;  // (the grid is sized for the table with the most workgroups)
@@ -176,9 +143,9 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
   const uint64_t* __restrict__ keys = d.keys;
   const float* __restrict__ vals = d.vals;
   float* __restrict__ out = d.out;
-  const bool record = CACHE && (d.cache_mode == kCacheOn || (BEHIND && d.cache_mode == kCacheOnBehind));
+  const bool record = CACHE && (d.cache_mode & kCacheRecords) == kCacheOn;
   if (CACHE && replay_blocked(st, d.tag)) return;
-  if (record && cache_same(st, d.tag)) {
+  if (record && __builtin_expect(cache_same(st, d.tag), BEHIND)) {
     // the keys are those of the cached request: position i of the request is position i of the cache
     float* __restrict__ cv = d.arena;
     if (PUSH && blockIdx.x == 0 && threadIdx.x == 0) st->dirty_epoch = d.tag.epoch;  // the slots fall behind
@@ -203,7 +170,7 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
     if (d.snap && blockIdx.x == 0 && threadIdx.x < 64) publish_snapshot(st, d.snap, d.snap_seq);
     return;
   }
-  if (BEHIND && d.cache_mode == kCacheOnBehind) write_back_together(d);
+  const bool ahead = BEHIND && d.cache_mode == kCacheOnBehind && st->behind_epoch == d.tag.epoch;
   if (record && blockIdx.x == 0 && threadIdx.x == 0) st->cache_epoch = d.tag.epoch;
   constexpr bool kPerKey = CACHE && PULL && !PUSH;
   bool per_key = false, differs = false;
@@ -295,13 +262,22 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
     if (!live || (i > 0 && before == key)) continue;  // past the end, or inside a run
     const bool run = i + 1 < n && after == key;
     if (PUSH && !PINNED) v = vals[i];
+    bool held = false;  // the cached value is the key's
+    float held_value = 0.0f;
+    if (BEHIND && ahead) {
+      uint64_t at = i;  // (a run names the cached key of one of its positions at most)
+      if (run)
+        while (at + 1 < n && keys[at + 1] == key && d.cache_keys[at] != key) ++at;
+      held = d.cache_keys[at] == key;
+      held_value = d.arena[at];
+    }
     bool is_new;
     uint64_t seen;
     uint64_t* p = find_or_insert(slots, mask, st, key, is_new, seen);
     if (record && (!p || run)) st->bad_epoch = d.tag.epoch;  // not a request the cache can stand for
     if (!p) continue;
     // an absent key starts from Val() == 0, then `+=` (kv_app.h:454): 0.0f + v, not a copy
-    float cur = is_new ? 0.0f : __uint_as_float((unsigned)seen);
+    float cur = is_new ? 0.0f : held ? held_value : __uint_as_float((unsigned)seen);
     if (PUSH) cur = cur + v;
     if (PULL) out[i] = cur;
     if (run) {  // the rest of the run, element by element like the reference's loop
@@ -310,7 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
         if (PULL) out[j] = cur;
       }
     }
-    if (PUSH || is_new) *reinterpret_cast<float*>(p) = cur;
+    if (PUSH || is_new || held) *reinterpret_cast<float*>(p) = cur;
     created += is_new ? 1u : 0u;
     if (record) {
       d.cache_keys[i] = key;
@@ -350,27 +326,28 @@ __global__ __launch_bounds__(kBlock) void k_scalar(HeadBatch<TABLES> b) {
   }
 }
 
+// Writes a cached value back to its slot.
+__device__ __forceinline__ void write_back(const TableHead& d, uint64_t i) {
+  const uint32_t slot = d.tile_key[i];
+  const float v = d.arena[i];
+  float* dst = slot == kSlotSpecial ? reinterpret_cast<float*>(&d.st->special_payload)
+                                    : reinterpret_cast<float*>(&d.slots[slot].payload);
+  *dst = v;
+}
+
 // Writes the cached values back to their slots. Launched before anything reads or changes the
-// slots of a table whose cache may be ahead of them: a request that does not repeat the cached
-// keys (kFlushUnlessSame: the comparison of that request has run), a growth, a dump.
-template <int TABLES>
-__global__ __launch_bounds__(kBlock) void k_scalar_flush(HeadBatch<TABLES> b) {
-  const TableHead& d = b.t[blockIdx.y];
+// slots of a table whose cache may be ahead of them: a request that is not compared with the cached
+// one, a growth, a dump.
+__global__ __launch_bounds__(kBlock) void k_scalar_flush(HeadBatch<1> b) {
+  const TableHead& d = b.t[0];
   if (blockIdx.x >= d.nblk) return;
   // nothing changes these two while this kernel runs except its own last workgroup, which writes
   // after every workgroup has read them
   const unsigned long long dirty = d.st->dirty_epoch;
   if (dirty <= d.st->clean_epoch) return;  // the slots are up to date
-  if (d.cache_mode == kFlushUnlessSame && (cache_same(d.st, d.tag) || d.tag.replay)) return;
   __shared__ unsigned s_last;
   const uint64_t stride = (uint64_t)d.nblk * kBlock;
-  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < d.n; i += stride) {
-    const uint32_t slot = d.tile_key[i];
-    const float v = d.arena[i];
-    float* dst = slot == kSlotSpecial ? reinterpret_cast<float*>(&d.st->special_payload)
-                                      : reinterpret_cast<float*>(&d.slots[slot].payload);
-    *dst = v;
-  }
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < d.n; i += stride) write_back(d, i);
   if (threadIdx.x == 0) s_last = ticket_last(d.st, d.nblk) ? 1u : 0u;
   __syncthreads();
   if (s_last && threadIdx.x == 0) d.st->clean_epoch = dirty;
@@ -445,6 +422,16 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
   bool differ = false;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) differ |= a[j] != c[j];
+  // Cached values that are ahead of the slots go back where the keys differ (a position past the end does not: both are 0).
+  // The request's own kernel sees to the others; which way it goes is not known here. (Nothing changes these two words in
+  // this launch before every workgroup has taken its ticket.)
+  if (__builtin_expect(differ, 0)) {
+    if (d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch) {
+#pragma unroll
+      for (int j = 0; j < kItems; ++j)
+        if (a[j] != c[j]) write_back(d, base + j);
+    }
+  }
   const int any = __syncthreads_or(differ ? 1 : 0);
   if (threadIdx.x == 0) {
     if (any) report_facts(st, kReqDiffer, d.nblk);
@@ -455,7 +442,10 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
   if (threadIdx.x >= 64) return;
   const bool same = (take_facts(st, d.nblk) & kReqDiffer) == 0u && cache_usable(st, tag);
   if (threadIdx.x == 0) {
-    st->flush_next = st->flush_done = 0;
+    if (!same && d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch) {
+      st->behind_epoch = tag.epoch;
+      st->clean_epoch = st->dirty_epoch;  // (by the end of the request)
+    }
     decide_same(st, tag, same, d.outcome);
   }
 }

@@ -356,6 +356,55 @@ def test_cached_values_written_back_by_the_request_that_differs(capi, orc, dev, 
     assert_bits_equal(t.dump()[2], o.dump()[2])
 
 
+@pytest.mark.parametrize("kind", ["push", "pull", "both"])
+@pytest.mark.parametrize("n", [2, 5, 1023, 1025, 70_001])
+def test_cached_values_of_keys_that_stay_where_they_are(capi, orc, dev, monkeypatch, kind, n):
+    """The slots lag behind the cache, and the request that differs names most keys at their cached positions, one or a few at
+    others, or one of them twice, with the cached position in front or behind."""
+    import torch
+    announce("write back, some stay", kind, n)
+    monkeypatch.setenv("PSKV_SCALAR_CACHE_MIN_KEYS", "1")
+    rng = np.random.default_rng(n)
+    pool = unique_keys(rng, 2 * n)
+    pool[-1] = 2**64 - 1
+    base = pool[::2].copy()
+    base[-1] = pool[-1]
+    others = []
+    for j in sorted({0, n // 2, n - 1}):
+        other = base.copy()
+        other[j] = pool[2 * j] + np.uint64(1) if 2 * j + 1 < 2 * n and pool[2 * j] + np.uint64(1) < pool[2 * j + 1] else other[j]
+        others.append(other)
+        if j + 1 < n:
+            for a, b in ((j, j + 1), (j + 1, j)):  # the key at b stands at both
+                other = base.copy()
+                other[a] = base[b]
+                others.append(other)
+            other = base.copy()  # everything behind j moves by one
+            other[j + 1:] = base[j:-1]
+            other[j] = base[j - 1] if j else base[0]
+            others.append(np.sort(other))
+    for turn, other in enumerate(others):
+        t, o = capi.Table(capi.MODE_SCALAR), orc.Store(orc.MODE_SCALAR)
+        for keys in (base, base, base, base, other):
+            vals = rng.standard_normal(n).astype(np.float32)
+            out = torch.zeros(n, device=dev)
+            torch.cuda.synchronize()
+            if kind == "both":
+                t.pushpull(to_dev(keys, dev), to_dev(vals, dev), out)
+                want = o.handle(True, True, keys, vals, out_cap=n)[1]
+            elif kind == "push" or keys is base:
+                t.push(to_dev(keys, dev), to_dev(vals, dev))
+                o.push(keys, vals)
+                continue
+            else:
+                t.pull(to_dev(keys, dev), out)
+                want = o.pull(keys)[0]
+            t.sync()
+            assert_bits_equal(out.cpu().numpy(), want, "turn %d" % turn)
+        t.sync()
+        assert_bits_equal(t.dump()[2], o.dump()[2], "turn %d" % turn)
+
+
 @pytest.mark.parametrize("S", [1, 3, 16, 31])
 @pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 30_001, 128 * 2048 + 1, 512 * 2048, 512 * 2048 + 1])
 def test_slices_with_lens_of_few_keys(capi, orc, dev, n, S):
