@@ -25,16 +25,17 @@ constexpr unsigned kVarParts = 256;
 constexpr uint64_t kStartFloats = 24u << 20;
 // Of a request that repeats the cached one two launches are short, for the second returns at once (100,000 rows over 16
 // tables, push and pull: 51 us against 54; pulls of 65,536 rows of 64 floats 16.3 -> 15.0 with one, of 256 31.1 -> 33.3; pushes
-// of 65,536 ragged rows of 45 in one table 23.9 -> 25.4 and 33.0 -> 35.2 with a wait behind each, of 20,000 17.9 -> 17.1 and
-// 27.8 -> 28.3, of 65,536 over 16 27.5 -> 23.8 and 37.1 -> 37.0).
+// of 65,536 ragged rows of 45 in one table 23.9 -> 25.4 and 33.0 -> 35.2 with a wait behind each, of 40,000 20.3 -> 19.2 and
+// 28.8 -> 29.9, of 65,536 over 16 27.5 -> 23.8 and 37.1 -> 37.0).
 constexpr uint64_t kStartRepeatKeys = 1u << 16, kStartRepeatFloats = 1u << 23;
 constexpr unsigned kStartFewTables = 4;
-constexpr uint64_t kStartRepeatKeysFew = 1u << 15;  // of a push
+constexpr uint64_t kStartRepeatKeysFew = 3u << 14;  // of a push
 // And k_var_push_start does not compare: it looks the keys up again, and the row kernel has no shortcut then (one table:
-// 65,536 rows of 64 floats 22.1 -> 26.6, of 1,024 153 -> 197, 20,000 of 256 22.7 -> 28.2, 5,000 of 64 13.2 -> 13.7 and 23.1 ->
-// 24.9 with a wait). That pays only where launches are most of a request, with several tables' arguments in each: push and pull
-// of 5,000 rows of 64 over four 23.3 -> 19.6, of 20,000 of 50 26.2 -> 24.8 but the push 11.8 -> 15.4; over 16, whose launches
-// carry 3.8 KB, 1,000 of 64 23 -> 18, pushes of 5,000 of 256 15.7 -> 15.6, of 20,000 of 64 15.3 -> 16.6.
+// 65,536 rows of 64 floats 22.1 -> 26.6 us, of 1,024 153 -> 197, 20,000 of 256 22.7 -> 28.2). That pays only where the
+// launches are most of a request: push and pull of 5,000 rows of 64 in one table 21.6 -> 19.7 and 32.1 -> 32.5 with a wait
+// behind each, over four 23.3 -> 19.6, slice, push and pull of 40,000 of 12 over three 26.5 -> 24.0 and 44.7 -> 46.3, but a
+// push of 20,000 of 50 over four 11.8 -> 15.4; over 16, whose launches carry 3.8 KB, push and pull of 1,000 of 64 23 -> 18,
+// pushes of 5,000 of 256 15.7 -> 15.6, of 20,000 of 64 15.3 -> 16.6.
 constexpr uint64_t kStartShortcutFloatsFew = 1u << 19, kStartShortcutFloats = 1u << 20;
 
 constexpr bool one_start(const StartOf& r) {
@@ -42,8 +43,7 @@ constexpr bool one_start(const StartOf& r) {
   if (!r.compared) return true;
   const bool few = r.tables <= kStartFewTables;
   if (r.keys > (r.push && few ? kStartRepeatKeysFew : kStartRepeatKeys) || r.floats > kStartRepeatFloats) return false;
-  if (!r.push || !r.shortcut) return true;
-  return r.tables > 1 && r.floats <= (few ? kStartShortcutFloatsFew : kStartShortcutFloats);
+  return !r.push || !r.shortcut || r.floats <= (few ? kStartShortcutFloatsFew : kStartShortcutFloats);
 }
 
 }  // namespace pskv
