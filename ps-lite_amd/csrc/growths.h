@@ -59,5 +59,23 @@ int move_growths(std::vector<Growth<Table, Slots>>& todo, unsigned most_tables, 
   return rc;
 }
 
+// The array that a table which needs `want` slots moves to: the spare one (`spare_cap` slots, or null) where that is large
+// enough, and `want` is its size then, or else a new one, and the spare goes. The table has no spare after it. Ops:
+//   int release(Slots*)     int allocate(uint64_t slots, Slots** fresh)
+template <typename Ops, typename Slots>
+int next_array(Slots*& spare, uint64_t& spare_cap, uint64_t& want, Slots*& fresh, Ops& ops) {
+  Slots* const was = spare;
+  const uint64_t cap = spare_cap;
+  spare = nullptr;
+  spare_cap = 0;
+  if (was && cap >= want) {
+    fresh = was;
+    want = cap;
+    return 0;
+  }
+  const int rc = was ? ops.release(was) : 0;
+  return rc ? rc : ops.allocate(want, &fresh);
+}
+
 }  // namespace pskv
 #endif  // PSKV_GROWTHS_H_

@@ -13,7 +13,6 @@
 #include <string>
 #include <thread>
 #include <tuple>
-#include <utility>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -706,22 +705,21 @@ int grow_slots(pskv_table* t, uint64_t keys_needed, Growths* growths) {
   }
   ++t->stats.growths;
   collect_spare(t, true);
-  if (t->spare && t->spare_cap >= want) {
-    ++t->stats.spare_used;
-    fresh = t->spare;
-    want = t->spare_cap;
-  } else {
-    if (t->spare) {  // too small after all
-      rc = array_release(std::exchange(t->spare, nullptr), t->stream);
-      if (rc) return rc;
+  struct {
+    pskv_table* t;
+    bool allocated;
+    int release(Slot* slots) { return array_release(slots, t->stream); }
+    int allocate(uint64_t n, Slot** to) {
+      allocated = true;
+      const auto a0 = std::chrono::steady_clock::now();
+      const int rc = alloc_slots(n, to, t->stream);
+      t->stats.alloc_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - a0).count();
+      return rc;
     }
-    const auto a0 = std::chrono::steady_clock::now();
-    rc = alloc_slots(want, &fresh, t->stream);
-    t->stats.alloc_us += std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - a0).count();
-    if (rc) return rc;
-  }
-  t->spare = nullptr;
-  t->spare_cap = 0;
+  } arrays{t, false};
+  rc = next_array(t->spare, t->spare_cap, want, fresh, arrays);
+  if (rc) return rc;
+  if (!arrays.allocated) ++t->stats.spare_used;
   growths->list.push_back({t, t->slots, t->cap, false});
   t->slots = fresh;
   t->cap = want;

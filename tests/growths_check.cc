@@ -44,6 +44,16 @@ struct Launches {
   }
 };
 
+struct Arrays {
+  Array* made;
+  int release_rc, allocate_rc;
+  int release(Array* a) { return ++a->released, release_rc; }
+  int allocate(uint64_t, Array** to) {
+    if (!allocate_rc) *to = made;
+    return allocate_rc;
+  }
+};
+
 int main(int argc, char** argv) {
   const bool forget = argc > 1 && !strcmp(argv[1], "--forget");
   for (unsigned tables : {0u, 1u, 3u, 16u, 17u, 40u}) {
@@ -76,6 +86,19 @@ int main(int argc, char** argv) {
         }
       }
     }
+  }
+  // the array that a table moves to: its spare one, or a new one, and where there is none no trace of the spare
+  for (int which = 0; which < 5; ++which) {
+    Array old, made;
+    Arrays ops{&made, which == 3 ? 5 : 0, which == 4 ? 6 : 0};
+    Array *spare = which == 0 ? nullptr : &old, *fresh = nullptr;
+    uint64_t cap = spare ? (which == 1 ? 512 : 128) : 0, want = 256;
+    const int rc = next_array(spare, cap, want, fresh, ops);
+    const bool large = which == 1, failed = which >= 3;
+    if (rc != (which == 3 ? 5 : which == 4 ? 6 : 0) || spare || cap) return printf("spare left: %d\n", which), 1;
+    if (old.released != (which >= 2 ? 1 : 0)) return printf("spare given back %d times\n", old.released), 1;
+    if (!failed && (fresh != (large ? &old : &made) || want != (large ? 512u : 256u))) return printf("array %d\n", which), 1;
+    if (failed && fresh) return printf("an array in spite of everything\n"), 1;
   }
   printf("ok\n");
   return 0;
