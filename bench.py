@@ -357,7 +357,7 @@ def run_sparse_lr(args, capi, dev):
                                      traffic("pull_scalar", keys_per_launch),
                                      traffic("pull_per_key", keys_per_launch)),
                         growth={"launches": st["growth"][0], "total_us": round(st["growth"][1] * 1e3, 1),
-                                "note": "k_regrow + k_regrow_rest of the sampled steps only"}),
+                                "note": "growths, and pushes that stream through the slots, of the sampled steps only"}),
     }
     if not args.no_extra:
         # the same steps on tables sized up front for every key of the run (no growth, lower fill)
@@ -866,9 +866,11 @@ def run_zipf(args, capi, dev, pushes=8):
                          bytes_per_key=28),
         # between a hit (28 B/key) and an insert (32 B/key); priced as inserts
         "kernels": {"push_scalar": dict(roofline(32.0 * n, push[0], push[1], traffic("push_scalar_zipf", n), push[2]),
-                                        kernel="k_scalar<push> (find-or-insert + add), 4M keys", bytes_per_key=32),
+                                        kernel="k_scalar<push> (find-or-insert + add), 4M keys, the pushes that go through the slots",
+                                        bytes_per_key=32),
                     "growth": {"launches": rehash[0], "total_us": round(rehash[1] * 1e3, 1),
-                               "kernels": "k_regrow + k_regrow_rest per growth"}},
+                               "kernels": "pushes that stream through the slots or make them grow: k_split, k_stream_push, "
+                                          "k_regrow_rest, k_push_left"}},
     }
     return res, (batches, probe)
 

@@ -73,7 +73,7 @@ extern "C" {
 #define PSKV_KERNEL_ROWS_ACC 2    /* push accumulate of rows (fixed-k and var-len) */
 #define PSKV_KERNEL_ROWS_GATHER 3 /* pull gather of rows */
 #define PSKV_KERNEL_LOOKUP 4      /* key -> row lookup / insert of the row modes */
-#define PSKV_KERNEL_REHASH 5
+#define PSKV_KERNEL_REHASH 5      /* passes over the slot array: growths, and pushes that stream through it */
 #define PSKV_KERNEL_COPY 6        /* the plain copy of pskv_copy_probe */
 #define PSKV_KERNEL_SAME_KEYS 7   /* comparison of a request's keys with the cached key set */
 #define PSKV_KERNEL_PULL_PER_KEY 8 /* SCALAR pull right behind the push that filled the key cache: keys

@@ -13,7 +13,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libpskv.so")
 NATIVE = os.path.join(HERE, "_native.so")
 SOURCES = ["table.hip", "slice.hip", "hostmem.hip", "stager.hip", "devpool.hip", "match.hip", "meta_codec.cc"]
-HEADERS = ["device_common.h", "devpool.h", "growths.h", "handover.h", "host_common.h", "one_launch.h", "parts.h", "quads.h", "scan.h", "search.h", "stager.h", "start_rule.h", "stream_choice.h", "table_kernels.h", "vote.h"]
+HEADERS = ["device_common.h", "devpool.h", "growths.h", "handover.h", "host_common.h", "one_launch.h", "parts.h", "quads.h", "scan.h", "search.h", "stager.h", "start_rule.h", "stream_choice.h", "stream_push.h", "stream_rule.h", "table_kernels.h", "vote.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -118,7 +118,12 @@ struct alignas(32) DevState {
   unsigned long long fresh_from;
   // k_fixed_own: a bit for every workgroup of a push that has left its rows to the last one, all zero between requests
   unsigned long long shares_left[8];
-  unsigned long long pad[6];
+  // stream_push.h: keys that the pass over the slots leaves to the kernel behind it (requests use the two in turn, the one that
+  // is not in use is zero), and the sum of the hashes of the keys of the newest such request (of the one in flight: next to
+  // each word of count_shard)
+  unsigned left_keys[2];
+  unsigned long long keys_sum;
+  unsigned long long pad[4];
   // one_launch.h: what the workgroups of a var-len request tell each other, all zero between requests
   unsigned long long parts[kVarParts];
 };

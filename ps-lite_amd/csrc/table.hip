@@ -23,6 +23,8 @@
 #include "one_launch.h"
 #include "scan.h"
 #include "stager.h"
+#include "stream_push.h"
+#include "stream_rule.h"
 #include "table_kernels.h"
 
 namespace pskv {
@@ -336,7 +338,7 @@ struct pskv_table {
   uint64_t arena_cap = 0;  // floats
   uint64_t row_len = 0;    // FIXED
 
-  GrowBuf ws;         // per-request workspace (row references, offsets)
+  GrowBuf ws;         // per-request workspace (row references, offsets; SCALAR: keys by bin, stream_push.h)
   GrowBuf tiles;      // VARLEN: first key of every request-side tile
   GrowBuf tiles_aff;  // VARLEN: one TileNote per tile
   Shell* shell = nullptr;     // what st, st_host, snap, outcome and small_* belong to
@@ -398,6 +400,8 @@ struct pskv_table {
   unsigned long long sc_seen = 0;         // the value of *outcome the host last looked at
   unsigned push_looks = 0;                // k_fixed_own: how often a workgroup looks for the verdict
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
+  int streams = -1;                       // pushes stream through the slot array: where it pays, or (0, 1) never, wherever they can
+  unsigned stream_turn = 0;               // the counter of left keys that the newest of them used
 
   bool prof = false;
   std::vector<EventPair> pending[PSKV_KERNEL_COUNT];
@@ -665,7 +669,7 @@ struct GrowthLaunches {
     for (unsigned i = 0; i < count; ++i) {
       const Growth<pskv_table, Slot>& g = *some[i];
       const uint64_t factor = g.t->cap / g.cap;
-      b.t[i] = RegrowOf{g.from, g.t->slots, g.cap - 1, g.t->cap - 1, g.t->st, factor};
+      b.t[i] = RegrowOf{g.from, g.t->slots, g.cap - 1, g.t->cap - 1, g.t->st, factor, kRegrowOld};
       most = std::max(most, g.cap);
       factors = std::max(factors, factor);
     }
@@ -1093,6 +1097,9 @@ bool scalar_cache_eligible(const pskv_table* t, const Request& r) {
   return t->sc_min_keys && r.n >= t->sc_min_keys && t->cap < (1ull << 32);
 }
 
+// pulls have been following the pushes of their keys and are not in a spell of failed comparisons
+bool pulls_follow(const pskv_table* t) { return t->sc_pairs >= 2 && t->sc_track[1].skip == 0; }
+
 ScalarCacheUse scalar_cache_use(pskv_table* t, const Request& r) {
   note_outcomes(t);
   const int kind = r.push ? 0 : 1;
@@ -1110,9 +1117,8 @@ ScalarCacheUse scalar_cache_use(pskv_table* t, const Request& r) {
       use = kScTry;
     } else if (kind == 0) {
       // a push is worth recording when its size repeats (the same keys may be coming again) or
-      // when pulls have been following the pushes and are not in a spell of failed comparisons
-      const bool pulls_follow = t->sc_pairs >= 2 && t->sc_track[1].skip == 0;
-      if ((compare && size_repeats) || pulls_follow) use = kScRecord;
+      // when pulls have been following the pushes
+      if ((compare && size_repeats) || pulls_follow(t)) use = kScRecord;
     } else if (compare && size_repeats && t->sc_last_kind == 1) {
       use = kScRecord;  // a pull behind a pull of the same size
     }
@@ -1122,11 +1128,150 @@ ScalarCacheUse scalar_cache_use(pskv_table* t, const Request& r) {
   return use;
 }
 
+// How a table's share of a SCALAR request is going to be served.
+struct ScalarPlan {
+  ScalarCacheUse use = kScPlain;
+  int kind_before = -1;  // of the request in front of it (pskv_table::sc_last_kind)
+  bool may_stream = false, streams = false;
+};
+
+// A table's share of a push that streams through its slot array.
+struct Streamed {
+  Item* it;
+  Growth<pskv_table, Slot> g;  // of the table, if `grows`
+  bool grows;
+  StreamShape shape;
+  uint32_t tiles() const { return (uint32_t)((it->r.n + kSplitTile - 1) / kSplitTile); }
+};
+
+size_t stream_room(const Streamed& s) {
+  return Carver::need((size_t)s.tiles() * kTileWords, 8) +
+         Carver::need((size_t)s.tiles() * (s.shape.bins + kStartsPad), 2) + Carver::need(s.it->r.n, sizeof(LeftKey));
+}
+
+// Those tables' shares of a push; the slot arrays that move for it have been allocated, nothing has been moved.
+int stream_push(Batch& bt, std::vector<Streamed>& todo) {
+  pskv_table* lead = lead_of(bt);
+  StreamBatch all;
+  RegrowBatch rest;
+  std::memset(&all, 0, sizeof(all));
+  std::memset(&rest, 0, sizeof(rest));
+  // the tables by what their arrays do: stay, become twice as large, or more
+  struct Kind {
+    StreamBatch b;
+    unsigned tables = 0, most_bins = 0;
+  } kinds[3];
+  unsigned most_tiles = 0, n_grow = 0;
+  uint64_t most_keys = 0, most_rest = 0;
+  for (size_t i = 0; i < todo.size(); ++i) {
+    Streamed& s = todo[i];
+    Item& it = *s.it;
+    pskv_table* t = it.t;
+    StreamOf& d = all.t[i];
+    d.slots = t->slots;
+    d.mask = t->cap - 1;
+    d.old_slots = s.grows ? s.g.from : t->slots;
+    d.old_mask = (s.grows ? s.g.cap : t->cap) - 1;
+    d.st = t->st;
+    d.keys = it.r.keys;
+    d.vals = it.r.vals;
+    d.n = it.r.n;
+    d.tiles = s.tiles();
+    d.bins = s.shape.bins;
+    d.bin_bits = s.shape.bin_bits;
+    d.images = s.shape.images;
+    Carver c(t->ws.ptr);
+    d.parts = c.take<unsigned long long>((size_t)d.tiles * kTileWords);
+    d.starts = c.take<uint16_t>((size_t)d.tiles * (d.bins + kStartsPad));
+    d.left = c.take<LeftKey>(it.r.n);
+    d.snap = it.pub.snap;
+    d.snap_seq = it.pub.seq;
+    d.told = t->outcome + 1;
+    d.turn = t->stream_turn ^= 1u;
+    most_tiles = std::max(most_tiles, d.tiles);
+    most_keys = std::max(most_keys, d.n);
+    const uint64_t factor = s.grows ? t->cap / s.g.cap : 1;
+    Kind& kind = kinds[factor == 1 ? 0 : factor == 2 ? 1 : 2];
+    kind.b.t[kind.tables++] = d;
+    kind.most_bins = std::max(kind.most_bins, d.bins);
+    if (s.grows) {
+      const uint64_t stretch = kImageSlots / factor;
+      rest.t[n_grow++] = RegrowOf{s.g.from, t->slots, s.g.cap - 1, t->cap - 1, t->st, factor, stretch};
+      most_rest = std::max(most_rest, s.g.cap / stretch);
+    }
+  }
+  const unsigned tables = (unsigned)todo.size();
+  int rc = launch(lead, PSKV_KERNEL_REHASH, k_split, dim3(most_tiles, tables), dim3(kSplitBlock), 0, all);
+  void (*const kernels[3])(StreamBatch) = {k_stream_push<4>, k_stream_push<2>, k_stream_push<1>};
+  bool begun[3] = {false, false, false};
+  for (int k = 0; k < 3 && !rc; ++k) {
+    if (!kinds[k].tables) continue;
+    rc = launch(lead, PSKV_KERNEL_REHASH, kernels[k], dim3(kinds[k].most_bins, kinds[k].tables),
+                dim3(kStreamBlock), 0, kinds[k].b);
+    begun[k] = !rc;
+  }
+  if (!rc && n_grow)
+    rc = launch(lead, PSKV_KERNEL_REHASH, k_regrow_rest, dim3((unsigned)((most_rest * kRestLanes + kBlock - 1) / kBlock), n_grow),
+                dim3(kBlock), 0, rest);
+  // (a lane for every 16th key would do where all of them were left; usually next to none is)
+  if (!rc)
+    rc = launch(lead, PSKV_KERNEL_REHASH, k_push_left, dim3(grid_for(most_keys, kBlock * 16, 512), tables), dim3(kBlock), 0, all);
+  for (Streamed& s : todo) {
+    pskv_table* t = s.it->t;
+    if (rc) (void)hipMemsetAsync(t->st->left_keys, 0, sizeof(t->st->left_keys), t->stream);  // (what was left is not looked up)
+    if (!s.grows) continue;
+    Slot* gone = s.g.from;
+    if (!begun[t->cap / s.g.cap == 2 ? 1 : 2]) {  // it keeps its old array, as in move_growths
+      gone = t->slots;
+      t->slots = s.g.from;
+      t->cap = s.g.cap;
+    }
+    const int r = GrowthLaunches().release(t, gone);
+    if (!rc) rc = r;
+  }
+  return rc;
+}
+
+// Picks the shares of a push that stream: out of `growths` the moves of their tables, which are part of it then. Takes
+// the room they need; one that there is no room for goes through the slots.
+std::vector<Streamed> pick_streamed(Batch& bt, const std::vector<ScalarPlan>& plan, Growths* growths) {
+  std::vector<Streamed> some;
+  double gain = 0.0;
+  for (size_t i = 0; i < bt.size(); ++i) {
+    pskv_table* t = bt[i].t;
+    const uint64_t n = bt[i].r.n;
+    if (!plan[i].may_stream || !n || !t->streams) continue;
+    Streamed s{&bt[i], {}, false, {}};
+    for (const Growth<pskv_table, Slot>& g : growths->list)
+      if (g.t == t && t->cap / g.cap <= (uint64_t)kRegrowMaxFactor) s.g = g, s.grows = true;
+    s.shape = stream_shape(n, t->cap);
+    if (!s.shape.bins) continue;
+    const double its =
+        t->streams > 0 ? kStreamLaunches : stream_gain(n, t->cap, t->share_known ? t->new_share : kFreshGuess, s.grows);
+    if (its <= 0.0) continue;
+    gain += its;
+    some.push_back(s);
+  }
+  if (gain < kStreamLaunches) return {};
+  std::vector<Streamed> todo;
+  for (const Streamed& s : some) {
+    if (grow(s.it->t, &s.it->t->ws, stream_room(s)) != PSKV_OK) {
+      clear_error();
+      continue;
+    }
+    todo.push_back(s);
+    auto& list = growths->list;
+    if (s.grows)
+      list.erase(std::find_if(list.begin(), list.end(), [&](const Growth<pskv_table, Slot>& g) { return g.t == s.it->t; }));
+  }
+  return todo;
+}
+
 int run_scalar(Batch& bt, bool push, bool pull) {
   Growths growths;
   uint64_t n_largest = 0;
   bool any_cache = false, behind = false;
-  std::vector<ScalarCacheUse> use(bt.size(), kScPlain);
+  std::vector<ScalarPlan> plan(bt.size());
   for (size_t i = 0; i < bt.size(); ++i) {
     Item& it = bt[i];
     pskv_table* t = it.t;
@@ -1137,7 +1282,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     // (a growth writes the cache back and drops it; a recorded repeat creates no key)
     int rc = r.replay == kReplayCapture ? PSKV_OK : reserve(t, r.n, 0, 0, &it.pub, &growths);
     if (rc) return rc;
-    const int kind_before = t->sc_last_kind;
+    plan[i].kind_before = t->sc_last_kind;
     if (r.replay) {
       // a request that is being recorded fills the key cache, or is compared with it, whatever its size
       if (t->cap >= (1ull << 32))
@@ -1145,21 +1290,46 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       const bool fits = t->cache_valid && t->cache_n == r.n;
       if (r.replay == kReplayCapture && !fits)
         return set_error(PSKV_ESTALE, "the key cache does not hold the request that is being recorded");
-      use[i] = fits ? kScTry : kScRecord;
+      plan[i].use = fits ? kScTry : kScRecord;
       t->sc_last_n = r.n;
       t->sc_last_kind = r.push ? 0 : 1;
     } else {
-      use[i] = scalar_cache_use(t, r);
+      plan[i].use = scalar_cache_use(t, r);
+      // A push that streams through the slots leaves no record. It gives way to one where pulls follow the pushes, and where the
+      // newest push that streamed named the keys of the one before it (as far as the host has been told).
+      const bool told_same = *static_cast<volatile unsigned long long*>(t->outcome + 1) != 0ull;
+      plan[i].may_stream = push && !pull && !r.pinned &&
+                      (plan[i].use == kScPlain || (plan[i].use == kScRecord && !pulls_follow(t) && !told_same));
     }
-    if (use[i] != kScTry) {
+  }
+  std::vector<Streamed> streamed = push && !pull ? pick_streamed(bt, plan, &growths) : std::vector<Streamed>();
+  for (const Streamed& s : streamed) plan[s.it - bt.data()].streams = true;
+  // (should the request end before they have: their arrays move with the others)
+  struct GiveBack {
+    std::vector<Streamed>& some;
+    Growths& growths;
+    ~GiveBack() {
+      for (const Streamed& s : some)
+        if (s.grows) growths.list.push_back(s.g);
+    }
+  } give_back_growths{streamed, growths};
+  for (size_t i = 0; i < bt.size(); ++i) {
+    Item& it = bt[i];
+    pskv_table* t = it.t;
+    Request& r = it.r;
+    if (r.n == 0) continue;
+    int rc = PSKV_OK;
+    if (plan[i].streams) plan[i].use = kScPlain;
+    if (plan[i].use != kScTry) {
       // the request goes through the slots, so they must be up to date; a push then makes the
       // cached values stale, a recording replaces them
       rc = flush_scalar_cache(t);
       if (rc) return rc;
-      if (push || use[i] == kScRecord) t->cache_valid = false;
+      if (push || plan[i].use == kScRecord) t->cache_valid = false;
     }
+    if (plan[i].streams) continue;
     TableReq& d = it.d;
-    if (use[i] == kScRecord) {
+    if (plan[i].use == kScRecord) {
       // Room for this request in the cache (it has been written back above; kScTry needs nothing:
       // the buffers have the cached request's size). Only a request that is going to be recorded
       // pays for it: a one-off pull of 16M keys would otherwise allocate 256 MB it never uses, and
@@ -1171,7 +1341,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       rc = grow(t, &t->sc_slots, r.n * sizeof(uint32_t));
       if (rc) return rc;
     }
-    if (use[i] == kScPlain) {
+    if (plan[i].use == kScPlain) {
       d.outcome = r.done;
       d.tag.epoch = r.done_seq;
     } else {
@@ -1185,7 +1355,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       // A pull right behind a push, with the slots up to date (the push went through them and
       // recorded itself): the pull kernel compares key by key and needs no launch in front of it.
       // (not in a recording: keys that differ would go through the slots there)
-      const bool per_key = use[i] == kScTry && !push && !t->sc_dirty && kind_before == 0 && r.replay != kReplayCapture;
+      const bool per_key = plan[i].use == kScTry && !push && !t->sc_dirty && plan[i].kind_before == 0 && r.replay != kReplayCapture;
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
       // (a recorded repeat is served from the cache or not at all: nothing to write back)
@@ -1205,9 +1375,15 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     d.snap_seq = it.pub.seq;
     n_largest = std::max(n_largest, r.n);
   }
-  if (!n_largest) return PSKV_OK;
+  if (!n_largest && streamed.empty()) return PSKV_OK;
   int rc = growths.move();
   if (rc) return rc;
+  if (!streamed.empty()) {
+    std::vector<Streamed> todo;
+    todo.swap(streamed);
+    rc = stream_push(bt, todo);
+    if (rc || !n_largest) return rc;
+  }
   // a recorded repeat, where the workgroups that compare it can wait for each other: one launch
   unsigned repeat_quads = 0;
   auto repeat_groups = [&](const Item& it) -> uint64_t {
@@ -1275,11 +1451,11 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   }
   if (rc) return rc;
   for (size_t i = 0; i < bt.size(); ++i) {
-    if (use[i] == kScPlain || !bt[i].r.n) continue;
+    if (plan[i].use == kScPlain || !bt[i].r.n) continue;
     pskv_table* t = bt[i].t;
     t->cache_valid = true;  // whichever way the device decides, the cache now stands for this request
     t->cache_n = bt[i].r.n;
-    if (push && use[i] == kScTry) t->sc_dirty = true;  // served from the cache: the slots lag behind
+    if (push && plan[i].use == kScTry) t->sc_dirty = true;  // served from the cache: the slots lag behind
   }
   return PSKV_OK;
 }
@@ -2237,6 +2413,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   // (the environment variable is for tests of workgroups that do not see the verdict)
   t->push_looks = kOwnLooks;
   if (const char* e = std::getenv("PSKV_PUSH_LOOKS")) t->push_looks = (unsigned)std::strtoul(e, nullptr, 10);
+  if (const char* e = std::getenv("PSKV_STREAM")) t->streams = std::atoi(e) != 0;  // (for tests)
   t->sc_min_keys = kScalarCacheMinKeys;
   if (const char* e = std::getenv("PSKV_SCALAR_CACHE_MIN_KEYS")) t->sc_min_keys = std::strtoull(e, nullptr, 10);
   auto fail = [&](int rc) {

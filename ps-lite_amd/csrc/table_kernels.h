@@ -1664,6 +1664,7 @@ struct RegrowOf {
   uint64_t old_mask, mask;
   DevState* st;
   uint64_t factor;
+  uint64_t stretch;  // old slots per workgroup: a multiple of kRestLanes
 };
 struct RegrowBatch {
   RegrowOf t[kMaxBatch];
@@ -1720,24 +1721,25 @@ __global__ __launch_bounds__(kBlock) void k_regrow(RegrowBatch b) {
   if (threadIdx.x == 0 && total < (unsigned long long)kRegrowOld) old_slots[a + total].key = kEmptyKey;
 }
 
-// Second pass of a growth by k_regrow: sixteen lanes per stretch of kRegrowOld old slots read the
-// keys the first pass left at its front, up to the first empty slot, and insert them the general way.
+// Second pass of a growth: sixteen lanes per stretch of old slots read the keys the first pass left at its front, up to the
+// first empty slot, and insert them the general way. A key that a pushed request has created in the new array meanwhile
+// (k_stream_push) gets both values: what was pushed came to 0.0f + v, and a stored value is never -0.0f.
 constexpr int kRestLanes = 16;
 __global__ __launch_bounds__(kBlock) void k_regrow_rest(RegrowBatch b) {
   const RegrowOf& d = b.t[blockIdx.y];
   const Slot* __restrict__ old_slots = d.old_slots;
   Slot* __restrict__ slots = d.slots;
-  const uint64_t old_cap = d.old_mask + 1, mask = d.mask;
+  const uint64_t old_cap = d.old_mask + 1, mask = d.mask, length = d.stretch;
   DevState* st = d.st;
   const uint64_t stretch = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) / kRestLanes;
   const unsigned l = threadIdx.x % kRestLanes;
   const unsigned group_shift = (threadIdx.x & 63) / kRestLanes * kRestLanes;
-  const uint64_t a = stretch * kRegrowOld;
+  const uint64_t a = stretch * length;
   bool more = a < old_cap;
-  for (unsigned c = 0; c < kRegrowOld / kRestLanes; ++c) {
+  for (uint64_t c = 0; c < length; c += kRestLanes) {
     u64x2 s;
     s.x = kEmptyKey, s.y = 0;
-    if (more) s = *reinterpret_cast<const u64x2*>(&old_slots[a + c * kRestLanes + l]);
+    if (more) s = *reinterpret_cast<const u64x2*>(&old_slots[a + c + l]);
     // the lanes of a wavefront stay together for the ballot; a group that is done reads nothing
     const unsigned long long ends = __ballot(more && s.x == kEmptyKey);
     const unsigned mine = (unsigned)(ends >> group_shift) & ((1u << kRestLanes) - 1u);
@@ -1746,14 +1748,22 @@ __global__ __launch_bounds__(kBlock) void k_regrow_rest(RegrowBatch b) {
       uint64_t h = home_slot(s.x, mask);
       bool placed = false;
       for (uint64_t probes = 0; probes <= mask; ++probes) {
-        if (slots[h].key == kEmptyKey) {
-          unsigned long long old = atomicCAS(reinterpret_cast<unsigned long long*>(&slots[h].key),
-                                             (unsigned long long)kEmptyKey, (unsigned long long)s.x);
-          if (old == kEmptyKey) {
+        unsigned long long k = slots[h].key;
+        if (k == kEmptyKey) {
+          k = atomicCAS(reinterpret_cast<unsigned long long*>(&slots[h].key), (unsigned long long)kEmptyKey,
+                        (unsigned long long)s.x);
+          if (k == kEmptyKey) {
             slots[h].payload = s.y;
             placed = true;
             break;
           }
+        }
+        if (k == s.x) {
+          float* sum = reinterpret_cast<float*>(&slots[h].payload);
+          *sum = *sum + __uint_as_float((unsigned)s.y);
+          atomicAdd(&st->count_shard[stretch % kCountShards * kShardStride], ~0ull);  // (it has been counted twice)
+          placed = true;
+          break;
         }
         h = (h + 1) & mask;
       }
