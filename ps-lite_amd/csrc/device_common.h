@@ -85,7 +85,7 @@ struct alignas(32) DevState {
   unsigned long long scan_total;       // grand total of the last lens scan
   unsigned int error;                  // sticky error bits of finished requests
   unsigned int req_error;              // error bits of the request in flight (follows `error`)
-  unsigned int misaligned;             // OR of (len & 3) over the lens of the current request
+  unsigned int misaligned;             // OR of (len & 3) over the lens of the current request; a push: kReqLong as well
   unsigned int req_flags;              // kReq* facts the workgroups of the kernel in flight have found
   // 32
   unsigned long long arena_top;        // FIXED: rows handed out; VARLEN: 16-byte units handed out
@@ -156,6 +156,7 @@ constexpr unsigned kReqMisaligned = 3u;  // OR of (len & 3)
 constexpr unsigned kReqBadLen = 4u;      // a length negative or above the maximum
 constexpr unsigned kReqDiffer = 8u;      // a key or length differs from the cached request
 constexpr unsigned kReqDuplicate = 16u;  // a key equals its left neighbour (requests are sorted)
+constexpr unsigned kReqLong = 32u;       // a row is much longer than the others (ByRow::longest)
 
 // Counters of the table as they are after request `seq`, written by the device into pinned host memory so that the host
 // can bound the counters without waiting for the stream. Both counters carry the low bits of the request's number above

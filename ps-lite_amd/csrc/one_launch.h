@@ -471,13 +471,13 @@ __device__ __forceinline__ OfAllParts meet_parts(DevState* st, unsigned nblk, un
     x.known = x.known && (w & kPartHere) != 0;
     x.all += sum;
     if (i < blockIdx.x) x.before += sum;
-    x.flags |= (unsigned)(w >> kPartFlagsAt) & 31u;
+    x.flags |= (unsigned)(w >> kPartFlagsAt) & 63u;
   }
   x.known = __syncthreads_and(x.known ? 1 : 0) != 0;
   if (x.known) reduce_parts(x, red);
   return x;
 }
-static_assert(kReqDuplicate == 16u && (kReqMisaligned | kReqBadLen | kReqDiffer) == 15u, "five bits of flags");
+static_assert(kReqLong == 32u && (kReqMisaligned | kReqBadLen | kReqDiffer | kReqDuplicate) == 31u, "six bits of flags");
 
 typedef int32_t i32x2u __attribute__((ext_vector_type(2), aligned(4)));
 struct TwoKeys {
@@ -528,6 +528,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
     len[j] = (unsigned long long)(uint32_t)l;
     s += len[j];
     flags |= (unsigned)l & kReqMisaligned;
+    flags |= longer_than(d, l) ? kReqLong : 0u;
     flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
     const bool has_left = base + j < n && base + j > 0;
     flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
@@ -540,6 +541,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
       of.all += (unsigned long long)(uint32_t)l;
       if (i < (uint64_t)blockIdx.x * kStartPart) of.before += (unsigned long long)(uint32_t)l;
       of.flags |= (unsigned)l & kReqMisaligned;
+      of.flags |= longer_than(d, l) ? kReqLong : 0u;
       of.flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
       of.flags |= i > 0 && d.keys[i] == d.keys[i - 1] ? kReqDuplicate : 0u;
     }
@@ -552,7 +554,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
     if (st->req_error) atomicOr(&st->error, st->req_error);
     st->req_error = bad;
     st->scan_total = of.all;
-    st->misaligned = of.flags & kReqMisaligned;
+    st->misaligned = of.flags & (kReqMisaligned | kReqLong);
     st->cache_epoch = d.tag.epoch;
     if (bad) st->bad_epoch = d.tag.epoch;
     tell_ragged(st, d.outcome, of.flags);

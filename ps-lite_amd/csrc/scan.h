@@ -127,7 +127,7 @@ __device__ __forceinline__ void scan_pass1_last(unsigned long long* part, DevSta
   const bool dup = (flags & kReqDuplicate) != 0u;
   st->req_error = (bad_len ? kDevErrBadLen : 0u) | (dup ? kDevErrDuplicate : 0u);
   if (bad_len || dup) st->bad_epoch = epoch;
-  st->misaligned = flags & kReqMisaligned;
+  st->misaligned = flags & (kReqMisaligned | kReqLong);
 }
 
 // Pass 2, the workgroup's part: every thread passes its kItems consecutive lens

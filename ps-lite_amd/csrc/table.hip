@@ -13,6 +13,7 @@
 #include <string>
 #include <thread>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include <hip/hip_ext.h>
@@ -1490,11 +1491,11 @@ int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
   auto nblk = [&](const Item&) { return blocks; };
   int rc;
   if (op == kOpAcc) {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true, false), nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false, false), nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true, false, false), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_ACC, PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false, false, false), nblk);
   } else {
-    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true, false), nblk)
-                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false, false), nblk);
+    rc = stream ? launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true, false, false), nblk)
+                : launch_batch(bt, PSKV_KERNEL_ROWS_GATHER, PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false, false, false), nblk);
   }
   it.d.tile_base = 0;
   return rc;
@@ -1528,18 +1529,33 @@ int launch_rows(Batch& bt, int op) {
     return PSKV_OK;
   }
   auto nblk = [&](const Item& it) {
-    if (VARLEN) return (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock + (it.d.started ? 1 : 0);
+    if (VARLEN) {
+      uint64_t blocks = (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock;
+      if (op == kOpAcc && it.d.k) {
+        const uint64_t rows = (uint64_t)kBlock >> ((it.d.k & ((1u << kByRowBits) - 1)) - 1);  // of a workgroup
+        blocks = std::max(blocks, (it.d.n + rows - 1) / rows);
+      }
+      return blocks + (it.d.started ? 1 : 0);
+    }
     return (it.d.ntiles + kQuadsFixed - 1) / kQuadsFixed;
   };
   const bool stream = floats >= kStreamFloats;
   bool started = false;
   for (const Item& it : bt) started = started || (VARLEN && it.d.started);
-  const KernelSet kernels =
-      op == kOpAcc
-          ? (started ? (stream ? PSKV_KSET_OF(k_rows, kOpAcc, true, true, true) : PSKV_KSET_OF(k_rows, kOpAcc, true, false, true))
-                     : (stream ? PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, true, false) : PSKV_KSET_OF(k_rows, kOpAcc, VARLEN, false, false)))
-          : (started ? (stream ? PSKV_KSET_OF(k_rows, kOpGather, true, true, true) : PSKV_KSET_OF(k_rows, kOpGather, true, false, true))
-                     : (stream ? PSKV_KSET_OF(k_rows, kOpGather, VARLEN, true, false) : PSKV_KSET_OF(k_rows, kOpGather, VARLEN, false, false)));
+  bool by_row = false;
+  for (const Item& it : bt) by_row = by_row || (VARLEN && op == kOpAcc && it.d.k);
+  auto pick = [&](auto op_, auto started_, auto by_row_) {
+    constexpr int OP = decltype(op_)::value;
+    constexpr bool STARTED = decltype(started_)::value, BY_ROW = decltype(by_row_)::value;
+    return stream ? PSKV_KSET_OF(k_rows, OP, VARLEN, true, STARTED, BY_ROW) : PSKV_KSET_OF(k_rows, OP, VARLEN, false, STARTED, BY_ROW);
+  };
+  using Acc = std::integral_constant<int, kOpAcc>;
+  using Gather = std::integral_constant<int, kOpGather>;
+  using No = std::false_type;
+  using Yes = std::integral_constant<bool, VARLEN>;
+  const KernelSet kernels = op == kOpAcc ? (by_row ? (started ? pick(Acc(), Yes(), Yes()) : pick(Acc(), No(), Yes()))
+                                                   : (started ? pick(Acc(), Yes(), No()) : pick(Acc(), No(), No())))
+                                         : (started ? pick(Gather(), Yes(), No()) : pick(Gather(), No(), No()));
   return launch_batch(bt, op == kOpAcc ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, nblk);
 }
 
@@ -1760,6 +1776,20 @@ bool start_together(const Batch& bt, bool push, F floats) {
   return one_start(r);
 }
 
+// How the rows of a push are added should they be ragged (rows_by_row), where the table's pushes have been so far as the host has
+// been told: about a lane per quad. Slice, push and pull, us: 2M rows of 1 to 20 floats in four tables 159 -> 146, 1M of 1 to 60 in
+// one 163 -> 148, 500,000 of 1 to 128 in 16, other ones every time, 210 -> 200 each. Not rows of a quad or two (300,000 of 1
+// to 10 in two tables 54 -> 56), of hundreds of floats, which fill wavefronts either way, nor requests that come in pieces, nor
+// (the device sees to that) where a row takes sixteen times as long as the others.
+constexpr uint64_t kByRowLeast = 8, kByRowMost = 128;
+uint64_t ragged_by_row(const pskv_table* t, const Request& r) {
+  const uint64_t mean = r.nvals / r.n;
+  if (!const_cast<volatile unsigned long long*>(t->outcome)[1] || r.pipe_in || mean < kByRowLeast || mean > kByRowMost) return 0;
+  unsigned shift = 2;
+  while ((1ull << shift) < (mean + 3) / 4) ++shift;
+  return by_row(shift, 16 * mean + 16);
+}
+
 // Launches per var-len request: a push takes three (compare + scan pass 1; scan pass 2 +
 // find-or-create + counter record; rows), a pull three (compare + stored lengths + scan pass 1;
 // scan pass 2 + tile table; rows), whatever the number of tables; a small one two (start_together).
@@ -1840,6 +1870,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_key = r.nvals ? static_cast<uint32_t*>(t->tiles.ptr) : nullptr;
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
+      d.k = ragged_by_row(t, r);
     }
     int rc = growths.move();
     if (rc) return rc;

@@ -57,7 +57,7 @@ struct TableReq : TableHead {
   // row kernels
   float* req;             // push: request values (read); pull: response values (written)
   uint64_t total;         // floats in req
-  uint64_t k;             // FIXED: floats per row
+  uint64_t k;             // FIXED: floats per row; VARLEN push: how the host would have ragged rows added (by_row)
   union {
     uint32_t cached;      // FIXED lookup: the first so many positions of cache_keys and ref belong together
     uint32_t started;     // VARLEN row kernels: workgroups of the k_var_*_start in front of this one, or 0
@@ -743,6 +743,14 @@ __device__ __forceinline__ void tell_ragged(DevState* st, unsigned long long* ou
   outcome[1] = ragged;
 }
 
+// TableReq::k of a VARLEN push whose rows the host takes to be ragged: 2^shift lanes per row, and the longest row for which that
+// will do; 0: a wavefront per 256 floats.
+constexpr unsigned kByRowBits = 8;
+__host__ __device__ constexpr uint64_t by_row(unsigned shift, uint64_t longest) { return longest << kByRowBits | (shift + 1); }
+__device__ __forceinline__ bool longer_than(const TableReq& d, int32_t len) {
+  return d.k && (uint64_t)(uint32_t)len > d.k >> kByRowBits;
+}
+
 // VARLEN push, first kernel: one pass over the request's keys and lens that
 //   - compares them with the cached request (when the host found the cache usable),
 //   - takes pass 1 of the lens scan (per-workgroup totals, flags),
@@ -785,6 +793,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
     const int32_t l = mine.v[j];
     s += (unsigned long long)(long long)l;
     flags |= (unsigned)l & kReqMisaligned;
+    flags |= longer_than(d, l) ? kReqLong : 0u;
     flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
     flags |= (mine.k[j] != old.k[j] || l != old.v[j]) ? kReqDiffer : 0u;
     // keys are sorted and must be unique (kv_app.h:17): a key that equals its left neighbour
@@ -1512,6 +1521,51 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
   }
 }
 
+// Ragged rows of a push, the other way round: 2^shift lanes a row (about as many as it has quads, by the host's reckoning),
+// a lane a quad of it, two turns asked for together. A wavefront that starts from its tile makes five trips to memory that follow
+// from each other (facts, tile table, offsets and references, rows, values), one that starts from its rows three; its
+// accesses to the arena are whole quads on their own boundaries (the end of a row's last one is nobody's), where a tile's
+// straddle them. Bound by the lines of the rows, which lie scattered: 200,000 of 600,000 rows of 1 to 100 floats 35 -> 29 us
+// (5.4 TB/s of lines), of 1 to 20 15 -> 11. Not for pulls (30 -> 33: their stores would be the ones that straddle), and not
+// where a row is far longer than the others, whose wavefront everybody would wait for.
+template <bool STREAM>
+__device__ __forceinline__ void rows_by_row(const RowsParams& p, uint64_t total, unsigned shift, bool rejected) {
+  const unsigned lane = threadIdx.x & 63, lanes = 1u << shift;
+  const uint64_t wave = (uint64_t)p.blk * (kBlock / 64) + (threadIdx.x >> 6);
+  const uint64_t row = (wave << (6 - shift)) + (lane >> shift);
+  if (row >= p.n) return;
+  const uint64_t first = p.off[row], end = p.off[row + 1], r = p.ref[row];
+  if (r == kRefAbsent) return;  // a key the lookup refused
+  const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
+  if (rejected && !fresh) return;
+  const uint32_t len = (uint32_t)(end - first), quads = (len + 3) >> 2;
+  float* dst = p.arena + (((r & ~kRefNew) >> kLenBits) << 2);
+  const float* side = p.req + first;
+  constexpr unsigned kTurns = 2;
+  for (uint32_t q0 = lane & (lanes - 1); q0 < quads; q0 += kTurns * lanes) {
+    f32x4 x[kTurns], y[kTurns];
+#pragma unroll
+    for (unsigned u = 0; u < kTurns; ++u) {
+      const uint32_t q = q0 + u * lanes;
+      x[u] = y[u] = (f32x4)(0.f);
+      if (q >= quads) continue;
+      if (!fresh) y[u] = load_quad<false>(dst + q * 4);
+      if (!rejected)  // (what follows a row's last float is the next row, but for the last row's)
+        x[u] = first + q * 4 + 4 <= total ? load_quad<STREAM>(side + q * 4) : load_part<STREAM>(side + q * 4, len - q * 4);
+    }
+#pragma unroll
+    for (unsigned u = 0; u < kTurns; ++u) {
+      const uint32_t q = q0 + u * lanes, left = len - q * 4;
+      if (q >= quads) continue;
+      f32x4 sum = rejected ? y[u] : y[u] + x[u];  // a created row is a zero row first (0.0f + v)
+      if (left < 2) sum.y = y[u].y;
+      if (left < 3) sum.z = y[u].z;
+      if (left < 4) sum.w = y[u].w;
+      store_quad<false>(sum, dst + q * 4);
+    }
+  }
+}
+
 // Quads per workgroup (fixed rows) and request-side floats per wavefront (var-len rows). One
 // 128-bit access per lane and many small workgroups stream fastest on this GPU (6.5 TB/s for
 // `row += in` against 5.5 TB/s with four accesses per lane).
@@ -1527,13 +1581,17 @@ __device__ __forceinline__ void finish_start(const TableReq& d) {
 
 // STARTED: VARLEN, behind one of those two kernels. (A kernel of its own: with the end of such a request in the way of the
 // others, 2M rows over 16 tables took 374 us to push and pull, not 357.)
-template <int OP, bool VARLEN, bool STREAM, bool STARTED, int TABLES>
+// BY_ROW: a push in which the host takes some table's rows to be ragged.
+template <int OP, bool VARLEN, bool STREAM, bool STARTED, bool BY_ROW, int TABLES>
 __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   // the grid is sized for the largest table of the launch: workgroups (VARLEN: wavefronts) past
   // this table's floats leave before they touch anything
+  const bool by_row = BY_ROW && d.k != 0;
   if (VARLEN) {
-    if ((((uint64_t)blockIdx.x + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total) {
+    const bool behind = by_row ? blockIdx.x + (STARTED && d.started ? 1u : 0u) >= d.nblk
+                               : (((uint64_t)blockIdx.x + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total;
+    if (behind) {
       if (STARTED && d.started && blockIdx.x == d.nblk - 1) finish_start(d);  // (a workgroup behind the last one with floats)
       return;
     }
@@ -1570,7 +1628,7 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
     uint64_t total = p.total;
     f32x4 x;
     TileNote aff = {kTileNotAffine, 0};
-    rows_wave_ask<OP, STREAM>(p, total, x, aff);
+    if (!by_row) rows_wave_ask<OP, STREAM>(p, total, x, aff);
     // a request served from the cached references creates nothing and cannot have been refused
     const bool same = facts.same_epoch == p.tag.epoch;
     if (p.tag.replay && !same) return;
@@ -1586,7 +1644,14 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
         return;
       }
     }
-    if (facts.misaligned != 0) {
+    if (by_row) {
+      if ((facts.misaligned & kReqMisaligned) && !(facts.misaligned & kReqLong)) {
+        rows_by_row<STREAM>(p, total, (unsigned)(d.k & ((1u << kByRowBits) - 1)) - 1, rejected);
+        return;
+      }
+      rows_wave_ask<OP, STREAM>(p, total, x, aff);  // (the host was wrong)
+    }
+    if (facts.misaligned & kReqMisaligned) {
       rows_wave_varlen<OP, true, STREAM>(p, total, s_off, s_ref, rejected, same, x);
     } else {
       if (same && rows_wave_affine<OP, STREAM>(p, total, x, aff)) return;

@@ -127,3 +127,46 @@ def test_requests_that_partly_repeat(capi, orc, dev, mode, n):
             torch.cuda.synchronize()
         assert_bits_equal(out.cpu().numpy(), want)
     assert_bits_equal(t.dump()[2], o.dump()[2])
+
+
+# mean lengths around the ones that lanes per row go by, a row sixteen times as long as the others, rows of nothing
+RAGGED = {"seven": lambda rng, n: rng.integers(5, 10, n), "nine": lambda rng, n: rng.integers(1, 18, n),
+          "with a long one": lambda rng, n: np.where(np.arange(n) == n // 2, 4099, rng.integers(0, 40, n)),
+          "up to the longest": lambda rng, n: np.where(np.arange(n) % 500 == 3, 290, rng.integers(0, 37, n)),
+          "hundreds": lambda rng, n: rng.integers(90, 165, n)}
+
+
+@pytest.mark.parametrize("n,S", [(700, 1), (30_001, 2), (140_003, 1)])
+@pytest.mark.parametrize("which", sorted(RAGGED))
+def test_ragged_pushes_row_by_row(capi, orc, dev, which, n, S):
+    """Pushes behind one that has told the host of ragged rows: held and new rows, the same again, one that is refused."""
+    announce("row by row", which, n, S)
+    rng = np.random.default_rng(n)
+    group, stores = capi.Group(S, capi.MODE_VARLEN), [orc.Store(orc.MODE_VARLEN) for _ in range(S)]
+    begin, end = capi.server_ranges(S)
+    keys = unique_keys(rng, 2 * n, S)
+    all_lens = RAGGED[which](rng, 2 * n).astype(np.int32)
+    all_lens[::13] += 1  # ragged in any case
+    for turn in range(5):
+        pick = np.sort(rng.choice(2 * n, n, replace=False)) if turn not in (2, 4) else pick
+        some, lens = keys[pick], all_lens[pick].copy()
+        if turn == 4:
+            lens[n // 3] += 4  # not the stored length: nothing of this table's share is applied
+        vals = rng.standard_normal(int(lens.sum())).astype(np.float32)
+        dk, dl = to_dev(some, dev), to_dev(lens, dev)
+        pos, val_pos, _ = capi.slice_keys(dk, begin, end, lens=dl, nvals=vals.size)
+        group.push(dk, pos, _off_by(vals, dev, turn % 3), val_pos, lens=dl)
+        if turn == 4:
+            with pytest.raises(capi.PskvError):
+                group.sync()
+        else:
+            group.sync()
+        for s in range(S):
+            part, floats = slice(int(pos[s]), int(pos[s + 1])), slice(int(val_pos[s]), int(val_pos[s + 1]))
+            if turn < 4 or not part.start <= n // 3 < part.stop:
+                stores[s].push(some[part], vals[floats], lens[part])
+    for s in range(S):
+        want_keys, want_lens, want = stores[s].dump()
+        got_keys, got_lens, got = group.tables[s].dump()
+        assert np.array_equal(got_keys, want_keys) and np.array_equal(got_lens, want_lens)
+        assert_bits_equal(got, want, "%s table %d" % (which, s))
