@@ -314,9 +314,8 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
     d.left[left_room(d.st, d.turn)] = LeftKey{words[at], reinterpret_cast<const float*>(words + kSplitTile)[at], kNoRun};
   }
   __syncthreads();
-  const float unset = __uint_as_float((unsigned)kPayloadUnset);
   if (GROW) {
-    for (unsigned j = threadIdx.x; j < kImageSlots; j += kStreamBlock) s_key[j] = kEmptyKey, s_val[j] = unset;
+    for (unsigned j = threadIdx.x; j < kImageSlots; j += kStreamBlock) s_key[j] = kEmptyKey, s_val[j] = 0.0f;
   }
   unsigned created = 0;
   for (unsigned image = 0; image < d.images; ++image) {
@@ -338,7 +337,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
         if (home_slot(s[q].x, d.old_mask) - old_base > at) continue;
         for (unsigned j = (unsigned)home_slot(s[q].x, mask) % kImageSlots; j < kImageSlots; ++j) {
           if (atomicCAS(&s_key[j], (unsigned long long)kEmptyKey, (unsigned long long)s[q].x) != kEmptyKey) continue;
-          s_val[j] = __uint_as_float((unsigned)s[q].y);
+          s_val[j] = stored_value(s[q].y);
           rest[q] = false;
           break;
         }
@@ -351,7 +350,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
       for (unsigned q = 0; q < SLOTS; ++q) {
         const unsigned j = q * kStreamBlock + threadIdx.x;
         s_key[j] = s[q].x;
-        s_val[j] = __uint_as_float((unsigned)s[q].y);
+        s_val[j] = stored_value(s[q].y);
       }
     }
     if (image + 1 < d.images) ask(image + 1);
@@ -386,9 +385,9 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
       const unsigned j = q * kStreamBlock + threadIdx.x;
       u64x2 w;
       w.x = s_key[j];
-      w.y = (kPayloadUnset ^ 0xffffffffull) | __float_as_uint(s_val[j]);
+      w.y = kPayloadUnset ^ __float_as_uint(s_val[j]);
       __builtin_nontemporal_store(w, &out[j]);
-      if (GROW) s_key[j] = kEmptyKey, s_val[j] = unset;
+      if (GROW) s_key[j] = kEmptyKey, s_val[j] = 0.0f;
     }
     // (what a lane writes in front of the next barrier, it has read itself)
   }
@@ -417,10 +416,10 @@ __global__ __launch_bounds__(kBlock) void k_push_left(StreamBatch b) {
     uint64_t seen;
     uint64_t* p = find_or_insert(d.slots, d.mask, st, l.key, is_new, seen);
     if (!p) continue;
-    float cur = (is_new ? 0.0f : __uint_as_float((unsigned)seen)) + l.v;
+    float cur = (is_new ? 0.0f : stored_value(seen)) + l.v;
     if (l.run != kNoRun)
       for (uint64_t j = (uint64_t)l.run + 1; j < d.n && d.keys[j] == l.key; ++j) cur = cur + d.vals[j];
-    *reinterpret_cast<float*>(p) = cur;
+    store_value(p, cur);
     created += is_new ? 1u : 0u;
   }
   if (blockIdx.x * kBlock < left) block_count_add(st, created, red);

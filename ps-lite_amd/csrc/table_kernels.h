@@ -97,7 +97,7 @@ __device__ __forceinline__ void arrived(T& x) {
 }
 
 // ---------------------------------------------------------------------------------
-// SCALAR mode: one float per key, kept in the low word of the slot payload so that a
+// SCALAR mode: one float per key, kept in the low word of the slot payload (stored_value) so that a
 // probe reads key and value with one 128-bit load.
 // One lane per key. Keys are unique within a request (kv_app.h:17), so the value word of a
 // slot is only ever touched by the lane that owns the key: no atomics on values, and the
@@ -224,10 +224,9 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
         uint64_t seen;
         uint64_t* p = find_or_insert(slots, mask, st, key, is_new, seen);
         if (!p) continue;
-        const float cur = is_new ? 0.0f : __uint_as_float((unsigned)seen);
+        const float cur = is_new ? 0.0f : stored_value(seen);
         out[j] = cur;
         for (uint64_t r = j + 1; r < n && keys[r] == key; ++r) out[r] = cur;
-        if (is_new) *reinterpret_cast<float*>(p) = cur;
         created += is_new ? 1u : 0u;
       }
     }
@@ -277,7 +276,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
     if (record && (!p || run)) st->bad_epoch = d.tag.epoch;  // not a request the cache can stand for
     if (!p) continue;
     // an absent key starts from Val() == 0, then `+=` (kv_app.h:454): 0.0f + v, not a copy
-    float cur = is_new ? 0.0f : held ? held_value : __uint_as_float((unsigned)seen);
+    float cur = is_new ? 0.0f : held ? held_value : stored_value(seen);
     if (PUSH) cur = cur + v;
     if (PULL) out[i] = cur;
     if (run) {  // the rest of the run, element by element like the reference's loop
@@ -286,7 +285,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
         if (PULL) out[j] = cur;
       }
     }
-    if (PUSH || is_new || held) *reinterpret_cast<float*>(p) = cur;
+    if (PUSH || held) store_value(p, cur);
     created += is_new ? 1u : 0u;
     if (record) {
       d.cache_keys[i] = key;
@@ -330,9 +329,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
 __device__ __forceinline__ void write_back(const TableHead& d, uint64_t i) {
   const uint32_t slot = d.tile_key[i];
   const float v = d.arena[i];
-  float* dst = slot == kSlotSpecial ? reinterpret_cast<float*>(&d.st->special_payload)
-                                    : reinterpret_cast<float*>(&d.slots[slot].payload);
-  *dst = v;
+  store_value(slot == kSlotSpecial ? reinterpret_cast<uint64_t*>(&d.st->special_payload) : &d.slots[slot].payload, v);
 }
 
 // Writes the cached values back to their slots. Launched before anything reads or changes the
@@ -1824,8 +1821,7 @@ __global__ __launch_bounds__(kBlock) void k_regrow_rest(RegrowBatch b) {
           }
         }
         if (k == s.x) {
-          float* sum = reinterpret_cast<float*>(&slots[h].payload);
-          *sum = *sum + __uint_as_float((unsigned)s.y);
+          store_value(&slots[h].payload, stored_value(slots[h].payload) + stored_value(s.y));
           atomicAdd(&st->count_shard[stretch % kCountShards * kShardStride], ~0ull);  // (it has been counted twice)
           placed = true;
           break;
