@@ -33,7 +33,8 @@ constexpr unsigned kMatchTurn = kMatchLds / kMatchBlock;  // source keys a lane 
 // A longer stretch than so many pieces is sampled, not staged. (Pieces follow from each other, but read in one go
 // what the sampled search reads key by key: they pay while there are workgroups enough to fill the GPU.)
 constexpr unsigned kMatchPieces = 8, kMatchPiecesFew = 3;
-constexpr unsigned kOwnSpans = 4096;
+// Tiles (of kMatchItems keys a lane, and of one) up to which the workgroups search for themselves, without a launch in front of them.
+constexpr unsigned kOwnSpans = 2560, kOwnSpansFew = 4096;
 constexpr uint64_t kNoMatch = ~0ull;
 constexpr unsigned kCounts = 64;        // counters of matched keys, each on a line of its own
 constexpr unsigned kCountStride = 16;
@@ -58,15 +59,19 @@ __device__ __forceinline__ f32x4 combine(int op, f32x4 d, f32x4 s) {
 // The match walks the tiles of one key set and finds their keys in the other. spans[t] = first key of the set that is
 // searched (`src`, n_src keys) not below the first key of tile t of the other; spans[tiles] = n_src.
 // The stretch of tile t is [spans[t], spans[t+1]): it may hold keys that lie between two
-// tiles, which match nothing. Bound by the round trips to memory that follow from each other: a workgroup
-// samples the whole source evenly into LDS (one round trip, the same lines for every workgroup), its
-// kSpanTiles tiles find the step they lie in there, and kSpanLanes lanes each narrow it down by a factor of 16
-// per round: four round trips in all for 16M keys. (A wavefront per tile with 64 probes per round takes as many
-// but reads 72 lines a tile.)
+// tiles, which match nothing. Bound by the lines it reads (16 probes for each of 15,625 tiles are 6 us) and by the round trips
+// that follow from each other: a workgroup samples the whole source evenly into LDS (one round trip, the same lines for every
+// workgroup), its kSpanTiles tiles find the step they lie in there, and kSpanLanes lanes per tile look at kSpanWindow keys,
+// a line or two or three, around the place where the tile's first key should be if the keys between the two that enclose it are spread evenly. A
+// step of 12,000 keys spread by a hash takes two or three looks; what is not found after kSpanLooks of them is narrowed down by a
+// factor of 16 per round. 12M into 16M keys: 17.5 us -> 10.6 (4,096 samples and three rounds of 16 probes without a guess), the
+// whole call 103 -> 96.5; into keys in 2,000 clusters, where guesses are no good, 96.3 -> 95.4, squares 89.8 -> 88.3.
 constexpr unsigned kSpanLanes = 16;
 constexpr unsigned kSpanTiles = 64;
 constexpr unsigned kSpanBlock = kSpanTiles * kSpanLanes;
-constexpr unsigned kSpanSamples = 4 * kSpanBlock;
+constexpr unsigned kSpanSamples = kSpanBlock;
+constexpr unsigned kSpanWindow = 2 * kSpanLanes;
+constexpr unsigned kSpanLooks = 4;
 __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __restrict__ src, uint64_t n_src,
                                                             const uint64_t* __restrict__ dst, uint64_t tiles,
                                                             unsigned tile, uint64_t* __restrict__ spans) {
@@ -77,14 +82,7 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
   const uint64_t key = live ? dst[t * tile] : 0;
   const uint64_t step = (n_src + kSpanSamples - 1) / kSpanSamples;
   const unsigned samples = (unsigned)((n_src + step - 1) / step);
-  uint64_t x[kSpanSamples / kSpanBlock];
-#pragma unroll
-  for (unsigned q = 0; q < kSpanSamples / kSpanBlock; ++q) {
-    const unsigned i = q * kSpanBlock + threadIdx.x;
-    x[q] = i < samples ? src[i * step] : 0;
-  }
-#pragma unroll
-  for (unsigned q = 0; q < kSpanSamples / kSpanBlock; ++q) s_sample[q * kSpanBlock + threadIdx.x] = x[q];
+  s_sample[threadIdx.x] = src[(threadIdx.x < samples ? threadIdx.x : samples - 1) * step];
   if (t == 0 && sub == 0) spans[tiles] = n_src;
   __syncthreads();
   unsigned a = 0, b = samples;  // samples before a are below the key, none from b on is
@@ -93,15 +91,38 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
     if (s_sample[mid] < key) a = mid + 1; else b = mid;
   }
   // every source key before lo is below the key, none from hi on is
-  uint64_t lo = a ? (a - 1) * step + 1 : 0, hi = a < samples ? a * step : n_src;
-  // (the lanes of a group stay together; a wavefront takes as many rounds as the longest of its groups)
-  while (__any(live && lo < hi)) {
+  uint64_t lo = a ? (a - 1) * step + 1 : 0, hi = !live ? lo : a < samples ? a * step : n_src;
+  if (a == 0) hi = lo;  // (the first sample is the first key)
+  const unsigned of_group = lane / kSpanLanes * kSpanLanes;
+  // (the lanes of a group stay together)
+  auto count = [&](bool x) { return (unsigned)__popcll((__ballot(x) >> of_group) & ((1ull << kSpanLanes) - 1)); };
+  const bool enclosed = a > 0 && a < samples;
+  uint64_t under = enclosed ? s_sample[a - 1] : 0, over = enclosed ? s_sample[a] : 0;  // the keys at lo - 1 and at hi
+  for (unsigned look = 0; look < kSpanLooks && __any(enclosed && lo < hi); ++look) {
+    const float share = (float)(key - under) / (float)(over - under);
+    const uint64_t guess = lo + (uint64_t)(fminf(fmaxf(share, 0.0f), 1.0f) * (float)(hi - lo));
+    uint64_t from = guess > lo + kSpanWindow / 2 ? guess - kSpanWindow / 2 : lo;
+    if (from + kSpanWindow > hi) from = hi - lo > kSpanWindow ? hi - kSpanWindow : lo;
+    const uint64_t p0 = from + sub, p1 = p0 + kSpanLanes;
+    const bool in0 = enclosed && p0 < hi, in1 = enclosed && p1 < hi;
+    const uint64_t x0 = in0 ? src[p0] : ~0ull, x1 = in1 ? src[p1] : ~0ull;
+    const unsigned looked = count(in0) + count(in1), below = count(in0 && x0 < key) + count(in1 && x1 < key);
+    const uint64_t first = __shfl(x0, (int)of_group), last = __shfl(x1, (int)(of_group + kSpanLanes - 1));
+    if (looked == 0) continue;  // found before
+    if (below == 0 && from > lo) {
+      hi = from, over = first;
+    } else if (below == looked && from + looked < hi) {
+      lo = from + looked, under = last;  // (a whole window: it ends before hi)
+    } else {
+      lo = hi = from + below;
+    }
+  }
+  // (a wavefront takes as many rounds as the longest of its groups)
+  while (__any(lo < hi)) {
     const uint64_t stride = (hi - lo + kSpanLanes - 1) / kSpanLanes;
     const uint64_t p = lo + sub * stride;
-    const bool below = live && p < hi && src[p] < key;
+    const unsigned cnt = count(p < hi && src[p] < key);
     // the probes are sorted: the first cnt are below
-    const unsigned cnt =
-        (unsigned)__popcll((__ballot(below) >> (lane / kSpanLanes * kSpanLanes)) & ((1ull << kSpanLanes) - 1));
     if (cnt == 0) {
       hi = lo;
     } else {
@@ -119,10 +140,10 @@ __global__ __launch_bounds__(kSpanBlock) void k_match_spans(const uint64_t* __re
 // other: 12M source against 16M destination keys, the whole call, took 125 us with one source key per lane asked for at a
 // time, 104.7 with three under a condition each, 101 without it, and 99.5 with all six that LDS has room for.
 // OWN: the workgroup finds where its stretch begins and ends itself (a wavefront each) instead of reading it from `spans`:
-// the search is hidden behind the keys of the tile, and a launch of 10 to 13 us in front of this one falls away, but every
+// the search is hidden behind the keys of the tile, and a launch in front of this one falls away, but every
 // workgroup reads lines for it that nobody else needs. Up to kOwnSpans tiles that is the better way (us per call:
-// 45,928 into 44,225 keys 16.6 -> 13.5, 1M into 1M 28.0 -> 21.4, 2.6M into 1.4M 39.3 -> 32.6, 4M into 4M 47.9 -> 46.2;
-// beyond it 6M into 6M 56.4 -> 58).
+// 45,928 into 44,225 keys 16.6 -> 13.5, 1M into 1M 28.0 -> 21.4, 2.6M into 1.4M 39.3 -> 32.6; against the search as it is now 3M
+// into 3M 41.3 -> 42.1, 4M into 4M 45.9 -> 50.3, but 1M into 16M, tiles of 256 keys, 70.7 -> 66.3).
 // K1: values are single floats and are combined here; otherwise where[i] receives the index in `far` of the match of
 // key i, or kNoMatch.
 template <bool K1, bool SWAP, unsigned ITEMS, bool OWN>
@@ -506,7 +527,7 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
   const bool few = n_near < kFewKeys || n_far / n_near >= 2;
   const unsigned tile = kMatchBlock * (few ? 1 : kMatchItems);
   const unsigned blocks = (unsigned)((n_near + tile - 1) / tile);
-  const bool own = blocks <= kOwnSpans;
+  const bool own = blocks <= (few ? kOwnSpansFew : kOwnSpans);
   if (!own) {
     int rc = room(&c->spans, ((size_t)blocks + 1) * sizeof(uint64_t), st);
     if (rc) return rc;

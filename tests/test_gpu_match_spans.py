@@ -38,3 +38,33 @@ def test_tiles_outside_the_other_set(capi, dev, n_dst):
         got = to_dev(dv, dev)
         assert capi.match(to_dev(sk, dev), to_dev(sv, dev), to_dev(dk, dev), got, 1, capi.OP_PLUS) == want_n
         assert_bits_equal(from_dev(got), want)
+
+
+def _sets(kind, rng, n):
+    if kind == "even":
+        return np.arange(n, dtype=np.uint64) * np.uint64(3)
+    if kind == "squares":
+        return np.arange(n, dtype=np.uint64) ** np.uint64(2)
+    if kind == "clusters":
+        return np.unique((rng.integers(0, 1 << 40, 700, dtype=np.uint64) << np.uint64(20))[:, None]
+                         + np.arange(n // 700 + 1, dtype=np.uint64)).ravel()
+    if kind == "far away":  # all but a few of the keys
+        return np.concatenate([np.arange(9, dtype=np.uint64), np.uint64(1 << 63) + np.arange(n, dtype=np.uint64)])
+    return np.unique(rng.integers(0, 1 << 64, n, dtype=np.uint64))
+
+
+@pytest.mark.parametrize("kind", ["even", "squares", "clusters", "far away", "any"])
+@pytest.mark.parametrize("n_src,n_dst", [(2_000_000, 2560 * 1024), (2_700_000, 2561 * 1024 + 3), (1100, 2_700_000)])
+def test_stretches_wherever_the_keys_lie(capi, dev, kind, n_src, n_dst):
+    """Searches that guess from the keys around: keys spread evenly, by the square, in clusters, and with a gap."""
+    announce("match guesses", kind, n_src, n_dst)
+    rng = np.random.default_rng(n_dst)
+    both = _sets(kind, rng, n_src + n_dst // 2)
+    sk = np.sort(rng.choice(both, min(n_src, both.size), replace=False))
+    dk = np.unique(np.concatenate([rng.choice(both, n_dst // 2, replace=False), both + np.uint64(1)]))[:n_dst]
+    sv = rng.integers(-50, 50, sk.size).astype(np.float32)
+    dv = rng.integers(-50, 50, dk.size).astype(np.float32)
+    want, want_n = numpy_model(sk, sv, dk, dv, 1, 1)
+    got = to_dev(dv, dev)
+    assert capi.match(to_dev(sk, dev), to_dev(sv, dev), to_dev(dk, dev), got, 1, capi.OP_PLUS) == want_n
+    assert_bits_equal(from_dev(got), want)
