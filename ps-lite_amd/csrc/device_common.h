@@ -131,7 +131,8 @@ struct alignas(32) DevState {
   // each word of count_shard)
   unsigned left_keys[2];
   unsigned long long keys_sum;
-  unsigned long long pad[4];
+  unsigned long long packed_epoch;  // the cached request whose keys are there packed as well (PackedKeys)
+  unsigned long long pad[3];
   // one_launch.h: what the workgroups of a var-len request tell each other, all zero between requests
   unsigned long long parts[kVarParts];
 };
@@ -164,7 +165,8 @@ constexpr unsigned kReqMisaligned = 3u;  // OR of (len & 3)
 constexpr unsigned kReqBadLen = 4u;      // a length negative or above the maximum
 constexpr unsigned kReqDiffer = 8u;      // a key or length differs from the cached request
 constexpr unsigned kReqDuplicate = 16u;  // a key equals its left neighbour (requests are sorted)
-constexpr unsigned kReqLong = 32u;       // a row is much longer than the others (ByRow::longest)
+constexpr unsigned kReqLong = 32u;       // a row is much longer than the others (by_row)
+constexpr unsigned kReqWide = 64u;       // two neighbouring keys are too far apart to be packed (PackedKeys)
 
 // Counters of the table as they are after request `seq`, written by the device into pinned host memory so that the host
 // can bound the counters without waiting for the stream. Both counters carry the low bits of the request's number above

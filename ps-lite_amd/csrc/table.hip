@@ -402,6 +402,7 @@ struct pskv_table {
   unsigned push_looks = 0;                // k_fixed_own: how often a workgroup looks for the verdict
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
   int streams = -1;                       // pushes stream through the slot array: where it pays, or (0, 1) never, wherever they can
+  bool packing = false;                   // a comparison has been asked to pack the cached keys (PackedKeys)
   unsigned stream_turn = 0;               // the counter of left keys that the newest of them used
 
   bool prof = false;
@@ -1048,6 +1049,7 @@ void note_outcomes(pskv_table* t) {
     tr.fail = std::min(tr.fail + 1u, 6u);
     tr.skip = 1u << tr.fail;
     tr.hit = false;
+    t->packing = false;
   }
 }
 
@@ -1080,6 +1082,10 @@ ReqTag next_tag(pskv_table* t, const Request& r, bool back_off = false) {
 // single short launch either way, and the cache would add two). The environment variable
 // PSKV_SCALAR_CACHE_MIN_KEYS, read when a table is created, overrides it (0 switches the cache off).
 constexpr uint64_t kScalarCacheMinKeys = 1u << 17;
+
+// Cached keys of at least this many are packed once a request has repeated them (8 MB of them: the time of smaller ones is the
+// launches'). Figures: PackedKeys.
+constexpr uint64_t kPackKeys = 1u << 20;
 
 // How a SCALAR request of one table relates to the table's key cache.
 enum ScalarCacheUse {
@@ -1271,7 +1277,7 @@ std::vector<Streamed> pick_streamed(Batch& bt, const std::vector<ScalarPlan>& pl
 int run_scalar(Batch& bt, bool push, bool pull) {
   Growths growths;
   uint64_t n_largest = 0;
-  bool any_cache = false, behind = false;
+  bool any_cache = false, behind = false, packs = false, packed = false;
   std::vector<ScalarPlan> plan(bt.size());
   for (size_t i = 0; i < bt.size(); ++i) {
     Item& it = bt[i];
@@ -1335,8 +1341,9 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       // the buffers have the cached request's size). Only a request that is going to be recorded
       // pays for it: a one-off pull of 16M keys would otherwise allocate 256 MB it never uses, and
       // wait for the stream to do so.
-      rc = grow(t, &t->cache_keys, r.n * sizeof(uint64_t));
+      rc = grow(t, &t->cache_keys, PackedKeys::bytes(r.n));
       if (rc) return rc;
+      t->packing = false;
       rc = grow(t, &t->sc_vals, r.n * sizeof(float));
       if (rc) return rc;
       rc = grow(t, &t->sc_slots, r.n * sizeof(uint32_t));
@@ -1359,6 +1366,16 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       const bool per_key = plan[i].use == kScTry && !push && !t->sc_dirty && plan[i].kind_before == 0 && r.replay != kReplayCapture;
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
+      if (!per_key && it.tag.try_cache && !r.replay && r.n >= kPackKeys) {
+        // (as far as the host has been told; the device looks)
+        const unsigned long long told = static_cast<volatile unsigned long long*>(t->outcome)[2];
+        if (told == kNoLongerPacked) t->packing = false;
+        if (!t->packing && t->sc_track[r.push ? 0 : 1].hit) {
+          t->packing = packs = true;
+        } else if (t->packing && told == kArePacked) {
+          packed = true;
+        }
+      }
       // (a recorded repeat is served from the cache or not at all: nothing to write back)
       if (!per_key && it.tag.try_cache && t->sc_dirty && r.replay != kReplayCapture) {
         d.cache_mode = kCacheOnBehind;
@@ -1402,9 +1419,12 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   }
   const bool one_launch = repeat_quads != 0;
   if (any_cache && !one_launch) {
-    rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, PSKV_KSET(k_same_keys), [](const Item& it) {
-      return ((it.d.cache_mode == kCacheOn || it.d.cache_mode == kCacheOnBehind) && it.tag.try_cache)
-                 ? (it.r.n + kBlock * kSameKeysItems - 1) / (kBlock * kSameKeysItems) : 0ull;
+    // (one kernel for all tables: the packed ones', where one of them has been told to be packed, compares the others' keys too)
+    const uint64_t per = packs || packed ? (uint64_t)kBlock * PackedKeys::kItems : (uint64_t)kBlock * kSameKeysItems;
+    const KernelSet kernels = packs    ? PSKV_KSET_OF(k_same_packed, true)
+                              : packed ? PSKV_KSET_OF(k_same_packed, false) : PSKV_KSET(k_same_keys);
+    rc = launch_batch(bt, PSKV_KERNEL_SAME_KEYS, kernels, [&](const Item& it) {
+      return ((it.d.cache_mode == kCacheOn || it.d.cache_mode == kCacheOnBehind) && it.tag.try_cache) ? (it.r.n + per - 1) / per : 0ull;
     });
     if (rc) return rc;
   }
@@ -2471,7 +2491,7 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   for (int q = 0; q < kSmallParts; ++q) t->small_done[q] = t->shell->done[q];
   std::memset(t->st_host, 0, sizeof(StateView));
   std::memset(t->snap, 0xFF, sizeof(Snapshot));  // names no request
-  t->outcome[0] = t->outcome[1] = 0ull;
+  t->outcome[0] = t->outcome[1] = t->outcome[2] = 0ull;
   const uint64_t keys = opts->initial_capacity ? opts->initial_capacity : kDefaultCapacity;
   t->cap = std::max(kMinSlots, next_pow2((uint64_t)((double)keys / t->max_load) + 1));
   int rc = alloc_slots(t->cap, &t->slots, t->stream);

@@ -379,6 +379,42 @@ __device__ __forceinline__ void decide_same(DevState* st, const ReqTag& tag, boo
   if (outcome && tag.try_cache) *outcome = (tag.epoch << 1) | (same ? 1ull : 0ull);
 }
 
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// What the workgroups of a comparison come to, found by the last of them. `how`: kComparesKeys, or kComparesPacked, or kPacksKeys,
+// with kReqWide where this lane's could not be packed.
+constexpr unsigned kComparesKeys = 0u, kComparesPacked = 1u, kPacksKeys = 2u;
+// what the host is told in outcome[2]: whether the keys are packed, or that a comparison has expected them to be
+constexpr unsigned long long kNotPacked = 0ull, kArePacked = 1ull, kNoLongerPacked = 2ull;
+__device__ __forceinline__ void same_keys_verdict(const TableHead& d, bool differ, unsigned how) {
+  DevState* st = d.st;
+  __shared__ unsigned s_last;
+  const int any = __syncthreads_or(differ ? 1 : 0);
+  const int wide = how & kPacksKeys ? __syncthreads_or(how & kReqWide ? 1 : 0) : 0;
+  if (threadIdx.x == 0) {
+    if (any || wide) report_facts(st, (any ? kReqDiffer : 0u) | (wide ? kReqWide : 0u), d.nblk);
+    s_last = ticket_last(st, d.nblk) ? 1u : 0u;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  if (threadIdx.x >= 64) return;
+  const unsigned found = take_facts(st, d.nblk);
+  const bool same = (found & kReqDiffer) == 0u && cache_usable(st, d.tag);
+  if (threadIdx.x != 0) return;
+  if (!same && d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch) {
+    st->behind_epoch = d.tag.epoch;
+    st->clean_epoch = st->dirty_epoch;  // (by the end of the request)
+  }
+  if (how & kPacksKeys) {
+    const bool packed = same && !(found & kReqWide);
+    st->packed_epoch = packed ? st->cache_epoch : 0ull;
+    if (d.outcome) d.outcome[2] = packed ? kArePacked : kNotPacked;
+  } else if (how == kComparesPacked && st->packed_epoch != st->cache_epoch) {
+    if (d.outcome) d.outcome[2] = kNoLongerPacked;
+  }
+  decide_same(st, d.tag, same, d.outcome);
+}
+
 // Compares the keys of a request with the cached ones and reaches the decision for the whole
 // request: the workgroup that finishes last sees whether any workgroup found a difference and
 // writes same_epoch. (A var-len push, whose lens count as well, compares in k_var_push_begin.)
@@ -391,8 +427,6 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
   const uint64_t* __restrict__ cache_keys = d.cache_keys;
   const uint64_t n = d.n;
   DevState* st = d.st;
-  const ReqTag tag = d.tag;
-  __shared__ unsigned s_last;
   constexpr int kItems = kSameKeysItems;
   static_assert(kItems % 2 == 0, "two keys per 128-bit load");
   const uint64_t base = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * kItems;
@@ -429,22 +463,110 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
         if (a[j] != c[j]) write_back(d, base + j);
     }
   }
-  const int any = __syncthreads_or(differ ? 1 : 0);
-  if (threadIdx.x == 0) {
-    if (any) report_facts(st, kReqDiffer, d.nblk);
-    s_last = ticket_last(st, d.nblk) ? 1u : 0u;
+  same_keys_verdict(d, differ, kComparesKeys);
+}
+
+// Cached keys are compared again and again while a request repeats, and of sorted keys not all has to be read for that.
+// SCALAR tables keep, behind the cached keys, what each of them is above the one in front of it, in 48 bits. A wavefront compares
+// its first key whole and the other 511 by what they add, which says that they are equal, or not, as surely; where they are
+// not it reads the cached keys themselves. They lie as the lanes read them: per wavefront and lane the lower 32 bits of its
+// eight keys, then the upper 16. PACK: a comparison with the cached keys themselves, which leaves them packed if they are the
+// request's, told to the host then; not where two neighbours are 2^48 or more apart, nor for keys that are not sorted.
+// Bound by memory: 14 B per key instead of 16. Push and pull of 16M repeated keys took 130 us and take 122.6 (three tables on three
+// streams in turn: 145.8 and 137), of 8M 73.1 and 69.1, of 2M 26 and 24.5, of 1M 18.6 and 18.4. The packed words are left in the
+// memory-side cache: loads that pass it by take 16M keys of three tables down to 121 us, but those of one alone up to 134-139.
+// 52 registers: with the cached keys themselves held as well (140) three wavefronts per SIMD took longer than what was read less.
+struct PackedKeys {
+  static constexpr int kItems = 8, kPairs = kItems / 2;  // keys of a lane: pairs of neighbours, 128 keys apart
+  static constexpr uint64_t kBlockKeys = 64 * kItems;
+  __host__ __device__ static constexpr uint64_t blocks(uint64_t n) { return (n + kBlockKeys - 1) / kBlockKeys; }
+  __host__ __device__ static constexpr size_t bytes(uint64_t n) { return blocks(n) * kBlockKeys * (8 + 6); }  // the keys' own included
+  __device__ static u32x4* block(uint64_t* keys, uint64_t n, uint64_t b) {
+    return reinterpret_cast<u32x4*>(keys + blocks(n) * kBlockKeys) + b * (kBlockKeys * 6 / 16);
   }
-  __syncthreads();
-  if (!s_last) return;
-  if (threadIdx.x >= 64) return;
-  const bool same = (take_facts(st, d.nblk) & kReqDiffer) == 0u && cache_usable(st, tag);
-  if (threadIdx.x == 0) {
-    if (!same && d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch) {
-      st->behind_epoch = tag.epoch;
-      st->clean_epoch = st->dirty_epoch;  // (by the end of the request)
+};
+template <bool PACK, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_same_packed(HeadBatch<TABLES> b) {
+  const TableHead& d = b.t[blockIdx.y];
+  if (blockIdx.x >= d.nblk) return;
+  const uint64_t* __restrict__ keys = d.keys;
+  uint64_t* const cache_keys = d.cache_keys;
+  const uint64_t n = d.n;
+  const DevState* st = d.st;
+  constexpr int kPairs = PackedKeys::kPairs;
+  const uint64_t wave = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const unsigned lane = threadIdx.x & 63;
+  const uint64_t base = wave * PackedKeys::kBlockKeys + lane * 2;
+  const bool there = wave * PackedKeys::kBlockKeys < n, first = lane == 0;
+  const bool packed = !PACK && st->packed_epoch == st->cache_epoch && st->cache_epoch != 0ull;
+  u32x4* const block = PackedKeys::block(cache_keys, n, wave);
+  const bool vec = (reinterpret_cast<uintptr_t>(keys) & 15) == 0;
+  auto key_pair = [&](int q) {
+    const uint64_t i = base + q * 128;
+    u64x2 x;
+    if (vec && i + 2 <= n) {
+      x = __builtin_nontemporal_load(reinterpret_cast<const u64x2*>(keys + i));
+    } else {
+      x.x = i < n ? keys[i] : 0, x.y = i + 1 < n ? keys[i + 1] : 0;
     }
-    decide_same(st, tag, same, d.outcome);
+    return x;
+  };
+  auto cached_pair = [&](int q) {
+    const uint64_t i = base + q * 128;
+    u64x2 y;
+    if (i + 2 <= n) {
+      y = *reinterpret_cast<const u64x2*>(cache_keys + i);
+    } else {
+      y.x = i < n ? cache_keys[i] : 0, y.y = 0;
+    }
+    return y;
+  };
+  u64x2 a[kPairs];
+  u32x4 word[3] = {(u32x4)(0u), (u32x4)(0u), (u32x4)(0u)};
+  uint64_t whole = 0;
+#pragma unroll
+  for (int q = 0; q < kPairs; ++q) a[q] = key_pair(q);
+  if (!PACK && there) {
+#pragma unroll
+    for (int w = 0; w < 3; ++w) word[w] = block[w * 64 + lane];
+    if (first) whole = cache_keys[base];
   }
+  bool differ = !PACK && !packed && there, wide = false;
+#pragma unroll
+  for (int q = 0; q < kPairs; ++q) {
+    const uint64_t i = base + q * 128;
+    uint64_t before = __shfl_up((unsigned long long)a[q].y, 1);
+    const uint64_t end = __shfl((unsigned long long)a[q ? q - 1 : 0].y, 63);
+    if (first) before = end;
+    const uint64_t x = a[q].x - before, y = a[q].y - a[q].x;
+    const bool alone = first && q == 0;  // (the wavefront's first key is compared whole)
+    if (!PACK) {
+      const unsigned high = word[2][q];
+      const bool equal = alone ? a[q].x == whole : x == ((uint64_t)(high & 0xffffu) << 32 | word[q / 2][q % 2 * 2]);
+      differ |= i < n && !equal;
+      differ |= i + 1 < n && y != ((uint64_t)(high >> 16) << 32 | word[q / 2][q % 2 * 2 + 1]);
+    } else {
+      wide |= (i < n && !alone && x >> 48) || (i + 1 < n && y >> 48);
+      word[q / 2][q % 2 * 2] = (unsigned)x, word[q / 2][q % 2 * 2 + 1] = (unsigned)y;
+      word[2][q] = (unsigned)(x >> 32 & 0xffffu) | (unsigned)(y >> 32) << 16;
+    }
+  }
+  if (PACK && there) {
+#pragma unroll
+    for (int w = 0; w < 3; ++w) block[w * 64 + lane] = word[w];
+  }
+  if (PACK || __any(differ)) {  // the keys themselves
+    differ = false;
+    const bool ahead = d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch;  // (as in k_same_keys)
+#pragma unroll 1  // (rare: it may not take registers from the others)
+    for (int q = 0; q < kPairs; ++q) {
+      const u64x2 x = key_pair(q), y = cached_pair(q);
+      differ |= x.x != y.x || x.y != y.y;
+      if (ahead && x.x != y.x) write_back(d, base + q * 128);
+      if (ahead && x.y != y.y) write_back(d, base + q * 128 + 1);
+    }
+  }
+  same_keys_verdict(d, differ, PACK ? kPacksKeys | (wide ? kReqWide : 0u) : kComparesPacked);
 }
 
 // A recorded SCALAR request of up to kRepeatGroups workgroups: comparison and values in ONE launch. Nothing
