@@ -1521,6 +1521,16 @@ int launch_rows_piece(Batch& bt, int op, uint64_t first, uint64_t floats) {
   return rc;
 }
 
+// FIXED: whether all rows of a launch are wide ones, and the kernels for them. (A request that is served in pieces waits for the host
+// link, whatever its kernel.)
+bool all_wide(const Batch& bt) {
+  return std::all_of(bt.begin(), bt.end(), [](const Item& it) { return !it.d.ntiles || it.d.k >= kWideRow; });
+}
+KernelSet wide_kernels(int op, bool stream) {
+  if (op == kOpAcc) return stream ? PSKV_KSET_OF(k_rows_wide, kOpAcc, true) : PSKV_KSET_OF(k_rows_wide, kOpAcc, false);
+  return stream ? PSKV_KSET_OF(k_rows_wide, kOpGather, true) : PSKV_KSET_OF(k_rows_wide, kOpGather, false);
+}
+
 // The row kernel over every table of the batch whose TableReq::total is not zero.
 template <bool VARLEN>
 int launch_rows(Batch& bt, int op) {
@@ -1560,6 +1570,8 @@ int launch_rows(Batch& bt, int op) {
     return (it.d.ntiles + kQuadsFixed - 1) / kQuadsFixed;
   };
   const bool stream = floats >= kStreamFloats;
+  const int kind = op == kOpAcc ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER;
+  if (!VARLEN && all_wide(bt)) return launch_batch(bt, kind, wide_kernels(op, stream), nblk);
   bool started = false;
   for (const Item& it : bt) started = started || (VARLEN && it.d.started);
   bool by_row = false;
@@ -1576,7 +1588,7 @@ int launch_rows(Batch& bt, int op) {
   const KernelSet kernels = op == kOpAcc ? (by_row ? (started ? pick(Acc(), Yes(), Yes()) : pick(Acc(), No(), Yes()))
                                                    : (started ? pick(Acc(), Yes(), No()) : pick(Acc(), No(), No())))
                                          : (started ? pick(Gather(), Yes(), No()) : pick(Gather(), No(), No()));
-  return launch_batch(bt, op == kOpAcc ? PSKV_KERNEL_ROWS_ACC : PSKV_KERNEL_ROWS_GATHER, kernels, nblk);
+  return launch_batch(bt, kind, kernels, nblk);
 }
 
 // Starts a row-mode request on every table with keys: numbers it and (`compare`: a recorded one), where the

@@ -1352,6 +1352,58 @@ __device__ __forceinline__ void rows_quads_fixed(const RowsParams& p, uint64_t q
   }
 }
 
+// The same for rows of kWideRow floats and more, which a workgroup meets one or two of. Bound by memory, as long as a wavefront asks
+// early: all arguments in one fetch, then the request's values, then the two references, through the scalar cache, so that nothing
+// waits for anything but the row for its reference. Above, arguments, facts and reference are four waits one behind the other
+// and the values are waited for with the reference: 64 rows of 4M floats, four pushes and a pull of three tables in turn, 2,460 us
+// against 2,395 here (6.1 and 6.3 TB/s), 300 of 100,010 318 and 308, 3 of 4.9M 178 and 170. Shorter rows, scattered over the
+// arena, gain nothing from it (64 floats 633 and 634-639, 48 floats 158 and 161: the memory has enough to do).
+constexpr uint64_t kWideRow = 1024;
+typedef const __attribute__((address_space(4))) uint64_t* ScalarWords;  // what no workgroup of this launch writes
+template <int OP, bool STREAM, bool REST>
+__device__ __forceinline__ void rows_quads_wide(const TableReq& d, uint64_t q0) {
+  // (asked for first, and not waited for before the references have come)
+  unsigned long long same_epoch = d.st->same_epoch, refused = OP == kOpAcc ? d.st->refused_epoch : 0ull;
+  const uint64_t quads = (d.k + 3) >> 2;
+  const unsigned rest = REST ? (unsigned)d.k & 3u : 0u;
+  if (threadIdx.x >= d.ntiles - q0) return;
+  f32x4 x = (f32x4)(0.f);
+  if (OP == kOpAcc && !REST) x = load_quad<STREAM>(d.req + (q0 + threadIdx.x) * 4);
+  const uint64_t row0 = q0 / quads;
+  const uint64_t c0 = q0 - row0 * quads + threadIdx.x;
+  const bool over = c0 >= quads;
+  const ScalarWords refs = (ScalarWords)reinterpret_cast<uintptr_t>(d.ref);
+  uint64_t ra = refs[row0], rb = refs[row0 + 1 < d.n ? row0 + 1 : row0];
+  const uint64_t row = row0 + (over ? 1u : 0u), c = over ? c0 - quads : c0;
+  const unsigned count = REST && c + 1 == quads ? rest : 4u;
+  float* side = d.req + row * d.k + c * 4;
+  if (OP == kOpAcc && REST)  // (as in rows_quads_fixed)
+    x = count == 4 || whole_quads(row + 1, d.k, d.n) ? load_quad<STREAM>(side) : load_part<STREAM>(side, rest);
+  asm volatile("" : "+s"(ra), "+s"(rb), "+v"(same_epoch), "+v"(refused));
+  const uint64_t r = over ? rb : ra;
+  const bool same = same_epoch == d.tag.epoch;
+  if (d.tag.replay && !same) return;
+  if (r == kRefAbsent) return;  // a key the lookup refused (duplicate in the request, full table)
+  const bool rejected = OP == kOpAcc && refused == d.tag.epoch;
+  const bool fresh = (r & kRefNew) != 0 && !d.ignore_new && !same;
+  float* dst = d.arena + (r & ~kRefNew) * d.k + c * 4;
+  f32x4 y = (f32x4)(0.f);
+  if (!fresh) y = load_quad<STREAM>(dst);
+  if (OP == kOpAcc) {
+    if (rejected) {
+      if (!fresh) return;
+    } else {
+      y = y + x;  // a created row is a zero row first (0.0f + v), kv_app.h:454
+    }
+    if (!REST || count == 4) store_quad<STREAM>(y, dst); else store_part<STREAM>(y, dst, rest);
+  } else {
+    if (!REST || count == 4) store_quad<STREAM>(y, side); else store_part<STREAM>(y, side, rest);
+    if (fresh) {  // pull created the row: zeros
+      if (!REST || count == 4) store_quad<STREAM>(y, dst); else store_part<STREAM>(y, dst, rest);
+    }
+  }
+}
+
 // VARLEN rows: a WAVEFRONT owns WTILE consecutive request-side floats. The tile table names
 // the first key that overlaps them; the wavefront stages the offsets and row references of
 // the keys that overlap its tile in its own piece of LDS (no workgroup barrier: the four
@@ -1791,6 +1843,22 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
     } else {
       rows_quads_fixed<OP, STREAM, false>(p, q0, d.ntiles);
     }
+  }
+}
+
+template <int OP, bool STREAM, int TABLES>
+__global__ __launch_bounds__(kBlock) void k_rows_wide(ReqBatch<TABLES> b) {
+  const TableReq& d = b.t[blockIdx.y];
+  unsigned blk = blockIdx.x;
+  // (the arguments asked for at once: fetched group by group where they are first used, each group is a wait)
+  asm("" : "+s"(blk) : "s"(d.nvals), "s"(d.ntiles), "s"(d.req), "s"(d.arena), "s"(d.ref), "s"(d.st), "s"(d.n), "s"(d.k),
+      "s"(d.ignore_new), "s"(d.tag.epoch), "s"(d.tag.replay));
+  const uint64_t q0 = d.nvals + (uint64_t)blk * kQuadsFixed;
+  if (q0 >= d.ntiles) return;
+  if (d.k & 3) {
+    rows_quads_wide<OP, STREAM, true>(d, q0);
+  } else {
+    rows_quads_wide<OP, STREAM, false>(d, q0);
   }
 }
 

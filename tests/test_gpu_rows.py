@@ -170,3 +170,58 @@ def test_ragged_pushes_row_by_row(capi, orc, dev, which, n, S):
         got_keys, got_lens, got = group.tables[s].dump()
         assert np.array_equal(got_keys, want_keys) and np.array_equal(got_lens, want_lens)
         assert_bits_equal(got, want, "%s table %d" % (which, s))
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("k,n", [(1024, 2100), (1025, 8300), (1027, 2100), (4098, 1100), (1_500_001, 3)])
+def test_rows_of_a_workgroup_or_more(capi, orc, dev, k, n, shift):
+    """Requests beyond what one launch serves: new rows and held ones, pushed, pulled and both, and a push that is refused."""
+    announce("wide rows", k, n, shift)
+    import torch
+    rng = np.random.default_rng(k)
+    t, o = capi.Table(capi.MODE_FIXED, row_len=k), orc.Store(orc.MODE_FIXED, k)
+    keys = unique_keys(rng, n + n // 2)
+    for turn in range(4):
+        some = np.sort(rng.choice(keys, n, replace=False))
+        vals = rng.standard_normal(n * k).astype(np.float32)
+        out = _off_by(np.full(n * k, 7, np.float32), dev, 3 * shift)
+        if turn == 1:
+            t.pull(to_dev(some, dev), out)
+            want = o.pull(some)[0]
+        elif turn == 2:
+            t.pushpull(to_dev(some, dev), _off_by(vals, dev, shift), out)
+            want = o.pushpull(some, vals)[0]
+        else:
+            if turn == 3:
+                some[n // 2] = some[n // 2 - 1]
+            t.push(to_dev(some, dev), _off_by(vals, dev, shift))
+            if turn == 3:
+                with pytest.raises(capi.PskvError):
+                    t.sync()
+                break
+            o.push(some, vals)
+            continue
+        t.sync()
+        assert_bits_equal(out.cpu().numpy(), want, "k = %d" % k)
+    o.pull(some)  # (the rows that a refused push has made stay, as zero rows)
+    for mine, theirs in zip(t.dump(), o.dump()):
+        assert np.array_equal(mine, theirs) if mine.dtype != np.float32 else assert_bits_equal(mine, theirs) is None
+
+
+@pytest.mark.parametrize("k", [1024, 1030])
+def test_recorded_rows_of_a_workgroup_or_more(capi, orc, dev, k):
+    announce("wide rows, recorded", k)
+    import torch
+    rng = np.random.default_rng(k)
+    n, S = 41, 2
+    keys, vals = unique_keys(rng, n, S), rng.standard_normal(n * k).astype(np.float32)
+    group, o = capi.Group(S, capi.MODE_FIXED, row_len=k), orc.Store(orc.MODE_FIXED, k)
+    dk, dv, out = to_dev(keys, dev), to_dev(vals, dev), torch.zeros(n * k, device=dev)
+    pos, val_pos, _ = capi.slice_keys(dk, *capi.server_ranges(S), nvals=n * k)
+    rec = group.record(capi.REPLAY_PUSH | capi.REPLAY_PULL, dk, pos, dv, val_pos, out=out)
+    o.push(keys, vals)
+    for _ in range(3):
+        rec.run()
+        group.sync()
+        o.push(keys, vals)
+        assert_bits_equal(out.cpu().numpy(), o.pull(keys)[0])
