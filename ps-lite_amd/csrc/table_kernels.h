@@ -1759,9 +1759,14 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   // the grid is sized for the largest table of the launch: workgroups (VARLEN: wavefronts) past
   // this table's floats leave before they touch anything
   const bool by_row = BY_ROW && d.k != 0;
+  unsigned blk = blockIdx.x;
   if (VARLEN) {
-    const bool behind = by_row ? blockIdx.x + (STARTED && d.started ? 1u : 0u) >= d.nblk
-                               : (((uint64_t)blockIdx.x + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total;
+    // every argument the common path uses, asked for at once (the compiler otherwise fetches them group by group where they
+    // are first used, one wait each)
+    asm("" : "+s"(blk) : "s"(d.tile_base), "s"(d.total), "s"(d.st), "s"(d.req), "s"(d.arena), "s"(d.tile_aff), "s"(d.total_on_device),
+        "s"(d.tag.epoch), "s"(d.tag.try_cache), "s"(d.tag.replay), "s"(d.ignore_new), "s"(d.ref), "s"(d.off), "s"(d.tile_key), "s"(d.n));
+    const bool behind = by_row ? blk + (STARTED && d.started ? 1u : 0u) >= d.nblk
+                               : (((uint64_t)blk + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total;
     if (behind) {
       if (STARTED && d.started && blockIdx.x == d.nblk - 1) finish_start(d);  // (a workgroup behind the last one with floats)
       return;
@@ -1782,7 +1787,7 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   p.k = d.k;
   p.ignore_new = d.ignore_new;
   p.total_on_device = d.total_on_device;
-  p.blk = blockIdx.x + d.tile_base;
+  p.blk = blk + d.tile_base;
   p.tag = d.tag;
   __shared__ int32_t s_off[VARLEN ? (kWaveSpan + 1) * (kBlock / 64) : 1];
   __shared__ uint64_t s_ref[VARLEN ? kWaveSpan * (kBlock / 64) : 1];
@@ -1790,10 +1795,6 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   const ReqFacts facts = load_req_facts(p.st);
   const unsigned long long refused = STARTED && OP == kOpAcc ? p.st->refused_epoch : 0ull;
   if (VARLEN) {
-    // every argument the common path uses, asked for at once (the compiler otherwise fetches them
-    // group by group where they are first used, one wait each)
-    asm volatile("" ::"s"(p.req), "s"(p.arena), "s"(p.tile_aff), "s"(p.total),
-                 "s"(p.total_on_device), "s"(p.tag.epoch));
     // the grid covers the room in the caller's buffer, which may be more than the data; the loads
     // that need no facts are on their way before the facts are looked at
     uint64_t total = p.total;
