@@ -476,7 +476,7 @@ def run_dense(args, capi, dev):
                    "keys_per_step": nk, "value_len": k},
         # 4 B in + 4 B row read + 4 B row write per float
         "roofline": dict(roofline(12.0 * floats, acc[0], acc[1], traffic("rows_acc_fixed", floats), acc[2]),
-                         kernel="k_rows<acc,fixed> (row += in)", bytes_per_float=12),
+                         kernel="k_rows_wide<acc> (row += in)", bytes_per_float=12),
         "kernels": {"rows_gather": dict(roofline(8.0 * floats, gat[0], gat[1],
                                                  traffic("rows_gather_fixed", floats), gat[2]),
                                         bytes_per_float=8),
@@ -977,9 +977,9 @@ def run_sparse_repeat(args, capi, dev):
         "kernels": {"pull_scalar_cached": dict(roofline(8.0 * n, pull[0], pull[1],
                                                         traffic("pull_scalar_cached", n), pull[2]),
                                                bytes_per_key=8),
-                    "same_keys": dict(roofline(16.0 * n, same[0], same[1], traffic("same_keys", n), same[2]),
-                                      kernel="k_same_keys (request keys against cached keys), once per "
-                                             "push and once per pull", bytes_per_key=16)},
+                    "same_keys": dict(roofline(14.0 * n, same[0], same[1], traffic("same_keys", n), same[2]),
+                                      kernel="k_same_packed (request keys against cached keys of 48 bits), once per "
+                                             "push and once per pull", bytes_per_key=14)},
     }
     return res, (keys, vals, n)
 
