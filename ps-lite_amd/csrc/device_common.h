@@ -9,6 +9,15 @@
 // Asks for all of a kernel's arguments at once (the compiler otherwise fetches them group by group where they are first
 // used, one wait each).
 #define PSKV_ASK_ARGS(...) asm volatile("" ::__VA_ARGS__)
+// The same in front of what `x`, a word that is the same for all lanes, is used for, and in the way of no scalar load behind it.
+// (The kernels are also compiled for the CPU, which knows no such registers.)
+#ifdef __HIP__
+#define PSKV_SCALAR "s"
+#define PSKV_ASK_ARGS_FOR(x, ...) asm("" : "+" PSKV_SCALAR(x) : __VA_ARGS__)
+#else
+#define PSKV_SCALAR "r"
+#define PSKV_ASK_ARGS_FOR(x, ...) (void)0
+#endif
 
 namespace pskv {
 

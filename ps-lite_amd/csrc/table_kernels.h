@@ -1379,7 +1379,7 @@ __device__ __forceinline__ void rows_quads_wide(const TableReq& d, uint64_t q0) 
   float* side = d.req + row * d.k + c * 4;
   if (OP == kOpAcc && REST)  // (as in rows_quads_fixed)
     x = count == 4 || whole_quads(row + 1, d.k, d.n) ? load_quad<STREAM>(side) : load_part<STREAM>(side, rest);
-  asm volatile("" : "+s"(ra), "+s"(rb), "+v"(same_epoch), "+v"(refused));
+  asm volatile("" : "+" PSKV_SCALAR(ra), "+" PSKV_SCALAR(rb), "+v"(same_epoch), "+v"(refused));
   const uint64_t r = over ? rb : ra;
   const bool same = same_epoch == d.tag.epoch;
   if (d.tag.replay && !same) return;
@@ -1763,7 +1763,7 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   if (VARLEN) {
     // every argument the common path uses, asked for at once (the compiler otherwise fetches them group by group where they
     // are first used, one wait each)
-    asm("" : "+s"(blk) : "s"(d.tile_base), "s"(d.total), "s"(d.st), "s"(d.req), "s"(d.arena), "s"(d.tile_aff), "s"(d.total_on_device),
+    PSKV_ASK_ARGS_FOR(blk, "s"(d.tile_base), "s"(d.total), "s"(d.st), "s"(d.req), "s"(d.arena), "s"(d.tile_aff), "s"(d.total_on_device),
         "s"(d.tag.epoch), "s"(d.tag.try_cache), "s"(d.tag.replay), "s"(d.ignore_new), "s"(d.ref), "s"(d.off), "s"(d.tile_key), "s"(d.n));
     const bool behind = by_row ? blk + (STARTED && d.started ? 1u : 0u) >= d.nblk
                                : (((uint64_t)blk + d.tile_base) * (kBlock / 64) + (threadIdx.x >> 6)) * kTileVar >= d.total;
@@ -1852,7 +1852,7 @@ __global__ __launch_bounds__(kBlock) void k_rows_wide(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   unsigned blk = blockIdx.x;
   // (the arguments asked for at once: fetched group by group where they are first used, each group is a wait)
-  asm("" : "+s"(blk) : "s"(d.nvals), "s"(d.ntiles), "s"(d.req), "s"(d.arena), "s"(d.ref), "s"(d.st), "s"(d.n), "s"(d.k),
+  PSKV_ASK_ARGS_FOR(blk, "s"(d.nvals), "s"(d.ntiles), "s"(d.req), "s"(d.arena), "s"(d.ref), "s"(d.st), "s"(d.n), "s"(d.k),
       "s"(d.ignore_new), "s"(d.tag.epoch), "s"(d.tag.replay));
   const uint64_t q0 = d.nvals + (uint64_t)blk * kQuadsFixed;
   if (q0 >= d.ntiles) return;
