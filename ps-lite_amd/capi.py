@@ -154,6 +154,10 @@ def _is_tensor(x):
     return hasattr(x, "data_ptr")
 
 
+class _Address(int):
+    """The address of an array, which lives as long as its address does (it may be a copy that nobody else holds)."""
+
+
 def _buf(x, dtype_np, dtype_name):
     """(pointer, element count, memkind or None) of a numpy array / torch tensor / None."""
     if x is None:
@@ -164,7 +168,10 @@ def _buf(x, dtype_np, dtype_name):
         kind = MEM_DEVICE if x.is_cuda else MEM_HOST
         return (x.data_ptr() if x.numel() else None), x.numel(), kind
     a = np.ascontiguousarray(x, dtype=dtype_np)
-    return (a.ctypes.data if a.size else None), a.size, MEM_HOST
+    at = _Address(a.ctypes.data) if a.size else None
+    if at:
+        at.of = a
+    return at, a.size, MEM_HOST
 
 
 def _memkind(*kinds):
