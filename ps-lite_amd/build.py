@@ -7,6 +7,8 @@ import os
 import subprocess
 import sysconfig
 
+import numpy
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
@@ -63,7 +65,7 @@ def build_lib(verbose=False):
 def build_native():
     """Compiles the per-request half of the Python binding (csrc/pymodule.cc) against the library."""
     cmd = ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
-           "-I" + os.path.join(REPO, "include"), "-I" + sysconfig.get_paths()["include"],
+           "-I" + os.path.join(REPO, "include"), "-I" + sysconfig.get_paths()["include"], "-I" + numpy.get_include(),
            os.path.join(CSRC, "pymodule.cc"), "-L" + HERE, "-lpskv", "-Wl,-rpath,$ORIGIN", "-L/opt/rocm/lib",
            "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-o", NATIVE]
     subprocess.run(cmd, check=True)

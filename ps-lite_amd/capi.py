@@ -560,14 +560,11 @@ def slice_keys(keys, range_begin, range_end, lens=None, nvals=0, device=0):
     if _native is None:
         load()
     if isinstance(range_begin, np.ndarray) and range_begin.ndim == 1:
-        S = range_begin.size
-        pos, val_pos = np.zeros((2, S + 1), np.uint64)
-        used = np.zeros(max(S, 1), np.uint8)
-        rc = _native.slice(device, keys, lens, nvals, range_begin, range_end, pos, val_pos, used)
-        if rc is not None:
-            if rc:
-                _check(rc)
-            return pos, val_pos, used if S else used[:0]
+        got = _native.slice(device, keys, lens, nvals, range_begin, range_end)
+        if got is not None:
+            if isinstance(got, int):
+                _check(got)
+            return got
     kp, n, k1 = _buf(keys, np.uint64, "int64")
     lp, nl, k2 = _buf(lens, np.int32, "int32")
     rb = np.ascontiguousarray(range_begin, dtype=np.uint64)

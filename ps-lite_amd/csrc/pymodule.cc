@@ -8,6 +8,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <hip/hip_runtime_api.h>
+#define NPY_NO_DEPRECATED_API NPY_1_7_API_VERSION
+#include <numpy/arrayobject.h>
 #include <stdint.h>
 
 #include "pskv/capi.h"
@@ -31,6 +33,9 @@ class Arg {
   // 1 taken, 0 not for the quick way, -1 a Python error is set
   int take(PyObject* o, char type) {
     if (o == Py_None) return 1;
+    // (a numpy array is looked at itself: its buffer costs 50 ns to ask for and to give back, and a slice of a request has six.
+    // The caller's arguments keep it.)
+    if (PyArray_CheckExact(o)) return array(reinterpret_cast<PyArrayObject*>(o), type);
     if (g_tensor_type && PyObject_TypeCheck(o, reinterpret_cast<PyTypeObject*>(g_tensor_type))) return tensor(o, type);
     if (!PyObject_CheckBuffer(o)) return 0;
     if (PyObject_GetBuffer(o, &view_, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) {
@@ -56,6 +61,18 @@ class Arg {
   PyObject* device_tensor = nullptr;  // borrowed
 
  private:
+  int array(PyArrayObject* a, char type) {
+    const int t = PyArray_TYPE(a);
+    const bool fits = type == 'k'   ? t == NPY_ULONG || t == NPY_ULONGLONG
+                      : type == 'f' ? t == NPY_FLOAT
+                      : type == 'b' ? t == NPY_UBYTE
+                                    : t == NPY_INT;
+    if (!fits || !PyArray_IS_C_CONTIGUOUS(a) || !PyArray_ISALIGNED(a) || !PyArray_ISNOTSWAPPED(a)) return 0;
+    n = (size_t)PyArray_SIZE(a);
+    ptr = n ? PyArray_DATA(a) : nullptr;
+    kind = kHost;
+    return 1;
+  }
   int tensor(PyObject* o, char type) {
     PyObject* d = PyObject_GetAttr(o, s_dtype);
     if (!d) return -1;
@@ -283,34 +300,41 @@ PyObject* group_pushpull(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(rc);
 }
 
-// slice(device, keys, lens, nvals, range_begin, range_end, pos, val_pos, used): the outputs are host arrays of
-// S+1, S+1 and at least S entries
+// slice(device, keys, lens, nvals, range_begin, range_end): (pos, val_pos, used), or a status
 PyObject* slice(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (!want(n, 9)) return nullptr;
+  if (!want(n, 6)) return nullptr;
   const long device = PyLong_AsLong(a[0]);
   const size_t nvals = PyLong_AsSize_t(a[3]);
   if (PyErr_Occurred()) {  // (a numpy integer, say)
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  Arg x[2], begin, end, pos, val_pos, used;
+  Arg x[2], begin, end;
   int kind, rc;
   NOT_QUICK(begin.take(a[4], 'k'));
   NOT_QUICK(end.take(a[5], 'k'));
-  NOT_QUICK(pos.take(a[6], 'k'));
-  NOT_QUICK(val_pos.take(a[7], 'k'));
-  NOT_QUICK(used.take(a[8], 'b'));
   const size_t S = begin.n;
-  if (begin.kind != kHost || end.kind != kHost || end.n != S || pos.n != S + 1 || val_pos.n != S + 1 || used.n < S)
-    Py_RETURN_NONE;
+  if (begin.kind != kHost || end.kind != kHost || end.n != S) Py_RETURN_NONE;
   NOT_QUICK(take_all(x, a + 1, "ki", 2, Py_None, &kind));
-  Py_BEGIN_ALLOW_THREADS;
-  rc = pskv_slice((int)device, static_cast<uint64_t*>(x[0].ptr), x[0].n, static_cast<int32_t*>(x[1].ptr), x[1].n,
-                  nvals, static_cast<uint64_t*>(begin.ptr), static_cast<uint64_t*>(end.ptr), S,
-                  static_cast<uint64_t*>(pos.ptr), static_cast<uint64_t*>(val_pos.ptr),
-                  static_cast<uint8_t*>(used.ptr), kind);
-  Py_END_ALLOW_THREADS;
-  return PyLong_FromLong(rc);
+  npy_intp bounds = (npy_intp)S + 1, ranges = (npy_intp)S;
+  PyObject* pos = PyArray_SimpleNew(1, &bounds, NPY_UINT64);
+  PyObject* val_pos = PyArray_SimpleNew(1, &bounds, NPY_UINT64);
+  PyObject* used = PyArray_SimpleNew(1, &ranges, NPY_UINT8);
+  PyObject* result = nullptr;
+  if (pos && val_pos && used) {
+    uint64_t* p = static_cast<uint64_t*>(PyArray_DATA(reinterpret_cast<PyArrayObject*>(pos)));
+    uint64_t* v = static_cast<uint64_t*>(PyArray_DATA(reinterpret_cast<PyArrayObject*>(val_pos)));
+    uint8_t* u = static_cast<uint8_t*>(PyArray_DATA(reinterpret_cast<PyArrayObject*>(used)));
+    Py_BEGIN_ALLOW_THREADS;
+    rc = pskv_slice((int)device, static_cast<uint64_t*>(x[0].ptr), x[0].n, static_cast<int32_t*>(x[1].ptr), x[1].n,
+                    nvals, static_cast<uint64_t*>(begin.ptr), static_cast<uint64_t*>(end.ptr), S, p, v, u, kind);
+    Py_END_ALLOW_THREADS;
+    result = rc ? PyLong_FromLong(rc) : PyTuple_Pack(3, pos, val_pos, used);
+  }
+  Py_XDECREF(pos);
+  Py_XDECREF(val_pos);
+  Py_XDECREF(used);
+  return result;
 }
 
 // match(device, src_keys, src_vals, dst_keys, dst_vals, k, op)
@@ -367,6 +391,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 }  // namespace
 
 PyMODINIT_FUNC PyInit__native(void) {
+  import_array();
   s_dtype = PyUnicode_InternFromString("dtype");
   s_is_cuda = PyUnicode_InternFromString("is_cuda");
   s_is_contiguous = PyUnicode_InternFromString("is_contiguous");
