@@ -134,9 +134,15 @@ __device__ __forceinline__ void arrived(T& x) {
 template <bool PUSH, bool PULL, bool CACHE, bool PINNED, bool BEHIND, int TABLES>
 __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
   const TableHead& d = b.t[blockIdx.y];
+  unsigned blk = blockIdx.x;
+  // (one fetch instead of three: a push of 1,000 keys from host memory occupies its stream for 4.22 us and not 4.45, a pull is back after
+  // 11.5 and not 11.7. The other variants gain nothing beyond noise.)
+  if (PINNED)
+    PSKV_ASK_ARGS_FOR(blk, "s"(d.n), "s"(d.nblk), "s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.vals), "s"(d.out),
+                      "s"(d.cache_mode), "s"(d.snap), "s"(d.snap_seq), "s"(d.tag.epoch));
   const uint64_t n = d.n;
   const unsigned nblk = d.nblk;  // (the grid is sized for the table with the most workgroups)
-  if (blockIdx.x >= nblk) return;
+  if (blk >= nblk) return;
   Slot* __restrict__ slots = d.slots;
   const uint64_t mask = d.mask;
   DevState* st = d.st;
@@ -148,10 +154,10 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
   if (record && __builtin_expect(cache_same(st, d.tag), BEHIND)) {
     // the keys are those of the cached request: position i of the request is position i of the cache
     float* __restrict__ cv = d.arena;
-    if (PUSH && blockIdx.x == 0 && threadIdx.x == 0) st->dirty_epoch = d.tag.epoch;  // the slots fall behind
+    if (PUSH && blk == 0 && threadIdx.x == 0) st->dirty_epoch = d.tag.epoch;  // the slots fall behind
     const bool vec = ((reinterpret_cast<uintptr_t>(vals) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
     const uint64_t stride = (uint64_t)nblk * kBlock * 4;
-    for (uint64_t i = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * 4; i < n; i += stride) {
+    for (uint64_t i = ((uint64_t)blk * kBlock + threadIdx.x) * 4; i < n; i += stride) {
       if (vec && i + 4 <= n) {
         f32x4 cur = *reinterpret_cast<const f32x4*>(cv + i);
         if (PUSH) cur = cur + __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(vals + i));
@@ -167,11 +173,11 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
       }
     }
     // (no key is created on this path: the counters are what they were)
-    if (d.snap && blockIdx.x == 0 && threadIdx.x < 64) publish_snapshot(st, d.snap, d.snap_seq);
+    if (d.snap && blk == 0 && threadIdx.x < 64) publish_snapshot(st, d.snap, d.snap_seq);
     return;
   }
   const bool ahead = BEHIND && d.cache_mode == kCacheOnBehind && st->behind_epoch == d.tag.epoch;
-  if (record && blockIdx.x == 0 && threadIdx.x == 0) st->cache_epoch = d.tag.epoch;
+  if (record && blk == 0 && threadIdx.x == 0) st->cache_epoch = d.tag.epoch;
   constexpr bool kPerKey = CACHE && PULL && !PUSH;
   bool per_key = false, differs = false;
   if (kPerKey) {
@@ -189,7 +195,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
     const bool kvec = (reinterpret_cast<uintptr_t>(keys) & 15) == 0;
     const bool ovec = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     const uint64_t stride4 = (uint64_t)nblk * kBlock * 4;
-    for (uint64_t i = ((uint64_t)blockIdx.x * kBlock + threadIdx.x) * 4; i < n; i += stride4) {
+    for (uint64_t i = ((uint64_t)blk * kBlock + threadIdx.x) * 4; i < n; i += stride4) {
       if (i + 4 <= n) {
         u64x2 x0, x1;
         if (kvec) {
@@ -236,7 +242,7 @@ __global__ __launch_bounds__(kBlock, 8) void k_scalar(HeadBatch<TABLES> b) {
   const uint64_t stride = (uint64_t)nblk * kBlock;
   const unsigned lane = threadIdx.x & 63;
   // whole wavefronts stay in the loop together: the shuffles below need every lane
-  for (uint64_t first = (uint64_t)blockIdx.x * kBlock; first < n_turns; first += stride) {
+  for (uint64_t first = (uint64_t)blk * kBlock; first < n_turns; first += stride) {
     const uint64_t i = first + threadIdx.x;
     const bool live = i < n;
     uint64_t outside = 0;  // PINNED: the key next to the wavefront's 64 keys on this lane's side
