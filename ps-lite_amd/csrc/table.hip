@@ -1367,13 +1367,14 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
       if (!per_key && it.tag.try_cache && !r.replay && r.n >= kPackKeys) {
-        // (as far as the host has been told; the device looks)
-        const unsigned long long told = static_cast<volatile unsigned long long*>(t->outcome)[2];
-        if (told == kNoLongerPacked) t->packing = false;
-        if (!t->packing && t->sc_track[r.push ? 0 : 1].hit) {
+        // (packed they are as soon as they have been asked for, further up the stream; the device looks, and says where it was not so)
+        volatile unsigned long long* const told = t->outcome + 2;
+        if (*told == kNotPacked) t->packing = false;
+        if (t->packing) {
+          packed = packed || *told != kNeverPacked;
+        } else if (t->sc_track[r.push ? 0 : 1].hit) {
           t->packing = packs = true;
-        } else if (t->packing && told == kArePacked) {
-          packed = true;
+          *told = 0ull;
         }
       }
       // (a recorded repeat is served from the cache or not at all: nothing to write back)

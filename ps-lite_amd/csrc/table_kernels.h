@@ -390,8 +390,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // What the workgroups of a comparison come to, found by the last of them. `how`: kComparesKeys, or kComparesPacked, or kPacksKeys,
 // with kReqWide where this lane's could not be packed.
 constexpr unsigned kComparesKeys = 0u, kComparesPacked = 1u, kPacksKeys = 2u;
-// what the host is told in outcome[2]: whether the keys are packed, or that a comparison has expected them to be
-constexpr unsigned long long kNotPacked = 0ull, kArePacked = 1ull, kNoLongerPacked = 2ull;
+// What the host is told in outcome[2] when it expects packed keys that are not there: packed again they may be, or, as they lie too
+// far apart, never (then DevState::packed_epoch is the cached request's number and kCannotBePacked).
+constexpr unsigned long long kNotPacked = 1ull, kNeverPacked = 2ull, kCannotBePacked = 1ull << 63;
 __device__ __forceinline__ void same_keys_verdict(const TableHead& d, bool differ, unsigned how) {
   DevState* st = d.st;
   __shared__ unsigned s_last;
@@ -412,12 +413,10 @@ __device__ __forceinline__ void same_keys_verdict(const TableHead& d, bool diffe
     st->clean_epoch = st->dirty_epoch;  // (by the end of the request)
   }
   if (how & kPacksKeys) {
-    const bool packed = same && !(found & kReqWide);
-    st->packed_epoch = packed ? st->cache_epoch : 0ull;
-    if (d.outcome) d.outcome[2] = packed ? kArePacked : kNotPacked;
-  } else if (how == kComparesPacked && st->packed_epoch != st->cache_epoch) {
-    if (d.outcome) d.outcome[2] = kNoLongerPacked;
+    st->packed_epoch = same ? st->cache_epoch | (found & kReqWide ? kCannotBePacked : 0ull) : 0ull;
   }
+  if (how != kComparesKeys && d.outcome && st->packed_epoch != st->cache_epoch)
+    d.outcome[2] = st->packed_epoch == (st->cache_epoch | kCannotBePacked) ? kNeverPacked : kNotPacked;
   decide_same(st, d.tag, same, d.outcome);
 }
 
