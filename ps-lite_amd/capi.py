@@ -174,6 +174,29 @@ def _buf(x, dtype_np, dtype_name):
     return at, a.size, MEM_HOST
 
 
+def _out(x, dtype_np, dtype_name):
+    """_buf() of an array that the call fills, and what takes the first entries of the answer to it where that is not the memory
+    itself that the library writes: arrays with strides, in another byte order, of another width."""
+    at, n, kind = _buf(x, dtype_np, dtype_name)
+    if x is None or _is_tensor(x):
+        return at, n, kind, lambda count: None
+    if not isinstance(x, np.ndarray):
+        try:
+            x = np.asarray(memoryview(x))
+        except TypeError:
+            raise TypeError("an answer goes to an array, not to a %s" % type(x).__name__) from None
+    if at is None or np.may_share_memory(at.of, x):
+        return at, n, kind, lambda count: None
+    if x.dtype.kind not in ("f" if dtype_np is np.float32 else "iuf"):
+        raise TypeError("an answer of %s does not go to an array of %s" % (np.dtype(dtype_np), x.dtype))
+    if not x.flags.writeable:
+        raise ValueError("the array that the answer goes to is read-only")
+
+    def give(count):
+        x.flat[:count] = at.of.ravel()[:count]
+    return at, n, kind, give
+
+
 def _memkind(*kinds):
     ks = {k for k in kinds if k is not None}
     assert len(ks) <= 1, "all buffers of a call must live in the same kind of memory"
@@ -261,14 +284,16 @@ class Table(_Holder):
         if got is not None:
             return self._sized(got)
         kp, n, k1 = _buf(keys, np.uint64, "int64")
-        op, cap, k2 = _buf(out, np.float32, "float32")
-        lp, _, k3 = _buf(out_lens, np.int32, "int32")
+        op, cap, k2, give = _out(out, np.float32, "float32")
+        lp, _, k3, give_lens = _out(out_lens, np.int32, "int32")
         got = ctypes.c_size_t(0)
         self.last_out_nvals = None
         self._hold(keys, out, out_lens)
         rc = self._lib.pskv_pull(self._h, kp, n, op, cap, lp, ctypes.byref(got), _memkind(k1, k2, k3))
         self.last_out_nvals = got.value
         _check(rc)
+        give(got.value)
+        give_lens(n)
         return got.value
 
     def _sized(self, got):
@@ -284,14 +309,16 @@ class Table(_Holder):
         kp, n, k1 = _buf(keys, np.uint64, "int64")
         vp, nv, k2 = _buf(vals, np.float32, "float32")
         lp, nl, k3 = _buf(lens, np.int32, "int32")
-        op, cap, k4 = _buf(out, np.float32, "float32")
-        olp, _, k5 = _buf(out_lens, np.int32, "int32")
+        op, cap, k4, give = _out(out, np.float32, "float32")
+        olp, _, k5, give_lens = _out(out_lens, np.int32, "int32")
         got = ctypes.c_size_t(0)
         self._hold(keys, vals, lens, out, out_lens)
         rc = self._lib.pskv_pushpull(self._h, kp, n, vp, nv, lp, nl, op, cap, olp, ctypes.byref(got),
                                      _memkind(k1, k2, k3, k4, k5))
         self.last_out_nvals = got.value
         _check(rc)
+        give(got.value)
+        give_lens(n)
         return got.value
 
     def push_raw(self, keys_ptr, n, vals_ptr, nvals, lens_ptr=None, nlens=0):
