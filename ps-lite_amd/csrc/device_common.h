@@ -82,6 +82,17 @@ __device__ __forceinline__ float stored_value(uint64_t payload) { return __uint_
 __device__ __forceinline__ void store_value(uint64_t* payload, float v) {
   *reinterpret_cast<unsigned*>(payload) = ~__float_as_uint(v);
 }
+// The sum of two values, of two NaNs the first. (Which of the operands of a `+` comes first the compiler chooses from kernel to kernel.
+// The kernels that take pushes past k_scalar leave what it leaves: the pushed NaN, and of a run the first.)
+__device__ __forceinline__ float sum_in_order(float first, float second) {
+#ifdef __HIP_DEVICE_COMPILE__
+  float sum;
+  asm("v_add_f32 %0, %1, %2" : "=v"(sum) : "v"(first), "v"(second));
+  return sum;
+#else
+  return first + second;
+#endif
+}
 
 // Counters that every workgroup bumps are spread over kCountShards cache lines:
 // atomics on one address are served one at a time, and a request can run thousands

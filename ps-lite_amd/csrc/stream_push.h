@@ -372,7 +372,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
           }
         }
         if (k == key[q]) {
-          s_val[j] = s_val[j] + v[q];
+          s_val[j] = sum_in_order(v[q], s_val[j]);
           placed = true;
         }
       }
@@ -416,9 +416,9 @@ __global__ __launch_bounds__(kBlock) void k_push_left(StreamBatch b) {
     uint64_t seen;
     uint64_t* p = find_or_insert(d.slots, d.mask, st, l.key, is_new, seen);
     if (!p) continue;
-    float cur = (is_new ? 0.0f : stored_value(seen)) + l.v;
+    float cur = sum_in_order(l.v, is_new ? 0.0f : stored_value(seen));
     if (l.run != kNoRun)
-      for (uint64_t j = (uint64_t)l.run + 1; j < d.n && d.keys[j] == l.key; ++j) cur = cur + d.vals[j];
+      for (uint64_t j = (uint64_t)l.run + 1; j < d.n && d.keys[j] == l.key; ++j) cur = sum_in_order(cur, d.vals[j]);
     store_value(p, cur);
     created += is_new ? 1u : 0u;
   }

@@ -2018,7 +2018,7 @@ __global__ __launch_bounds__(kBlock) void k_regrow_rest(RegrowBatch b) {
           }
         }
         if (k == s.x) {
-          store_value(&slots[h].payload, stored_value(slots[h].payload) + stored_value(s.y));
+          store_value(&slots[h].payload, sum_in_order(stored_value(slots[h].payload), stored_value(s.y)));
           atomicAdd(&st->count_shard[stretch % kCountShards * kShardStride], ~0ull);  // (it has been counted twice)
           placed = true;
           break;

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from conftest import announce
-from helpers import KMAX, to_dev, unique_keys
+from helpers import KMAX, assert_bits_equal, to_dev, unique_keys
 from test_gpu_store import _check_dump
 
 pytestmark = pytest.mark.gpu
@@ -136,3 +136,38 @@ def test_shares_of_a_request(capi, orc, dev, streaming, S):
                 stores[s].push(keys[part], vals[part])
     for s in range(S):
         _check_dump(group.tables[s], stores[s], "table %d" % s)
+
+
+@pytest.mark.parametrize("first,last", [(0.0, 1.0), (0.999, 1.0), (0.49, 0.51)])
+def test_values_that_are_no_numbers(capi, dev, monkeypatch, first, last):
+    """Infinities and NaNs, each with a payload of its own: what a push leaves that streams, with and without a growth, is to the bit
+    what one leaves that goes through the slots. (The sum of two NaNs is one of the two: which one depends on their order.)"""
+    announce("streamed NaNs", first, last)
+    rng = np.random.default_rng(int(first * 1000) + 7)
+    tables = []
+    for streams in ("0", "1"):
+        monkeypatch.setenv("PSKV_STREAM", streams)
+        tables.append(capi.Table(capi.MODE_SCALAR, initial_capacity=32_000, max_load=0.5))
+        tables[-1].prof_enable()
+    lo, hi = int(first * 2**64), min(int(last * 2**64), 2**64 - 1)
+    crowd = np.unique(unmixed(rng.integers(lo, hi, size=12_000, dtype=np.uint64)))
+    crowd = crowd[crowd != KMAX]
+
+    def push(keys, number):
+        bits = np.uint32(0x7FC00000 + number * 0x100000) + np.arange(keys.size, dtype=np.uint32)  # quiet, other ones every time
+        vals = np.where(rng.random(keys.size) < 0.7, bits.view(np.float32),
+                        rng.choice(np.array([np.inf, -np.inf, 1.5, -0.0], np.float32), keys.size))
+        vals[rng.random(keys.size) < 0.2] *= np.float32(-1)
+        for t in tables:
+            t.push(to_dev(keys, dev), to_dev(vals, dev))
+        a, b = (t.dump() for t in tables)
+        assert np.array_equal(a[0], b[0])
+        assert_bits_equal(b[2], a[2], "push %d" % number)
+
+    push(crowd, 0)
+    for number, size in ((1, 12_500), (2, 30_000)):  # (the second makes the tables grow)
+        others = np.setdiff1d(unique_keys(rng, size - 6_000), crowd)
+        runs = np.repeat(rng.choice(others, 50, replace=False), 2)
+        push(np.sort(np.concatenate([rng.choice(crowd, 6_000, replace=False), others, runs, np.full(2, KMAX, np.uint64)])), number)
+    assert streamed(tables[1], capi, 3)
+    assert tables[0].prof_read(capi.KERNEL_REHASH)[0] == 2  # (the growth)
