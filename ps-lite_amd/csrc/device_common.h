@@ -206,7 +206,7 @@ __host__ __device__ constexpr uint64_t record_word(uint64_t counter, uint64_t se
 // What a row-mode kernel needs to know about the request it belongs to.
 struct ReqTag {
   unsigned long long epoch;  // number of the request
-  unsigned int try_cache;    // the host found the key cache structurally usable for this request
+  unsigned int try_cache;    // not 0: the host found the key cache structurally usable for this request (kTry*)
   // The request is a replay of a recorded one (a node of a HIP graph, launched again and again with
   // the same arguments, this number included): it is only ever served from the cache. When the
   // comparison finds other keys than the cached ones, none of its kernels changes or answers
@@ -214,6 +214,10 @@ struct ReqTag {
   // for keys that it has not seen.
   unsigned int replay;
 };
+
+constexpr unsigned kTryKeys = 1u;     // compared key by key
+constexpr unsigned kTryPacked = 2u;   // SCALAR: the cached keys have been asked to be packed (PackedKeys)
+constexpr unsigned kTryAndPack = 3u;  // SCALAR: and this is who asks
 
 // True when request `tag` carries exactly the keys (and lens) of the cached request, so that
 // the row references, offsets and tile table still in the workspace are this request's too.

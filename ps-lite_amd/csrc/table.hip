@@ -1074,7 +1074,7 @@ ReqTag next_tag(pskv_table* t, const Request& r, bool back_off = false) {
       t->sc_kind[tag.epoch % pskv_table::kScKinds] = (unsigned char)kind;
     }
   }
-  tag.try_cache = compare ? 1u : 0u;
+  tag.try_cache = compare ? kTryKeys : 0u;
   return tag;
 }
 
@@ -1371,11 +1371,13 @@ int run_scalar(Batch& bt, bool push, bool pull) {
         volatile unsigned long long* const told = t->outcome + 2;
         if (*told == kNotPacked) t->packing = false;
         if (t->packing) {
-          packed = packed || *told != kNeverPacked;
+          if (*told != kNeverPacked) it.tag.try_cache = kTryPacked, packed = true;
         } else if (t->sc_track[r.push ? 0 : 1].hit) {
+          it.tag.try_cache = kTryAndPack;
           t->packing = packs = true;
           *told = 0ull;
         }
+        d.tag = it.tag;
       }
       // (a recorded repeat is served from the cache or not at all: nothing to write back)
       if (!per_key && it.tag.try_cache && t->sc_dirty && r.replay != kReplayCapture) {
@@ -1420,7 +1422,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
   }
   const bool one_launch = repeat_quads != 0;
   if (any_cache && !one_launch) {
-    // (one kernel for all tables: the packed ones', where one of them has been told to be packed, compares the others' keys too)
+    // (one kernel for all tables: the packed ones' compares the others' keys as they are, ReqTag::try_cache)
     const uint64_t per = packs || packed ? (uint64_t)kBlock * PackedKeys::kItems : (uint64_t)kBlock * kSameKeysItems;
     const KernelSet kernels = packs    ? PSKV_KSET_OF(k_same_packed, true)
                               : packed ? PSKV_KSET_OF(k_same_packed, false) : PSKV_KSET(k_same_keys);

@@ -476,8 +476,11 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
 // its first key whole and the other 511 by what they add, which says that they are equal, or not, as surely; where they are
 // not it reads the cached keys themselves. They lie as the lanes read them: per wavefront and lane the lower 32 bits of its
 // eight keys, then the upper 16. PACK: a comparison with the cached keys themselves, which leaves them packed if they are the
-// request's; not where two neighbours are 2^48 or more apart, nor for keys that are not sorted. A request whose keys are others
-// than the packed ones pays for it (30 B per key), once or twice: comparisons that fail are left out.
+// request's; not where two neighbours are 2^48 or more apart (one such gap is enough), nor for keys that are not sorted. A request
+// whose keys are others than the packed ones pays for it (30 B per key), once or twice: comparisons that fail are left out.
+// A table of the same launch whose keys are not packed is compared as by k_same_keys, 16 B per key. (With its words read for nothing and
+// its keys twice, 30 B, two tables of 8M keys of which one cannot be packed took 53 us to compare and 163 to push and pull. They take 36
+// and 127; as long as nothing was packed they took 38 and 131.)
 // Bound by memory: 14 B per key instead of 16. Push and pull of 16M repeated keys took 130 us and take 122.6 (three tables on three
 // streams in turn: 145.8 and 137), of 8M 73.1 and 69.1, of 2M 26 and 24.5, of 1M 18.6 and 18.4. The packed words are left in the
 // memory-side cache: loads that pass it by take 16M keys of three tables down to 121 us, but those of one alone up to 134-139.
@@ -504,7 +507,6 @@ __global__ __launch_bounds__(kBlock) void k_same_packed(HeadBatch<TABLES> b) {
   const unsigned lane = threadIdx.x & 63;
   const uint64_t base = wave * PackedKeys::kBlockKeys + lane * 2;
   const bool there = wave * PackedKeys::kBlockKeys < n, first = lane == 0;
-  const bool packed = !PACK && st->packed_epoch == st->cache_epoch && st->cache_epoch != 0ull;
   u32x4* const block = PackedKeys::block(cache_keys, n, wave);
   const bool vec = (reinterpret_cast<uintptr_t>(keys) & 15) == 0;
   auto key_pair = [&](int q) {
@@ -528,16 +530,35 @@ __global__ __launch_bounds__(kBlock) void k_same_packed(HeadBatch<TABLES> b) {
     return y;
   };
   u64x2 a[kPairs];
-  u32x4 word[3] = {(u32x4)(0u), (u32x4)(0u), (u32x4)(0u)};
-  uint64_t whole = 0;
 #pragma unroll
   for (int q = 0; q < kPairs; ++q) a[q] = key_pair(q);
+  // (one of the tables of the launch has been asked for this; whether its keys are there packed the device knows)
+  const bool asked = d.tag.try_cache == (PACK ? kTryAndPack : kTryPacked);
+  const bool packed = asked && (PACK || (st->packed_epoch == st->cache_epoch && st->cache_epoch != 0ull));
+  const bool ahead = d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch;  // (as in k_same_keys)
+  bool differ = false, wide = false;
+  if (!packed) {
+    u64x2 c[kPairs];
+#pragma unroll
+    for (int q = 0; q < kPairs; ++q) c[q] = cached_pair(q);
+#pragma unroll
+    for (int q = 0; q < kPairs; ++q) differ |= a[q].x != c[q].x || a[q].y != c[q].y;
+    if (__builtin_expect(differ && ahead, 0)) {
+#pragma unroll
+      for (int q = 0; q < kPairs; ++q) {
+        if (a[q].x != c[q].x) write_back(d, base + q * 128);
+        if (a[q].y != c[q].y) write_back(d, base + q * 128 + 1);
+      }
+    }
+    return same_keys_verdict(d, differ, asked ? kComparesPacked : kComparesKeys);
+  }
+  u32x4 word[3] = {(u32x4)(0u), (u32x4)(0u), (u32x4)(0u)};
+  uint64_t whole = 0;
   if (!PACK && there) {
 #pragma unroll
     for (int w = 0; w < 3; ++w) word[w] = block[w * 64 + lane];
     if (first) whole = cache_keys[base];
   }
-  bool differ = !PACK && !packed && there, wide = false;
 #pragma unroll
   for (int q = 0; q < kPairs; ++q) {
     const uint64_t i = base + q * 128;
@@ -563,7 +584,6 @@ __global__ __launch_bounds__(kBlock) void k_same_packed(HeadBatch<TABLES> b) {
   }
   if (PACK || __any(differ)) {  // the keys themselves
     differ = false;
-    const bool ahead = d.cache_mode == kCacheOnBehind && st->dirty_epoch > st->clean_epoch;  // (as in k_same_keys)
 #pragma unroll 1  // (rare: it may not take registers from the others)
     for (int q = 0; q < kPairs; ++q) {
       const u64x2 x = key_pair(q), y = cached_pair(q);
