@@ -1084,7 +1084,8 @@ ReqTag next_tag(pskv_table* t, const Request& r, bool back_off = false) {
 constexpr uint64_t kScalarCacheMinKeys = 1u << 17;
 
 // Cached keys of at least this many are packed once a request has repeated them (8 MB of them: the time of smaller ones is the
-// launches'). Figures: PackedKeys.
+// launches'). Figures: PackedKeys. Room for it, 6 B per key, is taken when such a request is recorded in the key cache; keys that a
+// recorded step left there (pskv_replay_*, which never packs) have none.
 constexpr uint64_t kPackKeys = 1u << 20;
 
 // How a SCALAR request of one table relates to the table's key cache.
@@ -1341,7 +1342,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       // the buffers have the cached request's size). Only a request that is going to be recorded
       // pays for it: a one-off pull of 16M keys would otherwise allocate 256 MB it never uses, and
       // wait for the stream to do so.
-      rc = grow(t, &t->cache_keys, PackedKeys::bytes(r.n));
+      rc = grow(t, &t->cache_keys, !r.replay && r.n >= kPackKeys ? PackedKeys::bytes(r.n) : r.n * sizeof(uint64_t));
       if (rc) return rc;
       t->packing = false;
       rc = grow(t, &t->sc_vals, r.n * sizeof(float));
@@ -1366,7 +1367,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       const bool per_key = plan[i].use == kScTry && !push && !t->sc_dirty && plan[i].kind_before == 0 && r.replay != kReplayCapture;
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
-      if (!per_key && it.tag.try_cache && !r.replay && r.n >= kPackKeys) {
+      if (!per_key && it.tag.try_cache && !r.replay && r.n >= kPackKeys && t->cache_keys.bytes >= PackedKeys::bytes(r.n)) {
         // (packed they are as soon as they have been asked for, further up the stream; the device looks, and says where it was not so)
         volatile unsigned long long* const told = t->outcome + 2;
         if (*told == kNotPacked) t->packing = false;

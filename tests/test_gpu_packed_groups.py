@@ -88,3 +88,39 @@ def test_a_packed_neighbour_costs_nothing(capi, dev):
     some = [keys_of(rng, n, wide=True) for _ in range(8)]
     alone, beside = fastest(some), fastest([packable] + some)
     assert beside < alone * (n * 8 * 16 + packable.size * 14) / (n * 8 * 16) * 1.25, (alone, beside)
+
+
+def test_keys_that_a_recorded_step_left(capi, orc, dev):
+    """Steps that are recorded leave no room behind the cached keys for packed ones: requests that name them the ordinary way are compared
+    with the keys themselves, until an ordinary request has left keys there."""
+    import torch
+    announce("packed behind a recording")
+    rng = np.random.default_rng(21)
+    n = (1 << 20) + 300
+    group, store = capi.Group(1, capi.MODE_SCALAR, initial_capacity=2 * n), orc.Store(orc.MODE_SCALAR)
+    keys, others = keys_of(rng, n), keys_of(rng, n)
+    pos = np.array([0, n], np.uint64)
+    dk, do, out = to_dev(keys, dev), to_dev(others, dev), torch.empty(n, dtype=torch.float32, device=dev)
+    vals = torch.zeros(n, dtype=torch.float32, device=dev)
+
+    def push(of, host, how):
+        new = rng.standard_normal(n).astype(np.float32)
+        vals.copy_(torch.from_numpy(new))
+        how(of)
+        store.push(host, new)
+        group.sync()
+
+    def ordinary(of):
+        group.push(of, pos, vals, pos)
+        group.pull(of, pos, out)
+
+    recordings = []
+    push(dk, keys, lambda of: recordings.append(group.record(capi.REPLAY_PUSH | capi.REPLAY_PULL, of, pos, vals, pos, out=out)))
+    push(dk, keys, lambda of: recordings[0].run())
+    for of, host in ((dk, keys), (do, others), (dk, keys)):
+        for _ in range(5):
+            push(of, host, ordinary)
+            assert_bits_equal(out.cpu().numpy(), store.pull(host)[0])
+    _check_dump(group.tables[0], store, "behind a recording")
+    recordings[0].close()
+    group.close()
