@@ -244,22 +244,16 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
   const unsigned tiles = d.tiles;
   unsigned total = 0;  // keys of the bin
   {
-    constexpr unsigned kTiles = kMostTiles / kStreamBlock;
-    unsigned first[kTiles], many[kTiles], mine = 0;
-#pragma unroll
-    for (unsigned q = 0; q < kTiles; ++q) {
-      const unsigned t = threadIdx.x * kTiles + q;
-      first[q] = many[q] = 0;
-      if (t < tiles) {
-        const uint16_t* row = d.starts + (uint64_t)t * (d.bins + kStartsPad) + bin;
-        first[q] = row[0];
-        many[q] = row[1] - first[q];
-      }
+    static_assert(kMostTiles == kStreamBlock, "a lane looks at a tile");
+    const unsigned t = threadIdx.x;
+    unsigned first = 0, many = 0;
+    if (t < tiles) {
+      const uint16_t* row = d.starts + (uint64_t)t * (d.bins + kStartsPad) + bin;
+      first = row[0];
+      many = row[1] - first;
     }
     ask(0);
-#pragma unroll
-    for (unsigned q = 0; q < kTiles; ++q) mine += many[q];
-    unsigned inc = mine;
+    unsigned inc = many;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const unsigned y = __shfl_up(inc, o);
@@ -267,19 +261,14 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
     }
     if (lane == 63) red[wave] = inc;
     __syncthreads();
-    unsigned run = inc - mine;
+    unsigned before = inc - many;
     for (unsigned x = 0; x < kStreamBlock / 64; ++x) {
-      if (x < wave) run += red[x];
+      if (x < wave) before += red[x];
       total += red[x];
     }
-#pragma unroll
-    for (unsigned q = 0; q < kTiles; ++q) {
-      const unsigned t = threadIdx.x * kTiles + q;
-      if (t < tiles) {
-        s_before[t] = run;
-        s_from[t] = (uint16_t)first[q];
-        run += many[q];
-      }
+    if (t < tiles) {
+      s_before[t] = before;
+      s_from[t] = (uint16_t)first;
     }
     __syncthreads();
   }

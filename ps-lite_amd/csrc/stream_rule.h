@@ -7,13 +7,14 @@ namespace pskv {
 
 constexpr unsigned kSplitTile = 8192;   // keys of a tile
 constexpr unsigned kTileWords = kSplitTile + kSplitTile / 2;  // 8-byte words it leaves: keys, and values behind them
-constexpr unsigned kMostTiles = 2048;
 constexpr unsigned kMostBins = 4096;
 constexpr unsigned kStartsPad = 2;      // 16-bit words behind a tile's row of starts: the number of its keys
 constexpr unsigned kImageSlots = 4096;
 constexpr unsigned kMostImages = 16;    // per bin: every image looks at all keys of the bin
 constexpr unsigned kBinKeys = 2048;     // that a workgroup holds
 constexpr unsigned kBinMean = kBinKeys - 64;  // keys of a bin on average, at most (a few bins then have some more than are held)
+constexpr unsigned kMostTiles = 1024;
+static_assert((uint64_t)kMostBins * kBinMean <= (uint64_t)kMostTiles * kSplitTile, "the keys of the most bins lie in the most tiles");
 
 struct StreamShape {
   uint32_t bins = 0;  // 0: the request does not fit
@@ -28,7 +29,7 @@ inline StreamShape stream_shape(uint64_t n, uint64_t cap) {
   uint64_t bins = cap / kImageSlots / 2;
   if (bins > kMostBins) bins = kMostBins;
   if (bins * kBinMean < n) bins *= 2;
-  if (bins < 2 || bins > kMostBins || bins * kBinMean < n || n > (uint64_t)kMostTiles * kSplitTile) return s;
+  if (bins < 2 || bins > kMostBins || bins * kBinMean < n) return s;
   const uint64_t images = cap / kImageSlots / bins;
   if (images > kMostImages) return s;
   s.bins = (uint32_t)bins;
