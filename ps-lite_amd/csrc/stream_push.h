@@ -68,7 +68,7 @@ __device__ __forceinline__ unsigned left_room(DevState* st, unsigned turn) {
   return __shfl(at, lead) + (unsigned)__popcll(lanes & ((1ull << lane) - 1ull));
 }
 
-// One workgroup per tile. Bound by memory (20 bytes read and written per key; 4M keys 17 us, 5.6 TB/s). A bin's place of a
+// One workgroup per tile. Bound by memory (12 bytes read and 12 written per key; 4M keys 24.4 us, 3.9 TB/s). A bin's place of a
 // key is its rank among the tile's keys of that bin (an LDS atomic per key, two 16-bit counters a word, which leaves LDS for
 // two workgroups per compute unit), keys and values travel through the same LDS one after the other, so that all
 // that is written is written in whole lines. With one atomic per key and tile to counters in memory in place of rows
