@@ -26,13 +26,10 @@ constexpr unsigned kSplitItems = kSplitTile / kSplitBlock;
 constexpr unsigned kStreamBlock = 1024;
 constexpr unsigned kStreamItems = kBinKeys / kStreamBlock;  // keys of its bin that a lane holds
 
-// A key that k_push_left looks up the general way.
-struct alignas(16) LeftKey {
-  unsigned long long key;
-  float v;
-  unsigned run;  // the key repeats: where in the request it first stands; else kNoRun
-};
-constexpr unsigned kNoRun = ~0u;
+// A key that k_push_left looks up the general way, by where it lies: its place among the tiles' keys, or, with kOfRequest, its index in
+// the request (where a run of it may follow).
+constexpr unsigned kOfRequest = 1u << 31;
+static_assert(kMostTiles * kSplitTile < kOfRequest, "places and indexes fit");
 
 struct StreamOf {
   Slot* slots;
@@ -45,7 +42,7 @@ struct StreamOf {
   uint64_t n;
   unsigned long long* parts;  // per tile: room for its keys, behind them for its values
   uint16_t* starts;           // per tile: where each bin's keys start in it, and its number of keys; a row is bins + kStartsPad
-  LeftKey* left;              // room for n
+  unsigned* left;             // room for n
   Snapshot* snap;             // counters after the request, or null
   uint64_t snap_seq;
   unsigned long long* told;   // pinned: whether the request named the keys of the one before it (by the sum of their hashes)
@@ -58,6 +55,14 @@ struct StreamBatch {
   StreamOf t[kMaxBatch];
 };
 static_assert(sizeof(StreamBatch) <= 3840, "kernel arguments are limited to 4 KiB");
+
+// The tiles' key and value at a place.
+__device__ __forceinline__ const unsigned long long* key_at(const StreamOf& d, unsigned at) {
+  return d.parts + (uint64_t)(at / kSplitTile) * kTileWords + at % kSplitTile;
+}
+__device__ __forceinline__ const float* value_at(const StreamOf& d, unsigned at) {
+  return reinterpret_cast<const float*>(d.parts + (uint64_t)(at / kSplitTile) * kTileWords + kSplitTile) + at % kSplitTile;
+}
 
 // Room for the left keys of the lanes that call it together.
 __device__ __forceinline__ unsigned left_room(DevState* st, unsigned turn) {
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split(StreamBatch b) {
     const uint64_t hash = mix64(key[q]);
     sum += hash;
     if (run || key[q] == kEmptyKey) {
-      place[q] = kInLeft | (run ? 1u << 30 : 0u) | atomicAdd(&s_left, 1u);
+      place[q] = kInLeft | atomicAdd(&s_left, 1u);
       continue;
     }
     const unsigned bin = (unsigned)(hash >> (64 - d.bin_bits)), half = (bin & 1) * 16;
@@ -175,8 +180,7 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split(StreamBatch b) {
   for (unsigned q = 0; q < kSplitItems; ++q) {
     if (place[q] == kNowhere) continue;
     if (place[q] & kInLeft) {
-      const unsigned i = (unsigned)(mine0 + q * 64);
-      d.left[s_left_at + (place[q] & 0xffffu)] = LeftKey{key[q], v[q], place[q] >> 30 & 1u ? i : kNoRun};
+      d.left[s_left_at + (place[q] & 0xffffu)] = kOfRequest | (unsigned)(mine0 + q * 64);
       place[q] = kNowhere;
       continue;
     }
@@ -204,7 +208,7 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split(StreamBatch b) {
   }
 }
 
-// One workgroup per bin: images of kImageSlots slots (keys and values, 48 KiB of LDS, so two workgroups of 1,024 lanes per
+// One workgroup per bin: images of kImageSlots slots (keys and values, 48 KiB of LDS, 54 in all, so two workgroups of 1,024 lanes per
 // compute unit: one streams while the other looks for its keys), the next one asked for while the keys of this one are
 // placed. Bound by memory: 4.7 to 5.2 TB/s of slots. 4M keys into 16M slots 105 us; workgroups of 512 lanes with images of
 // 2,048 slots 131, with 4,096 113, one image per bin instead of two 113 (as many lines read for half the keys). Keys whose
@@ -221,10 +225,9 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
   __shared__ float s_val[kImageSlots];
   __shared__ unsigned red[kStreamBlock / 64];
   __shared__ unsigned s_rest;
-  // (before there is an image: where each tile's keys of this bin lie)
-  static_assert(kMostTiles * (sizeof(unsigned) + sizeof(uint16_t)) <= sizeof(s_val), "the runs fit where the values go");
-  unsigned* s_before = reinterpret_cast<unsigned*>(s_val);
-  uint16_t* s_from = reinterpret_cast<uint16_t*>(s_before + kMostTiles);
+  // where each tile's keys of this bin lie
+  __shared__ unsigned s_before[kMostTiles];
+  __shared__ uint16_t s_from[kMostTiles];
   // (workgroups are dealt out to the eight XCDs in turn: bins next to each other, whose keys share lines, to one of them)
   const unsigned bin = d.bins % 8 == 0 ? blockIdx.x % 8 * (d.bins / 8) + blockIdx.x / 8 : blockIdx.x;
   const uint64_t mask = d.mask, base = (uint64_t)bin * d.images * kImageSlots;
@@ -272,8 +275,8 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
     }
     __syncthreads();
   }
-  // key j of the bin: its tile's words, and where it is among them
-  auto find = [&](unsigned j, unsigned& at) {
+  // key j of the bin: its place among the tiles' keys
+  auto find = [&](unsigned j) {
     unsigned t = 0;
     for (unsigned many = tiles; many > 1;) {
       const unsigned half = many >> 1;
@@ -281,8 +284,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
       t = up ? t + half : t;
       many = up ? many - half : half;
     }
-    at = s_from[t] + (j - s_before[t]);
-    return d.parts + (uint64_t)t * kTileWords;
+    return t * kSplitTile + s_from[t] + (j - s_before[t]);
   };
   unsigned long long key[kStreamItems];
   float v[kStreamItems];
@@ -291,18 +293,12 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
     const unsigned j = q * kStreamBlock + threadIdx.x;
     key[q] = 0, v[q] = 0.0f;
     if (j < total) {
-      unsigned at;
-      const unsigned long long* words = find(j, at);
-      key[q] = words[at];
-      v[q] = reinterpret_cast<const float*>(words + kSplitTile)[at];
+      const unsigned at = find(j);
+      key[q] = *key_at(d, at);
+      v[q] = *value_at(d, at);
     }
   }
-  for (unsigned j = kBinKeys + threadIdx.x; j < total; j += kStreamBlock) {
-    unsigned at;
-    const unsigned long long* words = find(j, at);
-    d.left[left_room(d.st, d.turn)] = LeftKey{words[at], reinterpret_cast<const float*>(words + kSplitTile)[at], kNoRun};
-  }
-  __syncthreads();
+  for (unsigned j = kBinKeys + threadIdx.x; j < total; j += kStreamBlock) d.left[left_room(d.st, d.turn)] = find(j);
   if (GROW) {
     for (unsigned j = threadIdx.x; j < kImageSlots; j += kStreamBlock) s_key[j] = kEmptyKey, s_val[j] = 0.0f;
   }
@@ -365,7 +361,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
           placed = true;
         }
       }
-      if (!placed) d.left[left_room(d.st, d.turn)] = LeftKey{key[q], v[q], kNoRun};
+      if (!placed) d.left[left_room(d.st, d.turn)] = find(q * kStreamBlock + threadIdx.x);
     }
     __syncthreads();
     u64x2* __restrict__ out = reinterpret_cast<u64x2*>(d.slots + base + (uint64_t)image * kImageSlots);
@@ -400,14 +396,17 @@ __global__ __launch_bounds__(kBlock) void k_push_left(StreamBatch b) {
   __shared__ unsigned red[kBlock / 64];
   unsigned created = 0;
   for (unsigned x = blockIdx.x * kBlock + threadIdx.x; x < left; x += gridDim.x * kBlock) {
-    const LeftKey l = d.left[x];
+    const unsigned at = d.left[x], i = at & ~kOfRequest;
+    const bool of_request = (at & kOfRequest) != 0;
+    const unsigned long long key = of_request ? d.keys[i] : *key_at(d, i);
+    const float v = of_request ? d.vals[i] : *value_at(d, i);
     bool is_new;
     uint64_t seen;
-    uint64_t* p = find_or_insert(d.slots, d.mask, st, l.key, is_new, seen);
+    uint64_t* p = find_or_insert(d.slots, d.mask, st, key, is_new, seen);
     if (!p) continue;
-    float cur = sum_in_order(l.v, is_new ? 0.0f : stored_value(seen));
-    if (l.run != kNoRun)
-      for (uint64_t j = (uint64_t)l.run + 1; j < d.n && d.keys[j] == l.key; ++j) cur = sum_in_order(cur, d.vals[j]);
+    float cur = sum_in_order(v, is_new ? 0.0f : stored_value(seen));
+    if (of_request)
+      for (uint64_t j = (uint64_t)i + 1; j < d.n && d.keys[j] == key; ++j) cur = sum_in_order(cur, d.vals[j]);
     store_value(p, cur);
     created += is_new ? 1u : 0u;
   }

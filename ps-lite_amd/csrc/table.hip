@@ -572,6 +572,14 @@ int grow(pskv_table* t, GrowBuf* b, size_t bytes) {
   return PSKV_OK;
 }
 
+// Gives back what grow() took.
+int drop(pskv_table* t, GrowBuf* b) {
+  void* const gone = b->ptr;
+  b->ptr = nullptr;
+  b->bytes = 0;
+  return array_release(gone, t->stream);
+}
+
 // Moves the base of the bounds forward to the newest record the device has published: the
 // counters after request `s1`.
 void adopt_snapshot(pskv_table* t) {
@@ -1154,7 +1162,7 @@ struct Streamed {
 
 size_t stream_room(const Streamed& s) {
   return Carver::need((size_t)s.tiles() * kTileWords, 8) +
-         Carver::need((size_t)s.tiles() * (s.shape.bins + kStartsPad), 2) + Carver::need(s.it->r.n, sizeof(LeftKey));
+         Carver::need((size_t)s.tiles() * (s.shape.bins + kStartsPad), 2) + Carver::need(s.it->r.n, sizeof(unsigned));
 }
 
 // Those tables' shares of a push; the slot arrays that move for it have been allocated, nothing has been moved.
@@ -1191,7 +1199,7 @@ int stream_push(Batch& bt, std::vector<Streamed>& todo) {
     Carver c(t->ws.ptr);
     d.parts = c.take<unsigned long long>((size_t)d.tiles * kTileWords);
     d.starts = c.take<uint16_t>((size_t)d.tiles * (d.bins + kStartsPad));
-    d.left = c.take<LeftKey>(it.r.n);
+    d.left = c.take<unsigned>(it.r.n);
     d.snap = it.pub.snap;
     d.snap_seq = it.pub.seq;
     d.told = t->outcome + 1;
@@ -1328,6 +1336,9 @@ int run_scalar(Batch& bt, bool push, bool pull) {
     if (r.n == 0) continue;
     int rc = PSKV_OK;
     if (plan[i].streams) plan[i].use = kScPlain;
+    // (17 B per key that a push that streamed has needed, and that nothing else of a SCALAR table does: a table that has been filled
+    // may be pulled from for long)
+    if (!plan[i].streams && t->ws.ptr && !t->capturing && (rc = drop(t, &t->ws))) return rc;
     if (plan[i].use != kScTry) {
       // the request goes through the slots, so they must be up to date; a push then makes the
       // cached values stale, a recording replaces them
