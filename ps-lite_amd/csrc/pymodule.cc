@@ -47,7 +47,6 @@ class Arg {
     if (!f || f[0] == 0 || f[1] != 0) return 0;
     const bool fits = type == 'k'   ? (f[0] == 'L' || f[0] == 'Q') && view_.itemsize == 8
                       : type == 'f' ? f[0] == 'f' && view_.itemsize == 4
-                      : type == 'b' ? f[0] == 'B' && view_.itemsize == 1
                                     : f[0] == 'i' && view_.itemsize == 4;
     if (!fits) return 0;
     n = (size_t)(view_.len / view_.itemsize);
@@ -65,7 +64,6 @@ class Arg {
     const int t = PyArray_TYPE(a);
     const bool fits = type == 'k'   ? t == NPY_ULONG || t == NPY_ULONGLONG
                       : type == 'f' ? t == NPY_FLOAT
-                      : type == 'b' ? t == NPY_UBYTE
                                     : t == NPY_INT;
     if (!fits || !PyArray_IS_C_CONTIGUOUS(a) || !PyArray_ISALIGNED(a) || !PyArray_ISNOTSWAPPED(a)) return 0;
     n = (size_t)PyArray_SIZE(a);
@@ -78,7 +76,7 @@ class Arg {
     if (!d) return -1;
     Py_DECREF(d);  // (dtypes live as long as torch does)
     const bool fits = type == 'k' ? d == g_int64 || d == g_uint64 : type == 'f' ? d == g_float32 : d == g_int32;
-    if (!fits || type == 'b') return 0;
+    if (!fits) return 0;
     PyObject* c = PyObject_CallMethodNoArgs(o, s_is_contiguous);
     if (!c) return -1;
     Py_DECREF(c);
