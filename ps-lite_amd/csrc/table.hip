@@ -401,7 +401,8 @@ struct pskv_table {
   unsigned long long sc_seen = 0;         // the value of *outcome the host last looked at
   unsigned push_looks = 0;                // k_fixed_own: how often a workgroup looks for the verdict
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
-  int streams = -1;                       // pushes stream through the slot array: where it pays, or (0, 1) never, wherever they can
+  // which pushes stream through the slot array (stream_push.h); PSKV_STREAM=0 and =1, read when a table is created, are for tests
+  enum class Streams { kNever, kWhereItPays, kWhereItFits } streams = Streams::kWhereItPays;
   bool packing = false;                   // a comparison has been asked to pack the cached keys (PackedKeys)
   unsigned stream_turn = 0;               // the counter of left keys that the newest of them used
 
@@ -1256,14 +1257,15 @@ std::vector<Streamed> pick_streamed(Batch& bt, const std::vector<ScalarPlan>& pl
   for (size_t i = 0; i < bt.size(); ++i) {
     pskv_table* t = bt[i].t;
     const uint64_t n = bt[i].r.n;
-    if (!plan[i].may_stream || !n || !t->streams) continue;
+    if (!plan[i].may_stream || !n || t->streams == pskv_table::Streams::kNever) continue;
     Streamed s{&bt[i], {}, false, {}};
     for (const Growth<pskv_table, Slot>& g : growths->list)
       if (g.t == t && t->cap / g.cap <= (uint64_t)kRegrowMaxFactor) s.g = g, s.grows = true;
     s.shape = stream_shape(n, t->cap);
     if (!s.shape.bins) continue;
-    const double its =
-        t->streams > 0 ? kStreamLaunches : stream_gain(n, t->cap, t->share_known ? t->new_share : kFreshGuess, s.grows);
+    const double its = t->streams == pskv_table::Streams::kWhereItFits
+                           ? kStreamLaunches
+                           : stream_gain(n, t->cap, t->share_known ? t->new_share : kFreshGuess, s.grows);
     if (its <= 0.0) continue;
     gain += its;
     some.push_back(s);
@@ -2491,7 +2493,8 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
   // (the environment variable is for tests of workgroups that do not see the verdict)
   t->push_looks = kOwnLooks;
   if (const char* e = std::getenv("PSKV_PUSH_LOOKS")) t->push_looks = (unsigned)std::strtoul(e, nullptr, 10);
-  if (const char* e = std::getenv("PSKV_STREAM")) t->streams = std::atoi(e) != 0;  // (for tests)
+  if (const char* e = std::getenv("PSKV_STREAM"))
+    t->streams = std::atoi(e) ? pskv_table::Streams::kWhereItFits : pskv_table::Streams::kNever;
   t->sc_min_keys = kScalarCacheMinKeys;
   if (const char* e = std::getenv("PSKV_SCALAR_CACHE_MIN_KEYS")) t->sc_min_keys = std::strtoull(e, nullptr, 10);
   auto fail = [&](int rc) {
