@@ -117,10 +117,12 @@ def test_the_same_keys_again_and_again(capi, orc, dev, streaming):
 
 @pytest.mark.parametrize("S", [2, 5])
 def test_shares_of_a_request(capi, orc, dev, streaming, S):
-    """Tables of a group, some of which stream, some of which grow, some of which do neither."""
+    """Tables of a group, all of which stream, some of which grow."""
     announce("streamed shares", S)
     rng = np.random.default_rng(S)
     group, stores = capi.Group(S, capi.MODE_SCALAR, initial_capacity=20_000), [orc.Store(orc.MODE_SCALAR) for _ in range(S)]
+    for t in group.tables:
+        t.prof_enable()
     begin, end = capi.server_ranges(S)
     for rep in range(5):
         keys = unique_keys(rng, 40_000 + 9_000 * rep, S)
@@ -136,6 +138,72 @@ def test_shares_of_a_request(capi, orc, dev, streaming, S):
                 stores[s].push(keys[part], vals[part])
     for s in range(S):
         _check_dump(group.tables[s], stores[s], "table %d" % s)
+    assert launches(group, capi.KERNEL_REHASH) >= 3 * 5 and launches(group, capi.KERNEL_PUSH_SCALAR) == 0
+
+
+def launches(group, kernel):
+    """By all tables of the group."""
+    return sum(t.prof_read(kernel)[0] for t in group.tables)
+
+
+def test_shares_that_stream_by_themselves(capi, orc, dev):
+    """A request of which the rule lets one share stream, with the growth that it asks for, and the others not: both ways in one request."""
+    announce("streamed shares by the rule")
+    rng = np.random.default_rng(77)
+    group, stores = capi.Group(3, capi.MODE_SCALAR, initial_capacity=1_000_000), [orc.Store(orc.MODE_SCALAR) for _ in range(3)]
+    for t in group.tables:
+        t.prof_enable()
+    sizes = (10_000, 2_000_000, 0)
+    parts = [unique_keys(rng, n) if n else np.zeros(0, np.uint64) for n in sizes]
+    pos = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint64)
+    vals = rng.standard_normal(int(pos[-1])).astype(np.float32)
+    group.push(to_dev(np.concatenate(parts), dev), pos, to_dev(vals, dev), pos)
+    # k_split, k_stream_push, k_regrow_rest and k_push_left; one k_scalar
+    assert launches(group, capi.KERNEL_REHASH) == 4 and launches(group, capi.KERNEL_PUSH_SCALAR) == 1
+    for s, keys in enumerate(parts):
+        if keys.size:
+            stores[s].push(keys, vals[int(pos[s]):int(pos[s + 1])])
+        _check_dump(group.tables[s], stores[s], "table %d" % s)
+
+
+@pytest.mark.parametrize("grows", [False, True])
+def test_cached_values_that_are_ahead_of_the_slots(capi, orc, dev, streaming, monkeypatch, grows):
+    """A push that streams reads the slots, which may lack what pushes of repeated keys have added to the key cache alone. Their values
+    go back first; the room that the push needs, which takes the key cache's buffers out of use, comes before that."""
+    announce("streamed behind repeats", grows)
+    monkeypatch.setenv("PSKV_SCALAR_CACHE_MIN_KEYS", "1000")
+    rng = np.random.default_rng(8)
+    n = 20_000
+    t, o = capi.Table(capi.MODE_SCALAR, initial_capacity=n if grows else 4 * n), orc.Store(orc.MODE_SCALAR)
+    t.prof_enable()
+    keys = np.concatenate([unique_keys(rng, n - 1), [np.uint64(KMAX)]])
+    for rep in range(3):
+        compared = t.prof_read(capi.KERNEL_SAME_KEYS)[0]
+        for _ in range(8):
+            push_both(t, o, dev, keys, rng.standard_normal(n).astype(np.float32))
+            t.sync()
+        assert t.prof_read(capi.KERNEL_SAME_KEYS)[0] > compared  # (the last ones have been served from the cache)
+        before = t.prof_read(capi.KERNEL_REHASH)[0]
+        others = np.unique(np.concatenate([rng.choice(keys, n // 2, replace=False), unique_keys(rng, n + 5_000 * rep)]))
+        push_both(t, o, dev, others, rng.standard_normal(others.size).astype(np.float32))
+        assert t.prof_read(capi.KERNEL_REHASH)[0] - before in ((3, 4) if grows else (3,))
+        _check_dump(t, o, "ahead %d" % rep)
+
+
+@pytest.mark.parametrize("capacity,images", [(30_000_000, 4), (60_000_000, 8), (120_000_000, 16)])
+def test_bins_of_many_images(capi, orc, dev, streaming, capacity, images):
+    """Arrays of 64M, 128M and 256M slots: the bins are as many as there may be, with four images each and more."""
+    announce("streamed images", images)
+    rng = np.random.default_rng(images)
+    t, o = capi.Table(capi.MODE_SCALAR, initial_capacity=capacity), orc.Store(orc.MODE_SCALAR)
+    t.prof_enable()
+    assert t.counters()["slots"] == 4096 * 4096 * images
+    universe = unique_keys(rng, 60_000)
+    for rep in range(3):
+        keys = np.sort(rng.choice(universe, 30_000 + rep, replace=False))
+        push_both(t, o, dev, keys, rng.standard_normal(keys.size).astype(np.float32))
+    assert t.prof_read(capi.KERNEL_REHASH)[0] == 9
+    _check_dump(t, o, "images")
 
 
 @pytest.mark.parametrize("first,last", [(0.0, 1.0), (0.999, 1.0), (0.49, 0.51)])
