@@ -225,3 +225,34 @@ def test_recorded_rows_of_a_workgroup_or_more(capi, orc, dev, k):
         group.sync()
         o.push(keys, vals)
         assert_bits_equal(out.cpu().numpy(), o.pull(keys)[0])
+
+
+@pytest.mark.parametrize("mode,n", [("ragged", 3_000), ("ragged", 60_000), ("wide", 40)])
+def test_rows_of_values_that_are_no_numbers(capi, orc, dev, mode, n):
+    """Infinities, and NaNs that meet numbers only (their payload stays then, whichever way round they are added), through the row kernels
+    that go by the rows and the wide ones; the ends of ragged rows, whose last quad is written whole, among them."""
+    announce("rows of NaNs", mode, n)
+    import torch
+    rng = np.random.default_rng(n)
+    keys = unique_keys(rng, n)
+    ragged, k = mode == "ragged", 1030
+    lens = rng.integers(1, 90, n).astype(np.int32) if ragged else None
+    total = int(lens.sum()) if ragged else n * k
+    t = capi.Table(capi.MODE_VARLEN) if ragged else capi.Table(capi.MODE_FIXED, row_len=k)
+    o = orc.Store(orc.MODE_VARLEN, 0) if ragged else orc.Store(orc.MODE_FIXED, k)
+    at = np.arange(total)
+    for turn in range(5):
+        vals = rng.standard_normal(total).astype(np.float32)
+        vals[at % 11 == turn] = (np.uint32(0x7FC00000) + (at[at % 11 == turn] & 0xFFFF).astype(np.uint32)).view(np.float32)
+        vals[at % 11 == 5] = np.inf
+        vals[at % 11 == 6] = -np.inf
+        vals[at % 11 == 7 + turn % 2] = -0.0
+        t.push(to_dev(keys, dev), _off_by(vals, dev, turn % 3), None if lens is None else to_dev(lens, dev))
+        o.push(keys, vals, lens)
+        t.sync()
+    out, out_lens = torch.empty(total, device=dev), torch.empty(n, dtype=torch.int32, device=dev)
+    t.pull(to_dev(keys, dev), out, out_lens if ragged else None)
+    t.sync()
+    assert_bits_equal(out.cpu().numpy(), o.pull(keys)[0])
+    for mine, theirs in zip(t.dump(), o.dump()):
+        assert np.array_equal(mine, theirs) if mine.dtype != np.float32 else assert_bits_equal(mine, theirs) is None
