@@ -306,7 +306,7 @@ def run_sparse_lr(args, capi, dev):
               "pull": kernel_stats(tables, capi.KERNEL_PULL_SCALAR),
               "same": kernel_stats(tables, capi.KERNEL_SAME_KEYS),
               "per_key": kernel_stats(tables, capi.KERNEL_PULL_PER_KEY),
-              "growth": kernel_stats(tables, capi.KERNEL_REHASH)}
+              "slot_passes": kernel_stats(tables, capi.KERNEL_REHASH)}
         for t in tables:
             t.prof_enable(False)
         # the last pull must hold exactly the pushed values, the tables every key of the run
@@ -356,8 +356,8 @@ def run_sparse_lr(args, capi, dev):
         "kernels": dict(pull_entries(keys_per_launch, st["pull"], st["same"], st["per_key"],
                                      traffic("pull_scalar", keys_per_launch),
                                      traffic("pull_per_key", keys_per_launch)),
-                        growth={"launches": st["growth"][0], "total_us": round(st["growth"][1] * 1e3, 1),
-                                "note": "growths, and pushes that stream through the slots, of the sampled steps only"}),
+                        slot_passes={"launches": st["slot_passes"][0], "total_us": round(st["slot_passes"][1] * 1e3, 1),
+                                     "note": "growths, and pushes that stream through the slots, of the sampled steps only"}),
     }
     if not args.no_extra:
         # the same steps on tables sized up front for every key of the run (no growth, lower fill)
@@ -868,9 +868,9 @@ def run_zipf(args, capi, dev, pushes=8):
         "kernels": {"push_scalar": dict(roofline(32.0 * n, push[0], push[1], traffic("push_scalar_zipf", n), push[2]),
                                         kernel="k_scalar<push> (find-or-insert + add), 4M keys, the pushes that go through the slots",
                                         bytes_per_key=32),
-                    "growth": {"launches": rehash[0], "total_us": round(rehash[1] * 1e3, 1),
-                               "kernels": "pushes that stream through the slots or make them grow: k_split, k_stream_push, "
-                                          "k_regrow_rest, k_push_left"}},
+                    "slot_passes": {"launches": rehash[0], "total_us": round(rehash[1] * 1e3, 1),
+                                    "kernels": "pushes that stream through the slots or make them grow: k_split, "
+                                               "k_stream_push, k_regrow_rest, k_push_left"}},
     }
     return res, (batches, probe)
 
