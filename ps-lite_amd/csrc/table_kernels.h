@@ -1382,7 +1382,8 @@ __device__ __forceinline__ void rows_quads_fixed(const RowsParams& p, uint64_t q
 // early: all arguments in one fetch, then the request's values, then the two references, through the scalar cache, so that nothing
 // waits for anything but the row for its reference. Above, arguments, facts and reference are four waits one behind the other
 // and the values are waited for with the reference: 64 rows of 4M floats, four pushes and a pull of three tables in turn, 2,460 us
-// against 2,395 here (6.1 and 6.3 TB/s), 300 of 100,010 318 and 308, 3 of 4.9M 178 and 170. Shorter rows, scattered over the
+// against 2,395 here (6.1 and 6.3 TB/s), 300 of 100,010 318 and 308, 3 of 4.9M 178 and 170. Pulls by themselves gain less: 300
+// rows of 100,010 41.2 and 39.0, 3 of 4.9M 20.9 and 20.0, 5,000 of 4,100 28.3 and 27.5, 64 of 4M 334 both. Shorter rows, scattered over the
 // arena, gain nothing from it (64 floats 633 and 634-639, 48 floats 158 and 161: the memory has enough to do).
 constexpr uint64_t kWideRow = 1024;
 typedef const __attribute__((address_space(4))) uint64_t* ScalarWords;  // what no workgroup of this launch writes
