@@ -302,7 +302,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
   if (GROW) {
     for (unsigned j = threadIdx.x; j < kImageSlots; j += kStreamBlock) s_key[j] = kEmptyKey, s_val[j] = 0.0f;
   }
-  unsigned created = 0;
+  unsigned created = 0, left = 0;  // left: a bit for each of the lane's keys that found no place
   for (unsigned image = 0; image < d.images; ++image) {
     if (GROW) {
       const uint64_t old_base = base / factor + (uint64_t)image * olds;
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
           placed = true;
         }
       }
-      if (!placed) d.left[left_room(d.st, d.turn)] = find(q * kStreamBlock + threadIdx.x);
+      if (!placed) left |= 1u << q;
     }
     __syncthreads();
     u64x2* __restrict__ out = reinterpret_cast<u64x2*>(d.slots + base + (uint64_t)image * kImageSlots);
@@ -376,6 +376,8 @@ __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) 
     }
     // (what a lane writes in front of the next barrier, it has read itself)
   }
+  for (unsigned q = 0; q < kStreamItems; ++q)
+    if (left >> q & 1u) d.left[left_room(d.st, d.turn)] = find(q * kStreamBlock + threadIdx.x);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) created += __shfl_xor(created, o);
   if (lane == 0) red[wave] = created;
