@@ -10,9 +10,9 @@
 //   k_regrow_rest  growing: the keys of the old array whose probe chains cross from stretch to stretch
 //   k_push_left    the keys of the request whose probe chains do, and those that the tiles do not carry: runs of one key,
 //                  the key that marks an empty slot
-// 4M keys, 40 % of them held, us (through the slots -> here): into 16M slots 258 -> 132, from 4M to 16M slots 348 -> 101, from 16M
-// to 32M 370 -> 195, from 32M to 64M 493 -> 340. The same bins with plain stores to the slots in place of the pass
-// over the array (no compare-and-swap): 250, not worth it.
+// 4M keys, 40 % of them held, us of all kernels (through the slots -> here): into 16M slots 232 -> 141, from 4M to 16M slots 290 -> 120, from
+// 16M to 32M 351 -> 201, from 32M to 64M 475 -> 334. The same bins with plain stores to the slots in place of the pass
+// over the array (no compare-and-swap): 250 for the first, not worth it.
 #ifndef PSKV_STREAM_PUSH_H_
 #define PSKV_STREAM_PUSH_H_
 #include "device_common.h"
@@ -210,11 +210,13 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split(StreamBatch b) {
 
 // One workgroup per bin: images of kImageSlots slots (keys and values, 48 KiB of LDS, 54 in all, so two workgroups of 1,024 lanes per
 // compute unit: one streams while the other looks for its keys), the next one asked for while the keys of this one are
-// placed. Bound by memory: 4.7 to 5.2 TB/s of slots. 4M keys into 16M slots 105 us; workgroups of 512 lanes with images of
+// placed. Bound by memory: 4.3 (from 4M to 16M) to 5.8 TB/s (32M that stay) of slots. 4M keys into 16M slots 105 us; workgroups of 512 lanes with images of
 // 2,048 slots 131, with 4,096 113, one image per bin instead of two 113 (as many lines read for half the keys). Keys whose
 // probe chains leave their image, and those of a bin that has more than its lanes hold, are left to k_push_left.
 // What a growth leaves in the old array is as with k_regrow: packed over the front of each image's old slots. A
 // key of the request may be among those; it is created in its image then, and k_regrow_rest adds the two up.
+// The runs of the bin's keys have LDS of their own, so that a key that is left can be named by its place (where the values go, they were
+// gone by then): from 16M to 32M slots 179 -> 158 us, from 32M to 64M 310 -> 293, arrays that stay as before.
 // SLOTS: of the array that the keys are in, per lane and image: 4 where it stays, 2 for one that becomes twice as large, 1 beyond.
 template <unsigned SLOTS>
 __global__ __launch_bounds__(kStreamBlock, 8) void k_stream_push(StreamBatch b) {

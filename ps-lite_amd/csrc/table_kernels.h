@@ -1723,8 +1723,8 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
 // a lane a quad of it, two turns asked for together. A wavefront that starts from its tile makes five trips to memory that follow
 // from each other (facts, tile table, offsets and references, rows, values), one that starts from its rows three; its
 // accesses to the arena are whole quads on their own boundaries (the end of a row's last one is nobody's), where a tile's
-// straddle them. Bound by the lines of the rows, which lie scattered: 200,000 of 600,000 rows of 1 to 100 floats 35 -> 29 us
-// (5.4 TB/s of lines), of 1 to 20 15 -> 11. Not for pulls (30 -> 33: their stores would be the ones that straddle), and not
+// straddle them. Bound by the lines of the rows, which lie scattered: 200,000 of 600,000 rows of 1 to 100 floats 32.5 -> 28.3 us
+// (5.2 TB/s of lines; the whole step, slice, push and pull, gains 1 to 2 %), of 1 to 20 15 -> 11. Not for pulls (30 -> 33: their stores would be the ones that straddle), and not
 // where a row is far longer than the others, whose wavefront everybody would wait for.
 template <bool STREAM>
 __device__ __forceinline__ void rows_by_row(const RowsParams& p, uint64_t total, unsigned shift, bool rejected) {
