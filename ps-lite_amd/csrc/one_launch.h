@@ -501,12 +501,13 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   PSKV_ASK_ARGS("s"(d.slots), "s"(d.mask), "s"(d.st), "s"(d.keys), "s"(d.lens), "s"(d.n), "s"(d.nvals), "s"(d.ref),
                 "s"(d.off), "s"(d.tile_key), "s"(d.ntiles), "s"(d.cache_keys), "s"(d.cache_lens), "s"(d.tag.epoch),
-                "s"(d.nblk));
+                "s"(d.nblk), "s"(d.ragged));
   const unsigned nblk = d.nblk;
   if (blockIdx.x >= nblk) return;
   DevState* st = d.st;
   const uint64_t n = d.n;
   constexpr unsigned max_len = PSKV_MAX_VARLEN_ROW;
+  const unsigned longest = longest_by_row(d);
   __shared__ PartRed red;
   __shared__ unsigned long long wsum[kBlock / 64 + 1];
   __shared__ unsigned cred[kBlock / 64];
@@ -528,7 +529,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
     len[j] = (unsigned long long)(uint32_t)l;
     s += len[j];
     flags |= (unsigned)l & kReqMisaligned;
-    flags |= longer_than(d, l) ? kReqLong : 0u;
+    flags |= (unsigned)l > longest ? kReqLong : 0u;
     flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
     const bool has_left = base + j < n && base + j > 0;
     flags |= (has_left && mine.k[j] == (j ? mine.k[j - 1] : left)) ? kReqDuplicate : 0u;
@@ -541,7 +542,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_start(ReqBatch<TABLES> b) {
       of.all += (unsigned long long)(uint32_t)l;
       if (i < (uint64_t)blockIdx.x * kStartPart) of.before += (unsigned long long)(uint32_t)l;
       of.flags |= (unsigned)l & kReqMisaligned;
-      of.flags |= longer_than(d, l) ? kReqLong : 0u;
+      of.flags |= (unsigned)l > longest ? kReqLong : 0u;
       of.flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
       of.flags |= i > 0 && d.keys[i] == d.keys[i - 1] ? kReqDuplicate : 0u;
     }

@@ -1578,8 +1578,8 @@ int launch_rows(Batch& bt, int op) {
   auto nblk = [&](const Item& it) {
     if (VARLEN) {
       uint64_t blocks = (it.d.total + kRowsVarPerBlock - 1) / kRowsVarPerBlock;
-      if (op == kOpAcc && it.d.k) {
-        const uint64_t rows = (uint64_t)kBlock >> ((it.d.k & ((1u << kByRowBits) - 1)) - 1);  // of a workgroup
+      if (op == kOpAcc && it.d.ragged) {
+        const uint64_t rows = (uint64_t)kBlock >> by_row_shift(it.d.ragged);  // of a workgroup
         blocks = std::max(blocks, (it.d.n + rows - 1) / rows);
       }
       return blocks + (it.d.started ? 1 : 0);
@@ -1592,7 +1592,7 @@ int launch_rows(Batch& bt, int op) {
   bool started = false;
   for (const Item& it : bt) started = started || (VARLEN && it.d.started);
   bool by_row = false;
-  for (const Item& it : bt) by_row = by_row || (VARLEN && op == kOpAcc && it.d.k);
+  for (const Item& it : bt) by_row = by_row || (VARLEN && op == kOpAcc && it.d.ragged);
   auto pick = [&](auto op_, auto started_, auto by_row_) {
     constexpr int OP = decltype(op_)::value;
     constexpr bool STARTED = decltype(started_)::value, BY_ROW = decltype(by_row_)::value;
@@ -1826,17 +1826,31 @@ bool start_together(const Batch& bt, bool push, F floats) {
 }
 
 // How the rows of a push are added should they be ragged (rows_by_row), where the table's pushes have been so far as the host has
-// been told: about a lane per quad. Slice, push and pull, us: 2M rows of 1 to 20 floats in four tables 159 -> 146, 1M of 1 to 60 in
-// one 163 -> 148, 500,000 of 1 to 128 in 16, other ones every time, 210 -> 200 each. Not rows of a quad or two (300,000 of 1
-// to 10 in two tables 54 -> 56), of hundreds of floats, which fill wavefronts either way, nor requests that come in pieces, nor
-// (the device sees to that) where a row takes sixteen times as long as the others.
-constexpr uint64_t kByRowLeast = 8, kByRowMost = 128;
-uint64_t ragged_by_row(const pskv_table* t, const Request& r) {
+// been told: so many lanes that two or three turns of them reach rows twice as long as the mean (lengths spread evenly from 1 on).
+// Slice, push and pull, us: 2M rows of 1 to 20 floats in four tables 159 -> 146, 1M of 1 to 60 in one 163 -> 148. With a lane or more per
+// quad of the mean and two turns always, the row kernel was no quicker than by tiles where the mean is a little above a power of two
+// quads: 600,000 rows of 1 to 70 floats by tiles 56.6, so 60.2, with three turns of half the lanes 45.8; of 1 to 80 62.6, 63.6, 53.2; of 1
+// to 180 129, 123, 107; 40,000 of 1 to 80 7.3, 8.6, 7.0.
+// Not rows of a quad or two (300,000 of 1 to 10 in two tables 54 -> 56), of hundreds of floats, which fill wavefronts either way, nor
+// requests that come in pieces, nor (the device sees to that) where a row takes sixteen times as long as the others. Nor requests that
+// repeat the cached one, whose rows lie as the request has them and stay in the caches, of 1.5M to 3.5M floats, slice, push and pull by
+// tiles and by the row: 55,000 rows of 1 to 100 34.4 and 36.0, 70,000 of 1 to 100 37.2 and 38.7, of 1 to 50 30.5 and 31.0; above and
+// below it pays (90,000 of 1 to 100 43.4 and 42.7, 120,000 50.5 and 47.7; 30,000 of 1 to 80 27.3 and 26.9), and so it does for short rows
+// (250,000 of 1 to 16 38.9 and 37.6). Whether a push repeats the cached one nobody knows that starts with one launch: 40,000 of 1
+// to 100 take 30.7 and 32.3 repeated, 33.0 and 32.4 with other rows in every step.
+constexpr uint64_t kByRowLeast = 8, kByRowMost = 128, kCachedLeast = 3ull << 19, kCachedMost = 7ull << 19, kCachedRow = 16;
+// `floats`: of the whole request
+uint64_t ragged_by_row(const Item& it, uint64_t floats) {
+  const pskv_table* t = it.t;
+  const Request& r = it.r;
   const uint64_t mean = r.nvals / r.n;
+  const bool repeats = it.tag.try_cache && t->sc_track[0].hit;
+  if (repeats && mean >= kCachedRow && floats >= kCachedLeast && floats < kCachedMost) return 0;
   if (!const_cast<volatile unsigned long long*>(t->outcome)[1] || r.pipe_in || mean < kByRowLeast || mean > kByRowMost) return 0;
+  const uint64_t quads = (mean + 3) / 4;
   unsigned shift = 2;
-  while ((1ull << shift) < (mean + 3) / 4) ++shift;
-  return by_row(shift, 16 * mean + 16);
+  while ((3ull << shift) < quads * 2) ++shift;
+  return by_row(shift, (1ull << shift) < quads, 16 * mean + 16);
 }
 
 // Launches per var-len request: a push takes three (compare + scan pass 1; scan pass 2 +
@@ -1852,8 +1866,8 @@ int run_varlen(Batch& bt, bool push, bool pull) {
   }
   if (!n_largest) return PSKV_OK;
   // (keys per thread of the key-by-key kernels: by the keys of the whole launch, not of its largest table)
-  uint64_t n_launch = 0;
-  for (const Item& it : bt) n_launch += it.r.n;
+  uint64_t n_launch = 0, floats = 0;
+  for (const Item& it : bt) n_launch += it.r.n, floats += it.r.nvals;
   const bool large = n_launch >= kVarLookupLargeKeys;
   const uint64_t chunk = kBlock * (large ? 4 : 1);  // keys per workgroup of the creating lookup
   const uint64_t pad_chunk = std::min(chunk, kStartPart);  // (and of k_var_push_start)
@@ -1919,7 +1933,7 @@ int run_varlen(Batch& bt, bool push, bool pull) {
       d.tile_key = r.nvals ? static_cast<uint32_t*>(t->tiles.ptr) : nullptr;
       d.tile_aff = static_cast<TileNote*>(t->tiles_aff.ptr);
       d.ntiles = it.tiles_cap;
-      d.k = ragged_by_row(t, r);
+      d.ragged = ragged_by_row(it, floats);
     }
     int rc = growths.move();
     if (rc) return rc;

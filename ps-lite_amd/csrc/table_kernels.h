@@ -26,7 +26,10 @@ struct TableHead {
   DevState* st;
   const uint64_t* keys;  // n sorted unique keys
   const float* vals;     // SCALAR push: n values
-  float* out;            // SCALAR pull: n values
+  union {
+    float* out;          // SCALAR pull: n values
+    uint64_t ragged;     // VARLEN push: how the host would have ragged rows added (by_row)
+  };
   uint64_t n;
   uint64_t* cache_keys;  // keys (and lens) of the request whose references the workspace holds
   // SCALAR key cache (a request that repeats the cached sorted key set is served from a
@@ -57,7 +60,7 @@ struct TableReq : TableHead {
   // row kernels
   float* req;             // push: request values (read); pull: response values (written)
   uint64_t total;         // floats in req
-  uint64_t k;             // FIXED: floats per row; VARLEN push: how the host would have ragged rows added (by_row)
+  uint64_t k;             // FIXED: floats per row
   union {
     uint32_t cached;      // FIXED lookup: the first so many positions of cache_keys and ref belong together
     uint32_t started;     // VARLEN row kernels: workgroups of the k_var_*_start in front of this one, or 0
@@ -888,13 +891,14 @@ __device__ __forceinline__ void tell_ragged(DevState* st, unsigned long long* ou
   outcome[1] = ragged;
 }
 
-// TableReq::k of a VARLEN push whose rows the host takes to be ragged: 2^shift lanes per row, and the longest row for which that
-// will do; 0: a wavefront per 256 floats.
-constexpr unsigned kByRowBits = 8;
-__host__ __device__ constexpr uint64_t by_row(unsigned shift, uint64_t longest) { return longest << kByRowBits | (shift + 1); }
-__device__ __forceinline__ bool longer_than(const TableReq& d, int32_t len) {
-  return d.k && (uint64_t)(uint32_t)len > d.k >> kByRowBits;
+// TableHead::ragged of a VARLEN push whose rows the host takes to be ragged: 2^shift lanes per row, two or three turns of them, and the longest
+// row for which that will do; 0: a wavefront per 256 floats.
+constexpr unsigned kByRowBits = 8, kByRowThree = 1u << 7;
+__host__ __device__ constexpr uint64_t by_row(unsigned shift, bool three, uint64_t longest) {
+  return longest << kByRowBits | (three ? kByRowThree : 0u) | (shift + 1);
 }
+__host__ __device__ constexpr unsigned by_row_shift(uint64_t ragged) { return ((unsigned)ragged & (kByRowThree - 1)) - 1; }
+__device__ __forceinline__ unsigned longest_by_row(const TableReq& d) { return d.ragged ? (unsigned)(d.ragged >> kByRowBits) : ~0u; }
 
 // VARLEN push, first kernel: one pass over the request's keys and lens that
 //   - compares them with the cached request (when the host found the cache usable),
@@ -915,6 +919,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
   unsigned long long* __restrict__ part = d.part;
   DevState* st = d.st;
   constexpr unsigned max_len = PSKV_MAX_VARLEN_ROW;
+  const unsigned longest = longest_by_row(d);
   const ReqTag tag = d.tag;
   __shared__ unsigned long long red[kBlock / 64];
   __shared__ unsigned fred[kBlock / 64];
@@ -938,7 +943,7 @@ __global__ __launch_bounds__(kBlock) void k_var_push_begin(ReqBatch<TABLES> b) {
     const int32_t l = mine.v[j];
     s += (unsigned long long)(long long)l;
     flags |= (unsigned)l & kReqMisaligned;
-    flags |= longer_than(d, l) ? kReqLong : 0u;
+    flags |= (unsigned)l > longest ? kReqLong : 0u;
     flags |= (l < 0 || (unsigned)l > max_len) ? kReqBadLen : 0u;
     flags |= (mine.k[j] != old.k[j] || l != old.v[j]) ? kReqDiffer : 0u;
     // keys are sorted and must be unique (kv_app.h:17): a key that equals its left neighbour
@@ -1719,27 +1724,33 @@ __device__ __forceinline__ void rows_wave_varlen(const RowsParams& p, uint64_t t
   }
 }
 
-// Ragged rows of a push, the other way round: 2^shift lanes a row (about as many as it has quads, by the host's reckoning),
-// a lane a quad of it, two turns asked for together. A wavefront that starts from its tile makes five trips to memory that follow
-// from each other (facts, tile table, offsets and references, rows, values), one that starts from its rows three; its
+// Ragged rows of a push, the other way round: 2^shift lanes a row (as many as it takes, by the host's reckoning, ragged_by_row),
+// a lane a quad of it, kTurns turns asked for together. A wavefront that starts from its tile makes five trips to memory that follow
+// from each other (facts, tile table, offsets and references, rows, values), one that starts from its rows two: what it needs of the offsets
+// and references is asked for with the facts (behind them the kernel took 27.3 us where it takes 25.8). Its
 // accesses to the arena are whole quads on their own boundaries (the end of a row's last one is nobody's), where a tile's
-// straddle them. Bound by the lines of the rows, which lie scattered: 200,000 of 600,000 rows of 1 to 100 floats 32.5 -> 28.3 us
-// (5.2 TB/s of lines; the whole step, slice, push and pull, gains 1 to 2 %), of 1 to 20 15 -> 11. Not for pulls (30 -> 33: their stores would be the ones that straddle), and not
+// straddle them. Bound by the lines of the rows, which lie scattered: 200,000 of 600,000 rows of 1 to 100 floats 31.8 -> 25.8 us,
+// of 1 to 16 10.6 -> 8.9. Not for pulls (30 -> 33: their stores would be the ones that straddle), and not
 // where a row is far longer than the others, whose wavefront everybody would wait for.
-template <bool STREAM>
-__device__ __forceinline__ void rows_by_row(const RowsParams& p, uint64_t total, unsigned shift, bool rejected) {
-  const unsigned lane = threadIdx.x & 63, lanes = 1u << shift;
+struct RowOfLane {
+  uint64_t first, end, ref;  // kRefAbsent behind the last row
+};
+__device__ __forceinline__ RowOfLane row_of_lane(const RowsParams& p, unsigned shift) {
   const uint64_t wave = (uint64_t)p.blk * (kBlock / 64) + (threadIdx.x >> 6);
-  const uint64_t row = (wave << (6 - shift)) + (lane >> shift);
-  if (row >= p.n) return;
-  const uint64_t first = p.off[row], end = p.off[row + 1], r = p.ref[row];
+  const uint64_t row = (wave << (6 - shift)) + ((threadIdx.x & 63) >> shift);
+  if (row >= p.n) return RowOfLane{0, 0, kRefAbsent};
+  return RowOfLane{p.off[row], p.off[row + 1], p.ref[row]};
+}
+template <bool STREAM, unsigned kTurns>
+__device__ __forceinline__ void rows_by_row(const RowsParams& p, uint64_t total, unsigned shift, const RowOfLane& mine, bool rejected) {
+  const unsigned lane = threadIdx.x & 63, lanes = 1u << shift;
+  const uint64_t first = mine.first, end = mine.end, r = mine.ref;
   if (r == kRefAbsent) return;  // a key the lookup refused
   const bool fresh = (r & kRefNew) != 0 && !p.ignore_new;
   if (rejected && !fresh) return;
   const uint32_t len = (uint32_t)(end - first), quads = (len + 3) >> 2;
   float* dst = p.arena + (((r & ~kRefNew) >> kLenBits) << 2);
   const float* side = p.req + first;
-  constexpr unsigned kTurns = 2;
   for (uint32_t q0 = lane & (lanes - 1); q0 < quads; q0 += kTurns * lanes) {
     f32x4 x[kTurns], y[kTurns];
 #pragma unroll
@@ -1785,7 +1796,7 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
   const TableReq& d = b.t[blockIdx.y];
   // the grid is sized for the largest table of the launch: workgroups (VARLEN: wavefronts) past
   // this table's floats leave before they touch anything
-  const bool by_row = BY_ROW && d.k != 0;
+  const bool by_row = BY_ROW && d.ragged != 0;
   unsigned blk = blockIdx.x;
   if (VARLEN) {
     // every argument the common path uses, asked for at once (the compiler otherwise fetches them group by group where they
@@ -1827,7 +1838,8 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
     uint64_t total = p.total;
     f32x4 x;
     TileNote aff = {kTileNotAffine, 0};
-    if (!by_row) rows_wave_ask<OP, STREAM>(p, total, x, aff);
+    RowOfLane mine;
+    if (by_row) mine = row_of_lane(p, by_row_shift(d.ragged)); else rows_wave_ask<OP, STREAM>(p, total, x, aff);
     // a request served from the cached references creates nothing and cannot have been refused
     const bool same = facts.same_epoch == p.tag.epoch;
     if (p.tag.replay && !same) return;
@@ -1845,7 +1857,10 @@ __global__ __launch_bounds__(kBlock) void k_rows(ReqBatch<TABLES> b) {
     }
     if (by_row) {
       if ((facts.misaligned & kReqMisaligned) && !(facts.misaligned & kReqLong)) {
-        rows_by_row<STREAM>(p, total, (unsigned)(d.k & ((1u << kByRowBits) - 1)) - 1, rejected);
+        if (d.ragged & kByRowThree)
+          rows_by_row<STREAM, 3>(p, total, by_row_shift(d.ragged), mine, rejected);
+        else
+          rows_by_row<STREAM, 2>(p, total, by_row_shift(d.ragged), mine, rejected);
         return;
       }
       rows_wave_ask<OP, STREAM>(p, total, x, aff);  // (the host was wrong)

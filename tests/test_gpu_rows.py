@@ -133,7 +133,10 @@ def test_requests_that_partly_repeat(capi, orc, dev, mode, n):
 RAGGED = {"seven": lambda rng, n: rng.integers(5, 10, n), "nine": lambda rng, n: rng.integers(1, 18, n),
           "with a long one": lambda rng, n: np.where(np.arange(n) == n // 2, 4099, rng.integers(0, 40, n)),
           "up to the longest": lambda rng, n: np.where(np.arange(n) % 500 == 3, 290, rng.integers(0, 37, n)),
-          "hundreds": lambda rng, n: rng.integers(90, 165, n)}
+          "hundreds": lambda rng, n: rng.integers(90, 165, n),
+          # (three turns of 4, 8 and 16 lanes: means of 6, 12 and 24 quads; rows of two such rounds among them)
+          "six quads": lambda rng, n: rng.integers(1, 47, n), "twelve quads": lambda rng, n: np.where(np.arange(n) % 97 == 5, 385, rng.integers(1, 88, n)),
+          "twenty-four quads": lambda rng, n: rng.integers(1, 188, n)}
 
 
 @pytest.mark.parametrize("n,S", [(700, 1), (30_001, 2), (140_003, 1)])
