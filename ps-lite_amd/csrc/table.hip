@@ -403,6 +403,7 @@ struct pskv_table {
   uint64_t sc_min_keys = 0;               // requests below this size leave the cache alone; 0 = no cache
   // which pushes stream through the slot array (stream_push.h); PSKV_STREAM=0 and =1, read when a table is created, are for tests
   enum class Streams { kNever, kWhereItPays, kWhereItFits } streams = Streams::kWhereItPays;
+  uint64_t pack_min_keys = 0;             // cached keys of at least this many are packed
   bool packing = false;                   // a comparison has been asked to pack the cached keys (PackedKeys)
   unsigned stream_turn = 0;               // the counter of left keys that the newest of them used
 
@@ -1092,10 +1093,12 @@ ReqTag next_tag(pskv_table* t, const Request& r, bool back_off = false) {
 // PSKV_SCALAR_CACHE_MIN_KEYS, read when a table is created, overrides it (0 switches the cache off).
 constexpr uint64_t kScalarCacheMinKeys = 1u << 17;
 
-// Cached keys of at least this many are packed once a request has repeated them (8 MB of them: the time of smaller ones is the
-// launches'). Figures: PackedKeys. Room for it, 6 B per key, is taken when such a request is recorded in the key cache; keys that a
+// Cached keys of at least this many are packed once a request has repeated them (12 MB of them: the time of smaller ones is the
+// launches', and the comparison of packed ones starts a little later: push and pull of 1.06M keys 19.8 -> 21.9 us, of 1.25M 21.3 -> 21.5-22.2,
+// of 1.5M 22.6 -> 22.4, of 1.75M 24.0 -> 23.8, of 2M 25.6 -> 24.9). The environment variable PSKV_PACK_MIN_KEYS, read when a table
+// is created, is for tests. Figures: PackedKeys. Room for it, 6 B per key, is taken when such a request is recorded in the key cache; keys that a
 // recorded step left there (pskv_replay_*, which never packs) have none.
-constexpr uint64_t kPackKeys = 1u << 20;
+constexpr uint64_t kPackKeys = 3u << 19;
 
 // How a SCALAR request of one table relates to the table's key cache.
 enum ScalarCacheUse {
@@ -1355,7 +1358,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       // the buffers have the cached request's size). Only a request that is going to be recorded
       // pays for it: a one-off pull of 16M keys would otherwise allocate 256 MB it never uses, and
       // wait for the stream to do so.
-      rc = grow(t, &t->cache_keys, !r.replay && r.n >= kPackKeys ? PackedKeys::bytes(r.n) : r.n * sizeof(uint64_t));
+      rc = grow(t, &t->cache_keys, !r.replay && r.n >= t->pack_min_keys ? PackedKeys::bytes(r.n) : r.n * sizeof(uint64_t));
       if (rc) return rc;
       t->packing = false;
       rc = grow(t, &t->sc_vals, r.n * sizeof(float));
@@ -1380,7 +1383,7 @@ int run_scalar(Batch& bt, bool push, bool pull) {
       const bool per_key = plan[i].use == kScTry && !push && !t->sc_dirty && plan[i].kind_before == 0 && r.replay != kReplayCapture;
       d.cache_mode = per_key ? kCachePerKey : kCacheOn;
       any_cache = true;
-      if (!per_key && it.tag.try_cache && !r.replay && r.n >= kPackKeys && t->cache_keys.bytes >= PackedKeys::bytes(r.n)) {
+      if (!per_key && it.tag.try_cache && !r.replay && r.n >= t->pack_min_keys && t->cache_keys.bytes >= PackedKeys::bytes(r.n)) {
         // (packed they are as soon as they have been asked for, further up the stream; the device looks, and says where it was not so)
         volatile unsigned long long* const told = t->outcome + 2;
         if (*told == kNotPacked) t->packing = false;
@@ -2511,6 +2514,8 @@ int pskv_table_create(pskv_table** out, const pskv_opts* opts) {
     t->streams = std::atoi(e) ? pskv_table::Streams::kWhereItFits : pskv_table::Streams::kNever;
   t->sc_min_keys = kScalarCacheMinKeys;
   if (const char* e = std::getenv("PSKV_SCALAR_CACHE_MIN_KEYS")) t->sc_min_keys = std::strtoull(e, nullptr, 10);
+  t->pack_min_keys = kPackKeys;
+  if (const char* e = std::getenv("PSKV_PACK_MIN_KEYS")) t->pack_min_keys = std::strtoull(e, nullptr, 10);
   auto fail = [&](int rc) {
     pskv_table_destroy(t);
     return rc;

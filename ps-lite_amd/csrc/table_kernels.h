@@ -485,7 +485,7 @@ __global__ __launch_bounds__(kBlock) void k_same_keys(HeadBatch<TABLES> b) {
 // its keys twice, 30 B, two tables of 8M keys of which one cannot be packed took 53 us to compare and 163 to push and pull. They take 36
 // and 127; as long as nothing was packed they took 38 and 131.)
 // Bound by memory: 14 B per key instead of 16. Push and pull of 16M repeated keys took 130 us and take 122.6 (three tables on three
-// streams in turn: 145.8 and 137), of 8M 73.1 and 69.1, of 2M 26 and 24.5, of 1M 18.6 and 18.4. The packed words are left in the
+// streams in turn: 145.8 and 137), of 8M 73.1 and 69.1, of 2M 26 and 24.5. The packed words are left in the
 // memory-side cache: loads that pass it by take 16M keys of three tables down to 121 us, but those of one alone up to 134-139.
 // 52 registers: with the cached keys themselves held as well (140) three wavefronts per SIMD took longer than what was read less.
 struct PackedKeys {

@@ -10,6 +10,11 @@ from test_gpu_store import _check_dump
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def packs_a_million(monkeypatch):
+    monkeypatch.setenv("PSKV_PACK_MIN_KEYS", str(1 << 20))
+
+
 def keys_of(rng, n, wide=False):
     keys = np.cumsum(rng.integers(2, 1 << 30, n, dtype=np.uint64))
     if wide:

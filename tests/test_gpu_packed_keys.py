@@ -1,4 +1,4 @@
-"""Requests of 1,048,576 keys and more that repeat the cached one, whose keys a SCALAR table then keeps packed, 48 bits each next to
+"""Requests of many keys that repeat the cached one, whose keys a SCALAR table then keeps packed, 48 bits each next to
 their neighbour: the same keys, keys that differ in single places, neighbours too far apart. Against the CPU oracle, bit for bit."""
 import numpy as np
 import pytest
@@ -8,6 +8,11 @@ from helpers import assert_bits_equal, to_dev
 from test_gpu_store import _check_dump
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def packs_a_million(monkeypatch):
+    monkeypatch.setenv("PSKV_PACK_MIN_KEYS", str(1 << 20))
 
 
 @pytest.mark.parametrize("n,skip", [(1 << 20, 0), ((1 << 20) + 1, 1), ((1 << 20) + 255, 0), ((1 << 20) + 1023, 0)])

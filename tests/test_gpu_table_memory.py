@@ -1,4 +1,6 @@
 """What requests leave allocated for a SCALAR table beside its slot array."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -11,6 +13,7 @@ pytestmark = pytest.mark.gpu
 def held_by(capi, make):
     """Bytes of device memory that what `make` returns holds on to."""
     import torch
+    gc.collect()  # (tables of earlier tests)
     torch.cuda.synchronize()
     capi.device_trim()
     before = torch.cuda.mem_get_info()[0]
@@ -21,12 +24,13 @@ def held_by(capi, make):
     return before - after
 
 
-def test_the_key_cache_of_keys_that_are_never_packed(capi, dev, monkeypatch):
-    """8 B for a cached key, 4 for its value and 4 for its slot number, an eighth to spare and the steps that the arrays come in (an
-    eighth of a power of two): 1.125 * 1.125 * 16 = 20.3 B per key. Beside each table 2 MiB for what the system rounds up."""
+@pytest.mark.parametrize("n,per_key", [(900_000, 16), ((3 << 19) - 1, 16), (3 << 19, 22)])
+def test_the_key_cache_and_its_packed_keys(capi, dev, monkeypatch, n, per_key):
+    """8 B for a cached key, 4 for its value and 4 for its slot number, 6 more where keys are packed; an eighth to spare, and the steps that
+    the arrays come in, an eighth of the next power of two: a quarter at most. Beside each table 2 MiB for what the system rounds up."""
     import torch
-    announce("key cache memory")
-    n, S = 900_000, 8
+    announce("key cache memory", n)
+    S = 4
     keys = [to_dev(unique_keys(np.random.default_rng(s), n), dev) for s in range(S)]
     all_keys, pos = torch.cat(keys), np.arange(S + 1, dtype=np.uint64) * n
     vals, out = (torch.zeros(S * n, device=dev) for _ in range(2))
@@ -42,7 +46,7 @@ def test_the_key_cache_of_keys_that_are_never_packed(capi, dev, monkeypatch):
     with_cache = held_by(capi, steps)
     monkeypatch.setenv("PSKV_SCALAR_CACHE_MIN_KEYS", "0")
     without = held_by(capi, steps)
-    assert 16 * n * S <= with_cache - without <= S * (20.3 * n + (2 << 20)), (with_cache - without) / (n * S)
+    assert per_key * n * S <= with_cache - without <= S * (1.125 * 1.25 * per_key * n + (2 << 20)), (with_cache - without) / (n * S)
 
 
 @pytest.mark.parametrize("then", ["nothing", "pull", "small push"])
@@ -53,23 +57,24 @@ def test_the_room_that_a_push_streams_through(capi, dev, monkeypatch, then):
     import torch
     announce("streaming memory", then)
     n = 4_000_000
-    keys = to_dev(unique_keys(np.random.default_rng(1), n), dev)
+    some = unique_keys(np.random.default_rng(1), n)
+    keys, some = to_dev(some, dev), some[:1000]
     vals, out = torch.zeros(n, device=dev), torch.zeros(n, device=dev)
 
     def filled():
-        t = capi.Table(capi.MODE_SCALAR, initial_capacity=n)
+        t = capi.Table(capi.MODE_SCALAR, initial_capacity=10_000_000)  # (no growth is near, nor an array for one)
         t.prof_enable()
         t.push(keys, vals)
-        t.size()  # (it is known then that the keys of the next request fit)
         if then == "pull":
-            t.pull(keys[:n // 64], out)
+            t.pull(keys, out)
         elif then == "small push":
-            t.push(keys[:1000], vals[:1000])
+            t.push(some, np.zeros(1000, np.float32))  # (from host memory: it does not stream)
         t.sync()
         return t
 
+    monkeypatch.setenv("PSKV_STREAM", "1")
     t = filled()
-    assert t.prof_read(capi.KERNEL_REHASH)[0] == 3  # (it streams: nobody asked for it)
+    assert t.prof_read(capi.KERNEL_REHASH)[0] == 3
     t.close()
     with_room = held_by(capi, filled)
     monkeypatch.setenv("PSKV_STREAM", "0")
