@@ -33,8 +33,16 @@ constexpr unsigned kMatchTurn = kMatchLds / kMatchBlock;  // source keys a lane 
 // A longer stretch than so many pieces is sampled, not staged. (Pieces follow from each other, but read in one go
 // what the sampled search reads key by key: they pay while there are workgroups enough to fill the GPU.)
 constexpr unsigned kMatchPieces = 8, kMatchPiecesFew = 3;
-// Tiles (of kMatchItems keys a lane, and of one) up to which the workgroups search for themselves, without a launch in front of them.
+// Tiles (of kMatchItems keys a lane, and of one) up to which the workgroups search for themselves, without a launch in front of them;
+// tiles of kMatchItems keys a lane up to as many as those of one, too, where the other set is small (own_search).
 constexpr unsigned kOwnSpans = 2560, kOwnSpansFew = 4096;
+// What the search in front costs a call hardly depends on the sets; the workgroups' own costs by the tiles and by how many rounds each
+// takes. us per call, with the launch in front and without: 30,000 into 3M keys 27.0 and 25.3, 1M into 3M 33.1 and 31.6, 2M into 3M 35.4
+// and 34.7, 2.6M into 3M 36.4 and 36.6; 1M into 3.5M 34.3 and 33.9, 1.5M into 3.5M 35.3 and 35.8; 100,000 into 4.1M 31.7 and 31.0, 700,000
+// into 4.1M 35.1 and 35.5.
+constexpr bool own_search(uint64_t n_near, uint64_t n_far, unsigned blocks, bool few) {
+  return blocks <= kOwnSpans || (blocks <= kOwnSpansFew && (few || n_near * 7 / 4 + n_far <= 29ull << 18));
+}
 constexpr uint64_t kNoMatch = ~0ull;
 constexpr unsigned kCounts = 64;        // counters of matched keys, each on a line of its own
 constexpr unsigned kCountStride = 16;
@@ -527,7 +535,7 @@ extern "C" int pskv_match(int device, const uint64_t* src_keys, size_t n_src, co
   const bool few = n_near < kFewKeys || n_far / n_near >= 2;
   const unsigned tile = kMatchBlock * (few ? 1 : kMatchItems);
   const unsigned blocks = (unsigned)((n_near + tile - 1) / tile);
-  const bool own = blocks <= (few ? kOwnSpansFew : kOwnSpans);
+  const bool own = own_search(n_near, n_far, blocks, few);
   if (!own) {
     int rc = room(&c->spans, ((size_t)blocks + 1) * sizeof(uint64_t), st);
     if (rc) return rc;

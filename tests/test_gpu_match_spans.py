@@ -1,6 +1,6 @@
-"""pskv_match where its workgroups stop finding their stretches themselves (2,560 tiles of 1,024 keys, or 4,096 of 256 where the
-other set is twice as large): as many tiles and one more, and tiles whose keys all lie in front of, behind or between those of
-the other set. Against numpy, bit for bit."""
+"""pskv_match where its workgroups stop finding their stretches themselves (2,560 tiles of 1,024 keys, 4,096 of them where the
+other set is small, or of 256 where it is twice as large): as many tiles and one more, and tiles whose keys all lie in front
+of, behind or between those of the other set. Against numpy, bit for bit."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n_src,n_dst", [(3_000_000, 4096 * 1024), (3_000_000, 4096 * 1024 + 1),
                                          (2_200_000, 4096 * 256), (2_200_000, 4096 * 256 + 1),
-                                         (1_900_000, 2560 * 1024), (1_900_000, 2560 * 1024 + 1)])
+                                         (3_200_000, 2560 * 1024), (3_200_000, 2560 * 1024 + 1),
+                                         ((29 << 18) - 5_250_000, 3_000_000), ((29 << 18) - 5_249_999, 3_000_000)])
 @pytest.mark.parametrize("k", [1, 3])
 def test_as_many_tiles_as_search_for_themselves(capi, dev, n_src, n_dst, k):
     announce("match own spans", n_src, n_dst, k)
